@@ -20,7 +20,7 @@
 extern "C" {
 #endif
 
-#define XS_ABI_VERSION 16
+#define XS_ABI_VERSION 17
 
 /* element types */
 enum { XS_F32 = 0, XS_BF16 = 1 };
@@ -170,6 +170,14 @@ size_t xs_slstm_workspace_bytes(int32_t B, int32_t T, int32_t NH, int32_t dh);
  * it runs the step kernel of xs_slstm_step (same bits, status.step_kernel = 1).
  */
 int xs_slstm_forward(const xs_slstm_args *args);
+
+/*
+ * The same with a word of pinned host memory (NULL: none) that becomes 1 when a bounded wait of the call ran out
+ * (status.aborted), written by the kernel itself: a caller that only wants to know whether one of its calls gave up
+ * looks at the word when it likes, with no copy of the status block and no event behind every call.  The library never
+ * clears it.  No counterpart in the reference.
+ */
+int xs_slstm_forward_watched(const xs_slstm_args *args, uint32_t *abort_host);
 
 /*
  * xs_slstm_forward for callers that cannot allocate device memory or pass a workspace (code under HIP graph

@@ -6,6 +6,8 @@ fails loudly with the command that builds it.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from typing import Optional
 
@@ -15,13 +17,14 @@ LIB_PATH = os.environ.get("XLSTM_AMD_LIB", os.path.join(PKG, "lib", "libxlstm_am
 XS_F32, XS_BF16 = 0, 1
 XS_ERR_UNSUPPORTED = -5
 STATIC_SCRATCH_BYTES = (4 << 20) + (64 << 10)
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 EXPORTS = (
     "xs_abi_version",
     "xs_last_error",
     "xs_slstm_workspace_bytes",
     "xs_slstm_forward",
+    "xs_slstm_forward_watched",
     "xs_slstm_step",
     "xs_slstm_forward_static",
     "xs_slstm_tile_r_for_steps",
@@ -199,6 +202,8 @@ def load() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.restype = ctypes.c_int
         fn.argtypes = [ctypes.POINTER(SlstmArgs)]
+    lib.xs_slstm_forward_watched.restype = ctypes.c_int
+    lib.xs_slstm_forward_watched.argtypes = [ctypes.POINTER(SlstmArgs), ctypes.c_void_p]
     for fn in (lib.xs_slstm_backward_prepare, lib.xs_slstm_backward, lib.xs_slstm_backward_params, lib.xs_slstm_backward_tile_r):
         fn.restype = ctypes.c_int
         fn.argtypes = [ctypes.POINTER(SlstmBwdArgs)]
@@ -220,3 +225,30 @@ def load() -> ctypes.CDLL:
 
 def last_error() -> str:
     return load().xs_last_error().decode()
+
+
+HOST_PATH = os.path.join(PKG, "lib", "_xlstm_host.so")
+_HOST = None
+
+
+def host():
+    """The native host path (``csrc/host_path.cpp``), bound to the loaded engine; raises if it has not been built."""
+    global _HOST
+    if _HOST is not None:
+        return _HOST
+    lib = load()
+    if not os.path.exists(HOST_PATH):
+        raise RuntimeError(f"xlstm_amd: native host path not built ({HOST_PATH} missing). Build it with `python -m xlstm_amd.build`.")
+    from torch.nn.modules import module as torch_module
+
+    from .functional import EngineError
+
+    spec = importlib.util.spec_from_loader("_xlstm_host", importlib.machinery.ExtensionFileLoader("_xlstm_host", HOST_PATH))
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    names = ("xs_slstm_step", "xs_slstm_forward_watched", "xs_slstm_workspace_bytes", "xs_last_error", "xs_causal_conv_silu",
+             "xs_headwise_gates", "xs_headwise_group_norm")
+    mod.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names}, EngineError,
+             torch_module._global_forward_hooks, torch_module._global_forward_pre_hooks)
+    _HOST = mod
+    return mod

@@ -14,6 +14,8 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
 SOURCES = [os.path.join(PKG, "csrc", "slstm_hip.hip")]
 LIB = os.path.join(PKG, "lib", "libxlstm_amd.so")
+HOST_SOURCE = os.path.join(PKG, "csrc", "host_path.cpp")
+HOST_LIB = os.path.join(PKG, "lib", "_xlstm_host.so")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-shared", "-fPIC",
@@ -44,6 +46,29 @@ def build(verbose: bool = False, extra_flags=(), out: str = LIB) -> str:
     return out
 
 
+def build_host(verbose: bool = False, out: str = HOST_LIB) -> str:
+    """Builds the native host path, a CPython extension over ATen (host code only: ``g++``)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    os.makedirs(os.path.dirname(out), exist_ok=True)
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-w",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-I", os.path.join(ROOT, "include"), "-I", sysconfig.get_paths()["include"],
+           *(f for p in cpp_extension.include_paths(device_type="cuda") for f in ("-isystem", p)),
+           HOST_SOURCE, "-o", out, "-L", libs, f"-Wl,-rpath,{libs}", "-L", "/opt/rocm/lib",
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-lamdhip64"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed ({res.returncode}):\n{res.stdout}")
+    return out
+
+
 if __name__ == "__main__":
     argv = sys.argv[1:]
     target = LIB
@@ -52,4 +77,6 @@ if __name__ == "__main__":
         target = os.path.abspath(argv[i + 1])
         del argv[i:i + 2]
     print(build(verbose=True, extra_flags=tuple(argv), out=target))
+    if target == LIB:
+        print(build_host(verbose=True))
     sys.exit(0)

@@ -28,6 +28,7 @@ What differs, on purpose:
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass, field
 from math import sqrt
 from typing import Callable, Literal, Optional, Sequence, Union
@@ -225,12 +226,11 @@ class _Runtime:
     calls in flight, the cached bf16 copy of R, the decode plan.  A copied or unpickled cell starts with none."""
 
     def __init__(self):
-        self.workspaces = {}
         self.status_ring = None
-        self.last_workspace = None
+        self.last_workspace = None  # of the latest call, or `native` where that call was the native path's
         self.r_bf16 = None
         self.step_plan = None
-        self.last_step = None  # (state tensor handed out by the last fast step, its version, h tensor, its version)
+        self.native = None  # the cell's native host path (_lib.host().CellPath), which also remembers the last fast step
 
     def __deepcopy__(self, memo):
         return _Runtime()
@@ -297,7 +297,7 @@ class sLSTMCell_hip(nn.Module):
         if not skip_backend_init:
             from . import _lib
 
-            _lib.load()  # fail loudly here, not at the first forward, if the engine is missing
+            _lib.host()  # fail loudly here, not at the first forward, if the engine or its host path is missing
 
     def __repr__(self):
         return (
@@ -422,15 +422,15 @@ class sLSTMCell_hip(nn.Module):
     def _workspace(self, B: int, device) -> torch.Tensor:
         """The cell's workspace for calls on the current stream of ``device`` (calls on one stream run one after the
         other, so they can share it; calls on different streams may overlap and get one each)."""
-        stream = torch.cuda.current_stream(device).cuda_stream
-        NH, dh = self.config.num_heads, self.head_dim
-        need = F_hip._lib.load().xs_slstm_workspace_bytes(B, 1, NH, dh)
-        key = (device, stream)
-        ws = self._rt.workspaces.get(key)
-        if ws is None or ws.numel() < need:
-            ws = torch.empty(need, dtype=torch.uint8, device=device)
-            self._rt.workspaces[key] = ws
-        return ws
+        return self._native().workspace(B, torch.empty(0, dtype=torch.uint8, device=device))
+
+    def _native(self):
+        """This cell's native host path: frequent calls (decode steps, inference calls) go through it in one hop."""
+        native = self._rt.native
+        if native is None:
+            native = F_hip._lib.host().CellPath(self._parameters, self.config.num_heads, self.head_dim)
+            self._rt.native = native
+        return native
 
     def _watch(self, workspace: torch.Tensor) -> None:
         """Queues a copy of the call's ``aborted`` word to pinned host memory behind the kernel and looks at the
@@ -460,11 +460,9 @@ class sLSTMCell_hip(nn.Module):
         ring["next"] = (i + 1) % self._STATUS_SLOTS
 
     def _poll_status(self, block: bool) -> None:
-        ring = self._rt.status_ring
-        if ring is None:
-            return
-        bad = False
-        for i, ev in enumerate(ring["events"]):
+        native, ring = self._rt.native, self._rt.status_ring
+        bad = native is not None and native.poll(block)  # (inference calls: the kernel itself tells the host)
+        for i, ev in enumerate(ring["events"] if ring is not None else ()):
             if ev is None:
                 continue
             if block:
@@ -489,6 +487,8 @@ class sLSTMCell_hip(nn.Module):
         ws = self._rt.last_workspace
         if ws is None:
             raise RuntimeError("the cell has not been called yet")
+        if ws is self._rt.native:  # (the latest call was a sequence call on the native path, which knows its workspace)
+            ws = ws.last_workspace()
         return F_hip.read_status(ws)
 
     def _run(self, input, state, reset_mask, step: bool, state_out=None):
@@ -543,8 +543,15 @@ class sLSTMCell_hip(nn.Module):
         del lengths  # unused, as in the reference
         if input.dim() == 3 and input.shape[1 if self.config.input_shape == "BSGNH" else 0] == 1:
             fast = self._step_fast(input, state, reset_mask, None)
+        else:
+            native = self._rt.native
+            if native is None and input.is_cuda:
+                native = self._native()
+            fast = native.forward(input, state, reset_mask, self.config, self.keep_state_fp32) if native is not None else None
             if fast is not None:
-                return fast
+                self._rt.last_workspace = native
+        if fast is not None:
+            return fast
         return self._run(input, state, reset_mask, step=False)
 
     def step(self, input: torch.Tensor, state: Optional[torch.Tensor] = None, reset_mask=None,
@@ -570,7 +577,14 @@ class sLSTMCell_hip(nn.Module):
 
     def _step_fast(self, input, state, reset_mask, state_out, h_out=None, h_prev=None):
         """The decode steady state (float32 state carried over, no mask, no autograd) through a cached
-        ``StepPlan``: the generic path spends more host time per token than the kernel runs."""
+        ``StepPlan`` and the native host path: the generic path spends more host time per token than the kernel runs."""
+        rt = self._rt
+        native = rt.native
+        if native is not None:
+            fast = native.step(input, state, reset_mask, state_out, h_out, h_prev, self.config, self.keep_state_fp32)
+            if fast is not None:
+                rt.last_workspace = rt.step_plan[1].workspace
+                return fast
         if (reset_mask is not None or state is None or state.dtype != torch.float32 or not state.is_contiguous()
                 or input.dtype not in (torch.float32, torch.bfloat16) or self.config.input_shape != "BSGNH"
                 or input.dim() != 3 or input.shape[1] != 1 or not input.is_contiguous() or not input.is_cuda
@@ -583,30 +597,31 @@ class sLSTMCell_hip(nn.Module):
         self._check_input(input)
         B = input.shape[0]
         self._check_state(B, state)
+        if not self._plan_step(B, input.dtype, input.device):
+            raise ValueError("the step's tensors do not fit the cell's parameters (device)")
+        if h_out is not None and (h_out.dtype != input.dtype or h_out.numel() != B * self.config.hidden_size
+                                  or not h_out.is_contiguous()):
+            raise ValueError("h_out must be a contiguous [1, B, H] tensor in the input dtype")
+        with torch.cuda.device(input.device):
+            fast = self._native().step(input, state, None, state_out, h_out, h_prev, self.config, self.keep_state_fp32)
+        if fast is None:
+            raise ValueError("h_prev or state_out does not fit the step (dtype, size or device)")
+        rt.last_workspace = rt.step_plan[1].workspace
+        return fast
+
+    def _plan_step(self, B: int, dtype: torch.dtype, device) -> bool:
+        """Makes the plan of decode steps of ``B`` rows from the current parameters and hands it to the native path."""
         r, b = self._recurrent_kernel_, self._bias_
-        key = (B, input.dtype, input.device, r.data_ptr(), r._version, b.data_ptr(), b._version)
+        if r.device != device or b.device != device:
+            return False
+        key = (B, dtype, device, r.data_ptr(), 0 if r.is_inference() else r._version, b.data_ptr(),
+               0 if b.is_inference() else b._version)
         cached = self._rt.step_plan
         if cached is None or cached[0] != key:
-            plan = F_hip.StepPlan(B, r.detach(), b.detach().view(self.config.num_heads, 4, self.head_dim), wx_dtype=input.dtype)
-            cached = (key, plan)
-            self._rt.step_plan = cached
-        H = self.config.hidden_size
-        h = h_out if h_out is not None else torch.empty((1, B, H), dtype=input.dtype, device=input.device)
-        if h.dtype != input.dtype or h.numel() != B * H or not h.is_contiguous():
-            raise ValueError("h_out must be a contiguous [1, B, H] tensor in the input dtype")
-        s_out = state_out if state_out is not None else torch.empty((4, B, H), dtype=torch.float32, device=input.device)
-        if h_prev is None and input.dtype == torch.bfloat16:
-            # The state this cell handed out last time comes back untouched: the h it returned with it is that state's
-            # y plane in bfloat16, the operand the step kernel wants (half the bytes, and the pipelined kernel).
-            last = self._rt.last_step
-            if (last is not None and last[0] is state and state._version == last[1] and last[2]._version == last[3]
-                    and last[2] is not h):
-                h_prev = last[2]
-        with torch.cuda.device(input.device):
-            cached[1](input, state, s_out, h, h_prev=h_prev)
-        self._rt.last_workspace = cached[1].workspace
-        self._rt.last_step = (s_out, s_out._version, h, h._version) if self.keep_state_fp32 else None
-        return self._permute_output(h), (s_out if self.keep_state_fp32 else s_out.to(input.dtype))
+            plan = F_hip.StepPlan(B, r.detach(), b.detach().view(self.config.num_heads, 4, self.head_dim), wx_dtype=dtype)
+            self._rt.step_plan = cached = (key, plan)
+            self._native().set_plan(plan, ctypes.addressof(plan._args), B, r, b)
+        return True
 
 
 def reference_cell_params_to_hip(recurrent_kernel_int: torch.Tensor, bias_int: torch.Tensor, source_backend: str,

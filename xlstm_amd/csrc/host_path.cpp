@@ -1,0 +1,734 @@
+// Native host path of the calls a program makes often: a decode step and an inference call of a cell, and the same of
+// a layer.  What the Python layers of cell.py, layer.py and functional.py do for such a call - look at dtypes, strides,
+// versions and modes, allocate the outputs, fill an argument block, launch - takes 15 us per cell call and 75 us per
+// layer call there, more than the kernels run; here it takes about 4 and 8.
+//
+// Every function returns None, with nothing launched, for a call that is not one of those it covers (autograd is
+// recording, hooks are registered, another dtype or layout ...): the caller then takes its general path.  The results
+// are those of the general path: the same kernels with the same arguments.
+//
+// A plain CPython extension over ATen (no pybind11: its argument casters cost as much as the rest of a step call).
+// The engine's C entry points come as addresses from the library that _lib.py has loaded, so that one loaded engine
+// serves both.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/autocast_mode.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <mutex>
+#include <unordered_map>
+#include <vector>
+
+#include "xlstm_amd.h"
+
+namespace {
+
+// ---- what bind() hands over from Python
+struct Engine {
+  decltype(&xs_slstm_step) step = nullptr;
+  decltype(&xs_slstm_forward_watched) forward = nullptr;
+  decltype(&xs_slstm_workspace_bytes) workspace_bytes = nullptr;
+  decltype(&xs_last_error) last_error = nullptr;
+  decltype(&xs_causal_conv_silu) conv = nullptr;
+  decltype(&xs_headwise_gates) gates = nullptr;
+  decltype(&xs_headwise_group_norm) norm = nullptr;
+  PyObject *error = nullptr;              // functional.EngineError
+  PyObject *global_hooks[2] = {nullptr, nullptr};  // hooks on every module of the process
+} g_engine;
+
+// interned attribute and dictionary keys
+struct Names {
+  PyObject *r, *b, *weight, *bias, *conv_state, *slstm_state, *input_shape, *output_shape, *keep_state_fp32, *config;
+  PyObject *modules, *parameters, *forward_hooks, *forward_pre_hooks, *training, *p, *eps, *conv1d, *conv, *fgate, *igate, *zgate, *ogate;
+  PyObject *group_norm, *slstm_cell, *dropout, *fused_pre_ops, *rt, *bsgnh;
+} g_names;
+
+struct PyRef {  // owns one reference
+  PyObject *o;
+  explicit PyRef(PyObject *p = nullptr) : o(p) {}
+  ~PyRef() { Py_XDECREF(o); }
+  PyRef(const PyRef &) = delete;
+  PyRef &operator=(const PyRef &) = delete;
+  PyObject *release() { PyObject *p = o; o = nullptr; return p; }
+};
+
+struct PythonError {};                                   // a Python exception is set
+struct NotCovered {};                                    // the general path takes this call
+[[noreturn]] void engine_failed(int rc) {
+  PyErr_Format(g_engine.error, "xlstm_amd error %d: %s", rc, g_engine.last_error());
+  throw PythonError{};
+}
+inline void launched(int rc) { if (rc != XS_OK) engine_failed(rc); }
+
+inline const at::Tensor &tensor_of(PyObject *o) {
+  if (!THPVariable_Check(o)) throw NotCovered{};
+  return THPVariable_Unpack(o);
+}
+inline bool absent(PyObject *o) { return o == nullptr || o == Py_None; }
+
+inline void *stream_of(const at::Device &d) { return (void *)c10::hip::getCurrentHIPStream(d.index()).stream(); }
+inline int dtype_code(at::ScalarType t) { return t == at::kBFloat16 ? XS_BF16 : XS_F32; }
+inline bool aligned(const void *p, uintptr_t n) { return ((uintptr_t)p) % n == 0; }
+
+// the version of a tensor's data, or 0 where none is kept (inference mode)
+inline uint32_t version_of(const at::Tensor &t) { return t.is_inference() ? 0u : t._version(); }
+inline bool versioned(const at::Tensor &t) { return !t.is_inference(); }
+
+// ---- abort words: pinned host words that a sequence kernel writes when one of its bounded waits ran out.  Pages of
+// words live as long as the process (a kernel of a cell that is gone may still be running), a word given back is the
+// last to be handed out again, and there are no more words than cells were alive at once (rounded up to a page).
+class WordPool {
+ public:
+  uint32_t *take() {
+    std::lock_guard<std::mutex> lock(mu_);
+    if (next_ == free_.size()) {
+      void *page = nullptr;
+      if (hipHostMalloc(&page, 4096, hipHostMallocDefault) != hipSuccess) return nullptr;
+      free_.clear(); next_ = 0;
+      for (int i = 0; i < 4096 / 64; ++i) free_.push_back((uint32_t *)((char *)page + 64 * i));
+    }
+    uint32_t *w = free_[next_++];
+    if (next_ > 1024) { free_.erase(free_.begin(), free_.begin() + (long)next_); next_ = 0; }
+    __atomic_store_n(w, 0u, __ATOMIC_RELEASE);
+    return w;
+  }
+  void give_back(uint32_t *w) {
+    std::lock_guard<std::mutex> lock(mu_);
+    free_.push_back(w);
+  }
+ private:
+  std::mutex mu_;
+  std::vector<uint32_t *> free_;  // [next_, end): free words, oldest first
+  size_t next_ = 0;
+} g_words;
+
+// ---- one cell
+struct CellPath {
+  PyObject *parameters = nullptr;  // its parameter dict
+  int64_t NH = 0, dh = 0;
+  // decode: the plan (functional.StepPlan) whose argument block is used, and what it was made for
+  PyObject *plan = nullptr;
+  xs_slstm_args *step_args = nullptr;
+  int64_t step_B = 0;
+  at::ScalarType step_dtype = at::kFloat;
+  at::Device device{at::kCPU};
+  const void *r_ptr = nullptr, *b_ptr = nullptr;
+  uint32_t r_version = 0, b_version = 0;
+  at::Tensor last_state, last_h;   // what the last step handed out (float32 state kept), and their versions
+  uint32_t last_state_version = 0, last_h_version = 0;
+  // sequences: a workspace per (device, stream), a float32 copy of the bias where the parameter is not float32
+  struct Workspace { int device; void *stream; at::Tensor t; };
+  std::vector<Workspace> workspaces;
+  at::Tensor bias32;
+  const void *bias32_of = nullptr;
+  uint32_t bias32_version = 0;
+  at::Tensor last_workspace;
+  uint32_t *abort_word = nullptr;
+  uint64_t devices_used = 0;
+
+  const at::Tensor &parameter(PyObject *name) const {
+    PyObject *o = PyDict_GetItem(parameters, name);
+    if (!o) throw NotCovered{};
+    return tensor_of(o);
+  }
+  ~CellPath() {
+    Py_XDECREF(parameters);
+    Py_XDECREF(plan);
+    if (abort_word) g_words.give_back(abort_word);
+  }
+
+  bool records(const at::Tensor &x, const at::Tensor *state, const at::Tensor &r, const at::Tensor &b) const {
+    return at::GradMode::is_enabled() && (x.requires_grad() || r.requires_grad() || b.requires_grad() || (state && state->requires_grad()));
+  }
+
+  at::Tensor &workspace(int64_t B, const at::Device &d) {
+    void *stream = stream_of(d);
+    const size_t need = g_engine.workspace_bytes((int32_t)B, 1, (int32_t)NH, (int32_t)dh);
+    Workspace *w = nullptr;
+    for (auto &it : workspaces)
+      if (it.device == d.index() && it.stream == stream) { w = &it; break; }
+    if (!w) {
+      // (a program that makes a new stream per call would otherwise collect workspaces without end; a stream's
+      // allocations are handed on in stream order by the caching allocator, so dropping the oldest is safe)
+      if (workspaces.size() >= 16) workspaces.erase(workspaces.begin());
+      workspaces.push_back(Workspace{(int)d.index(), stream, at::Tensor()});
+      w = &workspaces.back();
+    }
+    if (!w->t.defined() || (size_t)w->t.numel() < need)
+      w->t = at::empty({(int64_t)need}, at::TensorOptions().dtype(at::kByte).device(d));
+    return w->t;
+  }
+
+  void raise_if_aborted() {
+    if (abort_word && __atomic_load_n(abort_word, __ATOMIC_ACQUIRE)) {
+      __atomic_store_n(abort_word, 0u, __ATOMIC_RELEASE);
+      PyErr_SetString(g_engine.error,
+                      "an earlier sLSTM sequence call (forward or backward) on the hip backend gave up waiting for some of its "
+                      "compute units (they were held by other work on the GPU); its outputs were set to NaN");
+      throw PythonError{};
+    }
+  }
+};
+
+struct CellPathObject { PyObject_HEAD CellPath *c; };
+
+// the config's output_shape as the strides of [S,B,H] memory: 'BNSH', 'SBH', 'BSH' or 'SBNH'
+enum class OutShape { BNSH, SBH, BSH, SBNH };
+OutShape out_shape(PyObject *config) {
+  PyRef v(PyObject_GetAttr(config, g_names.output_shape));
+  if (!v.o) throw PythonError{};
+  const char *s = PyUnicode_Check(v.o) ? PyUnicode_AsUTF8(v.o) : nullptr;
+  if (!s) { PyErr_Clear(); throw NotCovered{}; }
+  if (!strcmp(s, "BNSH")) return OutShape::BNSH;
+  if (!strcmp(s, "SBH")) return OutShape::SBH;
+  if (!strcmp(s, "BSH")) return OutShape::BSH;
+  if (!strcmp(s, "SBNH")) return OutShape::SBNH;
+  throw NotCovered{};
+}
+struct Shape4 { std::array<int64_t, 4> size, stride; int n; };
+Shape4 shape_of(OutShape o, int64_t S, int64_t B, int64_t NH, int64_t dh) {
+  const int64_t H = NH * dh;
+  switch (o) {
+    case OutShape::BNSH: return {{B, NH, S, dh}, {H, dh, B * H, 1}, 4};
+    case OutShape::SBH: return {{S, B, H, 0}, {B * H, H, 1, 0}, 3};
+    case OutShape::BSH: return {{B, S, H, 0}, {H, B * H, 1, 0}, 3};
+    default: return {{S, B, NH, dh}, {B * H, H, dh, 1}, 4};
+  }
+}
+bool input_is_bsgnh(PyObject *config) {
+  PyRef v(PyObject_GetAttr(config, g_names.input_shape));
+  if (!v.o) throw PythonError{};
+  return v.o == g_names.bsgnh || PyUnicode_Compare(v.o, g_names.bsgnh) == 0;
+}
+
+// ---- one decode step into given buffers; the plan and the operand hint as sLSTMCell_hip._step_fast chooses them
+struct StepResult { at::Tensor h, state; };  // h: [1,B,H] memory, state: float32 [4,B,H]
+StepResult run_step(CellPath &c, const at::Tensor &x, const at::Tensor &state, const at::Tensor *state_out, const at::Tensor *h_out,
+                    const at::Tensor *h_prev, const Shape4 *h_shape, bool keep_state) {
+  const int64_t H = c.NH * c.dh;
+  const auto dt = x.scalar_type();
+  if (!c.plan || dt != c.step_dtype || !x.is_cuda() || x.device() != c.device || !x.is_contiguous() || x.dim() != 3 || x.size(1) != 1 ||
+      x.size(0) != c.step_B || x.size(2) != 4 * H)
+    throw NotCovered{};
+  const int64_t B = c.step_B;
+  if (state.scalar_type() != at::kFloat || !state.is_contiguous() || state.device() != c.device || state.dim() != 3 || state.size(0) != 4 ||
+      state.size(1) != B || state.size(2) != H)
+    throw NotCovered{};
+  const at::Tensor &r = c.parameter(g_names.r), &b = c.parameter(g_names.b);
+  if (r.data_ptr() != c.r_ptr || b.data_ptr() != c.b_ptr || version_of(r) != c.r_version || version_of(b) != c.b_version || c.records(x, &state, r, b))
+    throw NotCovered{};
+  StepResult out;
+  if (h_out) {
+    if (h_out->scalar_type() != dt || h_out->numel() != B * H || !h_out->is_contiguous() || h_out->device() != c.device) throw NotCovered{};
+    out.h = *h_out;
+  } else if (h_shape) {
+    out.h = at::empty_strided(at::IntArrayRef(h_shape->size.data(), h_shape->n), at::IntArrayRef(h_shape->stride.data(), h_shape->n), x.options());
+  } else {
+    out.h = at::empty({1, B, H}, x.options());
+  }
+  out.state = state_out ? *state_out : at::empty({4, B, H}, state.options());
+  xs_slstm_args &a = *c.step_args;
+  a.h_prev = nullptr;
+  if (dt == at::kBFloat16) {
+    if (h_prev) {
+      if (h_prev->scalar_type() != dt || h_prev->numel() != B * H || h_prev->device() != c.device) throw NotCovered{};
+      a.h_prev = h_prev->data_ptr();
+    } else if (c.last_state.defined() && c.last_state.is_same(state) && versioned(state) && version_of(state) == c.last_state_version &&
+               version_of(c.last_h) == c.last_h_version && c.last_h.data_ptr() != out.h.data_ptr()) {
+      // The state this cell handed out last time comes back untouched: the h it returned with it is that state's y
+      // plane in bfloat16, the operand the step kernel wants (half the bytes, and the pipelined kernel).
+      a.h_prev = c.last_h.data_ptr();
+    }
+  }
+  a.wx = x.data_ptr();
+  a.s0 = (const float *)state.data_ptr();
+  a.s_out = (float *)out.state.data_ptr();
+  a.h_out = out.h.data_ptr();
+  a.stream = stream_of(c.device);
+  launched(g_engine.step(&a));
+  if (keep_state && versioned(out.state) && versioned(out.h)) {
+    c.last_state = out.state; c.last_state_version = version_of(out.state);
+    c.last_h = out.h; c.last_h_version = version_of(out.h);
+  } else {
+    c.last_state.reset(); c.last_h.reset();
+  }
+  return out;
+}
+
+inline const at::Tensor *optional_tensor(PyObject *o) { return absent(o) ? nullptr : &tensor_of(o); }
+
+// step(input, state, reset_mask, state_out, h_out, h_prev, config, keep_state_fp32) -> (output, state) or None
+PyObject *cell_step_(CellPath &c, PyObject *const *args) {
+  if (!absent(args[2]) || absent(args[1]) || at::autocast::is_autocast_enabled(at::kCUDA)) throw NotCovered{};
+  const at::Tensor &x = tensor_of(args[0]), &state = tensor_of(args[1]);
+  if (!c.plan || !input_is_bsgnh(args[6])) throw NotCovered{};
+  const OutShape shape = out_shape(args[6]);
+  const bool keep = args[7] == Py_True;
+  c10::OptionalDeviceGuard guard(c.device);
+  const Shape4 s4 = shape_of(shape, 1, c.step_B, c.NH, c.dh);
+  const at::Tensor *h_out = optional_tensor(args[4]);
+  StepResult r = run_step(c, x, state, optional_tensor(args[3]), h_out, optional_tensor(args[5]), &s4, keep);
+  at::Tensor h = h_out ? r.h.as_strided(at::IntArrayRef(s4.size.data(), s4.n), at::IntArrayRef(s4.stride.data(), s4.n)) : r.h;
+  PyRef ph(THPVariable_Wrap(h)), ps(THPVariable_Wrap(keep || x.scalar_type() == at::kFloat ? r.state : r.state.to(x.scalar_type())));
+  if (!ph.o || !ps.o) throw PythonError{};
+  return PyTuple_Pack(2, ph.o, ps.o);
+}
+
+// ---- a sequence through the cell (no autograd), as sLSTMCell_hip._run and functional.slstm_forward do it
+struct Sequence { at::Tensor h, state; };  // h: [S,B,H] memory (with the strides of `shape` where given), state: float32
+at::Tensor mask_bytes(const at::Tensor &m, int64_t B, int64_t T) {
+  if (!m.is_cuda() || m.dim() != 2 || m.size(0) != B || m.size(1) != T) throw NotCovered{};
+  at::Tensor r = m;
+  if (r.scalar_type() == at::kBool) r = r.is_contiguous() ? r.view(at::kByte) : r.to(at::kByte);
+  else if (r.scalar_type() != at::kByte) r = r.ne(0).to(at::kByte);
+  return r.stride(1) != 1 ? r.contiguous() : r;
+}
+
+Sequence run_sequence(CellPath &c, at::Tensor x, const at::Tensor *state, const at::Tensor *mask, OutShape shape) {
+  const int64_t H = c.NH * c.dh, B = x.size(0), T = x.size(1);
+  const auto dt = x.scalar_type();
+  if ((dt != at::kFloat && dt != at::kBFloat16) || !x.is_cuda() || T < 2 || B < 1 || x.size(2) != 4 * H) throw NotCovered{};
+  at::Tensor r = c.parameter(g_names.r), b = c.parameter(g_names.b);
+  if (c.records(x, state, r, b) || r.device() != x.device() || b.device() != x.device() || !r.is_contiguous() || !b.is_contiguous()) throw NotCovered{};
+  if ((r.scalar_type() != at::kFloat && r.scalar_type() != at::kBFloat16) || r.numel() != c.NH * 4 * c.dh * c.dh || b.numel() != 4 * H) throw NotCovered{};
+  const size_t esz = x.element_size();
+  if (x.stride(2) != 1 || !aligned(x.data_ptr(), 16) || (x.stride(0) * esz) % 16 || (x.stride(1) * esz) % 16 || x.stride(1) < 4 * H ||
+      (B > 1 && x.stride(0) < 4 * H))
+    x = x.contiguous();
+  if (dt == at::kFloat && r.scalar_type() != at::kFloat) r = r.to(at::kFloat);
+  if (b.scalar_type() != at::kFloat) {
+    if (!c.bias32.defined() || c.bias32_of != b.data_ptr() || c.bias32_version != version_of(b) || !versioned(b) || c.bias32.device() != b.device()) {
+      c.bias32 = b.to(at::kFloat); c.bias32_of = b.data_ptr(); c.bias32_version = version_of(b);
+    }
+    b = c.bias32;
+  }
+  at::Tensor s0, m;
+  if (state) {
+    if (!state->is_cuda() || state->dim() != 3 || state->size(0) != 4 || state->size(1) != B || state->size(2) != H) throw NotCovered{};
+    s0 = state->to(at::kFloat).contiguous();
+  }
+  if (mask) m = mask_bytes(*mask, B, T);
+  const bool capturing = [&] {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing((hipStream_t)stream_of(x.device()), &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+  }();
+  if (!capturing) c.raise_if_aborted();
+  const Shape4 s4 = shape_of(shape, T, B, c.NH, c.dh);
+  Sequence out;
+  out.h = at::empty_strided(at::IntArrayRef(s4.size.data(), s4.n), at::IntArrayRef(s4.stride.data(), s4.n), x.options());
+  out.state = at::empty({4, B, H}, x.options().dtype(at::kFloat));
+  at::Tensor &ws = c.workspace(B, x.device());
+  if (!c.abort_word) c.abort_word = g_words.take();
+  if (!c.abort_word) throw NotCovered{};
+  xs_slstm_args a{};
+  a.B = (int32_t)B; a.T = (int32_t)T; a.NH = (int32_t)c.NH; a.dh = (int32_t)c.dh;
+  a.wx_dtype = dtype_code(dt); a.r_dtype = dtype_code(r.scalar_type());
+  a.wx = x.data_ptr(); a.wx_stride_b = x.stride(0); a.wx_stride_t = x.stride(1);
+  a.r = r.data_ptr(); a.bias = (const float *)b.data_ptr();
+  a.s0 = state ? (const float *)s0.data_ptr() : nullptr;
+  a.reset = mask ? (const uint8_t *)m.data_ptr() : nullptr; a.reset_stride_b = mask ? m.stride(0) : 0;
+  a.h_out = out.h.data_ptr(); a.s_out = (float *)out.state.data_ptr();
+  a.workspace = ws.data_ptr(); a.workspace_bytes = (size_t)ws.numel();
+  a.stream = stream_of(x.device());
+  launched(g_engine.forward(&a, capturing ? nullptr : c.abort_word));
+  c.last_workspace = ws;
+  if (x.device().index() < 64) c.devices_used |= 1ull << x.device().index();
+  return out;
+}
+
+// forward(input, state, reset_mask, config, keep_state_fp32) -> (output, state) or None
+PyObject *cell_forward_(CellPath &c, PyObject *const *args) {
+  if (at::autocast::is_autocast_enabled(at::kCUDA)) throw NotCovered{};
+  const at::Tensor &x = tensor_of(args[0]);
+  if (x.dim() != 3 || !x.is_cuda()) throw NotCovered{};
+  const at::Tensor *state = optional_tensor(args[1]), *mask = optional_tensor(args[2]);
+  const OutShape shape = out_shape(args[3]);
+  c10::OptionalDeviceGuard guard(x.device());
+  Sequence s = run_sequence(c, input_is_bsgnh(args[3]) ? x : x.permute({1, 0, 2}), state, mask, shape);
+  PyRef ph(THPVariable_Wrap(s.h)), ps(THPVariable_Wrap(args[4] == Py_True || x.scalar_type() == at::kFloat ? s.state : s.state.to(x.scalar_type())));
+  if (!ph.o || !ps.o) throw PythonError{};
+  return PyTuple_Pack(2, ph.o, ps.o);
+}
+
+template <PyObject *(*F)(CellPath &, PyObject *const *), int N>
+PyObject *cell_call(PyObject *self, PyObject *const *args, Py_ssize_t n) {
+  if (n != N) { PyErr_Format(PyExc_TypeError, "%d arguments expected, got %zd", N, n); return nullptr; }
+  try {
+    return F(*((CellPathObject *)self)->c, args);
+  } catch (const NotCovered &) {
+    Py_RETURN_NONE;
+  } catch (const PythonError &) {
+    return nullptr;
+  } catch (const std::exception &e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+}
+
+// set_plan(plan, address of its argument block, B, r, b): the next steps of that batch size and of these parameters
+PyObject *cell_set_plan_(CellPath &c, PyObject *const *args) {
+  const at::Tensor &r = tensor_of(args[3]), &b = tensor_of(args[4]);
+  Py_INCREF(args[0]);
+  Py_XDECREF(c.plan);
+  c.plan = args[0];
+  c.step_args = (xs_slstm_args *)PyLong_AsVoidPtr(args[1]);
+  c.step_B = PyLong_AsLongLong(args[2]);
+  c.step_dtype = c.step_args->wx_dtype == XS_BF16 ? at::kBFloat16 : at::kFloat;
+  c.device = r.device();
+  c.r_ptr = r.data_ptr(); c.b_ptr = b.data_ptr();
+  c.r_version = version_of(r); c.b_version = version_of(b);
+  Py_RETURN_NONE;
+}
+// workspace(B, a tensor on the device) -> the workspace of calls on that device's current stream
+PyObject *cell_workspace_(CellPath &c, PyObject *const *args) {
+  const at::Tensor &like = tensor_of(args[1]);
+  return THPVariable_Wrap(c.workspace(PyLong_AsLongLong(args[0]), like.device()));
+}
+// last_workspace() -> the workspace of the latest sequence call
+PyObject *cell_last_workspace_(CellPath &c, PyObject *const *) {
+  if (!c.last_workspace.defined()) Py_RETURN_NONE;
+  return THPVariable_Wrap(c.last_workspace);
+}
+// poll(block) -> whether a sequence call gave up since the last poll; block: waits for the calls in flight first
+PyObject *cell_poll_(CellPath &c, PyObject *const *args) {
+  if (args[0] == Py_True) {
+    for (int d = 0; d < 64; ++d)
+      if ((c.devices_used >> d) & 1) {
+        c10::OptionalDeviceGuard guard(at::Device(at::kCUDA, (c10::DeviceIndex)d));
+        Py_BEGIN_ALLOW_THREADS
+        (void)hipDeviceSynchronize();
+        Py_END_ALLOW_THREADS
+      }
+  }
+  if (c.abort_word && __atomic_exchange_n(c.abort_word, 0u, __ATOMIC_ACQ_REL)) Py_RETURN_TRUE;
+  Py_RETURN_FALSE;
+}
+
+PyObject *cell_new(PyTypeObject *type, PyObject *args, PyObject *) {
+  PyObject *parameters;
+  long long NH, dh;
+  if (!PyArg_ParseTuple(args, "O!LL", &PyDict_Type, &parameters, &NH, &dh)) return nullptr;
+  CellPathObject *self = (CellPathObject *)type->tp_alloc(type, 0);
+  if (!self) return nullptr;
+  self->c = new CellPath;
+  Py_INCREF(parameters);
+  self->c->parameters = parameters;
+  self->c->NH = NH; self->c->dh = dh;
+  return (PyObject *)self;
+}
+void cell_dealloc(PyObject *self) {
+  PyTypeObject *type = Py_TYPE(self);
+  delete ((CellPathObject *)self)->c;
+  type->tp_free(self);
+  Py_DECREF(type);
+}
+
+PyMethodDef cell_methods[] = {
+    {"step", (PyCFunction)(void *)cell_call<cell_step_, 8>, METH_FASTCALL, nullptr},
+    {"forward", (PyCFunction)(void *)cell_call<cell_forward_, 5>, METH_FASTCALL, nullptr},
+    {"set_plan", (PyCFunction)(void *)cell_call<cell_set_plan_, 5>, METH_FASTCALL, nullptr},
+    {"workspace", (PyCFunction)(void *)cell_call<cell_workspace_, 2>, METH_FASTCALL, nullptr},
+    {"last_workspace", (PyCFunction)(void *)cell_call<cell_last_workspace_, 0>, METH_FASTCALL, nullptr},
+    {"poll", (PyCFunction)(void *)cell_call<cell_poll_, 1>, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyType_Slot cell_slots[] = {{Py_tp_new, (void *)cell_new}, {Py_tp_dealloc, (void *)cell_dealloc}, {Py_tp_methods, cell_methods}, {0, nullptr}};
+PyType_Spec cell_spec = {"_xlstm_host.CellPath", sizeof(CellPathObject), 0, Py_TPFLAGS_DEFAULT, cell_slots};
+PyTypeObject *g_cell_type = nullptr;
+
+// ---- one layer: its submodules are looked up by name in the module dictionaries on every call (they may be replaced)
+PyObject *attribute(PyObject *o, PyObject *name) {  // new reference; nn.Module keeps these in its __dict__
+  PyObject *v = PyObject_GetAttr(o, name);
+  if (!v) throw PythonError{};
+  return v;
+}
+PyObject *submodule(PyObject *modules, PyObject *name) {  // borrowed
+  PyObject *m = PyDict_GetItem(modules, name);
+  if (!m) throw NotCovered{};
+  return m;
+}
+PyObject *module_dict(PyObject *module, PyObject *which) {  // borrowed from the module
+  PyRef d(attribute(module, which));
+  if (!PyDict_Check(d.o)) throw NotCovered{};
+  return d.o;  // (the module holds it)
+}
+at::Tensor parameter(PyObject *module, PyObject *name, bool optional = false) {
+  PyObject *o = PyDict_GetItem(module_dict(module, g_names.parameters), name);
+  if (absent(o)) {
+    if (optional) return at::Tensor();
+    throw NotCovered{};
+  }
+  return tensor_of(o);
+}
+bool has_hooks(PyObject *module) {
+  return PyDict_Size(module_dict(module, g_names.forward_hooks)) || PyDict_Size(module_dict(module, g_names.forward_pre_hooks));
+}
+
+struct LayerParts {
+  PyRef cell_config{nullptr};
+  CellPath *cell = nullptr;
+  bool keep_state = false;
+  at::Tensor conv_w, conv_b, gate[4], norm_w;
+  double eps = 1e-5;
+  int64_t K = 0, NH = 0, dh = 0, D = 0;
+};
+
+// what a layer call needs of its modules; NotCovered unless the engine's kernels apply (sLSTMLayer._fused) and no
+// gradient is recorded
+void collect(PyObject *layer, PyObject *cell_path, const at::Tensor &x, LayerParts &p) {
+  p.cell = ((CellPathObject *)cell_path)->c;
+  p.NH = p.cell->NH; p.dh = p.cell->dh; p.D = p.NH * p.dh;
+  if (x.dim() != 3 || x.scalar_type() != at::kBFloat16 || !x.is_cuda() || x.size(2) != p.D || p.dh % 64 || p.dh > 1024 ||
+      at::autocast::is_autocast_enabled(at::kCUDA))
+    throw NotCovered{};
+  for (PyObject *h : g_engine.global_hooks)
+    if (h && PyDict_Size(h)) throw NotCovered{};
+  PyObject *modules = module_dict(layer, g_names.modules);
+  PyObject *cell = submodule(modules, g_names.slstm_cell);
+  PyObject *conv1d = submodule(modules, g_names.conv1d);
+  PyObject *conv = submodule(module_dict(conv1d, g_names.modules), g_names.conv);
+  PyObject *norm = submodule(modules, g_names.group_norm), *dropout = submodule(modules, g_names.dropout);
+  if (has_hooks(cell) || has_hooks(dropout)) throw NotCovered{};
+  {
+    PyRef fused(attribute(layer, g_names.fused_pre_ops));
+    if (fused.o != Py_True) throw NotCovered{};
+    PyRef training(attribute(dropout, g_names.training)), rate(attribute(dropout, g_names.p));
+    const double dp = PyFloat_AsDouble(rate.o);
+    if (PyErr_Occurred()) { PyErr_Clear(); throw NotCovered{}; }
+    if (training.o == Py_True && dp != 0.0) throw NotCovered{};
+    PyRef keep(attribute(cell, g_names.keep_state_fp32)), eps(attribute(norm, g_names.eps));
+    p.keep_state = keep.o == Py_True;
+    p.eps = PyFloat_AsDouble(eps.o);
+    p.cell_config.o = attribute(cell, g_names.config);
+  }
+  if (!input_is_bsgnh(p.cell_config.o) || out_shape(p.cell_config.o) != OutShape::BNSH) throw NotCovered{};
+  p.conv_w = parameter(conv, g_names.weight);
+  p.conv_b = parameter(conv, g_names.bias, true);
+  // (the module called fgate feeds the i slot, igate the f slot)
+  PyObject *gates[4] = {g_names.fgate, g_names.igate, g_names.zgate, g_names.ogate};
+  bool needs_grad = x.requires_grad();
+  for (int g = 0; g < 4; ++g) {
+    p.gate[g] = parameter(submodule(modules, gates[g]), g_names.weight);
+    const at::Tensor &w = p.gate[g];
+    if (w.scalar_type() != at::kBFloat16 || !w.is_contiguous() || w.numel() != p.NH * p.dh * p.dh || w.device() != x.device() || !aligned(w.data_ptr(), 16)) throw NotCovered{};
+    needs_grad |= w.requires_grad();
+  }
+  p.norm_w = parameter(norm, g_names.weight, true);
+  for (const at::Tensor *t : {&p.conv_w, &p.conv_b, &p.norm_w}) {
+    if (!t->defined()) continue;
+    if (t->scalar_type() != at::kBFloat16 || !t->is_contiguous() || t->device() != x.device() || !aligned(t->data_ptr(), 16)) throw NotCovered{};
+    needs_grad |= t->requires_grad();
+  }
+  p.K = p.conv_w.numel() / p.D;
+  if (p.K < 2 || p.K > 4) throw NotCovered{};
+  if (at::GradMode::is_enabled() && needs_grad) throw NotCovered{};  // (the cell's own parameters: looked at where it runs)
+}
+
+void run_conv(const LayerParts &p, const at::Tensor &x, const void *taps, int64_t taps_stride, const at::Tensor *mask, void *out, void *ring, void *stream) {
+  xs_conv_args a{};
+  a.B = (int32_t)x.size(0); a.T = (int32_t)x.size(1); a.D = (int32_t)p.D; a.K = (int32_t)p.K;
+  a.dtype = XS_BF16;
+  a.x = x.data_ptr(); a.x_stride_b = x.stride(0); a.x_stride_t = x.stride(1);
+  a.conv_state = taps; a.conv_state_stride_b = taps && x.size(0) > 1 ? taps_stride : 0;
+  a.weight = p.conv_w.data_ptr(); a.bias = p.conv_b.defined() ? p.conv_b.data_ptr() : nullptr;
+  a.reset = mask ? (const uint8_t *)mask->data_ptr() : nullptr; a.reset_stride_b = mask ? mask->stride(0) : 0;
+  a.out = out; a.ring_out = ring; a.stream = stream;
+  launched(g_engine.conv(&a));
+}
+void run_gates(const LayerParts &p, const at::Tensor &x, const void *x_conv, void *out, void *stream) {
+  xs_gates_args a{};
+  a.M = (int32_t)(x.size(0) * x.size(1)); a.NH = (int32_t)p.NH; a.dh = (int32_t)p.dh;
+  a.dtype = XS_BF16;
+  a.x = x.data_ptr(); a.x_stride_row = p.D; a.x_conv = x_conv; a.x_conv_stride_row = p.D;
+  for (int g = 0; g < 4; ++g) a.w[g] = p.gate[g].data_ptr();
+  a.out = out; a.out_stride_row = 4 * p.D; a.stream = stream;
+  launched(g_engine.gates(&a));
+}
+void run_norm(const LayerParts &p, const at::Tensor &h, int64_t B, int64_t T, void *out, void *stream) {
+  xs_norm_args a{};
+  a.B = (int32_t)B; a.T = (int32_t)T; a.NH = (int32_t)p.NH; a.dh = (int32_t)p.dh;
+  a.dtype = XS_BF16; a.eps = (float)p.eps;
+  a.x = h.data_ptr(); a.x_stride_b = p.D; a.x_stride_h = p.dh; a.x_stride_t = B * p.D;  // [T,B,H] memory
+  a.weight = p.norm_w.defined() ? p.norm_w.data_ptr() : nullptr;
+  a.out = out; a.stream = stream;
+  launched(g_engine.norm(&a));
+}
+
+// the taps in front of the first token: a [B,n,D] tensor of which the last K-1 inputs count
+const void *taps_of(const LayerParts &p, const at::Tensor &t, int64_t B, int64_t *stride) {
+  const int64_t n = t.dim() == 3 ? t.size(1) : 0;
+  if (t.scalar_type() != at::kBFloat16 || n < p.K - 1 || t.size(0) != B || t.size(2) != p.D || t.stride(2) != 1 || t.stride(1) != p.D || t.stride(0) % 8 ||
+      !t.is_cuda() || !aligned(t.data_ptr(), 16))
+    throw NotCovered{};
+  *stride = t.stride(0);
+  return (const char *)t.data_ptr() + (n - (p.K - 1)) * p.D * 2;
+}
+
+PyObject *states_dict(PyObject *conv_state, const at::Tensor &state) {
+  PyRef s(THPVariable_Wrap(state)), d(PyDict_New());
+  if (!s.o || !d.o || !conv_state || PyDict_SetItem(d.o, g_names.conv_state, conv_state) || PyDict_SetItem(d.o, g_names.slstm_state, s.o)) throw PythonError{};
+  return d.release();
+}
+PyObject *first_of(PyObject *o) {  // a state that may come in a tuple or list of one
+  if (PyTuple_Check(o)) return PyTuple_GET_SIZE(o) ? PyTuple_GET_ITEM(o, 0) : Py_None;
+  if (PyList_Check(o)) return PyList_GET_SIZE(o) ? PyList_GET_ITEM(o, 0) : Py_None;
+  return o;
+}
+
+// layer_step(layer, cell path, x, conv_state, slstm_state, slstm_state_out, conv_state_out, h_out, h_prev, out)
+//   -> (out, {"conv_state": (ring,), "slstm_state": state}) or None
+PyObject *layer_step_(PyObject *const *args) {
+  const at::Tensor &x = tensor_of(args[2]);
+  if (absent(args[4])) throw NotCovered{};
+  LayerParts p;
+  collect(args[0], args[1], x, p);
+  const at::Tensor &state = tensor_of(args[4]);
+  const int64_t B = x.size(0);
+  if (x.size(1) != 1 || !x.is_contiguous() || !aligned(x.data_ptr(), 16) || B < 1) throw NotCovered{};
+  c10::OptionalDeviceGuard guard(x.device());
+  const void *taps = nullptr;
+  int64_t taps_stride = 0;
+  PyObject *prev = absent(args[3]) ? nullptr : first_of(args[3]);
+  if (!absent(prev)) {
+    const at::Tensor &t = tensor_of(prev);
+    if (t.dim() != 3 || (t.size(1) != p.K && t.size(1) != p.K - 1)) throw NotCovered{};  // (the general path asserts)
+    taps = taps_of(p, t, B, &taps_stride);
+  }
+  const at::Tensor *ring_out = optional_tensor(args[6]), *out_given = optional_tensor(args[9]);
+  const auto opts = x.options();
+  if (ring_out && (ring_out->scalar_type() != at::kBFloat16 || ring_out->dim() != 3 || ring_out->size(0) != B || ring_out->size(1) != p.K ||
+                   ring_out->size(2) != p.D || !ring_out->is_contiguous()))
+    throw NotCovered{};
+  if (out_given && (out_given->scalar_type() != at::kBFloat16 || out_given->numel() != B * p.D || !out_given->is_contiguous())) throw NotCovered{};
+  // the step's own conditions, before anything is launched
+  {
+    const at::Tensor *so = optional_tensor(args[5]), *ho = optional_tensor(args[7]), *hp = optional_tensor(args[8]);
+    if (so && (so->scalar_type() != at::kFloat || !so->is_contiguous() || so->dim() != 3 || so->size(0) != 4 || so->size(1) != B || so->size(2) != p.D)) throw NotCovered{};
+    if (ho && (ho->scalar_type() != at::kBFloat16 || ho->numel() != B * p.D || !ho->is_contiguous())) throw NotCovered{};
+    if (hp && (hp->scalar_type() != at::kBFloat16 || hp->numel() != B * p.D)) throw NotCovered{};
+    const at::Tensor &r = p.cell->parameter(g_names.r), &b = p.cell->parameter(g_names.b);
+    if (!p.cell->plan || p.cell->step_B != B || p.cell->step_dtype != at::kBFloat16 || p.cell->device != x.device() || r.data_ptr() != p.cell->r_ptr ||
+        b.data_ptr() != p.cell->b_ptr || version_of(r) != p.cell->r_version || version_of(b) != p.cell->b_version || p.cell->records(x, &state, r, b) ||
+        state.scalar_type() != at::kFloat || !state.is_contiguous() || state.device() != x.device() || state.dim() != 3 || state.size(0) != 4 ||
+        state.size(1) != B || state.size(2) != p.D)
+      throw NotCovered{};
+  }
+  void *stream = stream_of(x.device());
+  at::Tensor ring = ring_out ? *ring_out : at::empty({B, p.K, p.D}, opts);
+  at::Tensor wx = at::empty({B, 1, 4 * p.D}, opts), x_conv = at::empty({B, 1, p.D}, opts);
+  run_conv(p, x, taps, taps_stride, nullptr, x_conv.data_ptr(), ring.data_ptr(), stream);
+  run_gates(p, x, x_conv.data_ptr(), wx.data_ptr(), stream);
+  StepResult s = run_step(*p.cell, wx, state, optional_tensor(args[5]), optional_tensor(args[7]), optional_tensor(args[8]), nullptr, p.keep_state);
+  at::Tensor out = out_given ? *out_given : at::empty({B, 1, p.D}, opts);
+  run_norm(p, s.h, B, 1, out.data_ptr(), stream);
+  PyRef po(THPVariable_Wrap(out)), pr(THPVariable_Wrap(ring)), tuple(nullptr);
+  if (!po.o || !pr.o) throw PythonError{};
+  tuple.o = PyTuple_Pack(1, pr.o);
+  PyRef states(states_dict(tuple.o, p.keep_state ? s.state : s.state.to(at::kBFloat16)));
+  return PyTuple_Pack(2, po.o, states.o);
+}
+
+// layer_forward(layer, cell path, x, conv_state, slstm_state, return_last_state, reset_mask) -> the layer's result or None
+PyObject *layer_forward_(PyObject *const *args) {
+  const at::Tensor &x_in = tensor_of(args[2]);
+  LayerParts p;
+  collect(args[0], args[1], x_in, p);
+  const int64_t B = x_in.size(0), T = x_in.size(1);
+  if (T < 2 || B < 1) throw NotCovered{};
+  c10::OptionalDeviceGuard guard(x_in.device());
+  const void *taps = nullptr;
+  int64_t taps_stride = 0;
+  PyObject *prev = absent(args[3]) ? nullptr : first_of(args[3]);
+  if (!absent(prev)) taps = taps_of(p, tensor_of(prev), B, &taps_stride);
+  const bool last = args[5] == Py_True;
+  if (last && T < p.K - 1) throw NotCovered{};
+  const at::Tensor *state = optional_tensor(args[4]);
+  at::Tensor mask;
+  if (!absent(args[6])) mask = mask_bytes(tensor_of(args[6]), B, T);
+  const at::Tensor *maskp = mask.defined() ? &mask : nullptr;
+  {
+    const at::Tensor &r = p.cell->parameter(g_names.r), &b = p.cell->parameter(g_names.b);
+    if (p.cell->records(x_in, state, r, b)) throw NotCovered{};
+    if (state && (!state->is_cuda() || state->dim() != 3 || state->size(0) != 4 || state->size(1) != B || state->size(2) != p.D)) throw NotCovered{};
+  }
+  at::Tensor x = x_in.is_contiguous() && aligned(x_in.data_ptr(), 16) ? x_in : x_in.contiguous();
+  void *stream = stream_of(x.device());
+  at::Tensor wx = at::empty({B, T, 4 * p.D}, x.options()), x_conv = at::empty({B, T, p.D}, x.options());
+  run_conv(p, x, taps, taps_stride, maskp, x_conv.data_ptr(), nullptr, stream);
+  run_gates(p, x, x_conv.data_ptr(), wx.data_ptr(), stream);
+  Sequence s = run_sequence(*p.cell, wx, state, maskp, OutShape::SBH);
+  at::Tensor out = x_conv;  // (its last reader has been launched in front of the norm)
+  run_norm(p, s.h, B, T, out.data_ptr(), stream);
+  PyRef po(THPVariable_Wrap(out));
+  if (!po.o) throw PythonError{};
+  if (!last) return po.release();
+  // the last K-1 inputs: a tensor of their own where the call continued a state (x may be reused for the next chunk)
+  at::Tensor tail = x_in.narrow(1, T - (p.K - 1), p.K - 1);
+  PyRef pt(THPVariable_Wrap(taps ? tail.clone() : tail));
+  PyRef states(states_dict(pt.o, p.keep_state ? s.state : s.state.to(at::kBFloat16)));
+  return PyTuple_Pack(2, po.o, states.o);
+}
+
+template <PyObject *(*F)(PyObject *const *), int N>
+PyObject *layer_call(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  if (n != N) { PyErr_Format(PyExc_TypeError, "%d arguments expected, got %zd", N, n); return nullptr; }
+  if (!PyObject_TypeCheck(args[1], g_cell_type)) Py_RETURN_NONE;
+  try {
+    return F(args);
+  } catch (const NotCovered &) {
+    Py_RETURN_NONE;
+  } catch (const PythonError &) {
+    return nullptr;
+  } catch (const std::exception &e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+}
+
+// bind(addresses: dict name -> int, EngineError, the two dicts of global module hooks)
+PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  if (n != 4 || !PyDict_Check(args[0])) { PyErr_SetString(PyExc_TypeError, "bind(addresses, error, hooks, pre_hooks)"); return nullptr; }
+  auto get = [&](const char *name, auto &fn) {
+    PyObject *v = PyDict_GetItemString(args[0], name);
+    fn = v ? (std::decay_t<decltype(fn)>)PyLong_AsVoidPtr(v) : nullptr;
+    return fn != nullptr;
+  };
+  if (!get("xs_slstm_step", g_engine.step) || !get("xs_slstm_forward_watched", g_engine.forward) ||
+      !get("xs_slstm_workspace_bytes", g_engine.workspace_bytes) || !get("xs_last_error", g_engine.last_error) ||
+      !get("xs_causal_conv_silu", g_engine.conv) || !get("xs_headwise_gates", g_engine.gates) || !get("xs_headwise_group_norm", g_engine.norm)) {
+    PyErr_SetString(PyExc_KeyError, "an entry point of the engine is missing");
+    return nullptr;
+  }
+  for (int i = 1; i < 4; ++i) Py_INCREF(args[i]);
+  g_engine.error = args[1];
+  for (int i = 0; i < 2; ++i) g_engine.global_hooks[i] = PyDict_Check(args[2 + i]) ? args[2 + i] : nullptr;
+  Py_RETURN_NONE;
+}
+
+PyMethodDef module_methods[] = {
+    {"bind", (PyCFunction)(void *)bind, METH_FASTCALL, nullptr},
+    {"layer_step", (PyCFunction)(void *)layer_call<layer_step_, 10>, METH_FASTCALL, nullptr},
+    {"layer_forward", (PyCFunction)(void *)layer_call<layer_forward_, 7>, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_xlstm_host", "native host path of the cell's and the layer's frequent calls", -1, module_methods,
+                          nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__xlstm_host(void) {
+  auto s = [](const char *v) { return PyUnicode_InternFromString(v); };
+  g_names = Names{s("_recurrent_kernel_"), s("_bias_"), s("weight"), s("bias"), s("conv_state"), s("slstm_state"), s("input_shape"), s("output_shape"),
+                  s("keep_state_fp32"), s("config"), s("_modules"), s("_parameters"), s("_forward_hooks"), s("_forward_pre_hooks"), s("training"), s("p"),
+                  s("eps"), s("conv1d"), s("conv"), s("fgate"), s("igate"), s("zgate"), s("ogate"), s("group_norm"), s("slstm_cell"), s("dropout"),
+                  s("fused_pre_ops"), s("_rt"), s("BSGNH")};
+  PyObject *m = PyModule_Create(&module_def);
+  if (!m) return nullptr;
+  g_cell_type = (PyTypeObject *)PyType_FromSpec(&cell_spec);
+  if (!g_cell_type || PyModule_AddObject(m, "CellPath", (PyObject *)g_cell_type)) return nullptr;
+  Py_INCREF(g_cell_type);
+  return m;
+}

@@ -59,6 +59,12 @@ __device__ __forceinline__ bool mark_has_sentinel(uint32_t m) {
 __device__ __forceinline__ bool chunk_has_sentinel_bf16(const uint4 &v) { return mark_has_sentinel<true>(chunk_mark<true>(v)); }
 __device__ __forceinline__ bool chunk_has_sentinel_f32(const uint4 &v) { return mark_has_sentinel<false>(chunk_mark<false>(v)); }
 
+// Tells the host that a bounded wait ran out (a word in pinned memory that the caller reads when it likes: no copy and no
+// event behind every call).
+__device__ __forceinline__ void report_abort(unsigned int *host_word) {
+  if (host_word) __hip_atomic_store(host_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 struct CellState { float y, c, n, m; };
 
 // One exponential-gating update (vanilla/slstm.py:19-37; per-element n == 0 rule), the same code in
@@ -106,6 +112,15 @@ __global__ void fill_u32_kernel(uint32_t *p, size_t n, uint32_t v) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   for (; i < n; i += stride) p[i] = v;
+}
+
+// the two fills in front of a sequence launch as one kernel: the header (status block, placement words) zero, the
+// exchange ring "not written yet"
+__global__ void clear_workspace_kernel(uint32_t *header, size_t nh, uint32_t *ring, size_t nr) {
+  const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = i0; i < nh; i += stride) header[i] = 0u;
+  uint4 *const r4 = reinterpret_cast<uint4 *>(ring);  // (a ring is a multiple of 256 bytes)
+  for (size_t i = i0; i < nr / 4; i += stride) r4[i] = make_uint4(kSentinel32, kSentinel32, kSentinel32, kSentinel32);
 }
 
 __global__ void copy_state_kernel(const float *s0, float *s_out, size_t n) {

@@ -259,7 +259,7 @@ int run_step(const xs_slstm_args *a) {
 }
 
 // need != nullptr: launch nothing, only report the bytes of workspace the launches of this call touch
-int run_forward(const xs_slstm_args *a, size_t *need = nullptr) {
+int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_host = nullptr) {
   hipStream_t stream = (hipStream_t)a->stream;
   const int B = a->B, T = a->T, NH = a->NH, dh = a->dh;
   const long long H = (long long)NH * dh;
@@ -267,10 +267,10 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr) {
   const bool dry = need != nullptr;
   if (dry) *need = kHeaderBytes;
 
-  // status block + per-workgroup placement words start clean
-  if (!dry)
-    hipLaunchKernelGGL(fill_u32_kernel, dim3(4), dim3(256), 0, stream, (uint32_t *)a->workspace,
-                       (kStatusBytes + (size_t)kMaxWg * 4) / 4, 0u);
+  // status block + per-workgroup placement words start clean: with the exchange ring in front of the first launch, here
+  // where there is none
+  if (!dry && (B == 0 || T == 0))
+    hipLaunchKernelGGL(fill_u32_kernel, dim3(4), dim3(256), 0, stream, (uint32_t *)a->workspace, kHeaderBytes / 4, 0u);
   if (B == 0) return XS_OK;
   if (T == 0) {
     if (dry) return XS_OK;
@@ -372,18 +372,18 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr) {
       if (kHeaderBytes + ring > *need) *need = kHeaderBytes + ring;
       continue;
     }
-    if (launch_no++ > 0)  // the placement words of the previous launch must not pass for this one's
-      hipLaunchKernelGGL(fill_u32_kernel, dim3(4), dim3(256), 0, stream,
-                         (uint32_t *)((char *)a->workspace + kStatusBytes), (size_t)kMaxWg, 0u);
     // grid shapes of the three placements the kernel knows: one XCD per group, two XCDs per group, spread
     const int grid = G <= 32 ? 8 * G * ((ngroups + 7) / 8)
                              : ((G <= 64 && G % 2 == 0) ? 8 * (G / 2) * ((ngroups + 3) / 4) : ngroups * G);
     if (grid > kMaxWg) return fail(XS_ERR_UNSUPPORTED, "grid %d too large", grid);
-    {  // every word of the exchange ring starts as "not written yet"
-      const size_t words = ((size_t)kRing * ngroups * G * 16 * MT * 16 * (bf16 ? 2 : 4) + 3) / 4;
-      const int blocks = (int)((words + 256 * 4 - 1) / (256 * 4));
-      hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks < 1 ? 1 : (blocks > 1024 ? 1024 : blocks)), dim3(256), 0, stream,
-                         (uint32_t *)((char *)a->workspace + kHeaderBytes), words, kSentinel32);
+    {  // every word of the exchange ring starts as "not written yet"; the status block and the placement words are clear
+       // (a later launch of the call: the placement words alone, what the earlier ones said in the status block stays)
+      const size_t words = (size_t)kRing * ngroups * G * 16 * MT * 16 * (bf16 ? 2 : 4) / 4;
+      const int blocks = (int)((words / 4 + 255) / 256);
+      const size_t skip = launch_no++ > 0 ? kStatusBytes : 0;
+      hipLaunchKernelGGL(clear_workspace_kernel, dim3(blocks < 16 ? 16 : (blocks > 1024 ? 1024 : blocks)), dim3(256), 0, stream,
+                         (uint32_t *)((char *)a->workspace + skip), (kHeaderBytes - skip) / 4,
+                         (uint32_t *)((char *)a->workspace + kHeaderBytes), words);
     }
     SeqParams p;
     p.wx = a->wx; p.wx_sb = a->wx_stride_b; p.wx_st = a->wx_stride_t;
@@ -399,6 +399,7 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr) {
     p.head0 = head0; p.NHL = NHL;
     p.spin_limit = a->spin_limit;
     p.coef_out = a->coef_out;
+    p.abort_host = abort_host;
     // a prefetch wave issues 2 (bf16) or 4 (fp32) scalar loads per batch row of a tile; 8 per wave and iteration
     // and 16 in all are what the scalar cache sustains, a tile that needs more goes without (prefetch waves that
     // fall behind hold up the barriers: measured 2x slower)
@@ -1063,7 +1064,7 @@ size_t xs_slstm_workspace_bytes(int32_t B, int32_t T, int32_t NH, int32_t dh) {
   return kHeaderBytes + xbuf_elems(B, NH, dh) * 4;
 }
 
-int xs_slstm_forward(const xs_slstm_args *args) {
+int xs_slstm_forward_watched(const xs_slstm_args *args, uint32_t *abort_host) {
   g_err[0] = 0;
   const int rc = validate(args, false);
   if (rc != XS_OK) return rc;
@@ -1072,12 +1073,14 @@ int xs_slstm_forward(const xs_slstm_args *args) {
     size_t need = 0;
     const int rd = run_forward(args, &need);
     if (rd != XS_OK) return rd;
-    return run_forward(args);  // (also for one token: the step kernels keep no gate values)
+    return run_forward(args, nullptr, abort_host);  // (also for one token: the step kernels keep no gate values)
   }
   // one token: the tiled step kernel (no waits between compute units, bit-identical to the sequence kernel)
   if (args->T == 1 && args->B > 0 && args->r_dtype == args->wx_dtype) return run_step(args);
-  return run_forward(args);
+  return run_forward(args, nullptr, abort_host);
 }
+
+int xs_slstm_forward(const xs_slstm_args *args) { return xs_slstm_forward_watched(args, nullptr); }
 
 int xs_slstm_forward_static(const xs_slstm_args *args) {
   g_err[0] = 0;

@@ -27,6 +27,7 @@ struct SeqParams {
   int rows_per_wg;
   long long spin_limit;
   int prefetch;  // number of prefetch waves launched behind the six others (0 .. kMaxPrefetchWaves)
+  unsigned int *abort_host;  // a word in pinned host memory that a workgroup finishing after a give-up sets, or null
   float *coef_out;  // COEF variant: the backward pass's nine coefficients per step and element,
                     // [T][ceil(B/4)][NH][dh/64][4 rows][9][64 units] (what slstm_bwd_quad_kernel reads); else unused
 };
@@ -681,6 +682,7 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
     }
 #endif
     const bool poisoned = __hip_atomic_load(&p.status->aborted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
+    if (poisoned) report_abort(p.abort_host);
     if (gate_lane && brow < rend) {
       const long long o = (long long)brow * H + col;
       if (poisoned) st = CellState{kPoison, kPoison, kPoison, kPoison};
@@ -1138,6 +1140,7 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
 
   // ---- final state (NaN when a bounded wait ran out anywhere in the call: see the drainer)
   const bool poisoned = __hip_atomic_load(&p.status->aborted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
+  if (poisoned) report_abort(p.abort_host);
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int brow = rowbase + mt * 16 + pb;

@@ -450,6 +450,7 @@ __global__ __launch_bounds__(kRolesThreads) void slstm_seq_roles_kernel(SeqParam
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // ---- final state; NaN all over this workgroup's outputs when a bounded wait ran out anywhere in the call
     const bool poisoned = __hip_atomic_load(&p.status->aborted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
+    if (poisoned) report_abort(p.abort_host);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const int brow = rowbase + mt * 16 + pb;

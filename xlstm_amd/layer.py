@@ -206,6 +206,13 @@ class sLSTMLayer(nn.Module):
     def forward(self, x: torch.Tensor, conv_state: Optional[torch.Tensor] = None,
                 slstm_state: Optional[torch.Tensor] = None, return_last_state: bool = False,
                 reset_mask: Optional[torch.Tensor] = None, **kwargs):
+        if x.is_cuda:
+            cell = self.slstm_cell
+            native = cell._native()
+            fast = hipF._lib.host().layer_forward(self, native, x, conv_state, slstm_state, return_last_state, reset_mask)
+            if fast is not None:
+                cell._rt.last_workspace = native
+                return fast
         B, S, _ = x.shape
         if isinstance(conv_state, (tuple, list)):  # the ring a step returned (conv.py:131-157): oldest input first
             conv_state = conv_state[0]
@@ -241,6 +248,13 @@ class sLSTMLayer(nn.Module):
         ``slstm_state_out`` / ``h_out`` / ``h_prev`` are handed to the cell's ``step``; ``conv_state_out``
         ([B,k,D]) receives the new convolution ring and ``out`` ([B,1,D]) the result - both only on the engine's
         bfloat16 path (``_fused``), elsewhere fresh tensors are returned as usual."""
+        cell = self.slstm_cell
+        if x.is_cuda and cell._rt.step_plan is not None:
+            fast = hipF._lib.host().layer_step(self, cell._native(), x, conv_state, slstm_state, slstm_state_out, conv_state_out,
+                                               h_out, h_prev, out)
+            if fast is not None:
+                cell._rt.last_workspace = cell._rt.step_plan[1].workspace
+                return fast
         B, S, _ = x.shape
         fused = self._fused(x)
         if self.config.conv1d_kernel_size > 0 and fused:
