@@ -260,13 +260,33 @@ StepResult run_step(CellPath &c, const at::Tensor &x, const at::Tensor &state, c
   return out;
 }
 
+// Ordinary reasons for the general path, looked at in front of everything else: an exception costs tens of microseconds
+// in a process with as many libraries as this one, and a training loop or the first token of a batch size comes here on
+// every call.
+bool plan_fits(const CellPath &c, PyObject *x, PyObject *state) {
+  if (!c.plan || !THPVariable_Check(x) || !THPVariable_Check(state)) return false;
+  const at::Tensor &s = THPVariable_Unpack(state);
+  if (s.scalar_type() != at::kFloat || s.dim() != 3 || s.size(1) != c.step_B) return false;
+  PyObject *ro = PyDict_GetItem(c.parameters, g_names.r), *bo = PyDict_GetItem(c.parameters, g_names.b);
+  if (!ro || !bo || !THPVariable_Check(ro) || !THPVariable_Check(bo)) return false;
+  const at::Tensor &r = THPVariable_Unpack(ro), &b = THPVariable_Unpack(bo);
+  return r.data_ptr() == c.r_ptr && b.data_ptr() == c.b_ptr && version_of(r) == c.r_version && version_of(b) == c.b_version &&
+         THPVariable_Unpack(x).scalar_type() == c.step_dtype && !c.records(THPVariable_Unpack(x), &s, r, b);
+}
+bool recording(const CellPath &c, PyObject *x, PyObject *state) {
+  if (!at::GradMode::is_enabled()) return false;
+  PyObject *ro = PyDict_GetItem(c.parameters, g_names.r), *bo = PyDict_GetItem(c.parameters, g_names.b);
+  if (!ro || !bo || !THPVariable_Check(ro) || !THPVariable_Check(bo) || !THPVariable_Check(x)) return true;
+  return c.records(THPVariable_Unpack(x), !absent(state) && THPVariable_Check(state) ? &THPVariable_Unpack(state) : nullptr, THPVariable_Unpack(ro), THPVariable_Unpack(bo));
+}
+
 inline const at::Tensor *optional_tensor(PyObject *o) { return absent(o) ? nullptr : &tensor_of(o); }
 
 // step(input, state, reset_mask, state_out, h_out, h_prev, config, keep_state_fp32) -> (output, state) or None
 PyObject *cell_step_(CellPath &c, PyObject *const *args) {
-  if (!absent(args[2]) || absent(args[1]) || at::autocast::is_autocast_enabled(at::kCUDA)) throw NotCovered{};
+  if (!absent(args[2]) || absent(args[1]) || at::autocast::is_autocast_enabled(at::kCUDA) || !plan_fits(c, args[0], args[1])) Py_RETURN_NONE;
   const at::Tensor &x = tensor_of(args[0]), &state = tensor_of(args[1]);
-  if (!c.plan || !input_is_bsgnh(args[6])) throw NotCovered{};
+  if (!input_is_bsgnh(args[6])) throw NotCovered{};
   const OutShape shape = out_shape(args[6]);
   const bool keep = args[7] == Py_True;
   c10::OptionalDeviceGuard guard(c.device);
@@ -343,7 +363,7 @@ Sequence run_sequence(CellPath &c, at::Tensor x, const at::Tensor *state, const 
 
 // forward(input, state, reset_mask, config, keep_state_fp32) -> (output, state) or None
 PyObject *cell_forward_(CellPath &c, PyObject *const *args) {
-  if (at::autocast::is_autocast_enabled(at::kCUDA)) throw NotCovered{};
+  if (at::autocast::is_autocast_enabled(at::kCUDA) || recording(c, args[0], args[1])) Py_RETURN_NONE;
   const at::Tensor &x = tensor_of(args[0]);
   if (x.dim() != 3 || !x.is_cuda()) throw NotCovered{};
   const at::Tensor *state = optional_tensor(args[1]), *mask = optional_tensor(args[2]);
@@ -528,6 +548,12 @@ void collect(PyObject *layer, PyObject *cell_path, const at::Tensor &x, LayerPar
   if (at::GradMode::is_enabled() && needs_grad) throw NotCovered{};  // (the cell's own parameters: looked at where it runs)
 }
 
+// (the ordinary reasons, without an exception: see plan_fits)
+bool engine_layer(PyObject *const *args) {
+  return THPVariable_Check(args[2]) && THPVariable_Unpack(args[2]).scalar_type() == at::kBFloat16 &&
+         !recording(*((CellPathObject *)args[1])->c, args[2], nullptr);
+}
+
 void run_conv(const LayerParts &p, const at::Tensor &x, const void *taps, int64_t taps_stride, const at::Tensor *mask, void *out, void *ring, void *stream) {
   xs_conv_args a{};
   a.B = (int32_t)x.size(0); a.T = (int32_t)x.size(1); a.D = (int32_t)p.D; a.K = (int32_t)p.K;
@@ -582,8 +608,8 @@ PyObject *first_of(PyObject *o) {  // a state that may come in a tuple or list o
 // layer_step(layer, cell path, x, conv_state, slstm_state, slstm_state_out, conv_state_out, h_out, h_prev, out)
 //   -> (out, {"conv_state": (ring,), "slstm_state": state}) or None
 PyObject *layer_step_(PyObject *const *args) {
+  if (absent(args[4]) || !engine_layer(args) || !plan_fits(*((CellPathObject *)args[1])->c, args[2], args[4])) Py_RETURN_NONE;
   const at::Tensor &x = tensor_of(args[2]);
-  if (absent(args[4])) throw NotCovered{};
   LayerParts p;
   collect(args[0], args[1], x, p);
   const at::Tensor &state = tensor_of(args[4]);
@@ -634,6 +660,7 @@ PyObject *layer_step_(PyObject *const *args) {
 
 // layer_forward(layer, cell path, x, conv_state, slstm_state, return_last_state, reset_mask) -> the layer's result or None
 PyObject *layer_forward_(PyObject *const *args) {
+  if (!engine_layer(args)) Py_RETURN_NONE;
   const at::Tensor &x_in = tensor_of(args[2]);
   LayerParts p;
   collect(args[0], args[1], x_in, p);

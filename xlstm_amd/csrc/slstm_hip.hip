@@ -32,8 +32,8 @@
 #include "slstm_seq_roles_kernel.h"
 #include "slstm_step_kernel.h"
 #include "slstm_step_pipe_kernel.h"
-#include "slstm_layer_kernels.h"
 #include "slstm_backward_kernels.h"
+#include "slstm_layer_kernels.h"
 #include "slstm_backward_quad_kernel.h"
 #include "slstm_backward_step_kernel.h"
 #include "slstm_step_feed_kernel.h"
@@ -881,6 +881,39 @@ int run_conv(const xs_conv_args *a) {
   return XS_OK;
 }
 
+template <int BM, int BN, int D>
+int launch_gates(const xs_gates_args *a, GatesParams p, hipStream_t stream) {
+  p.n_tiles = 4 * a->NH * (a->dh / BN);
+  p.m_tiles = (a->M + BM - 1) / BM;
+  const int w_major = p.m_tiles <= 8;
+  const long long grid = w_major ? (long long)8 * ((p.n_tiles + 7) / 8) * p.m_tiles : (long long)8 * ((p.m_tiles + 7) / 8) * p.n_tiles;
+  if (grid > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many tiles for one launch");
+  if ((long long)BM * a->x_stride_row * 2 >= (1ll << 31) || (long long)BM * a->x_conv_stride_row * 2 >= (1ll << 31))
+    return fail(XS_ERR_UNSUPPORTED, "%d rows of x span 2 GiB or more", BM);
+  void (*kern)(GatesParams, int) = headwise_gates_kernel<BM, BN, D>;
+  const size_t lds = (size_t)D * (BM + BN) * 128;
+  if (lds > 64 * 1024) {
+    const int rc = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
+    if (rc != XS_OK) return rc;
+  }
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, stream, p, w_major);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? XS_OK : fail(XS_ERR_LAUNCH, "gate projection kernel launch failed: %s", hipGetErrorString(e));
+}
+
+// Tiles of the general kernel, by the number of tokens (us at 4 heads of 1024; the kernel before it in brackets):
+// up to 32 token tiles of 16 (M 1: 7.3 [101], M 30: 8.1 [103]); 128 x 128 tiles where the head dim allows them and they
+// fill the compute units (M 1024: 43 [215], M 16384: 786 [2828]); 64 x 64 in between and for the other head dims (M 64:
+// 9.3 [106]; 4 heads of 192, M 4096: 17.3 [40.7]).  A ring of few slots lets several workgroups share a compute unit,
+// which is worth more than slabs asked for further ahead.
+int launch_gates_tiles(const xs_gates_args *a, const GatesParams &p, hipStream_t stream) {
+  const int cus = device_cus();
+  if (cus <= 0) return fail(XS_ERR_DEVICE, "cannot query the device");
+  if (a->M <= 32) return launch_gates<16, 64, 4>(a, p, stream);
+  if (a->dh % 128 == 0 && (long long)((a->M + 127) / 128) * 4 * a->NH * (a->dh / 128) >= cus) return launch_gates<128, 128, 2>(a, p, stream);
+  return launch_gates<64, 64, 3>(a, p, stream);
+}
+
 int run_gates(const xs_gates_args *a) {
   if (!a) return fail(XS_ERR_NULL, "args is NULL");
   if (a->M < 0 || a->NH <= 0 || a->dh <= 0) return fail(XS_ERR_SHAPE, "bad dims M=%d NH=%d dh=%d", a->M, a->NH, a->dh);
@@ -903,43 +936,32 @@ int run_gates(const xs_gates_args *a) {
   p.out = (uint16_t *)a->out; p.out_sr = a->out_stride_row;
   p.M = a->M; p.NH = a->NH; p.dh = a->dh;
   hipStream_t stream = (hipStream_t)a->stream;
-  if (a->dh == 128 || a->dh == 256) {
-    // weights resident in registers, workgroups walk over token tiles
-    const int cus = device_cus();
-    if (cus <= 0) return fail(XS_ERR_DEVICE, "cannot query the device");
-    const int combos = 2 * a->NH;  // (head, operand)
-    const int bm = a->dh == 256 ? 64 : 32;  // tokens per tile: threads / 8
+  const int combos = 2 * a->NH;               // (head, operand)
+  const int bm = a->dh == 256 ? 64 : 32;      // the resident kernel's tokens per tile: threads / 8
+  const int cus = device_cus();
+  if (cus <= 0) return fail(XS_ERR_DEVICE, "cannot query the device");
+  const int parts = cus / combos > 1 ? cus / combos : 1;
+  if ((a->dh == 128 || a->dh == 256) && (a->M + bm - 1) / bm >= 4 * parts) {
+    // weights resident in registers, workgroups walk over token tiles: pays from four tiles per workgroup on (8 heads of
+    // 256, M 4096: 34 us against 49 with the general kernel; M 1024, one tile each: 16.7 against 13.6)
     p.m_tiles = (a->M + bm - 1) / bm;
     p.n_tiles = combos;
-    int parts = cus / combos;
-    if (parts < 1) parts = 1;
-    if (parts > p.m_tiles) parts = p.m_tiles;
-    if ((long long)((a->M + 63) / 64) * combos < cus) {
-      // too few token tiles to fill the device that way (a decode step): split the units instead
-      p.m_tiles = (a->M + 63) / 64;
-      p.n_tiles = 4 * a->NH * (a->dh / 64);
-      const size_t lds = (size_t)128 * (a->dh * 2 + 16);
-      void (*kern)(GatesParams) = a->dh == 256 ? headwise_gates_slab_kernel<4> : headwise_gates_slab_kernel<2>;
-      if (lds > 64 * 1024) {
-        const int rc = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
-        if (rc != XS_OK) return rc;
-      }
-      hipLaunchKernelGGL(kern, dim3((unsigned)(p.m_tiles * p.n_tiles)), dim3(256), lds, stream, p);
-    } else if (a->dh == 256)
-      hipLaunchKernelGGL(headwise_gates_resident_kernel<4>, dim3((unsigned)(combos * parts)), dim3(512), 0, stream, p, combos, parts);
-    else
-      hipLaunchKernelGGL(headwise_gates_resident_kernel<2>, dim3((unsigned)(combos * parts)), dim3(256), 0, stream, p, combos, parts);
+    if (a->dh == 256) hipLaunchKernelGGL(headwise_gates_resident_kernel<4>, dim3((unsigned)(combos * parts)), dim3(512), 0, stream, p, combos, parts);
+    else hipLaunchKernelGGL(headwise_gates_resident_kernel<2>, dim3((unsigned)(combos * parts)), dim3(256), 0, stream, p, combos, parts);
+  } else if ((a->dh == 128 || a->dh == 256) && a->M <= 256) {
+    // a decode step: every compute unit fetches its share of the weights once, the whole K range at once (8 heads of 128,
+    // M 256: 3.4 us against 3.8)
+    p.m_tiles = (a->M + 63) / 64;
+    p.n_tiles = 4 * a->NH * (a->dh / 64);
+    const size_t lds = (size_t)128 * (a->dh * 2 + 16);
+    void (*kern)(GatesParams) = a->dh == 256 ? headwise_gates_slab_kernel<4> : headwise_gates_slab_kernel<2>;
+    if (lds > 64 * 1024) {
+      const int rc = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
+      if (rc != XS_OK) return rc;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)(p.m_tiles * p.n_tiles)), dim3(256), lds, stream, p);
   } else {
-    // tile: 128 tokens when there are enough of them to fill the compute units, 128 units when dh allows
-    const int bn = a->dh % 128 == 0 ? 128 : 64;
-    const int bm = a->M >= 4096 ? 128 : 64;
-    p.m_tiles = (a->M + bm - 1) / bm;
-    p.n_tiles = 4 * a->NH * (a->dh / bn);
-    const long long grid = (long long)8 * ((p.m_tiles + 7) / 8) * p.n_tiles;
-    if (grid > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many tiles for one launch");
-    void (*kern)(GatesParams) = bm == 128 ? (bn == 128 ? headwise_gates_kernel<128, 128> : headwise_gates_kernel<128, 64>)
-                                          : (bn == 128 ? headwise_gates_kernel<64, 128> : headwise_gates_kernel<64, 64>);
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), 0, stream, p);
+    return launch_gates_tiles(a, p, stream);
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(XS_ERR_LAUNCH, "gate projection kernel launch failed: %s", hipGetErrorString(e));

@@ -113,12 +113,8 @@ __global__ __launch_bounds__(256) void causal_conv_silu_kernel(ConvParams p) {
 // the four headwise gate projections and their concatenation
 // (xlstm/blocks/slstm/layer.py:144-153, xlstm/components/linear_headwise.py:75-82):
 //   out[m, g*H + h*dh + o] = sum_d A_g[m, h*dh + d] * W_g[h, o, d]
-// with A_g = x_conv for the slots i and f, x for z and o.  A workgroup computes BM tokens x BN output
-// units of one (slot, head); K = dh is walked in stages of 64 inputs (128-byte rows), each staged
-// through LDS once; the loads of the next stage are in flight during the MFMAs of the current one.
-// Four waves as 2 x 2.  The product is formed transposed (units on the MFMA M axis), so a lane ends
-// with 4 consecutive units of one token.  Workgroup i runs on XCD i % 8: the tiles of one block of
-// tokens are given to ONE XCD, so that x and x_conv are fetched from HBM once.
+// with A_g = x_conv for the slots i and f, x for z and o.  The products are formed transposed (units on the MFMA M
+// axis), so a lane ends with 4 consecutive units of one token.
 // ---------------------------------------------------------------------------
 struct GatesParams {
   const uint16_t *x, *xc;
@@ -132,93 +128,93 @@ struct GatesParams {
 
 constexpr int kGateRowBytes = 144;  // 128 bytes of data + 16 of padding: conflict-free 16-byte reads
 
-template <int BM, int BN>
-__global__ __launch_bounds__(256) void headwise_gates_kernel(GatesParams p) {
-  constexpr int AI = BM * 8 / 256;  // 16-byte pieces of the token tile a thread stages per K stage
-  constexpr int WI = BN * 8 / 256;  // ... of the weight tile
-  constexpr int TM = BM / 32, TN = BN / 32;  // MFMA tiles of a wave: TM token tiles x TN unit tiles
-  __shared__ __attribute__((aligned(16))) unsigned char abuf[BM * kGateRowBytes];
-  __shared__ __attribute__((aligned(16))) unsigned char wbuf[BN * kGateRowBytes];
+// Every head dim (a multiple of 64) and every number of tokens.  A workgroup computes BM tokens x BN units of one (slot,
+// head); K is walked in slabs of 64 inputs (rows of 128 bytes) that the waves bring straight into a ring of D LDS slots,
+// D - 1 slabs ahead, with waits counted by hand and one barrier per slab.  A load that writes LDS fills 1 KiB in a row (8
+// rows), so the rows cannot be padded: piece g (16 bytes) of row r sits at position g ^ (r & 7), which keeps the MFMA
+// waves' 16-byte reads free of bank conflicts.  What bounds it is one pass over the weights (few tokens) or over x and
+// the output (many).  `w_major`: workgroup i runs on XCD i % 8, and with few token tiles all tiles of one block of
+// weights are given to ONE XCD (the weights are read once, and every XCD has work even for one token tile); with many,
+// all tiles of one block of tokens (x is read once).
+template <int BM, int BN, int D>
+__global__ __launch_bounds__(256) void headwise_gates_kernel(GatesParams p, int w_major) {
+  constexpr int SLOT = (BM + BN) * 128;
+  constexpr int NL = (BM + BN) / 8, ML = BM / 8;           // loads per slab, the token tile's first
+  constexpr int PW = (NL + 3) / 4;                         // loads of a wave per slab (where NL is no multiple of 4: the first waves')
+  constexpr int WM = BM == 16 ? 1 : 2, WN = 4 / WM;        // waves over tokens x over units
+  constexpr int TM = BM / 16 / WM, TN = BN / 16 / WN;      // MFMA tiles of a wave
+  extern __shared__ __attribute__((aligned(1024))) unsigned char gates_lds[];
 
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = (int)uniform((uint32_t)(tid >> 6));
   const int q = lane >> 4, r16 = lane & 15;
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / WN, wn = wave % WN;
 
-  const int xcd = blockIdx.x & 7;
-  const int jj = blockIdx.x >> 3;
-  const int mtile = (jj / p.n_tiles) * 8 + xcd;
-  if (mtile >= p.m_tiles) return;  // the whole workgroup leaves before any barrier
-  int nt = jj % p.n_tiles;
-  const int npu = p.dh / BN;  // unit tiles per (slot, head)
+  const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
+  int mtile, nt;
+  if (w_major) { nt = (jj / p.m_tiles) * 8 + xcd; mtile = jj % p.m_tiles; }
+  else { mtile = (jj / p.n_tiles) * 8 + xcd; nt = jj % p.n_tiles; }
+  if (mtile >= p.m_tiles || nt >= p.n_tiles) return;  // the whole workgroup leaves before any barrier
+  const int dh = p.dh, npu = dh / BN;  // unit tiles per (slot, head)
   const int ut = nt % npu; nt /= npu;
-  const int slot_in_pair = nt & 1; nt >>= 1;
-  const int pair = nt & 1;
-  const int head = nt >> 1;
-  const int slot = pair * 2 + slot_in_pair;
-  const int m0 = mtile * BM;
-  const int n0 = ut * BN;
-  const int dh = p.dh;
+  const int slot = nt & 3, head = nt >> 2;
+  const int m0 = mtile * BM, n0 = ut * BN;
+  const int rows = p.M - m0 < BM ? p.M - m0 : BM;
 
-  const uint16_t *abase = pair ? p.x : p.xc;
-  const long long asr = pair ? p.x_sr : p.xc_sr;
-  const uint16_t *wbase = p.w[slot] + ((long long)head * dh + n0) * dh;
+  const long long asr = slot >= 2 ? p.x_sr : p.xc_sr;
+  const unsigned long long ab = reinterpret_cast<unsigned long long>((slot >= 2 ? p.x : p.xc) + (long long)m0 * asr + (long long)head * dh);
+  const unsigned long long wb = reinterpret_cast<unsigned long long>(p.w[slot] + ((long long)head * dh + n0) * dh);
+  // (rows past the last token lie past the end of the descriptor: they read zeros)
+  const u32x4_t ars = {uniform((uint32_t)ab), uniform((uint32_t)(ab >> 32) & 0xFFFFu), uniform((uint32_t)((rows - 1) * asr * 2 + dh * 2)), 0x00020000u};
+  const u32x4_t wrs = {uniform((uint32_t)wb), uniform((uint32_t)(wb >> 32) & 0xFFFFu), (uint32_t)(BN * dh * 2), 0x00020000u};
+  const int sub = lane >> 3, swz = ((lane & 7) ^ sub) << 4;
+  const uint32_t avo = (uint32_t)(sub * asr * 2 + swz), wvo = (uint32_t)(sub * dh * 2 + swz);
+  const uint32_t lds0 = (uint32_t)(unsigned long long)((__attribute__((address_space(3))) unsigned char *)gates_lds);
 
-  const uint16_t *asrc[AI];
-  int adst[AI];
+  const int nslab = dh >> 6;
+  auto request = [&](int s) {
+    const uint32_t at = lds0 + (uint32_t)(s % D) * SLOT;
 #pragma unroll
-  for (int j = 0; j < AI; ++j) {
-    const int e = tid + 256 * j;
-    const int row = e >> 3, pc = e & 7;
-    const int m = m0 + row < p.M ? m0 + row : p.M - 1;
-    asrc[j] = abase + (long long)m * asr + (long long)head * dh + pc * 8;
-    adst[j] = row * kGateRowBytes + pc * 16;
-  }
-  const uint16_t *wsrc[WI];
-  int wdst[WI];
-#pragma unroll
-  for (int j = 0; j < WI; ++j) {
-    const int e = tid + 256 * j;
-    const int row = e >> 3, pc = e & 7;
-    wsrc[j] = wbase + (long long)row * dh + pc * 8;
-    wdst[j] = row * kGateRowBytes + pc * 16;
-  }
+    for (int k = 0; k < PW; ++k) {
+      const int l = wave + 4 * k;
+      if (NL % 4 && l >= NL) break;
+      if (l < ML) bwd_fetch_to_lds_b128(ars, uniform(at + l * 1024), avo + (uint32_t)(l * 16 * asr) + (uint32_t)s * 128u);
+      else bwd_fetch_to_lds_b128(wrs, uniform(at + l * 1024), wvo + (uint32_t)((l - ML) * 16 * dh) + (uint32_t)s * 128u);
+    }
+  };
+  // waits until at most `ahead` slabs' loads of this wave are in flight
+  const bool full = NL % 4 == 0 || wave < NL % 4;
+  auto landed = [&](int ahead) {
+    switch (ahead) {
+#define XS_GATES_WAIT(n) case n: if (n <= D - 2) { if (full) asm volatile("s_waitcnt vmcnt(%0)" :: "n"((n) * PW) : "memory"); \
+                                                   else asm volatile("s_waitcnt vmcnt(%0)" :: "n"((n) * (PW - 1)) : "memory"); } break;
+      XS_GATES_WAIT(0) XS_GATES_WAIT(1) XS_GATES_WAIT(2) XS_GATES_WAIT(3) XS_GATES_WAIT(4) XS_GATES_WAIT(5) XS_GATES_WAIT(6)
+#undef XS_GATES_WAIT
+    }
+  };
 
   f32x4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int arow = (wm * (BM / WM) + r16) * 128, wrow = (BM + wn * (BN / WN) + r16) * 128;
+  const int swr[2] = {((0 + q) ^ (r16 & 7)) << 4, ((4 + q) ^ (r16 & 7)) << 4};
 
-  uint4 areg[AI], wreg[WI];
-#pragma unroll
-  for (int j = 0; j < AI; ++j) areg[j] = *reinterpret_cast<const uint4 *>(asrc[j]);
-#pragma unroll
-  for (int j = 0; j < WI; ++j) wreg[j] = *reinterpret_cast<const uint4 *>(wsrc[j]);
-
-  const int nstage = dh >> 6;
-  for (int s = 0; s < nstage; ++s) {
-    if (s) __syncthreads();  // every wave is done reading the previous stage
-#pragma unroll
-    for (int j = 0; j < AI; ++j) *reinterpret_cast<uint4 *>(&abuf[adst[j]]) = areg[j];
-#pragma unroll
-    for (int j = 0; j < WI; ++j) *reinterpret_cast<uint4 *>(&wbuf[wdst[j]]) = wreg[j];
-    __syncthreads();
-    if (s + 1 < nstage) {
-#pragma unroll
-      for (int j = 0; j < AI; ++j) areg[j] = *reinterpret_cast<const uint4 *>(asrc[j] + (s + 1) * 64);
-#pragma unroll
-      for (int j = 0; j < WI; ++j) wreg[j] = *reinterpret_cast<const uint4 *>(wsrc[j] + (s + 1) * 64);
-    }
+  for (int s = 0; s < D - 1 && s < nslab; ++s) request(s);
+  for (int s = 0; s < nslab; ++s) {
+    const int left = nslab - 1 - s;
+    landed(left < D - 2 ? left : D - 2);
+    lds_barrier();  // slab s is in LDS, and every wave is done with slab s - 1, whose slot the next request fills
+    if (s + D - 1 < nslab) request(s + D - 1);
+    const unsigned char *b = gates_lds + (s % D) * SLOT;
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       uint4 av[TM], wv[TN];
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
-        av[i] = *reinterpret_cast<const uint4 *>(&abuf[(wm * (BM / 2) + 16 * i + r16) * kGateRowBytes + ks * 64 + q * 16]);
+      for (int i = 0; i < TM; ++i) av[i] = *reinterpret_cast<const uint4 *>(b + arow + 16 * i * 128 + swr[ks]);
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
-        wv[j] = *reinterpret_cast<const uint4 *>(&wbuf[(wn * (BN / 2) + 16 * j + r16) * kGateRowBytes + ks * 64 + q * 16]);
+      for (int j = 0; j < TN; ++j) wv[j] = *reinterpret_cast<const uint4 *>(b + wrow + 16 * j * 128 + swr[ks]);
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -227,11 +223,11 @@ __global__ __launch_bounds__(256) void headwise_gates_kernel(GatesParams p) {
     }
   }
 
-  // lane (r16, q) holds token m0 + wm*BM/2 + 16 i + r16, units n0 + wn*BN/2 + 16 j + 4 q .. +3
-  const long long colbase = (long long)slot * p.NH * dh + (long long)head * dh + n0 + wn * (BN / 2) + 4 * q;
+  // lane (r16, q) holds token m0 + wm*BM/WM + 16 i + r16, units n0 + wn*BN/WN + 16 j + 4 q .. +3
+  const long long colbase = (long long)slot * p.NH * dh + (long long)head * dh + n0 + wn * (BN / WN) + 4 * q;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    const int m = m0 + wm * (BM / 2) + 16 * i + r16;
+    const int m = m0 + wm * (BM / WM) + 16 * i + r16;
     if (m < p.M) {
       uint16_t *orow = p.out + (long long)m * p.out_sr + colbase;
 #pragma unroll

@@ -650,9 +650,9 @@ def headwise_gates(x: torch.Tensor, x_conv: torch.Tensor, weights, num_heads: in
     dh = H // num_heads
     x2 = x.reshape(-1, H)
     xc2 = x_conv.reshape(-1, H)
-    if x2.stride(1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
+    if x2.stride(1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16 or x2.stride(0) >= 1 << 22:
         x2 = x2.contiguous()
-    if xc2.stride(1) != 1 or xc2.stride(0) % 8 or xc2.data_ptr() % 16:
+    if xc2.stride(1) != 1 or xc2.stride(0) % 8 or xc2.data_ptr() % 16 or xc2.stride(0) >= 1 << 22:
         xc2 = xc2.contiguous()
     M = int(x2.shape[0])
     ws = []
