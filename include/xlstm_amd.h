@@ -382,11 +382,29 @@ int xs_slstm_backward_prepare(const xs_slstm_bwd_args *args);
 int xs_slstm_backward(const xs_slstm_bwd_args *args);
 
 /*
+ * Training at small head dims (multiples of 8 up to 128): a head stays in one compute unit, forward and backward, nothing
+ * waits for another compute unit and nothing can give up.
+ *   xs_slstm_train_coef_floats  floats of the coefficients such a training forward leaves, 0 where the pair below does
+ *                               not cover the call.
+ *   xs_slstm_train_forward      xs_slstm_forward (same bits) that also leaves the coefficients of the backward pass in
+ *                               `coef`, in an order of its own (slstm_local_kernel.h); coef_out must be NULL.
+ *   xs_slstm_train_backward     the reverse pass from them: reads B, T, NH, dh, dtype, coef, d_h (with its strides in
+ *                               elements, innermost H contiguous: the gradient as the layer behind the cell holds it
+ *                               needs no copy), d_s_final, r (the forward's layout and, with r_dtype XS_F32, its float32
+ *                               master), reset, recurrent_cut, recurrent_clipval; writes d_wx (d_wx_dtype) and d_s0.
+ * The gradients of r and the bias: xs_slstm_backward_params, as for the other kernels.
+ * Like coef_out, this takes the place of the state history and gate cache of the reference (slstm.cc:79-108).
+ */
+size_t xs_slstm_train_coef_floats(int32_t B, int32_t T, int32_t NH, int32_t dh, int32_t dtype);
+int xs_slstm_train_forward(const xs_slstm_args *args, float *coef);
+int xs_slstm_train_backward(const xs_slstm_bwd_args *args, int64_t d_h_stride_b, int64_t d_h_stride_t, int32_t r_dtype);
+
+/*
  * xs_slstm_backward_params   the gradients of the recurrent matrix and the bias from the gate deltas that
  *   xs_slstm_backward left in d_wx and the forward's outputs: d_r[h][g*dh+a][d] = sum over rows and steps of
  *   d_wx[b,t,g,h,a] * y_{t-1}[b,h,d] (y_{-1} the y plane of s0; zero where reset[b,t] is set), d_bias[h][g][a] = sum of
  *   d_wx[b,t,g,h,a].  Replaces the strided-batched GEMM and the bias aggregation behind the reference's time loop
- *   (slstm_backward.cu:381-386, 52-108).  Uses B, T, NH, dh (a multiple of 64), dtype, d_wx and its strides, h_out, s0,
+ *   (slstm_backward.cu:381-386, 52-108).  Uses B, T, NH, dh (a multiple of 8), dtype, d_wx and its strides, h_out, s0,
  *   reset, d_r, d_bias, stream.  With bf16 the deltas are rounded to bf16 for the product (float32 sums), as the
  *   reference's gate cache is.  The sums over slices of B*T are added with float atomics: their last bits depend on
  *   the order the compute units finish in.

@@ -36,6 +36,9 @@ EXPORTS = (
     "xs_headwise_gates",
     "xs_headwise_group_norm",
     "xs_measure_stage",
+    "xs_slstm_train_coef_floats",
+    "xs_slstm_train_forward",
+    "xs_slstm_train_backward",
 )
 
 
@@ -215,6 +218,12 @@ def load() -> ctypes.CDLL:
     lib.xs_headwise_gates.argtypes = [ctypes.POINTER(GatesArgs)]
     lib.xs_headwise_group_norm.restype = ctypes.c_int
     lib.xs_headwise_group_norm.argtypes = [ctypes.POINTER(NormArgs)]
+    lib.xs_slstm_train_coef_floats.restype = ctypes.c_size_t
+    lib.xs_slstm_train_coef_floats.argtypes = [ctypes.c_int32] * 5
+    lib.xs_slstm_train_forward.restype = ctypes.c_int
+    lib.xs_slstm_train_forward.argtypes = [ctypes.POINTER(SlstmArgs), ctypes.c_void_p]
+    lib.xs_slstm_train_backward.restype = ctypes.c_int
+    lib.xs_slstm_train_backward.argtypes = [ctypes.POINTER(SlstmBwdArgs), ctypes.c_int64, ctypes.c_int64, ctypes.c_int32]
     lib.xs_measure_stage.restype = ctypes.c_int
     lib.xs_measure_stage.argtypes = [ctypes.POINTER(MeasureArgs)]
     if lib.xs_abi_version() != ABI_VERSION:

@@ -511,11 +511,14 @@ class sLSTMCell_hip(nn.Module):
             or (state is not None and state.requires_grad)
         )
         args = (x, r, self._bias_.detach().view(self.config.num_heads, 4, self.head_dim), state, reset_mask)
-        coef = None
+        coef = h = s = None
         if wants_grad and self.keep_backward_coefficients and x.is_cuda and not step:
-            coef = F_hip.backward_coefficients_buffer(x, self.config.num_heads)
-        h = s = None
-        if coef is not None:
+            coef = F_hip.training_coefficients(x, self.config.num_heads)
+            if coef is not None:
+                h, s = F_hip.slstm_forward(*args, s_out=state_out, workspace=ws, train_coef=coef)
+            else:
+                coef = F_hip.backward_coefficients_buffer(x, self.config.num_heads)
+        if coef is not None and h is None:
             try:
                 h, s = F_hip.slstm_forward(*args, s_out=state_out, workspace=ws, coef_out=coef)
             except F_hip.CoefficientsUnsupported:  # (nothing has run: the plain forward, and the backward recomputes)

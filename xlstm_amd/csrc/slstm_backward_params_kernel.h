@@ -26,6 +26,7 @@ namespace {
 
 struct BwdParamParams {
   int B, T, NH, dh;
+  int dhp;                   // the head dim up to a multiple of 64: the result is tiled as if the heads had that many units
   const float *d_wx;         // [B,T,4,NH,dh] float32 (bf16 with d_wx_bf16), strides in elements: the gate deltas
   long long d_wx_sb, d_wx_st;
   int d_wx_bf16;
@@ -46,7 +47,7 @@ constexpr int bwd_param_lds_bytes(bool bf16, int nt) {
   return 2 * kParamKC * ((kParamMT + kParamPad) + (nt + kParamPad)) * (bf16 ? 2 : 4);
 }
 
-template <bool BF16, int NT>  // NT: columns of the result per workgroup (64, 128 or 256; dh is a multiple of it)
+template <bool BF16, int NT>  // NT: columns of the result per workgroup (64, 128 or 256; dhp is a multiple of it)
 __global__ __launch_bounds__(512) void slstm_bwd_param_kernel(BwdParamParams p) {
   typedef typename std::conditional<BF16, uint16_t, float>::type elem_t;
   constexpr int ESZ = BF16 ? 2 : 4;
@@ -60,8 +61,8 @@ __global__ __launch_bounds__(512) void slstm_bwd_param_kernel(BwdParamParams p) 
   elem_t *const As = reinterpret_cast<elem_t *>(param_lds);                        // [2][32 k][LDA]
   elem_t *const Bs = reinterpret_cast<elem_t *>(param_lds) + 2 * kParamKC * LDA;   // [2][32 k][LDB]
 
-  const int dh = p.dh, H = p.NH * dh;
-  const int tiles_m = 4 * dh / kParamMT, tiles_n = dh / NT, tiles = tiles_m * tiles_n;
+  const int dh = p.dh, dhp = p.dhp, H = p.NH * dh;
+  const int tiles_m = 4 * dhp / kParamMT, tiles_n = dhp / NT, tiles = tiles_m * tiles_n;
   // placement: the workgroups of one (head, K slice) share its stream of y chunks; they take consecutive slots of ONE
   // XCD (workgroup i runs on XCD i % 8), so that stream is fetched into one L2 once
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
@@ -80,9 +81,11 @@ __global__ __launch_bounds__(512) void slstm_bwd_param_kernel(BwdParamParams p) 
   // ---- staging roles.  delta: thread -> step tid / 16 of the chunk, 8 consecutive m from 8 (tid % 16); y: thread ->
   //      step (tid / NROWTHREADS) (+ 512 / NROWTHREADS per pass), 8 consecutive n
   const int dk = tid >> 4, dm = (tid & 15) * 8;
-  const int dcol = m0 + dm;                       // row of the head's result = gate * dh + unit
-  const long long d_off = (long long)(dcol / dh) * H + (long long)head * dh + dcol % dh;
+  const int dcol = m0 + dm;                       // row of the head's result = gate * dhp + unit
+  const bool d_there = dcol % dhp < dh;           // (8 units at a time: dh is a multiple of 8)
+  const long long d_off = (long long)(dcol / dhp) * H + (long long)head * dh + dcol % dhp;
   const int yk = tid / NROWTHREADS, yn = (tid % NROWTHREADS) * 8;
+  const bool y_there = n0 + yn < dh;
   const bool y_thread = tid < kParamKC * NROWTHREADS;  // (NT 64: 256 threads cover the chunk)
   float bsum[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
   const bool dbf16 = BF16 && p.d_wx_bf16 != 0;  // the deltas lie in bf16 (only with bf16 operands)
@@ -101,10 +104,10 @@ __global__ __launch_bounds__(512) void slstm_bwd_param_kernel(BwdParamParams p) 
       const char *base = reinterpret_cast<const char *>(p.d_wx) + ((long long)b * p.d_wx_sb + (long long)t0 * p.d_wx_st) * dsz;
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
           const_cast<char *>(base), 0, (int)(((long long)(nrows - 1) * p.d_wx_st + 4ll * H) * dsz), 0x00020000);
-      const int vo = (int)(((long long)dk * p.d_wx_st + d_off) * dsz);
+      const int vo = d_there ? (int)(((long long)dk * p.d_wx_st + d_off) * dsz) : (int)0x80000000;
       s.d[0] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, vo, 0, 0));
       // (deltas in bf16: the thread's 8 values are the first 16 bytes; the second load asks past the end and reads zeros)
-      s.d[1] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, dbf16 ? (int)0x80000000 : vo + 16, 0, 0));
+      s.d[1] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, dbf16 || !d_there ? (int)0x80000000 : vo + 16, 0, 0));
     }
     // y_{t-1}: the outputs of steps t0 - 1 .. (row -1, in front of step 0, lies in front of the descriptor: zeros)
     const int tb = t0 > 0 ? t0 - 1 : 0;  // the step the descriptor starts at
@@ -112,7 +115,7 @@ __global__ __launch_bounds__(512) void slstm_bwd_param_kernel(BwdParamParams p) 
     const char *ybase = reinterpret_cast<const char *>(p.h_out) + ((long long)tb * BH + (long long)b * H + col) * ESZ;
     const int yrows = t0 + nrows - 1 - tb;  // rows of h_out behind ybase that the chunk's steps use (0: only step 0)
     const __amdgpu_buffer_rsrc_t yrs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<char *>(ybase), 0, yrows > 0 ? (int)(((long long)(yrows - 1) * BH + NT) * ESZ) : 0, 0x00020000);
+        const_cast<char *>(ybase), 0, yrows > 0 ? (int)(((long long)(yrows - 1) * BH + (NT < dh - n0 ? NT : dh - n0)) * ESZ) : 0, 0x00020000);
     const __amdgpu_buffer_rsrc_t frs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t *>(p.reset ? p.reset + (long long)b * p.reset_sb + t0 : reinterpret_cast<const uint8_t *>(p.d_wx)), 0,
         p.reset ? nrows : 0, 0x00020000);
@@ -121,7 +124,7 @@ __global__ __launch_bounds__(512) void slstm_bwd_param_kernel(BwdParamParams p) 
       const int k = yk + ps * (512 / NROWTHREADS);          // the chunk's step t0 + k
       const int row = t0 + k - 1 - tb;                      // its operand's row behind ybase; -1 in front of step 0
       // (threads beyond the chunk - NT 64: the upper half of the workgroup - ask out of range too)
-      const int vo = (y_thread && row >= 0) ? (int)(((long long)row * BH + yn) * ESZ) : (int)0x80000000;
+      const int vo = (y_thread && y_there && row >= 0) ? (int)(((long long)row * BH + yn) * ESZ) : (int)0x80000000;
       s.y[ps][0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(yrs, vo, 0, 0));
       if (!BF16) s.y[ps][BF16 ? 0 : 1] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(yrs, vo, 16, 0));
       s.flag[ps] = __builtin_amdgcn_raw_buffer_load_b8(frs, y_thread ? k : (int)0x80000000, 0, 0);
@@ -133,7 +136,7 @@ __global__ __launch_bounds__(512) void slstm_bwd_param_kernel(BwdParamParams p) 
     {
       const int b = b0 + dk;
       s.d[0] = s.d[1] = float4{0.0f, 0.0f, 0.0f, 0.0f};
-      if (b < p.B) {
+      if (b < p.B && d_there) {
         const char *src = reinterpret_cast<const char *>(p.d_wx) + ((long long)b * p.d_wx_sb + d_off) * (dbf16 ? 2 : 4);
         s.d[0] = *reinterpret_cast<const float4 *>(src);
         if (!dbf16) s.d[1] = *reinterpret_cast<const float4 *>(src + 16);
@@ -145,7 +148,7 @@ __global__ __launch_bounds__(512) void slstm_bwd_param_kernel(BwdParamParams p) 
 #pragma unroll
       for (int e = 0; e < (BF16 ? 1 : 2); ++e) s.y[ps][e] = uint4{0u, 0u, 0u, 0u};
       s.flag[ps] = 0u;
-      if (!y_thread || b >= p.B) continue;
+      if (!y_thread || !y_there || b >= p.B) continue;
       if (p.reset) s.flag[ps] = p.reset[(long long)b * p.reset_sb];
       const long long col = (long long)head * dh + n0 + yn;
       const float4 lo = *reinterpret_cast<const float4 *>(p.s0 + (long long)b * H + col);
@@ -282,7 +285,7 @@ __global__ __launch_bounds__(512) void slstm_bwd_param_kernel(BwdParamParams p) 
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int row = m0 + wm * (MTILES * 16) + 16 * i + 4 * q + e, col = n0 + wn * 64 + 16 * j + r16;
-        atomicAdd(p.d_r + ((long long)head * 4 * dh + row) * dh + col, acc[i][j][e]);
+        if (row % dhp < dh && col < dh) atomicAdd(p.d_r + ((long long)head * 4 * dh + (row / dhp) * dh + row % dhp) * dh + col, acc[i][j][e]);
       }
   // ---- ... and of the bias (the workgroups of the first column tile): the 32 threads that staged a group of 8 m add
   //      up through LDS (the staging buffers are free behind the last barrier)
@@ -295,8 +298,8 @@ __global__ __launch_bounds__(512) void slstm_bwd_param_kernel(BwdParamParams p) 
       float sum = 0.0f;
 #pragma unroll 8
       for (int k = 0; k < kParamKC; ++k) sum += red[k * kParamMT + tid];
-      const int row = m0 + tid;  // = gate * dh + unit
-      atomicAdd(p.d_bias + (long long)head * 4 * dh + row, sum);
+      const int row = m0 + tid;  // = gate * dhp + unit
+      if (row % dhp < dh) atomicAdd(p.d_bias + (long long)head * 4 * dh + (row / dhp) * dh + row % dhp, sum);
     }
   }
 }

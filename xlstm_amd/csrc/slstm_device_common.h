@@ -123,6 +123,13 @@ __global__ void clear_workspace_kernel(uint32_t *header, size_t nh, uint32_t *ri
   for (size_t i = i0; i < nr / 4; i += stride) r4[i] = make_uint4(kSentinel32, kSentinel32, kSentinel32, kSentinel32);
 }
 
+// two regions of zeros in one launch
+__global__ void clear_two_kernel(uint32_t *a, size_t na, uint32_t *b, size_t nb) {
+  const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = i0; i < na; i += stride) a[i] = 0u;
+  for (size_t i = i0; i < nb; i += stride) b[i] = 0u;
+}
+
 __global__ void copy_state_kernel(const float *s0, float *s_out, size_t n) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const size_t stride = (size_t)gridDim.x * blockDim.x;

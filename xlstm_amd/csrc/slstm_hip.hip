@@ -34,6 +34,7 @@
 #include "slstm_step_pipe_kernel.h"
 #include "slstm_backward_kernels.h"
 #include "slstm_layer_kernels.h"
+#include "slstm_local_kernel.h"
 #include "slstm_backward_quad_kernel.h"
 #include "slstm_backward_step_kernel.h"
 #include "slstm_step_feed_kernel.h"
@@ -258,6 +259,104 @@ int run_step(const xs_slstm_args *a) {
   return XS_OK;
 }
 
+// the type of d_wx that a backward call asks for
+int d_wx_type(const xs_slstm_bwd_args *a, int *is_bf16) {
+  *is_bf16 = 0;
+  if (a->d_wx_dtype == XS_F32) return XS_OK;
+  if (a->d_wx_dtype != XS_BF16 || a->dtype != XS_BF16) return fail(XS_ERR_DTYPE, "d_wx_dtype must be XS_F32, or XS_BF16 with dtype XS_BF16");
+  if (a->d_wx && (((uintptr_t)a->d_wx % 16) || (a->d_wx_stride_b % 8) || (a->d_wx_stride_t % 8)))
+    return fail(XS_ERR_ALIGN, "d_wx in bf16 must be 16-byte aligned and its strides multiples of 8 elements");
+  *is_bf16 = 1;
+  return XS_OK;
+}
+
+// ---- small heads: the kernels that keep a head in one compute unit (slstm_local_kernel.h)
+inline bool local_head(int dh) { return dh <= kLocalMaxHeadDim; }
+// ... and where the forward alone is faster that way: float32 beyond head dim 64 has 1,024 cycles of MFMA per wave and step
+// in one compute unit (1.56 us a step at head dim 128, against 1.24 for slstm_seq_kernel over eight)
+inline bool local_forward(int dh, bool bf16) { return dh <= (bf16 ? kLocalMaxHeadDim : 64); }
+inline int local_waves(int dh) { return (dh + 15) / 16; }
+
+template <bool BF16, bool COEF>
+void (*pick_local(int w))(LocalParams) {
+  switch (w) {
+    case 1: return slstm_local_kernel<BF16, 1, COEF>;
+    case 2: return slstm_local_kernel<BF16, 2, COEF>;
+    case 3: return slstm_local_kernel<BF16, 3, COEF>;
+    case 4: return slstm_local_kernel<BF16, 4, COEF>;
+    case 5: return slstm_local_kernel<BF16, 5, COEF>;
+    case 6: return slstm_local_kernel<BF16, 6, COEF>;
+    case 7: return slstm_local_kernel<BF16, 7, COEF>;
+    default: return slstm_local_kernel<BF16, 8, COEF>;
+  }
+}
+template <bool BF16, bool DWX16>
+void (*pick_local_bwd(int w))(LocalBwdParams) {
+  switch (w) {
+    case 1: return slstm_local_bwd_kernel<BF16, 1, DWX16>;
+    case 2: return slstm_local_bwd_kernel<BF16, 2, DWX16>;
+    case 3: return slstm_local_bwd_kernel<BF16, 3, DWX16>;
+    case 4: return slstm_local_bwd_kernel<BF16, 4, DWX16>;
+    case 5: return slstm_local_bwd_kernel<BF16, 5, DWX16>;
+    case 6: return slstm_local_bwd_kernel<BF16, 6, DWX16>;
+    case 7: return slstm_local_bwd_kernel<BF16, 7, DWX16>;
+    default: return slstm_local_bwd_kernel<BF16, 8, DWX16>;
+  }
+}
+// workgroups of a launch over (row tile of 4 rows, head) pairs: a multiple of 8 (one range per XCD)
+inline long long local_grid(int B, int NH) { return ((long long)((B + 3) / 4) * NH + 7) / 8 * 8; }
+
+int run_local(const xs_slstm_args *a, float *coef) {
+  const bool bf16 = a->wx_dtype == XS_BF16;
+  const int w = local_waves(a->dh);
+  const long long grid = local_grid(a->B, a->NH);
+  if (grid > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many row tiles for one launch");
+  LocalParams p;
+  p.wx = a->wx; p.wx_sb = a->wx_stride_b; p.wx_st = a->wx_stride_t;
+  p.r = a->r; p.r_bf16 = a->r_dtype == XS_BF16;
+  p.bias = a->bias; p.s0 = a->s0; p.reset = a->reset; p.reset_sb = a->reset_stride_b;
+  p.h_out = a->h_out; p.s_out = a->s_out; p.status = (xs_slstm_status *)a->workspace; p.coef = coef;
+  p.B = a->B; p.T = a->T; p.NH = a->NH; p.dh = a->dh;
+  void (*k)(LocalParams);
+  if (coef) k = bf16 ? pick_local<true, true>(w) : pick_local<false, true>(w);
+  else k = bf16 ? pick_local<true, false>(w) : pick_local<false, false>(w);
+  hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(64 * w), 0, (hipStream_t)a->stream, p);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? XS_OK : fail(XS_ERR_LAUNCH, "sequence kernel launch failed: %s", hipGetErrorString(e));
+}
+
+int run_train_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_st, int r_dtype) {
+  if (!a) return fail(XS_ERR_NULL, "args is NULL");
+  if (a->B < 0 || a->T < 0 || a->NH <= 0 || a->dh <= 0) return fail(XS_ERR_SHAPE, "bad dims B=%d T=%d NH=%d dh=%d", a->B, a->T, a->NH, a->dh);
+  if (a->dtype != XS_F32 && a->dtype != XS_BF16) return fail(XS_ERR_DTYPE, "dtype must be XS_F32 or XS_BF16");
+  const bool bf16 = a->dtype == XS_BF16;
+  if (r_dtype != XS_F32 && !(r_dtype == XS_BF16 && bf16)) return fail(XS_ERR_DTYPE, "r_dtype must be XS_F32, or XS_BF16 with dtype XS_BF16");
+  if (a->dh % 8 != 0 || !local_head(a->dh)) return fail(XS_ERR_UNSUPPORTED, "head dim %d: a multiple of 8 up to %d", a->dh, kLocalMaxHeadDim);
+  if (a->B == 0 || a->T == 0) return XS_OK;
+  int dwx_bf16 = 0;
+  const int rc = d_wx_type(a, &dwx_bf16);
+  if (rc != XS_OK) return rc;
+  if (!a->coef || !a->d_h || !a->r || !a->d_wx || !a->d_s0) return fail(XS_ERR_NULL, "coef, d_h, r, d_wx and d_s0 are required");
+  if ((uintptr_t)a->coef % 16) return fail(XS_ERR_ALIGN, "coef must be 16-byte aligned");
+  const long long H = (long long)a->NH * a->dh;
+  if (a->d_wx_stride_t < 4 * H || (a->B > 1 && a->d_wx_stride_b < 4 * H)) return fail(XS_ERR_SHAPE, "d_wx strides overlap the innermost 4*H elements");
+  if (a->reset && a->reset_stride_b < a->T) return fail(XS_ERR_SHAPE, "reset row stride %lld < T", (long long)a->reset_stride_b);
+  const long long grid = local_grid(a->B, a->NH);
+  if (grid > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many row tiles for one launch");
+  const int w = local_waves(a->dh);
+  LocalBwdParams p;
+  p.coef = a->coef; p.d_h = a->d_h; p.d_h_sb = d_h_sb; p.d_h_st = d_h_st; p.d_s_final = a->d_s_final;
+  p.r = a->r; p.r_bf16 = r_dtype == XS_BF16; p.reset = a->reset; p.reset_sb = a->reset_stride_b;
+  p.d_wx = a->d_wx; p.d_wx_sb = a->d_wx_stride_b; p.d_wx_st = a->d_wx_stride_t; p.d_s0 = a->d_s0;
+  p.cut = a->recurrent_cut != 0;
+  p.clip = (a->recurrent_clipval > 0.0f && a->recurrent_clipval < __builtin_inff()) ? a->recurrent_clipval : 0.0f;
+  p.B = a->B; p.T = a->T; p.NH = a->NH; p.dh = a->dh;
+  void (*k)(LocalBwdParams) = bf16 ? (dwx_bf16 ? pick_local_bwd<true, true>(w) : pick_local_bwd<true, false>(w)) : pick_local_bwd<false, false>(w);
+  hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(64 * w), 0, (hipStream_t)a->stream, p);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? XS_OK : fail(XS_ERR_LAUNCH, "backward kernel launch failed: %s", hipGetErrorString(e));
+}
+
 // need != nullptr: launch nothing, only report the bytes of workspace the launches of this call touch
 int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_host = nullptr) {
   hipStream_t stream = (hipStream_t)a->stream;
@@ -321,6 +420,9 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
                              (!a->reset || 4ll * a->reset_stride_b < 0xFFFFFF00ll) && 16ll * NH * dh * esz < (1ll << 31);
     if (MT == 4 && !offsets_fit) MT = 2;
   }
+  // small heads stay in one compute unit, the whole call in one launch (nothing waits, so nothing has to be resident
+  // at once), unless the batch is one for the kernel of four row tiles
+  if (head0 == 0 && MT < 4 && !a->coef_out && local_forward(dh, bf16)) return dry ? XS_OK : run_local(a, nullptr);
   int rows_per_wg = 16 * MT;
   if (MT == 1) {  // spare compute units: smaller row tiles, smaller exchanges
     for (int r = 4; r < 16; r *= 2)
@@ -413,17 +515,6 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
     if (e != hipSuccess) return fail(XS_ERR_LAUNCH, "sequence kernel launch failed: %s", hipGetErrorString(e));
   }
   }  // heads of one launch
-  return XS_OK;
-}
-
-// the type of d_wx that a backward call asks for
-int d_wx_type(const xs_slstm_bwd_args *a, int *is_bf16) {
-  *is_bf16 = 0;
-  if (a->d_wx_dtype == XS_F32) return XS_OK;
-  if (a->d_wx_dtype != XS_BF16 || a->dtype != XS_BF16) return fail(XS_ERR_DTYPE, "d_wx_dtype must be XS_F32, or XS_BF16 with dtype XS_BF16");
-  if (a->d_wx && (((uintptr_t)a->d_wx % 16) || (a->d_wx_stride_b % 8) || (a->d_wx_stride_t % 8)))
-    return fail(XS_ERR_ALIGN, "d_wx in bf16 must be 16-byte aligned and its strides multiples of 8 elements");
-  *is_bf16 = 1;
   return XS_OK;
 }
 
@@ -774,7 +865,7 @@ int run_backward_params(const xs_slstm_bwd_args *a) {
   if (!a) return fail(XS_ERR_NULL, "args is NULL");
   if (a->B < 0 || a->T < 0 || a->NH <= 0 || a->dh <= 0) return fail(XS_ERR_SHAPE, "bad dims B=%d T=%d NH=%d dh=%d", a->B, a->T, a->NH, a->dh);
   if (a->dtype != XS_F32 && a->dtype != XS_BF16) return fail(XS_ERR_DTYPE, "dtype must be XS_F32 or XS_BF16");
-  if (a->dh % 64 != 0) return fail(XS_ERR_UNSUPPORTED, "backward pass: head dim %d is not a multiple of 64", a->dh);
+  if (a->dh % 8 != 0) return fail(XS_ERR_UNSUPPORTED, "backward pass: head dim %d is not a multiple of 8", a->dh);
   if (!a->d_r || !a->d_bias) return fail(XS_ERR_NULL, "d_r and d_bias are required");
   const bool bf16 = a->dtype == XS_BF16;
   const long long H = (long long)a->NH * a->dh;
@@ -799,17 +890,17 @@ int run_backward_params(const xs_slstm_bwd_args *a) {
       return fail(XS_ERR_UNSUPPORTED, "32 steps of d_wx or of the outputs span 2 GiB or more: run the batch in slices of rows");
   }
   // (the slices of K are added into the results: they start at zero)
-  hipLaunchKernelGGL(fill_u32_kernel, dim3(256), dim3(256), 0, stream, (uint32_t *)a->d_r, nr, 0u);
-  hipLaunchKernelGGL(fill_u32_kernel, dim3(4), dim3(256), 0, stream, (uint32_t *)a->d_bias, nb, 0u);
+  hipLaunchKernelGGL(clear_two_kernel, dim3(256), dim3(256), 0, stream, (uint32_t *)a->d_r, nr, (uint32_t *)a->d_bias, nb);
   if (!empty) {
     BwdParamParams p;
     p.B = a->B; p.T = a->T; p.NH = a->NH; p.dh = a->dh;
+    p.dhp = (a->dh + 63) / 64 * 64;
     p.d_wx = (const float *)a->d_wx; p.d_wx_sb = a->d_wx_stride_b; p.d_wx_st = a->d_wx_stride_t; p.d_wx_bf16 = dwx_bf16;
     p.h_out = a->h_out; p.s0 = a->s0; p.reset = a->reset; p.reset_sb = a->reset_stride_b;
     p.d_r = a->d_r; p.d_bias = a->d_bias;
     p.tchunks = (a->T + kParamKC - 1) / kParamKC;
-    const int nt = a->dh % 256 == 0 ? 256 : (a->dh % 128 == 0 ? 128 : 64);
-    const int tiles = (4 * a->dh / kParamMT) * (a->dh / nt);
+    const int nt = p.dhp % 256 == 0 ? 256 : (p.dhp % 128 == 0 ? 128 : 64);
+    const int tiles = (4 * p.dhp / kParamMT) * (p.dhp / nt);
     const long long nchunks = (long long)a->B * p.tchunks;
     // slices of K: enough workgroups for two per compute unit, no slice shorter than four chunks
     const int cus = device_cus() > 0 ? device_cus() : 256;
@@ -1121,6 +1212,27 @@ int xs_slstm_forward_static(const xs_slstm_args *args) {
     return fail(XS_ERR_WORKSPACE, "this call needs %zu bytes of scratch, the static array holds %zu: use xs_slstm_forward with a workspace",
                 need, (size_t)XS_STATIC_SCRATCH_BYTES);
   return run_forward(&a);
+}
+
+size_t xs_slstm_train_coef_floats(int32_t B, int32_t T, int32_t NH, int32_t dh, int32_t dtype) {
+  if (B < 1 || T < 1 || NH < 1 || dh < 8 || dh % 8 != 0 || (dtype != XS_F32 && dtype != XS_BF16) || !local_head(dh)) return 0;
+  return (size_t)T * ((B + 3) / 4) * NH * local_waves(dh) * 576;
+}
+
+int xs_slstm_train_forward(const xs_slstm_args *args, float *coef) {
+  g_err[0] = 0;
+  const int rc = validate(args, false);
+  if (rc != XS_OK) return rc;
+  if (!coef || ((uintptr_t)coef % 16)) return fail(coef ? XS_ERR_ALIGN : XS_ERR_NULL, "coef is required, 16-byte aligned");
+  if (args->coef_out) return fail(XS_ERR_UNSUPPORTED, "coef_out goes with xs_slstm_forward");
+  if (!xs_slstm_train_coef_floats(args->B, args->T, args->NH, args->dh, args->wx_dtype))
+    return fail(XS_ERR_UNSUPPORTED, "a training forward of this kind: head dims that are multiples of 8 up to %d, at least one row and step", kLocalMaxHeadDim);
+  return run_local(args, coef);
+}
+
+int xs_slstm_train_backward(const xs_slstm_bwd_args *args, int64_t d_h_stride_b, int64_t d_h_stride_t, int32_t r_dtype) {
+  g_err[0] = 0;
+  return run_train_backward(args, d_h_stride_b, d_h_stride_t, r_dtype);
 }
 
 int xs_slstm_step(const xs_slstm_args *args) {

@@ -100,6 +100,79 @@ def backward_coefficients_buffer(wx: torch.Tensor, num_heads: int) -> Optional[t
     return torch.empty((T, (B + 3) // 4 * 4, 9, H), dtype=torch.float32, device=wx.device)
 
 
+def training_coefficients(wx: torch.Tensor, num_heads: int) -> Optional[torch.Tensor]:
+    """The tensor a training forward at a small head dim (a multiple of 8 up to 128; ``slstm_forward(..., train_coef=)``)
+    leaves the backward pass's coefficients in, or ``None`` for other calls.  Such a head stays in one compute unit,
+    forward and backward (``xs_slstm_train_forward``)."""
+    B, T = int(wx.shape[0]), int(wx.shape[1])
+    n = _lib.load().xs_slstm_train_coef_floats(B, T, num_heads, int(wx.shape[2]) // 4 // num_heads, _DTYPE_CODE.get(wx.dtype, -1))
+    return torch.empty(n, dtype=torch.float32, device=wx.device) if n else None
+
+
+def _small_head_backward(lib, wx, r, bias, s0, reset_mask, h_out, d_h, d_s_final, coef, timings, recurrent_cut, recurrent_clipval,
+                         d_wx_dtype):
+    """The backward pass of a head that stays in one compute unit: ``coef`` from the training forward, or None (the forward
+    runs once more and leaves them)."""
+    NH, dh = int(r.shape[0]), int(r.shape[2])
+    B, T, H, dev = int(wx.shape[0]), int(wx.shape[1]), NH * dh, wx.device
+    bf16 = wx.dtype == torch.bfloat16
+    if d_wx_dtype not in (None, torch.float32) and not (d_wx_dtype == torch.bfloat16 and bf16):
+        raise TypeError("d_wx_dtype: float32, or bfloat16 with bfloat16 inputs")
+    marks = []
+
+    def mark():
+        if timings is not None:
+            marks.append(torch.cuda.Event(enable_timing=True))
+            marks[-1].record()
+
+    with torch.cuda.device(dev):
+        mark()
+        if coef is None:
+            coef = training_coefficients(wx, NH)
+            slstm_forward(wx, r, bias, s0, reset_mask, train_coef=coef)
+        if r.dtype != torch.float32 and not (bf16 and r.dtype == torch.bfloat16):
+            r = r.float()
+        r = r.contiguous()
+        if s0 is not None:
+            s0 = s0.to(torch.float32).contiguous()
+        if reset_mask is not None:
+            reset_mask = _mask_u8(reset_mask, B, T)
+        h_c = h_out if h_out.is_contiguous() and h_out.dtype == wx.dtype else h_out.to(wx.dtype).contiguous()
+        if d_h.dtype != wx.dtype or d_h.stride(2) != 1:
+            d_h = d_h.to(wx.dtype).contiguous()
+        if d_s_final is not None:
+            d_s_final = d_s_final.to(torch.float32).contiguous()
+        d_wx = torch.empty((B, T, 4 * H), dtype=d_wx_dtype or torch.float32, device=dev)
+        d_s0 = torch.empty((4, B, H), dtype=torch.float32, device=dev)
+        d_r = torch.empty((NH, 4 * dh, dh), dtype=torch.float32, device=dev)
+        d_bias = torch.empty((NH, 4, dh), dtype=torch.float32, device=dev)
+        a = _lib.SlstmBwdArgs()
+        a.B, a.T, a.NH, a.dh = B, T, NH, dh
+        a.dtype = _DTYPE_CODE[wx.dtype]
+        a.coef, a.d_h, a.r, a.h_out = coef.data_ptr(), d_h.data_ptr(), r.data_ptr(), h_c.data_ptr()
+        a.d_s_final = d_s_final.data_ptr() if d_s_final is not None else None
+        a.s0 = s0.data_ptr() if s0 is not None else None
+        a.reset = reset_mask.data_ptr() if reset_mask is not None else None
+        a.reset_stride_b = reset_mask.stride(0) if reset_mask is not None else 0
+        a.d_wx, a.d_wx_stride_b, a.d_wx_stride_t = d_wx.data_ptr(), d_wx.stride(0), d_wx.stride(1)
+        a.d_wx_dtype = _DTYPE_CODE[d_wx.dtype]
+        a.d_s0, a.d_r, a.d_bias = d_s0.data_ptr(), d_r.data_ptr(), d_bias.data_ptr()
+        a.recurrent_cut = 1 if recurrent_cut else 0
+        a.recurrent_clipval = float(recurrent_clipval) if recurrent_clipval is not None else 0.0
+        a.stream = torch.cuda.current_stream(dev).cuda_stream
+        mark()
+        rc = lib.xs_slstm_train_backward(ctypes.byref(a), d_h.stride(1), d_h.stride(0), _DTYPE_CODE[r.dtype])
+        if rc == 0:
+            mark()
+            rc = lib.xs_slstm_backward_params(ctypes.byref(a))
+        if rc != 0:
+            raise EngineError(f"xlstm_amd error {rc}: {_lib.last_error()}")
+        mark()
+    if timings is not None:
+        timings["events"] = marks
+    return d_wx, d_r, d_bias, d_s0
+
+
 def slstm_backward(
     wx: torch.Tensor,
     r: torch.Tensor,
@@ -142,7 +215,9 @@ def slstm_backward(
     input gradient in the type of its kernels; the reverse kernel then writes and the parameter kernel reads half the bytes.
     ``abort_sink``: a callable that takes the call's abort word (an int32 tensor of one element on the device) instead
     of this function reading it, which synchronises the host; the cell queues an asynchronous copy and raises at a later call.
-    ``coef``: what a training forward left (``slstm_forward(..., coef_out=)``); the forward walk is then skipped.
+    ``coef``: what a training forward left (``slstm_forward(..., coef_out=)`` or ``train_coef=``); the forward walk is then skipped.
+    Head dims up to 128 run ``xs_slstm_train_backward`` (a head in one compute unit) unless a kernel is asked for by one
+    of the overrides or ``spin_limit``.
     ``recurrent_cut`` and ``recurrent_clipval`` are the reference's ``gradient_recurrent_cut`` (no gradient from a step
     to the y it started from, ``slstm_backward_cut.cu:265-312``) and ``gradient_recurrent_clipval`` (that gradient
     clipped to +-value before ``d_h`` is added, ``slstm_pointwise.cu:136-143``).
@@ -157,6 +232,13 @@ def slstm_backward(
     bf16 = wx.dtype == torch.bfloat16
     if tuple(h_out.shape) != (T, B, H) or tuple(d_h.shape) != (T, B, H):
         raise ValueError(f"h_out and d_h must be [S, B, H] = {(T, B, H)}")
+    if coef is not None and coef.dim() == 1 and coef.numel() != lib.xs_slstm_train_coef_floats(B, T, NH, dh, _DTYPE_CODE[wx.dtype]):
+        raise ValueError("coef must be the tensor that the forward call of the same inputs filled")
+    # a small head stays in one compute unit (no choice of kernels, nothing waits): unless a kernel is asked for by name
+    if ((coef is None or coef.dim() == 1) and split_override is None and row_tile_override is None and not stepwise_override
+            and spin_limit == 0 and lib.xs_slstm_train_coef_floats(B, T, NH, dh, _DTYPE_CODE[wx.dtype])):
+        return _small_head_backward(lib, wx, r, bias, s0, reset_mask, h_out, d_h, d_s_final, coef, timings, recurrent_cut,
+                                    recurrent_clipval, d_wx_dtype)
     dh_k = backward_kernel_head_dim(dh, wx.dtype)
     if coef is not None and (dh_k != dh or not bf16 or tuple(coef.shape) != (T, (B + 3) // 4 * 4, 9, H)
                              or coef.dtype != torch.float32 or not coef.is_contiguous()):
@@ -371,12 +453,14 @@ def slstm_forward(
     spin_limit: int = 0,
     h_prev: Optional[torch.Tensor] = None,
     coef_out: Optional[torch.Tensor] = None,
+    train_coef: Optional[torch.Tensor] = None,
 ) -> Tuple[torch.Tensor, torch.Tensor]:
     """Runs the cell over ``wx`` and returns ``(h[S,B,H] in wx.dtype, state[4,B,H] float32)``.
 
     ``coef_out`` (a training forward; a float32 tensor from ``backward_coefficients_buffer``): the kernel also leaves
     the coefficients of the backward pass there, and ``slstm_backward(..., coef=coef_out)`` skips its own forward walk.
     Raises ``CoefficientsUnsupported`` (nothing has run) for calls that cannot: see ``backward_coefficients_buffer``.
+    ``train_coef`` (from ``training_coefficients``): the same for small head dims, whose kernels have a layout of their own.
 
     ``reset_mask[B,S]`` (bool/uint8) marks document starts: the row's state is
     zeroed before that step.  ``step=True`` uses the decode entry point (S == 1).
@@ -467,7 +551,10 @@ def slstm_forward(
             raise ValueError("coef_out must be the tensor backward_coefficients_buffer returns for this call")
         a.coef_out = coef_out.data_ptr()
     with torch.cuda.device(dev):
-        rc = (lib.xs_slstm_step if step else lib.xs_slstm_forward)(ctypes.byref(a))
+        if train_coef is not None:
+            rc = lib.xs_slstm_train_forward(ctypes.byref(a), train_coef.data_ptr())
+        else:
+            rc = (lib.xs_slstm_step if step else lib.xs_slstm_forward)(ctypes.byref(a))
     if rc != 0:
         if coef_out is not None and rc == _lib.XS_ERR_UNSUPPORTED:
             raise CoefficientsUnsupported(f"xlstm_amd error {rc}: {_lib.last_error()}")
