@@ -104,6 +104,16 @@ __device__ __forceinline__ void slstm_pointwise_keep(float iraw, float fraw, flo
   s.c = cnew; s.n = nnew; s.m = mnew;
 }
 
+// 4 x 4 transpose between four registers and the four groups of 16 lanes: in: register r of lane group g; out: register
+// g' of lane group r' = what register r' of lane group g' held
+__device__ __forceinline__ void transpose_lane_groups(float &x0, float &x1, float &x2, float &x3) {
+  auto s02 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x0), __float_as_uint(x2), false, false);
+  auto s13 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x1), __float_as_uint(x3), false, false);
+  auto lo = __builtin_amdgcn_permlane16_swap(s02[0], s13[0], false, false);
+  auto hi = __builtin_amdgcn_permlane16_swap(s02[1], s13[1], false, false);
+  x0 = __uint_as_float(lo[0]); x1 = __uint_as_float(lo[1]); x2 = __uint_as_float(hi[0]); x3 = __uint_as_float(hi[1]);
+}
+
 // ---------------------------------------------------------------------------
 // fill kernels (plain vector stores; also used instead of memset so that a
 // caller may capture the call in a graph)

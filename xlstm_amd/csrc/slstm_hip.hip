@@ -85,6 +85,17 @@ SeqKernel pick_mt(int MT, bool burst) {
   }
 }
 
+// (chunk counts below those here have head dims that stay in one compute unit: slstm_local_kernel.h)
+template <bool BF16, bool FULL>
+SeqKernel pick_quad(int nch) {
+  if (nch == 2) return slstm_seq_kernel<BF16, 2, 1, FULL, false, false, true>;
+  if (nch == 4) return slstm_seq_kernel<BF16, 4, 1, FULL, false, false, true>;
+  if constexpr (!BF16) {
+    if (nch == 8) return slstm_seq_kernel<BF16, 8, 1, FULL, false, false, true>;
+  }
+  return nullptr;
+}
+
 template <bool BF16, bool FULL>
 SeqKernel pick_roles_kernel(int nch) {
   switch (nch) {
@@ -99,7 +110,6 @@ SeqKernel pick_roles_kernel(int nch) {
 template <bool BF16, bool FULL>
 SeqKernel pick_kernel(int nch, int MT, bool burst) {
   switch (nch) {
-    case 1: return pick_mt<BF16, 1, FULL>(MT, burst);
     case 2: return pick_mt<BF16, 2, FULL>(MT, burst);
     case 4: return pick_mt<BF16, 4, FULL>(MT, burst);
     case 8: return pick_mt<BF16, 8, FULL>(MT, burst);
@@ -446,14 +456,11 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
     else
       kern = bf16 ? (full ? pick_kernel<true, true>(nch, MT, burst) : pick_kernel<true, false>(nch, MT, burst))
                   : (full ? pick_kernel<false, true>(nch, MT, burst) : pick_kernel<false, false>(nch, MT, burst));
-    // row tiles of at most 4 rows, bf16, whole K ranges up to 512: the compute waves split the columns by unit, not K
-    const bool quad = bf16 && MT == 1 && rows_per_wg == 4 && full && nch <= 4 && G <= 32;
-    if (quad) {
-      kern = nch == 1 ? slstm_seq_kernel<true, 1, 1, true, false, false, true>
-                      : (nch == 2 ? slstm_seq_kernel<true, 2, 1, true, false, false, true> : slstm_seq_kernel<true, 4, 1, true, false, false, true>);
-    }
+    // row tiles of at most 4 rows: the compute waves split the columns by unit, not K (head groups on one XCD)
+    const bool quad = MT == 1 && rows_per_wg == 4 && G <= 32;
+    if (quad) kern = bf16 ? (full ? pick_quad<true, true>(nch) : pick_quad<true, false>(nch)) : (full ? pick_quad<false, true>(nch) : pick_quad<false, false>(nch));
     if (a->coef_out) {  // a training forward: the same kernel, leaving the backward pass its coefficients
-      if (!quad || (dh != 128 && dh != 256) || rows_per_launch < B)
+      if (!quad || !bf16 || (dh != 128 && dh != 256) || rows_per_launch < B)
         return fail(XS_ERR_UNSUPPORTED, "coef_out: the call does not run in row tiles of 4 rows of one kernel (bf16, head dim 128 or 256, "
                                         "ceil(B/4) * NH * dh/16 workgroups on the device at once)");
       if (((uintptr_t)a->coef_out % 4)) return fail(XS_ERR_ALIGN, "coef_out must be 4-byte aligned");

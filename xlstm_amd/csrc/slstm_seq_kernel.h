@@ -156,15 +156,16 @@ __device__ __forceinline__ uint32_t seq_handshake(const SeqParams &p, int wg, in
 // 4 (fp32) inputs of every real row - fetched from the lane that holds them - into its own column's weights, and
 // the four lane groups' partial sums over K are added with two cross-lane steps.  The sums are formed in a different
 // order than the MFMA forms them, so the bits differ from the MFMA path (and from the decode kernel).
-// QUAD: row tiles of at most 4 rows (bf16, FULL, one row tile): the four compute waves split the workgroup's 64
-// columns by UNIT instead of splitting K, see "waves 0-3, QUAD" below.
+// QUAD: row tiles of at most 4 rows: the four compute waves split the workgroup's 64 columns by UNIT instead of splitting
+// K, see "waves 0-3, QUAD" below.
 // COEF (with QUAD): a training forward: the compute waves also leave the nine coefficients per step and element that the
 // backward pass would otherwise recompute in a forward walk of its own (slstm_bwd_prepare_kernel), see "COEF" below.
 template <bool BF16, int NCH, int MT, bool FULL, bool BURST, bool FMAC = false, bool QUAD = false, bool COEF = false>
 __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm_seq_kernel(SeqParams p) {
   static_assert(!COEF || QUAD, "coefficients for the backward pass come from the unit-split compute waves only");
   static_assert(!FMAC || MT == 1, "the FMA contraction is for one row tile of at most 4 rows");
-  static_assert(!QUAD || (BF16 && MT == 1 && FULL && !BURST && !FMAC), "the unit-split compute waves exist for bf16, one full row tile");
+  static_assert(!QUAD || (MT == 1 && !BURST && !FMAC), "the unit-split compute waves exist for one row tile of at most 4 rows");
+  static_assert(!COEF || (BF16 && FULL), "coefficients for the backward pass: bf16, head dims that fill the K range");
   constexpr int EPC = BF16 ? 8 : 4;      // elements per 16-byte chunk
   constexpr int KW = NCH * 4 * EPC;      // input units per wave
   constexpr int ESZ = BF16 ? 2 : 4;
@@ -453,25 +454,46 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
   // the four gates of a unit meet in the unit's lane through three row shifts (no LDS).  K is accumulated in the same
   // four quarters and folded in the same order as everywhere else: the same bits.  The barrier of the step (the
   // feeder's W.x, the drainer's h) is passed in front of the poll.  The exchange ring is [slot][member][4 rows]
-  // [16 units]: the group's h of a step is 8 dh bytes in a row.
+  // [16 units]: the group's h of a step is 8 dh bytes (float32: 16 dh) in a row.
+  // Without FULL the K range ends inside the four quarters: members past the last one lie past the end of the descriptor
+  // and read zeros, and units past the head dim publish zeros (they are polled like the others).
+  // float32 multiplies with v_mfma_f32_4x4x1, whose 16 blocks are 4 groups of columns x 4 quarters of K: a tile of 4 rows
+  // without padding takes a quarter of the cycles of v_mfma_f32_16x16x4 (head dim 128: 256 instead of 1,024 per wave and
+  // step), the operand is broadcast inside a quarter by the instruction, so that a lane polls only its own 16 bytes per 16
+  // inputs of a quarter, and the quarters meet in a 4 x 4 transpose across the lane groups.  B 4 x T 256 x 4 heads of 128: 311 us
+  // with K split over the waves, XS_F32_QUAD_US with this.
   // =========================================================================
   if constexpr (QUAD) {
     __builtin_amdgcn_s_setprio(3);
     constexpr int NK = 4 * NCH;                // MFMA k-steps over the head dim (dh = 32 NK)
     const int q = lane >> 4, r16 = lane & 15;
-    uint4 rreg[NK];
+    uint4 rreg[BF16 ? NK : 1];                 // bf16: the B operands of the k-steps
+    float rf[BF16 ? 1 : KW];                   // float32: the column's inputs of quarter q of K
     {
       const int a = a0 + 4 * wave + (r16 & 3);
-      const long long rowoff = ((long long)head * 4 * dh + (long long)(r16 >> 2) * dh + a) * dh;
+      const bool a_ok = FULL || a < dh;
+      const long long rowoff = ((long long)head * 4 * dh + (long long)(r16 >> 2) * dh + (a_ok ? a : 0)) * dh;
+      if constexpr (BF16) {
 #pragma unroll
-      for (int ks = 0; ks < NK; ++ks) {
-        const long long off = rowoff + ks * 32 + q * 8;
-        if (p.r_bf16) {
-          rreg[ks] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(p.r) + off);
-        } else {
-          const float4 lo = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(p.r) + off);
-          const float4 hi = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(p.r) + off + 4);
-          rreg[ks] = uint4{pack_bf16x2(lo.x, lo.y), pack_bf16x2(lo.z, lo.w), pack_bf16x2(hi.x, hi.y), pack_bf16x2(hi.z, hi.w)};
+        for (int ks = 0; ks < NK; ++ks) {
+          const int k = ks * 32 + q * 8;
+          if (!FULL && (!a_ok || k >= dh)) {
+            rreg[ks] = make_uint4(0, 0, 0, 0);
+          } else if (p.r_bf16) {
+            rreg[ks] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(p.r) + rowoff + k);
+          } else {
+            const float4 lo = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(p.r) + rowoff + k);
+            const float4 hi = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(p.r) + rowoff + k + 4);
+            rreg[ks] = uint4{pack_bf16x2(lo.x, lo.y), pack_bf16x2(lo.z, lo.w), pack_bf16x2(hi.x, hi.y), pack_bf16x2(hi.z, hi.w)};
+          }
+        }
+      } else {
+#pragma unroll
+        for (int k4 = 0; k4 < KW / 4; ++k4) {
+          const int k = q * KW + 4 * k4;
+          float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+          if (FULL || (a_ok && k < dh)) v = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(p.r) + rowoff + k);
+          rf[4 * k4] = v.x; rf[4 * k4 + 1] = v.y; rf[4 * k4 + 2] = v.z; rf[4 * k4 + 3] = v.w;
         }
       }
     }
@@ -479,12 +501,13 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
     const int gb = q, gu = 4 * wave + (r16 & 3);
     const bool gate_lane = r16 < 4;
     const int ua = a0 + gu, col = head * dh + ua;
+    const bool u_ok = FULL || ua < dh;
     const int brow = rowbase + gb;
     float bias_g[4];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) bias_g[g] = p.bias[((long long)head * 4 + g) * dh + ua];
+    for (int g = 0; g < 4; ++g) bias_g[g] = u_ok ? p.bias[((long long)head * 4 + g) * dh + ua] : 0.0f;
     CellState st{0.0f, 0.0f, 0.0f, 0.0f};
-    if (p.s0 && brow < rend) {
+    if (p.s0 && brow < rend && u_ok) {
       const long long o = (long long)brow * H + col;
       st.y = p.s0[o]; st.c = p.s0[BH + o]; st.n = p.s0[2 * BH + o]; st.m = p.s0[3 * BH + o];
     }
@@ -519,24 +542,30 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
 #endif
     lds_barrier();  // prologue barrier
     const bool cross = cross_s != 0u;
-    constexpr int QTILE = 4 * 16 * 2;          // bytes a member publishes per step
+    constexpr int QTILE = 4 * 16 * ESZ;        // bytes a member publishes per step
+    constexpr int NP = BF16 ? NK : NCH;        // 16-byte pieces of the group's h a lane polls per step
+    constexpr int PSTEP = BF16 ? 2 * QTILE : QTILE;  // ... and the distance between them
     const int xslot = p.G * QTILE;
     char *const xbase = reinterpret_cast<char *>(p.xbuf) + (long long)gi * kRing * xslot;
     // operand: MFMA row r16 is batch row r16 / 4 when r16 % 4 == 0, nothing otherwise; k-step ks, lane group q: units
     // 32 ks + 8 q .. + 7 = member 2 ks + q / 2, its units 8 (q % 2) .. + 7
-    const int arow = rowbase + (r16 >> 2);
-    const bool a_lane = (r16 & 3) == 0 && arow < rend;
-    const int xl = a_lane ? (q >> 1) * QTILE + (r16 >> 2) * 32 + (q & 1) * 16 : 0x7FFFFF00;
-    const long long xo = (long long)member * (QTILE / 2) + gb * 16 + gu;
+    // float32: lane (quarter q, piece r16 / 4, row r16 % 4), chunk c of the quarter: member q NCH + c, its units 4 (r16 / 4) .. + 3
+    const int orow = BF16 ? r16 >> 2 : r16 & 3;   // the batch row of the tile in this lane's operand
+    const int arow = rowbase + orow;
+    const bool a_lane = (!BF16 || (r16 & 3) == 0) && arow < rend;
+    const int xl = !a_lane ? 0x7FFFFF00 : (BF16 ? (q >> 1) * QTILE + orow * 32 + (q & 1) * 16 : q * NCH * QTILE + orow * 64 + (r16 >> 2) * 16);
+    const long long xo = (long long)member * (QTILE / ESZ) + gb * 16 + gu;
+    typedef typename std::conditional<BF16, uint16_t, uint32_t>::type word_t;
+    constexpr word_t kMissing = BF16 ? (word_t)kSentinel16 : (word_t)kSentinel32;
 #ifndef XS_QUAD_PAD
 #define XS_QUAD_PAD 4
 #endif
     asm volatile(".p2align 5\n\t.rept %0\n\ts_nop 0\n\t.endr" :: "n"(XS_QUAD_PAD));
     for (int t = 0; t < p.T; ++t) {
       const __amdgpu_buffer_rsrc_t hrs = __builtin_amdgcn_make_buffer_rsrc(xbase + ((t + kRing - 1) % kRing) * xslot, 0, xslot, 0x00020000);
-      uint16_t *const hcur = reinterpret_cast<uint16_t *>(xbase + (t % kRing) * xslot);
-      uint16_t *const hold = reinterpret_cast<uint16_t *>(xbase + ((t + kRing - 2) % kRing) * xslot);
-      uint4 areg[NK];
+      word_t *const hcur = reinterpret_cast<word_t *>(xbase + (t % kRing) * xslot);
+      word_t *const hold = reinterpret_cast<word_t *>(xbase + ((t + kRing - 2) % kRing) * xslot);
+      uint4 areg[NP];
       // The step's barrier and what the gating needs from LDS come FIRST, then one s_sleep, then the poll: whatever
       // stands between the poll's return and the MFMAs is on the chain.  Measured at B 16 x T 2048 x 4 heads of 256 (ms
       // per call): barrier and LDS reads under the poll 1.81, in front of it 1.63, with the s_sleep 1.52 (two of
@@ -553,7 +582,7 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
       XS_QTICK(2);
 #pragma unroll
       for (int g = 0; g < 4; ++g) wxv[g] = wxs[buf][g][gb * kTileStride + gu];
-      const bool row_reset = rfl[t & 3][r16 >> 2] != 0u;   // (the operand's row: it contributes R.0 = 0 exactly)
+      const bool row_reset = rfl[t & 3][orow] != 0u;       // (the operand's row: it contributes R.0 = 0 exactly)
       const bool gate_reset = rfl[t & 3][gb] != 0u;
 #ifndef XS_QUAD_SLEEP
 #define XS_QUAD_SLEEP 1
@@ -566,18 +595,23 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
       XS_QTICK(1);
       if (t > 0) {
 #pragma unroll
-        for (int ks = 0; ks < NK; ++ks)
-          areg[ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(hrs, xl, ks * 2 * QTILE, 16));
+        for (int ks = 0; ks < NP; ++ks)
+          areg[ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(hrs, xl, ks * PSTEP, 16));
         stage_coefficients(t - 1);  // (COEF; while the poll is on its way)
       } else {
 #pragma unroll
-        for (int ks = 0; ks < NK; ++ks) {
+        for (int ks = 0; ks < NP; ++ks) {
           areg[ks] = make_uint4(0, 0, 0, 0);
-          if (a_lane && p.s0) {
-            const float *src = p.s0 + (long long)arow * H + head * dh + ks * 32 + q * 8;
+          const int k = BF16 ? ks * 32 + q * 8 : q * KW + ks * 16 + (r16 >> 2) * 4;
+          if (a_lane && p.s0 && (FULL || k < dh)) {
+            const float *src = p.s0 + (long long)arow * H + head * dh + k;
             const float4 lo = *reinterpret_cast<const float4 *>(src);
-            const float4 hi = *reinterpret_cast<const float4 *>(src + 4);
-            areg[ks] = uint4{pack_bf16x2(lo.x, lo.y), pack_bf16x2(lo.z, lo.w), pack_bf16x2(hi.x, hi.y), pack_bf16x2(hi.z, hi.w)};
+            if constexpr (BF16) {
+              const float4 hi = *reinterpret_cast<const float4 *>(src + 4);
+              areg[ks] = uint4{pack_bf16x2(lo.x, lo.y), pack_bf16x2(lo.z, lo.w), pack_bf16x2(hi.x, hi.y), pack_bf16x2(hi.z, hi.w)};
+            } else {
+              areg[ks] = __builtin_bit_cast(uint4, lo);
+            }
           }
         }
       }
@@ -586,11 +620,11 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
         for (;;) {
           uint32_t ma = 0u;
 #pragma unroll
-          for (int ks = 0; ks < NK; ++ks) ma = mark_join<true>(ma, chunk_mark<true>(areg[ks]));
-          if (__builtin_amdgcn_ballot_w64(mark_has_sentinel<true>(ma)) == 0ull) break;
+          for (int ks = 0; ks < NP; ++ks) ma = mark_join<BF16>(ma, chunk_mark<BF16>(areg[ks]));
+          if (__builtin_amdgcn_ballot_w64(mark_has_sentinel<BF16>(ma)) == 0ull) break;
 #pragma unroll
-          for (int ks = 0; ks < NK; ++ks)
-            areg[ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(hrs, xl, ks * 2 * QTILE, 16));
+          for (int ks = 0; ks < NP; ++ks)
+            areg[ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(hrs, xl, ks * PSTEP, 16));
           spins += 1;
           if ((spins & 1023u) == 0u && __hip_atomic_load(&p.status->aborted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
             aborted = true;
@@ -613,23 +647,44 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
       XS_QTICK(0);
       if (__builtin_amdgcn_ballot_w64(row_reset) != 0ull) {
 #pragma unroll
-        for (int ks = 0; ks < NK; ++ks)
+        for (int ks = 0; ks < NP; ++ks)
           if (row_reset) areg[ks] = make_uint4(0, 0, 0, 0);
       }
-      // the four quarters of K, each its own chain from zero, folded in the order of the other kernels' waves
-      f32x4 acc[4];
+      float mine;
+      if constexpr (BF16) {
+        // the four quarters of K, each its own chain from zero, folded in the order of the other kernels' waves
+        f32x4 acc[4];
 #pragma unroll
-      for (int w4 = 0; w4 < 4; ++w4) acc[w4] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int w4 = 0; w4 < 4; ++w4) acc[w4] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int c = 0; c < NCH; ++c)
+        for (int c = 0; c < NCH; ++c)
 #pragma unroll
-        for (int w4 = 0; w4 < 4; ++w4)
-          acc[w4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, areg[w4 * NCH + c]),
-                                                            __builtin_bit_cast(bf16x8, rreg[w4 * NCH + c]), acc[w4], 0, 0, 0);
-      float mine = acc[0][0];
-      mine += acc[1][0];
-      mine += acc[2][0];
-      mine += acc[3][0];
+          for (int w4 = 0; w4 < 4; ++w4)
+            acc[w4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, areg[w4 * NCH + c]),
+                                                              __builtin_bit_cast(bf16x8, rreg[w4 * NCH + c]), acc[w4], 0, 0, 0);
+        mine = acc[0][0];
+        mine += acc[1][0];
+        mine += acc[2][0];
+        mine += acc[3][0];
+      } else {
+        // element e of the four 16-byte pieces of a chunk, in the order v_mfma_f32_16x16x4 takes them in the other kernels:
+        // lane group q accumulates quarter q of K for the four rows, then the quarters of a row meet in its lane group
+        f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+          const float hv[4] = {__uint_as_float(areg[c].x), __uint_as_float(areg[c].y), __uint_as_float(areg[c].z), __uint_as_float(areg[c].w)};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            acc = __builtin_amdgcn_mfma_f32_4x4x1f32(hv[e], rf[16 * c + e], acc, 2, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_4x4x1f32(hv[e], rf[16 * c + 4 + e], acc, 2, 1, 0);
+            acc = __builtin_amdgcn_mfma_f32_4x4x1f32(hv[e], rf[16 * c + 8 + e], acc, 2, 2, 0);
+            acc = __builtin_amdgcn_mfma_f32_4x4x1f32(hv[e], rf[16 * c + 12 + e], acc, 2, 3, 0);
+          }
+        }
+        float x0 = acc[0], x1 = acc[1], x2 = acc[2], x3 = acc[3];
+        transpose_lane_groups(x0, x1, x2, x3);
+        mine = ((x0 + x1) + x2) + x3;
+      }
       // lane (row, gate g, unit u) -> the unit's lane (row, 0, u): lanes 4, 8, 12 further on in the row of 16
       const int mi = __float_as_int(mine);
       const float ry1 = __int_as_float(__builtin_amdgcn_update_dpp(0, mi, 0x104, 0xF, 0xF, true));  // row_shl:4
@@ -655,18 +710,21 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
 #endif
       XS_QTICK(3);
       if (gate_lane) {
-        const uint16_t v = (uint16_t)float_to_bf16_bits(y);
+        word_t v;
+        if constexpr (BF16) v = (word_t)float_to_bf16_bits(y);
+        else v = __float_as_uint(y) == kSentinel32 ? 0x7FC00000u : __float_as_uint(y);
+        if (!u_ok) v = 0;
         if (cross) {
           __hip_atomic_store(hcur + xo, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          __hip_atomic_store(hold + xo, (uint16_t)kSentinel16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(hold + xo, kMissing, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
           hcur[xo] = v;
-          hold[xo] = (uint16_t)kSentinel16;
+          hold[xo] = kMissing;
         }
         hst[t & 3][gb * 16 + gu] = y;
       }
 #pragma unroll
-      for (int ks = 0; ks < NK; ++ks)  // (the operand registers stay reserved to the end of the iteration)
+      for (int ks = 0; ks < NP; ++ks)  // (the operand registers stay reserved to the end of the iteration)
         asm volatile("" :: "v"(areg[ks].x), "v"(areg[ks].y), "v"(areg[ks].z), "v"(areg[ks].w));
       XS_QTICK(4);
     }
@@ -683,7 +741,7 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
 #endif
     const bool poisoned = __hip_atomic_load(&p.status->aborted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
     if (poisoned) report_abort(p.abort_host);
-    if (gate_lane && brow < rend) {
+    if (gate_lane && brow < rend && u_ok) {
       const long long o = (long long)brow * H + col;
       if (poisoned) st = CellState{kPoison, kPoison, kPoison, kPoison};
       p.s_out[o] = st.y; p.s_out[BH + o] = st.c; p.s_out[2 * BH + o] = st.n; p.s_out[3 * BH + o] = st.m;
