@@ -382,20 +382,24 @@ int xs_slstm_backward_prepare(const xs_slstm_bwd_args *args);
 int xs_slstm_backward(const xs_slstm_bwd_args *args);
 
 /*
- * Training at small head dims (multiples of 8 up to 128): a head stays in one compute unit, forward and backward, nothing
- * waits for another compute unit and nothing can give up.
- *   xs_slstm_train_coef_floats  floats of the coefficients such a training forward leaves, 0 where the pair below does
- *                               not cover the call.
- *   xs_slstm_train_forward      xs_slstm_forward (same bits) that also leaves the coefficients of the backward pass in
- *                               `coef`, in an order of its own (slstm_local_kernel.h); coef_out must be NULL.
- *   xs_slstm_train_backward     the reverse pass from them: reads B, T, NH, dh, dtype, coef, d_h (with its strides in
- *                               elements, innermost H contiguous: the gradient as the layer behind the cell holds it
- *                               needs no copy), d_s_final, r (the forward's layout and, with r_dtype XS_F32, its float32
- *                               master), reset, recurrent_cut, recurrent_clipval; writes d_wx (d_wx_dtype) and d_s0.
+ * Training, every head dim of the forward (multiples of 8, up to 1024 with bf16 and 512 with f32): a forward that leaves the
+ * coefficients of the backward pass and a reverse pass of one launch (per slice of rows) that reads them.
+ *   xs_slstm_train_coef_floats    floats of those coefficients, 0 where the pair below does not cover the call.
+ *   xs_slstm_train_forward        xs_slstm_forward (same bits) that also leaves the coefficients in `coef`, in an order of
+ *                                 its own: [T][ceil(B/4)][NH][ceil(dh/16)][576]; coef_out must be NULL.
+ *   xs_slstm_train_exchange_bytes bytes of xs_slstm_bwd_args::exchange that the reverse pass needs (0: none, a head
+ *                                 stays in one compute unit; nothing waits and nothing can give up there); counters then
+ *                                 holds 1 + (compute units of the device) words, of which the first is as for split != 0.
+ *   xs_slstm_train_backward       the reverse pass: reads B, T, NH, dh, dtype, coef, d_h (with its strides in elements,
+ *                                 innermost H contiguous: the gradient as the layer behind the cell holds it needs no
+ *                                 copy; where exchange is needed, 16-byte aligned), d_s_final, r (the forward's layout and,
+ *                                 with r_dtype XS_F32, its float32 master), reset, recurrent_cut, recurrent_clipval,
+ *                                 exchange, counters, spin_limit; writes d_wx (d_wx_dtype) and d_s0.
  * The gradients of r and the bias: xs_slstm_backward_params, as for the other kernels.
  * Like coef_out, this takes the place of the state history and gate cache of the reference (slstm.cc:79-108).
  */
 size_t xs_slstm_train_coef_floats(int32_t B, int32_t T, int32_t NH, int32_t dh, int32_t dtype);
+size_t xs_slstm_train_exchange_bytes(int32_t B, int32_t NH, int32_t dh, int32_t dtype);
 int xs_slstm_train_forward(const xs_slstm_args *args, float *coef);
 int xs_slstm_train_backward(const xs_slstm_bwd_args *args, int64_t d_h_stride_b, int64_t d_h_stride_t, int32_t r_dtype);
 

@@ -37,6 +37,7 @@ EXPORTS = (
     "xs_headwise_group_norm",
     "xs_measure_stage",
     "xs_slstm_train_coef_floats",
+    "xs_slstm_train_exchange_bytes",
     "xs_slstm_train_forward",
     "xs_slstm_train_backward",
 )
@@ -220,6 +221,8 @@ def load() -> ctypes.CDLL:
     lib.xs_headwise_group_norm.argtypes = [ctypes.POINTER(NormArgs)]
     lib.xs_slstm_train_coef_floats.restype = ctypes.c_size_t
     lib.xs_slstm_train_coef_floats.argtypes = [ctypes.c_int32] * 5
+    lib.xs_slstm_train_exchange_bytes.restype = ctypes.c_size_t
+    lib.xs_slstm_train_exchange_bytes.argtypes = [ctypes.c_int32] * 4
     lib.xs_slstm_train_forward.restype = ctypes.c_int
     lib.xs_slstm_train_forward.argtypes = [ctypes.POINTER(SlstmArgs), ctypes.c_void_p]
     lib.xs_slstm_train_backward.restype = ctypes.c_int

@@ -513,11 +513,12 @@ class sLSTMCell_hip(nn.Module):
         args = (x, r, self._bias_.detach().view(self.config.num_heads, 4, self.head_dim), state, reset_mask)
         coef = h = s = None
         if wants_grad and self.keep_backward_coefficients and x.is_cuda and not step:
-            coef = F_hip.training_coefficients(x, self.config.num_heads)
-            if coef is not None:
-                h, s = F_hip.slstm_forward(*args, s_out=state_out, workspace=ws, train_coef=coef)
-            else:
+            if self.head_dim == 256:  # (bfloat16: row tiles of 4 rows x 64 units in the backward, where they fit)
                 coef = F_hip.backward_coefficients_buffer(x, self.config.num_heads)
+            if coef is None:
+                coef = F_hip.training_coefficients(x, self.config.num_heads)
+                if coef is not None:
+                    h, s = F_hip.slstm_forward(*args, s_out=state_out, workspace=ws, train_coef=coef)
         if coef is not None and h is None:
             try:
                 h, s = F_hip.slstm_forward(*args, s_out=state_out, workspace=ws, coef_out=coef)

@@ -104,6 +104,14 @@ __device__ __forceinline__ void slstm_pointwise_keep(float iraw, float fraw, flo
   s.c = cnew; s.n = nnew; s.m = mnew;
 }
 
+// The nine coefficients of the backward pass of one step and element (see slstm_bwd_prepare_kernel) into the 576 floats of
+// its 64 elements: coefficients 0-3 and 4-7 as 16 bytes per element, then coefficient 8
+__device__ __forceinline__ void store_coefficients(float *dst, int e, const GateValues &k, float y, float c, float n, float omf) {
+  *reinterpret_cast<f32x4 *>(dst + 4 * e) = f32x4{k.og * k.rn, y * k.rn, k.ig * k.tz, k.ig};
+  *reinterpret_cast<f32x4 *>(dst + 256 + 4 * e) = f32x4{k.fg * omf * c, k.fg * omf * n, k.ig * (1.0f - k.tz * k.tz), (1.0f - k.og) * y};
+  dst[512 + e] = k.fg;
+}
+
 // 4 x 4 transpose between four registers and the four groups of 16 lanes: in: register r of lane group g; out: register
 // g' of lane group r' = what register r' of lane group g' held
 __device__ __forceinline__ void transpose_lane_groups(float &x0, float &x1, float &x2, float &x3) {

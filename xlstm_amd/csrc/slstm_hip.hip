@@ -35,6 +35,7 @@
 #include "slstm_backward_kernels.h"
 #include "slstm_layer_kernels.h"
 #include "slstm_local_kernel.h"
+#include "slstm_backward_unit_kernel.h"
 #include "slstm_backward_quad_kernel.h"
 #include "slstm_backward_step_kernel.h"
 #include "slstm_step_feed_kernel.h"
@@ -94,6 +95,22 @@ SeqKernel pick_quad(int nch) {
     if (nch == 8) return slstm_seq_kernel<BF16, 8, 1, FULL, false, false, true>;
   }
   return nullptr;
+}
+
+// the kernels of a training forward beyond the head dims that stay in one compute unit
+template <bool BF16, int NCH, bool FULL>
+SeqKernel pick_train_n(bool quad, bool burst) {
+  if (quad) return slstm_seq_kernel<BF16, NCH, 1, FULL, false, false, NCH <= (BF16 ? 4 : 8), 2>;
+  return (burst && NCH <= 4) ? slstm_seq_kernel<BF16, NCH, 1, FULL, NCH <= 4, false, false, 2> : slstm_seq_kernel<BF16, NCH, 1, FULL, false, false, false, 2>;
+}
+template <bool BF16, bool FULL>
+SeqKernel pick_train(int nch, bool quad, bool burst) {
+  switch (nch) {
+    case 2: return pick_train_n<BF16, 2, FULL>(quad, burst);
+    case 4: return pick_train_n<BF16, 4, FULL>(quad, burst);
+    case 8: return pick_train_n<BF16, 8, FULL>(quad, burst);
+    default: return nullptr;
+  }
 }
 
 template <bool BF16, bool FULL>
@@ -281,36 +298,44 @@ int d_wx_type(const xs_slstm_bwd_args *a, int *is_bf16) {
 }
 
 // ---- small heads: the kernels that keep a head in one compute unit (slstm_local_kernel.h)
-inline bool local_head(int dh) { return dh <= kLocalMaxHeadDim; }
-// ... and where the forward alone is faster that way: float32 beyond head dim 64 has 1,024 cycles of MFMA per wave and step
-// in one compute unit (1.56 us a step at head dim 128, against 1.24 for slstm_seq_kernel over eight)
-inline bool local_forward(int dh, bool bf16) { return dh <= (bf16 ? kLocalMaxHeadDim : 64); }
+// (float32 beyond head dim 64 multiplies faster over several: 0.79 against 1.57 us a step at head dim 128)
+inline bool local_head(int dh, bool bf16) { return dh <= (bf16 ? kLocalMaxHeadDim : 64); }
+// the head dims that xs_slstm_train_forward / _backward cover
+inline bool trains(int dh, bool bf16) { return dh >= 8 && dh % 8 == 0 && dh <= (bf16 ? 1024 : 512); }
 inline int local_waves(int dh) { return (dh + 15) / 16; }
 
 template <bool BF16, bool COEF>
 void (*pick_local(int w))(LocalParams) {
+  if constexpr (BF16) {
+    switch (w) {
+      case 5: return slstm_local_kernel<BF16, 5, COEF>;
+      case 6: return slstm_local_kernel<BF16, 6, COEF>;
+      case 7: return slstm_local_kernel<BF16, 7, COEF>;
+      case 8: return slstm_local_kernel<BF16, 8, COEF>;
+    }
+  }
   switch (w) {
     case 1: return slstm_local_kernel<BF16, 1, COEF>;
     case 2: return slstm_local_kernel<BF16, 2, COEF>;
     case 3: return slstm_local_kernel<BF16, 3, COEF>;
-    case 4: return slstm_local_kernel<BF16, 4, COEF>;
-    case 5: return slstm_local_kernel<BF16, 5, COEF>;
-    case 6: return slstm_local_kernel<BF16, 6, COEF>;
-    case 7: return slstm_local_kernel<BF16, 7, COEF>;
-    default: return slstm_local_kernel<BF16, 8, COEF>;
+    default: return slstm_local_kernel<BF16, 4, COEF>;
   }
 }
 template <bool BF16, bool DWX16>
 void (*pick_local_bwd(int w))(LocalBwdParams) {
+  if constexpr (BF16) {
+    switch (w) {
+      case 5: return slstm_local_bwd_kernel<BF16, 5, DWX16>;
+      case 6: return slstm_local_bwd_kernel<BF16, 6, DWX16>;
+      case 7: return slstm_local_bwd_kernel<BF16, 7, DWX16>;
+      case 8: return slstm_local_bwd_kernel<BF16, 8, DWX16>;
+    }
+  }
   switch (w) {
     case 1: return slstm_local_bwd_kernel<BF16, 1, DWX16>;
     case 2: return slstm_local_bwd_kernel<BF16, 2, DWX16>;
     case 3: return slstm_local_bwd_kernel<BF16, 3, DWX16>;
-    case 4: return slstm_local_bwd_kernel<BF16, 4, DWX16>;
-    case 5: return slstm_local_bwd_kernel<BF16, 5, DWX16>;
-    case 6: return slstm_local_bwd_kernel<BF16, 6, DWX16>;
-    case 7: return slstm_local_bwd_kernel<BF16, 7, DWX16>;
-    default: return slstm_local_bwd_kernel<BF16, 8, DWX16>;
+    default: return slstm_local_bwd_kernel<BF16, 4, DWX16>;
   }
 }
 // workgroups of a launch over (row tile of 4 rows, head) pairs: a multiple of 8 (one range per XCD)
@@ -335,13 +360,105 @@ int run_local(const xs_slstm_args *a, float *coef) {
   return e == hipSuccess ? XS_OK : fail(XS_ERR_LAUNCH, "sequence kernel launch failed: %s", hipGetErrorString(e));
 }
 
+// ---- the unit-split reverse kernel (slstm_backward_unit_kernel.h): how a call is cut into launches
+struct UnitPlan { int G, W, CT, RT, heads, groups; };  // members of 16 CT units; row tile; heads of a launch; row tiles per head of a launch
+// The first form of the list with which all of a head slice's row tiles fit at once; tiles of 16 rows in several launches
+// where none does.  us a step (bf16): head dim 256, 64 rows 1.77 with {2, 8} and 2.91 with two launches of {2, 4}; head
+// dim 512, 32 rows 2.16 with {2, 8} and 3.31 with {2, 16}; head dim 1024, 16 rows 3.81 and 6.11.  A group of up to 32
+// members sits on one XCD, which members of 32 units give every head dim of bf16.
+int unit_plan(int B, int NH, int dh, bool bf16, UnitPlan &u) {
+  const int cus = device_cus();
+  if (cus <= 0) return fail(XS_ERR_DEVICE, "cannot query the device");
+  u.W = (dh + 15) / 16;
+  const int per_xcd = cus / 8;
+  static const int forms[2][4][2] = {{{1, 4}, {1, 16}}, {{1, 4}, {2, 4}, {2, 8}, {2, 16}}};  // {CT, RT}: float32, bf16
+  bool found = false;
+  for (int i = 0; i < (bf16 ? 4 : 2); ++i) {
+    const int ct = forms[bf16][i][0], rt = forms[bf16][i][1], members = (u.W + ct - 1) / ct, capacity = members > 32 ? 0 : 8 * (per_xcd / members);
+    if (capacity < 1) continue;
+    const int heads = NH < capacity ? NH : capacity, groups = capacity / heads, tiles = (B + rt - 1) / rt;
+    u.G = members; u.CT = ct; u.RT = rt; u.heads = heads; u.groups = groups < tiles ? groups : tiles;
+    found = true;
+    if (tiles <= groups) break;
+  }
+  if (!found) return fail(XS_ERR_DEVICE, "a head of %d units does not fit the compute units of this device's XCDs", dh);
+  return XS_OK;
+}
+inline size_t unit_ring_bytes(const UnitPlan &u, int esz) { return (size_t)kBwdRing * u.heads * u.groups * u.G * u.RT * 64 * u.CT * esz; }
+
+template <bool BF16, int RT, int CT, bool DWX16>
+void (*pick_unit_bwd(int gq))(UnitBwdParams) {
+  if constexpr (!BF16) {
+    if (gq <= 2) return slstm_bwd_unit_kernel<BF16, 2, RT, CT, DWX16>;
+  }
+  if constexpr (CT == 2) {
+    if (gq <= 2) return slstm_bwd_unit_kernel<BF16, 2, RT, CT, DWX16>;
+    if (gq <= 4) return slstm_bwd_unit_kernel<BF16, 4, RT, CT, DWX16>;
+    return nullptr;
+  } else {
+    if (gq <= 4) return slstm_bwd_unit_kernel<BF16, 4, RT, CT, DWX16>;
+    if (gq <= 8) return slstm_bwd_unit_kernel<BF16, 8, RT, CT, DWX16>;
+    return nullptr;
+  }
+}
+template <bool DWX16>
+void (*pick_unit_bwd_bf16(int rt, int ct, int gq))(UnitBwdParams) {
+  if (ct == 1) return pick_unit_bwd<true, 4, 1, DWX16>(gq);
+  return rt == 4 ? pick_unit_bwd<true, 4, 2, DWX16>(gq) : (rt == 8 ? pick_unit_bwd<true, 8, 2, DWX16>(gq) : pick_unit_bwd<true, 16, 2, DWX16>(gq));
+}
+
+int run_unit_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_st, int r_dtype, int dwx_bf16, float clip) {
+  const bool bf16 = a->dtype == XS_BF16;
+  const int esz = bf16 ? 2 : 4;
+  UnitPlan u;
+  int rc = unit_plan(a->B, a->NH, a->dh, bf16, u);
+  if (rc != XS_OK) return rc;
+  if (!a->exchange || !a->counters) return fail(XS_ERR_NULL, "exchange and counters are required at this head dim");
+  if (((uintptr_t)a->exchange % 16) || ((uintptr_t)a->d_h % 16) || (d_h_sb * esz) % 16 || (d_h_st * esz) % 16)
+    return fail(XS_ERR_ALIGN, "exchange, d_h and its strides must be 16-byte aligned");
+  if (16 * d_h_sb * esz >= (1ll << 31) || (a->reset && 16 * a->reset_stride_b + a->T >= (1ll << 31)))
+    return fail(XS_ERR_UNSUPPORTED, "rows of d_h or of the reset mask lie too far apart");
+  UnitBwdParams p;
+  p.coef = a->coef; p.d_h = a->d_h; p.d_h_sb = d_h_sb; p.d_h_st = d_h_st; p.d_s_final = a->d_s_final;
+  p.r = a->r; p.r_bf16 = r_dtype == XS_BF16; p.reset = a->reset; p.reset_sb = a->reset_stride_b;
+  p.d_wx = a->d_wx; p.d_wx_sb = a->d_wx_stride_b; p.d_wx_st = a->d_wx_stride_t; p.d_s0 = a->d_s0;
+  p.xch = (char *)a->exchange; p.abort_word = a->counters; p.placement = a->counters + 1;
+  p.spin_limit = a->spin_limit != 0 ? a->spin_limit : kDefaultSpinLimit;
+  p.cut = a->recurrent_cut != 0; p.clip = clip;
+  p.B = a->B; p.T = a->T; p.NH = a->NH; p.dh = a->dh; p.G = u.G; p.W = u.W;
+  const int gq = (u.G + 4 * u.CT - 1) / (4 * u.CT);  // members of a wave's share of K
+  void (*k)(UnitBwdParams);
+  if (bf16) k = dwx_bf16 ? pick_unit_bwd_bf16<true>(u.RT, u.CT, gq) : pick_unit_bwd_bf16<false>(u.RT, u.CT, gq);
+  else k = u.RT == 4 ? pick_unit_bwd<false, 4, 1, false>(gq) : pick_unit_bwd<false, 16, 1, false>(gq);
+  if (!k) return fail(XS_ERR_UNSUPPORTED, "no reverse kernel for head dim %d", a->dh);
+  const int lds = unit_bwd_lds_bytes(u.RT, u.CT, bf16);
+  rc = ensure_dynamic_lds((const void *)k, (size_t)lds);
+  if (rc != XS_OK) return rc;
+  hipStream_t stream = (hipStream_t)a->stream;
+  bool first = true;
+  for (int h0 = 0; h0 < a->NH; h0 += u.heads)
+    for (int b0 = 0; b0 < a->B; b0 += u.RT * u.groups) {
+      p.head0 = h0; p.NHL = h0 + u.heads <= a->NH ? u.heads : a->NH - h0;
+      p.b0 = b0; p.bend = b0 + u.RT * u.groups < a->B ? b0 + u.RT * u.groups : a->B;
+      p.NBT = (p.bend - b0 + u.RT - 1) / u.RT;
+      const int ng = p.NHL * p.NBT;
+      const long long n16 = (long long)kBwdRing * ng * u.G * u.RT * 64 * u.CT * esz / 16;
+      hipLaunchKernelGGL(slstm_bwd_arm_kernel, dim3((unsigned)((n16 + 255) / 256 < 1024 ? (n16 + 255) / 256 : 1024)), dim3(256), 0, stream,
+                         (uint4 *)p.xch, n16, first ? p.abort_word : p.placement, ng + (first ? 1 : 0));
+      first = false;
+      hipLaunchKernelGGL(k, dim3(8u * u.G * ((ng + 7) / 8)), dim3(unit_bwd_threads(u.CT)), lds, stream, p);
+    }
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? XS_OK : fail(XS_ERR_LAUNCH, "backward kernel launch failed: %s", hipGetErrorString(e));
+}
+
 int run_train_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_st, int r_dtype) {
   if (!a) return fail(XS_ERR_NULL, "args is NULL");
   if (a->B < 0 || a->T < 0 || a->NH <= 0 || a->dh <= 0) return fail(XS_ERR_SHAPE, "bad dims B=%d T=%d NH=%d dh=%d", a->B, a->T, a->NH, a->dh);
   if (a->dtype != XS_F32 && a->dtype != XS_BF16) return fail(XS_ERR_DTYPE, "dtype must be XS_F32 or XS_BF16");
   const bool bf16 = a->dtype == XS_BF16;
   if (r_dtype != XS_F32 && !(r_dtype == XS_BF16 && bf16)) return fail(XS_ERR_DTYPE, "r_dtype must be XS_F32, or XS_BF16 with dtype XS_BF16");
-  if (a->dh % 8 != 0 || !local_head(a->dh)) return fail(XS_ERR_UNSUPPORTED, "head dim %d: a multiple of 8 up to %d", a->dh, kLocalMaxHeadDim);
+  if (!trains(a->dh, bf16)) return fail(XS_ERR_UNSUPPORTED, "head dim %d: a multiple of 8 up to %d", a->dh, bf16 ? 1024 : 512);
   if (a->B == 0 || a->T == 0) return XS_OK;
   int dwx_bf16 = 0;
   const int rc = d_wx_type(a, &dwx_bf16);
@@ -351,6 +468,8 @@ int run_train_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_s
   const long long H = (long long)a->NH * a->dh;
   if (a->d_wx_stride_t < 4 * H || (a->B > 1 && a->d_wx_stride_b < 4 * H)) return fail(XS_ERR_SHAPE, "d_wx strides overlap the innermost 4*H elements");
   if (a->reset && a->reset_stride_b < a->T) return fail(XS_ERR_SHAPE, "reset row stride %lld < T", (long long)a->reset_stride_b);
+  const float clip = (a->recurrent_clipval > 0.0f && a->recurrent_clipval < __builtin_inff()) ? a->recurrent_clipval : 0.0f;
+  if (!local_head(a->dh, bf16)) return run_unit_backward(a, d_h_sb, d_h_st, r_dtype, dwx_bf16, clip);
   const long long grid = local_grid(a->B, a->NH);
   if (grid > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many row tiles for one launch");
   const int w = local_waves(a->dh);
@@ -358,8 +477,7 @@ int run_train_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_s
   p.coef = a->coef; p.d_h = a->d_h; p.d_h_sb = d_h_sb; p.d_h_st = d_h_st; p.d_s_final = a->d_s_final;
   p.r = a->r; p.r_bf16 = r_dtype == XS_BF16; p.reset = a->reset; p.reset_sb = a->reset_stride_b;
   p.d_wx = a->d_wx; p.d_wx_sb = a->d_wx_stride_b; p.d_wx_st = a->d_wx_stride_t; p.d_s0 = a->d_s0;
-  p.cut = a->recurrent_cut != 0;
-  p.clip = (a->recurrent_clipval > 0.0f && a->recurrent_clipval < __builtin_inff()) ? a->recurrent_clipval : 0.0f;
+  p.cut = a->recurrent_cut != 0; p.clip = clip;
   p.B = a->B; p.T = a->T; p.NH = a->NH; p.dh = a->dh;
   void (*k)(LocalBwdParams) = bf16 ? (dwx_bf16 ? pick_local_bwd<true, true>(w) : pick_local_bwd<true, false>(w)) : pick_local_bwd<false, false>(w);
   hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(64 * w), 0, (hipStream_t)a->stream, p);
@@ -368,7 +486,7 @@ int run_train_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_s
 }
 
 // need != nullptr: launch nothing, only report the bytes of workspace the launches of this call touch
-int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_host = nullptr) {
+int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_host = nullptr, float *train_coef = nullptr) {
   hipStream_t stream = (hipStream_t)a->stream;
   const int B = a->B, T = a->T, NH = a->NH, dh = a->dh;
   const long long H = (long long)NH * dh;
@@ -420,7 +538,8 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
   const int tiles = (B + 15) / 16;
   const int max_groups_per_head = capacity / NHL;  // >= 1
   int MT = 1;
-  while (MT < 4 && (tiles + MT - 1) / MT > max_groups_per_head) MT *= 2;
+  // (a training forward that leaves its coefficients: one row tile per workgroup, more launches)
+  while (!train_coef && MT < 4 && (tiles + MT - 1) / MT > max_groups_per_head) MT *= 2;
   {
     // The gating waves of the kernel of four row tiles address W.x, the mask and h_out as a scalar base plus a 32-bit
     // offset per lane inside four rows / one row tile.  Where four rows span more than that (sequences of a gigabyte
@@ -432,7 +551,7 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
   }
   // small heads stay in one compute unit, the whole call in one launch (nothing waits, so nothing has to be resident
   // at once), unless the batch is one for the kernel of four row tiles
-  if (head0 == 0 && MT < 4 && !a->coef_out && local_forward(dh, bf16)) return dry ? XS_OK : run_local(a, nullptr);
+  if (head0 == 0 && MT < 4 && !a->coef_out && !train_coef && local_head(dh, bf16)) return dry ? XS_OK : run_local(a, nullptr);
   int rows_per_wg = 16 * MT;
   if (MT == 1) {  // spare compute units: smaller row tiles, smaller exchanges
     for (int r = 4; r < 16; r *= 2)
@@ -459,12 +578,14 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
     // row tiles of at most 4 rows: the compute waves split the columns by unit, not K (head groups on one XCD)
     const bool quad = MT == 1 && rows_per_wg == 4 && G <= 32;
     if (quad) kern = bf16 ? (full ? pick_quad<true, true>(nch) : pick_quad<true, false>(nch)) : (full ? pick_quad<false, true>(nch) : pick_quad<false, false>(nch));
+    if (train_coef) kern = bf16 ? (full ? pick_train<true, true>(nch, quad, burst) : pick_train<true, false>(nch, quad, burst))
+                                : (full ? pick_train<false, true>(nch, quad, burst) : pick_train<false, false>(nch, quad, burst));
     if (a->coef_out) {  // a training forward: the same kernel, leaving the backward pass its coefficients
       if (!quad || !bf16 || (dh != 128 && dh != 256) || rows_per_launch < B)
         return fail(XS_ERR_UNSUPPORTED, "coef_out: the call does not run in row tiles of 4 rows of one kernel (bf16, head dim 128 or 256, "
                                         "ceil(B/4) * NH * dh/16 workgroups on the device at once)");
       if (((uintptr_t)a->coef_out % 4)) return fail(XS_ERR_ALIGN, "coef_out must be 4-byte aligned");
-      kern = nch == 1 ? slstm_seq_kernel<true, 1, 1, true, false, false, true, true> : slstm_seq_kernel<true, 2, 1, true, false, false, true, true>;
+      kern = nch == 1 ? slstm_seq_kernel<true, 1, 1, true, false, false, true, 1> : slstm_seq_kernel<true, 2, 1, true, false, false, true, 1>;
     }
 #ifdef XS_SMALL_BATCH_FMA
     // the measured alternative for small batches (see the kernel): only in a library built for that measurement
@@ -507,7 +628,7 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
     p.b0 = b0; p.bend = bend; p.G = G; p.NBT = NBT; p.rows_per_wg = rows_per_wg;
     p.head0 = head0; p.NHL = NHL;
     p.spin_limit = a->spin_limit;
-    p.coef_out = a->coef_out;
+    p.coef_out = train_coef ? train_coef : a->coef_out;
     p.abort_host = abort_host;
     // a prefetch wave issues 2 (bf16) or 4 (fp32) scalar loads per batch row of a tile; 8 per wave and iteration
     // and 16 in all are what the scalar cache sustains, a tile that needs more goes without (prefetch waves that
@@ -1222,8 +1343,14 @@ int xs_slstm_forward_static(const xs_slstm_args *args) {
 }
 
 size_t xs_slstm_train_coef_floats(int32_t B, int32_t T, int32_t NH, int32_t dh, int32_t dtype) {
-  if (B < 1 || T < 1 || NH < 1 || dh < 8 || dh % 8 != 0 || (dtype != XS_F32 && dtype != XS_BF16) || !local_head(dh)) return 0;
-  return (size_t)T * ((B + 3) / 4) * NH * local_waves(dh) * 576;
+  if (B < 1 || T < 1 || NH < 1 || (dtype != XS_F32 && dtype != XS_BF16) || !trains(dh, dtype == XS_BF16)) return 0;
+  return (size_t)T * ((B + 3) / 4) * NH * ((dh + 15) / 16) * 576;
+}
+
+size_t xs_slstm_train_exchange_bytes(int32_t B, int32_t NH, int32_t dh, int32_t dtype) {
+  if (B < 1 || NH < 1 || (dtype != XS_F32 && dtype != XS_BF16) || !trains(dh, dtype == XS_BF16) || local_head(dh, dtype == XS_BF16)) return 0;
+  UnitPlan u;
+  return unit_plan(B, NH, dh, dtype == XS_BF16, u) == XS_OK ? unit_ring_bytes(u, dtype == XS_BF16 ? 2 : 4) : 0;
 }
 
 int xs_slstm_train_forward(const xs_slstm_args *args, float *coef) {
@@ -1233,8 +1360,10 @@ int xs_slstm_train_forward(const xs_slstm_args *args, float *coef) {
   if (!coef || ((uintptr_t)coef % 16)) return fail(coef ? XS_ERR_ALIGN : XS_ERR_NULL, "coef is required, 16-byte aligned");
   if (args->coef_out) return fail(XS_ERR_UNSUPPORTED, "coef_out goes with xs_slstm_forward");
   if (!xs_slstm_train_coef_floats(args->B, args->T, args->NH, args->dh, args->wx_dtype))
-    return fail(XS_ERR_UNSUPPORTED, "a training forward of this kind: head dims that are multiples of 8 up to %d, at least one row and step", kLocalMaxHeadDim);
-  return run_local(args, coef);
+    return fail(XS_ERR_UNSUPPORTED, "a training forward: at least one row and step, head dims up to 1024 (bf16) and 512 (float32)");
+  // (float32 between head dim 64 and 128 multiplies faster over several compute units, see local_forward)
+  if (local_head(args->dh, args->wx_dtype == XS_BF16)) return run_local(args, coef);
+  return run_forward(args, nullptr, nullptr, coef);
 }
 
 int xs_slstm_train_backward(const xs_slstm_bwd_args *args, int64_t d_h_stride_b, int64_t d_h_stride_t, int32_t r_dtype) {

@@ -1,6 +1,6 @@
 // Small heads: a whole head in ONE compute unit.  Included by slstm_hip.hip only, behind slstm_backward_kernels.h.
 //
-// Up to head dim 128 the recurrent matrix of a head fits the register file of a compute unit (bf16: 128 KiB of 512), and
+// Up to head dim 128 (bf16; 64 in float32) the recurrent matrix of a head is small enough for one compute unit (bf16: 128 KiB of 512 of registers), and
 // then nothing has to cross between compute units: the exchange of h that takes two thirds of a step of
 // slstm_seq_kernel (0.5 us of 0.75) becomes a pass through LDS, and so does the exchange of the gate deltas in the
 // reverse pass.  A workgroup owns four batch rows of one head; wave w owns the 16 units 16 w .. 16 w + 15 with all four
@@ -21,9 +21,10 @@
 //
 // What bounds a step is a chain again - LDS read, MFMAs, gating (some 300 cycles), LDS write, barrier - of 0.28 us at head dim
 // 16 to 0.60 at 128.  Measured, us per step at T 512, 4 heads, B 16 (slstm_seq_kernel and slstm_bwd_split / quad_kernel before
-// it): forward bf16 head dim 64 0.38 (0.73), 128 0.60 (0.75), float32 head dim 64 0.59 (1.20; at 128 1.57 against 1.24: there
-// only when training); reverse pass bf16 head dim 64 0.72 (0.90, and 0.25 for the forward walk in front of it), float32
-// head dim 96 1.70 (3.3, run as 128, and 0.43 for the walk).  Large batches are bound by the coefficients' 36 bytes per element.
+// it): forward bf16 head dim 64 0.38 (0.73), 128 0.60 (0.75), float32 head dim 64 0.59 (1.20); reverse pass bf16 head dim
+// 64 0.72 (0.90, and 0.25 for the forward walk in front of it).  float32 beyond 64 is bound by the matrix instructions of one
+// compute unit (1,024 cycles per wave and step at head dim 128: 1.57 forward, 1.70 reverse at 96, against 0.79 and 1.00 over
+// several).  Large batches are bound by the coefficients' 36 bytes per element.
 //
 // W.x (the coefficients, d_h) is fetched by the lanes that use it, kLocalAhead (kLocalBwdAhead) steps ahead into a ring
 // of registers; without polls there is nothing that these misses could hold up.
@@ -79,9 +80,9 @@ __device__ __forceinline__ bool local_place(int n, int NH, int &head, int &tile)
 template <bool BF16, int W, bool COEF>
 __global__ __launch_bounds__(64 * W) void slstm_local_kernel(LocalParams p) {
   typedef typename std::conditional<BF16, uint16_t, float>::type elem_t;
-  constexpr int KS = BF16 ? (W + 1) / 2 : (W + 3) / 4;  // bf16: MFMA k-steps of 32; float32: chunks of 16 inputs per quarter of K
-  constexpr int KW = 16 * KS;                           // (float32) inputs per quarter; nch of the other kernels: 1 up to 64, 2 up to 128
-  static_assert(BF16 || KS == 1 || KS == 2, "the quarters of K are 16 or 32 inputs");
+  static_assert(BF16 || W <= 4, "float32: head dims up to 64");
+  constexpr int KS = BF16 ? (W + 1) / 2 : 1;            // bf16: MFMA k-steps of 32
+  constexpr int KW = 16 * KS;                           // (float32) inputs per quarter of K
   // elements between the rows of the h tile in LDS: bf16 16 bytes of padding; float32 16 words beyond a multiple of 64
   // (the 16 lanes of a quarter of K read 4 rows x 16 words: all banks once)
   constexpr int HS = BF16 ? KS * 32 + 8 : 4 * KW + (4 * KW % 64 == 0 ? 16 : 80 - 4 * KW % 64);
@@ -171,7 +172,7 @@ __global__ __launch_bounds__(64 * W) void slstm_local_kernel(LocalParams p) {
   long long coef_step = 0;
   if constexpr (COEF) {
     coef_step = (long long)ntiles * p.NH * W * 576;
-    cfp = p.coef + (((long long)tile * p.NH + head) * W + wave) * 576 + lane * 4;
+    cfp = p.coef + (((long long)tile * p.NH + head) * W + wave) * 576;
   }
   elem_t *hop = reinterpret_cast<elem_t *>(p.h_out) + so;
   elem_t h_bits = 0;
@@ -179,10 +180,7 @@ __global__ __launch_bounds__(64 * W) void slstm_local_kernel(LocalParams p) {
     if (mine) __builtin_nontemporal_store(h_bits, hop + (long long)t * BH);
     if constexpr (COEF) {
       const float omf = __builtin_amdgcn_rcpf(1.0f + __expf(kept_f));  // 1 - sigmoid(f)
-      float *dst = cfp + t * coef_step;
-      *reinterpret_cast<f32x4 *>(dst) = f32x4{kept.og * kept.rn, kept_y * kept.rn, kept.ig * kept.tz, kept.ig};
-      *reinterpret_cast<f32x4 *>(dst + 256) = f32x4{kept.fg * omf * kept_c, kept.fg * omf * kept_n, kept.ig * (1.0f - kept.tz * kept.tz), (1.0f - kept.og) * kept_y};
-      dst[512 - 3 * lane] = kept.fg;
+      store_coefficients(cfp + t * coef_step, lane, kept, kept_y, kept_c, kept_n, omf);
     }
   };
 

@@ -28,7 +28,7 @@ struct SeqParams {
   long long spin_limit;
   int prefetch;  // number of prefetch waves launched behind the six others (0 .. kMaxPrefetchWaves)
   unsigned int *abort_host;  // a word in pinned host memory that a workgroup finishing after a give-up sets, or null
-  float *coef_out;  // COEF variant: the backward pass's nine coefficients per step and element,
+  float *coef_out;  // COEF variants: the backward pass's nine coefficients per step and element, 1:
                     // [T][ceil(B/4)][NH][dh/64][4 rows][9][64 units] (what slstm_bwd_quad_kernel reads); else unused
 };
 
@@ -158,14 +158,15 @@ __device__ __forceinline__ uint32_t seq_handshake(const SeqParams &p, int wg, in
 // order than the MFMA forms them, so the bits differ from the MFMA path (and from the decode kernel).
 // QUAD: row tiles of at most 4 rows: the four compute waves split the workgroup's 64 columns by UNIT instead of splitting
 // K, see "waves 0-3, QUAD" below.
-// COEF (with QUAD): a training forward: the compute waves also leave the nine coefficients per step and element that the
+// COEF: a training forward (1: in the layout slstm_bwd_quad_kernel reads, 2: in that of slstm_local_kernel, per row tile of
+// 4 rows, head and workgroup 576 floats; then also with K split over the waves and row tiles of 8 and 16 rows): the compute waves also leave the nine coefficients per step and element that the
 // backward pass would otherwise recompute in a forward walk of its own (slstm_bwd_prepare_kernel), see "COEF" below.
-template <bool BF16, int NCH, int MT, bool FULL, bool BURST, bool FMAC = false, bool QUAD = false, bool COEF = false>
+template <bool BF16, int NCH, int MT, bool FULL, bool BURST, bool FMAC = false, bool QUAD = false, int COEF = 0>
 __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm_seq_kernel(SeqParams p) {
-  static_assert(!COEF || QUAD, "coefficients for the backward pass come from the unit-split compute waves only");
+  static_assert(!COEF || MT == 1, "coefficients for the backward pass: one row tile per workgroup");
   static_assert(!FMAC || MT == 1, "the FMA contraction is for one row tile of at most 4 rows");
   static_assert(!QUAD || (MT == 1 && !BURST && !FMAC), "the unit-split compute waves exist for one row tile of at most 4 rows");
-  static_assert(!COEF || (BF16 && FULL), "coefficients for the backward pass: bf16, head dims that fill the K range");
+  static_assert(COEF != 1 || (QUAD && BF16 && FULL), "the layout of slstm_bwd_quad_kernel: bf16, row tiles of 4 rows, head dims that fill the K range");
   constexpr int EPC = BF16 ? 8 : 4;      // elements per 16-byte chunk
   constexpr int KW = NCH * 4 * EPC;      // input units per wave
   constexpr int ESZ = BF16 ? 2 : 4;
@@ -176,7 +177,9 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
   __shared__ float part[2][4][4][kTileFloats];  // [buffer][wave][gate][unit*stride + row]
   __shared__ float wxs[2][4][kTileFloats];      // [slot][gate][row*stride + unit]   W.x of one iteration
   __shared__ float hst[4][256];                 // [slot][row*16 + unit]             h on its way to HBM
-  __shared__ float cst[COEF ? 4 : 1][COEF ? 9 * 64 : 1];  // [slot][coefficient][row*16 + unit]  (COEF) on their way to HBM
+  constexpr int CSETS = COEF ? (QUAD ? 1 : 4) : 0;  // sets of 4 rows whose coefficients are staged
+  // (COEF) coefficients on their way to HBM: [slot][set]; 1: [coefficient][row*16 + unit]; 2: as they lie in memory
+  __shared__ __attribute__((aligned(16))) float cst[COEF ? 4 : 1][COEF ? CSETS * 576 : 1];
   __shared__ uint32_t rfl[4][16];               // [slot][row]                       reset flags
   __shared__ uint32_t cross_s;
 
@@ -354,18 +357,32 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
     // poll), between barriers #t+1 and #t+2, and leave three iterations behind: 4 rows x 9 coefficients x 16 units into
     // the piece of the (row tile, head, slice of 64 units) that the backward's reverse kernel reads per step
     float *coef_dst = nullptr;
-    long long coef_step = 0;
-    if constexpr (COEF) {
+    long long coef_step = 0, coef_set = 0;
+    if constexpr (COEF == 1) {
       const int ntiles = (p.B + 3) >> 2, S = dh >> 6;
       coef_step = (long long)ntiles * p.NH * S * (4 * 9 * 64);
       coef_dst = p.coef_out + ((((long long)(rowbase >> 2)) * p.NH + head) * S + (a0 >> 6)) * (4 * 9 * 64)
                  + (lane >> 4) * (9 * 64) + (a0 & 63) + (lane & 15);
+    } else if constexpr (COEF == 2) {
+      coef_set = (long long)p.NH * p.G * 576;
+      coef_step = (long long)((p.B + 3) >> 2) * coef_set;
+      coef_dst = p.coef_out + (long long)(rowbase >> 2) * coef_set + ((long long)head * p.G + member) * 576;
     }
     auto drain_coef = [&](int t) {
-      if constexpr (COEF) {
+      if constexpr (COEF == 1) {
         float *dst = coef_dst + t * coef_step;
 #pragma unroll
         for (int j = 0; j < 9; ++j) dst[j * 64] = cst[t & 3][j * 64 + lane];
+      } else if constexpr (COEF == 2) {
+#pragma unroll
+        for (int s = 0; s < CSETS; ++s) {
+          if (rowbase + 4 * s >= rend) break;
+          float *dst = coef_dst + t * coef_step + s * coef_set;
+          const float *src = cst[t & 3] + s * 576;
+          *reinterpret_cast<f32x4 *>(dst + 4 * lane) = *reinterpret_cast<const f32x4 *>(src + 4 * lane);
+          *reinterpret_cast<f32x4 *>(dst + 256 + 4 * lane) = *reinterpret_cast<const f32x4 *>(src + 256 + 4 * lane);
+          dst[512 + lane] = src[512 + lane];
+        }
       }
     };
     lds_barrier();  // prologue barrier
@@ -375,7 +392,8 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
 #endif
     for (int j = 0; j < NITpad; ++j) {
       if (j >= 2 && j - 2 < NIT) drain(j - 2);
-      if (COEF && j >= 3 && j - 3 < NIT) drain_coef(j - 3);
+      if (COEF && QUAD && j >= 3 && j - 3 < NIT) drain_coef(j - 3);
+      if (COEF && !QUAD && j >= 2 && j - 2 < NIT) drain_coef(j - 2);
 #ifdef XS_PROFILE
       { const long long now_ = clock64(); dprof[0] += now_ - dt; dt = now_; }
 #endif
@@ -387,7 +405,7 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
     lds_barrier();  // final barrier
     for (int it = (NITpad >= 2 ? NITpad - 2 : 0); it < NIT; ++it) drain(it);
     if (COEF)
-      for (int it = (NITpad >= 3 ? NITpad - 3 : 0); it < NIT; ++it) drain_coef(it);
+      for (int it = (NITpad >= (QUAD ? 3 : 2) ? NITpad - (QUAD ? 3 : 2) : 0); it < NIT; ++it) drain_coef(it);
     // A bounded wait ran out somewhere: whatever this workgroup computed from then on is built on operands that
     // never arrived.  A caller that does not read the status block must not mistake it for a result, so the
     // workgroup's part of h_out becomes NaN (the compute waves do the same to s_out).  Any workgroup that consumed
@@ -461,7 +479,7 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
   // without padding takes a quarter of the cycles of v_mfma_f32_16x16x4 (head dim 128: 256 instead of 1,024 per wave and
   // step), the operand is broadcast inside a quarter by the instruction, so that a lane polls only its own 16 bytes per 16
   // inputs of a quarter, and the quarters meet in a 4 x 4 transpose across the lane groups.  B 4 x T 256 x 4 heads of 128: 311 us
-  // with K split over the waves, XS_F32_QUAD_US with this.
+  // with K split over the waves, 199 us with this.
   // =========================================================================
   if constexpr (QUAD) {
     __builtin_amdgcn_s_setprio(3);
@@ -520,16 +538,20 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
       if constexpr (COEF) {
         const float omf = __builtin_amdgcn_rcpf(1.0f + __expf(kept_f));  // 1 - sigmoid(f)
         if (gate_lane) {
-          float *dst = &cst[t & 3][gb * 16 + gu];
-          dst[0 * 64] = kept.og * kept.rn;
-          dst[1 * 64] = kept_y * kept.rn;
-          dst[2 * 64] = kept.ig * kept.tz;
-          dst[3 * 64] = kept.ig;
-          dst[4 * 64] = kept.fg * omf * kept_c;
-          dst[5 * 64] = kept.fg * omf * kept_n;
-          dst[6 * 64] = kept.ig * (1.0f - kept.tz * kept.tz);
-          dst[7 * 64] = (1.0f - kept.og) * kept_y;
-          dst[8 * 64] = kept.fg;
+          if constexpr (COEF == 1) {
+            float *dst = &cst[t & 3][gb * 16 + gu];
+            dst[0 * 64] = kept.og * kept.rn;
+            dst[1 * 64] = kept_y * kept.rn;
+            dst[2 * 64] = kept.ig * kept.tz;
+            dst[3 * 64] = kept.ig;
+            dst[4 * 64] = kept.fg * omf * kept_c;
+            dst[5 * 64] = kept.fg * omf * kept_n;
+            dst[6 * 64] = kept.ig * (1.0f - kept.tz * kept.tz);
+            dst[7 * 64] = (1.0f - kept.og) * kept_y;
+            dst[8 * 64] = kept.fg;
+          } else {
+            store_coefficients(&cst[t & 3][0], gb * 16 + gu, kept, kept_y, kept_c, kept_n, omf);
+          }
         }
       }
     };
@@ -1144,7 +1166,10 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
         raw[g] = (wxs[buf][g][pb * kTileStride + pa] + ry) + bias_g[g];
       }
       if (rfl[it & 3][pb] != 0u) st[mt] = CellState{0.0f, 0.0f, 0.0f, 0.0f};
-      slstm_pointwise(raw[0], raw[1], raw[2], raw[3], st[mt]);
+      GateValues kept{0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+      const float kept_c = st[mt].c, kept_n = st[mt].n;
+      if constexpr (COEF != 0) slstm_pointwise_keep(raw[0], raw[1], raw[2], raw[3], st[mt], kept);
+      else slstm_pointwise(raw[0], raw[1], raw[2], raw[3], st[mt]);
 #ifdef XS_PROFILE
       asm volatile("" :: "v"(st[mt].y));
 #endif
@@ -1178,6 +1203,8 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
         }
       }
       hst[it & 3][tid] = y;
+      if constexpr (COEF != 0)  // (h is on its way)
+        store_coefficients(&cst[it & 3][(pb >> 2) * 576], (pb & 3) * 16 + pa, kept, y, kept_c, kept_n, __builtin_amdgcn_rcpf(1.0f + __expf(raw[1])));
       if (MT == 1) {
         // (the operand registers stay reserved to the end of the iteration: measured as fast or faster)
 #pragma unroll

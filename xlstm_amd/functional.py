@@ -91,28 +91,30 @@ def backward_coefficients_buffer(wx: torch.Tensor, num_heads: int) -> Optional[t
     B, T = int(wx.shape[0]), int(wx.shape[1])
     H = int(wx.shape[2]) // 4
     dh = H // num_heads
-    if wx.dtype != torch.bfloat16 or dh not in (128, 256) or B < 1 or T < 2:
-        return None
-    cus = _compute_units(wx.device)
-    groups4 = num_heads * ((B + 3) // 4)
-    if (groups4 + 7) // 8 * 8 * (dh // 16) > cus or (groups4 + 7) // 8 * 8 * (dh // 64) + 8 > cus:
+    if wx.dtype != torch.bfloat16 or dh not in (128, 256) or B < 1 or T < 2 or not _quad_fits(B, T, num_heads, dh, wx.device):
         return None
     return torch.empty((T, (B + 3) // 4 * 4, 9, H), dtype=torch.float32, device=wx.device)
 
 
+def _quad_fits(B: int, T: int, NH: int, dh: int, device) -> bool:
+    """Whether forward and backward of a bf16 call fit the device in row tiles of 4 rows, prefetching workgroups included."""
+    cus = _compute_units(device)
+    groups = (NH * ((B + 3) // 4) + 7) // 8 * 8
+    return groups * (dh // 16) <= cus and groups * (dh // 64) + 8 <= cus
+
+
 def training_coefficients(wx: torch.Tensor, num_heads: int) -> Optional[torch.Tensor]:
-    """The tensor a training forward at a small head dim (a multiple of 8 up to 128; ``slstm_forward(..., train_coef=)``)
-    leaves the backward pass's coefficients in, or ``None`` for other calls.  Such a head stays in one compute unit,
-    forward and backward (``xs_slstm_train_forward``)."""
+    """The tensor a training forward (``slstm_forward(..., train_coef=)``) leaves the backward pass's coefficients in, 36
+    bytes per step and element, or ``None`` for calls without a forward kernel (``xs_slstm_train_forward``)."""
     B, T = int(wx.shape[0]), int(wx.shape[1])
     n = _lib.load().xs_slstm_train_coef_floats(B, T, num_heads, int(wx.shape[2]) // 4 // num_heads, _DTYPE_CODE.get(wx.dtype, -1))
     return torch.empty(n, dtype=torch.float32, device=wx.device) if n else None
 
 
-def _small_head_backward(lib, wx, r, bias, s0, reset_mask, h_out, d_h, d_s_final, coef, timings, recurrent_cut, recurrent_clipval,
-                         d_wx_dtype):
-    """The backward pass of a head that stays in one compute unit: ``coef`` from the training forward, or None (the forward
-    runs once more and leaves them)."""
+def _train_backward(lib, wx, r, bias, s0, reset_mask, h_out, d_h, d_s_final, coef, timings, recurrent_cut, recurrent_clipval,
+                    d_wx_dtype, spin_limit, abort_sink):
+    """The backward pass by ``xs_slstm_train_backward``: ``coef`` from the training forward, or None (the forward runs once
+    more and leaves them)."""
     NH, dh = int(r.shape[0]), int(r.shape[2])
     B, T, H, dev = int(wx.shape[0]), int(wx.shape[1]), NH * dh, wx.device
     bf16 = wx.dtype == torch.bfloat16
@@ -138,8 +140,12 @@ def _small_head_backward(lib, wx, r, bias, s0, reset_mask, h_out, d_h, d_s_final
         if reset_mask is not None:
             reset_mask = _mask_u8(reset_mask, B, T)
         h_c = h_out if h_out.is_contiguous() and h_out.dtype == wx.dtype else h_out.to(wx.dtype).contiguous()
-        if d_h.dtype != wx.dtype or d_h.stride(2) != 1:
+        esz = wx.element_size()
+        if (d_h.dtype != wx.dtype or d_h.stride(2) != 1 or d_h.data_ptr() % 16 or (d_h.stride(0) * esz) % 16
+                or (d_h.stride(1) * esz) % 16 or d_h.stride(1) >= 1 << 25):
             d_h = d_h.to(wx.dtype).contiguous()
+        if reset_mask is not None and reset_mask.stride(0) >= 1 << 26:
+            reset_mask = reset_mask.contiguous()
         if d_s_final is not None:
             d_s_final = d_s_final.to(torch.float32).contiguous()
         d_wx = torch.empty((B, T, 4 * H), dtype=d_wx_dtype or torch.float32, device=dev)
@@ -159,6 +165,12 @@ def _small_head_backward(lib, wx, r, bias, s0, reset_mask, h_out, d_h, d_s_final
         a.d_s0, a.d_r, a.d_bias = d_s0.data_ptr(), d_r.data_ptr(), d_bias.data_ptr()
         a.recurrent_cut = 1 if recurrent_cut else 0
         a.recurrent_clipval = float(recurrent_clipval) if recurrent_clipval is not None else 0.0
+        a.spin_limit = int(spin_limit)
+        xbytes = lib.xs_slstm_train_exchange_bytes(B, NH, dh, a.dtype)
+        exchange = None
+        if xbytes:  # a head spread over compute units: the ring its members exchange through, behind the abort word
+            exchange = torch.empty(4096 + xbytes, dtype=torch.uint8, device=dev)
+            a.counters, a.exchange = exchange.data_ptr(), exchange.data_ptr() + 4096
         a.stream = torch.cuda.current_stream(dev).cuda_stream
         mark()
         rc = lib.xs_slstm_train_backward(ctypes.byref(a), d_h.stride(1), d_h.stride(0), _DTYPE_CODE[r.dtype])
@@ -170,7 +182,18 @@ def _small_head_backward(lib, wx, r, bias, s0, reset_mask, h_out, d_h, d_s_final
         mark()
     if timings is not None:
         timings["events"] = marks
+    if exchange is not None:
+        word = exchange[:4].view(torch.int32)
+        if abort_sink is not None:
+            abort_sink(word)
+        elif timings is None and int(word.item()):  # (a synchronisation)
+            raise EngineError(_GAVE_UP)
     return d_wx, d_r, d_bias, d_s0
+
+
+_GAVE_UP = ("xlstm_amd: a wait between the compute units of a head ran out in the backward pass "
+            "(other work held compute units, or the workgroups of a head were not placed on one XCD); "
+            "the gradients are invalid")
 
 
 def slstm_backward(
@@ -216,8 +239,8 @@ def slstm_backward(
     ``abort_sink``: a callable that takes the call's abort word (an int32 tensor of one element on the device) instead
     of this function reading it, which synchronises the host; the cell queues an asynchronous copy and raises at a later call.
     ``coef``: what a training forward left (``slstm_forward(..., coef_out=)`` or ``train_coef=``); the forward walk is then skipped.
-    Head dims up to 128 run ``xs_slstm_train_backward`` (a head in one compute unit) unless a kernel is asked for by one
-    of the overrides or ``spin_limit``.
+    Without an override most calls run ``xs_slstm_train_backward`` (one launch, from the coefficients of a training forward,
+    which runs again where ``coef`` is not given).
     ``recurrent_cut`` and ``recurrent_clipval`` are the reference's ``gradient_recurrent_cut`` (no gradient from a step
     to the y it started from, ``slstm_backward_cut.cu:265-312``) and ``gradient_recurrent_clipval`` (that gradient
     clipped to +-value before ``d_h`` is added, ``slstm_pointwise.cu:136-143``).
@@ -234,11 +257,13 @@ def slstm_backward(
         raise ValueError(f"h_out and d_h must be [S, B, H] = {(T, B, H)}")
     if coef is not None and coef.dim() == 1 and coef.numel() != lib.xs_slstm_train_coef_floats(B, T, NH, dh, _DTYPE_CODE[wx.dtype]):
         raise ValueError("coef must be the tensor that the forward call of the same inputs filled")
-    # a small head stays in one compute unit (no choice of kernels, nothing waits): unless a kernel is asked for by name
+    # Unless a kernel is asked for by name: the reverse pass of one launch from a training forward's coefficients.  bf16 at
+    # head dim 256 keeps the kernel for row tiles of 4 rows x 64 units (its prefetching workgroups: 1.03 us a step) where it fits
     if ((coef is None or coef.dim() == 1) and split_override is None and row_tile_override is None and not stepwise_override
-            and spin_limit == 0 and lib.xs_slstm_train_coef_floats(B, T, NH, dh, _DTYPE_CODE[wx.dtype])):
-        return _small_head_backward(lib, wx, r, bias, s0, reset_mask, h_out, d_h, d_s_final, coef, timings, recurrent_cut,
-                                    recurrent_clipval, d_wx_dtype)
+            and not (coef is None and bf16 and dh == 256 and _quad_fits(B, T, NH, dh, wx.device))
+            and lib.xs_slstm_train_coef_floats(B, T, NH, dh, _DTYPE_CODE[wx.dtype])):
+        return _train_backward(lib, wx, r, bias, s0, reset_mask, h_out, d_h, d_s_final, coef, timings, recurrent_cut,
+                               recurrent_clipval, d_wx_dtype, spin_limit, abort_sink)
     dh_k = backward_kernel_head_dim(dh, wx.dtype)
     if coef is not None and (dh_k != dh or not bf16 or tuple(coef.shape) != (T, (B + 3) // 4 * 4, 9, H)
                              or coef.dtype != torch.float32 or not coef.is_contiguous()):
@@ -418,9 +443,7 @@ def slstm_backward(
     if split and abort_sink is not None:  # (the caller looks at the call's abort word later: no synchronisation here)
         abort_sink(counters[:1])
     elif split and timings is None and int(counters[0].item()):  # (a synchronisation)
-        raise EngineError("xlstm_amd: a wait between the compute units of a head ran out in the backward pass "
-                          "(other work held compute units, or the workgroups of a head were not placed on one XCD); "
-                          "the gradients are invalid")
+        raise EngineError(_GAVE_UP)
     return d_wx, d_r, d_bias, d_s0
 
 
