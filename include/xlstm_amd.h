@@ -395,13 +395,14 @@ int xs_slstm_backward(const xs_slstm_bwd_args *args);
  *                                 copy; where exchange is needed, 16-byte aligned), d_s_final, r (the forward's layout and,
  *                                 with r_dtype XS_F32, its float32 master), reset, recurrent_cut, recurrent_clipval,
  *                                 exchange, counters, spin_limit; writes d_wx (d_wx_dtype) and d_s0.
+ * abort_host: NULL, or a pinned host word (as for xs_slstm_forward_watched) that becomes 1 when a wait ran out.
  * The gradients of r and the bias: xs_slstm_backward_params, as for the other kernels.
  * Like coef_out, this takes the place of the state history and gate cache of the reference (slstm.cc:79-108).
  */
 size_t xs_slstm_train_coef_floats(int32_t B, int32_t T, int32_t NH, int32_t dh, int32_t dtype);
 size_t xs_slstm_train_exchange_bytes(int32_t B, int32_t NH, int32_t dh, int32_t dtype);
-int xs_slstm_train_forward(const xs_slstm_args *args, float *coef);
-int xs_slstm_train_backward(const xs_slstm_bwd_args *args, int64_t d_h_stride_b, int64_t d_h_stride_t, int32_t r_dtype);
+int xs_slstm_train_forward(const xs_slstm_args *args, float *coef, uint32_t *abort_host);
+int xs_slstm_train_backward(const xs_slstm_bwd_args *args, int64_t d_h_stride_b, int64_t d_h_stride_t, int32_t r_dtype, uint32_t *abort_host);
 
 /*
  * xs_slstm_backward_params   the gradients of the recurrent matrix and the bias from the gate deltas that

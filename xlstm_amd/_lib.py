@@ -224,9 +224,9 @@ def load() -> ctypes.CDLL:
     lib.xs_slstm_train_exchange_bytes.restype = ctypes.c_size_t
     lib.xs_slstm_train_exchange_bytes.argtypes = [ctypes.c_int32] * 4
     lib.xs_slstm_train_forward.restype = ctypes.c_int
-    lib.xs_slstm_train_forward.argtypes = [ctypes.POINTER(SlstmArgs), ctypes.c_void_p]
+    lib.xs_slstm_train_forward.argtypes = [ctypes.POINTER(SlstmArgs), ctypes.c_void_p, ctypes.c_void_p]
     lib.xs_slstm_train_backward.restype = ctypes.c_int
-    lib.xs_slstm_train_backward.argtypes = [ctypes.POINTER(SlstmBwdArgs), ctypes.c_int64, ctypes.c_int64, ctypes.c_int32]
+    lib.xs_slstm_train_backward.argtypes = [ctypes.POINTER(SlstmBwdArgs), ctypes.c_int64, ctypes.c_int64, ctypes.c_int32, ctypes.c_void_p]
     lib.xs_measure_stage.restype = ctypes.c_int
     lib.xs_measure_stage.argtypes = [ctypes.POINTER(MeasureArgs)]
     if lib.xs_abi_version() != ABI_VERSION:
@@ -259,7 +259,8 @@ def host():
     mod = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(mod)
     names = ("xs_slstm_step", "xs_slstm_forward_watched", "xs_slstm_workspace_bytes", "xs_last_error", "xs_causal_conv_silu",
-             "xs_headwise_gates", "xs_headwise_group_norm")
+             "xs_headwise_gates", "xs_headwise_group_norm", "xs_slstm_train_coef_floats", "xs_slstm_train_exchange_bytes",
+             "xs_slstm_train_forward", "xs_slstm_train_backward", "xs_slstm_backward_params")
     mod.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names}, EngineError,
              torch_module._global_forward_hooks, torch_module._global_forward_pre_hooks)
     _HOST = mod

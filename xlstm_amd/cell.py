@@ -38,6 +38,8 @@ from torch import nn
 
 from . import functional as F_hip
 
+_ENGINE_BACKWARD = F_hip.slstm_backward
+
 DTYPE_DICT = {
     "bfloat16": torch.bfloat16,
     "float16": torch.float16,
@@ -552,11 +554,22 @@ class sLSTMCell_hip(nn.Module):
             if native is None and input.is_cuda:
                 native = self._native()
             fast = native.forward(input, state, reset_mask, self.config, self.keep_state_fp32) if native is not None else None
+            if fast is None and native is not None and torch.is_grad_enabled() and self._trains_natively(input):
+                fast = native.train(input, state, reset_mask, self.config, self.keep_state_fp32)
             if fast is not None:
                 self._rt.last_workspace = native
         if fast is not None:
             return fast
         return self._run(input, state, reset_mask, step=False)
+
+    def _trains_natively(self, input: torch.Tensor) -> bool:
+        """Whether a training call takes the native host path.  Not where the coefficients are not to be kept, where
+        ``functional.slstm_backward`` has been replaced (whoever did so sees every backward call), and for long bfloat16
+        sequences at head dim 256: forward and backward in row tiles of 4 rows x 64 units save 0.07 us a step there
+        and take three more launches."""
+        return (self.keep_backward_coefficients and F_hip.slstm_backward is _ENGINE_BACKWARD
+                and not (self.head_dim == 256 and input.dtype == torch.bfloat16
+                         and input.shape[1 if self.config.input_shape == "BSGNH" else 0] >= 384))
 
     def step(self, input: torch.Tensor, state: Optional[torch.Tensor] = None, reset_mask=None,
              state_out: Optional[torch.Tensor] = None, h_out: Optional[torch.Tensor] = None,

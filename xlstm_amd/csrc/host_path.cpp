@@ -1,5 +1,5 @@
-// Native host path of the calls a program makes often: a decode step and an inference call of a cell, and the same of
-// a layer.  What the Python layers of cell.py, layer.py and functional.py do for such a call - look at dtypes, strides,
+// Native host path of the calls a program makes often: a decode step, an inference call and a training call of a cell,
+// and the first two of a layer.  What the Python layers of cell.py, layer.py and functional.py do for such a call - look at dtypes, strides,
 // versions and modes, allocate the outputs, fill an argument block, launch - takes 15 us per cell call and 75 us per
 // layer call there, more than the kernels run; here it takes about 4 and 8.
 //
@@ -18,10 +18,14 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/saved_variable.h>
 
+#include <memory>
 #include <mutex>
-#include <unordered_map>
 #include <vector>
 
 #include "xlstm_amd.h"
@@ -37,6 +41,11 @@ struct Engine {
   decltype(&xs_causal_conv_silu) conv = nullptr;
   decltype(&xs_headwise_gates) gates = nullptr;
   decltype(&xs_headwise_group_norm) norm = nullptr;
+  decltype(&xs_slstm_train_coef_floats) coef_floats = nullptr;
+  decltype(&xs_slstm_train_exchange_bytes) exchange_bytes = nullptr;
+  decltype(&xs_slstm_train_forward) train_forward = nullptr;
+  decltype(&xs_slstm_train_backward) train_backward = nullptr;
+  decltype(&xs_slstm_backward_params) backward_params = nullptr;
   PyObject *error = nullptr;              // functional.EngineError
   PyObject *global_hooks[2] = {nullptr, nullptr};  // hooks on every module of the process
 } g_engine;
@@ -45,7 +54,7 @@ struct Engine {
 struct Names {
   PyObject *r, *b, *weight, *bias, *conv_state, *slstm_state, *input_shape, *output_shape, *keep_state_fp32, *config;
   PyObject *modules, *parameters, *forward_hooks, *forward_pre_hooks, *training, *p, *eps, *conv1d, *conv, *fgate, *igate, *zgate, *ogate;
-  PyObject *group_norm, *slstm_cell, *dropout, *fused_pre_ops, *rt, *bsgnh;
+  PyObject *group_norm, *slstm_cell, *dropout, *fused_pre_ops, *bsgnh, *cut, *clipval;
 } g_names;
 
 struct PyRef {  // owns one reference
@@ -106,6 +115,11 @@ class WordPool {
   std::vector<uint32_t *> free_;  // [next_, end): free words, oldest first
   size_t next_ = 0;
 } g_words;
+using AbortWord = std::shared_ptr<uint32_t>;  // a cell's, and its backward calls' that are still to come
+AbortWord take_word() {
+  uint32_t *w = g_words.take();
+  return w ? AbortWord(w, [](uint32_t *p) { g_words.give_back(p); }) : nullptr;
+}
 
 // ---- one cell
 struct CellPath {
@@ -128,7 +142,7 @@ struct CellPath {
   const void *bias32_of = nullptr;
   uint32_t bias32_version = 0;
   at::Tensor last_workspace;
-  uint32_t *abort_word = nullptr;
+  AbortWord abort_word;
   uint64_t devices_used = 0;
 
   const at::Tensor &parameter(PyObject *name) const {
@@ -139,7 +153,6 @@ struct CellPath {
   ~CellPath() {
     Py_XDECREF(parameters);
     Py_XDECREF(plan);
-    if (abort_word) g_words.give_back(abort_word);
   }
 
   bool records(const at::Tensor &x, const at::Tensor *state, const at::Tensor &r, const at::Tensor &b) const {
@@ -165,8 +178,8 @@ struct CellPath {
   }
 
   void raise_if_aborted() {
-    if (abort_word && __atomic_load_n(abort_word, __ATOMIC_ACQUIRE)) {
-      __atomic_store_n(abort_word, 0u, __ATOMIC_RELEASE);
+    if (abort_word && __atomic_load_n(abort_word.get(), __ATOMIC_ACQUIRE)) {
+      __atomic_store_n(abort_word.get(), 0u, __ATOMIC_RELEASE);
       PyErr_SetString(g_engine.error,
                       "an earlier sLSTM sequence call (forward or backward) on the hip backend gave up waiting for some of its "
                       "compute units (they were held by other work on the GPU); its outputs were set to NaN");
@@ -300,7 +313,7 @@ PyObject *cell_step_(CellPath &c, PyObject *const *args) {
 }
 
 // ---- a sequence through the cell (no autograd), as sLSTMCell_hip._run and functional.slstm_forward do it
-struct Sequence { at::Tensor h, state; };  // h: [S,B,H] memory (with the strides of `shape` where given), state: float32
+struct Sequence { at::Tensor h, state, coef, mask; };  // h: [S,B,H] memory with the strides of `shape`, state: float32
 at::Tensor mask_bytes(const at::Tensor &m, int64_t B, int64_t T) {
   if (!m.is_cuda() || m.dim() != 2 || m.size(0) != B || m.size(1) != T) throw NotCovered{};
   at::Tensor r = m;
@@ -309,12 +322,18 @@ at::Tensor mask_bytes(const at::Tensor &m, int64_t B, int64_t T) {
   return r.stride(1) != 1 ? r.contiguous() : r;
 }
 
-Sequence run_sequence(CellPath &c, at::Tensor x, const at::Tensor *state, const at::Tensor *mask, OutShape shape) {
+bool capturing(const at::Device &d) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing((hipStream_t)stream_of(d), &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
+// train: the forward of a training call, which also leaves the backward pass its coefficients (no graph is recorded here)
+Sequence run_sequence(CellPath &c, at::Tensor x, const at::Tensor *state, const at::Tensor *mask, OutShape shape, bool train = false) {
   const int64_t H = c.NH * c.dh, B = x.size(0), T = x.size(1);
   const auto dt = x.scalar_type();
   if ((dt != at::kFloat && dt != at::kBFloat16) || !x.is_cuda() || T < 2 || B < 1 || x.size(2) != 4 * H) throw NotCovered{};
   at::Tensor r = c.parameter(g_names.r), b = c.parameter(g_names.b);
-  if (c.records(x, state, r, b) || r.device() != x.device() || b.device() != x.device() || !r.is_contiguous() || !b.is_contiguous()) throw NotCovered{};
+  if ((!train && c.records(x, state, r, b)) || r.device() != x.device() || b.device() != x.device() || !r.is_contiguous() || !b.is_contiguous()) throw NotCovered{};
   if ((r.scalar_type() != at::kFloat && r.scalar_type() != at::kBFloat16) || r.numel() != c.NH * 4 * c.dh * c.dh || b.numel() != 4 * H) throw NotCovered{};
   const size_t esz = x.element_size();
   if (x.stride(2) != 1 || !aligned(x.data_ptr(), 16) || (x.stride(0) * esz) % 16 || (x.stride(1) * esz) % 16 || x.stride(1) < 4 * H ||
@@ -333,17 +352,19 @@ Sequence run_sequence(CellPath &c, at::Tensor x, const at::Tensor *state, const 
     s0 = state->to(at::kFloat).contiguous();
   }
   if (mask) m = mask_bytes(*mask, B, T);
-  const bool capturing = [&] {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing((hipStream_t)stream_of(x.device()), &st) != hipSuccess || st != hipStreamCaptureStatusNone;
-  }();
-  if (!capturing) c.raise_if_aborted();
+  const bool in_graph = capturing(x.device());
+  if (!in_graph) c.raise_if_aborted();
   const Shape4 s4 = shape_of(shape, T, B, c.NH, c.dh);
   Sequence out;
   out.h = at::empty_strided(at::IntArrayRef(s4.size.data(), s4.n), at::IntArrayRef(s4.stride.data(), s4.n), x.options());
   out.state = at::empty({4, B, H}, x.options().dtype(at::kFloat));
+  if (train) {
+    const size_t n = g_engine.coef_floats((int32_t)B, (int32_t)T, (int32_t)c.NH, (int32_t)c.dh, dtype_code(dt));
+    if (!n) throw NotCovered{};
+    out.coef = at::empty({(int64_t)n}, out.state.options());
+  }
   at::Tensor &ws = c.workspace(B, x.device());
-  if (!c.abort_word) c.abort_word = g_words.take();
+  if (!c.abort_word) c.abort_word = take_word();
   if (!c.abort_word) throw NotCovered{};
   xs_slstm_args a{};
   a.B = (int32_t)B; a.T = (int32_t)T; a.NH = (int32_t)c.NH; a.dh = (int32_t)c.dh;
@@ -355,7 +376,9 @@ Sequence run_sequence(CellPath &c, at::Tensor x, const at::Tensor *state, const 
   a.h_out = out.h.data_ptr(); a.s_out = (float *)out.state.data_ptr();
   a.workspace = ws.data_ptr(); a.workspace_bytes = (size_t)ws.numel();
   a.stream = stream_of(x.device());
-  launched(g_engine.forward(&a, capturing ? nullptr : c.abort_word));
+  uint32_t *word = in_graph ? nullptr : c.abort_word.get();
+  launched(train ? g_engine.train_forward(&a, (float *)out.coef.data_ptr(), word) : g_engine.forward(&a, word));
+  out.mask = m;
   c.last_workspace = ws;
   if (x.device().index() < 64) c.devices_used |= 1ull << x.device().index();
   return out;
@@ -375,6 +398,159 @@ PyObject *cell_forward_(CellPath &c, PyObject *const *args) {
   return PyTuple_Pack(2, ph.o, ps.o);
 }
 
+// ---- training: the engine's two backward calls (reverse pass, gradients of R and bias) as a node of the autograd graph,
+// the way _CellFunction and functional._train_backward do it
+struct ReverseInputs {
+  at::Tensor r, h, state, mask, coef;  // as the forward used them; h: [T,B,H] memory
+  AbortWord word;
+  int64_t B, T, NH, dh;
+  bool cut;
+  double clip;
+};
+struct CellGradients { at::Tensor d_wx, d_r, d_bias, d_s0; };
+// d_h: [T,B,H] with the strides (d_sb, d_st); d_s: float32 or undefined.  Called without the GIL
+[[noreturn]] void engine_failed_in_backward(int rc) {
+  const std::string what = g_engine.last_error();
+  PyGILState_STATE gil = PyGILState_Ensure();
+  PyErr_Format(g_engine.error, "xlstm_amd error %d: %s", rc, what.c_str());
+  python_error e;
+  e.persist();
+  PyGILState_Release(gil);
+  throw e;
+}
+CellGradients run_reverse(const ReverseInputs &in, const at::Tensor &d_h, int64_t d_sb, int64_t d_st, const at::Tensor &d_s) {
+  const int64_t B = in.B, T = in.T, NH = in.NH, dh = in.dh, H = NH * dh;
+  const auto dt = in.h.scalar_type();
+  const auto f32 = in.h.options().dtype(at::kFloat);
+  at::Tensor r = in.r;
+  if (!(r.scalar_type() == at::kFloat || (r.scalar_type() == at::kBFloat16 && dt == at::kBFloat16))) r = r.to(at::kFloat);
+  CellGradients g;
+  g.d_wx = at::empty({B, T, 4 * H}, in.h.options());
+  g.d_s0 = at::empty({4, B, H}, f32);
+  g.d_r = at::empty({NH, 4 * dh, dh}, f32);
+  g.d_bias = at::empty({4 * H}, f32);
+  xs_slstm_bwd_args a{};
+  a.B = (int32_t)B; a.T = (int32_t)T; a.NH = (int32_t)NH; a.dh = (int32_t)dh;
+  a.dtype = dtype_code(dt);
+  a.coef = (float *)in.coef.data_ptr(); a.d_h = d_h.data_ptr(); a.r = r.data_ptr(); a.h_out = in.h.data_ptr();
+  at::Tensor d_s32, s0;
+  if (d_s.defined()) { d_s32 = d_s.to(at::kFloat).contiguous(); a.d_s_final = (const float *)d_s32.data_ptr(); }
+  if (in.state.defined()) { s0 = in.state.to(at::kFloat).contiguous(); a.s0 = (const float *)s0.data_ptr(); }
+  if (in.mask.defined()) { a.reset = (const uint8_t *)in.mask.data_ptr(); a.reset_stride_b = in.mask.stride(0); }
+  a.d_wx = (float *)g.d_wx.data_ptr(); a.d_wx_stride_b = g.d_wx.stride(0); a.d_wx_stride_t = g.d_wx.stride(1);
+  a.d_wx_dtype = dtype_code(dt);
+  a.d_s0 = (float *)g.d_s0.data_ptr(); a.d_r = (float *)g.d_r.data_ptr(); a.d_bias = (float *)g.d_bias.data_ptr();
+  a.recurrent_cut = in.cut; a.recurrent_clipval = (float)in.clip;
+  const size_t xbytes = g_engine.exchange_bytes((int32_t)B, (int32_t)NH, (int32_t)dh, a.dtype);
+  at::Tensor exchange;
+  if (xbytes) {  // a head spread over compute units: the ring its members exchange through, behind the abort word
+    exchange = at::empty({(int64_t)(4096 + xbytes)}, in.h.options().dtype(at::kByte));
+    a.counters = (unsigned int *)exchange.data_ptr();
+    a.exchange = (char *)exchange.data_ptr() + 4096;
+  }
+  a.stream = stream_of(in.h.device());
+  int rc = g_engine.train_backward(&a, d_sb, d_st, dtype_code(r.scalar_type()), capturing(in.h.device()) ? nullptr : in.word.get());
+  if (rc == XS_OK) rc = g_engine.backward_params(&a);
+  if (rc != XS_OK) engine_failed_in_backward(rc);
+  return g;
+}
+
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+struct CellBackward : public torch::autograd::Node {
+  SavedVariable r, h, state;
+  bool has_state = false, transposed_input = false;
+  ReverseInputs in;  // (its saved tensors are filled in when the backward runs)
+  OutShape shape = OutShape::BNSH;
+  at::ScalarType r_dtype = at::kFloat, b_dtype = at::kFloat, s_dtype = at::kFloat;
+
+  std::string name() const override { return "sLSTMCellBackward"; }
+  void release_variables() override {
+    r.reset_data(); h.reset_data(); state.reset_data();
+    in.coef.reset(); in.mask.reset();
+  }
+  variable_list apply(variable_list &&grads) override {
+    at::NoGradGuard no_grad;
+    ReverseInputs call = in;
+    const at::Tensor h_saved = h.unpack(shared_from_this());
+    c10::OptionalDeviceGuard guard(h_saved.device());
+    const int64_t B = in.B, T = in.T, dh = in.dh, H = in.NH * dh;
+    // [S,B,H] views of the output and its gradient
+    auto sbh = [&](const at::Tensor &t) {
+      switch (shape) {
+        case OutShape::BNSH: return t.permute({2, 0, 1, 3});
+        case OutShape::SBH: return t.unsqueeze(2);
+        case OutShape::BSH: return t.permute({1, 0, 2}).unsqueeze(2);
+        default: return t;
+      }
+    };
+    call.h = h_saved;
+    call.r = r.unpack();
+    if (has_state) call.state = state.unpack();
+    at::Tensor d = grads[0].defined() ? sbh(grads[0]) : at::zeros({T, B, 1, H}, h_saved.options());  // [S,B,NH,dh] or [S,B,1,H]
+    const int64_t esz = h_saved.element_size();
+    int64_t sb = B > 1 ? d.stride(1) : H, st = d.stride(0);
+    if (d.scalar_type() != h_saved.scalar_type() || d.stride(3) != 1 || (d.size(2) > 1 && d.stride(2) != dh) || !aligned(d.data_ptr(), 16) ||
+        (sb * esz) % 16 || (st * esz) % 16 || sb >= (1 << 25) || sb < 0 || st < 0) {
+      d = d.to(h_saved.scalar_type()).contiguous();
+      sb = H; st = B * H;
+    }
+    CellGradients g = run_reverse(call, d, sb, st, grads[1]);
+    variable_list out(has_state ? 4 : 3);
+    out[0] = transposed_input ? g.d_wx.permute({1, 0, 2}) : g.d_wx;
+    out[1] = g.d_r.to(r_dtype);
+    out[2] = g.d_bias.to(b_dtype);
+    if (has_state) out[3] = g.d_s0.to(s_dtype);
+    return out;
+  }
+};
+
+// train(input, state, reset_mask, config, keep_state_fp32) -> (output, state) with their place in the graph, or None
+PyObject *cell_train_(CellPath &c, PyObject *const *args) {
+  if (at::autocast::is_autocast_enabled(at::kCUDA) || !THPVariable_Check(args[0]) || !recording(c, args[0], args[1])) Py_RETURN_NONE;
+  const at::Tensor &x = tensor_of(args[0]);
+  const bool bsgnh = input_is_bsgnh(args[3]);
+  if (x.dim() != 3 || !x.is_cuda() || x.size(bsgnh ? 1 : 0) < 2 || x.size(bsgnh ? 0 : 1) < 1) Py_RETURN_NONE;
+  if ((x.scalar_type() != at::kFloat && x.scalar_type() != at::kBFloat16) ||
+      !g_engine.coef_floats(1, 1, (int32_t)c.NH, (int32_t)c.dh, dtype_code(x.scalar_type())))
+    Py_RETURN_NONE;
+  const at::Tensor *state = optional_tensor(args[1]), *mask = optional_tensor(args[2]);
+  const OutShape shape = out_shape(args[3]);
+  PyRef cut(PyObject_GetAttr(args[3], g_names.cut)), clip(PyObject_GetAttr(args[3], g_names.clipval));
+  if (!cut.o || !clip.o) throw PythonError{};
+  const int cut_on = PyObject_IsTrue(cut.o);
+  const double clipval = clip.o == Py_None ? 0.0 : PyFloat_AsDouble(clip.o);
+  if (PyErr_Occurred()) throw PythonError{};
+  c10::OptionalDeviceGuard guard(x.device());
+  Sequence s;
+  at::Tensor s_out;
+  {
+    const at::Tensor r = c.parameter(g_names.r), b = c.parameter(g_names.b);
+    {
+      at::NoGradGuard no_grad;
+      s = run_sequence(c, bsgnh ? x : x.permute({1, 0, 2}), state, mask, shape, true);
+    }
+    auto node = std::shared_ptr<CellBackward>(new CellBackward(), torch::autograd::deleteNode);
+    node->set_next_edges(state ? torch::autograd::collect_next_edges(x, r, b, *state) : torch::autograd::collect_next_edges(x, r, b));
+    node->r = SavedVariable(r, false);
+    node->has_state = state != nullptr;
+    if (state) { node->state = SavedVariable(*state, false); node->s_dtype = state->scalar_type(); }
+    node->transposed_input = !bsgnh;
+    node->shape = shape;
+    node->r_dtype = r.scalar_type(); node->b_dtype = b.scalar_type();
+    node->in.mask = s.mask; node->in.coef = s.coef; node->in.word = c.abort_word;
+    node->in.B = s.state.size(1); node->in.T = x.size(bsgnh ? 1 : 0); node->in.NH = c.NH; node->in.dh = c.dh;
+    node->in.cut = cut_on != 0; node->in.clip = clipval;
+    torch::autograd::set_history(s.h, node);
+    torch::autograd::set_history(s.state, node);
+    node->h = SavedVariable(s.h, true);
+  }
+  PyRef ph(THPVariable_Wrap(s.h)), ps(THPVariable_Wrap(args[4] == Py_True || x.scalar_type() == at::kFloat ? s.state : s.state.to(x.scalar_type())));
+  if (!ph.o || !ps.o) throw PythonError{};
+  return PyTuple_Pack(2, ph.o, ps.o);
+}
+
 template <PyObject *(*F)(CellPath &, PyObject *const *), int N>
 PyObject *cell_call(PyObject *self, PyObject *const *args, Py_ssize_t n) {
   if (n != N) { PyErr_Format(PyExc_TypeError, "%d arguments expected, got %zd", N, n); return nullptr; }
@@ -383,6 +559,9 @@ PyObject *cell_call(PyObject *self, PyObject *const *args, Py_ssize_t n) {
   } catch (const NotCovered &) {
     Py_RETURN_NONE;
   } catch (const PythonError &) {
+    return nullptr;
+  } catch (python_error &e) {
+    e.restore();
     return nullptr;
   } catch (const std::exception &e) {
     PyErr_SetString(PyExc_RuntimeError, e.what());
@@ -425,7 +604,7 @@ PyObject *cell_poll_(CellPath &c, PyObject *const *args) {
         Py_END_ALLOW_THREADS
       }
   }
-  if (c.abort_word && __atomic_exchange_n(c.abort_word, 0u, __ATOMIC_ACQ_REL)) Py_RETURN_TRUE;
+  if (c.abort_word && __atomic_exchange_n(c.abort_word.get(), 0u, __ATOMIC_ACQ_REL)) Py_RETURN_TRUE;
   Py_RETURN_FALSE;
 }
 
@@ -451,6 +630,7 @@ void cell_dealloc(PyObject *self) {
 PyMethodDef cell_methods[] = {
     {"step", (PyCFunction)(void *)cell_call<cell_step_, 8>, METH_FASTCALL, nullptr},
     {"forward", (PyCFunction)(void *)cell_call<cell_forward_, 5>, METH_FASTCALL, nullptr},
+    {"train", (PyCFunction)(void *)cell_call<cell_train_, 5>, METH_FASTCALL, nullptr},
     {"set_plan", (PyCFunction)(void *)cell_call<cell_set_plan_, 5>, METH_FASTCALL, nullptr},
     {"workspace", (PyCFunction)(void *)cell_call<cell_workspace_, 2>, METH_FASTCALL, nullptr},
     {"last_workspace", (PyCFunction)(void *)cell_call<cell_last_workspace_, 0>, METH_FASTCALL, nullptr},
@@ -710,6 +890,9 @@ PyObject *layer_call(PyObject *, PyObject *const *args, Py_ssize_t n) {
     Py_RETURN_NONE;
   } catch (const PythonError &) {
     return nullptr;
+  } catch (python_error &e) {
+    e.restore();
+    return nullptr;
   } catch (const std::exception &e) {
     PyErr_SetString(PyExc_RuntimeError, e.what());
     return nullptr;
@@ -726,7 +909,10 @@ PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
   };
   if (!get("xs_slstm_step", g_engine.step) || !get("xs_slstm_forward_watched", g_engine.forward) ||
       !get("xs_slstm_workspace_bytes", g_engine.workspace_bytes) || !get("xs_last_error", g_engine.last_error) ||
-      !get("xs_causal_conv_silu", g_engine.conv) || !get("xs_headwise_gates", g_engine.gates) || !get("xs_headwise_group_norm", g_engine.norm)) {
+      !get("xs_causal_conv_silu", g_engine.conv) || !get("xs_headwise_gates", g_engine.gates) || !get("xs_headwise_group_norm", g_engine.norm) ||
+      !get("xs_slstm_train_coef_floats", g_engine.coef_floats) || !get("xs_slstm_train_exchange_bytes", g_engine.exchange_bytes) ||
+      !get("xs_slstm_train_forward", g_engine.train_forward) || !get("xs_slstm_train_backward", g_engine.train_backward) ||
+      !get("xs_slstm_backward_params", g_engine.backward_params)) {
     PyErr_SetString(PyExc_KeyError, "an entry point of the engine is missing");
     return nullptr;
   }
@@ -751,7 +937,7 @@ PyMODINIT_FUNC PyInit__xlstm_host(void) {
   g_names = Names{s("_recurrent_kernel_"), s("_bias_"), s("weight"), s("bias"), s("conv_state"), s("slstm_state"), s("input_shape"), s("output_shape"),
                   s("keep_state_fp32"), s("config"), s("_modules"), s("_parameters"), s("_forward_hooks"), s("_forward_pre_hooks"), s("training"), s("p"),
                   s("eps"), s("conv1d"), s("conv"), s("fgate"), s("igate"), s("zgate"), s("ogate"), s("group_norm"), s("slstm_cell"), s("dropout"),
-                  s("fused_pre_ops"), s("_rt"), s("BSGNH")};
+                  s("fused_pre_ops"), s("BSGNH"), s("gradient_recurrent_cut"), s("gradient_recurrent_clipval")};
   PyObject *m = PyModule_Create(&module_def);
   if (!m) return nullptr;
   g_cell_type = (PyTypeObject *)PyType_FromSpec(&cell_spec);

@@ -41,6 +41,7 @@ struct UnitBwdParams {
   float *d_s0;
   char *xch;                 // exchange ring [kBwdRing][groups of the launch][member][RT rows][16 CT units][4 gates]
   unsigned int *abort_word, *placement;
+  unsigned int *abort_host;  // a pinned host word that a wait that ran out is reported in, or null
   long long spin_limit;
   int cut;
   float clip;
@@ -369,8 +370,9 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
     const bool mixed = !p.cut && (seen & (seen - 1u)) != 0u;  // (the plain stores reach one XCD's L2 only)
     if (mixed && tid == 0) __hip_atomic_store(p.abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     dy = (p.cut || after) ? 0.0f : add_up(p.T - 1);
+    const bool poisoned = mixed || __hip_atomic_load(p.abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
+    if (poisoned && p.abort_host && lane == 0) __hip_atomic_store(p.abort_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (mine) {
-      const bool poisoned = mixed || __hip_atomic_load(p.abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
       p.d_s0[so] = poisoned ? kPoison : dy;
       p.d_s0[BH + so] = poisoned ? kPoison : dc;
       p.d_s0[2 * BH + so] = poisoned ? kPoison : dn;

@@ -407,7 +407,7 @@ void (*pick_unit_bwd_bf16(int rt, int ct, int gq))(UnitBwdParams) {
   return rt == 4 ? pick_unit_bwd<true, 4, 2, DWX16>(gq) : (rt == 8 ? pick_unit_bwd<true, 8, 2, DWX16>(gq) : pick_unit_bwd<true, 16, 2, DWX16>(gq));
 }
 
-int run_unit_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_st, int r_dtype, int dwx_bf16, float clip) {
+int run_unit_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_st, int r_dtype, int dwx_bf16, float clip, uint32_t *abort_host) {
   const bool bf16 = a->dtype == XS_BF16;
   const int esz = bf16 ? 2 : 4;
   UnitPlan u;
@@ -422,7 +422,7 @@ int run_unit_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_st
   p.coef = a->coef; p.d_h = a->d_h; p.d_h_sb = d_h_sb; p.d_h_st = d_h_st; p.d_s_final = a->d_s_final;
   p.r = a->r; p.r_bf16 = r_dtype == XS_BF16; p.reset = a->reset; p.reset_sb = a->reset_stride_b;
   p.d_wx = a->d_wx; p.d_wx_sb = a->d_wx_stride_b; p.d_wx_st = a->d_wx_stride_t; p.d_s0 = a->d_s0;
-  p.xch = (char *)a->exchange; p.abort_word = a->counters; p.placement = a->counters + 1;
+  p.xch = (char *)a->exchange; p.abort_word = a->counters; p.placement = a->counters + 1; p.abort_host = abort_host;
   p.spin_limit = a->spin_limit != 0 ? a->spin_limit : kDefaultSpinLimit;
   p.cut = a->recurrent_cut != 0; p.clip = clip;
   p.B = a->B; p.T = a->T; p.NH = a->NH; p.dh = a->dh; p.G = u.G; p.W = u.W;
@@ -452,7 +452,7 @@ int run_unit_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_st
   return e == hipSuccess ? XS_OK : fail(XS_ERR_LAUNCH, "backward kernel launch failed: %s", hipGetErrorString(e));
 }
 
-int run_train_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_st, int r_dtype) {
+int run_train_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_st, int r_dtype, uint32_t *abort_host) {
   if (!a) return fail(XS_ERR_NULL, "args is NULL");
   if (a->B < 0 || a->T < 0 || a->NH <= 0 || a->dh <= 0) return fail(XS_ERR_SHAPE, "bad dims B=%d T=%d NH=%d dh=%d", a->B, a->T, a->NH, a->dh);
   if (a->dtype != XS_F32 && a->dtype != XS_BF16) return fail(XS_ERR_DTYPE, "dtype must be XS_F32 or XS_BF16");
@@ -469,7 +469,7 @@ int run_train_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_s
   if (a->d_wx_stride_t < 4 * H || (a->B > 1 && a->d_wx_stride_b < 4 * H)) return fail(XS_ERR_SHAPE, "d_wx strides overlap the innermost 4*H elements");
   if (a->reset && a->reset_stride_b < a->T) return fail(XS_ERR_SHAPE, "reset row stride %lld < T", (long long)a->reset_stride_b);
   const float clip = (a->recurrent_clipval > 0.0f && a->recurrent_clipval < __builtin_inff()) ? a->recurrent_clipval : 0.0f;
-  if (!local_head(a->dh, bf16)) return run_unit_backward(a, d_h_sb, d_h_st, r_dtype, dwx_bf16, clip);
+  if (!local_head(a->dh, bf16)) return run_unit_backward(a, d_h_sb, d_h_st, r_dtype, dwx_bf16, clip, abort_host);
   const long long grid = local_grid(a->B, a->NH);
   if (grid > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many row tiles for one launch");
   const int w = local_waves(a->dh);
@@ -1353,7 +1353,7 @@ size_t xs_slstm_train_exchange_bytes(int32_t B, int32_t NH, int32_t dh, int32_t 
   return unit_plan(B, NH, dh, dtype == XS_BF16, u) == XS_OK ? unit_ring_bytes(u, dtype == XS_BF16 ? 2 : 4) : 0;
 }
 
-int xs_slstm_train_forward(const xs_slstm_args *args, float *coef) {
+int xs_slstm_train_forward(const xs_slstm_args *args, float *coef, uint32_t *abort_host) {
   g_err[0] = 0;
   const int rc = validate(args, false);
   if (rc != XS_OK) return rc;
@@ -1361,14 +1361,13 @@ int xs_slstm_train_forward(const xs_slstm_args *args, float *coef) {
   if (args->coef_out) return fail(XS_ERR_UNSUPPORTED, "coef_out goes with xs_slstm_forward");
   if (!xs_slstm_train_coef_floats(args->B, args->T, args->NH, args->dh, args->wx_dtype))
     return fail(XS_ERR_UNSUPPORTED, "a training forward: at least one row and step, head dims up to 1024 (bf16) and 512 (float32)");
-  // (float32 between head dim 64 and 128 multiplies faster over several compute units, see local_forward)
   if (local_head(args->dh, args->wx_dtype == XS_BF16)) return run_local(args, coef);
-  return run_forward(args, nullptr, nullptr, coef);
+  return run_forward(args, nullptr, abort_host, coef);
 }
 
-int xs_slstm_train_backward(const xs_slstm_bwd_args *args, int64_t d_h_stride_b, int64_t d_h_stride_t, int32_t r_dtype) {
+int xs_slstm_train_backward(const xs_slstm_bwd_args *args, int64_t d_h_stride_b, int64_t d_h_stride_t, int32_t r_dtype, uint32_t *abort_host) {
   g_err[0] = 0;
-  return run_train_backward(args, d_h_stride_b, d_h_stride_t, r_dtype);
+  return run_train_backward(args, d_h_stride_b, d_h_stride_t, r_dtype, abort_host);
 }
 
 int xs_slstm_step(const xs_slstm_args *args) {

@@ -173,7 +173,7 @@ def _train_backward(lib, wx, r, bias, s0, reset_mask, h_out, d_h, d_s_final, coe
             a.counters, a.exchange = exchange.data_ptr(), exchange.data_ptr() + 4096
         a.stream = torch.cuda.current_stream(dev).cuda_stream
         mark()
-        rc = lib.xs_slstm_train_backward(ctypes.byref(a), d_h.stride(1), d_h.stride(0), _DTYPE_CODE[r.dtype])
+        rc = lib.xs_slstm_train_backward(ctypes.byref(a), d_h.stride(1), d_h.stride(0), _DTYPE_CODE[r.dtype], None)
         if rc == 0:
             mark()
             rc = lib.xs_slstm_backward_params(ctypes.byref(a))
@@ -575,7 +575,7 @@ def slstm_forward(
         a.coef_out = coef_out.data_ptr()
     with torch.cuda.device(dev):
         if train_coef is not None:
-            rc = lib.xs_slstm_train_forward(ctypes.byref(a), train_coef.data_ptr())
+            rc = lib.xs_slstm_train_forward(ctypes.byref(a), train_coef.data_ptr(), None)
         else:
             rc = (lib.xs_slstm_step if step else lib.xs_slstm_forward)(ctypes.byref(a))
     if rc != 0:
