@@ -88,6 +88,11 @@ inline bool aligned(const void *p, uintptr_t n) { return ((uintptr_t)p) % n == 0
 inline uint32_t version_of(const at::Tensor &t) { return t.is_inference() ? 0u : t._version(); }
 inline bool versioned(const at::Tensor &t) { return !t.is_inference(); }
 
+bool capturing(const at::Device &d) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing((hipStream_t)stream_of(d), &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
 // ---- abort words: pinned host words that a sequence kernel writes when one of its bounded waits ran out.  Pages of
 // words live as long as the process (a kernel of a cell that is gone may still be running), a word given back is the
 // last to be handed out again, and there are no more words than cells were alive at once (rounded up to a page).
@@ -135,12 +140,10 @@ struct CellPath {
   uint32_t r_version = 0, b_version = 0;
   at::Tensor last_state, last_h;   // what the last step handed out (float32 state kept), and their versions
   uint32_t last_state_version = 0, last_h_version = 0;
-  // sequences: a workspace per (device, stream), a float32 copy of the bias where the parameter is not float32
-  struct Workspace { int device; void *stream; at::Tensor t; };
+  // sequences: a workspace per (device, stream)
+  struct Workspace { int device; void *stream; at::Tensor t; bool captured = false; };
   std::vector<Workspace> workspaces;
-  at::Tensor bias32;
-  const void *bias32_of = nullptr;
-  uint32_t bias32_version = 0;
+  std::vector<at::Tensor> captured;  // workspaces that a recorded graph writes and that a larger one has replaced
   at::Tensor last_workspace;
   AbortWord abort_word;
   uint64_t devices_used = 0;
@@ -167,13 +170,19 @@ struct CellPath {
       if (it.device == d.index() && it.stream == stream) { w = &it; break; }
     if (!w) {
       // (a program that makes a new stream per call would otherwise collect workspaces without end; a stream's
-      // allocations are handed on in stream order by the caching allocator, so dropping the oldest is safe)
-      if (workspaces.size() >= 16) workspaces.erase(workspaces.begin());
+      // allocations are handed on in stream order by the caching allocator, so dropping the oldest is safe - unless
+      // it was used under capture: replays of the graph write it for as long as the graph lives)
+      if (workspaces.size() >= 16)
+        for (auto it = workspaces.begin(); it != workspaces.end(); ++it)
+          if (!it->captured) { workspaces.erase(it); break; }
       workspaces.push_back(Workspace{(int)d.index(), stream, at::Tensor()});
       w = &workspaces.back();
     }
-    if (!w->t.defined() || (size_t)w->t.numel() < need)
+    if (!w->t.defined() || (size_t)w->t.numel() < need) {
+      if (w->captured) captured.push_back(w->t);
       w->t = at::empty({(int64_t)need}, at::TensorOptions().dtype(at::kByte).device(d));
+    }
+    w->captured |= capturing(d);
     return w->t;
   }
 
@@ -322,11 +331,6 @@ at::Tensor mask_bytes(const at::Tensor &m, int64_t B, int64_t T) {
   return r.stride(1) != 1 ? r.contiguous() : r;
 }
 
-bool capturing(const at::Device &d) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing((hipStream_t)stream_of(d), &st) != hipSuccess || st != hipStreamCaptureStatusNone;
-}
-
 // train: the forward of a training call, which also leaves the backward pass its coefficients (no graph is recorded here)
 Sequence run_sequence(CellPath &c, at::Tensor x, const at::Tensor *state, const at::Tensor *mask, OutShape shape, bool train = false) {
   const int64_t H = c.NH * c.dh, B = x.size(0), T = x.size(1);
@@ -340,12 +344,7 @@ Sequence run_sequence(CellPath &c, at::Tensor x, const at::Tensor *state, const 
       (B > 1 && x.stride(0) < 4 * H))
     x = x.contiguous();
   if (dt == at::kFloat && r.scalar_type() != at::kFloat) r = r.to(at::kFloat);
-  if (b.scalar_type() != at::kFloat) {
-    if (!c.bias32.defined() || c.bias32_of != b.data_ptr() || c.bias32_version != version_of(b) || !versioned(b) || c.bias32.device() != b.device()) {
-      c.bias32 = b.to(at::kFloat); c.bias32_of = b.data_ptr(); c.bias32_version = version_of(b);
-    }
-    b = c.bias32;
-  }
+  if (b.scalar_type() != at::kFloat) b = b.to(at::kFloat);  // (on every call: a copy kept would be another stream's, and a graph's)
   at::Tensor s0, m;
   if (state) {
     if (!state->is_cuda() || state->dim() != 3 || state->size(0) != 4 || state->size(1) != B || state->size(2) != H) throw NotCovered{};
@@ -364,8 +363,10 @@ Sequence run_sequence(CellPath &c, at::Tensor x, const at::Tensor *state, const 
     out.coef = at::empty({(int64_t)n}, out.state.options());
   }
   at::Tensor &ws = c.workspace(B, x.device());
-  if (!c.abort_word) c.abort_word = take_word();
-  if (!c.abort_word) throw NotCovered{};
+  if (!in_graph) {  // (under capture no host memory is allocated, and a replay reports to nobody)
+    if (!c.abort_word) c.abort_word = take_word();
+    if (!c.abort_word) throw NotCovered{};
+  }
   xs_slstm_args a{};
   a.B = (int32_t)B; a.T = (int32_t)T; a.NH = (int32_t)c.NH; a.dh = (int32_t)c.dh;
   a.wx_dtype = dtype_code(dt); a.r_dtype = dtype_code(r.scalar_type());
