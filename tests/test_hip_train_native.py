@@ -68,3 +68,61 @@ def test_native_training_call_equals_the_python_path(monkeypatch, dtype, in_shap
         with torch.no_grad():
             cell._recurrent_kernel_.mul_(1.0)
         torch.autograd.grad(out, x, torch.ones_like(out))
+
+
+def _small_cell(NH=2, dh=64):
+    from xlstm_amd.cell import sLSTMCell, sLSTMCellConfig
+
+    torch.manual_seed(dh)
+    cell = sLSTMCell(sLSTMCellConfig(hidden_size=NH * dh, num_heads=NH, backend="hip", recurrent_weight_init="standard")).to(DEV)
+    return cell, torch.randn(3, 5, 4 * NH * dh, device=DEV, requires_grad=True)
+
+
+def test_forward_mode_is_refused():
+    print("case forward mode", flush=True)
+    cell, x = _small_cell()
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            cell(dual)
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("dh", [64, 128])
+def test_checkpointing_and_hooks_see_what_is_saved(monkeypatch, native, dh):
+    """Checkpointing keeps nothing of the first forward; hooks pack the coefficients as well; gradients stay the same."""
+    from torch.utils.checkpoint import checkpoint
+
+    from xlstm_amd import cell as cell_module
+
+    print("case saved tensors", native, dh, flush=True)
+    if not native:
+        plain = cell_module.F_hip.slstm_backward
+        monkeypatch.setattr(cell_module.F_hip, "slstm_backward", lambda *a, **kw: plain(*a, **kw))
+    cell, x = _small_cell(dh=dh)
+    leaves = [x, *cell.parameters()]
+    out, _ = cell(x)
+    d = torch.randn_like(out)
+    want = torch.autograd.grad(out, leaves, d)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.numel()), t.cpu())[1], lambda t: t.to(DEV)):
+        hooked = torch.autograd.grad(cell(x)[0], leaves, d)
+    coef = cell_module.F_hip.training_coefficients(x, 2).numel()
+    assert coef in packed and x.numel() in packed and cell._bias_.numel() in packed
+    again = torch.autograd.grad(checkpoint(lambda v: cell(v)[0], x, use_reentrant=False), leaves, d)
+    for a, b, c in zip(want, hooked, again):
+        # (sums over rows and steps by float atomics: 15 terms of order 1)
+        torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5)
+        torch.testing.assert_close(a, c, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("which", ["input", "_bias_", "_recurrent_kernel_"])
+def test_changes_in_front_of_the_backward_are_refused(which):
+    print("case in place", which, flush=True)
+    cell, leaf = _small_cell()
+    x = leaf * 1.0
+    out, _ = cell(x)
+    with torch.no_grad():
+        (x if which == "input" else getattr(cell, which)).mul_(1.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.sum().backward()

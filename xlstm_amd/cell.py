@@ -202,20 +202,23 @@ class _CellFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, r, bias, state, h, s, mask, num_heads, cut, clipval, coef, abort_sink):
-        ctx.save_for_backward(x, r, bias, h, *(() if state is None else (state,)))
+        own = coef if coef is not None and coef.dim() == 1 else None  # (read, not consumed: hooks may pack it, the graph run twice)
+        ctx.has_state = state is not None
+        ctx.save_for_backward(x, r, bias, h, *(() if state is None else (state,)), *(() if own is None else (own,)))
         ctx.mask, ctx.num_heads, ctx.cut, ctx.clipval = mask, num_heads, cut, clipval
-        ctx.coef = coef  # (what a training forward left for the backward pass, or None: see keep_backward_coefficients)
+        ctx.coef = coef if own is None else None  # (what a training forward left for the backward pass, or None: see keep_backward_coefficients)
         ctx.abort_sink = abort_sink  # (takes the backward call's abort word: the cell looks at it later, without a synchronisation)
         return h.view_as(h), s.view_as(s)
 
     @staticmethod
     def backward(ctx, d_h, d_s):
         x, r, bias, h = ctx.saved_tensors[:4]
-        state = ctx.saved_tensors[4] if len(ctx.saved_tensors) > 4 else None
+        state = ctx.saved_tensors[4] if ctx.has_state else None
+        coef = ctx.saved_tensors[-1] if len(ctx.saved_tensors) > 4 + ctx.has_state else ctx.coef
         NH, dh = ctx.num_heads, r.shape[2]
         d_wx, d_r, d_bias, d_s0 = F_hip.slstm_backward(
             x.detach(), r.detach(), bias.detach().view(NH, 4, dh), None if state is None else state.detach(), ctx.mask,
-            h, d_h, d_s, recurrent_cut=ctx.cut, recurrent_clipval=ctx.clipval, coef=ctx.coef,
+            h, d_h, d_s, recurrent_cut=ctx.cut, recurrent_clipval=ctx.clipval, coef=coef,
             d_wx_dtype=torch.bfloat16 if x.dtype == torch.bfloat16 else None,  # (the input's gradient in the input's type)
             abort_sink=ctx.abort_sink)
         ctx.coef = None

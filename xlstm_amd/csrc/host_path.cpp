@@ -437,7 +437,11 @@ CellGradients run_reverse(const ReverseInputs &in, const at::Tensor &d_h, int64_
   at::Tensor d_s32, s0;
   if (d_s.defined()) { d_s32 = d_s.to(at::kFloat).contiguous(); a.d_s_final = (const float *)d_s32.data_ptr(); }
   if (in.state.defined()) { s0 = in.state.to(at::kFloat).contiguous(); a.s0 = (const float *)s0.data_ptr(); }
-  if (in.mask.defined()) { a.reset = (const uint8_t *)in.mask.data_ptr(); a.reset_stride_b = in.mask.stride(0); }
+  at::Tensor mask = in.mask;
+  if (mask.defined()) {
+    if (mask.stride(0) >= (1 << 26)) mask = mask.contiguous();  // (the reverse kernel's offsets are 31-bit)
+    a.reset = (const uint8_t *)mask.data_ptr(); a.reset_stride_b = mask.stride(0);
+  }
   a.d_wx = (float *)g.d_wx.data_ptr(); a.d_wx_stride_b = g.d_wx.stride(0); a.d_wx_stride_t = g.d_wx.stride(1);
   a.d_wx_dtype = dtype_code(dt);
   a.d_s0 = (float *)g.d_s0.data_ptr(); a.d_r = (float *)g.d_r.data_ptr(); a.d_bias = (float *)g.d_bias.data_ptr();
@@ -460,7 +464,9 @@ using torch::autograd::SavedVariable;
 using torch::autograd::variable_list;
 
 struct CellBackward : public torch::autograd::Node {
-  SavedVariable r, h, state;
+  // (input and bias are not read again: a change of theirs in front of the backward is refused like one of R.  The
+  // coefficients are saved like a tensor of the caller's, so that checkpointing and offloading hooks see them)
+  SavedVariable x, r, b, h, state, coef;
   bool has_state = false, transposed_input = false;
   ReverseInputs in;  // (its saved tensors are filled in when the backward runs)
   OutShape shape = OutShape::BNSH;
@@ -468,12 +474,16 @@ struct CellBackward : public torch::autograd::Node {
 
   std::string name() const override { return "sLSTMCellBackward"; }
   void release_variables() override {
-    r.reset_data(); h.reset_data(); state.reset_data();
-    in.coef.reset(); in.mask.reset();
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (SavedVariable *v : {&x, &r, &b, &h, &state, &coef}) v->reset_data();
+    in.mask.reset();
   }
   variable_list apply(variable_list &&grads) override {
+    std::lock_guard<std::mutex> lock(mutex_);
     at::NoGradGuard no_grad;
     ReverseInputs call = in;
+    x.unpack();
+    b.unpack();
     const at::Tensor h_saved = h.unpack(shared_from_this());
     c10::OptionalDeviceGuard guard(h_saved.device());
     const int64_t B = in.B, T = in.T, dh = in.dh, H = in.NH * dh;
@@ -488,6 +498,7 @@ struct CellBackward : public torch::autograd::Node {
     };
     call.h = h_saved;
     call.r = r.unpack();
+    call.coef = coef.unpack();
     if (has_state) call.state = state.unpack();
     at::Tensor d = grads[0].defined() ? sbh(grads[0]) : at::zeros({T, B, 1, H}, h_saved.options());  // [S,B,NH,dh] or [S,B,1,H]
     const int64_t esz = h_saved.element_size();
@@ -517,6 +528,8 @@ PyObject *cell_train_(CellPath &c, PyObject *const *args) {
       !g_engine.coef_floats(1, 1, (int32_t)c.NH, (int32_t)c.dh, dtype_code(x.scalar_type())))
     Py_RETURN_NONE;
   const at::Tensor *state = optional_tensor(args[1]), *mask = optional_tensor(args[2]);
+  for (const at::Tensor *t : {&x, &c.parameter(g_names.r), &c.parameter(g_names.b), state})
+    if (t && t->_fw_grad(0).defined()) Py_RETURN_NONE;  // (forward mode: the general path refuses it)
   const OutShape shape = out_shape(args[3]);
   PyRef cut(PyObject_GetAttr(args[3], g_names.cut)), clip(PyObject_GetAttr(args[3], g_names.clipval));
   if (!cut.o || !clip.o) throw PythonError{};
@@ -534,13 +547,16 @@ PyObject *cell_train_(CellPath &c, PyObject *const *args) {
     }
     auto node = std::shared_ptr<CellBackward>(new CellBackward(), torch::autograd::deleteNode);
     node->set_next_edges(state ? torch::autograd::collect_next_edges(x, r, b, *state) : torch::autograd::collect_next_edges(x, r, b));
+    node->x = SavedVariable(x, false);
     node->r = SavedVariable(r, false);
+    node->b = SavedVariable(b, false);
+    node->coef = SavedVariable(s.coef, false);
     node->has_state = state != nullptr;
     if (state) { node->state = SavedVariable(*state, false); node->s_dtype = state->scalar_type(); }
     node->transposed_input = !bsgnh;
     node->shape = shape;
     node->r_dtype = r.scalar_type(); node->b_dtype = b.scalar_type();
-    node->in.mask = s.mask; node->in.coef = s.coef; node->in.word = c.abort_word;
+    node->in.mask = s.mask; node->in.word = c.abort_word;
     node->in.B = s.state.size(1); node->in.T = x.size(bsgnh ? 1 : 0); node->in.NH = c.NH; node->in.dh = c.dh;
     node->in.cut = cut_on != 0; node->in.clip = clipval;
     torch::autograd::set_history(s.h, node);
