@@ -126,3 +126,30 @@ def test_changes_in_front_of_the_backward_are_refused(which):
         (x if which == "input" else getattr(cell, which)).mul_(1.0)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         out.sum().backward()
+
+
+@pytest.mark.parametrize("dtype,dh", [(torch.bfloat16, 64), (torch.float32, 96), (torch.bfloat16, 256), (torch.bfloat16, 512)])
+def test_coefficients_beyond_what_is_kept(monkeypatch, dtype, dh):
+    """Coefficients of a size that is not kept: the backward call makes them again, in slices of rows."""
+    from xlstm_amd import cell as cell_module
+
+    print("case coefficients not kept", dtype, dh, flush=True)
+    cell, _ = _small_cell(dh=dh)
+    B, T = 37, 4
+    x = torch.randn(B, T, 8 * dh, device=DEV).to(dtype).requires_grad_(True)
+    state = torch.randn(4, B, 2 * dh, device=DEV)
+    state[2] = state[2].abs() + 1.0
+    state = state.to(dtype).requires_grad_(True)
+    mask = torch.from_numpy(geometric_reset_mask(1, B, T, 3)).to(DEV).bool()
+    leaves = [x, state, *cell.parameters()]
+    out, _ = cell(x, state, reset_mask=mask)
+    d = torch.randn_like(out)
+    want = torch.autograd.grad(out, leaves, d)
+    for bound in ("KEPT_COEFFICIENT_BYTES", "RECOMPUTED_COEFFICIENT_BYTES"):
+        monkeypatch.setattr(cell_module.F_hip, bound, 36 * T * 2 * dh * 16)
+    out2, _ = cell(x, state, reset_mask=mask)
+    assert torch.equal(out, out2) and "sLSTMCell" not in out2.grad_fn.name()
+    for a, b in zip(want, torch.autograd.grad(out2, leaves, d)):
+        # (row tiles of other heights sum in another order, and bfloat16 deltas round once: 2^-8)
+        tol = 2e-2 if dtype == torch.bfloat16 else 1e-4
+        torch.testing.assert_close(a, b, rtol=tol, atol=tol)

@@ -258,8 +258,8 @@ class sLSTMCell_hip(nn.Module):
     config_class = sLSTMCellConfig
 
     #: Training: let the forward call leave the backward pass its coefficients (36 bytes per step and element, held
-    #: until the backward has run) where it can - bfloat16 inputs, head dim 128 or 256, a batch whose row tiles of 4
-    #: rows fit the device - instead of having the backward pass recompute them in a forward walk of its own.  The
+    #: until the backward has run) up to ``functional.KEPT_COEFFICIENT_BYTES`` instead of having the backward pass run the
+    #: forward once more for them (beyond: bfloat16 at head dim 256 where the row tiles of 4 rows fit the device).  The
     #: reference's native forward always keeps its states and gate values when it trains (slstm.cc:79-108); set this to
     #: False to keep nothing (the memory then goes to the backward call alone).  The gradients are the same either way.
     keep_backward_coefficients: bool = True
@@ -520,7 +520,7 @@ class sLSTMCell_hip(nn.Module):
         if wants_grad and self.keep_backward_coefficients and x.is_cuda and not step:
             if self.head_dim == 256:  # (bfloat16: row tiles of 4 rows x 64 units in the backward, where they fit)
                 coef = F_hip.backward_coefficients_buffer(x, self.config.num_heads)
-            if coef is None:
+            if coef is None and 9 * x.numel() <= F_hip.KEPT_COEFFICIENT_BYTES:
                 coef = F_hip.training_coefficients(x, self.config.num_heads)
                 if coef is not None:
                     h, s = F_hip.slstm_forward(*args, s_out=state_out, workspace=ws, train_coef=coef)
@@ -571,6 +571,7 @@ class sLSTMCell_hip(nn.Module):
         sequences at head dim 256: forward and backward in row tiles of 4 rows x 64 units save 0.07 us a step there
         and take three more launches."""
         return (self.keep_backward_coefficients and F_hip.slstm_backward is _ENGINE_BACKWARD
+                and 9 * input.numel() <= F_hip.KEPT_COEFFICIENT_BYTES
                 and not (self.head_dim == 256 and input.dtype == torch.bfloat16
                          and input.shape[1 if self.config.input_shape == "BSGNH" else 0] >= 384))
 

@@ -103,6 +103,13 @@ def _quad_fits(B: int, T: int, NH: int, dh: int, device) -> bool:
     return groups * (dh // 16) <= cus and groups * (dh // 64) + 8 <= cus
 
 
+#: A training forward leaves the backward pass its coefficients up to this size (of 36 bytes per step and element: 16 rows x
+#: 2048 steps x 1024 units take 1.2 GB), so that a stack of layers that fits without them still fits.  Beyond, the backward
+#: call runs the forward once more, in slices of rows whose coefficients take up to the second size.
+KEPT_COEFFICIENT_BYTES = 4 << 30
+RECOMPUTED_COEFFICIENT_BYTES = 24 << 30
+
+
 def training_coefficients(wx: torch.Tensor, num_heads: int) -> Optional[torch.Tensor]:
     """The tensor a training forward (``slstm_forward(..., train_coef=)``) leaves the backward pass's coefficients in, 36
     bytes per step and element, or ``None`` for calls without a forward kernel (``xs_slstm_train_forward``)."""
@@ -255,13 +262,24 @@ def slstm_backward(
     bf16 = wx.dtype == torch.bfloat16
     if tuple(h_out.shape) != (T, B, H) or tuple(d_h.shape) != (T, B, H):
         raise ValueError(f"h_out and d_h must be [S, B, H] = {(T, B, H)}")
-    if coef is not None and coef.dim() == 1 and coef.numel() != lib.xs_slstm_train_coef_floats(B, T, NH, dh, _DTYPE_CODE[wx.dtype]):
-        raise ValueError("coef must be the tensor that the forward call of the same inputs filled")
     # Unless a kernel is asked for by name: the reverse pass of one launch from a training forward's coefficients.  bf16 at
     # head dim 256 keeps the kernel for row tiles of 4 rows x 64 units (its prefetching workgroups: 1.03 us a step) where it fits
-    if ((coef is None or coef.dim() == 1) and split_override is None and row_tile_override is None and not stepwise_override
-            and not (coef is None and bf16 and dh == 256 and _quad_fits(B, T, NH, dh, wx.device))
-            and lib.xs_slstm_train_coef_floats(B, T, NH, dh, _DTYPE_CODE[wx.dtype])):
+    from_training = ((coef is None or coef.dim() == 1) and split_override is None and row_tile_override is None and not stepwise_override
+                     and not (coef is None and bf16 and dh == 256 and _quad_fits(B, T, NH, dh, wx.device))
+                     and lib.xs_slstm_train_coef_floats(B, T, NH, dh, _DTYPE_CODE[wx.dtype]))
+    if from_training and coef is None and timings is None:
+        rows = max(16, RECOMPUTED_COEFFICIENT_BYTES // (36 * T * H) // 16 * 16)
+        if rows < B:
+            parts = [slstm_backward(wx[b0:b0 + rows], r, bias, None if s0 is None else s0[:, b0:b0 + rows],
+                                    None if reset_mask is None else reset_mask[b0:b0 + rows], h_out[:, b0:b0 + rows],
+                                    d_h[:, b0:b0 + rows], None if d_s_final is None else d_s_final[:, b0:b0 + rows],
+                                    spin_limit=spin_limit, recurrent_cut=recurrent_cut, recurrent_clipval=recurrent_clipval,
+                                    d_wx_dtype=d_wx_dtype, abort_sink=abort_sink) for b0 in range(0, B, rows)]
+            return (torch.cat([q[0] for q in parts], 0), sum(q[1] for q in parts), sum(q[2] for q in parts),
+                    torch.cat([q[3] for q in parts], 1))
+    if coef is not None and coef.dim() == 1 and coef.numel() != lib.xs_slstm_train_coef_floats(B, T, NH, dh, _DTYPE_CODE[wx.dtype]):
+        raise ValueError("coef must be the tensor that the forward call of the same inputs filled")
+    if from_training:
         return _train_backward(lib, wx, r, bias, s0, reset_mask, h_out, d_h, d_s_final, coef, timings, recurrent_cut,
                                recurrent_clipval, d_wx_dtype, spin_limit, abort_sink)
     dh_k = backward_kernel_head_dim(dh, wx.dtype)
