@@ -68,3 +68,41 @@ def test_workspace_of_a_graph_outlives_many_streams(warm):
         for t in held:
             assert t.data_ptr() != ptr and bool((t == 0xA5).all())
     cell.check_status()
+
+
+def test_modules_put_in_the_place_of_a_layers_are_called():
+    """A dropout without a rate, a wrapped cell: the layer runs them as modules."""
+    from xlstm_amd.layer import sLSTMLayer, sLSTMLayerConfig
+
+    print("case replaced modules", flush=True)
+    torch.manual_seed(0)
+    layer = sLSTMLayer(sLSTMLayerConfig(embedding_dim=128, num_heads=2, conv1d_kernel_size=4, backend="hip",
+                                        recurrent_weight_init="standard")).to(DEV, torch.bfloat16).eval()
+    x = torch.randn(2, 6, 128, device=DEV, dtype=torch.bfloat16)
+
+    class Doubled(torch.nn.Module):
+        def forward(self, y):
+            return y * 2
+
+    class Wrapped(torch.nn.Module):
+        def __init__(self, cell):
+            super().__init__()
+            self.inner, self.calls = cell, 0
+
+        def forward(self, *args, **kw):
+            self.calls += 1
+            return self.inner(*args, **kw)
+
+    with torch.no_grad():
+        want = layer(x)
+        layer.dropout = torch.nn.Identity()
+        assert torch.equal(layer(x), want)
+        layer.group_norm.weight.data.fill_(0.25)
+        layer.group_norm.eps, eps = 10.0, layer.group_norm.eps  # (the norm then sees the scale of its input)
+        plain = layer(x)
+        layer.dropout = Doubled()
+        assert not torch.equal(layer(x), plain)
+        layer.dropout, layer.group_norm.eps = torch.nn.Dropout(0.0), eps
+        plain = layer(x)
+        layer.slstm_cell = Wrapped(layer.slstm_cell)
+        assert torch.equal(layer(x), plain) and layer.slstm_cell.calls == 1

@@ -28,7 +28,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from . import functional as hipF
-from .cell import sLSTMCell, sLSTMCellConfig
+from .cell import sLSTMCell, sLSTMCell_hip, sLSTMCellConfig
 
 
 @dataclass
@@ -193,6 +193,11 @@ class sLSTMLayer(nn.Module):
             return hipF.headwise_group_norm(y, self.group_norm.weight, self.group_norm.eps)
         return self.group_norm(y).transpose(1, 2).reshape(B, S, -1)
 
+    def _own_modules(self) -> bool:
+        """Whether cell and dropout are what the constructor made, which the native host path runs without calling them
+        (a wrapper or a subclass put in their place is called)."""
+        return type(self.slstm_cell) is sLSTMCell_hip and type(self.dropout) is nn.Dropout
+
     def _engine_ops_allowed(self, t) -> bool:
         # the engine's kernels record no autograd graph: under grad mode the PyTorch ops run, and a backward pass
         # reaches the cell, which raises (inference engine)
@@ -206,7 +211,7 @@ class sLSTMLayer(nn.Module):
     def forward(self, x: torch.Tensor, conv_state: Optional[torch.Tensor] = None,
                 slstm_state: Optional[torch.Tensor] = None, return_last_state: bool = False,
                 reset_mask: Optional[torch.Tensor] = None, **kwargs):
-        if x.is_cuda:
+        if x.is_cuda and self._own_modules():
             cell = self.slstm_cell
             native = cell._native()
             fast = hipF._lib.host().layer_forward(self, native, x, conv_state, slstm_state, return_last_state, reset_mask)
@@ -249,7 +254,7 @@ class sLSTMLayer(nn.Module):
         ([B,k,D]) receives the new convolution ring and ``out`` ([B,1,D]) the result - both only on the engine's
         bfloat16 path (``_fused``), elsewhere fresh tensors are returned as usual."""
         cell = self.slstm_cell
-        if x.is_cuda and cell._rt.step_plan is not None:
+        if x.is_cuda and self._own_modules() and cell._rt.step_plan is not None:
             fast = hipF._lib.host().layer_step(self, cell._native(), x, conv_state, slstm_state, slstm_state_out, conv_state_out,
                                                h_out, h_prev, out)
             if fast is not None:
