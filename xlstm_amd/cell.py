@@ -212,9 +212,9 @@ class _CellFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, d_h, d_s):
-        x, r, bias, h = ctx.saved_tensors[:4]
-        state = ctx.saved_tensors[4] if ctx.has_state else None
-        coef = ctx.saved_tensors[-1] if len(ctx.saved_tensors) > 4 + ctx.has_state else ctx.coef
+        x, r, bias, h, *more = ctx.saved_tensors  # (once: hooks may refuse to unpack a second time)
+        state = more[0] if ctx.has_state else None
+        coef = more[-1] if len(more) > ctx.has_state else ctx.coef
         NH, dh = ctx.num_heads, r.shape[2]
         d_wx, d_r, d_bias, d_s0 = F_hip.slstm_backward(
             x.detach(), r.detach(), bias.detach().view(NH, 4, dh), None if state is None else state.detach(), ctx.mask,
