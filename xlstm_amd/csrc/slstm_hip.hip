@@ -40,6 +40,7 @@
 #include "slstm_backward_step_kernel.h"
 #include "slstm_step_feed_kernel.h"
 #include "slstm_backward_params_kernel.h"
+#include "slstm_backward_params_slab_kernel.h"
 #include "slstm_serial_bound.h"
 
 // ---------------------------------------------------------------------------
@@ -1023,16 +1024,21 @@ int run_backward_params(const xs_slstm_bwd_args *a) {
     BwdParamParams p;
     p.B = a->B; p.T = a->T; p.NH = a->NH; p.dh = a->dh;
     p.dhp = (a->dh + 63) / 64 * 64;
-    p.d_wx = (const float *)a->d_wx; p.d_wx_sb = a->d_wx_stride_b; p.d_wx_st = a->d_wx_stride_t; p.d_wx_bf16 = dwx_bf16;
+    p.d_wx = (const float *)a->d_wx; p.d_wx_sb = a->d_wx_stride_b; p.d_wx_st = a->d_wx_stride_t;
     p.h_out = a->h_out; p.s0 = a->s0; p.reset = a->reset; p.reset_sb = a->reset_stride_b;
     p.d_r = a->d_r; p.d_bias = a->d_bias;
     p.tchunks = (a->T + kParamKC - 1) / kParamKC;
     const int nt = p.dhp % 256 == 0 ? 256 : (p.dhp % 128 == 0 ? 128 : 64);
-    const int tiles = (4 * p.dhp / kParamMT) * (p.dhp / nt);
+    const bool slab = dwx_bf16 != 0;  // deltas in bf16: the kernel whose operands go straight to LDS
+    const int tiles = (4 * p.dhp / (slab ? kSlabMT : kParamMT)) * (p.dhp / nt);
     const long long nchunks = (long long)a->B * p.tchunks;
-    // slices of K: enough workgroups for two per compute unit, no slice shorter than four chunks
+    if (nchunks > 0x7FFFFFFF - 8) return fail(XS_ERR_UNSUPPORTED, "too many chunks of 32 steps for one launch");
+    // slices of K: enough workgroups for two per compute unit (slab: its LDS takes a compute unit to itself), no slice
+    // shorter than four chunks
     const int cus = device_cus() > 0 ? device_cus() : 256;
-    long long ks = (2ll * cus + (long long)a->NH * tiles - 1) / ((long long)a->NH * tiles);  // (4 or 8 per compute unit: 10 to 30 % slower)
+    const long long base = (long long)a->NH * tiles;
+    long long ks = slab ? cus / base : (2ll * cus + base - 1) / base;  // (4 or 8 per compute unit: 10 to 30 % slower)
+    if (ks < 1) ks = 1;
     // (head, slice) groups are dealt out over the XCDs, group i on XCD i % 8: a multiple of 8 of them keeps every XCD
     // busy (4 heads of 1024 are 512 tiles and one slice each by the rule above: four XCDs idle, twice the time)
     while ((a->NH * ks) % 8 != 0 && a->NH * ks < 64) ++ks;
@@ -1045,7 +1051,11 @@ int run_backward_params(const xs_slstm_bwd_args *a) {
     void (*kern)(BwdParamParams);
     if (bf16) kern = nt == 256 ? slstm_bwd_param_kernel<true, 256> : (nt == 128 ? slstm_bwd_param_kernel<true, 128> : slstm_bwd_param_kernel<true, 64>);
     else kern = nt == 256 ? slstm_bwd_param_kernel<false, 256> : (nt == 128 ? slstm_bwd_param_kernel<false, 128> : slstm_bwd_param_kernel<false, 64>);
-    const size_t lds = (size_t)bwd_param_lds_bytes(bf16, nt);
+    size_t lds = (size_t)bwd_param_lds_bytes(bf16, nt);
+    if (slab) {
+      kern = nt == 256 ? slstm_bwd_param_slab_kernel<256> : (nt == 128 ? slstm_bwd_param_slab_kernel<128> : slstm_bwd_param_slab_kernel<64>);
+      lds = (size_t)param_slab_lds_bytes(nt);
+    }
     if (lds > 64 * 1024) {
       const int rc = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds);
       if (rc != XS_OK) return rc;
