@@ -32,6 +32,7 @@
 #include "slstm_seq_roles_kernel.h"
 #include "slstm_step_kernel.h"
 #include "slstm_step_pipe_kernel.h"
+#include "slstm_step_small_kernel.h"
 #include "slstm_backward_kernels.h"
 #include "slstm_layer_kernels.h"
 #include "slstm_local_kernel.h"
@@ -224,6 +225,22 @@ int run_step(const xs_slstm_args *a) {
   p.spin_limit = a->spin_limit > 0 ? (a->spin_limit < (1ll << 30) ? (int)a->spin_limit : (1 << 30)) : (1 << 22);
   const long long nwg = (long long)NH * p.n_unit_tiles * p.n_row_tiles;
   if (nwg > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many tiles for one step launch");
+  // Small batches: workgroups of 16 rows x 16 units (slstm_step_small_kernel.h), as long as there are at most so many of
+  // them per compute unit; beyond, what every row tile reads of R costs more than the other kernels' longer way.  us a step
+  // replayed from a graph, this kernel / the others, on either side of the line: bf16 4 heads of 512, 64 rows (2 per compute unit) 8.3 / 10.5,
+  // 80 rows 10.7 / 10.5; 8 heads of 256, 64 rows (2) 5.0 / 5.5, 128 rows 8.0 / 6.0; 4 heads of 1024, 16 rows (1) 7.8 / 9.9, 32 rows
+  // 12.6 / 11.0; float32 4 heads of 256, 256 rows (4) 14.7 / 16.6, 512 rows 24.0 / 17.4.
+  const int small_rows = (B + 15) / 16, small_units = (dh + 15) / 16;
+  if ((long long)NH * small_units * small_rows <= (long long)device_cus() * (bf16 ? (nch == 8 ? 1 : 2) : 4)) {
+    p.n_unit_tiles = small_units;
+    p.n_row_tiles = small_rows;
+    p.h_prev = bf16 && a->s0 && !a->reset ? a->h_prev : nullptr;
+    void (*k)(StepParams) = bf16 ? (p.h_prev ? pick_step_small<true, true>(nch) : pick_step_small<true, false>(nch)) : pick_step_small<false, false>(nch);
+    hipLaunchKernelGGL(k, dim3((unsigned)(NH * p.n_unit_tiles * p.n_row_tiles)), dim3(256), 0, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(XS_ERR_LAUNCH, "step kernel launch failed: %s", hipGetErrorString(e));
+    return XS_OK;
+  }
   const dim3 grid((unsigned)nwg);
   int nch_log2 = 0;
   while ((1 << nch_log2) < nch) ++nch_log2;
