@@ -198,7 +198,7 @@ class _CellFunction(torch.autograd.Function):
     """Joins the results of a forward call of the engine to the autograd graph.  The backward runs the engine's two
     backward kernels (``functional.slstm_backward``): the gradient by the rule of the reference's native kernel
     (``slstm_pointwise.cu:118-196``; what ``sLSTMFunc.backward`` returns, ``slstm.cc:137-304``).  ``h`` and ``s`` are
-    what the forward call returned for ``x, r, bias, state, mask``; nothing else is stored for the backward."""
+    what the forward call returned for ``x, r, bias, state, mask``; beside them only ``coef`` is stored, where there is one."""
 
     @staticmethod
     def forward(ctx, x, r, bias, state, h, s, mask, num_heads, cut, clipval, coef, abort_sink):
