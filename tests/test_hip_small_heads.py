@@ -65,3 +65,33 @@ def test_small_heads_against_the_oracles(bf16, B, T, NH, dh, masked, opts):
     if bf16:
         short = F.slstm_backward(wx_t, r_t, b_t, s0_t, m_t, h, d_h_t, torch.from_numpy(d_sf).to(DEV), coef=coef, d_wx_dtype=dt, **opts)
         assert torch.equal(short[0], got[0].to(dt)) and torch.equal(short[3], got[3])
+
+
+@pytest.mark.parametrize("bf16,B,NH,dh", [(True, 64, 40, 128), (True, 33, 33, 128), (True, 40, 72, 64), (False, 40, 72, 64), (True, 65, 129, 24)])
+def test_more_heads_than_one_launch_holds(bf16, B, NH, dh):
+    """The heads in front run in the kernel of four row tiles, the last few in one compute unit each: every head against the
+    oracle and bit for bit against the step kernel."""
+    from xlstm_amd import functional as F
+
+    print("case heads in several launches", bf16, B, NH, dh, flush=True)
+    T = 4
+    wx, r, b, s0 = make_problem(700 + dh, B, T, NH, dh, rscale=2.0, bf16=bf16, with_state=True)
+    reset = geometric_reset_mask(dh, B, T, 3)
+    if bf16:
+        r = torch.from_numpy(r).bfloat16().float().numpy()
+    dt = torch.bfloat16 if bf16 else torch.float32
+    wx_t = torch.from_numpy(wx).to(DEV).to(dt)
+    r_t, b_t = r_ext_to_kernel(torch.from_numpy(r)).to(DEV), torch.from_numpy(b).to(DEV)
+    s0_t, m_t = torch.from_numpy(s0).to(DEV), torch.from_numpy(reset).to(DEV)
+    ws = F.workspace_for(B, T, NH, dh, DEV)
+    h, s = F.slstm_forward(wx_t, r_t, b_t, s0_t, m_t, workspace=ws)
+    status = F.read_status(ws)
+    assert status["launches"] > 1 and status["rows_per_workgroup"] == 4 and status["aborted"] == 0, status
+    st = s0_t
+    for t in range(T):
+        ht, st = F.slstm_forward(wx_t[:, t:t + 1], r_t.to(dt), b_t, st, m_t[:, t:t + 1], step=True)
+        assert torch.equal(ht[0], h[t]), t
+    assert torch.equal(st, s)
+    h_ref, s_ref = so.slstm_forward(wx, r, b, s0, reset)
+    tol = 2e-2 if bf16 else 1e-5
+    assert max_err(h.float().cpu().numpy(), h_ref) <= tol and max_err(s.cpu().numpy(), s_ref) <= tol

@@ -359,17 +359,18 @@ void (*pick_local_bwd(int w))(LocalBwdParams) {
 // workgroups of a launch over (row tile of 4 rows, head) pairs: a multiple of 8 (one range per XCD)
 inline long long local_grid(int B, int NH) { return ((long long)((B + 3) / 4) * NH + 7) / 8 * 8; }
 
-int run_local(const xs_slstm_args *a, float *coef) {
+// heads head0 .. NH - 1 (head0 > 0: behind launches of other kernels for the heads in front)
+int run_local(const xs_slstm_args *a, float *coef, int head0 = 0) {
   const bool bf16 = a->wx_dtype == XS_BF16;
   const int w = local_waves(a->dh);
-  const long long grid = local_grid(a->B, a->NH);
+  const long long grid = local_grid(a->B, a->NH - head0);
   if (grid > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many row tiles for one launch");
   LocalParams p;
   p.wx = a->wx; p.wx_sb = a->wx_stride_b; p.wx_st = a->wx_stride_t;
   p.r = a->r; p.r_bf16 = a->r_dtype == XS_BF16;
   p.bias = a->bias; p.s0 = a->s0; p.reset = a->reset; p.reset_sb = a->reset_stride_b;
   p.h_out = a->h_out; p.s_out = a->s_out; p.status = (xs_slstm_status *)a->workspace; p.coef = coef;
-  p.B = a->B; p.T = a->T; p.NH = a->NH; p.dh = a->dh;
+  p.B = a->B; p.T = a->T; p.NH = a->NH; p.dh = a->dh; p.head0 = head0;
   void (*k)(LocalParams);
   if (coef) k = bf16 ? pick_local<true, true>(w) : pick_local<false, true>(w);
   else k = bf16 ? pick_local<true, false>(w) : pick_local<false, false>(w);
@@ -503,7 +504,8 @@ int run_train_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_s
   return e == hipSuccess ? XS_OK : fail(XS_ERR_LAUNCH, "backward kernel launch failed: %s", hipGetErrorString(e));
 }
 
-// need != nullptr: launch nothing, only report the bytes of workspace the launches of this call touch
+// need != nullptr: launch nothing, only say whether a kernel takes every launch of this call and how many bytes of
+// workspace they touch
 int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_host = nullptr, float *train_coef = nullptr) {
   hipStream_t stream = (hipStream_t)a->stream;
   const int B = a->B, T = a->T, NH = a->NH, dh = a->dh;
@@ -548,6 +550,11 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
   // Heads are independent (block-diagonal R): when the groups of all heads do not fit at once, the heads go in
   // several launches, as many per launch as fit.
   const int heads_per_launch = NH < capacity ? NH : capacity;
+  if (!dry && heads_per_launch < NH) {  // a call is refused as a whole: no slice of heads after another has been launched
+    size_t bytes = 0;
+    const int rc = run_forward(a, &bytes, nullptr, train_coef);
+    if (rc != XS_OK) return rc;
+  }
   int launch_no = 0;
   for (int head0 = 0; head0 < NH; head0 += heads_per_launch) {
   const int NHL = head0 + heads_per_launch <= NH ? heads_per_launch : NH - head0;
@@ -567,9 +574,10 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
                              (!a->reset || 4ll * a->reset_stride_b < 0xFFFFFF00ll) && 16ll * NH * dh * esz < (1ll << 31);
     if (MT == 4 && !offsets_fit) MT = 2;
   }
-  // small heads stay in one compute unit, the whole call in one launch (nothing waits, so nothing has to be resident
-  // at once), unless the batch is one for the kernel of four row tiles
-  if (head0 == 0 && MT < 4 && !a->coef_out && !train_coef && local_head(dh, bf16)) return dry ? XS_OK : run_local(a, nullptr);
+  // small heads stay in one compute unit, all heads that are left in one launch (nothing waits, so nothing has to be
+  // resident at once), unless the batch is one for the kernel of four row tiles.  (The slices of heads but the last are of
+  // one size: where the first goes to that kernel, a last one of fewer heads may still come here.)
+  if (MT < 4 && !a->coef_out && !train_coef && local_head(dh, bf16)) return dry ? XS_OK : run_local(a, nullptr, head0);
   int rows_per_wg = 16 * MT;
   if (MT == 1) {  // spare compute units: smaller row tiles, smaller exchanges
     for (int r = 4; r < 16; r *= 2)
@@ -615,15 +623,15 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
     if (!kern) return fail(XS_ERR_UNSUPPORTED, "no kernel for nch=%d MT=%d", nch, MT);
     const int NBT = (bend - b0 + rows_per_wg - 1) / rows_per_wg;
     const int ngroups = NHL * NBT;
+    // grid shapes of the three placements the kernel knows: one XCD per group, two XCDs per group, spread
+    const int grid = G <= 32 ? 8 * G * ((ngroups + 7) / 8)
+                             : ((G <= 64 && G % 2 == 0) ? 8 * (G / 2) * ((ngroups + 3) / 4) : ngroups * G);
+    if (grid > kMaxWg) return fail(XS_ERR_UNSUPPORTED, "grid %d too large", grid);
     if (dry) {
       const size_t ring = (size_t)kRing * ngroups * G * 16 * MT * 16 * (bf16 ? 2 : 4);
       if (kHeaderBytes + ring > *need) *need = kHeaderBytes + ring;
       continue;
     }
-    // grid shapes of the three placements the kernel knows: one XCD per group, two XCDs per group, spread
-    const int grid = G <= 32 ? 8 * G * ((ngroups + 7) / 8)
-                             : ((G <= 64 && G % 2 == 0) ? 8 * (G / 2) * ((ngroups + 3) / 4) : ngroups * G);
-    if (grid > kMaxWg) return fail(XS_ERR_UNSUPPORTED, "grid %d too large", grid);
     {  // every word of the exchange ring starts as "not written yet"; the status block and the placement words are clear
        // (a later launch of the call: the placement words alone, what the earlier ones said in the status block stays)
       const size_t words = (size_t)kRing * ngroups * G * 16 * MT * 16 * (bf16 ? 2 : 4) / 4;

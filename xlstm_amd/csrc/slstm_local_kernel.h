@@ -50,6 +50,7 @@ struct LocalParams {
   xs_slstm_status *status;   // or null
   float *coef;               // COEF: [T][ceil(B/4)][NH][waves][{64 lanes x 4}, {64 x 4}, {64 x 1}]: coefficients 0-3, 4-7, 8
   int B, T, NH, dh;
+  int head0;                 // the heads of this launch: head0 .. NH - 1
 };
 
 struct LocalBwdParams {
@@ -91,7 +92,8 @@ __global__ __launch_bounds__(64 * W) void slstm_local_kernel(LocalParams p) {
 
   int head, tile;
   const int ntiles = (p.B + 3) >> 2;
-  if (!local_place(ntiles * p.NH, p.NH, head, tile)) return;  // the whole workgroup leaves before any barrier
+  if (!local_place(ntiles * (p.NH - p.head0), p.NH - p.head0, head, tile)) return;  // the whole workgroup leaves before any barrier
+  head += p.head0;
   const int tid = threadIdx.x, lane = tid & 63, wave = (int)uniform((uint32_t)(tid >> 6));
   const int b = lane >> 4, n = lane & 15;
   const int dh = p.dh, H = p.NH * dh;
@@ -100,7 +102,12 @@ __global__ __launch_bounds__(64 * W) void slstm_local_kernel(LocalParams p) {
   const bool mine = a < dh && brow < p.B;
   const int ac = a < dh ? a : dh - 1, bc = brow < p.B ? brow : p.B - 1;
   const long long so = (long long)bc * H + head * dh + ac;
-  if (p.status && blockIdx.x == 0 && tid < 16) reinterpret_cast<uint32_t *>(p.status)[tid] = tid == 5 ? 1u : (tid == 7 ? 4u : 0u);
+  if (p.status && blockIdx.x == 0 && tid < 16) {
+    uint32_t *const word = reinterpret_cast<uint32_t *>(p.status) + tid;
+    if (p.head0 == 0) *word = tid == 5 ? 1u : (tid == 7 ? 4u : 0u);
+    else if (tid == 5) *word += 1u;  // (behind the launches of the heads in front: what they said stays)
+    else if (tid == 7) *word = 4u;
+  }
 
   // ---- R: bf16: column n of gate g is unit 16 w + n, k-step ks, lane group q = b: inputs 32 ks + 8 q .. + 7
   //      float32: lane (quarter kq = b, column n): inputs kq KW .. + KW - 1 of its unit's row
