@@ -106,3 +106,43 @@ def test_modules_put_in_the_place_of_a_layers_are_called():
         plain = layer(x)
         layer.slstm_cell = Wrapped(layer.slstm_cell)
         assert torch.equal(layer(x), plain) and layer.slstm_cell.calls == 1
+
+
+@pytest.mark.parametrize("module,method,where", [
+    (module, method, where) for module, method in (("slstm_cell", "forward"), ("slstm_cell", "step"), ("dropout", "forward"))
+    for where in ("instance", "class", "compiled") if (method, where) != ("step", "compiled")])
+def test_methods_put_in_the_place_of_a_modules_are_called(monkeypatch, module, method, where):
+    """A layer calls a ``forward`` or ``step`` that was replaced on its cell or dropout, or on their class, and a module that
+    was compiled in place - behind calls that went through the native host path."""
+    from xlstm_amd.layer import sLSTMLayer, sLSTMLayerConfig
+
+    print("case replaced method", where, module, method, flush=True)
+    torch.manual_seed(0)
+    layer = sLSTMLayer(sLSTMLayerConfig(embedding_dim=128, num_heads=2, conv1d_kernel_size=4, backend="hip",
+                                        recurrent_weight_init="standard")).to(DEV, torch.bfloat16).eval()
+    layer.slstm_cell.keep_state_fp32 = True
+    x = torch.randn(2, 6, 128, device=DEV, dtype=torch.bfloat16)
+    calls = []
+
+    def run():
+        with torch.no_grad():
+            out, states = layer(x[:, :4], return_last_state=True)
+            outs = [out]
+            for t in (4, 5):
+                out, states = layer.step(x[:, t:t + 1].contiguous(), **states)
+                outs.append(out)
+        return torch.cat(outs, 1)
+
+    want = run()
+    target = getattr(layer, module)
+    if where == "compiled":  # what Module.compile leaves on the module
+        plain = target._call_impl
+        target._compiled_call_impl = lambda *a, **kw: (calls.append(1), plain(*a, **kw))[1]
+    elif where == "instance":
+        plain = getattr(target, method)
+        setattr(target, method, lambda *a, **kw: (calls.append(1), plain(*a, **kw))[1])
+    else:
+        plain = getattr(type(target), method)
+        monkeypatch.setattr(type(target), method, lambda self, *a, **kw: (calls.append(1), plain(self, *a, **kw))[1])
+    # (the dropout runs behind the sequence and behind every step, the cell's forward and step once per call of that kind)
+    assert torch.equal(run(), want) and len(calls) == {"forward": 3 if module == "dropout" else 1, "step": 2}[method]

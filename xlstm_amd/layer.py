@@ -151,6 +151,11 @@ class MultiHeadLayerNorm(nn.Module):
         return out.view(B, S, NH, DH).transpose(1, 2)
 
 
+# the methods that the native host path of a layer stands in for, and what replaces them in a module's own dictionary
+_STOOD_IN_FOR = (sLSTMCell_hip.forward, sLSTMCell_hip.step, nn.Dropout.forward)
+_REPLACEABLE = frozenset(("forward", "step", "_compiled_call_impl"))
+
+
 class sLSTMLayer(nn.Module):
     config_class = sLSTMLayerConfig
 
@@ -194,9 +199,13 @@ class sLSTMLayer(nn.Module):
         return self.group_norm(y).transpose(1, 2).reshape(B, S, -1)
 
     def _own_modules(self) -> bool:
-        """Whether cell and dropout are what the constructor made, which the native host path runs without calling them
-        (a wrapper or a subclass put in their place is called)."""
-        return type(self.slstm_cell) is sLSTMCell_hip and type(self.dropout) is nn.Dropout
+        """Whether cell and dropout are what the constructor made, which the native host path runs without calling them (a
+        wrapper or a subclass in their place, a method replaced on the module or its class, a module compiled in place
+        is called)."""
+        cell, dropout = self.slstm_cell, self.dropout
+        return (type(cell) is sLSTMCell_hip and type(dropout) is nn.Dropout
+                and _REPLACEABLE.isdisjoint(cell.__dict__) and _REPLACEABLE.isdisjoint(dropout.__dict__)
+                and (sLSTMCell_hip.forward, sLSTMCell_hip.step, nn.Dropout.forward) == _STOOD_IN_FOR)
 
     def _engine_ops_allowed(self, t) -> bool:
         # the engine's kernels record no autograd graph: under grad mode the PyTorch ops run, and a backward pass
