@@ -155,3 +155,25 @@ def test_cell_can_be_copied_and_pickled():
         assert torch.equal(other.recurrent_kernel[:], c.recurrent_kernel[:]) and torch.equal(other.bias[:], c.bias[:])
         other.bias[0, 1] = torch.zeros(16)
         assert not torch.equal(other.bias[:], c.bias[:])
+
+
+def test_a_cell_in_a_cycle_is_collected():
+    """A hook on a parameter whose closure refers to the module: a cycle through the native host path's reference to the
+    cell's parameters, which the collector has to see."""
+    import gc
+    import weakref
+
+    from xlstm_amd import _lib
+
+    cell = _cell(hidden_size=16, num_heads=2)
+    native = cell._native()
+    assert gc.is_tracked(native) and cell._parameters in gc.get_referents(native)
+    cell._bias_.register_hook(lambda grad, cell=cell: grad)
+    gone = weakref.ref(cell)
+    del cell, native
+    gc.collect()
+    assert gone() is None
+    # a path without parameters (as the collector leaves one to finalizers): nothing runs, nothing crashes
+    path = _lib.host().CellPath({}, 2, 8)
+    x = torch.zeros(1, 3, 64)
+    assert path.step(x[:, :1], x, None, None, None, None, None, False) is None and path.poll(False) is False

@@ -148,8 +148,9 @@ struct CellPath {
   AbortWord abort_word;
   uint64_t devices_used = 0;
 
+  PyObject *parameter_object(PyObject *name) const { return parameters ? PyDict_GetItem(parameters, name) : nullptr; }  // borrowed
   const at::Tensor &parameter(PyObject *name) const {
-    PyObject *o = PyDict_GetItem(parameters, name);
+    PyObject *o = parameter_object(name);
     if (!o) throw NotCovered{};
     return tensor_of(o);
   }
@@ -289,7 +290,7 @@ bool plan_fits(const CellPath &c, PyObject *x, PyObject *state) {
   if (!c.plan || !THPVariable_Check(x) || !THPVariable_Check(state)) return false;
   const at::Tensor &s = THPVariable_Unpack(state);
   if (s.scalar_type() != at::kFloat || s.dim() != 3 || s.size(1) != c.step_B) return false;
-  PyObject *ro = PyDict_GetItem(c.parameters, g_names.r), *bo = PyDict_GetItem(c.parameters, g_names.b);
+  PyObject *ro = c.parameter_object(g_names.r), *bo = c.parameter_object(g_names.b);
   if (!ro || !bo || !THPVariable_Check(ro) || !THPVariable_Check(bo)) return false;
   const at::Tensor &r = THPVariable_Unpack(ro), &b = THPVariable_Unpack(bo);
   return r.data_ptr() == c.r_ptr && b.data_ptr() == c.b_ptr && version_of(r) == c.r_version && version_of(b) == c.b_version &&
@@ -297,7 +298,7 @@ bool plan_fits(const CellPath &c, PyObject *x, PyObject *state) {
 }
 bool recording(const CellPath &c, PyObject *x, PyObject *state) {
   if (!at::GradMode::is_enabled()) return false;
-  PyObject *ro = PyDict_GetItem(c.parameters, g_names.r), *bo = PyDict_GetItem(c.parameters, g_names.b);
+  PyObject *ro = c.parameter_object(g_names.r), *bo = c.parameter_object(g_names.b);
   if (!ro || !bo || !THPVariable_Check(ro) || !THPVariable_Check(bo) || !THPVariable_Check(x)) return true;
   return c.records(THPVariable_Unpack(x), !absent(state) && THPVariable_Check(state) ? &THPVariable_Unpack(state) : nullptr, THPVariable_Unpack(ro), THPVariable_Unpack(bo));
 }
@@ -589,15 +590,14 @@ PyObject *cell_call(PyObject *self, PyObject *const *args, Py_ssize_t n) {
 // set_plan(plan, address of its argument block, B, r, b): the next steps of that batch size and of these parameters
 PyObject *cell_set_plan_(CellPath &c, PyObject *const *args) {
   const at::Tensor &r = tensor_of(args[3]), &b = tensor_of(args[4]);
-  Py_INCREF(args[0]);
-  Py_XDECREF(c.plan);
-  c.plan = args[0];
   c.step_args = (xs_slstm_args *)PyLong_AsVoidPtr(args[1]);
   c.step_B = PyLong_AsLongLong(args[2]);
   c.step_dtype = c.step_args->wx_dtype == XS_BF16 ? at::kBFloat16 : at::kFloat;
   c.device = r.device();
   c.r_ptr = r.data_ptr(); c.b_ptr = b.data_ptr();
   c.r_version = version_of(r); c.b_version = version_of(b);
+  Py_INCREF(args[0]);
+  Py_XSETREF(c.plan, args[0]);
   Py_RETURN_NONE;
 }
 // workspace(B, a tensor on the device) -> the workspace of calls on that device's current stream
@@ -637,8 +637,28 @@ PyObject *cell_new(PyTypeObject *type, PyObject *args, PyObject *) {
   self->c->NH = NH; self->c->dh = dh;
   return (PyObject *)self;
 }
+// (the parameters' hooks may refer to the cell, which holds this path: the collector has to see through it)
+int cell_traverse(PyObject *self, visitproc visit, void *arg) {
+  CellPath *c = ((CellPathObject *)self)->c;
+  Py_VISIT(Py_TYPE(self));
+  if (c) {
+    Py_VISIT(c->parameters);
+    Py_VISIT(c->plan);
+  }
+  return 0;
+}
+int cell_clear(PyObject *self) {
+  CellPath *c = ((CellPathObject *)self)->c;
+  if (c) {
+    c->step_args = nullptr;  // (the plan's)
+    Py_CLEAR(c->parameters);
+    Py_CLEAR(c->plan);
+  }
+  return 0;
+}
 void cell_dealloc(PyObject *self) {
   PyTypeObject *type = Py_TYPE(self);
+  PyObject_GC_UnTrack(self);
   delete ((CellPathObject *)self)->c;
   type->tp_free(self);
   Py_DECREF(type);
@@ -653,8 +673,9 @@ PyMethodDef cell_methods[] = {
     {"last_workspace", (PyCFunction)(void *)cell_call<cell_last_workspace_, 0>, METH_FASTCALL, nullptr},
     {"poll", (PyCFunction)(void *)cell_call<cell_poll_, 1>, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
-PyType_Slot cell_slots[] = {{Py_tp_new, (void *)cell_new}, {Py_tp_dealloc, (void *)cell_dealloc}, {Py_tp_methods, cell_methods}, {0, nullptr}};
-PyType_Spec cell_spec = {"_xlstm_host.CellPath", sizeof(CellPathObject), 0, Py_TPFLAGS_DEFAULT, cell_slots};
+PyType_Slot cell_slots[] = {{Py_tp_new, (void *)cell_new}, {Py_tp_dealloc, (void *)cell_dealloc},
+                            {Py_tp_traverse, (void *)cell_traverse}, {Py_tp_clear, (void *)cell_clear}, {Py_tp_methods, cell_methods}, {0, nullptr}};
+PyType_Spec cell_spec = {"_xlstm_host.CellPath", sizeof(CellPathObject), 0, Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC, cell_slots};
 PyTypeObject *g_cell_type = nullptr;
 
 // ---- one layer: its submodules are looked up by name in the module dictionaries on every call (they may be replaced)
