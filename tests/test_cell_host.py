@@ -177,3 +177,78 @@ def test_a_cell_in_a_cycle_is_collected():
     path = _lib.host().CellPath({}, 2, 8)
     x = torch.zeros(1, 3, 64)
     assert path.step(x[:, :1], x, None, None, None, None, None, False) is None and path.poll(False) is False
+
+
+_COUNTER = r"""
+#include <dlfcn.h>
+static int thrown;
+void __cxa_throw(void *object, void *type, void (*destructor)(void *)) {
+  ++thrown;
+  ((void (*)(void *, void *, void (*)(void *)))dlsym(dlopen("libstdc++.so.6", RTLD_NOW), "__cxa_throw"))(object, type, destructor);
+}
+int count_thrown(void) { int n = thrown; thrown = 0; return n; }
+"""
+
+_CALLS = r"""
+import ctypes, sys
+counter = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # (in front of every library that throws)
+import torch
+from xlstm_amd import _lib
+from xlstm_amd.cell import sLSTMCell, sLSTMCellConfig
+from xlstm_amd.layer import sLSTMLayer, sLSTMLayerConfig
+
+host = _lib.host()
+
+def layer_calls(dtype=torch.bfloat16, dh=64, T=3, hook=False, **kw):
+    layer = sLSTMLayer(sLSTMLayerConfig(embedding_dim=2 * dh, num_heads=2, backend="hip", **kw)).to(dtype)
+    if hook:
+        layer.slstm_cell.register_forward_hook(lambda *a: None)
+    x = torch.zeros(2, T, 2 * dh, dtype=dtype)
+    with torch.no_grad():
+        native = layer.slstm_cell._native()
+        assert host.layer_forward(layer, native, x, None, None, True, None) is None
+        assert host.layer_step(layer, native, x[:, :1], None, torch.zeros(4, 2, 2 * dh), None, None, None, None, None) is None
+
+def cell_calls(x, state=None, mask=None, **kw):
+    cell = sLSTMCell(sLSTMCellConfig(hidden_size=32, num_heads=2, backend="hip", **kw))
+    native = cell._native()
+    for grad in (False, True):
+        with torch.set_grad_enabled(grad):
+            assert native.forward(x, state, mask, cell.config, False) is None
+            assert native.train(x, state, mask, cell.config, False) is None
+            assert native.step(x, state, mask, None, None, None, cell.config, False) is None
+
+try:  # (an error of the library's own throws: the counter counts)
+    torch.empty(1).reshape(2)
+except RuntimeError:
+    pass
+assert counter.count_thrown() > 0
+layer_calls(), layer_calls(torch.float32), layer_calls(dh=48), layer_calls(T=1), layer_calls(conv1d_kernel_size=0), layer_calls(dropout=0.5)
+layer_calls(conv1d_kernel_size=6), layer_calls(group_norm_weight=False), layer_calls(output_shape="SBH"), layer_calls(hook=True)
+x = torch.zeros(3, 4, 128)
+state = torch.zeros(4, 3, 32)
+cell_calls(x), cell_calls(x.half()), cell_calls(x.bfloat16(), state.bfloat16()), cell_calls(x[:, :1], state), cell_calls(x, state, torch.zeros(3, 4))
+cell_calls(x.double(), input_shape="SBGNH"), cell_calls(x[0]), cell_calls(x[:, :1], state, input_shape="SBGNH"), cell_calls(x[:, :0])
+cell_calls(x, output_shape="nope"), cell_calls(x, state, 3), cell_calls(x, "state")
+print("thrown", counter.count_thrown())
+"""
+
+
+def test_calls_of_the_general_path_cost_no_exception(tmp_path):
+    """Half precision, other head dims, no convolution, dropout, one-token calls, other layouts: the native host path says
+    that it does not cover them by a return value."""
+    import os
+    import shutil
+    import subprocess
+    import sys
+
+    from tests.conftest import ROOT
+
+    if shutil.which("gcc") is None:
+        pytest.skip("needs a C compiler")
+    source, counter = tmp_path / "counter.c", tmp_path / "libcounter.so"
+    source.write_text(_COUNTER)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-w", "-o", str(counter), str(source), "-ldl"], check=True)
+    res = subprocess.run([sys.executable, "-c", _CALLS, str(counter)], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
+                         timeout=300, env=dict(os.environ, PYTHONPATH=ROOT))
+    assert res.returncode == 0 and "thrown 0" in res.stdout, res.stdout

@@ -4,8 +4,10 @@
 // layer call there, more than the kernels run; here it takes about 4 and 8.
 //
 // Every function returns None, with nothing launched, for a call that is not one of those it covers (autograd is
-// recording, hooks are registered, another dtype or layout ...): the caller then takes its general path.  The results
-// are those of the general path: the same kernels with the same arguments.
+// recording, hooks are registered, another dtype or layout ...): the caller then takes its general path.  That is looked at
+// in front of everything else and said by return values: an exception costs 7 us and more in a process with as many
+// libraries as this one, and programs whose calls all take the general path pay for it on every one.  The results are
+// those of the general path: the same kernels with the same arguments.
 //
 // A plain CPython extension over ATen (no pybind11: its argument casters cost as much as the rest of a step call).
 // The engine's C entry points come as addresses from the library that _lib.py has loaded, so that one loaded engine
@@ -66,19 +68,19 @@ struct PyRef {  // owns one reference
   PyObject *release() { PyObject *p = o; o = nullptr; return p; }
 };
 
-struct PythonError {};                                   // a Python exception is set
-struct NotCovered {};                                    // the general path takes this call
+struct PythonError {};  // a Python exception is set
 [[noreturn]] void engine_failed(int rc) {
   PyErr_Format(g_engine.error, "xlstm_amd error %d: %s", rc, g_engine.last_error());
   throw PythonError{};
 }
 inline void launched(int rc) { if (rc != XS_OK) engine_failed(rc); }
 
-inline const at::Tensor &tensor_of(PyObject *o) {
-  if (!THPVariable_Check(o)) throw NotCovered{};
-  return THPVariable_Unpack(o);
-}
+inline const at::Tensor *tensor_of(PyObject *o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }  // or null
 inline bool absent(PyObject *o) { return o == nullptr || o == Py_None; }
+inline bool optional_tensor(PyObject *o, const at::Tensor *&t) {  // false: neither a tensor nor None
+  t = absent(o) ? nullptr : tensor_of(o);
+  return t || absent(o);
+}
 
 inline void *stream_of(const at::Device &d) { return (void *)c10::hip::getCurrentHIPStream(d.index()).stream(); }
 inline int dtype_code(at::ScalarType t) { return t == at::kBFloat16 ? XS_BF16 : XS_F32; }
@@ -148,11 +150,9 @@ struct CellPath {
   AbortWord abort_word;
   uint64_t devices_used = 0;
 
-  PyObject *parameter_object(PyObject *name) const { return parameters ? PyDict_GetItem(parameters, name) : nullptr; }  // borrowed
-  const at::Tensor &parameter(PyObject *name) const {
-    PyObject *o = parameter_object(name);
-    if (!o) throw NotCovered{};
-    return tensor_of(o);
+  bool weights(const at::Tensor *&r, const at::Tensor *&b) const {
+    PyObject *ro = parameters ? PyDict_GetItem(parameters, g_names.r) : nullptr, *bo = parameters ? PyDict_GetItem(parameters, g_names.b) : nullptr;
+    return ro && bo && (r = tensor_of(ro)) && (b = tensor_of(bo));
   }
   ~CellPath() {
     Py_XDECREF(parameters);
@@ -202,16 +202,17 @@ struct CellPathObject { PyObject_HEAD CellPath *c; };
 
 // the config's output_shape as the strides of [S,B,H] memory: 'BNSH', 'SBH', 'BSH' or 'SBNH'
 enum class OutShape { BNSH, SBH, BSH, SBNH };
-OutShape out_shape(PyObject *config) {
+bool out_shape(PyObject *config, OutShape &shape) {
   PyRef v(PyObject_GetAttr(config, g_names.output_shape));
   if (!v.o) throw PythonError{};
   const char *s = PyUnicode_Check(v.o) ? PyUnicode_AsUTF8(v.o) : nullptr;
-  if (!s) { PyErr_Clear(); throw NotCovered{}; }
-  if (!strcmp(s, "BNSH")) return OutShape::BNSH;
-  if (!strcmp(s, "SBH")) return OutShape::SBH;
-  if (!strcmp(s, "BSH")) return OutShape::BSH;
-  if (!strcmp(s, "SBNH")) return OutShape::SBNH;
-  throw NotCovered{};
+  if (!s) { PyErr_Clear(); return false; }
+  if (!strcmp(s, "BNSH")) shape = OutShape::BNSH;
+  else if (!strcmp(s, "SBH")) shape = OutShape::SBH;
+  else if (!strcmp(s, "BSH")) shape = OutShape::BSH;
+  else if (!strcmp(s, "SBNH")) shape = OutShape::SBNH;
+  else return false;
+  return true;
 }
 struct Shape4 { std::array<int64_t, 4> size, stride; int n; };
 Shape4 shape_of(OutShape o, int64_t S, int64_t B, int64_t NH, int64_t dh) {
@@ -230,37 +231,42 @@ bool input_is_bsgnh(PyObject *config) {
 }
 
 // ---- one decode step into given buffers; the plan and the operand hint as sLSTMCell_hip._step_fast chooses them
+struct StepBuffers { const at::Tensor *state_out = nullptr, *h_out = nullptr, *h_prev = nullptr; };
+bool step_buffers(PyObject *state_out, PyObject *h_out, PyObject *h_prev, StepBuffers &s) {
+  return optional_tensor(state_out, s.state_out) && optional_tensor(h_out, s.h_out) && optional_tensor(h_prev, s.h_prev);
+}
+// whether the cell's plan covers a step of B rows of x (the cell's input, or what a layer makes it from)
+bool step_fits(const CellPath &c, const at::Tensor &x, const at::Tensor &state, const StepBuffers &s) {
+  const at::Tensor *r, *b;
+  if (!c.plan || !c.weights(r, b) || r->data_ptr() != c.r_ptr || b->data_ptr() != c.b_ptr || version_of(*r) != c.r_version ||
+      version_of(*b) != c.b_version)
+    return false;
+  const int64_t B = c.step_B, H = c.NH * c.dh;
+  const auto dt = c.step_dtype;
+  if (x.scalar_type() != dt || !x.is_cuda() || x.device() != c.device || !x.is_contiguous() || x.dim() != 3 || x.size(0) != B || x.size(1) != 1 ||
+      c.records(x, &state, *r, *b))
+    return false;
+  auto state_like = [&](const at::Tensor &t) {
+    return t.scalar_type() == at::kFloat && t.is_contiguous() && t.device() == c.device && t.dim() == 3 && t.size(0) == 4 && t.size(1) == B && t.size(2) == H;
+  };
+  auto h_like = [&](const at::Tensor &t) { return t.scalar_type() == dt && t.numel() == B * H && t.device() == c.device; };
+  return state_like(state) && (!s.state_out || state_like(*s.state_out)) && (!s.h_out || (h_like(*s.h_out) && s.h_out->is_contiguous())) &&
+         (!s.h_prev || dt != at::kBFloat16 || h_like(*s.h_prev));
+}
 struct StepResult { at::Tensor h, state; };  // h: [1,B,H] memory, state: float32 [4,B,H]
-StepResult run_step(CellPath &c, const at::Tensor &x, const at::Tensor &state, const at::Tensor *state_out, const at::Tensor *h_out,
-                    const at::Tensor *h_prev, const Shape4 *h_shape, bool keep_state) {
-  const int64_t H = c.NH * c.dh;
-  const auto dt = x.scalar_type();
-  if (!c.plan || dt != c.step_dtype || !x.is_cuda() || x.device() != c.device || !x.is_contiguous() || x.dim() != 3 || x.size(1) != 1 ||
-      x.size(0) != c.step_B || x.size(2) != 4 * H)
-    throw NotCovered{};
-  const int64_t B = c.step_B;
-  if (state.scalar_type() != at::kFloat || !state.is_contiguous() || state.device() != c.device || state.dim() != 3 || state.size(0) != 4 ||
-      state.size(1) != B || state.size(2) != H)
-    throw NotCovered{};
-  const at::Tensor &r = c.parameter(g_names.r), &b = c.parameter(g_names.b);
-  if (r.data_ptr() != c.r_ptr || b.data_ptr() != c.b_ptr || version_of(r) != c.r_version || version_of(b) != c.b_version || c.records(x, &state, r, b))
-    throw NotCovered{};
+// (wx: contiguous [B,1,4H]; everything else as step_fits has found it)
+StepResult run_step(CellPath &c, const at::Tensor &wx, const at::Tensor &state, const StepBuffers &s, const Shape4 *h_shape, bool keep_state) {
+  const int64_t B = c.step_B, H = c.NH * c.dh;
   StepResult out;
-  if (h_out) {
-    if (h_out->scalar_type() != dt || h_out->numel() != B * H || !h_out->is_contiguous() || h_out->device() != c.device) throw NotCovered{};
-    out.h = *h_out;
-  } else if (h_shape) {
-    out.h = at::empty_strided(at::IntArrayRef(h_shape->size.data(), h_shape->n), at::IntArrayRef(h_shape->stride.data(), h_shape->n), x.options());
-  } else {
-    out.h = at::empty({1, B, H}, x.options());
-  }
-  out.state = state_out ? *state_out : at::empty({4, B, H}, state.options());
+  if (s.h_out) out.h = *s.h_out;
+  else if (h_shape) out.h = at::empty_strided(at::IntArrayRef(h_shape->size.data(), h_shape->n), at::IntArrayRef(h_shape->stride.data(), h_shape->n), wx.options());
+  else out.h = at::empty({1, B, H}, wx.options());
+  out.state = s.state_out ? *s.state_out : at::empty({4, B, H}, state.options());
   xs_slstm_args &a = *c.step_args;
   a.h_prev = nullptr;
-  if (dt == at::kBFloat16) {
-    if (h_prev) {
-      if (h_prev->scalar_type() != dt || h_prev->numel() != B * H || h_prev->device() != c.device) throw NotCovered{};
-      a.h_prev = h_prev->data_ptr();
+  if (c.step_dtype == at::kBFloat16) {
+    if (s.h_prev) {
+      a.h_prev = s.h_prev->data_ptr();
     } else if (c.last_state.defined() && c.last_state.is_same(state) && versioned(state) && version_of(state) == c.last_state_version &&
                version_of(c.last_h) == c.last_h_version && c.last_h.data_ptr() != out.h.data_ptr()) {
       // The state this cell handed out last time comes back untouched: the h it returned with it is that state's y
@@ -268,7 +274,7 @@ StepResult run_step(CellPath &c, const at::Tensor &x, const at::Tensor &state, c
       a.h_prev = c.last_h.data_ptr();
     }
   }
-  a.wx = x.data_ptr();
+  a.wx = wx.data_ptr();
   a.s0 = (const float *)state.data_ptr();
   a.s_out = (float *)out.state.data_ptr();
   a.h_out = out.h.data_ptr();
@@ -283,63 +289,65 @@ StepResult run_step(CellPath &c, const at::Tensor &x, const at::Tensor &state, c
   return out;
 }
 
-// Ordinary reasons for the general path, looked at in front of everything else: an exception costs tens of microseconds
-// in a process with as many libraries as this one, and a training loop or the first token of a batch size comes here on
-// every call.
-bool plan_fits(const CellPath &c, PyObject *x, PyObject *state) {
-  if (!c.plan || !THPVariable_Check(x) || !THPVariable_Check(state)) return false;
-  const at::Tensor &s = THPVariable_Unpack(state);
-  if (s.scalar_type() != at::kFloat || s.dim() != 3 || s.size(1) != c.step_B) return false;
-  PyObject *ro = c.parameter_object(g_names.r), *bo = c.parameter_object(g_names.b);
-  if (!ro || !bo || !THPVariable_Check(ro) || !THPVariable_Check(bo)) return false;
-  const at::Tensor &r = THPVariable_Unpack(ro), &b = THPVariable_Unpack(bo);
-  return r.data_ptr() == c.r_ptr && b.data_ptr() == c.b_ptr && version_of(r) == c.r_version && version_of(b) == c.b_version &&
-         THPVariable_Unpack(x).scalar_type() == c.step_dtype && !c.records(THPVariable_Unpack(x), &s, r, b);
-}
-bool recording(const CellPath &c, PyObject *x, PyObject *state) {
+bool recording(const CellPath &c, const at::Tensor &x, const at::Tensor *state) {
   if (!at::GradMode::is_enabled()) return false;
-  PyObject *ro = c.parameter_object(g_names.r), *bo = c.parameter_object(g_names.b);
-  if (!ro || !bo || !THPVariable_Check(ro) || !THPVariable_Check(bo) || !THPVariable_Check(x)) return true;
-  return c.records(THPVariable_Unpack(x), !absent(state) && THPVariable_Check(state) ? &THPVariable_Unpack(state) : nullptr, THPVariable_Unpack(ro), THPVariable_Unpack(bo));
+  const at::Tensor *r, *b;
+  return !c.weights(r, b) || c.records(x, state, *r, *b);
 }
-
-inline const at::Tensor *optional_tensor(PyObject *o) { return absent(o) ? nullptr : &tensor_of(o); }
 
 // step(input, state, reset_mask, state_out, h_out, h_prev, config, keep_state_fp32) -> (output, state) or None
 PyObject *cell_step_(CellPath &c, PyObject *const *args) {
-  if (!absent(args[2]) || absent(args[1]) || at::autocast::is_autocast_enabled(at::kCUDA) || !plan_fits(c, args[0], args[1])) Py_RETURN_NONE;
-  const at::Tensor &x = tensor_of(args[0]), &state = tensor_of(args[1]);
-  if (!input_is_bsgnh(args[6])) throw NotCovered{};
-  const OutShape shape = out_shape(args[6]);
+  const at::Tensor *x = tensor_of(args[0]), *state = tensor_of(args[1]);
+  StepBuffers s;
+  if (!absent(args[2]) || !x || !state || at::autocast::is_autocast_enabled(at::kCUDA) || !step_buffers(args[3], args[4], args[5], s) ||
+      !step_fits(c, *x, *state, s) || x->size(2) != 4 * c.NH * c.dh)
+    Py_RETURN_NONE;
+  OutShape shape;
+  if (!input_is_bsgnh(args[6]) || !out_shape(args[6], shape)) Py_RETURN_NONE;
   const bool keep = args[7] == Py_True;
   c10::OptionalDeviceGuard guard(c.device);
   const Shape4 s4 = shape_of(shape, 1, c.step_B, c.NH, c.dh);
-  const at::Tensor *h_out = optional_tensor(args[4]);
-  StepResult r = run_step(c, x, state, optional_tensor(args[3]), h_out, optional_tensor(args[5]), &s4, keep);
-  at::Tensor h = h_out ? r.h.as_strided(at::IntArrayRef(s4.size.data(), s4.n), at::IntArrayRef(s4.stride.data(), s4.n)) : r.h;
-  PyRef ph(THPVariable_Wrap(h)), ps(THPVariable_Wrap(keep || x.scalar_type() == at::kFloat ? r.state : r.state.to(x.scalar_type())));
+  StepResult r = run_step(c, *x, *state, s, &s4, keep);
+  at::Tensor h = s.h_out ? r.h.as_strided(at::IntArrayRef(s4.size.data(), s4.n), at::IntArrayRef(s4.stride.data(), s4.n)) : r.h;
+  PyRef ph(THPVariable_Wrap(h)), ps(THPVariable_Wrap(keep || x->scalar_type() == at::kFloat ? r.state : r.state.to(x->scalar_type())));
   if (!ph.o || !ps.o) throw PythonError{};
   return PyTuple_Pack(2, ph.o, ps.o);
 }
 
 // ---- a sequence through the cell (no autograd), as sLSTMCell_hip._run and functional.slstm_forward do it
 struct Sequence { at::Tensor h, state, coef, mask; };  // h: [S,B,H] memory with the strides of `shape`, state: float32
-at::Tensor mask_bytes(const at::Tensor &m, int64_t B, int64_t T) {
-  if (!m.is_cuda() || m.dim() != 2 || m.size(0) != B || m.size(1) != T) throw NotCovered{};
+bool mask_fits(const at::Tensor *m, int64_t B, int64_t T) { return !m || (m->is_cuda() && m->dim() == 2 && m->size(0) == B && m->size(1) == T); }
+at::Tensor mask_bytes(const at::Tensor &m) {
   at::Tensor r = m;
   if (r.scalar_type() == at::kBool) r = r.is_contiguous() ? r.view(at::kByte) : r.to(at::kByte);
   else if (r.scalar_type() != at::kByte) r = r.ne(0).to(at::kByte);
   return r.stride(1) != 1 ? r.contiguous() : r;
 }
 
+// whether the sequence kernels take these tensors; x: [B,T,..] on the GPU
+bool sequence_fits(const CellPath &c, const at::Tensor &x, int64_t B, int64_t T, const at::Tensor *state, const at::Tensor *mask) {
+  const int64_t H = c.NH * c.dh;
+  const auto dt = x.scalar_type();
+  const at::Tensor *r, *b;
+  if ((dt != at::kFloat && dt != at::kBFloat16) || T < 2 || B < 1 || !mask_fits(mask, B, T) || !c.weights(r, b)) return false;
+  if (state && (!state->is_cuda() || state->dim() != 3 || state->size(0) != 4 || state->size(1) != B || state->size(2) != H)) return false;
+  return r->device() == x.device() && b->device() == x.device() && r->is_contiguous() && b->is_contiguous() &&
+         (r->scalar_type() == at::kFloat || r->scalar_type() == at::kBFloat16) && r->numel() == c.NH * 4 * c.dh * c.dh && b->numel() == 4 * H;
+}
+// the cell's abort word, made on first use (under capture there is none: no host memory is allocated, and a replay reports to nobody)
+bool have_word(CellPath &c, const at::Device &d) {
+  if (!c.abort_word && !capturing(d)) c.abort_word = take_word();
+  return c.abort_word || capturing(d);
+}
+
 // train: the forward of a training call, which also leaves the backward pass its coefficients (no graph is recorded here)
+// (x: [B,T,4H] as sequence_fits has found it)
 Sequence run_sequence(CellPath &c, at::Tensor x, const at::Tensor *state, const at::Tensor *mask, OutShape shape, bool train = false) {
   const int64_t H = c.NH * c.dh, B = x.size(0), T = x.size(1);
   const auto dt = x.scalar_type();
-  if ((dt != at::kFloat && dt != at::kBFloat16) || !x.is_cuda() || T < 2 || B < 1 || x.size(2) != 4 * H) throw NotCovered{};
-  at::Tensor r = c.parameter(g_names.r), b = c.parameter(g_names.b);
-  if ((!train && c.records(x, state, r, b)) || r.device() != x.device() || b.device() != x.device() || !r.is_contiguous() || !b.is_contiguous()) throw NotCovered{};
-  if ((r.scalar_type() != at::kFloat && r.scalar_type() != at::kBFloat16) || r.numel() != c.NH * 4 * c.dh * c.dh || b.numel() != 4 * H) throw NotCovered{};
+  const at::Tensor *rp, *bp;
+  if (!c.weights(rp, bp)) { PyErr_SetString(PyExc_RuntimeError, "the cell has lost its parameters"); throw PythonError{}; }
+  at::Tensor r = *rp, b = *bp;
   const size_t esz = x.element_size();
   if (x.stride(2) != 1 || !aligned(x.data_ptr(), 16) || (x.stride(0) * esz) % 16 || (x.stride(1) * esz) % 16 || x.stride(1) < 4 * H ||
       (B > 1 && x.stride(0) < 4 * H))
@@ -347,11 +355,8 @@ Sequence run_sequence(CellPath &c, at::Tensor x, const at::Tensor *state, const 
   if (dt == at::kFloat && r.scalar_type() != at::kFloat) r = r.to(at::kFloat);
   if (b.scalar_type() != at::kFloat) b = b.to(at::kFloat);  // (on every call: a copy kept would be another stream's, and a graph's)
   at::Tensor s0, m;
-  if (state) {
-    if (!state->is_cuda() || state->dim() != 3 || state->size(0) != 4 || state->size(1) != B || state->size(2) != H) throw NotCovered{};
-    s0 = state->to(at::kFloat).contiguous();
-  }
-  if (mask) m = mask_bytes(*mask, B, T);
+  if (state) s0 = state->to(at::kFloat).contiguous();
+  if (mask) m = mask_bytes(*mask);
   const bool in_graph = capturing(x.device());
   if (!in_graph) c.raise_if_aborted();
   const Shape4 s4 = shape_of(shape, T, B, c.NH, c.dh);
@@ -360,14 +365,9 @@ Sequence run_sequence(CellPath &c, at::Tensor x, const at::Tensor *state, const 
   out.state = at::empty({4, B, H}, x.options().dtype(at::kFloat));
   if (train) {
     const size_t n = g_engine.coef_floats((int32_t)B, (int32_t)T, (int32_t)c.NH, (int32_t)c.dh, dtype_code(dt));
-    if (!n) throw NotCovered{};
     out.coef = at::empty({(int64_t)n}, out.state.options());
   }
   at::Tensor &ws = c.workspace(B, x.device());
-  if (!in_graph) {  // (under capture no host memory is allocated, and a replay reports to nobody)
-    if (!c.abort_word) c.abort_word = take_word();
-    if (!c.abort_word) throw NotCovered{};
-  }
   xs_slstm_args a{};
   a.B = (int32_t)B; a.T = (int32_t)T; a.NH = (int32_t)c.NH; a.dh = (int32_t)c.dh;
   a.wx_dtype = dtype_code(dt); a.r_dtype = dtype_code(r.scalar_type());
@@ -388,13 +388,17 @@ Sequence run_sequence(CellPath &c, at::Tensor x, const at::Tensor *state, const 
 
 // forward(input, state, reset_mask, config, keep_state_fp32) -> (output, state) or None
 PyObject *cell_forward_(CellPath &c, PyObject *const *args) {
-  if (at::autocast::is_autocast_enabled(at::kCUDA) || recording(c, args[0], args[1])) Py_RETURN_NONE;
-  const at::Tensor &x = tensor_of(args[0]);
-  if (x.dim() != 3 || !x.is_cuda()) throw NotCovered{};
-  const at::Tensor *state = optional_tensor(args[1]), *mask = optional_tensor(args[2]);
-  const OutShape shape = out_shape(args[3]);
+  const at::Tensor *xp = tensor_of(args[0]), *state, *mask;
+  if (!xp || xp->dim() != 3 || !xp->is_cuda() || !optional_tensor(args[1], state) || !optional_tensor(args[2], mask) ||
+      at::autocast::is_autocast_enabled(at::kCUDA) || recording(c, *xp, state))
+    Py_RETURN_NONE;
+  const at::Tensor &x = *xp;
+  OutShape shape;
+  const bool bsgnh = input_is_bsgnh(args[3]);
+  if (!out_shape(args[3], shape) || x.size(2) != 4 * c.NH * c.dh || !sequence_fits(c, x, x.size(bsgnh ? 0 : 1), x.size(bsgnh ? 1 : 0), state, mask)) Py_RETURN_NONE;
   c10::OptionalDeviceGuard guard(x.device());
-  Sequence s = run_sequence(c, input_is_bsgnh(args[3]) ? x : x.permute({1, 0, 2}), state, mask, shape);
+  if (!have_word(c, x.device())) Py_RETURN_NONE;
+  Sequence s = run_sequence(c, bsgnh ? x : x.permute({1, 0, 2}), state, mask, shape);
   PyRef ph(THPVariable_Wrap(s.h)), ps(THPVariable_Wrap(args[4] == Py_True || x.scalar_type() == at::kFloat ? s.state : s.state.to(x.scalar_type())));
   if (!ph.o || !ps.o) throw PythonError{};
   return PyTuple_Pack(2, ph.o, ps.o);
@@ -521,27 +525,28 @@ struct CellBackward : public torch::autograd::Node {
 
 // train(input, state, reset_mask, config, keep_state_fp32) -> (output, state) with their place in the graph, or None
 PyObject *cell_train_(CellPath &c, PyObject *const *args) {
-  if (at::autocast::is_autocast_enabled(at::kCUDA) || !THPVariable_Check(args[0]) || !recording(c, args[0], args[1])) Py_RETURN_NONE;
-  const at::Tensor &x = tensor_of(args[0]);
+  const at::Tensor *xp = tensor_of(args[0]), *state, *mask, *rp, *bp;
+  if (!xp || xp->dim() != 3 || !xp->is_cuda() || !optional_tensor(args[1], state) || !optional_tensor(args[2], mask) ||
+      at::autocast::is_autocast_enabled(at::kCUDA) || !c.weights(rp, bp) || !recording(c, *xp, state))
+    Py_RETURN_NONE;
+  const at::Tensor &x = *xp;
+  OutShape shape;
   const bool bsgnh = input_is_bsgnh(args[3]);
-  if (x.dim() != 3 || !x.is_cuda() || x.size(bsgnh ? 1 : 0) < 2 || x.size(bsgnh ? 0 : 1) < 1) Py_RETURN_NONE;
-  if ((x.scalar_type() != at::kFloat && x.scalar_type() != at::kBFloat16) ||
+  if (!out_shape(args[3], shape) || x.size(2) != 4 * c.NH * c.dh || !sequence_fits(c, x, x.size(bsgnh ? 0 : 1), x.size(bsgnh ? 1 : 0), state, mask) ||
       !g_engine.coef_floats(1, 1, (int32_t)c.NH, (int32_t)c.dh, dtype_code(x.scalar_type())))
     Py_RETURN_NONE;
-  const at::Tensor *state = optional_tensor(args[1]), *mask = optional_tensor(args[2]);
-  for (const at::Tensor *t : {&x, &c.parameter(g_names.r), &c.parameter(g_names.b), state})
+  for (const at::Tensor *t : {&x, rp, bp, state})
     if (t && t->_fw_grad(0).defined()) Py_RETURN_NONE;  // (forward mode: the general path refuses it)
-  const OutShape shape = out_shape(args[3]);
   PyRef cut(PyObject_GetAttr(args[3], g_names.cut)), clip(PyObject_GetAttr(args[3], g_names.clipval));
   if (!cut.o || !clip.o) throw PythonError{};
   const int cut_on = PyObject_IsTrue(cut.o);
   const double clipval = clip.o == Py_None ? 0.0 : PyFloat_AsDouble(clip.o);
   if (PyErr_Occurred()) throw PythonError{};
   c10::OptionalDeviceGuard guard(x.device());
+  if (!have_word(c, x.device())) Py_RETURN_NONE;
   Sequence s;
-  at::Tensor s_out;
   {
-    const at::Tensor r = c.parameter(g_names.r), b = c.parameter(g_names.b);
+    const at::Tensor r = *rp, b = *bp;
     {
       at::NoGradGuard no_grad;
       s = run_sequence(c, bsgnh ? x : x.permute({1, 0, 2}), state, mask, shape, true);
@@ -574,8 +579,6 @@ PyObject *cell_call(PyObject *self, PyObject *const *args, Py_ssize_t n) {
   if (n != N) { PyErr_Format(PyExc_TypeError, "%d arguments expected, got %zd", N, n); return nullptr; }
   try {
     return F(*((CellPathObject *)self)->c, args);
-  } catch (const NotCovered &) {
-    Py_RETURN_NONE;
   } catch (const PythonError &) {
     return nullptr;
   } catch (python_error &e) {
@@ -589,7 +592,9 @@ PyObject *cell_call(PyObject *self, PyObject *const *args, Py_ssize_t n) {
 
 // set_plan(plan, address of its argument block, B, r, b): the next steps of that batch size and of these parameters
 PyObject *cell_set_plan_(CellPath &c, PyObject *const *args) {
-  const at::Tensor &r = tensor_of(args[3]), &b = tensor_of(args[4]);
+  const at::Tensor *rp = tensor_of(args[3]), *bp = tensor_of(args[4]);
+  if (!rp || !bp) { PyErr_SetString(PyExc_TypeError, "set_plan: r and b are tensors"); throw PythonError{}; }
+  const at::Tensor &r = *rp, &b = *bp;
   c.step_args = (xs_slstm_args *)PyLong_AsVoidPtr(args[1]);
   c.step_B = PyLong_AsLongLong(args[2]);
   c.step_dtype = c.step_args->wx_dtype == XS_BF16 ? at::kBFloat16 : at::kFloat;
@@ -602,8 +607,9 @@ PyObject *cell_set_plan_(CellPath &c, PyObject *const *args) {
 }
 // workspace(B, a tensor on the device) -> the workspace of calls on that device's current stream
 PyObject *cell_workspace_(CellPath &c, PyObject *const *args) {
-  const at::Tensor &like = tensor_of(args[1]);
-  return THPVariable_Wrap(c.workspace(PyLong_AsLongLong(args[0]), like.device()));
+  const at::Tensor *like = tensor_of(args[1]);
+  if (!like) { PyErr_SetString(PyExc_TypeError, "workspace: a tensor on the device"); throw PythonError{}; }
+  return THPVariable_Wrap(c.workspace(PyLong_AsLongLong(args[0]), like->device()));
 }
 // last_workspace() -> the workspace of the latest sequence call
 PyObject *cell_last_workspace_(CellPath &c, PyObject *const *) {
@@ -684,26 +690,25 @@ PyObject *attribute(PyObject *o, PyObject *name) {  // new reference; nn.Module 
   if (!v) throw PythonError{};
   return v;
 }
-PyObject *submodule(PyObject *modules, PyObject *name) {  // borrowed
-  PyObject *m = PyDict_GetItem(modules, name);
-  if (!m) throw NotCovered{};
-  return m;
-}
-PyObject *module_dict(PyObject *module, PyObject *which) {  // borrowed from the module
+PyObject *module_dict(PyObject *module, PyObject *which) {  // borrowed from the module, or null
   PyRef d(attribute(module, which));
-  if (!PyDict_Check(d.o)) throw NotCovered{};
-  return d.o;  // (the module holds it)
+  return PyDict_Check(d.o) ? d.o : nullptr;  // (the module holds it)
 }
-at::Tensor parameter(PyObject *module, PyObject *name, bool optional = false) {
-  PyObject *o = PyDict_GetItem(module_dict(module, g_names.parameters), name);
-  if (absent(o)) {
-    if (optional) return at::Tensor();
-    throw NotCovered{};
-  }
-  return tensor_of(o);
+PyObject *submodule(PyObject *module, PyObject *name) {  // borrowed, or null
+  PyObject *modules = module_dict(module, g_names.modules), *m = modules ? PyDict_GetItem(modules, name) : nullptr;
+  return absent(m) ? nullptr : m;
+}
+// a parameter of a module in the type and place of x; absent: an undefined tensor.  false: another type, layout or device
+bool parameter(PyObject *module, PyObject *name, const at::Tensor &x, at::Tensor &out) {
+  PyObject *parameters = module_dict(module, g_names.parameters), *o = parameters ? PyDict_GetItem(parameters, name) : nullptr;
+  const at::Tensor *t;
+  if (!parameters || !optional_tensor(o, t)) return false;
+  if (t) out = *t;
+  return !t || (t->scalar_type() == at::kBFloat16 && t->is_contiguous() && t->device() == x.device() && aligned(t->data_ptr(), 16));
 }
 bool has_hooks(PyObject *module) {
-  return PyDict_Size(module_dict(module, g_names.forward_hooks)) || PyDict_Size(module_dict(module, g_names.forward_pre_hooks));
+  PyObject *after = module_dict(module, g_names.forward_hooks), *before = module_dict(module, g_names.forward_pre_hooks);
+  return !after || !before || PyDict_Size(after) || PyDict_Size(before);
 }
 
 struct LayerParts {
@@ -715,61 +720,49 @@ struct LayerParts {
   int64_t K = 0, NH = 0, dh = 0, D = 0;
 };
 
-// what a layer call needs of its modules; NotCovered unless the engine's kernels apply (sLSTMLayer._fused) and no
-// gradient is recorded
-void collect(PyObject *layer, PyObject *cell_path, const at::Tensor &x, LayerParts &p) {
+// what a layer call needs of its modules; false unless the engine's kernels apply (sLSTMLayer._fused) and no gradient is
+// recorded
+bool collect(PyObject *layer, PyObject *cell_path, const at::Tensor &x, LayerParts &p) {
   p.cell = ((CellPathObject *)cell_path)->c;
   p.NH = p.cell->NH; p.dh = p.cell->dh; p.D = p.NH * p.dh;
   if (x.dim() != 3 || x.scalar_type() != at::kBFloat16 || !x.is_cuda() || x.size(2) != p.D || p.dh % 64 || p.dh > 1024 ||
-      at::autocast::is_autocast_enabled(at::kCUDA))
-    throw NotCovered{};
+      at::autocast::is_autocast_enabled(at::kCUDA) || recording(*p.cell, x, nullptr))
+    return false;
   for (PyObject *h : g_engine.global_hooks)
-    if (h && PyDict_Size(h)) throw NotCovered{};
-  PyObject *modules = module_dict(layer, g_names.modules);
-  PyObject *cell = submodule(modules, g_names.slstm_cell);
-  PyObject *conv1d = submodule(modules, g_names.conv1d);
-  PyObject *conv = submodule(module_dict(conv1d, g_names.modules), g_names.conv);
-  PyObject *norm = submodule(modules, g_names.group_norm), *dropout = submodule(modules, g_names.dropout);
-  if (has_hooks(cell) || has_hooks(dropout)) throw NotCovered{};
+    if (h && PyDict_Size(h)) return false;
+  PyObject *cell = submodule(layer, g_names.slstm_cell), *conv1d = submodule(layer, g_names.conv1d);
+  PyObject *conv = conv1d ? submodule(conv1d, g_names.conv) : nullptr;
+  PyObject *norm = submodule(layer, g_names.group_norm), *dropout = submodule(layer, g_names.dropout);
+  if (!cell || !conv || !norm || !dropout || has_hooks(cell) || has_hooks(dropout)) return false;
   {
     PyRef fused(attribute(layer, g_names.fused_pre_ops));
-    if (fused.o != Py_True) throw NotCovered{};
+    if (fused.o != Py_True) return false;
     PyRef training(attribute(dropout, g_names.training)), rate(attribute(dropout, g_names.p));
     const double dp = PyFloat_AsDouble(rate.o);
-    if (PyErr_Occurred()) { PyErr_Clear(); throw NotCovered{}; }
-    if (training.o == Py_True && dp != 0.0) throw NotCovered{};
+    if (PyErr_Occurred()) { PyErr_Clear(); return false; }
+    if (training.o == Py_True && dp != 0.0) return false;
     PyRef keep(attribute(cell, g_names.keep_state_fp32)), eps(attribute(norm, g_names.eps));
     p.keep_state = keep.o == Py_True;
     p.eps = PyFloat_AsDouble(eps.o);
+    if (PyErr_Occurred()) throw PythonError{};
     p.cell_config.o = attribute(cell, g_names.config);
   }
-  if (!input_is_bsgnh(p.cell_config.o) || out_shape(p.cell_config.o) != OutShape::BNSH) throw NotCovered{};
-  p.conv_w = parameter(conv, g_names.weight);
-  p.conv_b = parameter(conv, g_names.bias, true);
+  OutShape shape;
+  if (!input_is_bsgnh(p.cell_config.o) || !out_shape(p.cell_config.o, shape) || shape != OutShape::BNSH) return false;
+  if (!parameter(conv, g_names.weight, x, p.conv_w) || !p.conv_w.defined() || !parameter(conv, g_names.bias, x, p.conv_b) ||
+      !parameter(norm, g_names.weight, x, p.norm_w))
+    return false;
   // (the module called fgate feeds the i slot, igate the f slot)
   PyObject *gates[4] = {g_names.fgate, g_names.igate, g_names.zgate, g_names.ogate};
   bool needs_grad = x.requires_grad();
   for (int g = 0; g < 4; ++g) {
-    p.gate[g] = parameter(submodule(modules, gates[g]), g_names.weight);
-    const at::Tensor &w = p.gate[g];
-    if (w.scalar_type() != at::kBFloat16 || !w.is_contiguous() || w.numel() != p.NH * p.dh * p.dh || w.device() != x.device() || !aligned(w.data_ptr(), 16)) throw NotCovered{};
-    needs_grad |= w.requires_grad();
+    PyObject *gate = submodule(layer, gates[g]);
+    if (!gate || !parameter(gate, g_names.weight, x, p.gate[g]) || !p.gate[g].defined() || p.gate[g].numel() != p.NH * p.dh * p.dh) return false;
+    needs_grad |= p.gate[g].requires_grad();
   }
-  p.norm_w = parameter(norm, g_names.weight, true);
-  for (const at::Tensor *t : {&p.conv_w, &p.conv_b, &p.norm_w}) {
-    if (!t->defined()) continue;
-    if (t->scalar_type() != at::kBFloat16 || !t->is_contiguous() || t->device() != x.device() || !aligned(t->data_ptr(), 16)) throw NotCovered{};
-    needs_grad |= t->requires_grad();
-  }
+  for (const at::Tensor *t : {&p.conv_w, &p.conv_b, &p.norm_w}) needs_grad |= t->defined() && t->requires_grad();
   p.K = p.conv_w.numel() / p.D;
-  if (p.K < 2 || p.K > 4) throw NotCovered{};
-  if (at::GradMode::is_enabled() && needs_grad) throw NotCovered{};  // (the cell's own parameters: looked at where it runs)
-}
-
-// (the ordinary reasons, without an exception: see plan_fits)
-bool engine_layer(PyObject *const *args) {
-  return THPVariable_Check(args[2]) && THPVariable_Unpack(args[2]).scalar_type() == at::kBFloat16 &&
-         !recording(*((CellPathObject *)args[1])->c, args[2], nullptr);
+  return p.K >= 2 && p.K <= 4 && !(at::GradMode::is_enabled() && needs_grad);  // (the cell's own parameters: recording)
 }
 
 void run_conv(const LayerParts &p, const at::Tensor &x, const void *taps, int64_t taps_stride, const at::Tensor *mask, void *out, void *ring, void *stream) {
@@ -803,13 +796,14 @@ void run_norm(const LayerParts &p, const at::Tensor &h, int64_t B, int64_t T, vo
 }
 
 // the taps in front of the first token: a [B,n,D] tensor of which the last K-1 inputs count
-const void *taps_of(const LayerParts &p, const at::Tensor &t, int64_t B, int64_t *stride) {
+bool taps_of(const LayerParts &p, const at::Tensor &t, int64_t B, const void *&taps, int64_t &stride) {
   const int64_t n = t.dim() == 3 ? t.size(1) : 0;
   if (t.scalar_type() != at::kBFloat16 || n < p.K - 1 || t.size(0) != B || t.size(2) != p.D || t.stride(2) != 1 || t.stride(1) != p.D || t.stride(0) % 8 ||
       !t.is_cuda() || !aligned(t.data_ptr(), 16))
-    throw NotCovered{};
-  *stride = t.stride(0);
-  return (const char *)t.data_ptr() + (n - (p.K - 1)) * p.D * 2;
+    return false;
+  stride = t.stride(0);
+  taps = (const char *)t.data_ptr() + (n - (p.K - 1)) * p.D * 2;
+  return true;
 }
 
 PyObject *states_dict(PyObject *conv_state, const at::Tensor &state) {
@@ -826,47 +820,36 @@ PyObject *first_of(PyObject *o) {  // a state that may come in a tuple or list o
 // layer_step(layer, cell path, x, conv_state, slstm_state, slstm_state_out, conv_state_out, h_out, h_prev, out)
 //   -> (out, {"conv_state": (ring,), "slstm_state": state}) or None
 PyObject *layer_step_(PyObject *const *args) {
-  if (absent(args[4]) || !engine_layer(args) || !plan_fits(*((CellPathObject *)args[1])->c, args[2], args[4])) Py_RETURN_NONE;
-  const at::Tensor &x = tensor_of(args[2]);
+  const at::Tensor *xp = tensor_of(args[2]), *statep = tensor_of(args[4]), *ring_out, *out_given;
+  CellPath &c = *((CellPathObject *)args[1])->c;
+  StepBuffers buffers;
+  if (!xp || !statep || !step_buffers(args[5], args[7], args[8], buffers) || !optional_tensor(args[6], ring_out) || !optional_tensor(args[9], out_given) ||
+      !step_fits(c, *xp, *statep, buffers))
+    Py_RETURN_NONE;
+  const at::Tensor &x = *xp, &state = *statep;
   LayerParts p;
-  collect(args[0], args[1], x, p);
-  const at::Tensor &state = tensor_of(args[4]);
+  if (!aligned(x.data_ptr(), 16) || !collect(args[0], args[1], x, p)) Py_RETURN_NONE;
   const int64_t B = x.size(0);
-  if (x.size(1) != 1 || !x.is_contiguous() || !aligned(x.data_ptr(), 16) || B < 1) throw NotCovered{};
-  c10::OptionalDeviceGuard guard(x.device());
+  if (B < 1) Py_RETURN_NONE;
   const void *taps = nullptr;
   int64_t taps_stride = 0;
   PyObject *prev = absent(args[3]) ? nullptr : first_of(args[3]);
   if (!absent(prev)) {
-    const at::Tensor &t = tensor_of(prev);
-    if (t.dim() != 3 || (t.size(1) != p.K && t.size(1) != p.K - 1)) throw NotCovered{};  // (the general path asserts)
-    taps = taps_of(p, t, B, &taps_stride);
+    const at::Tensor *t = tensor_of(prev);
+    if (!t || t->dim() != 3 || (t->size(1) != p.K && t->size(1) != p.K - 1) || !taps_of(p, *t, B, taps, taps_stride)) Py_RETURN_NONE;  // (the general path asserts)
   }
-  const at::Tensor *ring_out = optional_tensor(args[6]), *out_given = optional_tensor(args[9]);
   const auto opts = x.options();
   if (ring_out && (ring_out->scalar_type() != at::kBFloat16 || ring_out->dim() != 3 || ring_out->size(0) != B || ring_out->size(1) != p.K ||
                    ring_out->size(2) != p.D || !ring_out->is_contiguous()))
-    throw NotCovered{};
-  if (out_given && (out_given->scalar_type() != at::kBFloat16 || out_given->numel() != B * p.D || !out_given->is_contiguous())) throw NotCovered{};
-  // the step's own conditions, before anything is launched
-  {
-    const at::Tensor *so = optional_tensor(args[5]), *ho = optional_tensor(args[7]), *hp = optional_tensor(args[8]);
-    if (so && (so->scalar_type() != at::kFloat || !so->is_contiguous() || so->dim() != 3 || so->size(0) != 4 || so->size(1) != B || so->size(2) != p.D)) throw NotCovered{};
-    if (ho && (ho->scalar_type() != at::kBFloat16 || ho->numel() != B * p.D || !ho->is_contiguous())) throw NotCovered{};
-    if (hp && (hp->scalar_type() != at::kBFloat16 || hp->numel() != B * p.D)) throw NotCovered{};
-    const at::Tensor &r = p.cell->parameter(g_names.r), &b = p.cell->parameter(g_names.b);
-    if (!p.cell->plan || p.cell->step_B != B || p.cell->step_dtype != at::kBFloat16 || p.cell->device != x.device() || r.data_ptr() != p.cell->r_ptr ||
-        b.data_ptr() != p.cell->b_ptr || version_of(r) != p.cell->r_version || version_of(b) != p.cell->b_version || p.cell->records(x, &state, r, b) ||
-        state.scalar_type() != at::kFloat || !state.is_contiguous() || state.device() != x.device() || state.dim() != 3 || state.size(0) != 4 ||
-        state.size(1) != B || state.size(2) != p.D)
-      throw NotCovered{};
-  }
+    Py_RETURN_NONE;
+  if (out_given && (out_given->scalar_type() != at::kBFloat16 || out_given->numel() != B * p.D || !out_given->is_contiguous())) Py_RETURN_NONE;
+  c10::OptionalDeviceGuard guard(x.device());
   void *stream = stream_of(x.device());
   at::Tensor ring = ring_out ? *ring_out : at::empty({B, p.K, p.D}, opts);
   at::Tensor wx = at::empty({B, 1, 4 * p.D}, opts), x_conv = at::empty({B, 1, p.D}, opts);
   run_conv(p, x, taps, taps_stride, nullptr, x_conv.data_ptr(), ring.data_ptr(), stream);
   run_gates(p, x, x_conv.data_ptr(), wx.data_ptr(), stream);
-  StepResult s = run_step(*p.cell, wx, state, optional_tensor(args[5]), optional_tensor(args[7]), optional_tensor(args[8]), nullptr, p.keep_state);
+  StepResult s = run_step(c, wx, state, buffers, nullptr, p.keep_state);
   at::Tensor out = out_given ? *out_given : at::empty({B, 1, p.D}, opts);
   run_norm(p, s.h, B, 1, out.data_ptr(), stream);
   PyRef po(THPVariable_Wrap(out)), pr(THPVariable_Wrap(ring)), tuple(nullptr);
@@ -878,28 +861,27 @@ PyObject *layer_step_(PyObject *const *args) {
 
 // layer_forward(layer, cell path, x, conv_state, slstm_state, return_last_state, reset_mask) -> the layer's result or None
 PyObject *layer_forward_(PyObject *const *args) {
-  if (!engine_layer(args)) Py_RETURN_NONE;
-  const at::Tensor &x_in = tensor_of(args[2]);
+  const at::Tensor *xp = tensor_of(args[2]), *state, *mask_in;
+  if (!xp || !optional_tensor(args[4], state) || !optional_tensor(args[6], mask_in)) Py_RETURN_NONE;
+  const at::Tensor &x_in = *xp;
   LayerParts p;
-  collect(args[0], args[1], x_in, p);
+  if (x_in.dim() != 3 || x_in.size(1) < 2 || !collect(args[0], args[1], x_in, p)) Py_RETURN_NONE;
   const int64_t B = x_in.size(0), T = x_in.size(1);
-  if (T < 2 || B < 1) throw NotCovered{};
-  c10::OptionalDeviceGuard guard(x_in.device());
+  if (!sequence_fits(*p.cell, x_in, B, T, state, mask_in) || recording(*p.cell, x_in, state)) Py_RETURN_NONE;
   const void *taps = nullptr;
   int64_t taps_stride = 0;
   PyObject *prev = absent(args[3]) ? nullptr : first_of(args[3]);
-  if (!absent(prev)) taps = taps_of(p, tensor_of(prev), B, &taps_stride);
-  const bool last = args[5] == Py_True;
-  if (last && T < p.K - 1) throw NotCovered{};
-  const at::Tensor *state = optional_tensor(args[4]);
-  at::Tensor mask;
-  if (!absent(args[6])) mask = mask_bytes(tensor_of(args[6]), B, T);
-  const at::Tensor *maskp = mask.defined() ? &mask : nullptr;
-  {
-    const at::Tensor &r = p.cell->parameter(g_names.r), &b = p.cell->parameter(g_names.b);
-    if (p.cell->records(x_in, state, r, b)) throw NotCovered{};
-    if (state && (!state->is_cuda() || state->dim() != 3 || state->size(0) != 4 || state->size(1) != B || state->size(2) != p.D)) throw NotCovered{};
+  if (!absent(prev)) {
+    const at::Tensor *t = tensor_of(prev);
+    if (!t || !taps_of(p, *t, B, taps, taps_stride)) Py_RETURN_NONE;
   }
+  const bool last = args[5] == Py_True;
+  if (last && T < p.K - 1) Py_RETURN_NONE;
+  c10::OptionalDeviceGuard guard(x_in.device());
+  if (!have_word(*p.cell, x_in.device())) Py_RETURN_NONE;
+  at::Tensor mask;
+  if (mask_in) mask = mask_bytes(*mask_in);
+  const at::Tensor *maskp = mask_in ? &mask : nullptr;
   at::Tensor x = x_in.is_contiguous() && aligned(x_in.data_ptr(), 16) ? x_in : x_in.contiguous();
   void *stream = stream_of(x.device());
   at::Tensor wx = at::empty({B, T, 4 * p.D}, x.options()), x_conv = at::empty({B, T, p.D}, x.options());
@@ -924,8 +906,6 @@ PyObject *layer_call(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (!PyObject_TypeCheck(args[1], g_cell_type)) Py_RETURN_NONE;
   try {
     return F(args);
-  } catch (const NotCovered &) {
-    Py_RETURN_NONE;
   } catch (const PythonError &) {
     return nullptr;
   } catch (python_error &e) {
