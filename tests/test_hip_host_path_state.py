@@ -146,3 +146,23 @@ def test_methods_put_in_the_place_of_a_modules_are_called(monkeypatch, module, m
         monkeypatch.setattr(type(target), method, lambda self, *a, **kw: (calls.append(1), plain(self, *a, **kw))[1])
     # (the dropout runs behind the sequence and behind every step, the cell's forward and step once per call of that kind)
     assert torch.equal(run(), want) and len(calls) == {"forward": 3 if module == "dropout" else 1, "step": 2}[method]
+
+
+@pytest.mark.parametrize("trains", [False, True])
+def test_out_of_memory_is_reported_as_such(trains):
+    """Programs catch ``torch.OutOfMemoryError`` to go on with a smaller batch."""
+    print("case out of memory", trains, flush=True)
+    cell = _cell(2, 64)
+    x = torch.randn(8, 4096, 512, device=DEV, requires_grad=trains)
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)
+    try:
+        with torch.set_grad_enabled(trains), pytest.raises(torch.OutOfMemoryError):
+            held = [cell(x) for _ in range(64)]  # (16 MiB of outputs each)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    with torch.set_grad_enabled(trains):
+        assert bool(torch.isfinite(cell(x)[0]).all())
+    cell.check_status()

@@ -581,11 +581,8 @@ PyObject *cell_call(PyObject *self, PyObject *const *args, Py_ssize_t n) {
     return F(*((CellPathObject *)self)->c, args);
   } catch (const PythonError &) {
     return nullptr;
-  } catch (python_error &e) {
-    e.restore();
-    return nullptr;
-  } catch (const std::exception &e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
+  } catch (...) {  // (out of memory and the like: as the type that torch raises for it)
+    torch::translate_exception_to_python(std::current_exception());
     return nullptr;
   }
 }
@@ -908,11 +905,8 @@ PyObject *layer_call(PyObject *, PyObject *const *args, Py_ssize_t n) {
     return F(args);
   } catch (const PythonError &) {
     return nullptr;
-  } catch (python_error &e) {
-    e.restore();
-    return nullptr;
-  } catch (const std::exception &e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
+  } catch (...) {  // (out of memory and the like: as the type that torch raises for it)
+    torch::translate_exception_to_python(std::current_exception());
     return nullptr;
   }
 }
