@@ -70,6 +70,7 @@ enum {
  *                             ring through which the compute units of a head
  *                             pass h_t to each other (a few MiB).  Two calls
  *                             that may overlap in time need different workspaces;
+ *                             calls of several host threads on one stream may share one;
  *                             two sequence calls that overlap on one GPU also
  *                             compete for its compute units (each needs all of
  *                             its workgroups running at once), so one of them

@@ -626,7 +626,11 @@ class sLSTMCell_hip(nn.Module):
         with torch.cuda.device(input.device):
             fast = self._native().step(input, state, None, state_out, h_out, h_prev, self.config, self.keep_state_fp32)
         if fast is None:
-            raise ValueError("h_prev or state_out does not fit the step (dtype, size or device)")
+            size = B * self.config.hidden_size
+            if (any(t is not None and t.device != input.device for t in (state_out, h_out, h_prev)) or h_prev is not None
+                    and input.dtype == torch.bfloat16 and (h_prev.dtype != input.dtype or h_prev.numel() != size)):
+                raise ValueError("h_prev or state_out does not fit the step (dtype, size or device)")
+            return None  # (another thread has planned steps of another batch size meanwhile)
         rt.last_workspace = rt.step_plan[1].workspace
         return fast
 
@@ -641,7 +645,8 @@ class sLSTMCell_hip(nn.Module):
         if cached is None or cached[0] != key:
             plan = F_hip.StepPlan(B, r.detach(), b.detach().view(self.config.num_heads, 4, self.head_dim), wx_dtype=dtype)
             self._rt.step_plan = cached = (key, plan)
-            self._native().set_plan(plan, ctypes.addressof(plan._args), B, r, b)
+        plan = cached[1]
+        self._native().set_plan(plan, ctypes.addressof(plan._args), B, r, b)
         return True
 
 

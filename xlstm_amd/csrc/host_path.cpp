@@ -69,11 +69,22 @@ struct PyRef {  // owns one reference
 };
 
 struct PythonError {};  // a Python exception is set
-[[noreturn]] void engine_failed(int rc) {
-  PyErr_Format(g_engine.error, "xlstm_amd error %d: %s", rc, g_engine.last_error());
-  throw PythonError{};
+struct EngineFailed { std::string what; };  // an entry point of the engine said no (thrown without the GIL)
+inline void launched(int rc) {
+  if (rc != XS_OK) throw EngineFailed{"xlstm_amd error " + std::to_string(rc) + ": " + g_engine.last_error()};
 }
-inline void launched(int rc) { if (rc != XS_OK) engine_failed(rc); }
+
+// The GIL is given up around allocations (which may reach the driver) and launches (which block when a queue is full), so
+// that the other Python threads of a serving process run on.  What a call has of a cell is therefore taken with the GIL
+// held - tensors and argument blocks by value, the plan by a reference of its own - and what it leaves there is written
+// with the GIL held again: another thread may be in the same cell meanwhile.
+struct WithoutGil {
+  PyThreadState *state = PyEval_SaveThread();
+  WithoutGil() = default;
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+  WithoutGil(const WithoutGil &) = delete;
+  WithoutGil &operator=(const WithoutGil &) = delete;
+};
 
 inline const at::Tensor *tensor_of(PyObject *o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }  // or null
 inline bool absent(PyObject *o) { return o == nullptr || o == Py_None; }
@@ -163,25 +174,35 @@ struct CellPath {
     return at::GradMode::is_enabled() && (x.requires_grad() || r.requires_grad() || b.requires_grad() || (state && state->requires_grad()));
   }
 
-  at::Tensor &workspace(int64_t B, const at::Device &d) {
+  at::Tensor workspace(int64_t B, const at::Device &d) {
     void *stream = stream_of(d);
     const size_t need = g_engine.workspace_bytes((int32_t)B, 1, (int32_t)NH, (int32_t)dh);
-    Workspace *w = nullptr;
-    for (auto &it : workspaces)
-      if (it.device == d.index() && it.stream == stream) { w = &it; break; }
-    if (!w) {
-      // (a program that makes a new stream per call would otherwise collect workspaces without end; a stream's
-      // allocations are handed on in stream order by the caching allocator, so dropping the oldest is safe - unless
-      // it was used under capture: replays of the graph write it for as long as the graph lives)
-      if (workspaces.size() >= 16)
-        for (auto it = workspaces.begin(); it != workspaces.end(); ++it)
-          if (!it->captured) { workspaces.erase(it); break; }
-      workspaces.push_back(Workspace{(int)d.index(), stream, at::Tensor()});
-      w = &workspaces.back();
-    }
-    if (!w->t.defined() || (size_t)w->t.numel() < need) {
-      if (w->captured) captured.push_back(w->t);
-      w->t = at::empty({(int64_t)need}, at::TensorOptions().dtype(at::kByte).device(d));
+    auto find = [&]() -> Workspace * {
+      for (auto &it : workspaces)
+        if (it.device == d.index() && it.stream == stream) return &it;
+      return nullptr;
+    };
+    Workspace *w = find();
+    if (!w || (size_t)w->t.numel() < need) {
+      at::Tensor fresh;
+      {
+        WithoutGil no_gil;
+        fresh = at::empty({(int64_t)need}, at::TensorOptions().dtype(at::kByte).device(d));
+      }
+      w = find();
+      if (!w) {
+        // (a program that makes a new stream per call would otherwise collect workspaces without end; a stream's
+        // allocations are handed on in stream order by the caching allocator, so dropping the oldest is safe - unless
+        // it was used under capture: replays of the graph write it for as long as the graph lives)
+        if (workspaces.size() >= 16)
+          for (auto it = workspaces.begin(); it != workspaces.end(); ++it)
+            if (!it->captured) { workspaces.erase(it); break; }
+        workspaces.push_back(Workspace{(int)d.index(), stream, fresh});
+        w = &workspaces.back();
+      } else if ((size_t)w->t.numel() < need) {
+        if (w->captured) captured.push_back(w->t);
+        w->t = fresh;
+      }
     }
     w->captured |= capturing(d);
     return w->t;
@@ -253,41 +274,57 @@ bool step_fits(const CellPath &c, const at::Tensor &x, const at::Tensor &state, 
   return state_like(state) && (!s.state_out || state_like(*s.state_out)) && (!s.h_out || (h_like(*s.h_out) && s.h_out->is_contiguous())) &&
          (!s.h_prev || dt != at::kBFloat16 || h_like(*s.h_prev));
 }
-struct StepResult { at::Tensor h, state; };  // h: [1,B,H] memory, state: float32 [4,B,H]
-// (wx: contiguous [B,1,4H]; everything else as step_fits has found it)
-StepResult run_step(CellPath &c, const at::Tensor &wx, const at::Tensor &state, const StepBuffers &s, const Shape4 *h_shape, bool keep_state) {
-  const int64_t B = c.step_B, H = c.NH * c.dh;
-  StepResult out;
-  if (s.h_out) out.h = *s.h_out;
-  else if (h_shape) out.h = at::empty_strided(at::IntArrayRef(h_shape->size.data(), h_shape->n), at::IntArrayRef(h_shape->stride.data(), h_shape->n), wx.options());
-  else out.h = at::empty({1, B, H}, wx.options());
-  out.state = s.state_out ? *s.state_out : at::empty({4, B, H}, state.options());
-  xs_slstm_args &a = *c.step_args;
-  a.h_prev = nullptr;
-  if (c.step_dtype == at::kBFloat16) {
-    if (s.h_prev) {
-      a.h_prev = s.h_prev->data_ptr();
-    } else if (c.last_state.defined() && c.last_state.is_same(state) && versioned(state) && version_of(state) == c.last_state_version &&
-               version_of(c.last_h) == c.last_h_version && c.last_h.data_ptr() != out.h.data_ptr()) {
-      // The state this cell handed out last time comes back untouched: the h it returned with it is that state's y
-      // plane in bfloat16, the operand the step kernel wants (half the bytes, and the pipelined kernel).
-      a.h_prev = c.last_h.data_ptr();
+// one decode step of the cell's plan: made and left with the GIL held, run without it
+struct Step {
+  CellPath &c;
+  PyRef plan;        // (it owns the R and the bias that the argument block points to)
+  xs_slstm_args a;
+  const int64_t B, H;
+  const at::Device device;
+  const at::ScalarType dtype;
+  at::Tensor last_state, last_h;
+  uint32_t last_state_version, last_h_version;
+  at::Tensor h, state;  // h: [1,B,H] memory, state: float32 [4,B,H]
+
+  explicit Step(CellPath &cell)
+      : c(cell), plan(cell.plan), a(*cell.step_args), B(cell.step_B), H(cell.NH * cell.dh), device(cell.device), dtype(cell.step_dtype),
+        last_state(cell.last_state), last_h(cell.last_h), last_state_version(cell.last_state_version), last_h_version(cell.last_h_version) {
+    Py_INCREF(plan.o);
+  }
+  // wx: contiguous [B,1,4H]; everything else as step_fits has found it
+  void run(const at::Tensor &wx, const at::Tensor &s0, const StepBuffers &s, const Shape4 *h_shape) {
+    if (s.h_out) h = *s.h_out;
+    else if (h_shape) h = at::empty_strided(at::IntArrayRef(h_shape->size.data(), h_shape->n), at::IntArrayRef(h_shape->stride.data(), h_shape->n), wx.options());
+    else h = at::empty({1, B, H}, wx.options());
+    state = s.state_out ? *s.state_out : at::empty({4, B, H}, s0.options());
+    a.h_prev = nullptr;
+    if (dtype == at::kBFloat16) {
+      if (s.h_prev) {
+        a.h_prev = s.h_prev->data_ptr();
+      } else if (last_state.defined() && last_state.is_same(s0) && versioned(s0) && version_of(s0) == last_state_version &&
+                 version_of(last_h) == last_h_version && last_h.data_ptr() != h.data_ptr()) {
+        // The state this cell handed out last time comes back untouched: the h it returned with it is that state's y
+        // plane in bfloat16, the operand the step kernel wants (half the bytes, and the pipelined kernel).
+        a.h_prev = last_h.data_ptr();
+      }
+    }
+    a.wx = wx.data_ptr();
+    a.s0 = (const float *)s0.data_ptr();
+    a.s_out = (float *)state.data_ptr();
+    a.h_out = h.data_ptr();
+    a.stream = stream_of(device);
+    launched(g_engine.step(&a));
+  }
+  void leave(bool keep_state) {
+    if (c.plan == plan.o) *c.step_args = a;  // (the plan's block describes its last step)
+    if (keep_state && versioned(state) && versioned(h)) {
+      c.last_state = state; c.last_state_version = version_of(state);
+      c.last_h = h; c.last_h_version = version_of(h);
+    } else {
+      c.last_state.reset(); c.last_h.reset();
     }
   }
-  a.wx = wx.data_ptr();
-  a.s0 = (const float *)state.data_ptr();
-  a.s_out = (float *)out.state.data_ptr();
-  a.h_out = out.h.data_ptr();
-  a.stream = stream_of(c.device);
-  launched(g_engine.step(&a));
-  if (keep_state && versioned(out.state) && versioned(out.h)) {
-    c.last_state = out.state; c.last_state_version = version_of(out.state);
-    c.last_h = out.h; c.last_h_version = version_of(out.h);
-  } else {
-    c.last_state.reset(); c.last_h.reset();
-  }
-  return out;
-}
+};
 
 bool recording(const CellPath &c, const at::Tensor &x, const at::Tensor *state) {
   if (!at::GradMode::is_enabled()) return false;
@@ -307,15 +344,21 @@ PyObject *cell_step_(CellPath &c, PyObject *const *args) {
   const bool keep = args[7] == Py_True;
   c10::OptionalDeviceGuard guard(c.device);
   const Shape4 s4 = shape_of(shape, 1, c.step_B, c.NH, c.dh);
-  StepResult r = run_step(c, *x, *state, s, &s4, keep);
-  at::Tensor h = s.h_out ? r.h.as_strided(at::IntArrayRef(s4.size.data(), s4.n), at::IntArrayRef(s4.stride.data(), s4.n)) : r.h;
-  PyRef ph(THPVariable_Wrap(h)), ps(THPVariable_Wrap(keep || x->scalar_type() == at::kFloat ? r.state : r.state.to(x->scalar_type())));
+  Step step(c);
+  at::Tensor h, state_out;
+  {
+    WithoutGil no_gil;
+    step.run(*x, *state, s, &s4);
+    h = s.h_out ? step.h.as_strided(at::IntArrayRef(s4.size.data(), s4.n), at::IntArrayRef(s4.stride.data(), s4.n)) : step.h;
+    state_out = keep || step.dtype == at::kFloat ? step.state : step.state.to(step.dtype);
+  }
+  step.leave(keep);
+  PyRef ph(THPVariable_Wrap(h)), ps(THPVariable_Wrap(state_out));
   if (!ph.o || !ps.o) throw PythonError{};
   return PyTuple_Pack(2, ph.o, ps.o);
 }
 
 // ---- a sequence through the cell (no autograd), as sLSTMCell_hip._run and functional.slstm_forward do it
-struct Sequence { at::Tensor h, state, coef, mask; };  // h: [S,B,H] memory with the strides of `shape`, state: float32
 bool mask_fits(const at::Tensor *m, int64_t B, int64_t T) { return !m || (m->is_cuda() && m->dim() == 2 && m->size(0) == B && m->size(1) == T); }
 at::Tensor mask_bytes(const at::Tensor &m) {
   at::Tensor r = m;
@@ -336,55 +379,71 @@ bool sequence_fits(const CellPath &c, const at::Tensor &x, int64_t B, int64_t T,
 }
 // the cell's abort word, made on first use (under capture there is none: no host memory is allocated, and a replay reports to nobody)
 bool have_word(CellPath &c, const at::Device &d) {
-  if (!c.abort_word && !capturing(d)) c.abort_word = take_word();
-  return c.abort_word || capturing(d);
+  if (c.abort_word || capturing(d)) return true;
+  AbortWord word;
+  {
+    WithoutGil no_gil;
+    word = take_word();
+  }
+  if (!c.abort_word) c.abort_word = std::move(word);
+  return c.abort_word != nullptr;
 }
 
-// train: the forward of a training call, which also leaves the backward pass its coefficients (no graph is recorded here)
-// (x: [B,T,4H] as sequence_fits has found it)
-Sequence run_sequence(CellPath &c, at::Tensor x, const at::Tensor *state, const at::Tensor *mask, OutShape shape, bool train = false) {
-  const int64_t H = c.NH * c.dh, B = x.size(0), T = x.size(1);
-  const auto dt = x.scalar_type();
-  const at::Tensor *rp, *bp;
-  if (!c.weights(rp, bp)) { PyErr_SetString(PyExc_RuntimeError, "the cell has lost its parameters"); throw PythonError{}; }
-  at::Tensor r = *rp, b = *bp;
-  const size_t esz = x.element_size();
-  if (x.stride(2) != 1 || !aligned(x.data_ptr(), 16) || (x.stride(0) * esz) % 16 || (x.stride(1) * esz) % 16 || x.stride(1) < 4 * H ||
-      (B > 1 && x.stride(0) < 4 * H))
-    x = x.contiguous();
-  if (dt == at::kFloat && r.scalar_type() != at::kFloat) r = r.to(at::kFloat);
-  if (b.scalar_type() != at::kFloat) b = b.to(at::kFloat);  // (on every call: a copy kept would be another stream's, and a graph's)
-  at::Tensor s0, m;
-  if (state) s0 = state->to(at::kFloat).contiguous();
-  if (mask) m = mask_bytes(*mask);
-  const bool in_graph = capturing(x.device());
-  if (!in_graph) c.raise_if_aborted();
-  const Shape4 s4 = shape_of(shape, T, B, c.NH, c.dh);
-  Sequence out;
-  out.h = at::empty_strided(at::IntArrayRef(s4.size.data(), s4.n), at::IntArrayRef(s4.stride.data(), s4.n), x.options());
-  out.state = at::empty({4, B, H}, x.options().dtype(at::kFloat));
-  if (train) {
-    const size_t n = g_engine.coef_floats((int32_t)B, (int32_t)T, (int32_t)c.NH, (int32_t)c.dh, dtype_code(dt));
-    out.coef = at::empty({(int64_t)n}, out.state.options());
+// A sequence through the cell: made and left with the GIL held, run without it.  train: the forward of a training call, which
+// also leaves the backward pass its coefficients (no graph is recorded here)
+struct Sequence {
+  CellPath &c;
+  at::Tensor r, b;
+  const bool in_graph;
+  AbortWord word;
+  at::Tensor ws;
+  at::Tensor h, state, coef, mask;  // h: [T,B,H] memory with the strides of `shape`, state: float32, mask: bytes
+
+  Sequence(CellPath &cell, const at::Device &device, int64_t B) : c(cell), in_graph(capturing(device)) {
+    const at::Tensor *rp, *bp;
+    if (!c.weights(rp, bp)) { PyErr_SetString(PyExc_RuntimeError, "the cell has lost its parameters"); throw PythonError{}; }
+    r = *rp; b = *bp;
+    if (!in_graph) c.raise_if_aborted();
+    word = in_graph ? nullptr : c.abort_word;
+    ws = c.workspace(B, device);
   }
-  at::Tensor &ws = c.workspace(B, x.device());
-  xs_slstm_args a{};
-  a.B = (int32_t)B; a.T = (int32_t)T; a.NH = (int32_t)c.NH; a.dh = (int32_t)c.dh;
-  a.wx_dtype = dtype_code(dt); a.r_dtype = dtype_code(r.scalar_type());
-  a.wx = x.data_ptr(); a.wx_stride_b = x.stride(0); a.wx_stride_t = x.stride(1);
-  a.r = r.data_ptr(); a.bias = (const float *)b.data_ptr();
-  a.s0 = state ? (const float *)s0.data_ptr() : nullptr;
-  a.reset = mask ? (const uint8_t *)m.data_ptr() : nullptr; a.reset_stride_b = mask ? m.stride(0) : 0;
-  a.h_out = out.h.data_ptr(); a.s_out = (float *)out.state.data_ptr();
-  a.workspace = ws.data_ptr(); a.workspace_bytes = (size_t)ws.numel();
-  a.stream = stream_of(x.device());
-  uint32_t *word = in_graph ? nullptr : c.abort_word.get();
-  launched(train ? g_engine.train_forward(&a, (float *)out.coef.data_ptr(), word) : g_engine.forward(&a, word));
-  out.mask = m;
-  c.last_workspace = ws;
-  if (x.device().index() < 64) c.devices_used |= 1ull << x.device().index();
-  return out;
-}
+  // x: [B,T,4H] as sequence_fits has found it
+  void run(at::Tensor x, const at::Tensor *s_in, const at::Tensor *mask_in, OutShape shape, bool train = false) {
+    const int64_t H = c.NH * c.dh, B = x.size(0), T = x.size(1);
+    const auto dt = x.scalar_type();
+    const size_t esz = x.element_size();
+    if (x.stride(2) != 1 || !aligned(x.data_ptr(), 16) || (x.stride(0) * esz) % 16 || (x.stride(1) * esz) % 16 || x.stride(1) < 4 * H ||
+        (B > 1 && x.stride(0) < 4 * H))
+      x = x.contiguous();
+    if (dt == at::kFloat && r.scalar_type() != at::kFloat) r = r.to(at::kFloat);
+    if (b.scalar_type() != at::kFloat) b = b.to(at::kFloat);  // (on every call: a copy kept would be another stream's, and a graph's)
+    at::Tensor s0;
+    if (s_in) s0 = s_in->to(at::kFloat).contiguous();
+    if (mask_in) mask = mask_bytes(*mask_in);
+    const Shape4 s4 = shape_of(shape, T, B, c.NH, c.dh);
+    h = at::empty_strided(at::IntArrayRef(s4.size.data(), s4.n), at::IntArrayRef(s4.stride.data(), s4.n), x.options());
+    state = at::empty({4, B, H}, x.options().dtype(at::kFloat));
+    if (train) {
+      const size_t n = g_engine.coef_floats((int32_t)B, (int32_t)T, (int32_t)c.NH, (int32_t)c.dh, dtype_code(dt));
+      coef = at::empty({(int64_t)n}, state.options());
+    }
+    xs_slstm_args a{};
+    a.B = (int32_t)B; a.T = (int32_t)T; a.NH = (int32_t)c.NH; a.dh = (int32_t)c.dh;
+    a.wx_dtype = dtype_code(dt); a.r_dtype = dtype_code(r.scalar_type());
+    a.wx = x.data_ptr(); a.wx_stride_b = x.stride(0); a.wx_stride_t = x.stride(1);
+    a.r = r.data_ptr(); a.bias = (const float *)b.data_ptr();
+    a.s0 = s_in ? (const float *)s0.data_ptr() : nullptr;
+    a.reset = mask_in ? (const uint8_t *)mask.data_ptr() : nullptr; a.reset_stride_b = mask_in ? mask.stride(0) : 0;
+    a.h_out = h.data_ptr(); a.s_out = (float *)state.data_ptr();
+    a.workspace = ws.data_ptr(); a.workspace_bytes = (size_t)ws.numel();
+    a.stream = stream_of(x.device());
+    launched(train ? g_engine.train_forward(&a, (float *)coef.data_ptr(), word.get()) : g_engine.forward(&a, word.get()));
+  }
+  void leave() {
+    c.last_workspace = ws;
+    if (ws.device().index() < 64) c.devices_used |= 1ull << ws.device().index();
+  }
+};
 
 // forward(input, state, reset_mask, config, keep_state_fp32) -> (output, state) or None
 PyObject *cell_forward_(CellPath &c, PyObject *const *args) {
@@ -398,8 +457,16 @@ PyObject *cell_forward_(CellPath &c, PyObject *const *args) {
   if (!out_shape(args[3], shape) || x.size(2) != 4 * c.NH * c.dh || !sequence_fits(c, x, x.size(bsgnh ? 0 : 1), x.size(bsgnh ? 1 : 0), state, mask)) Py_RETURN_NONE;
   c10::OptionalDeviceGuard guard(x.device());
   if (!have_word(c, x.device())) Py_RETURN_NONE;
-  Sequence s = run_sequence(c, bsgnh ? x : x.permute({1, 0, 2}), state, mask, shape);
-  PyRef ph(THPVariable_Wrap(s.h)), ps(THPVariable_Wrap(args[4] == Py_True || x.scalar_type() == at::kFloat ? s.state : s.state.to(x.scalar_type())));
+  const bool keep = args[4] == Py_True || x.scalar_type() == at::kFloat;
+  Sequence s(c, x.device(), x.size(bsgnh ? 0 : 1));
+  at::Tensor state_out;
+  {
+    WithoutGil no_gil;
+    s.run(bsgnh ? x : x.permute({1, 0, 2}), state, mask, shape);
+    state_out = keep ? s.state : s.state.to(x.scalar_type());
+  }
+  s.leave();
+  PyRef ph(THPVariable_Wrap(s.h)), ps(THPVariable_Wrap(state_out));
   if (!ph.o || !ps.o) throw PythonError{};
   return PyTuple_Pack(2, ph.o, ps.o);
 }
@@ -544,12 +611,15 @@ PyObject *cell_train_(CellPath &c, PyObject *const *args) {
   if (PyErr_Occurred()) throw PythonError{};
   c10::OptionalDeviceGuard guard(x.device());
   if (!have_word(c, x.device())) Py_RETURN_NONE;
-  Sequence s;
+  const bool keep = args[4] == Py_True || x.scalar_type() == at::kFloat;
+  Sequence s(c, x.device(), x.size(bsgnh ? 0 : 1));
+  const at::Tensor r = s.r, b = s.b;
+  at::Tensor state_out;
   {
-    const at::Tensor r = *rp, b = *bp;
+    WithoutGil no_gil;
     {
       at::NoGradGuard no_grad;
-      s = run_sequence(c, bsgnh ? x : x.permute({1, 0, 2}), state, mask, shape, true);
+      s.run(bsgnh ? x : x.permute({1, 0, 2}), state, mask, shape, true);
     }
     auto node = std::shared_ptr<CellBackward>(new CellBackward(), torch::autograd::deleteNode);
     node->set_next_edges(state ? torch::autograd::collect_next_edges(x, r, b, *state) : torch::autograd::collect_next_edges(x, r, b));
@@ -562,14 +632,16 @@ PyObject *cell_train_(CellPath &c, PyObject *const *args) {
     node->transposed_input = !bsgnh;
     node->shape = shape;
     node->r_dtype = r.scalar_type(); node->b_dtype = b.scalar_type();
-    node->in.mask = s.mask; node->in.word = c.abort_word;
+    node->in.mask = s.mask; node->in.word = s.word;
     node->in.B = s.state.size(1); node->in.T = x.size(bsgnh ? 1 : 0); node->in.NH = c.NH; node->in.dh = c.dh;
     node->in.cut = cut_on != 0; node->in.clip = clipval;
     torch::autograd::set_history(s.h, node);
     torch::autograd::set_history(s.state, node);
     node->h = SavedVariable(s.h, true);
+    state_out = keep ? s.state : s.state.to(x.scalar_type());
   }
-  PyRef ph(THPVariable_Wrap(s.h)), ps(THPVariable_Wrap(args[4] == Py_True || x.scalar_type() == at::kFloat ? s.state : s.state.to(x.scalar_type())));
+  s.leave();
+  PyRef ph(THPVariable_Wrap(s.h)), ps(THPVariable_Wrap(state_out));
   if (!ph.o || !ps.o) throw PythonError{};
   return PyTuple_Pack(2, ph.o, ps.o);
 }
@@ -580,6 +652,9 @@ PyObject *cell_call(PyObject *self, PyObject *const *args, Py_ssize_t n) {
   try {
     return F(*((CellPathObject *)self)->c, args);
   } catch (const PythonError &) {
+    return nullptr;
+  } catch (const EngineFailed &e) {
+    PyErr_SetString(g_engine.error, e.what.c_str());
     return nullptr;
   } catch (...) {  // (out of memory and the like: as the type that torch raises for it)
     torch::translate_exception_to_python(std::current_exception());
@@ -830,10 +905,12 @@ PyObject *layer_step_(PyObject *const *args) {
   if (B < 1) Py_RETURN_NONE;
   const void *taps = nullptr;
   int64_t taps_stride = 0;
+  at::Tensor before;  // (held: it may come in a list, which another thread may change)
   PyObject *prev = absent(args[3]) ? nullptr : first_of(args[3]);
   if (!absent(prev)) {
     const at::Tensor *t = tensor_of(prev);
     if (!t || t->dim() != 3 || (t->size(1) != p.K && t->size(1) != p.K - 1) || !taps_of(p, *t, B, taps, taps_stride)) Py_RETURN_NONE;  // (the general path asserts)
+    before = *t;
   }
   const auto opts = x.options();
   if (ring_out && (ring_out->scalar_type() != at::kBFloat16 || ring_out->dim() != 3 || ring_out->size(0) != B || ring_out->size(1) != p.K ||
@@ -841,18 +918,25 @@ PyObject *layer_step_(PyObject *const *args) {
     Py_RETURN_NONE;
   if (out_given && (out_given->scalar_type() != at::kBFloat16 || out_given->numel() != B * p.D || !out_given->is_contiguous())) Py_RETURN_NONE;
   c10::OptionalDeviceGuard guard(x.device());
-  void *stream = stream_of(x.device());
-  at::Tensor ring = ring_out ? *ring_out : at::empty({B, p.K, p.D}, opts);
-  at::Tensor wx = at::empty({B, 1, 4 * p.D}, opts), x_conv = at::empty({B, 1, p.D}, opts);
-  run_conv(p, x, taps, taps_stride, nullptr, x_conv.data_ptr(), ring.data_ptr(), stream);
-  run_gates(p, x, x_conv.data_ptr(), wx.data_ptr(), stream);
-  StepResult s = run_step(c, wx, state, buffers, nullptr, p.keep_state);
-  at::Tensor out = out_given ? *out_given : at::empty({B, 1, p.D}, opts);
-  run_norm(p, s.h, B, 1, out.data_ptr(), stream);
+  Step step(c);
+  at::Tensor ring, out, state_out;
+  {
+    WithoutGil no_gil;
+    void *stream = stream_of(x.device());
+    ring = ring_out ? *ring_out : at::empty({B, p.K, p.D}, opts);
+    at::Tensor wx = at::empty({B, 1, 4 * p.D}, opts), x_conv = at::empty({B, 1, p.D}, opts);
+    run_conv(p, x, taps, taps_stride, nullptr, x_conv.data_ptr(), ring.data_ptr(), stream);
+    run_gates(p, x, x_conv.data_ptr(), wx.data_ptr(), stream);
+    step.run(wx, state, buffers, nullptr);
+    out = out_given ? *out_given : at::empty({B, 1, p.D}, opts);
+    run_norm(p, step.h, B, 1, out.data_ptr(), stream);
+    state_out = p.keep_state ? step.state : step.state.to(at::kBFloat16);
+  }
+  step.leave(p.keep_state);
   PyRef po(THPVariable_Wrap(out)), pr(THPVariable_Wrap(ring)), tuple(nullptr);
   if (!po.o || !pr.o) throw PythonError{};
   tuple.o = PyTuple_Pack(1, pr.o);
-  PyRef states(states_dict(tuple.o, p.keep_state ? s.state : s.state.to(at::kBFloat16)));
+  PyRef states(states_dict(tuple.o, state_out));
   return PyTuple_Pack(2, po.o, states.o);
 }
 
@@ -867,33 +951,45 @@ PyObject *layer_forward_(PyObject *const *args) {
   if (!sequence_fits(*p.cell, x_in, B, T, state, mask_in) || recording(*p.cell, x_in, state)) Py_RETURN_NONE;
   const void *taps = nullptr;
   int64_t taps_stride = 0;
+  at::Tensor before;  // (held: it may come in a list, which another thread may change)
   PyObject *prev = absent(args[3]) ? nullptr : first_of(args[3]);
   if (!absent(prev)) {
     const at::Tensor *t = tensor_of(prev);
     if (!t || !taps_of(p, *t, B, taps, taps_stride)) Py_RETURN_NONE;
+    before = *t;
   }
   const bool last = args[5] == Py_True;
   if (last && T < p.K - 1) Py_RETURN_NONE;
   c10::OptionalDeviceGuard guard(x_in.device());
   if (!have_word(*p.cell, x_in.device())) Py_RETURN_NONE;
-  at::Tensor mask;
-  if (mask_in) mask = mask_bytes(*mask_in);
-  const at::Tensor *maskp = mask_in ? &mask : nullptr;
-  at::Tensor x = x_in.is_contiguous() && aligned(x_in.data_ptr(), 16) ? x_in : x_in.contiguous();
-  void *stream = stream_of(x.device());
-  at::Tensor wx = at::empty({B, T, 4 * p.D}, x.options()), x_conv = at::empty({B, T, p.D}, x.options());
-  run_conv(p, x, taps, taps_stride, maskp, x_conv.data_ptr(), nullptr, stream);
-  run_gates(p, x, x_conv.data_ptr(), wx.data_ptr(), stream);
-  Sequence s = run_sequence(*p.cell, wx, state, maskp, OutShape::SBH);
-  at::Tensor out = x_conv;  // (its last reader has been launched in front of the norm)
-  run_norm(p, s.h, B, T, out.data_ptr(), stream);
+  Sequence s(*p.cell, x_in.device(), B);
+  at::Tensor out, tail, state_out;
+  {
+    WithoutGil no_gil;
+    at::Tensor mask;
+    if (mask_in) mask = mask_bytes(*mask_in);
+    const at::Tensor *maskp = mask_in ? &mask : nullptr;
+    at::Tensor x = x_in.is_contiguous() && aligned(x_in.data_ptr(), 16) ? x_in : x_in.contiguous();
+    void *stream = stream_of(x.device());
+    at::Tensor wx = at::empty({B, T, 4 * p.D}, x.options()), x_conv = at::empty({B, T, p.D}, x.options());
+    run_conv(p, x, taps, taps_stride, maskp, x_conv.data_ptr(), nullptr, stream);
+    run_gates(p, x, x_conv.data_ptr(), wx.data_ptr(), stream);
+    s.run(wx, state, maskp, OutShape::SBH);
+    out = x_conv;  // (its last reader has been launched in front of the norm)
+    run_norm(p, s.h, B, T, out.data_ptr(), stream);
+    if (last) {
+      // the last K-1 inputs: a tensor of their own where the call continued a state (x may be reused for the next chunk)
+      tail = x_in.narrow(1, T - (p.K - 1), p.K - 1);
+      if (taps) tail = tail.clone();
+      state_out = p.keep_state ? s.state : s.state.to(at::kBFloat16);
+    }
+  }
+  s.leave();
   PyRef po(THPVariable_Wrap(out));
   if (!po.o) throw PythonError{};
   if (!last) return po.release();
-  // the last K-1 inputs: a tensor of their own where the call continued a state (x may be reused for the next chunk)
-  at::Tensor tail = x_in.narrow(1, T - (p.K - 1), p.K - 1);
-  PyRef pt(THPVariable_Wrap(taps ? tail.clone() : tail));
-  PyRef states(states_dict(pt.o, p.keep_state ? s.state : s.state.to(at::kBFloat16)));
+  PyRef pt(THPVariable_Wrap(tail));
+  PyRef states(states_dict(pt.o, state_out));
   return PyTuple_Pack(2, po.o, states.o);
 }
 
@@ -904,6 +1000,9 @@ PyObject *layer_call(PyObject *, PyObject *const *args, Py_ssize_t n) {
   try {
     return F(args);
   } catch (const PythonError &) {
+    return nullptr;
+  } catch (const EngineFailed &e) {
+    PyErr_SetString(g_engine.error, e.what.c_str());
     return nullptr;
   } catch (...) {  // (out of memory and the like: as the type that torch raises for it)
     torch::translate_exception_to_python(std::current_exception());

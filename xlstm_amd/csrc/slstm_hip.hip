@@ -504,6 +504,14 @@ int run_train_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_s
   return e == hipSuccess ? XS_OK : fail(XS_ERR_LAUNCH, "backward kernel launch failed: %s", hipGetErrorString(e));
 }
 
+// Calls of several host threads that share a workspace and a stream run one after the other on the device, but only if the
+// launches of one call - the workspace is cleared, then used - are not interleaved with another's: a call holds the lock of
+// its workspace while it launches.
+std::mutex &launches_into(const void *workspace) {
+  static std::mutex mu[64];
+  return mu[((uintptr_t)workspace >> 8) % 64];
+}
+
 // need != nullptr: launch nothing, only say whether a kernel takes every launch of this call and how many bytes of
 // workspace they touch
 int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_host = nullptr, float *train_coef = nullptr) {
@@ -555,6 +563,8 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
     const int rc = run_forward(a, &bytes, nullptr, train_coef);
     if (rc != XS_OK) return rc;
   }
+  std::unique_lock<std::mutex> launches;
+  if (!dry) launches = std::unique_lock<std::mutex>(launches_into(a->workspace));
   int launch_no = 0;
   for (int head0 = 0; head0 < NH; head0 += heads_per_launch) {
   const int NHL = head0 + heads_per_launch <= NH ? heads_per_launch : NH - head0;
