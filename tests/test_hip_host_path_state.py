@@ -166,3 +166,43 @@ def test_out_of_memory_is_reported_as_such(trains):
     with torch.set_grad_enabled(trains):
         assert bool(torch.isfinite(cell(x)[0]).all())
     cell.check_status()
+
+
+@pytest.mark.parametrize("trains", [False, True])
+def test_check_status_waits_for_the_cells_own_calls(trains):
+    """All of them, and not what other streams of the device run."""
+    import time
+
+    print("case check_status", trains, flush=True)
+    cell = _cell(2, 64)
+    x = torch.randn(2, 16384, 512, device=DEV, requires_grad=trains)  # (some 8 ms in one direction)
+    a = torch.randn(8192, 8192, device=DEV, dtype=torch.bfloat16)
+    others, own = torch.cuda.Event(), torch.cuda.Event()
+
+    def busy_elsewhere():  # some 0.3 s on a stream whose hardware queue is not the current stream's
+        for side in [torch.cuda.Stream() for _ in range(8)]:
+            torch.cuda.synchronize()
+            with torch.cuda.stream(side):
+                for _ in range(400):
+                    a @ a
+                others.record()
+            a[0].clone()
+            own.record()
+            own.synchronize()
+            if not others.query():
+                return
+        pytest.skip("every stream shares the current one's hardware queue")
+
+    with torch.set_grad_enabled(trains):
+        torch.autograd.grad(cell(x)[0].sum(), x) if trains else cell(x)  # (loads the kernels)
+        busy_elsewhere()
+        begin = time.perf_counter()
+        out, _ = cell(x)
+        if trains:
+            torch.autograd.grad(out, x, torch.ones_like(out))
+        cell.check_status()
+        waited, pending = time.perf_counter() - begin, not others.query()
+        own.record()
+        own.synchronize()
+        rest = time.perf_counter() - begin - waited
+    assert pending and waited > 4e-3 and rest < 0.5 * waited, (pending, waited, rest)
