@@ -151,9 +151,8 @@ class MultiHeadLayerNorm(nn.Module):
         return out.view(B, S, NH, DH).transpose(1, 2)
 
 
-# the methods that the native host path of a layer stands in for, and what replaces them in a module's own dictionary
-_STOOD_IN_FOR = (sLSTMCell_hip.forward, sLSTMCell_hip.step, nn.Dropout.forward)
-_REPLACEABLE = frozenset(("forward", "step", "_compiled_call_impl"))
+# the methods that the native host path of a layer stands in for
+_CELL_FORWARD, _CELL_STEP, _DROPOUT_FORWARD = sLSTMCell_hip.forward, sLSTMCell_hip.step, nn.Dropout.forward
 
 
 class sLSTMLayer(nn.Module):
@@ -202,10 +201,14 @@ class sLSTMLayer(nn.Module):
         """Whether cell and dropout are what the constructor made, which the native host path runs without calling them (a
         wrapper or a subclass in their place, a method replaced on the module or its class, a module compiled in place
         is called)."""
-        cell, dropout = self.slstm_cell, self.dropout
-        return (type(cell) is sLSTMCell_hip and type(dropout) is nn.Dropout
-                and _REPLACEABLE.isdisjoint(cell.__dict__) and _REPLACEABLE.isdisjoint(dropout.__dict__)
-                and (sLSTMCell_hip.forward, sLSTMCell_hip.step, nn.Dropout.forward) == _STOOD_IN_FOR)
+        cell, dropout = self._modules["slstm_cell"], self._modules["dropout"]
+        if type(cell) is not sLSTMCell_hip or type(dropout) is not nn.Dropout:
+            return False
+        of_cell, of_dropout = cell.__dict__, dropout.__dict__
+        return ("forward" not in of_cell and "step" not in of_cell and "_compiled_call_impl" not in of_cell
+                and "forward" not in of_dropout and "_compiled_call_impl" not in of_dropout
+                and sLSTMCell_hip.forward is _CELL_FORWARD and sLSTMCell_hip.step is _CELL_STEP
+                and nn.Dropout.forward is _DROPOUT_FORWARD)
 
     def _engine_ops_allowed(self, t) -> bool:
         # the engine's kernels record no autograd graph: under grad mode the PyTorch ops run, and a backward pass
