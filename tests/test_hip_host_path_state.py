@@ -108,6 +108,31 @@ def test_modules_put_in_the_place_of_a_layers_are_called():
         assert torch.equal(layer(x), plain) and layer.slstm_cell.calls == 1
 
 
+def test_plan_of_a_graph_outlives_other_batch_sizes():
+    """A decoder's graphs, then eager steps of another batch size and of changed parameters on the same layer, with every block
+    that is free given back to the driver: replays still read the R and the bias that they were recorded with."""
+    from xlstm_amd.decode import GraphedLayerDecoder
+    from xlstm_amd.layer import sLSTMLayer, sLSTMLayerConfig
+
+    print("case graph and plans", flush=True)
+    torch.manual_seed(0)
+    layer = sLSTMLayer(sLSTMLayerConfig(embedding_dim=1024, num_heads=2, conv1d_kernel_size=4, backend="hip",
+                                        recurrent_weight_init="standard")).to(DEV, torch.bfloat16).eval()
+    xs = [torch.randn(4, 1, 1024, device=DEV, dtype=torch.bfloat16) for _ in range(4)]
+    dec = GraphedLayerDecoder(layer, 4)
+    want = [dec.step(x).clone() for x in xs]
+    dec.reset()
+    with torch.no_grad():
+        for B in (6, 7):
+            layer.step(torch.randn(B, 1, 1024, device=DEV, dtype=torch.bfloat16), slstm_state=torch.zeros(4, B, 1024, device=DEV))
+        layer.slstm_cell._recurrent_kernel_.mul_(1.0)
+        layer.step(xs[0], slstm_state=torch.zeros(4, 4, 1024, device=DEV))
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    for x, w in zip(xs, want):
+        assert torch.equal(dec.step(x), w)
+
+
 @pytest.mark.parametrize("module,method,where", [
     (module, method, where) for module, method in (("slstm_cell", "forward"), ("slstm_cell", "step"), ("dropout", "forward"))
     for where in ("instance", "class", "compiled") if (method, where) != ("step", "compiled")])

@@ -26,6 +26,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
 
+#include <algorithm>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -103,7 +104,8 @@ inline bool versioned(const at::Tensor &t) { return !t.is_inference(); }
 
 bool capturing(const at::Device &d) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing((hipStream_t)stream_of(d), &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+  const hipStream_t stream = (hipStream_t)stream_of(d);  // (the null stream cannot be captured)
+  return stream && (hipStreamIsCapturing(stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone);
 }
 
 // ---- abort words: pinned host words that a sequence kernel writes when one of its bounded waits ran out.  Pages of
@@ -176,6 +178,7 @@ struct CellPath {
   int64_t NH = 0, dh = 0;
   // decode: the plan (functional.StepPlan) whose argument block is used, and what it was made for
   PyObject *plan = nullptr;
+  std::vector<PyObject *> recorded_plans;  // plans that a recorded graph reads, for as long as the cell lives
   xs_slstm_args *step_args = nullptr;
   int64_t step_B = 0;
   at::ScalarType step_dtype = at::kFloat;
@@ -199,6 +202,7 @@ struct CellPath {
   ~CellPath() {
     Py_XDECREF(parameters);
     Py_XDECREF(plan);
+    for (PyObject *o : recorded_plans) Py_DECREF(o);
   }
 
   bool records(const at::Tensor &x, const at::Tensor *state, const at::Tensor &r, const at::Tensor &b) const {
@@ -321,6 +325,10 @@ struct Step {
       : c(cell), plan(cell.plan), a(*cell.step_args), B(cell.step_B), H(cell.NH * cell.dh), device(cell.device), dtype(cell.step_dtype),
         last_state(cell.last_state), last_h(cell.last_h), last_state_version(cell.last_state_version), last_h_version(cell.last_h_version) {
     Py_INCREF(plan.o);
+    if (capturing(device) && std::find(c.recorded_plans.begin(), c.recorded_plans.end(), plan.o) == c.recorded_plans.end()) {
+      c.recorded_plans.push_back(plan.o);  // (steps of another batch size or of changed parameters replace the plan, replays read on)
+      Py_INCREF(plan.o);
+    }
   }
   // wx: contiguous [B,1,4H]; everything else as step_fits has found it
   void run(const at::Tensor &wx, const at::Tensor &s0, const StepBuffers &s, const Shape4 *h_shape) {
@@ -750,6 +758,7 @@ int cell_traverse(PyObject *self, visitproc visit, void *arg) {
   if (c) {
     Py_VISIT(c->parameters);
     Py_VISIT(c->plan);
+    for (PyObject *o : c->recorded_plans) Py_VISIT(o);
   }
   return 0;
 }
@@ -759,6 +768,9 @@ int cell_clear(PyObject *self) {
     c->step_args = nullptr;  // (the plan's)
     Py_CLEAR(c->parameters);
     Py_CLEAR(c->plan);
+    std::vector<PyObject *> recorded;
+    recorded.swap(c->recorded_plans);
+    for (PyObject *o : recorded) Py_DECREF(o);
   }
   return 0;
 }
