@@ -133,6 +133,35 @@ def test_plan_of_a_graph_outlives_other_batch_sizes():
         assert torch.equal(dec.step(x), w)
 
 
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_first_step_of_a_cell_under_capture(dtype, masked):
+    """A decode step whose first call is recorded (nothing of it has run when it returns), then eager steps in front of any
+    replay, other parameters, replays."""
+    print("case first step under capture", dtype, masked, flush=True)
+    x = torch.randn(3, 1, 8 * 256, device=DEV, dtype=dtype)
+    state = torch.rand(4, 3, 512, device=DEV) + 0.5
+    mask = torch.tensor([[True], [False], [False]], device=DEV) if masked else None
+    cells = [_cell(2, 256) for _ in range(2)]
+    for cell in cells:
+        cell.keep_state_fp32 = True
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.no_grad():
+        want = cells[1].step(x, state, mask)  # (loads the kernels: a cell of its own)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            out = cells[0].step(x, state, mask)
+        got = cells[0].step(x, state, mask)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        for _ in range(3):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(out, want))
+            out[0].zero_()
+            got = cells[0].step(x, state, mask)
+            assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 @pytest.mark.parametrize("module,method,where", [
     (module, method, where) for module, method in (("slstm_cell", "forward"), ("slstm_cell", "step"), ("dropout", "forward"))
     for where in ("instance", "class", "compiled") if (method, where) != ("step", "compiled")])

@@ -234,6 +234,7 @@ class _Runtime:
         self.status_ring = None
         self.last_workspace = None  # of the latest call, or `native` where that call was the native path's
         self.r_bf16 = None
+        self.recorded = []  # bf16 copies of R that recorded graphs read
         self.step_plan = None
         self.native = None  # the cell's native host path (_lib.host().CellPath), which also remembers the last fast step
 
@@ -412,13 +413,18 @@ class sLSTMCell_hip(nn.Module):
 
     # ------------------------------------------------------------------ forward
     def _bf16_recurrent_kernel(self) -> torch.Tensor:
-        """bf16 copy of R for decoding, refreshed when the parameter changes."""
+        """bf16 copy of R for decoding, refreshed when the parameter changes.  Under capture: a copy at hand is kept for the
+        graph that reads it, a new one is made within the graph and not kept here (nothing has run yet)."""
         p = self._recurrent_kernel_
-        key = (p.data_ptr(), p._version, p.device)
+        key = (p.data_ptr(), 0 if p.is_inference() else p._version, p.device)
         cache = self._rt.r_bf16
+        capturing = p.is_cuda and torch.cuda.is_current_stream_capturing()
         if cache is None or cache[0] != key:
             cache = (key, p.detach().to(torch.bfloat16).contiguous())
-            self._rt.r_bf16 = cache
+            if not capturing:
+                self._rt.r_bf16 = cache
+        elif capturing and not any(t is cache[1] for t in self._rt.recorded):
+            self._rt.recorded.append(cache[1])
         return cache[1]
 
     # ------------------------------------------------------------------ status of calls in flight
@@ -618,6 +624,8 @@ class sLSTMCell_hip(nn.Module):
         self._check_input(input)
         B = input.shape[0]
         self._check_state(B, state)
+        if torch.cuda.is_current_stream_capturing():
+            return None  # (a plan made here would be filled by replays only, in memory of the graph's)
         if not self._plan_step(B, input.dtype, input.device):
             raise ValueError("the step's tensors do not fit the cell's parameters (device)")
         if h_out is not None and (h_out.dtype != input.dtype or h_out.numel() != B * self.config.hidden_size
@@ -635,7 +643,8 @@ class sLSTMCell_hip(nn.Module):
         return fast
 
     def _plan_step(self, B: int, dtype: torch.dtype, device) -> bool:
-        """Makes the plan of decode steps of ``B`` rows from the current parameters and hands it to the native path."""
+        """Makes the plan of decode steps of ``B`` rows from the current parameters and hands it to the native path.  False
+        where the parameters live elsewhere."""
         r, b = self._recurrent_kernel_, self._bias_
         if r.device != device or b.device != device:
             return False
