@@ -108,6 +108,43 @@ def test_modules_put_in_the_place_of_a_layers_are_called():
         assert torch.equal(layer(x), plain) and layer.slstm_cell.calls == 1
 
 
+def test_graphs_of_a_cell_have_workspaces_of_their_own():
+    """Two graphs recorded on one stream, replayed on two streams at a time, beside eager calls on the stream of the capture."""
+    print("case workspaces of graphs", flush=True)
+    cell = _cell(2, 256, torch.bfloat16)
+    xs = [torch.randn(3, 40, 8 * 256, device=DEV, dtype=torch.bfloat16) for _ in range(3)]
+    side, streams = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(2)]
+    with torch.no_grad():
+        want = [_cell(2, 256, torch.bfloat16)(x) for x in xs]
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            cell(xs[2])
+        used = {cell._native().last_workspace().data_ptr()}
+        torch.cuda.synchronize()
+        graphs, outs, held = [], [], []
+        for x in xs[:2]:
+            graphs.append(torch.cuda.CUDAGraph())
+            with torch.cuda.graph(graphs[-1], stream=side):
+                outs.append(cell(x))
+            held.append(cell._native().last_workspace())
+            used.add(held[-1].data_ptr())
+        assert len(used) == 3
+        del held
+        for _ in range(10):
+            torch.cuda.synchronize()
+            for g, s in zip(graphs, streams):
+                with torch.cuda.stream(s):
+                    g.replay()
+            with torch.cuda.stream(side):
+                got = cell(xs[2])
+            torch.cuda.synchronize()
+            for a, b in zip([*outs, got], want):
+                assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+            for o in outs:
+                o[0].zero_()
+    cell.check_status()
+
+
 def test_plan_of_a_graph_outlives_other_batch_sizes():
     """A decoder's graphs, then eager steps of another batch size and of changed parameters on the same layer, with every block
     that is free given back to the driver: replays still read the R and the bias that they were recorded with."""

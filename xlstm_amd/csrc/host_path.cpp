@@ -187,10 +187,10 @@ struct CellPath {
   uint32_t r_version = 0, b_version = 0;
   at::Tensor last_state, last_h;   // what the last step handed out (float32 state kept), and their versions
   uint32_t last_state_version = 0, last_h_version = 0;
-  // sequences: a workspace per (device, stream)
-  struct Workspace { int device; void *stream; at::Tensor t; bool captured = false; };
+  // sequences: a workspace per (device, stream); a call under capture has one of its own, which is the graph's (graphs that
+  // were recorded on one stream may be replayed on several, beside eager calls on that stream)
+  struct Workspace { int device; void *stream; at::Tensor t; };
   std::vector<Workspace> workspaces;
-  std::vector<at::Tensor> captured;  // workspaces that a recorded graph writes and that a larger one has replaced
   at::Tensor last_workspace;
   AbortWord abort_word;
   std::shared_ptr<CallsInFlight> calls = std::make_shared<CallsInFlight>();
@@ -218,28 +218,25 @@ struct CellPath {
       return nullptr;
     };
     Workspace *w = find();
-    if (!w || (size_t)w->t.numel() < need) {
+    const bool in_graph = capturing(d);
+    if (in_graph || !w || (size_t)w->t.numel() < need) {
       at::Tensor fresh;
       {
         WithoutGil no_gil;
         fresh = at::empty({(int64_t)need}, at::TensorOptions().dtype(at::kByte).device(d));
       }
+      if (in_graph) return fresh;
       w = find();
       if (!w) {
         // (a program that makes a new stream per call would otherwise collect workspaces without end; a stream's
-        // allocations are handed on in stream order by the caching allocator, so dropping the oldest is safe - unless
-        // it was used under capture: replays of the graph write it for as long as the graph lives)
-        if (workspaces.size() >= 16)
-          for (auto it = workspaces.begin(); it != workspaces.end(); ++it)
-            if (!it->captured) { workspaces.erase(it); break; }
+        // allocations are handed on in stream order by the caching allocator, so dropping the oldest is safe)
+        if (workspaces.size() >= 16) workspaces.erase(workspaces.begin());
         workspaces.push_back(Workspace{(int)d.index(), stream, fresh});
         w = &workspaces.back();
       } else if ((size_t)w->t.numel() < need) {
-        if (w->captured) captured.push_back(w->t);
         w->t = fresh;
       }
     }
-    w->captured |= capturing(d);
     return w->t;
   }
 
