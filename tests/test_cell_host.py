@@ -215,7 +215,7 @@ def cell_calls(x, state=None, mask=None, **kw):
     for grad in (False, True):
         with torch.set_grad_enabled(grad):
             assert native.forward(x, state, mask, cell.config, False) is None
-            assert native.train(x, state, mask, cell.config, False) is None
+            assert native.train(x, state, mask, cell.config, False, 1 << 40) is None
             assert native.step(x, state, mask, None, None, None, cell.config, False) is None
 
 try:  # (an error of the library's own throws: the counter counts)

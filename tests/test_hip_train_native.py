@@ -153,3 +153,49 @@ def test_coefficients_beyond_what_is_kept(monkeypatch, dtype, dh):
         # (row tiles of other heights sum in another order, and bfloat16 deltas round once: 2^-8)
         tol = 2e-2 if dtype == torch.bfloat16 else 1e-4
         torch.testing.assert_close(a, b, rtol=tol, atol=tol)
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("dtype,dh", [(torch.float32, 64), (torch.bfloat16, 128), (torch.bfloat16, 256)])
+def test_a_stack_keeps_what_a_device_may_hold(monkeypatch, native, dtype, dh):
+    """Four layers one behind the other and room for the coefficients of two: the others are made again by their backward
+    calls, the gradients are the same, and everything is given back - behind the backward, and where none is run."""
+    from xlstm_amd import _lib
+    from xlstm_amd import cell as cell_module
+    from xlstm_amd.cell import sLSTMCell, sLSTMCellConfig
+
+    print("case stack", native, dtype, dh, flush=True)
+    if not native:
+        monkeypatch.setattr(cell_module.sLSTMCell_hip, "_trains_natively", lambda self, input: False)
+    host, F, H, B, T = _lib.host(), cell_module.F_hip, 2 * dh, 4, 400 if dh == 256 else 8
+    torch.manual_seed(dh)
+    cells = [sLSTMCell(sLSTMCellConfig(hidden_size=H, num_heads=2, backend="hip", recurrent_weight_init="standard",
+                                       output_shape="BSH")).to(DEV) for _ in range(4)]
+    x0 = torch.randn(B, T, 4 * H, device=DEV, dtype=dtype)
+    leaves = [p for cell in cells for p in cell.parameters()]
+
+    def run():
+        x, held = x0, []
+        for cell in cells:
+            out, _ = cell(x)
+            x = x0 + out.repeat(1, 1, 4)
+            held.append(host.kept(0))
+        return x, held
+
+    assert host.kept(0) == 0
+    x, held = run()
+    each = held[0]
+    assert 0 < each <= 36 * B * T * H and held == [each, 2 * each, 3 * each, 4 * each]
+    want = torch.autograd.grad(x.float().square().mean(), leaves)
+    assert host.kept(0) == 0  # (the graph's outputs are still there, what it saved is not)
+    monkeypatch.setattr(F, "KEPT_COEFFICIENT_BYTES_PER_DEVICE", 2 * each + each // 2)
+    x, held = run()
+    assert held == [each, 2 * each, 2 * each, 2 * each]
+    got = torch.autograd.grad(x.float().square().mean(), leaves, retain_graph=True)
+    assert host.kept(0) == (2 * each if dh != 256 else 0)  # (a graph that is kept keeps them, but for the row tiles of 4 rows)
+    del x
+    assert host.kept(0) == 0
+    for a, b in zip(want, got):
+        # (other row tiles sum in another order; bfloat16 deltas round once, 2^-8, and so do the gradients between layers)
+        tol = (1e-4 if dtype == torch.float32 else 3e-2) * float(a.abs().max())
+        torch.testing.assert_close(a, b, rtol=0, atol=tol)

@@ -259,8 +259,9 @@ class sLSTMCell_hip(nn.Module):
     config_class = sLSTMCellConfig
 
     #: Training: let the forward call leave the backward pass its coefficients (36 bytes per step and element, held
-    #: until the backward has run) up to ``functional.KEPT_COEFFICIENT_BYTES`` instead of having the backward pass run the
-    #: forward once more for them (beyond: bfloat16 at head dim 256 where the row tiles of 4 rows fit the device).  The
+    #: until the backward has run) up to ``functional.KEPT_COEFFICIENT_BYTES`` (bfloat16 at head dim 256 in row tiles of 4
+    #: rows: also beyond) and, with all others that wait on the device, ``functional.KEPT_COEFFICIENT_BYTES_PER_DEVICE``, instead
+    #: of having the backward pass run the forward once more for them.  The
     #: reference's native forward always keeps its states and gate values when it trains (slstm.cc:79-108); set this to
     #: False to keep nothing (the memory then goes to the backward call alone).  The gradients are the same either way.
     keep_backward_coefficients: bool = True
@@ -525,9 +526,9 @@ class sLSTMCell_hip(nn.Module):
         coef = h = s = None
         if wants_grad and self.keep_backward_coefficients and x.is_cuda and not step:
             if self.head_dim == 256:  # (bfloat16: row tiles of 4 rows x 64 units in the backward, where they fit)
-                coef = F_hip.backward_coefficients_buffer(x, self.config.num_heads)
+                coef = F_hip.backward_coefficients_buffer(x, self.config.num_heads, kept=True)
             if coef is None and 9 * x.numel() <= F_hip.KEPT_COEFFICIENT_BYTES:
-                coef = F_hip.training_coefficients(x, self.config.num_heads)
+                coef = F_hip.training_coefficients(x, self.config.num_heads, kept=True)
                 if coef is not None:
                     h, s = F_hip.slstm_forward(*args, s_out=state_out, workspace=ws, train_coef=coef)
         if coef is not None and h is None:
@@ -564,7 +565,8 @@ class sLSTMCell_hip(nn.Module):
                 native = self._native()
             fast = native.forward(input, state, reset_mask, self.config, self.keep_state_fp32) if native is not None else None
             if fast is None and native is not None and torch.is_grad_enabled() and self._trains_natively(input):
-                fast = native.train(input, state, reset_mask, self.config, self.keep_state_fp32)
+                fast = native.train(input, state, reset_mask, self.config, self.keep_state_fp32,
+                                    F_hip.KEPT_COEFFICIENT_BYTES_PER_DEVICE)
             if fast is not None:
                 self._rt.last_workspace = native
         if fast is not None:

@@ -27,6 +27,7 @@
 #include <torch/csrc/autograd/saved_variable.h>
 
 #include <algorithm>
+#include <atomic>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -140,6 +141,26 @@ AbortWord take_word() {
   uint32_t *w = g_words.take();
   return w ? AbortWord(w, [](uint32_t *p) { g_words.give_back(p); }) : nullptr;
 }
+
+// ---- the bytes that training forwards have left, per device, for backward calls that are still to come: a share of what a
+// device may hold is taken with the coefficients and goes with them
+std::atomic<int64_t> g_kept_bytes[64];
+class Share {
+ public:
+  static std::shared_ptr<Share> take(int device, int64_t bytes, int64_t limit) {  // null: that would be more than `limit`
+    if (device < 0 || device >= 64) return nullptr;
+    int64_t held = g_kept_bytes[device].load();
+    do {
+      if (bytes > limit - held) return nullptr;
+    } while (!g_kept_bytes[device].compare_exchange_weak(held, held + bytes));
+    return std::shared_ptr<Share>(new Share(device, bytes));
+  }
+  ~Share() { g_kept_bytes[device_] -= bytes_; }
+ private:
+  Share(int device, int64_t bytes) : device_(device), bytes_(bytes) {}
+  const int device_;
+  const int64_t bytes_;
+};
 
 // ---- where calls of a cell may still be running: the streams they went to.  Shared with the backward calls that are still to
 // come; used without the GIL.  (An event behind every call would say it to the call, and costs 5 us on the device each:
@@ -577,6 +598,7 @@ struct CellBackward : public torch::autograd::Node {
   // coefficients are saved like a tensor of the caller's, so that checkpointing and offloading hooks see them)
   SavedVariable x, r, b, h, state, coef;
   bool has_state = false, transposed_input = false;
+  std::shared_ptr<Share> share;  // the coefficients'
   ReverseInputs in;  // (its saved tensors are filled in when the backward runs)
   OutShape shape = OutShape::BNSH;
   at::ScalarType r_dtype = at::kFloat, b_dtype = at::kFloat, s_dtype = at::kFloat;
@@ -586,6 +608,7 @@ struct CellBackward : public torch::autograd::Node {
     std::lock_guard<std::mutex> lock(mutex_);
     for (SavedVariable *v : {&x, &r, &b, &h, &state, &coef}) v->reset_data();
     in.mask.reset();
+    share.reset();
   }
   variable_list apply(variable_list &&grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
@@ -627,7 +650,8 @@ struct CellBackward : public torch::autograd::Node {
   }
 };
 
-// train(input, state, reset_mask, config, keep_state_fp32) -> (output, state) with their place in the graph, or None
+// train(input, state, reset_mask, config, keep_state_fp32, bytes of coefficients that a device may hold) -> (output, state) with
+// their place in the graph, or None
 PyObject *cell_train_(CellPath &c, PyObject *const *args) {
   const at::Tensor *xp = tensor_of(args[0]), *state, *mask, *rp, *bp;
   if (!xp || xp->dim() != 3 || !xp->is_cuda() || !optional_tensor(args[1], state) || !optional_tensor(args[2], mask) ||
@@ -649,6 +673,11 @@ PyObject *cell_train_(CellPath &c, PyObject *const *args) {
   c10::OptionalDeviceGuard guard(x.device());
   if (!have_word(c, x.device())) Py_RETURN_NONE;
   const bool keep = args[4] == Py_True || x.scalar_type() == at::kFloat;
+  const int64_t limit = PyLong_AsLongLong(args[5]);
+  if (PyErr_Occurred()) throw PythonError{};
+  std::shared_ptr<Share> share = Share::take(x.device().index(), 4 * (int64_t)g_engine.coef_floats((int32_t)x.size(bsgnh ? 0 : 1), (int32_t)x.size(bsgnh ? 1 : 0),
+                                             (int32_t)c.NH, (int32_t)c.dh, dtype_code(x.scalar_type())), limit);
+  if (!share) Py_RETURN_NONE;  // (the backward call of the general path makes them again)
   Sequence s(c, x.device(), x.size(bsgnh ? 0 : 1));
   const at::Tensor r = s.r, b = s.b;
   at::Tensor state_out;
@@ -664,6 +693,7 @@ PyObject *cell_train_(CellPath &c, PyObject *const *args) {
     node->r = SavedVariable(r, false);
     node->b = SavedVariable(b, false);
     node->coef = SavedVariable(s.coef, false);
+    node->share = std::move(share);
     node->has_state = state != nullptr;
     if (state) { node->state = SavedVariable(*state, false); node->s_dtype = state->scalar_type(); }
     node->transposed_input = !bsgnh;
@@ -782,7 +812,7 @@ void cell_dealloc(PyObject *self) {
 PyMethodDef cell_methods[] = {
     {"step", (PyCFunction)(void *)cell_call<cell_step_, 8>, METH_FASTCALL, nullptr},
     {"forward", (PyCFunction)(void *)cell_call<cell_forward_, 5>, METH_FASTCALL, nullptr},
-    {"train", (PyCFunction)(void *)cell_call<cell_train_, 5>, METH_FASTCALL, nullptr},
+    {"train", (PyCFunction)(void *)cell_call<cell_train_, 6>, METH_FASTCALL, nullptr},
     {"set_plan", (PyCFunction)(void *)cell_call<cell_set_plan_, 5>, METH_FASTCALL, nullptr},
     {"workspace", (PyCFunction)(void *)cell_call<cell_workspace_, 2>, METH_FASTCALL, nullptr},
     {"last_workspace", (PyCFunction)(void *)cell_call<cell_last_workspace_, 0>, METH_FASTCALL, nullptr},
@@ -1047,6 +1077,24 @@ PyObject *layer_call(PyObject *, PyObject *const *args, Py_ssize_t n) {
   }
 }
 
+// keep(device, bytes, limit) -> a share of what the device may hold, given back when the object goes, or None beyond the limit
+void share_gone(PyObject *capsule) { delete (std::shared_ptr<Share> *)PyCapsule_GetPointer(capsule, "share"); }
+PyObject *keep(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  if (n != 3) { PyErr_SetString(PyExc_TypeError, "keep(device, bytes, limit)"); return nullptr; }
+  const long long device = PyLong_AsLongLong(args[0]), bytes = PyLong_AsLongLong(args[1]), limit = PyLong_AsLongLong(args[2]);
+  if (PyErr_Occurred()) return nullptr;
+  std::shared_ptr<Share> share = Share::take((int)device, bytes, limit);
+  if (!share) Py_RETURN_NONE;
+  return PyCapsule_New(new std::shared_ptr<Share>(std::move(share)), "share", share_gone);
+}
+// kept(device) -> the bytes that are held now
+PyObject *kept(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  const long long device = n == 1 ? PyLong_AsLongLong(args[0]) : -1;
+  if (PyErr_Occurred()) return nullptr;
+  if (device < 0 || device >= 64) { PyErr_SetString(PyExc_ValueError, "kept(device)"); return nullptr; }
+  return PyLong_FromLongLong(g_kept_bytes[device].load());
+}
+
 // bind(addresses: dict name -> int, EngineError, the two dicts of global module hooks)
 PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (n != 4 || !PyDict_Check(args[0])) { PyErr_SetString(PyExc_TypeError, "bind(addresses, error, hooks, pre_hooks)"); return nullptr; }
@@ -1072,6 +1120,8 @@ PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
 
 PyMethodDef module_methods[] = {
     {"bind", (PyCFunction)(void *)bind, METH_FASTCALL, nullptr},
+    {"keep", (PyCFunction)(void *)keep, METH_FASTCALL, nullptr},
+    {"kept", (PyCFunction)(void *)kept, METH_FASTCALL, nullptr},
     {"layer_step", (PyCFunction)(void *)layer_call<layer_step_, 10>, METH_FASTCALL, nullptr},
     {"layer_forward", (PyCFunction)(void *)layer_call<layer_forward_, 7>, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};

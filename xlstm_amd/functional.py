@@ -12,6 +12,7 @@ Layouts are the external ones of the reference cell:
 from __future__ import annotations
 
 import ctypes
+import math
 from typing import Optional, Tuple
 
 import torch
@@ -82,18 +83,19 @@ class CoefficientsUnsupported(EngineError):
     """A forward call was asked to leave the backward pass its coefficients and is not one of those that can."""
 
 
-def backward_coefficients_buffer(wx: torch.Tensor, num_heads: int) -> Optional[torch.Tensor]:
+def backward_coefficients_buffer(wx: torch.Tensor, num_heads: int, kept: bool = False) -> Optional[torch.Tensor]:
     """The tensor a training forward (``slstm_forward(..., coef_out=)``) leaves the backward pass's coefficients in, or
     ``None`` where the forward cannot: it takes bfloat16 inputs, a head dim of 128 or 256 and a batch whose row tiles of
     4 rows fit the device in the forward (``ceil(B/4) * NH * dh/16`` workgroups) and, with their prefetching workgroups,
     in the backward.  36 bytes per step and element, held from the forward to the backward (the reference keeps the
-    states and gate values of every step instead, ``slstm.cc:79-108``); without it the backward pass recomputes them."""
+    states and gate values of every step instead, ``slstm.cc:79-108``); without it the backward pass recomputes them.
+    ``kept``: for a backward call to come, within ``KEPT_COEFFICIENT_BYTES_PER_DEVICE`` (``None`` beyond)."""
     B, T = int(wx.shape[0]), int(wx.shape[1])
     H = int(wx.shape[2]) // 4
     dh = H // num_heads
     if wx.dtype != torch.bfloat16 or dh not in (128, 256) or B < 1 or T < 2 or not _quad_fits(B, T, num_heads, dh, wx.device):
         return None
-    return torch.empty((T, (B + 3) // 4 * 4, 9, H), dtype=torch.float32, device=wx.device)
+    return _coefficients((T, (B + 3) // 4 * 4, 9, H), wx.device, kept)
 
 
 def _quad_fits(B: int, T: int, NH: int, dh: int, device) -> bool:
@@ -104,18 +106,34 @@ def _quad_fits(B: int, T: int, NH: int, dh: int, device) -> bool:
 
 
 #: A training forward leaves the backward pass its coefficients up to this size (of 36 bytes per step and element: 16 rows x
-#: 2048 steps x 1024 units take 1.2 GB), so that a stack of layers that fits without them still fits.  Beyond, the backward
-#: call runs the forward once more, in slices of rows whose coefficients take up to the second size.
+#: 2048 steps x 1024 units take 1.2 GB), and as long as all that wait for their backward call on a device, of every layer of a
+#: stack and of every cell, stay within the second (a sixteenth of 288 GB: so that a stack that fits without them still fits).
+#: Beyond either, the backward call runs the forward once more, in slices of rows whose coefficients take up to the third.
 KEPT_COEFFICIENT_BYTES = 4 << 30
+KEPT_COEFFICIENT_BYTES_PER_DEVICE = 16 << 30
 RECOMPUTED_COEFFICIENT_BYTES = 24 << 30
 
 
-def training_coefficients(wx: torch.Tensor, num_heads: int) -> Optional[torch.Tensor]:
+def _coefficients(shape, device, kept: bool) -> Optional[torch.Tensor]:
+    share = None
+    if kept:
+        bytes_ = 4 * math.prod(shape)
+        share = _lib.host().keep(device.index, bytes_, KEPT_COEFFICIENT_BYTES_PER_DEVICE)
+        if share is None:
+            return None
+    coef = torch.empty(shape, dtype=torch.float32, device=device)
+    if kept:
+        coef.share = share  # (goes with the tensor: when the graph that holds it is done, or a hook has packed it elsewhere)
+    return coef
+
+
+def training_coefficients(wx: torch.Tensor, num_heads: int, kept: bool = False) -> Optional[torch.Tensor]:
     """The tensor a training forward (``slstm_forward(..., train_coef=)``) leaves the backward pass's coefficients in, 36
-    bytes per step and element, or ``None`` for calls without a forward kernel (``xs_slstm_train_forward``)."""
+    bytes per step and element, or ``None`` for calls without a forward kernel (``xs_slstm_train_forward``).  ``kept``: as in
+    ``backward_coefficients_buffer``."""
     B, T = int(wx.shape[0]), int(wx.shape[1])
     n = _lib.load().xs_slstm_train_coef_floats(B, T, num_heads, int(wx.shape[2]) // 4 // num_heads, _DTYPE_CODE.get(wx.dtype, -1))
-    return torch.empty(n, dtype=torch.float32, device=wx.device) if n else None
+    return _coefficients((n,), wx.device, kept) if n else None
 
 
 def _train_backward(lib, wx, r, bias, s0, reset_mask, h_out, d_h, d_s_final, coef, timings, recurrent_cut, recurrent_clipval,
