@@ -157,6 +157,22 @@ def test_cell_can_be_copied_and_pickled():
         assert not torch.equal(other.bias[:], c.bias[:])
 
 
+def test_the_choice_of_the_training_path_is_by_the_call_alone(monkeypatch):
+    """Sizes, types and the cell's own setting; not what has become of a function of the package."""
+    from xlstm_amd import cell as cell_module
+
+    cell = _cell(hidden_size=512, num_heads=2)
+    short, long = torch.zeros(1, 8, 2048), torch.zeros(1, 400, 2048)
+    for watch in (False, True):
+        if watch:
+            plain = cell_module.F_hip.slstm_backward
+            monkeypatch.setattr(cell_module.F_hip, "slstm_backward", lambda *a, **kw: plain(*a, **kw))
+        assert cell._trains_natively(short) and cell._trains_natively(long) and cell._trains_natively(short.bfloat16())
+        assert not cell._trains_natively(long.bfloat16())  # (row tiles of 4 rows x 64 units, forward and backward)
+    cell.keep_backward_coefficients = False
+    assert not cell._trains_natively(short)
+
+
 def test_a_cell_in_a_cycle_is_collected():
     """A hook on a parameter whose closure refers to the module: a cycle through the native host path's reference to the
     cell's parameters, which the collector has to see."""

@@ -1,5 +1,5 @@
-"""Training calls of a cell through the native host path against the Python one (which a replaced
-``functional.slstm_backward`` takes): every layout of input and output, states, masks, options, gradients of any strides."""
+"""Training calls of a cell through the native host path against the Python one (the tests replace the cell's choice
+between them): every layout of input and output, states, masks, options, gradients of any strides."""
 import pytest
 import torch
 
@@ -37,8 +37,7 @@ def test_native_training_call_equals_the_python_path(monkeypatch, dtype, in_shap
         results = []
         for native in (True, False):
             if not native:
-                plain = cell_module.F_hip.slstm_backward
-                monkeypatch.setattr(cell_module.F_hip, "slstm_backward", lambda *a, **kw: plain(*a, **kw))
+                monkeypatch.setattr(cell_module.sLSTMCell_hip, "_trains_natively", lambda self, input: False)
             x = x0.clone().requires_grad_(True)
             st = s0.to(dtype).requires_grad_(True) if extra.get("state") else None
             out, state = cell(x, st, reset_mask=mask)
@@ -97,8 +96,7 @@ def test_checkpointing_and_hooks_see_what_is_saved(monkeypatch, native, dh):
 
     print("case saved tensors", native, dh, flush=True)
     if not native:
-        plain = cell_module.F_hip.slstm_backward
-        monkeypatch.setattr(cell_module.F_hip, "slstm_backward", lambda *a, **kw: plain(*a, **kw))
+        monkeypatch.setattr(cell_module.sLSTMCell_hip, "_trains_natively", lambda self, input: False)
     cell, x = _small_cell(dh=dh)
     leaves = [x, *cell.parameters()]
     out, _ = cell(x)

@@ -38,8 +38,6 @@ from torch import nn
 
 from . import functional as F_hip
 
-_ENGINE_BACKWARD = F_hip.slstm_backward
-
 DTYPE_DICT = {
     "bfloat16": torch.bfloat16,
     "float16": torch.float16,
@@ -574,12 +572,10 @@ class sLSTMCell_hip(nn.Module):
         return self._run(input, state, reset_mask, step=False)
 
     def _trains_natively(self, input: torch.Tensor) -> bool:
-        """Whether a training call takes the native host path.  Not where the coefficients are not to be kept, where
-        ``functional.slstm_backward`` has been replaced (whoever did so sees every backward call), and for long bfloat16
-        sequences at head dim 256: forward and backward in row tiles of 4 rows x 64 units save 0.07 us a step there
+        """Whether a training call takes the native host path.  Not where the coefficients are not to be kept, and for long
+        bfloat16 sequences at head dim 256: forward and backward in row tiles of 4 rows x 64 units save 0.07 us a step there
         and take three more launches."""
-        return (self.keep_backward_coefficients and F_hip.slstm_backward is _ENGINE_BACKWARD
-                and 9 * input.numel() <= F_hip.KEPT_COEFFICIENT_BYTES
+        return (self.keep_backward_coefficients and 9 * input.numel() <= F_hip.KEPT_COEFFICIENT_BYTES
                 and not (self.head_dim == 256 and input.dtype == torch.bfloat16
                          and input.shape[1 if self.config.input_shape == "BSGNH" else 0] >= 384))
 
