@@ -37,7 +37,7 @@ def test_step_of_a_small_batch(bf16, B, NH, dh):
 def _run(F, so, x, wx, r_t, r, b_t, b, mask, m, T, bf16):
     h_seq, s_seq = F.slstm_forward(x, r_t, b_t, None, m)
     h_ref, s_ref = so.slstm_forward(wx, r, b, None, mask)
-    tol = 2e-2 if bf16 else 1e-4  # (the bars of the cell's parity tests)
+    tol = 2e-2 if bf16 else 1e-5  # (the bars of the cell's parity tests; float32: K products of order 1 / sqrt(K) and three steps of gating, a few 2^-24 each)
     state, h_prev = None, None
     for t in range(T):
         mt = None if m is None else m[:, t:t + 1]
