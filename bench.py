@@ -325,10 +325,10 @@ def bench_backward(device, iters=3):
 
 
 def bench_backward_large(device, T=4096, iters=2):
-    """The backward pass at BASELINE config 5's shape (B=64, 4 heads of 1024, bf16): the kernels of one launch per step
-    (``split == 3`` of the C ABI), the whole call and its three parts by HIP events.  Per step the walk and the reverse
-    pass each read R once (32 MiB: it does not stay in any cache level below the Infinity Cache) and the operand rows
-    once per tile of 32 units; the roofline line prices those bytes of the reverse kernel against the HBM peak."""
+    """The backward pass at BASELINE config 5's shape (B=64, 4 heads of 1024, bf16) without coefficients from the forward:
+    the forward runs once more and leaves them, the reverse kernel (32 units per workgroup, R in registers, one launch per
+    slice of rows) and the gradients of R and the bias follow; the whole call and its three parts by HIP events.  The
+    roofline line prices the bytes that the reverse pass cannot do without against the HBM peak."""
     import numpy as np
     import torch
 
@@ -363,17 +363,16 @@ def bench_backward_large(device, T=4096, iters=2):
         finite = bool(torch.isfinite(out[0][:, -1]).all() and torch.isfinite(out[3]).all())
         del out
     rev_ms = float(np.median(rev))
-    # a launch of the reverse kernel: R transposed once, nine coefficients in and four gate deltas out per element in
-    # float32, the deltas in bf16 out and (the step behind's) in, d_h in bf16, the gradients of c and n in and out
-    nbytes = NH * 4 * dh * dh * 2 + (9 * 4 + 4 * 4 + 2 + 2 + 2 + 4 * 4) * B * H
-    return {"workload": "backward pass at config 5's shape: B=64 T=%d D=4096 NH=4 bf16, one launch per step" % T,
-            "ms": float(np.median(total)), "forward_walk_ms": float(np.median(prep)), "reverse_ms": rev_ms,
+    # the reverse pass: R once, and per step and element nine coefficients in and four gate deltas out in float32, d_h in bf16
+    nbytes = NH * 4 * dh * dh * 4 + T * (9 * 4 + 4 * 4 + 2) * B * H
+    return {"workload": "backward pass at config 5's shape: B=64 T=%d D=4096 NH=4 bf16, the forward once more for the coefficients" % T,
+            "ms": float(np.median(total)), "forward_again_ms": float(np.median(prep)), "reverse_ms": rev_ms,
             "parameter_gradient_kernel_ms": float(np.median(par)),
-            "us_per_step": {"forward_walk": float(np.median(prep)) * 1e3 / T, "reverse": rev_ms * 1e3 / (T + 1)},
+            "us_per_step": {"forward_again": float(np.median(prep)) * 1e3 / T, "reverse": rev_ms * 1e3 / T},
             "finite": finite,
-            "roofline": {"bound": "hbm", "achieved": nbytes / (rev_ms / (T + 1) * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                         "frac": nbytes / (rev_ms / (T + 1) * 1e-3) / 1e9 / HBM_PEAK_GBS, "traffic": None,
-                         "kernel": "slstm_bwd_step_kernel<bf16>", "algorithmic_bytes_per_launch": nbytes}}
+            "roofline": {"bound": "hbm", "achieved": nbytes / (rev_ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                         "frac": nbytes / (rev_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "traffic": None,
+                         "kernel": "slstm_bwd_unit_kernel<bf16>, its launches together", "algorithmic_bytes": nbytes}}
 
 
 def bench_decode_other_head_dims(device, steps=300):

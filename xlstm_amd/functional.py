@@ -519,7 +519,7 @@ def slstm_forward(
     ``coef_out`` (a training forward; a float32 tensor from ``backward_coefficients_buffer``): the kernel also leaves
     the coefficients of the backward pass there, and ``slstm_backward(..., coef=coef_out)`` skips its own forward walk.
     Raises ``CoefficientsUnsupported`` (nothing has run) for calls that cannot: see ``backward_coefficients_buffer``.
-    ``train_coef`` (from ``training_coefficients``): the same for small head dims, whose kernels have a layout of their own.
+    ``train_coef`` (from ``training_coefficients``): the same for every head dim, in the layout of ``xs_slstm_train_backward``.
 
     ``reset_mask[B,S]`` (bool/uint8) marks document starts: the row's state is
     zeroed before that step.  ``step=True`` uses the decode entry point (S == 1).
