@@ -125,3 +125,32 @@ def test_threads_share_a_cell(streams):
         t.join()
     assert not failures, failures[:5]
     cell.check_status()
+
+
+@pytest.mark.parametrize("of_layer", [False, True])
+def test_a_plan_replaced_while_a_step_is_looked_at(of_layer):
+    """Python code that runs in the middle of a step (here an attribute of the cell's config that steps the cell with another
+    batch size, as another thread may at that point): the step takes the plan of its own batch size."""
+    print("case plan replaced", of_layer, flush=True)
+    layer = _layer()
+    cell = layer.slstm_cell
+    steps = {True: lambda x, s: layer.step(x, slstm_state=s), False: cell.step}[of_layer]
+    xs = [torch.randn(B, 1, 128 if of_layer else 512, device=DEV, dtype=torch.bfloat16) for B in (3, 7)]
+    states = [torch.rand(4, x.shape[0], 128, device=DEV) + 0.5 for x in xs]
+
+    class Config:
+        def __init__(self, config):
+            self.config, self.armed = config, False
+
+        def __getattr__(self, name):
+            if name == "output_shape" and self.armed:
+                self.armed = False
+                steps(xs[1], states[1])
+            return getattr(self.config, name)
+
+    with torch.no_grad():
+        want = steps(xs[0], states[0])[0]
+        cell.config = Config(cell.config)
+        assert torch.equal(steps(xs[0], states[0])[0], want)
+        cell.config.armed = True
+        assert torch.equal(steps(xs[0], states[0])[0], want) and not cell.config.armed

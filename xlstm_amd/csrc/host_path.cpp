@@ -309,7 +309,8 @@ struct StepBuffers { const at::Tensor *state_out = nullptr, *h_out = nullptr, *h
 bool step_buffers(PyObject *state_out, PyObject *h_out, PyObject *h_prev, StepBuffers &s) {
   return optional_tensor(state_out, s.state_out) && optional_tensor(h_out, s.h_out) && optional_tensor(h_prev, s.h_prev);
 }
-// whether the cell's plan covers a step of B rows of x (the cell's input, or what a layer makes it from)
+// whether the cell's plan covers a step of B rows of x (the cell's input, or what a layer makes it from).  Looked at right in front
+// of the Step: an attribute read in between may run Python code, and with it another thread that replaces the plan
 bool step_fits(const CellPath &c, const at::Tensor &x, const at::Tensor &state, const StepBuffers &s) {
   const at::Tensor *r, *b;
   if (!c.plan || !c.weights(r, b) || r->data_ptr() != c.r_ptr || b->data_ptr() != c.b_ptr || version_of(*r) != c.r_version ||
@@ -393,11 +394,10 @@ bool recording(const CellPath &c, const at::Tensor &x, const at::Tensor *state) 
 PyObject *cell_step_(CellPath &c, PyObject *const *args) {
   const at::Tensor *x = tensor_of(args[0]), *state = tensor_of(args[1]);
   StepBuffers s;
-  if (!absent(args[2]) || !x || !state || at::autocast::is_autocast_enabled(at::kCUDA) || !step_buffers(args[3], args[4], args[5], s) ||
-      !step_fits(c, *x, *state, s) || x->size(2) != 4 * c.NH * c.dh)
-    Py_RETURN_NONE;
   OutShape shape;
-  if (!input_is_bsgnh(args[6]) || !out_shape(args[6], shape)) Py_RETURN_NONE;
+  if (!absent(args[2]) || !x || !state || !c.plan || at::autocast::is_autocast_enabled(at::kCUDA) || !step_buffers(args[3], args[4], args[5], s) ||
+      !input_is_bsgnh(args[6]) || !out_shape(args[6], shape) || !step_fits(c, *x, *state, s) || x->size(2) != 4 * c.NH * c.dh)
+    Py_RETURN_NONE;
   const bool keep = args[7] == Py_True;
   c10::OptionalDeviceGuard guard(c.device);
   const Shape4 s4 = shape_of(shape, 1, c.step_B, c.NH, c.dh);
@@ -962,12 +962,12 @@ PyObject *layer_step_(PyObject *const *args) {
   const at::Tensor *xp = tensor_of(args[2]), *statep = tensor_of(args[4]), *ring_out, *out_given;
   CellPath &c = *((CellPathObject *)args[1])->c;
   StepBuffers buffers;
-  if (!xp || !statep || !step_buffers(args[5], args[7], args[8], buffers) || !optional_tensor(args[6], ring_out) || !optional_tensor(args[9], out_given) ||
-      !step_fits(c, *xp, *statep, buffers))
+  if (!xp || !statep || !c.plan || !step_buffers(args[5], args[7], args[8], buffers) || !optional_tensor(args[6], ring_out) ||
+      !optional_tensor(args[9], out_given))
     Py_RETURN_NONE;
   const at::Tensor &x = *xp, &state = *statep;
   LayerParts p;
-  if (!aligned(x.data_ptr(), 16) || !collect(args[0], args[1], x, p)) Py_RETURN_NONE;
+  if (!collect(args[0], args[1], x, p) || !step_fits(c, x, state, buffers) || !aligned(x.data_ptr(), 16)) Py_RETURN_NONE;
   const int64_t B = x.size(0);
   if (B < 1) Py_RETURN_NONE;
   const void *taps = nullptr;
