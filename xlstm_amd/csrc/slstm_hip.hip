@@ -366,11 +366,13 @@ int run_local(const xs_slstm_args *a, float *coef, int head0 = 0) {
   const long long grid = local_grid(a->B, a->NH - head0);
   if (grid > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many row tiles for one launch");
   LocalParams p;
-  p.wx = a->wx; p.wx_sb = a->wx_stride_b; p.wx_st = a->wx_stride_t;
-  p.r = a->r; p.r_bf16 = a->r_dtype == XS_BF16;
-  p.bias = a->bias; p.s0 = a->s0; p.reset = a->reset; p.reset_sb = a->reset_stride_b;
-  p.h_out = a->h_out; p.s_out = a->s_out; p.status = (xs_slstm_status *)a->workspace; p.coef = coef;
-  p.B = a->B; p.T = a->T; p.NH = a->NH; p.dh = a->dh; p.head0 = head0;
+  const size_t esz = bf16 ? 2 : 4, units = (size_t)head0 * a->dh;  // (an offset of the pointers: the kernel has no head of its own to add)
+  p.wx = (const char *)a->wx + units * esz; p.wx_sb = a->wx_stride_b; p.wx_st = a->wx_stride_t;
+  p.r_bf16 = a->r_dtype == XS_BF16;
+  p.r = (const char *)a->r + units * 4 * a->dh * (p.r_bf16 ? 2 : 4);
+  p.bias = a->bias + 4 * units; p.s0 = a->s0 ? a->s0 + units : nullptr; p.reset = a->reset; p.reset_sb = a->reset_stride_b;
+  p.h_out = (char *)a->h_out + units * esz; p.s_out = a->s_out + units; p.status = (xs_slstm_status *)a->workspace; p.coef = coef;
+  p.B = a->B; p.T = a->T; p.NH = a->NH; p.dh = a->dh; p.heads = a->NH - head0;
   void (*k)(LocalParams);
   if (coef) k = bf16 ? pick_local<true, true>(w) : pick_local<false, true>(w);
   else k = bf16 ? pick_local<true, false>(w) : pick_local<false, false>(w);

@@ -50,7 +50,7 @@ struct LocalParams {
   xs_slstm_status *status;   // or null
   float *coef;               // COEF: [T][ceil(B/4)][NH][waves][{64 lanes x 4}, {64 x 4}, {64 x 1}]: coefficients 0-3, 4-7, 8
   int B, T, NH, dh;
-  int head0;                 // the heads of this launch: head0 .. NH - 1
+  int heads;                 // of this launch: the last ones, whose first one every pointer but coef and status names
 };
 
 struct LocalBwdParams {
@@ -92,8 +92,7 @@ __global__ __launch_bounds__(64 * W) void slstm_local_kernel(LocalParams p) {
 
   int head, tile;
   const int ntiles = (p.B + 3) >> 2;
-  if (!local_place(ntiles * (p.NH - p.head0), p.NH - p.head0, head, tile)) return;  // the whole workgroup leaves before any barrier
-  head += p.head0;
+  if (!local_place(ntiles * p.heads, p.heads, head, tile)) return;  // the whole workgroup leaves before any barrier
   const int tid = threadIdx.x, lane = tid & 63, wave = (int)uniform((uint32_t)(tid >> 6));
   const int b = lane >> 4, n = lane & 15;
   const int dh = p.dh, H = p.NH * dh;
@@ -104,7 +103,7 @@ __global__ __launch_bounds__(64 * W) void slstm_local_kernel(LocalParams p) {
   const long long so = (long long)bc * H + head * dh + ac;
   if (p.status && blockIdx.x == 0 && tid < 16) {
     uint32_t *const word = reinterpret_cast<uint32_t *>(p.status) + tid;
-    if (p.head0 == 0) *word = tid == 5 ? 1u : (tid == 7 ? 4u : 0u);
+    if (p.heads == p.NH) *word = tid == 5 ? 1u : (tid == 7 ? 4u : 0u);
     else if (tid == 5) *word += 1u;  // (behind the launches of the heads in front: what they said stays)
     else if (tid == 7) *word = 4u;
   }
