@@ -109,13 +109,14 @@ def test_modules_put_in_the_place_of_a_layers_are_called():
 
 
 def test_graphs_of_a_cell_have_workspaces_of_their_own():
-    """Two graphs recorded on one stream, replayed on two streams at a time, beside eager calls on the stream of the capture."""
+    """Two graphs recorded on one stream, replayed on two streams at a time, beside eager calls on the stream of the capture
+    (a head is spread over 9 compute units: three calls at a time fit an XCD)."""
     print("case workspaces of graphs", flush=True)
-    cell = _cell(2, 256, torch.bfloat16)
-    xs = [torch.randn(3, 40, 8 * 256, device=DEV, dtype=torch.bfloat16) for _ in range(3)]
+    cell = _cell(2, 136, torch.bfloat16)
+    xs = [torch.randn(3, 40, 8 * 136, device=DEV, dtype=torch.bfloat16) for _ in range(3)]
     side, streams = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(2)]
     with torch.no_grad():
-        want = [_cell(2, 256, torch.bfloat16)(x) for x in xs]
+        want = [_cell(2, 136, torch.bfloat16)(x) for x in xs]
         torch.cuda.synchronize()
         with torch.cuda.stream(side):
             cell(xs[2])

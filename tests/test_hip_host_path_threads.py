@@ -78,7 +78,7 @@ def test_threads_share_a_cell(streams):
     from xlstm_amd.cell import sLSTMCell, sLSTMCellConfig
 
     torch.manual_seed(0)
-    NH, dh, T = 2, 256, 24
+    NH, dh, T = 2, 136, 24  # (a head is spread over 9 compute units: the calls of all threads fit an XCD at a time)
     cell = sLSTMCell(sLSTMCellConfig(hidden_size=NH * dh, num_heads=NH, backend="hip", recurrent_weight_init="standard")).to(DEV)
     cell.keep_state_fp32 = True
     xs = [torch.randn(B, T, 4 * NH * dh, device=DEV).bfloat16() for B in (3, 5, 8, 8)]
