@@ -1,5 +1,5 @@
-"""What the native host path keeps between the calls of a cell: a workspace that a recorded graph writes, nothing of the
-parameters."""
+"""What the native host path keeps between the calls of a cell (the plans that recorded graphs read, nothing of the parameters),
+what it gives graphs of their own, whom it calls, what it waits for and how it fails."""
 import pytest
 import torch
 
