@@ -20,7 +20,7 @@
 extern "C" {
 #endif
 
-#define XS_ABI_VERSION 17
+#define XS_ABI_VERSION 18
 
 /* element types */
 enum { XS_F32 = 0, XS_BF16 = 1 };
@@ -287,6 +287,47 @@ typedef struct xs_norm_args {
 } xs_norm_args;
 
 int xs_headwise_group_norm(const xs_norm_args *args);
+
+/*
+ * The operations around the cell of a FLOAT32 layer, forward and backward (same formulas as above; everything held and
+ * summed in float32): what a layer's training call and its float32 inference call consist of besides the cell's own calls.
+ *   xs_layer_front           x_conv = silu(conv(x)) and the cell's input wx = the four projections.  Two kernels.
+ *   xs_layer_norm            out = group norm of h.  One kernel.
+ *   xs_layer_front_backward  from d_wx (what xs_slstm_train_backward left): d_x, d_gate_w, d_conv_w and d_conv_b.  Four kernels.
+ *                            d_x_conv is its intermediate, scratch holds xs_layer_scratch_floats floats.
+ * The reference leaves these gradients to PyTorch's autograd (xlstm/blocks/slstm/layer.py:123-155).  Sums over tokens are added
+ * up in a fixed order.
+ */
+typedef struct xs_layer_args {
+  int32_t B, T, NH, dh;      /* dh a multiple of 4, at most 512; D = NH*dh */
+  int32_t K;                 /* taps, 2..4 */
+  float eps;
+  const float *x;            /* [B,T,D], strides in elements (multiples of 4), innermost contiguous */
+  int64_t x_stride_b, x_stride_t;
+  const float *conv_state;   /* front: as for xs_causal_conv_silu, or NULL */
+  int64_t conv_state_stride_b;
+  const float *conv_w;       /* [D,K] */
+  const float *conv_b;       /* [D] or NULL */
+  const float *gate_w[4];    /* each [NH,dh,dh], slot order i, f, z, o */
+  const float *norm_w;       /* [D] or NULL */
+  const uint8_t *reset;      /* [B,T] or NULL, row stride reset_stride_b bytes */
+  int64_t reset_stride_b;
+  float *x_conv;             /* [B,T,D] contiguous: written by front, read by front_backward */
+  float *wx;                 /* [B,T,4D] contiguous (front) */
+  const float *h;            /* [T,B,D] contiguous: the cell's output (norm) */
+  float *out;                /* [B,T,D] contiguous (norm) */
+  const float *d_wx;         /* [B,T,4D] contiguous (front_backward) */
+  float *d_x_conv;           /* [B,T,D] contiguous (front_backward) */
+  float *d_x;                /* [B,T,D] contiguous (front_backward) */
+  float *d_conv_w, *d_conv_b, *d_gate_w[4]; /* in the parameters' layouts; d_conv_b NULL where there is no bias */
+  float *scratch;
+  void *stream;
+} xs_layer_args;
+
+int xs_layer_front(const xs_layer_args *args);
+int xs_layer_norm(const xs_layer_args *args);
+size_t xs_layer_scratch_floats(int32_t B, int32_t T, int32_t NH, int32_t dh, int32_t K);
+int xs_layer_front_backward(const xs_layer_args *args);
 
 /*
  * Backward pass of the cell (training), by the rule of the reference's native kernel: the stabiliser m is a

@@ -17,7 +17,7 @@ LIB_PATH = os.environ.get("XLSTM_AMD_LIB", os.path.join(PKG, "lib", "libxlstm_am
 XS_F32, XS_BF16 = 0, 1
 XS_ERR_UNSUPPORTED = -5
 STATIC_SCRATCH_BYTES = (4 << 20) + (64 << 10)
-ABI_VERSION = 17
+ABI_VERSION = 18
 
 EXPORTS = (
     "xs_abi_version",
@@ -35,6 +35,10 @@ EXPORTS = (
     "xs_causal_conv_silu",
     "xs_headwise_gates",
     "xs_headwise_group_norm",
+    "xs_layer_front",
+    "xs_layer_norm",
+    "xs_layer_scratch_floats",
+    "xs_layer_front_backward",
     "xs_measure_stage",
     "xs_slstm_train_coef_floats",
     "xs_slstm_train_exchange_bytes",
@@ -155,6 +159,38 @@ class NormArgs(ctypes.Structure):
     ]
 
 
+class LayerArgs(ctypes.Structure):
+    """Mirror of ``xs_layer_args``."""
+
+    _fields_ = [
+        ("B", ctypes.c_int32), ("T", ctypes.c_int32), ("NH", ctypes.c_int32), ("dh", ctypes.c_int32),
+        ("K", ctypes.c_int32),
+        ("eps", ctypes.c_float),
+        ("x", ctypes.c_void_p),
+        ("x_stride_b", ctypes.c_int64), ("x_stride_t", ctypes.c_int64),
+        ("conv_state", ctypes.c_void_p),
+        ("conv_state_stride_b", ctypes.c_int64),
+        ("conv_w", ctypes.c_void_p),
+        ("conv_b", ctypes.c_void_p),
+        ("gate_w", ctypes.c_void_p * 4),
+        ("norm_w", ctypes.c_void_p),
+        ("reset", ctypes.c_void_p),
+        ("reset_stride_b", ctypes.c_int64),
+        ("x_conv", ctypes.c_void_p),
+        ("wx", ctypes.c_void_p),
+        ("h", ctypes.c_void_p),
+        ("out", ctypes.c_void_p),
+        ("d_wx", ctypes.c_void_p),
+        ("d_x_conv", ctypes.c_void_p),
+        ("d_x", ctypes.c_void_p),
+        ("d_conv_w", ctypes.c_void_p),
+        ("d_conv_b", ctypes.c_void_p),
+        ("d_gate_w", ctypes.c_void_p * 4),
+        ("scratch", ctypes.c_void_p),
+        ("stream", ctypes.c_void_p),
+    ]
+
+
 STAGE_EXCHANGE, STAGE_CONTRACTION, STAGE_GATING, STAGE_LAUNCH, STAGE_CHAIN = 0, 1, 2, 3, 4
 
 
@@ -219,6 +255,11 @@ def load() -> ctypes.CDLL:
     lib.xs_headwise_gates.argtypes = [ctypes.POINTER(GatesArgs)]
     lib.xs_headwise_group_norm.restype = ctypes.c_int
     lib.xs_headwise_group_norm.argtypes = [ctypes.POINTER(NormArgs)]
+    for fn in (lib.xs_layer_front, lib.xs_layer_norm, lib.xs_layer_front_backward):
+        fn.restype = ctypes.c_int
+        fn.argtypes = [ctypes.POINTER(LayerArgs)]
+    lib.xs_layer_scratch_floats.restype = ctypes.c_size_t
+    lib.xs_layer_scratch_floats.argtypes = [ctypes.c_int32] * 5
     lib.xs_slstm_train_coef_floats.restype = ctypes.c_size_t
     lib.xs_slstm_train_coef_floats.argtypes = [ctypes.c_int32] * 5
     lib.xs_slstm_train_exchange_bytes.restype = ctypes.c_size_t
@@ -260,7 +301,8 @@ def host():
     spec.loader.exec_module(mod)
     names = ("xs_slstm_step", "xs_slstm_forward_watched", "xs_slstm_workspace_bytes", "xs_last_error", "xs_causal_conv_silu",
              "xs_headwise_gates", "xs_headwise_group_norm", "xs_slstm_train_coef_floats", "xs_slstm_train_exchange_bytes",
-             "xs_slstm_train_forward", "xs_slstm_train_backward", "xs_slstm_backward_params")
+             "xs_slstm_train_forward", "xs_slstm_train_backward", "xs_slstm_backward_params", "xs_layer_front", "xs_layer_norm",
+             "xs_layer_scratch_floats", "xs_layer_front_backward")
     mod.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names}, EngineError,
              torch_module._global_forward_hooks, torch_module._global_forward_pre_hooks)
     _HOST = mod

@@ -1,5 +1,5 @@
-// Native host path of the calls a program makes often: a decode step, an inference call and a training call of a cell,
-// and the first two of a layer.  What the Python layers of cell.py, layer.py and functional.py do for such a call - look at dtypes, strides,
+// Native host path of the calls a program makes often: a decode step, an inference call and a training call of a cell
+// and of a layer (training: in float32).  What the Python layers of cell.py, layer.py and functional.py do for such a call - look at dtypes, strides,
 // versions and modes, allocate the outputs, fill an argument block, launch - takes 15 us per cell call and 75 us per
 // layer call there, more than the kernels run; here it takes about 4 and 8.
 //
@@ -50,6 +50,10 @@ struct Engine {
   decltype(&xs_slstm_train_forward) train_forward = nullptr;
   decltype(&xs_slstm_train_backward) train_backward = nullptr;
   decltype(&xs_slstm_backward_params) backward_params = nullptr;
+  decltype(&xs_layer_front) layer_front = nullptr;
+  decltype(&xs_layer_norm) layer_norm = nullptr;
+  decltype(&xs_layer_scratch_floats) layer_scratch = nullptr;
+  decltype(&xs_layer_front_backward) layer_front_backward = nullptr;
   PyObject *error = nullptr;              // functional.EngineError
   PyObject *global_hooks[2] = {nullptr, nullptr};  // hooks on every module of the process
 } g_engine;
@@ -58,7 +62,7 @@ struct Engine {
 struct Names {
   PyObject *r, *b, *weight, *bias, *conv_state, *slstm_state, *input_shape, *output_shape, *keep_state_fp32, *config;
   PyObject *modules, *parameters, *forward_hooks, *forward_pre_hooks, *training, *p, *eps, *conv1d, *conv, *fgate, *igate, *zgate, *ogate;
-  PyObject *group_norm, *slstm_cell, *dropout, *fused_pre_ops, *bsgnh, *cut, *clipval;
+  PyObject *group_norm, *slstm_cell, *dropout, *fused_pre_ops, *bsgnh, *cut, *clipval, *gradients_with_graph;
 } g_names;
 
 struct PyRef {  // owns one reference
@@ -590,6 +594,29 @@ CellGradients run_reverse(const ReverseInputs &in, const at::Tensor &d_h, int64_
   return g;
 }
 
+// the gradient of the output as the reverse pass reads it: [S,B,NH,dh] or [S,B,1,H] of the output's type, with the strides of a
+// row and of a step
+at::Tensor output_gradient(const ReverseInputs &in, OutShape shape, const at::Tensor &given, int64_t &sb, int64_t &st) {
+  const int64_t H = in.NH * in.dh;
+  auto sbh = [&](const at::Tensor &t) {
+    switch (shape) {
+      case OutShape::BNSH: return t.permute({2, 0, 1, 3});
+      case OutShape::SBH: return t.unsqueeze(2);
+      case OutShape::BSH: return t.permute({1, 0, 2}).unsqueeze(2);
+      default: return t;
+    }
+  };
+  at::Tensor d = given.defined() ? sbh(given) : at::zeros({in.T, in.B, 1, H}, in.h.options());
+  const int64_t esz = in.h.element_size();
+  sb = in.B > 1 ? d.stride(1) : H; st = d.stride(0);
+  if (d.scalar_type() != in.h.scalar_type() || d.stride(3) != 1 || (d.size(2) > 1 && d.stride(2) != in.dh) || !aligned(d.data_ptr(), 16) ||
+      (sb * esz) % 16 || (st * esz) % 16 || sb >= (1 << 25) || sb < 0 || st < 0) {
+    d = d.to(in.h.scalar_type()).contiguous();
+    sb = H; st = in.B * H;
+  }
+  return d;
+}
+
 using torch::autograd::SavedVariable;
 using torch::autograd::variable_list;
 
@@ -616,30 +643,13 @@ struct CellBackward : public torch::autograd::Node {
     ReverseInputs call = in;
     x.unpack();
     b.unpack();
-    const at::Tensor h_saved = h.unpack(shared_from_this());
-    c10::OptionalDeviceGuard guard(h_saved.device());
-    const int64_t B = in.B, T = in.T, dh = in.dh, H = in.NH * dh;
-    // [S,B,H] views of the output and its gradient
-    auto sbh = [&](const at::Tensor &t) {
-      switch (shape) {
-        case OutShape::BNSH: return t.permute({2, 0, 1, 3});
-        case OutShape::SBH: return t.unsqueeze(2);
-        case OutShape::BSH: return t.permute({1, 0, 2}).unsqueeze(2);
-        default: return t;
-      }
-    };
-    call.h = h_saved;
+    call.h = h.unpack(shared_from_this());
+    c10::OptionalDeviceGuard guard(call.h.device());
     call.r = r.unpack();
     call.coef = coef.unpack();
     if (has_state) call.state = state.unpack();
-    at::Tensor d = grads[0].defined() ? sbh(grads[0]) : at::zeros({T, B, 1, H}, h_saved.options());  // [S,B,NH,dh] or [S,B,1,H]
-    const int64_t esz = h_saved.element_size();
-    int64_t sb = B > 1 ? d.stride(1) : H, st = d.stride(0);
-    if (d.scalar_type() != h_saved.scalar_type() || d.stride(3) != 1 || (d.size(2) > 1 && d.stride(2) != dh) || !aligned(d.data_ptr(), 16) ||
-        (sb * esz) % 16 || (st * esz) % 16 || sb >= (1 << 25) || sb < 0 || st < 0) {
-      d = d.to(h_saved.scalar_type()).contiguous();
-      sb = H; st = B * H;
-    }
+    int64_t sb, st;
+    const at::Tensor d = output_gradient(call, shape, grads[0], sb, st);
     CellGradients g = run_reverse(call, d, sb, st, grads[1]);
     variable_list out(has_state ? 4 : 3);
     out[0] = transposed_input ? g.d_wx.permute({1, 0, 2}) : g.d_wx;
@@ -837,13 +847,14 @@ PyObject *submodule(PyObject *module, PyObject *name) {  // borrowed, or null
   PyObject *modules = module_dict(module, g_names.modules), *m = modules ? PyDict_GetItem(modules, name) : nullptr;
   return absent(m) ? nullptr : m;
 }
-// a parameter of a module in the type and place of x; absent: an undefined tensor.  false: another type, layout or device
+// a parameter of a module in the type and place of x; None: an undefined tensor.  false: another type, layout or device, or no
+// parameter of that name (it may be a plain attribute meanwhile, made from other tensors)
 bool parameter(PyObject *module, PyObject *name, const at::Tensor &x, at::Tensor &out) {
   PyObject *parameters = module_dict(module, g_names.parameters), *o = parameters ? PyDict_GetItem(parameters, name) : nullptr;
   const at::Tensor *t;
-  if (!parameters || !optional_tensor(o, t)) return false;
+  if (!o || !optional_tensor(o, t)) return false;
   if (t) out = *t;
-  return !t || (t->scalar_type() == at::kBFloat16 && t->is_contiguous() && t->device() == x.device() && aligned(t->data_ptr(), 16));
+  return !t || (t->scalar_type() == x.scalar_type() && t->is_contiguous() && t->device() == x.device() && aligned(t->data_ptr(), 16));
 }
 bool has_hooks(PyObject *module) {
   PyObject *after = module_dict(module, g_names.forward_hooks), *before = module_dict(module, g_names.forward_pre_hooks);
@@ -857,29 +868,33 @@ struct LayerParts {
   at::Tensor conv_w, conv_b, gate[4], norm_w;
   double eps = 1e-5;
   int64_t K = 0, NH = 0, dh = 0, D = 0;
+  bool float32 = false;
 };
 
-// what a layer call needs of its modules; false unless the engine's kernels apply (sLSTMLayer._fused) and no gradient is
-// recorded
-bool collect(PyObject *layer, PyObject *cell_path, const at::Tensor &x, LayerParts &p) {
+// what a layer call needs of its modules; false unless the engine's kernels apply (bfloat16: sLSTMLayer._fused) and a gradient is
+// recorded (`train`: dropout and norm behind the cell are called as modules then) or none is
+bool collect(PyObject *layer, PyObject *cell_path, const at::Tensor &x, LayerParts &p, bool train = false) {
   p.cell = ((CellPathObject *)cell_path)->c;
   p.NH = p.cell->NH; p.dh = p.cell->dh; p.D = p.NH * p.dh;
-  if (x.dim() != 3 || x.scalar_type() != at::kBFloat16 || !x.is_cuda() || x.size(2) != p.D || p.dh % 64 || p.dh > 1024 ||
-      at::autocast::is_autocast_enabled(at::kCUDA) || recording(*p.cell, x, nullptr))
+  p.float32 = x.scalar_type() == at::kFloat;
+  if (x.dim() != 3 || (!p.float32 && x.scalar_type() != at::kBFloat16) || !x.is_cuda() || x.size(2) != p.D ||
+      (p.float32 ? p.dh % 4 || p.dh > 512 : p.dh % 64 || p.dh > 1024) || at::autocast::is_autocast_enabled(at::kCUDA))
     return false;
+  bool records = recording(*p.cell, x, nullptr);
+  if (records && !train) return false;
   for (PyObject *h : g_engine.global_hooks)
     if (h && PyDict_Size(h)) return false;
   PyObject *cell = submodule(layer, g_names.slstm_cell), *conv1d = submodule(layer, g_names.conv1d);
   PyObject *conv = conv1d ? submodule(conv1d, g_names.conv) : nullptr;
   PyObject *norm = submodule(layer, g_names.group_norm), *dropout = submodule(layer, g_names.dropout);
-  if (!cell || !conv || !norm || !dropout || has_hooks(cell) || has_hooks(dropout)) return false;
+  if (!cell || !conv || !norm || !dropout || has_hooks(cell) || (!train && has_hooks(dropout))) return false;
   {
     PyRef fused(attribute(layer, g_names.fused_pre_ops));
     if (fused.o != Py_True) return false;
     PyRef training(attribute(dropout, g_names.training)), rate(attribute(dropout, g_names.p));
     const double dp = PyFloat_AsDouble(rate.o);
     if (PyErr_Occurred()) { PyErr_Clear(); return false; }
-    if (training.o == Py_True && dp != 0.0) return false;
+    if (!train && training.o == Py_True && dp != 0.0) return false;
     PyRef keep(attribute(cell, g_names.keep_state_fp32)), eps(attribute(norm, g_names.eps));
     p.keep_state = keep.o == Py_True;
     p.eps = PyFloat_AsDouble(eps.o);
@@ -889,19 +904,18 @@ bool collect(PyObject *layer, PyObject *cell_path, const at::Tensor &x, LayerPar
   OutShape shape;
   if (!input_is_bsgnh(p.cell_config.o) || !out_shape(p.cell_config.o, shape) || shape != OutShape::BNSH) return false;
   if (!parameter(conv, g_names.weight, x, p.conv_w) || !p.conv_w.defined() || !parameter(conv, g_names.bias, x, p.conv_b) ||
-      !parameter(norm, g_names.weight, x, p.norm_w))
+      (!train && !parameter(norm, g_names.weight, x, p.norm_w)))
     return false;
   // (the module called fgate feeds the i slot, igate the f slot)
   PyObject *gates[4] = {g_names.fgate, g_names.igate, g_names.zgate, g_names.ogate};
-  bool needs_grad = x.requires_grad();
   for (int g = 0; g < 4; ++g) {
     PyObject *gate = submodule(layer, gates[g]);
     if (!gate || !parameter(gate, g_names.weight, x, p.gate[g]) || !p.gate[g].defined() || p.gate[g].numel() != p.NH * p.dh * p.dh) return false;
-    needs_grad |= p.gate[g].requires_grad();
   }
-  for (const at::Tensor *t : {&p.conv_w, &p.conv_b, &p.norm_w}) needs_grad |= t->defined() && t->requires_grad();
+  for (const at::Tensor *t : {&p.conv_w, &p.conv_b, &p.norm_w, &p.gate[0], &p.gate[1], &p.gate[2], &p.gate[3]})
+    records |= at::GradMode::is_enabled() && t->defined() && t->requires_grad();
   p.K = p.conv_w.numel() / p.D;
-  return p.K >= 2 && p.K <= 4 && !(at::GradMode::is_enabled() && needs_grad);  // (the cell's own parameters: recording)
+  return p.K >= 2 && p.K <= 4 && records == train;
 }
 
 void run_conv(const LayerParts &p, const at::Tensor &x, const void *taps, int64_t taps_stride, const at::Tensor *mask, void *out, void *ring, void *stream) {
@@ -934,14 +948,30 @@ void run_norm(const LayerParts &p, const at::Tensor &h, int64_t B, int64_t T, vo
   launched(g_engine.norm(&a));
 }
 
+// the float32 kernels' argument block, with what a pass in either direction needs; x: contiguous
+xs_layer_args float32_args(const LayerParts &p, const at::Tensor &x, const at::Tensor &x_conv, const at::Tensor *mask) {
+  xs_layer_args a{};
+  a.B = (int32_t)x.size(0); a.T = (int32_t)x.size(1); a.NH = (int32_t)p.NH; a.dh = (int32_t)p.dh; a.K = (int32_t)p.K;
+  a.eps = (float)p.eps;
+  auto ptr = [](const at::Tensor &t) { return t.defined() ? (const float *)t.data_ptr() : nullptr; };
+  a.x = ptr(x); a.x_stride_b = x.stride(0); a.x_stride_t = x.stride(1);
+  a.conv_w = ptr(p.conv_w); a.conv_b = ptr(p.conv_b); a.norm_w = ptr(p.norm_w);
+  for (int g = 0; g < 4; ++g) a.gate_w[g] = ptr(p.gate[g]);
+  a.reset = mask ? (const uint8_t *)mask->data_ptr() : nullptr; a.reset_stride_b = mask ? mask->stride(0) : 0;
+  a.x_conv = (float *)x_conv.data_ptr();
+  a.stream = stream_of(x.device());
+  return a;
+}
+
 // the taps in front of the first token: a [B,n,D] tensor of which the last K-1 inputs count
 bool taps_of(const LayerParts &p, const at::Tensor &t, int64_t B, const void *&taps, int64_t &stride) {
   const int64_t n = t.dim() == 3 ? t.size(1) : 0;
-  if (t.scalar_type() != at::kBFloat16 || n < p.K - 1 || t.size(0) != B || t.size(2) != p.D || t.stride(2) != 1 || t.stride(1) != p.D || t.stride(0) % 8 ||
-      !t.is_cuda() || !aligned(t.data_ptr(), 16))
+  const int64_t esz = p.float32 ? 4 : 2;
+  if (t.scalar_type() != (p.float32 ? at::kFloat : at::kBFloat16) || n < p.K - 1 || t.size(0) != B || t.size(2) != p.D || t.stride(2) != 1 ||
+      t.stride(1) != p.D || t.stride(0) * esz % 16 || !t.is_cuda() || !aligned(t.data_ptr(), 16))
     return false;
   stride = t.stride(0);
-  taps = (const char *)t.data_ptr() + (n - (p.K - 1)) * p.D * 2;
+  taps = (const char *)t.data_ptr() + (n - (p.K - 1)) * p.D * esz;
   return true;
 }
 
@@ -967,7 +997,7 @@ PyObject *layer_step_(PyObject *const *args) {
     Py_RETURN_NONE;
   const at::Tensor &x = *xp, &state = *statep;
   LayerParts p;
-  if (!collect(args[0], args[1], x, p) || !step_fits(c, x, state, buffers) || !aligned(x.data_ptr(), 16)) Py_RETURN_NONE;
+  if (!collect(args[0], args[1], x, p) || p.float32 || !step_fits(c, x, state, buffers) || !aligned(x.data_ptr(), 16)) Py_RETURN_NONE;
   const int64_t B = x.size(0);
   if (B < 1) Py_RETURN_NONE;
   const void *taps = nullptr;
@@ -1039,16 +1069,26 @@ PyObject *layer_forward_(PyObject *const *args) {
     at::Tensor x = x_in.is_contiguous() && aligned(x_in.data_ptr(), 16) ? x_in : x_in.contiguous();
     void *stream = stream_of(x.device());
     at::Tensor wx = at::empty({B, T, 4 * p.D}, x.options()), x_conv = at::empty({B, T, p.D}, x.options());
-    run_conv(p, x, taps, taps_stride, maskp, x_conv.data_ptr(), nullptr, stream);
-    run_gates(p, x, x_conv.data_ptr(), wx.data_ptr(), stream);
-    s.run(wx, state, maskp, OutShape::SBH);
     out = x_conv;  // (its last reader has been launched in front of the norm)
-    run_norm(p, s.h, B, T, out.data_ptr(), stream);
+    if (p.float32) {
+      xs_layer_args a = float32_args(p, x, x_conv, maskp);
+      a.conv_state = (const float *)taps; a.conv_state_stride_b = taps && B > 1 ? taps_stride : 0;
+      a.wx = (float *)wx.data_ptr();
+      launched(g_engine.layer_front(&a));
+      s.run(wx, state, maskp, OutShape::SBH);
+      a.h = (const float *)s.h.data_ptr(); a.out = (float *)out.data_ptr();
+      launched(g_engine.layer_norm(&a));
+    } else {
+      run_conv(p, x, taps, taps_stride, maskp, x_conv.data_ptr(), nullptr, stream);
+      run_gates(p, x, x_conv.data_ptr(), wx.data_ptr(), stream);
+      s.run(wx, state, maskp, OutShape::SBH);
+      run_norm(p, s.h, B, T, out.data_ptr(), stream);
+    }
     if (last) {
       // the last K-1 inputs: a tensor of their own where the call continued a state (x may be reused for the next chunk)
       tail = x_in.narrow(1, T - (p.K - 1), p.K - 1);
       if (taps) tail = tail.clone();
-      state_out = p.keep_state ? s.state : s.state.to(at::kBFloat16);
+      state_out = p.keep_state || p.float32 ? s.state : s.state.to(at::kBFloat16);
     }
   }
   s.leave();
@@ -1058,6 +1098,191 @@ PyObject *layer_forward_(PyObject *const *args) {
   PyRef pt(THPVariable_Wrap(tail));
   PyRef states(states_dict(pt.o, state_out));
   return PyTuple_Pack(2, po.o, states.o);
+}
+
+// ---- training of a float32 layer: one node of the autograd graph for everything between x and the cell's output
+struct PythonObject {  // a reference that is given back with the GIL held
+  PyObject *o;
+  explicit PythonObject(PyObject *p) : o(p) { Py_INCREF(o); }
+  ~PythonObject() {
+    if (!Py_IsInitialized()) return;
+    PyGILState_STATE gil = PyGILState_Ensure();
+    Py_DECREF(o);
+    PyGILState_Release(gil);
+  }
+  PythonObject(const PythonObject &) = delete;
+  PythonObject &operator=(const PythonObject &) = delete;
+};
+
+struct LayerBackward : public torch::autograd::Node {
+  // the inputs in the order of the gradients: x, convolution weight and bias, the four gate weights, R, b, state
+  enum { X, CONV_W, CONV_B, GATE, R = GATE + 4, BIAS, STATE, INPUTS };
+  SavedVariable inputs[INPUTS], x_conv, h, coef;
+  bool given[INPUTS] = {};
+  std::shared_ptr<Share> share;  // the coefficients'
+  ReverseInputs in;  // (its saved tensors are filled in when the backward runs)
+  int64_t K = 0;
+  at::ScalarType r_dtype = at::kFloat, b_dtype = at::kFloat, s_dtype = at::kFloat;
+  std::unique_ptr<PythonObject> layer;
+
+  std::string name() const override { return "sLSTMLayerBackward"; }
+  void release_variables() override {
+    std::unique_ptr<PythonObject> last;  // (given back behind the lock: that may run Python code)
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (SavedVariable &v : inputs) v.reset_data();
+    for (SavedVariable *v : {&x_conv, &h, &coef}) v->reset_data();
+    in.mask.reset();
+    share.reset();
+    last = std::move(layer);
+  }
+
+  // A backward that is itself recorded (create_graph): the layer's operations once more, one by one, and their gradients
+  variable_list with_graph(PyObject *module, const at::Tensor (&t)[INPUTS], const at::Tensor &reset, const variable_list &grads) {
+    struct Gil { PyGILState_STATE g = PyGILState_Ensure(); ~Gil() { PyGILState_Release(g); } } gil;
+    PyRef held(module);
+    auto wrapped = [](const at::Tensor &v) {
+      if (v.defined()) return THPVariable_Wrap(v);
+      Py_INCREF(Py_None);
+      return Py_None;
+    };
+    PyRef list(PyTuple_New(INPUTS)), d_out(wrapped(grads[0])), d_state(wrapped(grads[1])), mask(wrapped(reset));
+    if (list.o)
+      for (int i = 0; i < INPUTS; ++i) PyTuple_SET_ITEM(list.o, i, wrapped(t[i]));
+    PyRef result(list.o && module ? PyObject_CallMethodObjArgs(module, g_names.gradients_with_graph, list.o, mask.o, d_out.o, d_state.o, nullptr) : nullptr);
+    variable_list out(INPUTS);
+    if (!result.o || !PyTuple_Check(result.o) || PyTuple_GET_SIZE(result.o) != INPUTS) {
+      if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "the gradients of the layer are missing");
+      python_error e;
+      e.persist();
+      throw e;
+    }
+    for (int i = 0; i < INPUTS; ++i)
+      if (const at::Tensor *g = tensor_of(PyTuple_GET_ITEM(result.o, i))) out[i] = *g;
+    return out;
+  }
+
+  variable_list apply(variable_list &&grads) override {
+    at::Tensor t[INPUTS], xc;
+    ReverseInputs call;
+    PyObject *module = nullptr;
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      for (int i = 0; i < INPUTS; ++i)
+        if (given[i]) t[i] = inputs[i].unpack();
+      call = in;
+      call.h = h.unpack(shared_from_this());
+      call.coef = coef.unpack();
+      xc = x_conv.unpack();
+      if (at::GradMode::is_enabled() && layer) {
+        PyGILState_STATE gil = PyGILState_Ensure();
+        module = layer->o;
+        Py_INCREF(module);
+        PyGILState_Release(gil);
+      }
+    }
+    c10::OptionalDeviceGuard guard(call.h.device());
+    if (at::GradMode::is_enabled()) return with_graph(module, t, call.mask, grads);
+    at::NoGradGuard no_grad;
+    call.r = t[R];
+    if (given[STATE]) call.state = t[STATE];
+    const int64_t B = in.B, T = in.T, D = in.NH * in.dh;
+    int64_t sb, st;
+    const at::Tensor d = output_gradient(call, OutShape::BNSH, grads[0], sb, st);
+    CellGradients g = run_reverse(call, d, sb, st, grads[1]);
+    const auto f32 = call.h.options();
+    const at::Tensor x = t[X].is_contiguous() && aligned(t[X].data_ptr(), 16) ? t[X] : t[X].clone(at::MemoryFormat::Contiguous);
+    LayerParts p;
+    p.NH = in.NH; p.dh = in.dh; p.D = D; p.K = K;
+    p.conv_w = t[CONV_W]; p.conv_b = t[CONV_B];
+    for (int i = 0; i < 4; ++i) p.gate[i] = t[GATE + i];
+    xs_layer_args a = float32_args(p, x, xc, call.mask.defined() ? &call.mask : nullptr);
+    variable_list out(INPUTS);
+    for (int i = CONV_W; i < R; ++i)
+      if (given[i]) out[i] = at::empty(t[i].sizes(), f32);
+    out[X] = at::empty({B, T, D}, f32);
+    const at::Tensor d_x_conv = at::empty({B, T, D}, f32);
+    const at::Tensor scratch = at::empty({(int64_t)g_engine.layer_scratch((int32_t)B, (int32_t)T, (int32_t)in.NH, (int32_t)in.dh, (int32_t)K)}, f32);
+    auto ptr = [](const at::Tensor &v) { return v.defined() ? (float *)v.data_ptr() : nullptr; };
+    a.scratch = ptr(scratch);
+    a.d_wx = ptr(g.d_wx); a.d_x = ptr(out[X]);
+    a.d_x_conv = ptr(d_x_conv);
+    a.d_conv_w = ptr(out[CONV_W]); a.d_conv_b = ptr(out[CONV_B]);
+    for (int i = 0; i < 4; ++i) a.d_gate_w[i] = ptr(out[GATE + i]);
+    const int rc = g_engine.layer_front_backward(&a);
+    if (rc != XS_OK) engine_failed_in_backward(rc);
+    out[R] = g.d_r.to(r_dtype);
+    out[BIAS] = g.d_bias.to(b_dtype);
+    if (given[STATE]) out[STATE] = g.d_s0.to(s_dtype);
+    return out;
+  }
+};
+
+// layer_train(layer, cell path, x, slstm_state, reset_mask, bytes of coefficients that a device may hold) -> (the cell's output,
+// state) with their place in the graph, or None.  The caller has looked at the modules (sLSTMLayer._plain_modules)
+PyObject *layer_train_(PyObject *const *args) {
+  const at::Tensor *xp = tensor_of(args[2]), *state, *mask_in;
+  if (!xp || !optional_tensor(args[3], state) || !optional_tensor(args[4], mask_in)) Py_RETURN_NONE;
+  const at::Tensor &x_in = *xp;
+  LayerParts p;
+  if (x_in.dim() != 3 || x_in.size(1) < 2 || x_in.scalar_type() != at::kFloat || !collect(args[0], args[1], x_in, p, true)) Py_RETURN_NONE;
+  CellPath &c = *p.cell;
+  const int64_t B = x_in.size(0), T = x_in.size(1);
+  const at::Tensor *rp, *bp;
+  if (!sequence_fits(c, x_in, B, T, state, mask_in) || !g_engine.coef_floats(1, 1, (int32_t)p.NH, (int32_t)p.dh, XS_F32) || !c.weights(rp, bp))
+    Py_RETURN_NONE;
+  const at::Tensor given[LayerBackward::INPUTS] = {x_in, p.conv_w, p.conv_b, p.gate[0], p.gate[1], p.gate[2], p.gate[3], *rp, *bp, state ? *state : at::Tensor()};
+  for (const at::Tensor &t : given)
+    if (t.defined() && t._fw_grad(0).defined()) Py_RETURN_NONE;  // (forward mode: the general path refuses it)
+  PyRef cut(PyObject_GetAttr(p.cell_config.o, g_names.cut)), clip(PyObject_GetAttr(p.cell_config.o, g_names.clipval));
+  if (!cut.o || !clip.o) throw PythonError{};
+  const int cut_on = PyObject_IsTrue(cut.o);
+  const double clipval = clip.o == Py_None ? 0.0 : PyFloat_AsDouble(clip.o);
+  const int64_t limit = PyLong_AsLongLong(args[5]);
+  if (PyErr_Occurred()) throw PythonError{};
+  c10::OptionalDeviceGuard guard(x_in.device());
+  if (!have_word(c, x_in.device())) Py_RETURN_NONE;
+  std::shared_ptr<Share> share = Share::take(x_in.device().index(), 4 * (int64_t)g_engine.coef_floats((int32_t)B, (int32_t)T, (int32_t)p.NH, (int32_t)p.dh, XS_F32), limit);
+  if (!share) Py_RETURN_NONE;
+  Sequence s(c, x_in.device(), B);
+  auto layer = std::make_unique<PythonObject>(args[0]);
+  {
+    WithoutGil no_gil;
+    at::Tensor x_conv;
+    {
+      at::NoGradGuard no_grad;
+      at::Tensor mask;
+      if (mask_in) mask = mask_bytes(*mask_in);
+      const at::Tensor *maskp = mask_in ? &mask : nullptr;
+      const at::Tensor x = x_in.is_contiguous() && aligned(x_in.data_ptr(), 16) ? x_in.detach() : x_in.clone(at::MemoryFormat::Contiguous);
+      const at::Tensor wx = at::empty({B, T, 4 * p.D}, x.options());
+      x_conv = at::empty({B, T, p.D}, x.options());
+      xs_layer_args a = float32_args(p, x, x_conv, maskp);
+      a.wx = (float *)wx.data_ptr();
+      launched(g_engine.layer_front(&a));
+      s.run(wx, state, maskp, OutShape::BNSH, true);
+    }
+    auto node = std::shared_ptr<LayerBackward>(new LayerBackward(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(given[0], given[1], given[2], given[3], given[4], given[5], given[6], given[7], given[8], given[9]));
+    for (int i = 0; i < LayerBackward::INPUTS; ++i)
+      if ((node->given[i] = given[i].defined())) node->inputs[i] = SavedVariable(given[i], false);
+    node->x_conv = SavedVariable(x_conv, false);
+    node->coef = SavedVariable(s.coef, false);
+    node->share = std::move(share);
+    node->K = p.K;
+    node->r_dtype = rp->scalar_type(); node->b_dtype = bp->scalar_type();
+    if (state) node->s_dtype = state->scalar_type();
+    node->in.mask = s.mask; node->in.word = s.word; node->in.calls = c.calls;
+    node->in.B = B; node->in.T = T; node->in.NH = p.NH; node->in.dh = p.dh;
+    node->in.cut = cut_on != 0; node->in.clip = clipval;
+    node->layer = std::move(layer);
+    torch::autograd::set_history(s.h, node);
+    torch::autograd::set_history(s.state, node);
+    node->h = SavedVariable(s.h, true);
+  }
+  s.leave();
+  PyRef ph(THPVariable_Wrap(s.h)), ps(THPVariable_Wrap(s.state));
+  if (!ph.o || !ps.o) throw PythonError{};
+  return PyTuple_Pack(2, ph.o, ps.o);
 }
 
 template <PyObject *(*F)(PyObject *const *), int N>
@@ -1108,7 +1333,9 @@ PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
       !get("xs_causal_conv_silu", g_engine.conv) || !get("xs_headwise_gates", g_engine.gates) || !get("xs_headwise_group_norm", g_engine.norm) ||
       !get("xs_slstm_train_coef_floats", g_engine.coef_floats) || !get("xs_slstm_train_exchange_bytes", g_engine.exchange_bytes) ||
       !get("xs_slstm_train_forward", g_engine.train_forward) || !get("xs_slstm_train_backward", g_engine.train_backward) ||
-      !get("xs_slstm_backward_params", g_engine.backward_params)) {
+      !get("xs_slstm_backward_params", g_engine.backward_params) || !get("xs_layer_front", g_engine.layer_front) ||
+      !get("xs_layer_norm", g_engine.layer_norm) || !get("xs_layer_scratch_floats", g_engine.layer_scratch) ||
+      !get("xs_layer_front_backward", g_engine.layer_front_backward)) {
     PyErr_SetString(PyExc_KeyError, "an entry point of the engine is missing");
     return nullptr;
   }
@@ -1124,6 +1351,7 @@ PyMethodDef module_methods[] = {
     {"kept", (PyCFunction)(void *)kept, METH_FASTCALL, nullptr},
     {"layer_step", (PyCFunction)(void *)layer_call<layer_step_, 10>, METH_FASTCALL, nullptr},
     {"layer_forward", (PyCFunction)(void *)layer_call<layer_forward_, 7>, METH_FASTCALL, nullptr},
+    {"layer_train", (PyCFunction)(void *)layer_call<layer_train_, 6>, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_xlstm_host", "native host path of the cell's and the layer's frequent calls", -1, module_methods,
                           nullptr, nullptr, nullptr, nullptr};
@@ -1135,7 +1363,7 @@ PyMODINIT_FUNC PyInit__xlstm_host(void) {
   g_names = Names{s("_recurrent_kernel_"), s("_bias_"), s("weight"), s("bias"), s("conv_state"), s("slstm_state"), s("input_shape"), s("output_shape"),
                   s("keep_state_fp32"), s("config"), s("_modules"), s("_parameters"), s("_forward_hooks"), s("_forward_pre_hooks"), s("training"), s("p"),
                   s("eps"), s("conv1d"), s("conv"), s("fgate"), s("igate"), s("zgate"), s("ogate"), s("group_norm"), s("slstm_cell"), s("dropout"),
-                  s("fused_pre_ops"), s("BSGNH"), s("gradient_recurrent_cut"), s("gradient_recurrent_clipval")};
+                  s("fused_pre_ops"), s("BSGNH"), s("gradient_recurrent_cut"), s("gradient_recurrent_clipval"), s("_gradients_with_graph")};
   PyObject *m = PyModule_Create(&module_def);
   if (!m) return nullptr;
   g_cell_type = (PyTypeObject *)PyType_FromSpec(&cell_spec);

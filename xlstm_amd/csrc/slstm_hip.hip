@@ -23,6 +23,8 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
+#include <initializer_list>
 #include <mutex>
 
 #include "xlstm_amd.h"
@@ -35,6 +37,7 @@
 #include "slstm_step_small_kernel.h"
 #include "slstm_backward_kernels.h"
 #include "slstm_layer_kernels.h"
+#include "slstm_layer_f32_kernels.h"
 #include "slstm_local_kernel.h"
 #include "slstm_backward_unit_kernel.h"
 #include "slstm_backward_quad_kernel.h"
@@ -1258,6 +1261,158 @@ int run_group_norm(const xs_norm_args *a) {
   return XS_OK;
 }
 
+// ---- the float32 layer around the cell (slstm_layer_f32_kernels.h)
+int layer_launched(const char *what) {
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? XS_OK : fail(XS_ERR_LAUNCH, "%s launch failed: %s", what, hipGetErrorString(e));
+}
+bool layer_misaligned(std::initializer_list<const void *> ptrs) {
+  for (const void *q : ptrs)
+    if ((uintptr_t)q % 16) return true;
+  return false;
+}
+int layer_check(const xs_layer_args *a) {
+  if (!a) return fail(XS_ERR_NULL, "args is NULL");
+  if (a->B < 0 || a->T < 0 || a->NH <= 0 || a->dh <= 0) return fail(XS_ERR_SHAPE, "bad dims B=%d T=%d NH=%d dh=%d", a->B, a->T, a->NH, a->dh);
+  if (a->dh % 4 || a->dh > 512) return fail(XS_ERR_UNSUPPORTED, "head dim %d is not a multiple of 4 up to 512", a->dh);
+  if ((long long)a->B * a->T > (1ll << 29)) return fail(XS_ERR_UNSUPPORTED, "too many tokens for one call");
+  return XS_OK;
+}
+// how a backward pass splits its sums over tokens
+struct LayerSplit { int conv_blocks, slices, slice_tokens; size_t gate_floats, conv_floats; };
+LayerSplit layer_split(int B, int T, int NH, int dh, int K) {
+  LayerSplit s;
+  const long long M = (long long)B * T, D = (long long)NH * dh, up = (dh + 63) / 64;
+  s.conv_blocks = (int)(((long long)B * ((T + kConvBackRun - 1) / kConvBackRun) + 7) / 8);
+  // 1024 workgroups, four a compute unit, but slices of 256 tokens and more (us at 4096 tokens x 4 heads of 128 in 8, 16, 32
+  // slices 31.0, 28.5, 29.5; 6732 x 8 of 256 in 1, 2, 4: 346, 303, 295)
+  const long long tiles = 4 * NH * up * up, want = std::max(1ll, std::min(1024 / tiles, (M + 255) / 256));
+  s.slice_tokens = (int)(((M + want - 1) / want + kProductK - 1) / kProductK * kProductK);
+  s.slices = (int)((M + s.slice_tokens - 1) / s.slice_tokens);
+  s.gate_floats = s.slices > 1 ? (size_t)s.slices * 4 * D * dh : 0;
+  s.conv_floats = (size_t)s.conv_blocks * D * (K + 1);
+  return s;
+}
+LayerConvParams layer_conv_params(const xs_layer_args *a) {
+  LayerConvParams p{};
+  p.B = a->B; p.T = a->T; p.D = a->NH * a->dh;
+  p.x = a->x; p.x_sb = a->x_stride_b; p.x_st = a->x_stride_t;
+  p.state = a->conv_state; p.state_sb = a->conv_state_stride_b ? a->conv_state_stride_b : (long long)(a->K - 1) * p.D;
+  p.w = a->conv_w; p.bias = a->conv_b;
+  p.reset = a->reset; p.reset_sb = a->reset_stride_b;
+  return p;
+}
+LayerProductParams layer_product_params(const xs_layer_args *a) {
+  LayerProductParams p{};
+  const long long D = (long long)a->NH * a->dh;
+  p.a[0] = a->x_conv; p.a_sb[0] = a->T * D; p.a_st[0] = D;
+  p.a[1] = a->x; p.a_sb[1] = a->x_stride_b; p.a_st[1] = a->x_stride_t;
+  for (int g = 0; g < 4; ++g) { p.w[g] = a->gate_w[g]; p.d_w[g] = a->d_gate_w[g]; }
+  p.wx = a->wx; p.d_wx = a->d_wx; p.d_a[0] = a->d_x_conv; p.d_a[1] = a->d_x;
+  p.M = a->B * a->T; p.T = a->T; p.NH = a->NH; p.dh = a->dh;
+  p.m_tiles = (p.M + 63) / 64; p.slices = 1; p.slice_tokens = p.M;
+  return p;
+}
+template <LayerProduct MODE>
+int launch_layer_product(LayerProductParams p, hipStream_t stream) {
+  const int up = (p.dh + 63) / 64;
+  p.tiles = MODE == LayerProduct::WEIGHTS ? 4 * up * up : (MODE == LayerProduct::INPUTS ? 2 : 4) * up;
+  const long long pairs = (long long)p.NH * (MODE == LayerProduct::WEIGHTS ? p.slices : p.m_tiles);
+  const long long grid = 8 * ((pairs + 7) / 8) * p.tiles;
+  if (grid > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many tiles for one launch");
+  p.pairs = (int)pairs; p.pairs_per_xcd = (int)((pairs + 7) / 8);
+  hipLaunchKernelGGL(layer_product_f32_kernel<MODE>, dim3((unsigned)grid), dim3(256), 0, stream, p);
+  return layer_launched("projection kernel");
+}
+
+int layer_front_check(const xs_layer_args *a) {
+  const long long D = (long long)a->NH * a->dh;
+  if (a->K < 2 || a->K > 4) return fail(XS_ERR_UNSUPPORTED, "convolution of %d taps not supported (2..4)", a->K);
+  if (!a->x || !a->conv_w || !a->gate_w[0] || !a->gate_w[1] || !a->gate_w[2] || !a->gate_w[3] || !a->x_conv)
+    return fail(XS_ERR_NULL, "x, the weights and x_conv are required");
+  if (a->x_stride_t < D || (a->B > 1 && a->x_stride_b < D)) return fail(XS_ERR_SHAPE, "x strides overlap the innermost D elements");
+  if (a->x_stride_b % 4 || a->x_stride_t % 4 || layer_misaligned({a->x, a->conv_w, a->conv_b, a->gate_w[0], a->gate_w[1], a->gate_w[2], a->gate_w[3], a->x_conv}))
+    return fail(XS_ERR_ALIGN, "x, its strides, the weights and x_conv must be 16-byte aligned");
+  return XS_OK;
+}
+
+int run_layer_front(const xs_layer_args *a) {
+  int rc = layer_check(a);
+  if (rc != XS_OK || a->B == 0 || a->T == 0) return rc;
+  if ((rc = layer_front_check(a)) != XS_OK) return rc;
+  const long long D = (long long)a->NH * a->dh;
+  if (!a->wx) return fail(XS_ERR_NULL, "wx is required");
+  if (a->conv_state && a->conv_state_stride_b && (a->conv_state_stride_b < (a->K - 1) * D || a->conv_state_stride_b % 4))
+    return fail(XS_ERR_SHAPE, "conv_state row stride %lld too small or not 16-byte aligned", (long long)a->conv_state_stride_b);
+  if (layer_misaligned({a->conv_state, a->wx})) return fail(XS_ERR_ALIGN, "conv_state and wx must be 16-byte aligned");
+  LayerConvParams c = layer_conv_params(a);
+  c.out = a->x_conv;
+  const long long threads = (long long)a->B * ((a->T + kConvRun - 1) / kConvRun) * (D / 4), blocks = (threads + 255) / 256;
+  if (blocks > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many tokens for one launch");
+  void (*kern)(LayerConvParams) = a->K == 2 ? layer_conv_f32_kernel<2> : (a->K == 3 ? layer_conv_f32_kernel<3> : layer_conv_f32_kernel<4>);
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)a->stream, c);
+  if ((rc = layer_launched("convolution kernel")) != XS_OK) return rc;
+  return launch_layer_product<LayerProduct::PROJECT>(layer_product_params(a), (hipStream_t)a->stream);
+}
+
+template <int L, int P>
+void launch_layer_norm(const LayerNormParams &p, hipStream_t stream) {
+  const long long groups = (long long)p.B * p.T * p.NH;
+  hipLaunchKernelGGL((layer_norm_f32_kernel<L, P>), dim3((unsigned)((groups + 256 / L - 1) / (256 / L))), dim3(256), 0, stream, p);
+}
+int run_layer_norm(const xs_layer_args *a) {
+  const int rc = layer_check(a);
+  if (rc != XS_OK || a->B == 0 || a->T == 0) return rc;
+  if (!a->h || !a->out) return fail(XS_ERR_NULL, "h and out are required");
+  if (layer_misaligned({a->h, a->norm_w, a->out})) return fail(XS_ERR_ALIGN, "h, norm_w and out must be 16-byte aligned");
+  if ((long long)a->B * a->T * a->NH > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many tokens for one launch");
+  LayerNormParams p{};
+  p.y = a->h; p.weight = a->norm_w; p.out = a->out; p.eps = a->eps;
+  p.B = a->B; p.T = a->T; p.NH = a->NH; p.dh = a->dh;
+  hipStream_t stream = (hipStream_t)a->stream;
+  if (a->dh <= 64) launch_layer_norm<16, 1>(p, stream);
+  else if (a->dh <= 128) launch_layer_norm<32, 1>(p, stream);
+  else if (a->dh <= 256) launch_layer_norm<64, 1>(p, stream);
+  else launch_layer_norm<64, 2>(p, stream);
+  return layer_launched("group norm kernel");
+}
+
+int run_layer_front_backward(const xs_layer_args *a) {
+  int rc = layer_check(a);
+  if (rc != XS_OK || a->B == 0 || a->T == 0) return rc;
+  if ((rc = layer_front_check(a)) != XS_OK) return rc;
+  if (!a->d_wx || !a->d_x_conv || !a->d_x || !a->scratch || !a->d_conv_w || (a->conv_b && !a->d_conv_b) ||
+      !a->d_gate_w[0] || !a->d_gate_w[1] || !a->d_gate_w[2] || !a->d_gate_w[3])
+    return fail(XS_ERR_NULL, "d_wx, d_x_conv, d_x, scratch and the gradients of the parameters are required");
+  if (a->conv_state) return fail(XS_ERR_UNSUPPORTED, "no gradient through a convolution that continues from a state");
+  if (layer_misaligned({a->d_wx, a->d_x_conv, a->d_x, a->scratch, a->d_gate_w[0], a->d_gate_w[1], a->d_gate_w[2], a->d_gate_w[3]}))
+    return fail(XS_ERR_ALIGN, "d_wx, d_x_conv, d_x, scratch and d_gate_w must be 16-byte aligned");
+  const LayerSplit split = layer_split(a->B, a->T, a->NH, a->dh, a->K);
+  hipStream_t stream = (hipStream_t)a->stream;
+  const long long D = (long long)a->NH * a->dh;
+  LayerProductParams g = layer_product_params(a);
+  if ((rc = launch_layer_product<LayerProduct::INPUTS>(g, stream)) != XS_OK) return rc;
+  g.slices = split.slices; g.slice_tokens = split.slice_tokens; g.partial = a->scratch;
+  if ((rc = launch_layer_product<LayerProduct::WEIGHTS>(g, stream)) != XS_OK) return rc;
+  LayerConvParams c = layer_conv_params(a);
+  c.state = nullptr;
+  c.d_out = a->d_x_conv; c.d_x = a->d_x; c.partial = a->scratch + split.gate_floats;
+  const int piece_blocks = (int)((D / 4 + 31) / 32);
+  if ((long long)piece_blocks * split.conv_blocks > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many tokens for one launch");
+  void (*kern)(LayerConvParams, int) = a->K == 2 ? layer_conv_backward_f32_kernel<2> : (a->K == 3 ? layer_conv_backward_f32_kernel<3> : layer_conv_backward_f32_kernel<4>);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(piece_blocks * split.conv_blocks)), dim3(256), 0, stream, c, piece_blocks);
+  if ((rc = layer_launched("convolution gradient kernel")) != XS_OK) return rc;
+  LayerReduceParams r{};
+  auto region = [](const float *partial, long long n, int parts) { return LayerReduceParams::Region{partial, n, parts, (int)((n + 63) / 64)}; };
+  r.region[0] = region(a->scratch, split.slices > 1 ? 4 * D * a->dh : 0, split.slices);
+  r.region[1] = region(c.partial, D * (a->K + 1), split.conv_blocks);
+  for (int i = 0; i < 4; ++i) r.d_w[i] = a->d_gate_w[i];
+  r.d_conv_w = a->d_conv_w; r.d_conv_b = a->conv_b ? a->d_conv_b : nullptr;
+  r.per_gate = D * a->dh; r.taps = a->K;
+  hipLaunchKernelGGL(layer_reduce_kernel, dim3((unsigned)(r.region[0].blocks + r.region[1].blocks)), dim3(256), 0, stream, r);
+  return layer_launched("sum kernel");
+}
+
 // ---- measurement: one stage of the dependency chain of a timestep, alone (slstm_serial_bound.h)
 int run_stage(const xs_measure_args *a) {
   if (!a) return fail(XS_ERR_NULL, "args is NULL");
@@ -1476,6 +1631,27 @@ int xs_headwise_gates(const xs_gates_args *args) {
 int xs_headwise_group_norm(const xs_norm_args *args) {
   g_err[0] = 0;
   return run_group_norm(args);
+}
+
+int xs_layer_front(const xs_layer_args *args) {
+  g_err[0] = 0;
+  return run_layer_front(args);
+}
+
+int xs_layer_norm(const xs_layer_args *args) {
+  g_err[0] = 0;
+  return run_layer_norm(args);
+}
+
+size_t xs_layer_scratch_floats(int32_t B, int32_t T, int32_t NH, int32_t dh, int32_t K) {
+  if (B <= 0 || T <= 0 || NH <= 0 || dh <= 0 || K <= 0) return 0;
+  const LayerSplit s = layer_split(B, T, NH, dh, K);
+  return s.gate_floats + s.conv_floats;
+}
+
+int xs_layer_front_backward(const xs_layer_args *args) {
+  g_err[0] = 0;
+  return run_layer_front_backward(args);
 }
 
 }  // extern "C"

@@ -13,7 +13,9 @@ external views, ``cell.reference_state_dict_to_hip``).
 For bfloat16 inputs with a head dim that is a multiple of 64 the ops in front of the cell run
 as two HIP kernels of the engine (convolution + SiLU; the four projections written straight into the
 cell's input), see ``functional.causal_conv_silu`` / ``functional.headwise_gates``, and so does the
-group norm behind it (``functional.headwise_group_norm``); otherwise they are PyTorch-ROCm ops.
+group norm behind it (``functional.headwise_group_norm``).  A float32 layer of the modules below runs on
+kernels of the engine around the cell as well; in its training calls everything up to the cell's output is
+one node of the autograd graph.  Otherwise they are PyTorch-ROCm ops.
 New: ``reset_mask[B,S]`` (document starts of packed rows) reaches the cell, and
 the causal convolution does not look across a document start either.
 """
@@ -26,6 +28,7 @@ from typing import Optional
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.nn.modules import module as torch_module
 
 from . import functional as hipF
 from .cell import sLSTMCell, sLSTMCell_hip, sLSTMCellConfig
@@ -135,7 +138,10 @@ class LinearHeadwiseExpand(nn.Module):
 
 
 class MultiHeadLayerNorm(nn.Module):
-    """Per-head group norm of [B,NH,S,DH] with residual weight (components/ln.py:8-68)."""
+    """Per-head group norm of [B,NH,S,DH] with residual weight (components/ln.py:8-68).  Its gradients are PyTorch's.
+    Measured with PyTorch 2.10 on ROCm 7: beyond 128 tokens (B*S) the gradient of the WEIGHT that ``F.group_norm`` hands back
+    on the GPU is off by its own size (relative 2-norm error 0.9 to 1.05 against float64 on the CPU; up to 128 tokens
+    2e-7; the gradient of the input is right throughout)."""
 
     def __init__(self, ndim: int, weight: bool = True, eps: float = 1e-5):
         super().__init__()
@@ -151,6 +157,24 @@ class MultiHeadLayerNorm(nn.Module):
         return out.view(B, S, NH, DH).transpose(1, 2)
 
 
+class _UpToTheCell(nn.Module):
+    """A layer's modules up to the cell, one by one, for calls with other tensors in place of its parameters
+    (``torch.func.functional_call``)."""
+
+    def __init__(self, layer: "sLSTMLayer"):
+        super().__init__()
+        self.layer = layer
+
+    def forward(self, x, slstm_state, reset_mask):
+        x_conv = self.layer.conv_act_fn(self.layer.conv1d(x, reset_mask=reset_mask))
+        return self.layer._cell_output(x, x_conv, slstm_state, reset_mask)
+
+
+# the modules that the float32 path of a layer stands in for, and their methods
+_PLAIN = {"conv1d": CausalConv1d, "fgate": LinearHeadwiseExpand, "igate": LinearHeadwiseExpand, "zgate": LinearHeadwiseExpand,
+          "ogate": LinearHeadwiseExpand, "conv_act_fn": nn.SiLU}
+_PLAIN_NORM = {"group_norm": MultiHeadLayerNorm}  # (inference)
+_PLAIN_FORWARD = {cls: cls.forward for cls in (*_PLAIN.values(), MultiHeadLayerNorm, nn.Conv1d)}
 # the methods that the native host path of a layer stands in for
 _CELL_FORWARD, _CELL_STEP, _DROPOUT_FORWARD = sLSTMCell_hip.forward, sLSTMCell_hip.step, nn.Dropout.forward
 
@@ -210,6 +234,44 @@ class sLSTMLayer(nn.Module):
                 and sLSTMCell_hip.forward is _CELL_FORWARD and sLSTMCell_hip.step is _CELL_STEP
                 and nn.Dropout.forward is _DROPOUT_FORWARD)
 
+    def _plain_modules(self, train: bool) -> bool:
+        """Whether the modules in front of the cell (inference: and the norm behind it) are what the constructor made, with
+        nothing that wants them called one by one (hooks, replaced methods).  Looked at for float32, whose path covers
+        training."""
+        modules = self._modules
+        found = [(modules.get(name), cls) for names in ((_PLAIN,) if train else (_PLAIN, _PLAIN_NORM)) for name, cls in names.items()]
+        if any(type(m) is not cls for m, cls in found):
+            return False
+        conv = modules["conv1d"]._modules.get("conv")
+        if (type(conv) is not nn.Conv1d or conv.stride != (1,) or conv.dilation != (1,) or conv.padding != (modules["conv1d"].pad,)
+                or conv.padding_mode != "zeros" or conv.groups != self.config.embedding_dim
+                or conv.kernel_size != (modules["conv1d"].pad + 1,) or torch_module._global_backward_hooks
+                or torch_module._global_backward_pre_hooks or torch.jit.is_tracing()):
+            return False
+        for m, cls in (*found, (conv, nn.Conv1d)):
+            if ("forward" in m.__dict__ or "_compiled_call_impl" in m.__dict__ or cls.forward is not _PLAIN_FORWARD[cls]
+                    or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks):
+                return False
+        cell = modules["slstm_cell"]
+        return not (cell._backward_hooks or cell._backward_pre_hooks)
+
+    def _cell_output(self, x, x_conv, slstm_state, reset_mask):
+        return self.slstm_cell(self._gates(x, x_conv), state=slstm_state, reset_mask=reset_mask)
+
+    def _gradients_with_graph(self, inputs, reset_mask, d_y, d_state):
+        """The gradients of a training call for a backward pass that is itself recorded: its operations once more with the
+        call's own tensors (x, convolution weight and bias, the gates', R, b, state), one by one."""
+        x, state = inputs[0], inputs[-1]
+        names = ("conv1d.conv.weight", "conv1d.conv.bias", "fgate.weight", "igate.weight", "zgate.weight", "ogate.weight",
+                 "slstm_cell._recurrent_kernel_", "slstm_cell._bias_")
+        params = {"layer." + n: t for n, t in zip(names, inputs[1:-1]) if t is not None}
+        with torch.enable_grad():
+            y, new_state = torch.func.functional_call(_UpToTheCell(self), params, (x, state, reset_mask))
+            pairs = [(o, g) for o, g in ((y, d_y), (new_state, d_state)) if g is not None]
+            wanted = [t for t in inputs if t is not None and t.requires_grad]
+            grads = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs], create_graph=True, allow_unused=True))
+        return tuple(next(grads) if t is not None and t.requires_grad else None for t in inputs)
+
     def _engine_ops_allowed(self, t) -> bool:
         # the engine's kernels record no autograd graph: under grad mode the PyTorch ops run, and a backward pass
         # reaches the cell, which raises (inference engine)
@@ -226,10 +288,21 @@ class sLSTMLayer(nn.Module):
         if x.is_cuda and self._own_modules():
             cell = self.slstm_cell
             native = cell._native()
-            fast = hipF._lib.host().layer_forward(self, native, x, conv_state, slstm_state, return_last_state, reset_mask)
-            if fast is not None:
-                cell._rt.last_workspace = native
-                return fast
+            if x.dtype != torch.float32 or self._plain_modules(train=False):
+                fast = hipF._lib.host().layer_forward(self, native, x, conv_state, slstm_state, return_last_state, reset_mask)
+                if fast is not None:
+                    cell._rt.last_workspace = native
+                    return fast
+            if (x.dtype == torch.float32 and conv_state is None and torch.is_grad_enabled() and cell.keep_backward_coefficients
+                    and 36 * x.numel() <= hipF.KEPT_COEFFICIENT_BYTES and self._plain_modules(train=True)):
+                fast = hipF._lib.host().layer_train(self, native, x, slstm_state, reset_mask, hipF.KEPT_COEFFICIENT_BYTES_PER_DEVICE)
+                if fast is not None:
+                    cell._rt.last_workspace = native
+                    y, slstm_state = fast
+                    out = self._norm(self.dropout(y), x.shape[0], x.shape[1])
+                    if return_last_state:
+                        return out, {"conv_state": x[:, -self.conv1d.pad:], "slstm_state": slstm_state}
+                    return out
         B, S, _ = x.shape
         if isinstance(conv_state, (tuple, list)):  # the ring a step returned (conv.py:131-157): oldest input first
             conv_state = conv_state[0]
@@ -251,7 +324,7 @@ class sLSTMLayer(nn.Module):
             x_conv = self.conv_act_fn(x_conv)
         else:
             x_conv = x
-        y, slstm_state = self.slstm_cell(self._gates(x, x_conv), state=slstm_state, reset_mask=reset_mask)
+        y, slstm_state = self._cell_output(x, x_conv, slstm_state, reset_mask)
         out = self._norm(self.dropout(y), B, S)
         if return_last_state:
             return out, {"conv_state": conv_state, "slstm_state": slstm_state}
