@@ -20,7 +20,7 @@
 extern "C" {
 #endif
 
-#define XS_ABI_VERSION 18
+#define XS_ABI_VERSION 19
 
 /* element types */
 enum { XS_F32 = 0, XS_BF16 = 1 };
@@ -287,6 +287,29 @@ typedef struct xs_norm_args {
 } xs_norm_args;
 
 int xs_headwise_group_norm(const xs_norm_args *args);
+
+/*
+ * xs_layer_step: one decoded token of a bf16 layer (xlstm/blocks/slstm/layer.py:92-121) up to its hidden state in ONE kernel -
+ * convolution + SiLU with the ring of the next step, the four projections, the cell's step - with the results, bit for bit,
+ * of xs_causal_conv_silu, xs_headwise_gates and xs_slstm_step called one behind the other.  XS_ERR_UNSUPPORTED, with nothing launched,
+ * where xs_layer_step_fits() is 0: those three are the faster way there.
+ *   cell         as for xs_slstm_step with bf16 wx and r, a state (s0) and no mask; wx and its strides are not read
+ *   x            [B,D] contiguous, not overlapping ring_out;  conv_state, conv_w, conv_b, ring_out (required) as for
+ *                xs_causal_conv_silu, K = 4;  gate_w as for xs_headwise_gates
+ */
+typedef struct xs_layer_step_args {
+  xs_slstm_args cell;
+  const void *x;
+  const void *conv_state;
+  int64_t conv_state_stride_b;
+  const void *conv_w, *conv_b;
+  void *ring_out;
+  const void *gate_w[4];
+  int32_t K;
+} xs_layer_step_args;
+
+int xs_layer_step_fits(int32_t B, int32_t NH, int32_t dh, int32_t K);
+int xs_layer_step(const xs_layer_step_args *args);
 
 /*
  * The operations around the cell of a FLOAT32 layer, forward and backward (same formulas as above; everything held and

@@ -17,7 +17,7 @@ LIB_PATH = os.environ.get("XLSTM_AMD_LIB", os.path.join(PKG, "lib", "libxlstm_am
 XS_F32, XS_BF16 = 0, 1
 XS_ERR_UNSUPPORTED = -5
 STATIC_SCRATCH_BYTES = (4 << 20) + (64 << 10)
-ABI_VERSION = 18
+ABI_VERSION = 19
 
 EXPORTS = (
     "xs_abi_version",
@@ -35,6 +35,8 @@ EXPORTS = (
     "xs_causal_conv_silu",
     "xs_headwise_gates",
     "xs_headwise_group_norm",
+    "xs_layer_step_fits",
+    "xs_layer_step",
     "xs_layer_front",
     "xs_layer_norm",
     "xs_layer_scratch_floats",
@@ -159,6 +161,22 @@ class NormArgs(ctypes.Structure):
     ]
 
 
+class LayerStepArgs(ctypes.Structure):
+    """Mirror of ``xs_layer_step_args``."""
+
+    _fields_ = [
+        ("cell", SlstmArgs),
+        ("x", ctypes.c_void_p),
+        ("conv_state", ctypes.c_void_p),
+        ("conv_state_stride_b", ctypes.c_int64),
+        ("conv_w", ctypes.c_void_p),
+        ("conv_b", ctypes.c_void_p),
+        ("ring_out", ctypes.c_void_p),
+        ("gate_w", ctypes.c_void_p * 4),
+        ("K", ctypes.c_int32),
+    ]
+
+
 class LayerArgs(ctypes.Structure):
     """Mirror of ``xs_layer_args``."""
 
@@ -258,6 +276,10 @@ def load() -> ctypes.CDLL:
     for fn in (lib.xs_layer_front, lib.xs_layer_norm, lib.xs_layer_front_backward):
         fn.restype = ctypes.c_int
         fn.argtypes = [ctypes.POINTER(LayerArgs)]
+    lib.xs_layer_step_fits.restype = ctypes.c_int
+    lib.xs_layer_step_fits.argtypes = [ctypes.c_int32] * 4
+    lib.xs_layer_step.restype = ctypes.c_int
+    lib.xs_layer_step.argtypes = [ctypes.POINTER(LayerStepArgs)]
     lib.xs_layer_scratch_floats.restype = ctypes.c_size_t
     lib.xs_layer_scratch_floats.argtypes = [ctypes.c_int32] * 5
     lib.xs_slstm_train_coef_floats.restype = ctypes.c_size_t
@@ -301,7 +323,8 @@ def host():
     spec.loader.exec_module(mod)
     names = ("xs_slstm_step", "xs_slstm_forward_watched", "xs_slstm_workspace_bytes", "xs_last_error", "xs_causal_conv_silu",
              "xs_headwise_gates", "xs_headwise_group_norm", "xs_slstm_train_coef_floats", "xs_slstm_train_exchange_bytes",
-             "xs_slstm_train_forward", "xs_slstm_train_backward", "xs_slstm_backward_params", "xs_layer_front", "xs_layer_norm",
+             "xs_slstm_train_forward", "xs_slstm_train_backward", "xs_slstm_backward_params", "xs_layer_step_fits", "xs_layer_step",
+             "xs_layer_front", "xs_layer_norm",
              "xs_layer_scratch_floats", "xs_layer_front_backward")
     mod.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names}, EngineError,
              torch_module._global_forward_hooks, torch_module._global_forward_pre_hooks)

@@ -50,10 +50,13 @@ struct Engine {
   decltype(&xs_slstm_train_forward) train_forward = nullptr;
   decltype(&xs_slstm_train_backward) train_backward = nullptr;
   decltype(&xs_slstm_backward_params) backward_params = nullptr;
+  decltype(&xs_layer_step_fits) layer_step_fits = nullptr;
+  decltype(&xs_layer_step) layer_step = nullptr;
   decltype(&xs_layer_front) layer_front = nullptr;
   decltype(&xs_layer_norm) layer_norm = nullptr;
   decltype(&xs_layer_scratch_floats) layer_scratch = nullptr;
   decltype(&xs_layer_front_backward) layer_front_backward = nullptr;
+  bool own_parts = true;                  // the parts of a layer's step are the engine's own: one kernel may stand for them
   PyObject *error = nullptr;              // functional.EngineError
   PyObject *global_hooks[2] = {nullptr, nullptr};  // hooks on every module of the process
 } g_engine;
@@ -355,9 +358,15 @@ struct Step {
   }
   // wx: contiguous [B,1,4H]; everything else as step_fits has found it
   void run(const at::Tensor &wx, const at::Tensor &s0, const StepBuffers &s, const Shape4 *h_shape) {
+    fill(wx.options(), s0, s, h_shape);
+    a.wx = wx.data_ptr();
+    launched(g_engine.step(&a));
+  }
+  // the argument block but for wx
+  void fill(const at::TensorOptions &opts, const at::Tensor &s0, const StepBuffers &s, const Shape4 *h_shape) {
     if (s.h_out) h = *s.h_out;
-    else if (h_shape) h = at::empty_strided(at::IntArrayRef(h_shape->size.data(), h_shape->n), at::IntArrayRef(h_shape->stride.data(), h_shape->n), wx.options());
-    else h = at::empty({1, B, H}, wx.options());
+    else if (h_shape) h = at::empty_strided(at::IntArrayRef(h_shape->size.data(), h_shape->n), at::IntArrayRef(h_shape->stride.data(), h_shape->n), opts);
+    else h = at::empty({1, B, H}, opts);
     state = s.state_out ? *s.state_out : at::empty({4, B, H}, s0.options());
     a.h_prev = nullptr;
     if (dtype == at::kBFloat16) {
@@ -370,12 +379,10 @@ struct Step {
         a.h_prev = last_h.data_ptr();
       }
     }
-    a.wx = wx.data_ptr();
     a.s0 = (const float *)s0.data_ptr();
     a.s_out = (float *)state.data_ptr();
     a.h_out = h.data_ptr();
     a.stream = stream_of(device);
-    launched(g_engine.step(&a));
   }
   void leave(bool keep_state) {
     if (c.plan == plan.o) *c.step_args = a;  // (the plan's block describes its last step)
@@ -975,6 +982,11 @@ bool taps_of(const LayerParts &p, const at::Tensor &t, int64_t B, const void *&t
   return true;
 }
 
+bool overlap(const at::Tensor &a, const at::Tensor &b) {  // contiguous tensors
+  const char *pa = (const char *)a.data_ptr(), *pb = (const char *)b.data_ptr();
+  return pa < pb + b.nbytes() && pb < pa + a.nbytes();
+}
+
 PyObject *states_dict(PyObject *conv_state, const at::Tensor &state) {
   PyRef s(THPVariable_Wrap(state)), d(PyDict_New());
   if (!s.o || !d.o || !conv_state || PyDict_SetItem(d.o, g_names.conv_state, conv_state) || PyDict_SetItem(d.o, g_names.slstm_state, s.o)) throw PythonError{};
@@ -1021,11 +1033,23 @@ PyObject *layer_step_(PyObject *const *args) {
     WithoutGil no_gil;
     void *stream = stream_of(x.device());
     ring = ring_out ? *ring_out : at::empty({B, p.K, p.D}, opts);
-    at::Tensor wx = at::empty({B, 1, 4 * p.D}, opts), x_conv = at::empty({B, 1, p.D}, opts);
-    run_conv(p, x, taps, taps_stride, nullptr, x_conv.data_ptr(), ring.data_ptr(), stream);
-    run_gates(p, x, x_conv.data_ptr(), wx.data_ptr(), stream);
-    step.run(wx, state, buffers, nullptr);
     out = out_given ? *out_given : at::empty({B, 1, p.D}, opts);
+    if (g_engine.own_parts && g_engine.layer_step_fits((int32_t)B, (int32_t)p.NH, (int32_t)p.dh, (int32_t)p.K) && !overlap(x, ring)) {
+      step.fill(opts, state, buffers, nullptr);
+      xs_layer_step_args a{};
+      a.cell = step.a;
+      a.x = x.data_ptr();
+      a.conv_state = taps; a.conv_state_stride_b = taps && B > 1 ? taps_stride : 0;
+      a.conv_w = p.conv_w.data_ptr(); a.conv_b = p.conv_b.defined() ? p.conv_b.data_ptr() : nullptr;
+      a.ring_out = ring.data_ptr(); a.K = (int32_t)p.K;
+      for (int g = 0; g < 4; ++g) a.gate_w[g] = p.gate[g].data_ptr();
+      launched(g_engine.layer_step(&a));
+    } else {
+      at::Tensor wx = at::empty({B, 1, 4 * p.D}, opts), x_conv = at::empty({B, 1, p.D}, opts);
+      run_conv(p, x, taps, taps_stride, nullptr, x_conv.data_ptr(), ring.data_ptr(), stream);
+      run_gates(p, x, x_conv.data_ptr(), wx.data_ptr(), stream);
+      step.run(wx, state, buffers, nullptr);
+    }
     run_norm(p, step.h, B, 1, out.data_ptr(), stream);
     state_out = p.keep_state ? step.state : step.state.to(at::kBFloat16);
   }
@@ -1334,11 +1358,15 @@ PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
       !get("xs_slstm_train_coef_floats", g_engine.coef_floats) || !get("xs_slstm_train_exchange_bytes", g_engine.exchange_bytes) ||
       !get("xs_slstm_train_forward", g_engine.train_forward) || !get("xs_slstm_train_backward", g_engine.train_backward) ||
       !get("xs_slstm_backward_params", g_engine.backward_params) || !get("xs_layer_front", g_engine.layer_front) ||
+      !get("xs_layer_step_fits", g_engine.layer_step_fits) || !get("xs_layer_step", g_engine.layer_step) ||
       !get("xs_layer_norm", g_engine.layer_norm) || !get("xs_layer_scratch_floats", g_engine.layer_scratch) ||
       !get("xs_layer_front_backward", g_engine.layer_front_backward)) {
     PyErr_SetString(PyExc_KeyError, "an entry point of the engine is missing");
     return nullptr;
   }
+  // (whoever binds other entry points for the parts of a layer's step, to watch them or to stand in for them, has them called)
+  static const Engine first = g_engine;
+  g_engine.own_parts = g_engine.step == first.step && g_engine.conv == first.conv && g_engine.gates == first.gates;
   for (int i = 1; i < 4; ++i) Py_INCREF(args[i]);
   g_engine.error = args[1];
   for (int i = 0; i < 2; ++i) g_engine.global_hooks[i] = PyDict_Check(args[2 + i]) ? args[2 + i] : nullptr;

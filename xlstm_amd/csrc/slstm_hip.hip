@@ -24,6 +24,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <initializer_list>
 #include <mutex>
 
@@ -35,6 +36,7 @@
 #include "slstm_step_kernel.h"
 #include "slstm_step_pipe_kernel.h"
 #include "slstm_step_small_kernel.h"
+#include "slstm_layer_step_kernel.h"
 #include "slstm_backward_kernels.h"
 #include "slstm_layer_kernels.h"
 #include "slstm_layer_f32_kernels.h"
@@ -178,12 +180,14 @@ int validate(const xs_slstm_args *a, bool step, bool own_scratch = false) {
   return XS_OK;
 }
 
-// compute units of the current device (an attribute query: no device synchronisation, cheap per call)
+// compute units of the current device (asked for once: a decoded token looks at it several times)
 int device_cus() {
+  static std::atomic<int> known[64];  // (0: not asked yet)
   int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return -1;
+  if (hipGetDevice(&dev) != hipSuccess) return -1;
+  if (dev >= 0 && dev < 64 && (cus = known[dev].load(std::memory_order_relaxed)) > 0) return cus;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return -1;
+  if (dev >= 0 && dev < 64) known[dev].store(cus, std::memory_order_relaxed);
   return cus;
 }
 
@@ -205,6 +209,22 @@ int ensure_dynamic_lds(const void *kernel, size_t bytes) {
   return XS_OK;
 }
 
+StepParams step_params(const xs_slstm_args *a) {
+  StepParams p;
+  p.wx = a->wx; p.wx_sb = a->wx_stride_b;
+  p.r = a->r; p.r_bf16 = a->r_dtype == XS_BF16;
+  p.bias = a->bias; p.s0 = a->s0;
+  p.reset = a->reset; p.reset_sb = a->reset_stride_b;
+  p.h_out = a->h_out; p.s_out = a->s_out;
+  p.status = (xs_slstm_status *)a->workspace;
+  p.B = a->B; p.NH = a->NH; p.dh = a->dh;
+  p.n_unit_tiles = (a->dh + 31) / 32;
+  p.n_row_tiles = (a->B + 63) / 64;
+  p.h_prev = nullptr;
+  p.spin_limit = a->spin_limit > 0 ? (a->spin_limit < (1ll << 30) ? (int)a->spin_limit : (1 << 30)) : (1 << 22);
+  return p;
+}
+
 int run_step(const xs_slstm_args *a) {
   hipStream_t stream = (hipStream_t)a->stream;
   const int B = a->B, NH = a->NH, dh = a->dh;
@@ -215,17 +235,7 @@ int run_step(const xs_slstm_args *a) {
   while (nch * 16 * epc < dh) nch *= 2;  // the sequence kernel's K quarters are nch slabs wide
   if (nch > 8) return fail(XS_ERR_UNSUPPORTED, "head dim %d too large for %s operands (max %d)", dh, bf16 ? "bf16" : "fp32", 8 * 16 * epc);
   if ((long long)B * 4 * NH * dh * (bf16 ? 2 : 4) < 32) return fail(XS_ERR_SHAPE, "wx too small");
-  StepParams p;
-  p.wx = a->wx; p.wx_sb = a->wx_stride_b;
-  p.r = a->r; p.r_bf16 = a->r_dtype == XS_BF16;
-  p.bias = a->bias; p.s0 = a->s0;
-  p.reset = a->reset; p.reset_sb = a->reset_stride_b;
-  p.h_out = a->h_out; p.s_out = a->s_out;
-  p.status = (xs_slstm_status *)a->workspace;
-  p.B = B; p.NH = NH; p.dh = dh;
-  p.n_unit_tiles = (dh + 31) / 32;
-  p.n_row_tiles = (B + 63) / 64;
-  p.spin_limit = a->spin_limit > 0 ? (a->spin_limit < (1ll << 30) ? (int)a->spin_limit : (1 << 30)) : (1 << 22);
+  StepParams p = step_params(a);
   const long long nwg = (long long)NH * p.n_unit_tiles * p.n_row_tiles;
   if (nwg > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many tiles for one step launch");
   // Small batches: workgroups of 16 rows x 16 units (slstm_step_small_kernel.h), as long as there are at most so many of
@@ -1107,7 +1117,7 @@ int run_backward_params(const xs_slstm_bwd_args *a) {
   return XS_OK;
 }
 
-int run_conv(const xs_conv_args *a) {
+int check_conv(const xs_conv_args *a) {
   if (!a) return fail(XS_ERR_NULL, "args is NULL");
   if (a->B < 0 || a->T < 0 || a->D <= 0) return fail(XS_ERR_SHAPE, "bad dims B=%d T=%d D=%d", a->B, a->T, a->D);
   if (a->dtype != XS_BF16) return fail(XS_ERR_DTYPE, "xs_causal_conv_silu computes on bf16 tensors only");
@@ -1130,6 +1140,12 @@ int run_conv(const xs_conv_args *a) {
   if (((uintptr_t)a->x % 16) || ((a->x_stride_b * 2) % 16) || ((a->x_stride_t * 2) % 16) || ((uintptr_t)a->conv_state % 16) ||
       ((uintptr_t)a->weight % 16) || ((uintptr_t)a->bias % 16) || ((uintptr_t)a->out % 16))
     return fail(XS_ERR_ALIGN, "x and its strides, conv_state, weight, bias and out must be 16-byte aligned");
+  return XS_OK;
+}
+
+int run_conv(const xs_conv_args *a) {
+  const int rc = check_conv(a);
+  if (rc != XS_OK || a->B == 0 || a->T == 0) return rc;
   const long long threads = (long long)a->B * a->T * (a->D / 8);
   const long long blocks = ((threads + 255) / 256 + 7) / 8 * 8;  // a multiple of 8: the kernel deals them out by XCD
   if (blocks > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many tokens for one launch");
@@ -1183,7 +1199,7 @@ int launch_gates_tiles(const xs_gates_args *a, const GatesParams &p, hipStream_t
   return launch_gates<64, 64, 3>(a, p, stream);
 }
 
-int run_gates(const xs_gates_args *a) {
+int check_gates(const xs_gates_args *a) {
   if (!a) return fail(XS_ERR_NULL, "args is NULL");
   if (a->M < 0 || a->NH <= 0 || a->dh <= 0) return fail(XS_ERR_SHAPE, "bad dims M=%d NH=%d dh=%d", a->M, a->NH, a->dh);
   if (a->dtype != XS_BF16) return fail(XS_ERR_DTYPE, "xs_headwise_gates computes on bf16 tensors only");
@@ -1198,6 +1214,12 @@ int run_gates(const xs_gates_args *a) {
       ((a->x_conv_stride_row * 2) % 16) || ((a->out_stride_row * 2) % 16) || ((uintptr_t)a->w[0] % 16) ||
       ((uintptr_t)a->w[1] % 16) || ((uintptr_t)a->w[2] % 16) || ((uintptr_t)a->w[3] % 16))
     return fail(XS_ERR_ALIGN, "x, x_conv, out, their row strides and the weights must be 16-byte aligned");
+  return XS_OK;
+}
+
+int run_gates(const xs_gates_args *a) {
+  const int rc = check_gates(a);
+  if (rc != XS_OK || a->M == 0) return rc;
   GatesParams p;
   p.x = (const uint16_t *)a->x; p.xc = (const uint16_t *)a->x_conv;
   p.x_sr = a->x_stride_row; p.xc_sr = a->x_conv_stride_row;
@@ -1258,6 +1280,75 @@ int run_group_norm(const xs_norm_args *a) {
   hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)a->stream, p);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(XS_ERR_LAUNCH, "group norm kernel launch failed: %s", hipGetErrorString(e));
+  return XS_OK;
+}
+
+// ---- one decoded token of a layer up to its hidden state (slstm_layer_step_kernel.h)
+// How its kernel splits it; ut 0: not at all, the kernels of its parts are the faster way.
+// us a token with the group norm behind it, replayed from a graph, the parts' kernels -> this one.  One workgroup of 16 units
+// a compute unit: 4 heads of 64, 7 rows 11.9 -> 6.7, 4 of 256, 64 rows 14.5 -> 9.6, 4 of 512, 7 rows 16.0 -> 12.6.  Up to two, as one of
+// 32 units: 8 of 256, 64 rows 15.6 -> 11.0 (as two 13.0), 4 of 512, 64 rows 22.2 -> 17.4 (24.8).  Beyond, several row tiles
+// a workgroup of 32 units: 8 of 256, 128 rows 18.5 -> 14.3, 256 rows 23.0 -> 20.8, 16 of 256, 256 rows (16 a compute unit, each
+// as many again 5.6 us against 4.2) 34.4 -> 32.0.  Head dims beyond 256 have no registers for several row tiles, 1024 (its
+// whole head in a convolution, 32 products in one chain) gains nothing: 1 row 24.0 -> 24.0, 16 rows 26.0 -> 27.3.
+struct LayerStepSplit { int nch, ut, row_groups; bool loop; };
+LayerStepSplit layer_step_split(int B, int NH, int dh, int K) {
+  LayerStepSplit s{1, 0, (B + 15) / 16, false};
+  while (s.nch * 128 < dh) s.nch *= 2;
+  const long long cus = device_cus(), wgs = (long long)NH * (dh / 16) * s.row_groups;  // workgroups of 16 rows x 16 units
+  if (K != 4 || s.nch > 4 || cus <= 0 || wgs > (s.nch <= 2 ? 16 : 2) * cus) return s;
+  s.ut = wgs <= cus ? 1 : 2;
+  if (wgs > 2 * cus) {
+    s.loop = true;
+    s.row_groups = (int)std::min<long long>(s.row_groups, std::max(1ll, cus / ((long long)NH * (dh / 32))));
+  }
+  return s;
+}
+int run_layer_step(const xs_layer_step_args *a) {
+  if (!a) return fail(XS_ERR_NULL, "args is NULL");
+  xs_slstm_args cell = a->cell;
+  const int B = cell.B, NH = cell.NH, dh = cell.dh;
+  const long long D = (long long)NH * dh;
+  if (cell.wx_dtype != XS_BF16) return fail(XS_ERR_DTYPE, "xs_layer_step computes on bf16 tensors only");
+  if (NH <= 0 || dh <= 0 || dh % 64) return fail(XS_ERR_UNSUPPORTED, "head dim %d is not a multiple of 64", dh);
+  if (!cell.s0 || cell.reset) return fail(XS_ERR_UNSUPPORTED, "a layer's step goes with a state and without a mask");
+  if (B > 0 && (!a->x || !a->ring_out)) return fail(XS_ERR_NULL, "x and ring_out are required");
+  cell.wx = a->x; cell.wx_stride_b = cell.wx_stride_t = 4 * D;  // (not read)
+  int rc = validate(&cell, true);
+  if (rc != XS_OK || B == 0) return rc;
+  const LayerStepSplit split = layer_step_split(B, NH, dh, a->K);
+  if (!split.ut) return fail(XS_ERR_UNSUPPORTED, "xs_layer_step does not take %d rows of %d heads of %d with %d taps", B, NH, dh, a->K);
+  xs_conv_args conv{};
+  conv.B = B; conv.T = 1; conv.D = (int32_t)D; conv.K = a->K; conv.dtype = XS_BF16;
+  conv.x = a->x; conv.x_stride_b = conv.x_stride_t = D;
+  conv.conv_state = a->conv_state; conv.conv_state_stride_b = a->conv_state_stride_b;
+  conv.weight = a->conv_w; conv.bias = a->conv_b; conv.out = conv.ring_out = a->ring_out;
+  xs_gates_args gates{};
+  gates.M = B; gates.NH = NH; gates.dh = dh; gates.dtype = XS_BF16;
+  gates.x = gates.x_conv = a->x; gates.x_stride_row = gates.x_conv_stride_row = D;
+  for (int g = 0; g < 4; ++g) gates.w[g] = a->gate_w[g];
+  gates.out = a->ring_out; gates.out_stride_row = 4 * D;
+  if ((rc = check_conv(&conv)) != XS_OK || (rc = check_gates(&gates)) != XS_OK) return rc;
+  const uintptr_t x0 = (uintptr_t)a->x, r0 = (uintptr_t)a->ring_out, nx = (uintptr_t)B * D * 2;
+  if (x0 < r0 + 4 * nx && r0 < x0 + nx) return fail(XS_ERR_SHAPE, "ring_out must not overlap x");  // (other workgroups still read it)
+  LayerStepParams p;
+  p.step = step_params(&cell);
+  p.step.n_unit_tiles = dh / (16 * split.ut);
+  p.step.n_row_tiles = split.row_groups;
+  p.step.h_prev = cell.h_prev;
+  p.row_tiles = (B + 15) / 16;
+  p.x = (const uint16_t *)a->x;
+  p.state = (const uint16_t *)a->conv_state;
+  p.state_sb = a->conv_state_stride_b ? a->conv_state_stride_b : 3 * D;
+  p.conv_w = (const uint16_t *)a->conv_w; p.conv_b = (const uint16_t *)a->conv_b;
+  for (int g = 0; g < 4; ++g) p.gate_w[g] = (const uint16_t *)a->gate_w[g];
+  p.ring_out = (uint16_t *)a->ring_out;
+  const LayerStepKernel kern = cell.h_prev ? pick_layer_step<true>(split.nch, split.ut, split.loop) : pick_layer_step<false>(split.nch, split.ut, split.loop);
+  const size_t lds = (size_t)layer_step_lds_bytes(split.nch);
+  if (lds + 25600 * split.ut > 64 * 1024 && (rc = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds)) != XS_OK) return rc;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(NH * p.step.n_unit_tiles * p.step.n_row_tiles)), dim3(256 * split.ut), lds, (hipStream_t)cell.stream, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(XS_ERR_LAUNCH, "layer step kernel launch failed: %s", hipGetErrorString(e));
   return XS_OK;
 }
 
@@ -1641,6 +1732,15 @@ int xs_layer_front(const xs_layer_args *args) {
 int xs_layer_norm(const xs_layer_args *args) {
   g_err[0] = 0;
   return run_layer_norm(args);
+}
+
+int xs_layer_step_fits(int32_t B, int32_t NH, int32_t dh, int32_t K) {
+  return B > 0 && NH > 0 && dh > 0 && dh % 64 == 0 && layer_step_split(B, NH, dh, K).ut > 0;
+}
+
+int xs_layer_step(const xs_layer_step_args *args) {
+  g_err[0] = 0;
+  return run_layer_step(args);
 }
 
 size_t xs_layer_scratch_floats(int32_t B, int32_t T, int32_t NH, int32_t dh, int32_t K) {
