@@ -1,11 +1,15 @@
-"""Decode loop for one sLSTM layer replayed from HIP graphs.
+"""Decode loop for one sLSTM layer without allocations: kernels launched directly, or replayed from HIP graphs.
 
 The reference decodes by calling ``sLSTMLayer.step`` once per token from Python
 (``xlstm/blocks/slstm/layer.py:92-121`` via ``xlstm_block_stack.py:126-137``).  One such
 step is a dozen small launches, so the host sets the pace.  ``GraphedLayerDecoder`` captures
 the step twice - once reading state set 0 and writing set 1, once the other way round -
 and replays the two graphs alternately: no allocation, no state copy and no Python between
-the launches of a token.
+the launches of a token.  Where the layer's native host path takes the step, its two to four
+launches go out directly: launching a graph costs 15 us on the host, whatever it holds, and a
+token from elsewhere has to be copied to where the graph reads it (8 heads of 256, 256 rows:
+30.5 -> 20.8 us a token; 3 rows of 4 heads of 256: 25 -> 12).  The graphs serve what that path
+leaves to others (other types and head dims, parameters changed since, hooks, autocast).
 
 Only kernels are recorded (the engine's entry points enqueue nothing else); the state
 buffers are cleared with ``zero_()``, which is a fill kernel.
@@ -16,6 +20,7 @@ from typing import Optional
 
 import torch
 
+from . import _lib
 from .layer import sLSTMLayer
 
 
@@ -81,13 +86,33 @@ class GraphedLayerDecoder:
 
     def step(self, x: Optional[torch.Tensor] = None) -> torch.Tensor:
         """``x`` [B,1,D] -> the layer's output for this token (a buffer that the next call overwrites).
-        With ``x=None`` the token is taken from ``self.x``, where its producer has written it: one copy
-        kernel (and the gap in front of the graph) less per token."""
+        With ``x=None`` the token is taken from ``self.x``, where its producer has written it (from the graphs: one copy
+        kernel and the gap in front of the graph less per token)."""
+        if not torch.cuda.is_current_stream_capturing() and self._launch(self.x if x is None else x):
+            return self.out
         if x is not None and x.data_ptr() != self.x.data_ptr():
             self.x.copy_(x)
+            if not torch.cuda.is_current_stream_capturing() and self._launch(self.x):
+                return self.out
         self.graphs[self.cur].replay()
         self.cur ^= 1
         return self.out
+
+    def _launch(self, x: torch.Tensor) -> bool:
+        """The step through the layer's native host path, into the buffers that the graphs use; False where it does not
+        take it."""
+        layer, k = self.layer, self.cur
+        cell = layer.slstm_cell
+        if x.shape != self.x.shape or not layer._own_modules() or cell._rt.step_plan is None:
+            return False
+        with torch.no_grad():
+            done = _lib.host().layer_step(layer, cell._native(), x, self.conv[k], self.slstm[k], self.slstm[1 - k], self.conv[1 - k],
+                                          self.h[1 - k], self.h[k], self.out)
+        if done is None:
+            return False
+        cell._rt.last_workspace = cell._rt.step_plan[1].workspace
+        self.cur = 1 - k
+        return True
 
     def state(self):
         """Current state in the reference's per-block format (xlstm_block_stack.py:126-137)."""
