@@ -466,11 +466,16 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
   // waves 0-3, QUAD: row tiles of at most 4 rows.  With K split over the four waves (below), a step's chain runs
   // through LDS: partial tiles out, a barrier, sixteen partial values back in and added up, and only one of the four
   // waves gates real rows.  Here wave w owns units 4 w .. 4 w + 3 of the workgroup's 16 with all four gates (16
-  // columns) and the WHOLE of K: it polls the whole h tile of the group (4 rows x dh, 16 bytes per lane from the 16
-  // lanes whose MFMA row is a real one), multiplies, and gates its own 16 elements; nothing crosses between the waves.
-  // The batch rows sit at MFMA rows 0, 4, 8, 12, so the sum of (row b, column n) arrives in lane group b, lane n, and
+  // columns) and the WHOLE of K: it polls the whole h tile of the group (4 rows x dh), multiplies, and gates its own
+  // 16 elements; nothing crosses between the waves.  bf16: batch row b takes the four MFMA rows 4 b .. 4 b + 3, each with
+  // ANOTHER QUARTER of K, so that no lane of a poll is a row that is not there; a quarter's MFMAs make sums of all sixteen
+  // rows, of which the four that hold that quarter are the right ones: row 4 b + w of quarter w, which is register w of
+  // lane group b.  So the sum of (row b, column n) arrives in lane group b, lane n, and
   // the four gates of a unit meet in the unit's lane through three row shifts (no LDS).  K is accumulated in the same
-  // four quarters and folded in the same order as everywhere else: the same bits.  The barrier of the step (the
+  // four quarters and folded in the same order as everywhere else: the same bits.  A poll is 2 loads a wave at head dim 256;
+  // with the batch rows at MFMA rows 0, 4, 8, 12 and zeros between it was 8, three quarters of their lanes empty, and the
+  // loads of the four waves held each other up in the compute unit's one return path (us a call, before -> after: B 16 x T 2048 x 4 heads
+  // of 256 1527 -> 1464, a layer at B 7 x T 333 x 4 heads of 192 286 -> 257, B 1 x T 500 x 8 heads of 256 379 -> 310).  The barrier of the step (the
   // feeder's W.x, the drainer's h) is passed in front of the poll.  The exchange ring is [slot][member][4 rows]
   // [16 units]: the group's h of a step is 8 dh bytes (float32: 16 dh) in a row.
   // Without FULL the K range ends inside the four quarters: members past the last one lie past the end of the descriptor
@@ -565,17 +570,17 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
     lds_barrier();  // prologue barrier
     const bool cross = cross_s != 0u;
     constexpr int QTILE = 4 * 16 * ESZ;        // bytes a member publishes per step
-    constexpr int NP = BF16 ? NK : NCH;        // 16-byte pieces of the group's h a lane polls per step
+    constexpr int NP = NCH;                    // 16-byte pieces of the group's h a lane polls per step
     constexpr int PSTEP = BF16 ? 2 * QTILE : QTILE;  // ... and the distance between them
     const int xslot = p.G * QTILE;
     char *const xbase = reinterpret_cast<char *>(p.xbuf) + (long long)gi * kRing * xslot;
-    // operand: MFMA row r16 is batch row r16 / 4 when r16 % 4 == 0, nothing otherwise; k-step ks, lane group q: units
-    // 32 ks + 8 q .. + 7 = member 2 ks + q / 2, its units 8 (q % 2) .. + 7
+    // operand: lane (q, MFMA row r16) holds batch row r16 / 4 and quarter r16 % 4 of K: chunk c of the quarter, units
+    // 32 (NCH (r16 % 4) + c) + 8 q .. + 7 = member 2 (NCH (r16 % 4) + c) + q / 2, its units 8 (q % 2) .. + 7
     // float32: lane (quarter q, piece r16 / 4, row r16 % 4), chunk c of the quarter: member q NCH + c, its units 4 (r16 / 4) .. + 3
     const int orow = BF16 ? r16 >> 2 : r16 & 3;   // the batch row of the tile in this lane's operand
     const int arow = rowbase + orow;
-    const bool a_lane = (!BF16 || (r16 & 3) == 0) && arow < rend;
-    const int xl = !a_lane ? 0x7FFFFF00 : (BF16 ? (q >> 1) * QTILE + orow * 32 + (q & 1) * 16 : q * NCH * QTILE + orow * 64 + (r16 >> 2) * 16);
+    const bool a_lane = arow < rend;
+    const int xl = !a_lane ? 0x7FFFFF00 : (BF16 ? (2 * NCH * (r16 & 3) + (q >> 1)) * QTILE + orow * 32 + (q & 1) * 16 : q * NCH * QTILE + orow * 64 + (r16 >> 2) * 16);
     const long long xo = (long long)member * (QTILE / ESZ) + gb * 16 + gu;
     typedef typename std::conditional<BF16, uint16_t, uint32_t>::type word_t;
     constexpr word_t kMissing = BF16 ? (word_t)kSentinel16 : (word_t)kSentinel32;
@@ -596,7 +601,9 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
       // barrier (1.52 - 1.53) - but the issue slots: a wave asleep leaves its SIMD to the feeder, drainer and prefetch
       // waves, which these waves' raised priority otherwise keeps waiting (no s_sleep but priority 0 from the barrier
       // to the poll: 1.53).  Then the loop's start moved over the eight phases of a 32-byte line of code:
-      // 1.517 .. 1.573, the best one taken.  (K split over the waves, below: 1.70.)
+      // 1.517 .. 1.573, the best one taken.  (K split over the waves, below: 1.70.)  With the shorter polls, ms: 1.457 with one
+      // s_sleep, 1.52 with two, 1.60 with three; head dim 512 (B 4 x T 700), whose peers come later, 0.77, 0.73 and 0.76.  One
+      // barrier for two or four steps, W.x and h in rings of as many: 1.51 and 1.55 (the waves beside these then come in bursts).
       const int buf = t & 1;
       float wxv[4];
       XS_QTICK(5);
@@ -607,7 +614,7 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
       const bool row_reset = rfl[t & 3][orow] != 0u;       // (the operand's row: it contributes R.0 = 0 exactly)
       const bool gate_reset = rfl[t & 3][gb] != 0u;
 #ifndef XS_QUAD_SLEEP
-#define XS_QUAD_SLEEP 1
+#define XS_QUAD_SLEEP (BF16 && NCH == 4 ? 2 : 1)
 #endif
       if (XS_QUAD_SLEEP > 0) __builtin_amdgcn_s_sleep(XS_QUAD_SLEEP);
       asm volatile("");  // (the compiler keeps what stands in front of this statement in front of the poll)
@@ -624,7 +631,7 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
 #pragma unroll
         for (int ks = 0; ks < NP; ++ks) {
           areg[ks] = make_uint4(0, 0, 0, 0);
-          const int k = BF16 ? ks * 32 + q * 8 : q * KW + ks * 16 + (r16 >> 2) * 4;
+          const int k = BF16 ? ((r16 & 3) * NCH + ks) * 32 + q * 8 : q * KW + ks * 16 + (r16 >> 2) * 4;
           if (a_lane && p.s0 && (FULL || k < dh)) {
             const float *src = p.s0 + (long long)arow * H + head * dh + k;
             const float4 lo = *reinterpret_cast<const float4 *>(src);
@@ -682,12 +689,12 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
         for (int c = 0; c < NCH; ++c)
 #pragma unroll
           for (int w4 = 0; w4 < 4; ++w4)
-            acc[w4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, areg[w4 * NCH + c]),
+            acc[w4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, areg[c]),
                                                               __builtin_bit_cast(bf16x8, rreg[w4 * NCH + c]), acc[w4], 0, 0, 0);
-        mine = acc[0][0];
-        mine += acc[1][0];
-        mine += acc[2][0];
-        mine += acc[3][0];
+        mine = acc[0][0];  // (MFMA row 4 q + w4)
+        mine += acc[1][1];
+        mine += acc[2][2];
+        mine += acc[3][3];
       } else {
         // element e of the four 16-byte pieces of a chunk, in the order v_mfma_f32_16x16x4 takes them in the other kernels:
         // lane group q accumulates quarter q of K for the four rows, then the quarters of a row meet in its lane group

@@ -91,17 +91,17 @@ __global__ __launch_bounds__(256) void stage_exchange_kernel(StageParams p) {
 }
 
 // ---- (1b) the exchange as the kernel for row tiles of 4 rows makes it: [slot][member][4 rows][16 units], EVERY wave
-//      polls the group's whole tile (NK chunks of 16 bytes from the 16 lanes whose MFMA row is a real one) and publishes
-//      its own 16 values; the step's barrier and a pause of 64 cycles in front of the poll
+//      polls the group's whole tile (NK / 4 chunks of 16 bytes a lane) and publishes its own 16 values; the step's barrier
+//      and a pause of 64 cycles in front of the poll
 template <int NK>
 __global__ __launch_bounds__(256) void stage_exchange_quad_kernel(StageParams p) {
   const int wg = blockIdx.x, xcd = wg & 7, member = wg >> 3;
   if (xcd != 0 || member >= p.members) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, r16 = lane & 15;
-  constexpr int QTILE = 4 * 16 * 2;
+  constexpr int QTILE = 4 * 16 * 2, NCH = NK / 4;
   const int xslot = p.members * QTILE;
-  const bool a_lane = (r16 & 3) == 0 && (r16 >> 2) < p.rows;
-  const int xl = a_lane ? (q >> 1) * QTILE + (r16 >> 2) * 32 + (q & 1) * 16 : 0x7FFFFF00;
+  const bool a_lane = (r16 >> 2) < p.rows;
+  const int xl = a_lane ? (2 * NCH * (r16 & 3) + (q >> 1)) * QTILE + (r16 >> 2) * 32 + (q & 1) * 16 : 0x7FFFFF00;
   const long long xo = (long long)member * (QTILE / 2) + q * 16 + 4 * wave + (r16 & 3);
   uint32_t carry = (uint32_t)tid, max_spins = 0;
   bool dead = false;
@@ -115,15 +115,15 @@ __global__ __launch_bounds__(256) void stage_exchange_quad_kernel(StageParams p)
     __syncthreads();
     __builtin_amdgcn_s_sleep(1);
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char *>(cur), 0, xslot, 0x00020000);
-    uint4 areg[NK];
+    uint4 areg[NCH];
     uint32_t spins = 0;
     for (;;) {
 #pragma unroll
-      for (int ks = 0; ks < NK; ++ks)
+      for (int ks = 0; ks < NCH; ++ks)
         areg[ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, xl, ks * 2 * QTILE, 16));
       uint32_t ma = 0u;
 #pragma unroll
-      for (int ks = 0; ks < NK; ++ks) ma = mark_join<true>(ma, chunk_mark<true>(areg[ks]));
+      for (int ks = 0; ks < NCH; ++ks) ma = mark_join<true>(ma, chunk_mark<true>(areg[ks]));
       if (__builtin_amdgcn_ballot_w64(mark_has_sentinel<true>(ma)) == 0ull || dead) break;
       if (++spins >= (uint32_t)p.spin_limit ||
           ((spins & 1023u) == 0u && __hip_atomic_load(p.words, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)) {
@@ -133,10 +133,10 @@ __global__ __launch_bounds__(256) void stage_exchange_quad_kernel(StageParams p)
       }
     }
     max_spins = spins > max_spins ? spins : max_spins;
-    // (every lane's next word depends on a polled one: lanes 0-3 of a row of 16 publish, lanes 0, 4, 8, 12 poll)
+    // (every lane's next word depends on a polled one: lanes 0-3 of a row of 16 publish, all of them poll)
     uint32_t mix = areg[0].x;
 #pragma unroll
-    for (int ks = 1; ks < NK; ++ks) mix ^= areg[ks].x;
+    for (int ks = 1; ks < NCH; ++ks) mix ^= areg[ks].x;
     carry += mix + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)mix, 0x104, 0xF, 0xF, true);
   }
   if (lane == 0 && max_spins) atomicMax(p.words + 1, max_spins);
@@ -205,8 +205,8 @@ __global__ __launch_bounds__(256) void stage_chain_kernel(StageParams p) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, r16 = lane & 15;
   const int xslot = p.members * QTILE;
   char *const xbase = p.ring + (long long)group * kRing * xslot;
-  const bool a_lane = (r16 & 3) == 0 && (r16 >> 2) < p.rows;
-  const int xl = a_lane ? (q >> 1) * QTILE + (r16 >> 2) * 32 + (q & 1) * 16 : 0x7FFFFF00;
+  const bool a_lane = (r16 >> 2) < p.rows;
+  const int xl = a_lane ? (2 * NCH * (r16 & 3) + (q >> 1)) * QTILE + (r16 >> 2) * 32 + (q & 1) * 16 : 0x7FFFFF00;
   const long long xo = (long long)member * (QTILE / 2) + q * 16 + 4 * wave + (r16 & 3);
   uint4 rreg[NK];
 #pragma unroll
@@ -219,9 +219,9 @@ __global__ __launch_bounds__(256) void stage_chain_kernel(StageParams p) {
   uint32_t max_spins = 0;
   bool dead = false;
   // (the loop's start relative to a 32-byte line of code, chosen like the product kernel's: the best of the eight,
-  // 0.64 us per step; the others 0.67 (three of them) and 0.78 (four))
+  // 0.638 us per step; five others 0.64, two 0.81)
 #ifndef XS_CHAIN_PAD
-#define XS_CHAIN_PAD 4
+#define XS_CHAIN_PAD 6
 #endif
   asm volatile(".p2align 5\n\t.rept %0\n\ts_nop 0\n\t.endr" :: "n"(XS_CHAIN_PAD));
   for (int t = 0; t < p.steps; ++t) {
@@ -229,20 +229,20 @@ __global__ __launch_bounds__(256) void stage_chain_kernel(StageParams p) {
     uint16_t *const old = reinterpret_cast<uint16_t *>(xbase + ((t + kRing - 2) % kRing) * xslot);
     lds_barrier();
     __builtin_amdgcn_s_sleep(1);
-    uint4 areg[NK];
+    uint4 areg[NCH];
     if (t == 0) {
 #pragma unroll
-      for (int ks = 0; ks < NK; ++ks) areg[ks] = make_uint4(0, 0, 0, 0);
+      for (int ks = 0; ks < NCH; ++ks) areg[ks] = make_uint4(0, 0, 0, 0);
     } else {
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(xbase + ((t + kRing - 1) % kRing) * xslot, 0, xslot, 0x00020000);
       uint32_t spins = 0;
       for (;;) {
 #pragma unroll
-        for (int ks = 0; ks < NK; ++ks)
+        for (int ks = 0; ks < NCH; ++ks)
           areg[ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, xl, ks * 2 * QTILE, 16));
         uint32_t ma = 0u;
 #pragma unroll
-        for (int ks = 0; ks < NK; ++ks) ma = mark_join<true>(ma, chunk_mark<true>(areg[ks]));
+        for (int ks = 0; ks < NCH; ++ks) ma = mark_join<true>(ma, chunk_mark<true>(areg[ks]));
         if (__builtin_amdgcn_ballot_w64(mark_has_sentinel<true>(ma)) == 0ull || dead) break;
         if (++spins >= (uint32_t)p.spin_limit ||
             ((spins & 1023u) == 0u && __hip_atomic_load(p.words, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)) {
@@ -260,12 +260,12 @@ __global__ __launch_bounds__(256) void stage_chain_kernel(StageParams p) {
     for (int c = 0; c < NCH; ++c)
 #pragma unroll
       for (int w4 = 0; w4 < 4; ++w4)
-        acc[w4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, areg[w4 * NCH + c]),
+        acc[w4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, areg[c]),
                                                           __builtin_bit_cast(bf16x8, rreg[w4 * NCH + c]), acc[w4], 0, 0, 0);
     float mine = acc[0][0];
-    mine += acc[1][0];
-    mine += acc[2][0];
-    mine += acc[3][0];
+    mine += acc[1][1];
+    mine += acc[2][2];
+    mine += acc[3][3];
     const int mi = __float_as_int(mine);
     const float ry1 = __int_as_float(__builtin_amdgcn_update_dpp(0, mi, 0x104, 0xF, 0xF, true));
     const float ry2 = __int_as_float(__builtin_amdgcn_update_dpp(0, mi, 0x108, 0xF, 0xF, true));
