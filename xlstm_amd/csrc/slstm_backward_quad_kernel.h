@@ -175,9 +175,10 @@ __global__ __launch_bounds__(kBwdQuadThreads) void slstm_bwd_quad_kernel(BwdSpli
   }
   const int pub_off = prow * (K * 2) + (s * UW + pu) * 8;
   const int wave_u = (int)uniform((uint32_t)wave);
-  // + k-step * 64; the lanes between the real rows ask past the end of the slot and get zeros without a request to the L2
-  // (with copies of the real rows there a look moved four times the bytes through the compute unit's one return path)
-  const int poll_off = (r16 & 3) == 0 ? (r16 >> 2) * (K * 2) + q * 16 : 0x7FFFFF00;
+  // MFMA row r16 holds k-step r16 % 4 (+ 4 a load) of batch row r16 / 4: a load brings four k-steps, no lane of it is a row that
+  // is not there (one k-step a load, its rows at MFMA rows 0, 4, 8, 12: 2.11 ms at B 16 x T 2048 x 4 heads of 256, 2.01 with this)
+  constexpr int LOADS = (KSTEPS + 3) / 4;
+  const int poll_off = (r16 & 3) < KSTEPS ? (r16 >> 2) * (K * 2) + (r16 & 3) * 64 + q * 16 : 0x7FFFFF00;
   char *const ring = reinterpret_cast<char *>(p.xch) + (long long)group * SLOT;
   const long long ring_stride = (long long)ngroups * SLOT;
   const bool cut = p.cut != 0;
@@ -266,25 +267,30 @@ __global__ __launch_bounds__(kBwdQuadThreads) void slstm_bwd_quad_kernel(BwdSpli
       //      Two sets of tiles, used in turn: a wave writes the tiles of step n + 2 only after a peer has published step
       //      n + 2, for which that peer needed all of this workgroup's deltas of step n + 1, which were computed from the
       //      sums of step n.
-      auto multiply = [&](const u32x4_t (&a)[KSTEPS]) {
+      auto multiply = [&](const u32x4_t (&a)[LOADS]) {
         XS_BTICK(3);
-        f32x4 acc[4];
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb) acc[cb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        constexpr int CH = KSTEPS < 4 ? KSTEPS : 4;  // a chain per MFMA row of a batch row: its sums arrive in register j of lane group q
+        f32x4 acc[CH][4];
 #pragma unroll
         for (int ks = 0; ks < KSTEPS; ++ks)
 #pragma unroll
           for (int cb = 0; cb < 4; ++cb)
-            acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[ks]), __builtin_bit_cast(bf16x8, bq[ks][cb]), acc[cb], 0, 0, 0);
+            acc[ks % 4][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[ks / 4]), __builtin_bit_cast(bf16x8, bq[ks][cb]),
+                                                                      ks < 4 ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : acc[ks % 4][cb], 0, 0, 0);
         float *const tiles = part + (n & 1) * 8 * PART + wave * PART + q * kBwdPartStride + r16;
 #pragma unroll
-        for (int cb = 0; cb < 4; ++cb) tiles[cb * 16] = acc[cb][0];
+        for (int cb = 0; cb < 4; ++cb) {
+          float sum = acc[0][cb][0];
+#pragma unroll
+          for (int j = 1; j < CH; ++j) sum += acc[j][cb][j];
+          tiles[cb * 16] = sum;
+        }
       };
       // (a negative spin limit is the host's way to make every wait run out at its first look: the error path, forced)
-      auto complete = [&](const u32x4_t (&a)[KSTEPS]) {
+      auto complete = [&](const u32x4_t (&a)[LOADS]) {
         uint32_t mark = 0u;
 #pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks) mark = mark_join<true>(mark, chunk_mark<true>(__builtin_bit_cast(uint4, a[ks])));
+        for (int i = 0; i < LOADS; ++i) mark = mark_join<true>(mark, chunk_mark<true>(__builtin_bit_cast(uint4, a[i])));
         return (__builtin_amdgcn_ballot_w64(mark_has_sentinel<true>(mark)) == 0ull && p.spin_limit >= 0) || gave_up;
       };
       long long spins = 0;
@@ -301,7 +307,7 @@ __global__ __launch_bounds__(kBwdQuadThreads) void slstm_bwd_quad_kernel(BwdSpli
       // (two looks in flight half a round trip apart, so that an incomplete one is followed sooner: 0.15 to 0.4 ms slower,
       // as was every variant that asks more often)
       {
-        u32x4_t areg[KSTEPS];
+        u32x4_t areg[LOADS];
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(ring + (n % kBwdRing) * ring_stride, 0, SLOT, 0x00020000);
         constexpr int kPastL1 = 16;  // (the load's scope bits: served by the L2)
         if (lane == 0) look_step[wave] = n + 1;
@@ -310,8 +316,8 @@ __global__ __launch_bounds__(kBwdQuadThreads) void slstm_bwd_quad_kernel(BwdSpli
           blook = clock64() - btick;
 #endif
 #pragma unroll
-          for (int ks = 0; ks < KSTEPS; ++ks)
-            areg[ks] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, poll_off, (wave_u * KSTEPS + ks) * 64, kPastL1));
+          for (int i = 0; i < LOADS; ++i)
+            areg[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, poll_off, (wave_u * KSTEPS + 4 * i) * 64, kPastL1));
           if (complete(areg)) break;
           another_round();
         }

@@ -22,7 +22,9 @@
 //
 // Bound by the chain of a step (publish, poll, MFMA, barrier: about 1 us); us a step at NH heads x head dim, batch, the
 // forward's coefficients included, against the walk and the reverse kernel before: float32 4x256 B16 1.5 (9.0), bf16
-// 4x192 B16 1.0, 4x512 B8 1.3, 4x512 B64 3.5, 4x1024 B16 3.8 (18.0).
+// 4x192 B16 1.0, 4x512 B8 1.3, 4x512 B64 3.5, 4x1024 B16 3.8 (18.0).  Polls whose lanes are all rows that are there (row tiles
+// of 4 and 8 rows in bf16: below), us a training call before -> after: 4x1024 B16 T512 3609 -> 2997 (the reverse pass 3.8 -> 2.6 a
+// step), 8x384 B8 T300 785 -> 660, 4x256 B6 T300 601 -> 557, 4x512 B16 T256 815 -> 763.
 #pragma once
 
 namespace {
@@ -73,7 +75,10 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
   constexpr int PSTRIDE = unit_part_stride(CT), PWAVE = RT * PSTRIDE;
   constexpr int COEFS = SETS * CT * 2304;     // bytes of a step's coefficients: [set of 4 rows][16 units][576 floats]
   constexpr int NLD = BF16 ? 2 * CT * GQ : GQ;  // 16-byte pieces of deltas a lane polls per step (float32: per set of four rows)
-  constexpr int BATCH = NLD < 16 ? NLD : 16;  // ... in one go
+  // bf16, row tiles of fewer than 16 rows: PK MFMA rows per batch row, each of which takes another piece, so that a load has
+  // no lane without a row; NPL loads for the NLD pieces
+  constexpr int PK = BF16 ? 16 / RT : 1, NPL = (NLD + PK - 1) / PK;
+  constexpr int BATCH = NPL < 16 ? NPL : 16;  // ... in one go
   constexpr int NPASS = BF16 ? 1 : SETS;
   extern __shared__ __attribute__((aligned(1024))) unsigned char unit_lds[];
   float *const part = reinterpret_cast<float *>(unit_lds);          // [2][NW waves][RT][PSTRIDE]
@@ -198,13 +203,16 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
   char *const ring = p.xch + (long long)gi * xslot;
   const long long ring_stride = (long long)ngroups * xslot;
   const int pub = member * MB + prow * EB + pu * 4 * ESZ;
-  // poll: bf16: piece j: member wave GQ + j / (2 CT), units 8 (j % (2 CT)) + 2 q, + 1 of MFMA row r16's batch row; float32: piece c:
-  // member wave GQ + c, unit 4 q + r16 / 4 of row r16 % 4.  Members past the last one, and (RT 4) the rows between the
-  // real ones, lie past the end of the descriptor: zeros
+  // poll: bf16: piece j: member wave GQ + j / (2 CT), units 8 (j % (2 CT)) + 2 q, + 1 of a batch row; MFMA row r16 holds pieces
+  // r16 % PK, + PK, ... of batch row r16 / PK; float32: piece c: member wave GQ + c, unit 4 q + r16 / 4 of row r16 % 4.  Members
+  // past the last one and pieces that are another wave's lie past the end of the descriptor: zeros
   int vo;
-  constexpr int STEP = 16 / RT;               // MFMA rows per batch row (bf16)
-  if constexpr (BF16) vo = r16 % STEP == 0 ? (r16 / STEP) * EB + q * 16 : 0x40000000;
-  else vo = (r16 & 3) * EB + q * 64 + (r16 >> 2) * 16;
+  if constexpr (BF16) {
+    const int j = r16 % PK;
+    vo = j < NLD ? r16 / PK * EB + q * 16 + j / (2 * CT) * MB + j % (2 * CT) * 64 : 0x40000000;
+  } else {
+    vo = (r16 & 3) * EB + q * 64 + (r16 >> 2) * 16;
+  }
   vo += wave * GQ * MB;
 
   f32x4 cA{0, 0, 0, 0}, cB{0, 0, 0, 0};
@@ -287,17 +295,19 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
       float *const tiles = part + (n & 1) * (NW * PWAVE) + wave * PWAVE;
 #pragma unroll
       for (int ps = 0; ps < NPASS; ++ps) {
-        f32x4 acc[BF16 ? 4 : 1];  // (bf16: four chains, CT 2: two per column tile)
+        // bf16: a chain per column tile and MFMA row of a batch row (RT 16: four chains, CT 2: two per column tile)
+        constexpr int CH = PK == 1 ? 4 / CT : PK;
+        f32x4 acc[BF16 ? CT * CH : 1];
 #pragma unroll
-        for (int i = 0; i < (BF16 ? 4 : 1); ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int i = 0; i < (BF16 ? CT * CH : 1); ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int b0 = 0; b0 < NLD; b0 += BATCH) {
+        for (int b0 = 0; b0 < NPL; b0 += BATCH) {
           uint4 areg[BATCH];
           long long spins = 0;
           for (;;) {
 #pragma unroll
             for (int i = 0; i < BATCH; ++i) {
-              const int j = b0 + i;
+              const int j = (b0 + i) * PK;
               const int off = BF16 ? j / (2 * CT) * MB + j % (2 * CT) * 64 : j * MB + ps * 4 * EB;
               areg[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, vo + off, 0, 16));
             }
@@ -314,10 +324,14 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
 #pragma unroll
             for (int i = 0; i < BATCH; ++i)
 #pragma unroll
-              for (int ct = 0; ct < CT; ++ct) {
-                f32x4 &c = acc[CT == 1 ? i & 3 : 2 * ct + (i & 1)];
-                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, areg[i]), __builtin_bit_cast(bf16x8, rb[b0 + i][ct]), c, 0, 0, 0);
-              }
+              for (int j = 0; j < PK; ++j)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) {
+                  const int piece = (b0 + i) * PK + j;
+                  if (piece >= NLD) continue;
+                  f32x4 &c = acc[ct * CH + (PK == 1 ? i % CH : j)];
+                  c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, areg[i]), __builtin_bit_cast(bf16x8, rb[piece][ct]), c, 0, 0, 0);
+                }
           } else {
 #pragma unroll
             for (int i = 0; i < BATCH; ++i) {
@@ -334,19 +348,21 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
           }
         }
         if constexpr (BF16) {
-          // lane group q holds MFMA rows 4 q .. 4 q + 3: batch rows (4 q + i) / STEP
-          if constexpr (CT == 1) {
-            const f32x4 sum = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+          // lane group q holds MFMA rows 4 q .. 4 q + 3: batch rows (4 q + i) / PK, the sums of chain j in row j of the PK
 #pragma unroll
-            for (int i = 0; i < 4; i += STEP) tiles[(4 * q + i) / STEP * PSTRIDE + r16] = sum[i];
-          } else {
-            const f32x4 s0 = acc[0] + acc[1], s1 = acc[2] + acc[3];
+          for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-            for (int i = 0; i < 4; i += STEP) {
-              tiles[(4 * q + i) / STEP * PSTRIDE + r16] = s0[i];
-              tiles[(4 * q + i) / STEP * PSTRIDE + 16 + r16] = s1[i];
+            for (int i = 0; i < 4; i += PK) {
+              float sum = acc[ct * CH][i];
+              if constexpr (PK == 1) {
+                if constexpr (CH == 4) sum = (sum + acc[1][i]) + (acc[2][i] + acc[3][i]);
+                else sum += acc[ct * CH + 1][i];
+              } else {
+#pragma unroll
+                for (int j = 1; j < PK; ++j) sum += acc[ct * CH + j][i + j];
+              }
+              tiles[(4 * q + i) / PK * PSTRIDE + 16 * ct + r16] = sum;
             }
-          }
         } else {
           float x0 = acc[0][0], x1 = acc[0][1], x2 = acc[0][2], x3 = acc[0][3];
           transpose_lane_groups(x0, x1, x2, x3);
