@@ -14,8 +14,8 @@
 // K is ordered (unit of the head, gate): the four deltas of an element are 8 bytes in a row and a thread publishes them
 // with one store; a group's slot is [4 rows][K] bf16, a wave's store 512 bytes in a row.  Wave w multiplies k-steps
 // 4w ... 4w + 3 (at head dim 256), i.e. the deltas of units 32w ... 32w + 31 of the head: it polls ONE publisher's
-// half.  The four batch rows sit at MFMA rows 0, 4, 8, 12 (the rows between are zero), so the sum of (row b, column n)
-// arrives in lane group b, lane n, first element.
+// half.  Batch row b takes the MFMA rows 4 b .. 4 b + 3, each with another of the wave's k-steps, so that no lane of a poll is
+// a row that is not there; the sum of (row b, column n) over k-step j arrives in lane group b, lane n, element j.
 #pragma once
 
 namespace {
@@ -30,14 +30,16 @@ constexpr int kBwdQuadDepth = 6;                   // steps the feeder waves req
 static_assert(kBwdQuadDepth >= 3 && kBwdQuadDepth <= kBwdQuadSlots && kBwdQuadDepth <= kBwdQuadFeeders + 2, "feeder depth");
 constexpr int kBwdQuadThreads = (8 + kBwdQuadFeeders) * 64;
 constexpr int kBwdQuadPart = 4 * kBwdPartStride;   // floats of a wave's partial tile
-constexpr int bwd_quad_lds_bytes() { return 2 * 8 * kBwdQuadPart * 4 + kBwdQuadSlots * kBwdQuadSlot; }
+constexpr int kBwdQuadStash = 4 * 64 * 16;         // a step's deltas on their way to d_wx: four values per element
+constexpr int bwd_quad_lds_bytes() { return 2 * 8 * kBwdQuadPart * 4 + kBwdQuadSlots * kBwdQuadSlot + 2 * kBwdQuadStash; }
 
 // s_sleep units (64 cycles each) in front of a wave's first look at the step's deltas: of the waves that do not form the
 // step's gradient (they leave the barrier with nothing else to do, a quarter of a step before anything is published),
 // and of the waves that have just published.  Reverse kernel at B 16, T 2048, 4 heads of 256, ms: (0, 0) 2.43, (4, 0)
 // 2.42, (6, 2) 2.31, (8, 2) 2.20, (8, 4) 2.17, (10, 0) 2.24, (12, 2) 2.20, (16, 4) 2.33; at half the batch (one group per
 // XCD) 2.13, 2.21, 2.09, 2.02, 2.09, 2.04, 2.10, 2.32.  A look that comes back incomplete costs its whole round trip, and
-// so does every cycle slept past the arrival.
+// so does every cycle slept past the arrival.  (With the polls and stores of the kernel as it is now, ms a training call:
+// (8, 2) 3.70, (8, 4) 3.76, (8, 6) 3.85, (6, 2) 3.72, (10, 4) 3.77.)
 constexpr int kBwdQuadSleepIdle = 8, kBwdQuadSleepPublished = 2;
 
 template <int S, bool DWX16 = false>  // S workgroups per group, dh = 64 S; DWX16: d_wx takes the gate deltas rounded to bf16
@@ -67,6 +69,10 @@ __global__ __launch_bounds__(kBwdQuadThreads) void slstm_bwd_quad_kernel(BwdSpli
   const int row0 = (group / p.NH) * 4;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, r16 = lane & 15;
   char *const feed = reinterpret_cast<char *>(part + 2 * 8 * PART);
+  // the deltas of the step before, for the feeder waves to write to d_wx: [2][row][64 units][4 gates].  (Stores of the waves
+  // that form the gradient stood in front of their look at the peers' deltas, which waits for their acknowledgement.)
+  typedef typename std::conditional<DWX16, uint16_t, float>::type wx_t;
+  wx_t *const stash = reinterpret_cast<wx_t *>(feed + kBwdQuadSlots * kBwdQuadSlot);
   bwd_note_placement(p, group);
   // look_step[w]: 1 + the step of the call whose first look compute wave w has issued (for the feeder waves, see there)
   __shared__ volatile int look_step[8];
@@ -115,7 +121,15 @@ __global__ __launch_bounds__(kBwdQuadThreads) void slstm_bwd_quad_kernel(BwdSpli
 #ifdef XS_PROFILE
       fprof[4] += clock64() - ftick;  // (the wait, if it was this wave's turn)
 #endif
-      __syncthreads();  // A(m)
+      lds_barrier();  // A(m)
+      // feeder wave f writes the step's deltas of row f, and the first the group's progress
+      if (s == 0 && f == 0 && lane == 0 && m + 1 < p.T) p.progress[group] = (unsigned int)(m + 1);
+      if (f < rows_there) {
+        const long long wo = (long long)(row0 + f) * p.d_wx_sb + (long long)(p.T - 1 - m) * p.d_wx_st + (long long)head * dh + s * UW + lane;
+        const wx_t *const mine = stash + (((m & 1) * 4 + f) * 64 + lane) * 4;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) reinterpret_cast<wx_t *>(p.d_wx)[wo + (long long)g * H] = mine[g];
+      }
 #ifdef XS_PROFILE
       fprof[5] += clock64() - ftick;  // (the step)
       ftick = clock64();
@@ -244,18 +258,12 @@ __global__ __launch_bounds__(kBwdQuadThreads) void slstm_bwd_quad_kernel(BwdSpli
         *reinterpret_cast<uint2 *>(ring + ((n + kBwdRing - 2) % kBwdRing) * ring_stride + pub_off) = uint2{0xFFFFFFFFu, 0xFFFFFFFFu};
       }
       XS_BTICK(1);
-      // ---- while the deltas are on their way: d_wx, the progress word, the next step's inputs
-      //      (with the first look issued in front of these instead of behind them, and a longer sleep in front of it, the
-      //      kernel took 2.33 ms at config 2 instead of 2.20: the look then waits for the stores behind it as well)
-      if (s == 0 && tid == 0) p.progress[group] = (unsigned int)n;
-      if (there) {
-        const long long wo = (long long)row * p.d_wx_sb + (long long)t * p.d_wx_st + ecol;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          if constexpr (DWX16) reinterpret_cast<uint16_t *>(p.d_wx)[wo + (long long)g * H] = (uint16_t)(pack_bf16x2(delta[g], 0.0f) & 0xFFFFu);
-          else p.d_wx[wo + (long long)g * H] = delta[g];
-        }
-      }
+      // ---- while the deltas are on their way: their copies for the feeder waves, the next step's inputs.  (A look right
+      //      behind the publication, these under it: it comes too early and its repetition is late, 4.18 ms a training
+      //      call at B 16 x T 2048 x 4 heads of 256 against 3.70; five units of sleep more, 3.98.)
+      wx_t *const copy = stash + (((n & 1) * 4 + prow) * 64 + pu) * 4;
+      if constexpr (DWX16) *reinterpret_cast<uint2 *>(copy) = uint2{pack_bf16x2(delta[0], delta[1]), pack_bf16x2(delta[2], delta[3])};
+      else *reinterpret_cast<f32x4 *>(copy) = f32x4{delta[0], delta[1], delta[2], delta[3]};
       if (n + 1 < p.T) read_inputs(n + 1);
       if (!cut && S > 1) __builtin_amdgcn_s_sleep(kBwdQuadSleepPublished);
     } else {
@@ -328,7 +336,7 @@ __global__ __launch_bounds__(kBwdQuadThreads) void slstm_bwd_quad_kernel(BwdSpli
       }
     }
     XS_BTICK(4);
-    __syncthreads();  // A(n)
+    lds_barrier();  // A(n)
     XS_BTICK(5);
   }
   // ---- gradient w.r.t. the initial state (the stabiliser's part is zero by the rule; NaN all over when a wait ran out)

@@ -60,6 +60,12 @@ constexpr int unit_bwd_lds_bytes(int rt, int ct, bool bf16) {
   return 2 * 4 * ct * rt * unit_part_stride(ct) * 4 + 2 * unit_bwd_burst(rt, ct) * unit_bwd_slot(rt, ct, bf16);
 }
 
+// s_sleep units (64 cycles each) in front of a wave's first look at the step's deltas: of the waves that have just published,
+// and of the others.  A look that comes back incomplete costs its whole round trip.  Head dim 1024 in row tiles of 8 rows has
+// the longest step (B 16 x T 512 x 4 heads, us a training call): (2, 8) 3006, (2, 12) 2924, (4, 12) 2917, (6, 16) 2881, (9, 16) 2883,
+// (6, 20) 2905, (9, 24) 2933; the others lose with more than (2, 8): 4 heads of 256, 6 rows, T 300 (2, 8) 558, (4, 10) 570, (6, 16) 597.
+constexpr int unit_bwd_sleep(int rt, int ct, int gq, bool published) { return rt == 8 && ct == 2 && gq == 4 ? (published ? 6 : 16) : (published ? 2 : 8); }
+
 template <bool BF16, int GQ, int RT, int CT, bool DWX16>  // GQ: members of a wave's share of K (rounded up)
 __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(UnitBwdParams p) {
   static_assert(RT == 4 || (RT == 16 && BF16 == (CT == 2)) || (RT == 8 && CT == 2), "row tiles of 4, 8 (bf16) or 16 rows");
@@ -286,9 +292,9 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
         }
       }
       if (n + 1 < p.T) read_inputs(n + 1);
-      if (!p.cut) __builtin_amdgcn_s_sleep(2);
+      if (!p.cut) __builtin_amdgcn_s_sleep(unit_bwd_sleep(RT, CT, GQ, true));
     } else {
-      if (!p.cut) __builtin_amdgcn_s_sleep(8);
+      if (!p.cut) __builtin_amdgcn_s_sleep(unit_bwd_sleep(RT, CT, GQ, false));
     }
     if (!p.cut) {
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(ring + (n % kBwdRing) * ring_stride, 0, xslot, 0x00020000);
