@@ -33,6 +33,7 @@
 #include "slstm_device_common.h"
 #include "slstm_seq_kernel.h"
 #include "slstm_seq_roles_kernel.h"
+#include "slstm_seq_pair_kernel.h"
 #include "slstm_step_kernel.h"
 #include "slstm_step_pipe_kernel.h"
 #include "slstm_step_small_kernel.h"
@@ -527,6 +528,26 @@ std::mutex &launches_into(const void *workspace) {
   return mu[((uintptr_t)workspace >> 8) % 64];
 }
 
+SeqKernel pick_pair(int MT, int rows, bool coef) {
+  if (MT == 2) return coef ? slstm_seq_pair_kernel<2, 16, 2> : slstm_seq_pair_kernel<2, 16, 0>;
+  if (rows == 4) return coef ? slstm_seq_pair_kernel<1, 4, 2> : slstm_seq_pair_kernel<1, 4, 0>;
+  if (rows == 8) return coef ? slstm_seq_pair_kernel<1, 8, 2> : slstm_seq_pair_kernel<1, 8, 0>;
+  return coef ? slstm_seq_pair_kernel<1, 16, 2> : slstm_seq_pair_kernel<1, 16, 0>;
+}
+
+// Do two workgroups of every form of slstm_seq_pair_kernel share a compute unit, as its placement needs?
+bool pair_resident() {
+  static const bool resident = [] {
+    for (int form = 0; form < 8; ++form) {
+      const SeqKernel k = pick_pair(form >> 1 == 3 ? 2 : 1, 4 << (form >> 1), form & 1);
+      int n = 0;
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(k), kPairThreads, 0) != hipSuccess || n < 2) return false;
+    }
+    return true;
+  }();
+  return resident;
+}
+
 // need != nullptr: launch nothing, only say whether a kernel takes every launch of this call and how many bytes of
 // workspace they touch
 int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_host = nullptr, float *train_coef = nullptr) {
@@ -565,8 +586,23 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
   // (one workgroup per compute unit), not per device: with 24 workgroups per group an XCD of 32 compute units
   // holds one group, not 32 * 8 / 24 of the device's.
   const int cus_per_xcd = cus / 8 > 0 ? cus / 8 : 1;
+  // The gating waves of the kernel of four row tiles, and the kernel with two workgroups per compute unit, address W.x, the
+  // mask and h_out as a scalar base plus a 32-bit offset per lane inside four rows / one row tile.
+  const long long esz = bf16 ? 2 : 4;
+  const bool offsets_fit = 4ll * a->wx_stride_b * esz + 4ll * NH * dh * esz < 0xFFFFFF00ll &&
+                           (!a->reset || 4ll * a->reset_stride_b < 0xFFFFFF00ll) && 16ll * NH * dh * esz < (1ll << 31);
+  // Heads of more workgroups than an XCD has compute units, sequences that are not short: two workgroups per compute unit and a head on
+  // one XCD (slstm_seq_pair_kernel).  R is then read once for every 32 rows instead of 64 before the first step, and 64 peers shake
+  // hands: 4 heads of 1024, us a call, on XCD pairs / on one XCD: B 64 T 40 143 / 151, T 100 361 / 346, T 300 1016 / 937; B 16 T 17 68 / 76, T 40
+  // 119 / 114, T 300 700 / 514; B 2 T 9 49 / 47; 4 x 768 B 64 T 40 161 / 137.  (A training forward takes one row tile per workgroup on XCD
+  // pairs, four times the launches.)
+  const int pair_groups = 8 * (2 * cus_per_xcd / G), pair_heads = NH < pair_groups ? NH : pair_groups;
+  const bool pair = bf16 && G > 32 && pair_groups > 0 && offsets_fit &&
+                    T >= (train_coef || (B + 15) / 16 <= pair_groups / pair_heads ? 32 : 64) && pair_resident();
+  const int span = pair ? 64 : 32;
   int capacity;  // head groups per launch
-  if (G <= 32) capacity = 8 * (cus_per_xcd / G);
+  if (pair) capacity = pair_groups;
+  else if (G <= 32) capacity = 8 * (cus_per_xcd / G);
   else if (G <= 64 && G % 2 == 0) capacity = 4 * ((2 * cus_per_xcd) / G);
   else capacity = cus / G;
   if (capacity < 1) return fail(XS_ERR_DEVICE, "a head group of %d workgroups does not fit the %d compute units of this device's XCDs", G, cus);
@@ -589,16 +625,10 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
   const int max_groups_per_head = capacity / NHL;  // >= 1
   int MT = 1;
   // (a training forward that leaves its coefficients: one row tile per workgroup, more launches)
-  while (!train_coef && MT < 4 && (tiles + MT - 1) / MT > max_groups_per_head) MT *= 2;
-  {
-    // The gating waves of the kernel of four row tiles address W.x, the mask and h_out as a scalar base plus a 32-bit
-    // offset per lane inside four rows / one row tile.  Where four rows span more than that (sequences of a gigabyte
-    // per row), the batch goes through the kernel of two row tiles in more launches instead.
-    const long long esz = bf16 ? 2 : 4;
-    const bool offsets_fit = 4ll * a->wx_stride_b * esz + 4ll * NH * dh * esz < 0xFFFFFF00ll &&
-                             (!a->reset || 4ll * a->reset_stride_b < 0xFFFFFF00ll) && 16ll * NH * dh * esz < (1ll << 31);
-    if (MT == 4 && !offsets_fit) MT = 2;
-  }
+  while ((pair || !train_coef) && MT < (pair ? 2 : 4) && (tiles + MT - 1) / MT > max_groups_per_head) MT *= 2;
+  // (where four rows span more than 32-bit offsets reach - sequences of a gigabyte per row -, the batch goes through the kernel of
+  // two row tiles in more launches instead)
+  if (MT == 4 && !offsets_fit) MT = 2;
   // small heads stay in one compute unit, all heads that are left in one launch (nothing waits, so nothing has to be
   // resident at once), unless the batch is one for the kernel of four row tiles.  (The slices of heads but the last are of
   // one size: where the first goes to that kernel, a last one of fewer heads may still come here.)
@@ -629,7 +659,8 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
     // row tiles of at most 4 rows: the compute waves split the columns by unit, not K (head groups on one XCD)
     const bool quad = MT == 1 && rows_per_wg == 4 && G <= 32;
     if (quad) kern = bf16 ? (full ? pick_quad<true, true>(nch) : pick_quad<true, false>(nch)) : (full ? pick_quad<false, true>(nch) : pick_quad<false, false>(nch));
-    if (train_coef) kern = bf16 ? (full ? pick_train<true, true>(nch, quad, burst) : pick_train<true, false>(nch, quad, burst))
+    if (pair) kern = pick_pair(MT, rows_per_wg, train_coef != nullptr);
+    else if (train_coef) kern = bf16 ? (full ? pick_train<true, true>(nch, quad, burst) : pick_train<true, false>(nch, quad, burst))
                                 : (full ? pick_train<false, true>(nch, quad, burst) : pick_train<false, false>(nch, quad, burst));
     if (a->coef_out) {  // a training forward: the same kernel, leaving the backward pass its coefficients
       if (!quad || !bf16 || (dh != 128 && dh != 256) || rows_per_launch < B)
@@ -649,7 +680,7 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
     const int NBT = (bend - b0 + rows_per_wg - 1) / rows_per_wg;
     const int ngroups = NHL * NBT;
     // grid shapes of the three placements the kernel knows: one XCD per group, two XCDs per group, spread
-    const int grid = G <= 32 ? 8 * G * ((ngroups + 7) / 8)
+    const int grid = G <= span ? 8 * G * ((ngroups + 7) / 8)
                              : ((G <= 64 && G % 2 == 0) ? 8 * (G / 2) * ((ngroups + 3) / 4) : ngroups * G);
     if (grid > kMaxWg) return fail(XS_ERR_UNSUPPORTED, "grid %d too large", grid);
     if (dry) {
@@ -676,7 +707,7 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
     p.wg_xcc = (uint32_t *)((char *)a->workspace + kStatusBytes);
     p.xbuf = (char *)a->workspace + kHeaderBytes;
     p.B = B; p.T = T; p.NH = NH; p.dh = dh;
-    p.b0 = b0; p.bend = bend; p.G = G; p.NBT = NBT; p.rows_per_wg = rows_per_wg;
+    p.b0 = b0; p.bend = bend; p.G = G; p.span = span; p.NBT = NBT; p.rows_per_wg = rows_per_wg;
     p.head0 = head0; p.NHL = NHL;
     p.spin_limit = a->spin_limit;
     p.coef_out = train_coef ? train_coef : a->coef_out;
@@ -689,7 +720,7 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
       const int want = (rows_in_tile * (bf16 ? 2 : 4) + 7) / 8;
       p.prefetch = want <= max_prefetch_waves(nch) ? want : 0;
     }
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(roles ? kRolesThreads : kThreads + 64 * p.prefetch), 0, stream, p);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(pair ? kPairThreads : (roles ? kRolesThreads : kThreads + 64 * p.prefetch)), 0, stream, p);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(XS_ERR_LAUNCH, "sequence kernel launch failed: %s", hipGetErrorString(e));
   }

@@ -21,6 +21,7 @@ struct SeqParams {
   int B, T, NH, dh;
   int b0, bend;  // batch rows [b0, bend) handled by this launch
   int G;         // workgroups per head group
+  int span;      // workgroups that one XCD holds: 32, or 64 where two share a compute unit (slstm_seq_pair_kernel)
   int NBT;       // batch tiles (independent groups) per head
   int head0;     // first head of this launch (more heads than fit the device at once go in several launches)
   int NHL;       // heads of this launch
@@ -84,7 +85,7 @@ __device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgc
 // ---- role of a workgroup (XCD-aware: workgroup i is dispatched to XCD i % 8; a head group takes consecutive slots of
 //      ONE XCD so its exchange stays in one L2): head group index and position inside the group
 __device__ __forceinline__ void seq_place(const SeqParams &p, int wg, int &gi, int &member) {
-  if (p.G <= 32) {
+  if (p.G <= p.span) {
     const int xcd = wg & 7;
     const int local = wg >> 3;
     const int slot = local / p.G;
@@ -106,41 +107,41 @@ __device__ __forceinline__ void seq_place(const SeqParams &p, int wg, int &gi, i
   }
 }
 
-// ---- placement handshake (one thread of the workgroup): do all members of this head group share one XCD (one L2)?
+// ---- placement handshake (the first wave of the workgroup): do all members of this head group share one XCD (one L2)?
 //      If so h is published with plain stores (they land in that L2); otherwise with device-scope stores that are
-//      written through to memory.  Returns 1 for "more than one XCD".
+//      written through to memory.  Returns 1 for "more than one XCD".  A lane looks at one peer.
 __device__ __forceinline__ uint32_t seq_handshake(const SeqParams &p, int wg, int gi, long long spin_limit) {
-  const bool one_xcd_layout = p.G <= 32;
-  if (wg == 0) {
-    atomicAdd(&p.status->launches, 1u);  // a long batch is run as several launches of row chunks
-    p.status->rows_per_workgroup = (uint32_t)p.rows_per_wg;
-  }
+  const bool one_xcd_layout = p.G <= p.span;
+  const int lane = threadIdx.x & 63;
   const uint32_t my_xcc = __builtin_amdgcn_s_getreg(20 | (3 << 11)) & 0xFu;  // XCC_ID, bits [3:0]
-  __hip_atomic_store(&p.wg_xcc[wg], 0x80000000u | ((uint32_t)gi << 8) | my_xcc, __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
-  uint32_t cross = one_xcd_layout ? 0u : 1u;
-  if (one_xcd_layout) {
-    const int xcd = wg & 7;
-    const int slot = (wg >> 3) / p.G;
-    for (int j = 0; j < p.G; ++j) {
-      const int peer = ((slot * p.G + j) << 3) | xcd;
-      uint32_t w = 0;
-      long long spins = 0;
-      while (((w = __hip_atomic_load(&p.wg_xcc[peer], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) & 0x80000000u) == 0u) {
-        if (++spins >= spin_limit) {  // a peer never started: the grid is not co-resident
-          if (atomicExch(&p.status->aborted, 1u) == 0u) {
-            p.status->abort_wg = (uint32_t)wg;
-            p.status->abort_step = 0xFFFFFFFFu;
-          }
-          cross = 1u;
-          break;
-        }
-      }
-      if ((w & 0xFu) != my_xcc) cross = 1u;
+  if (lane == 0) {
+    if (wg == 0) {
+      atomicAdd(&p.status->launches, 1u);  // a long batch is run as several launches of row chunks
+      p.status->rows_per_workgroup = (uint32_t)p.rows_per_wg;
     }
-    if (cross) atomicAdd(&p.status->xcd_mixed, 1u);
+    __hip_atomic_store(&p.wg_xcc[wg], 0x80000000u | ((uint32_t)gi << 8) | my_xcc, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
   }
-  return cross;
+  if (!one_xcd_layout) return 1u;
+  bool elsewhere = false;
+  if (lane < p.G) {
+    const int peer = (((wg >> 3) / p.G * p.G + lane) << 3) | (wg & 7);
+    uint32_t w = 0;
+    long long spins = 0;
+    while (((w = __hip_atomic_load(&p.wg_xcc[peer], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) & 0x80000000u) == 0u) {
+      if (++spins >= spin_limit) {  // a peer never started: the grid is not co-resident
+        if (atomicExch(&p.status->aborted, 1u) == 0u) {
+          p.status->abort_wg = (uint32_t)wg;
+          p.status->abort_step = 0xFFFFFFFFu;
+        }
+        break;
+      }
+    }
+    elsewhere = (w & 0x80000000u) == 0u || (w & 0xFu) != my_xcc;
+  }
+  const bool cross = __builtin_amdgcn_ballot_w64(elsewhere) != 0ull;
+  if (cross && lane == 0) atomicAdd(&p.status->xcd_mixed, 1u);
+  return cross ? 1u : 0u;
 }
 
 // FULL: the head dim fills the K range of the four waves exactly (dh == 16 * NCH * elements per chunk) and, with
@@ -197,7 +198,10 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
   const int lane = tid & 63;
   const long long spin_limit = p.spin_limit > 0 ? p.spin_limit : kDefaultSpinLimit;
 
-  if (tid == 0) cross_s = seq_handshake(p, wg, gi, spin_limit);
+  if (tid < 64) {
+    const uint32_t verdict = seq_handshake(p, wg, gi, spin_limit);
+    if (tid == 0) cross_s = verdict;
+  }
 
   const int dh = p.dh;
   const int H = p.NH * dh;

@@ -85,7 +85,10 @@ __global__ __launch_bounds__(kRolesThreads) void slstm_seq_roles_kernel(SeqParam
   const int wave = (int)uniform((uint32_t)(tid >> 6));
   const int lane = tid & 63;
   const long long spin_limit = p.spin_limit > 0 ? p.spin_limit : kDefaultSpinLimit;
-  if (tid == 0) cross_s = seq_handshake(p, wg, gi, spin_limit);
+  if (tid < 64) {
+    const uint32_t verdict = seq_handshake(p, wg, gi, spin_limit);
+    if (tid == 0) cross_s = verdict;
+  }
 
   const int dh = p.dh;
   const int H = p.NH * dh;
