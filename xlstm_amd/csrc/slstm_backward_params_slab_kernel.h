@@ -16,7 +16,9 @@
 //
 // Bound: at NT 256 a chunk is 1,024 cycles of MFMA per SIMD, about as many of LDS (128 KiB read, 32 written), and 32 KiB from the L2 per compute unit.
 // Measured against the kernel it replaces: B 16 x T 512 x 4 heads of 1024 762 -> 357 us (0.77 PFLOP/s), B 16 x T 2048 x 4
-// heads of 256 229 -> 137 us (335 MB of operands, 0.50 PFLOP/s).
+// heads of 256 229 -> 137 us (335 MB of operands, 0.50 PFLOP/s); with chunks stepped by additions instead of 90 scalar instructions of products,
+// and asked for behind the MFMAs (alone, in a loop): 371 -> 355, 131 -> 125 us.  Of the 355 the requests with the barriers alone take 220, MFMAs and LDS
+// reads without memory 309: the eight waves of a compute unit do both in step, so the two add up where they should overlap.
 #pragma once
 
 namespace {
@@ -80,32 +82,42 @@ __global__ __launch_bounds__(512) void slstm_bwd_param_slab_kernel(BwdParamParam
     b_off[i] = b_col[i] >= 0 ? (uint32_t)((k * BH + yn) * 2) : kNone;
   }
   const uint32_t lds0 = (uint32_t)(unsigned long long)((__attribute__((address_space(3))) unsigned char *)slab_lds);
-  auto descriptor = [&](const void *base, uint32_t bytes) {
-    const unsigned long long v = reinterpret_cast<unsigned long long>(base);
-    return u32x4_t{uniform((uint32_t)v), uniform((uint32_t)(v >> 32) & 0xFFFFu), uniform(bytes), 0x00020000u};
+  // the next chunk to ask for: its place and what its descriptors cover, stepped with additions (nearly all chunks follow the last one in
+  // their batch row)
+  int f_left = c_hi - c_lo, f_b = c_lo / p.tchunks, f_t = c_lo % p.tchunks;
+  uint32_t f_dst = lds0;
+  const int tail = p.T - (p.tchunks - 1) * KC, bwidth = NT < dh - n0 ? NT : dh - n0;
+  const uint32_t a_step = (uint32_t)(KC * p.d_wx_st * 2), b_step = (uint32_t)(KC * BH * 2);
+  const uint32_t a_full = (uint32_t)(((KC - 1) * p.d_wx_st + 4ll * H) * 2), a_tail = (uint32_t)(((tail - 1) * p.d_wx_st + 4ll * H) * 2);
+  const uint32_t b_full = (uint32_t)(((KC - 1) * BH + bwidth) * 2), b_tail = (uint32_t)(((tail - 1) * BH + bwidth) * 2);
+  unsigned long long a_at = 0, b_at = 0, r_at = 0;
+  auto row_start = [&](int t) {
+    a_at = reinterpret_cast<unsigned long long>(p.d_wx) + ((long long)f_b * p.d_wx_sb + (long long)t * KC * p.d_wx_st) * 2;
+    b_at = reinterpret_cast<unsigned long long>(p.h_out) + (((long long)t * KC - 1) * BH + (long long)f_b * H + (long long)head * dh + n0) * 2;
+    r_at = p.reset ? reinterpret_cast<unsigned long long>(p.reset) + (long long)f_b * p.reset_sb + (long long)t * KC : 0;
   };
-  int f_chunk = c_lo, f_b = c_lo / p.tchunks, f_t = c_lo % p.tchunks, f_stage = 0;  // the next chunk to ask for
+  if (f_left > 0) row_start(f_t);
+  auto descriptor = [&](unsigned long long v, uint32_t bytes) { return u32x4_t{uniform((uint32_t)v), uniform((uint32_t)(v >> 32) & 0xFFFFu), uniform(bytes), 0x00020000u}; };
   auto request = [&]() {
-    const int t0 = f_t * KC;
-    const int nrows = f_chunk < c_hi ? (p.T - t0 < KC ? p.T - t0 : KC) : 0;
-    const int b = nrows ? f_b : 0, t = nrows ? t0 : 0;
-    const uint32_t dst = lds0 + (uint32_t)(f_stage * STAGE);
-    const u32x4_t ars = descriptor(reinterpret_cast<const uint16_t *>(reinterpret_cast<const void *>(p.d_wx)) + (long long)b * p.d_wx_sb + (long long)t * p.d_wx_st,
-                                   nrows ? (uint32_t)(((long long)(nrows - 1) * p.d_wx_st + 4ll * H) * 2) : 0u);
+    const bool there = f_left > 0, last = f_t == p.tchunks - 1;
+    const u32x4_t ars = descriptor(a_at, there ? (last ? a_tail : a_full) : 0u);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) bwd_fetch_to_lds_b128(ars, uniform(dst + (uint32_t)(wave * 1024 + 8192 * i)), a_off[i]);
+    for (int i = 0; i < 2; ++i) bwd_fetch_to_lds_b128(ars, uniform(f_dst + (uint32_t)(wave * 1024 + 8192 * i)), a_off[i]);
     // y_{t-1}: step t's operand is row t - 1 of the outputs (in front of step 0: nothing, see below)
-    const u32x4_t brs = descriptor(reinterpret_cast<const uint16_t *>(p.h_out) + ((long long)t - 1) * BH + (long long)b * H + (long long)head * dh + n0,
-                                   nrows ? (uint32_t)(((long long)(nrows - 1) * BH + (NT < dh - n0 ? NT : dh - n0)) * 2) : 0u);
+    const u32x4_t brs = descriptor(b_at, there ? (last ? b_tail : b_full) : 0u);
 #pragma unroll
     for (int i = 0; i < NB; ++i)
       if (lane < BLANES)
-        bwd_fetch_to_lds_b128(brs, uniform(dst + BOFF + (uint32_t)(wave * BLANES * 16 + 8192 * i)), t == 0 && b_row[i] == 0 ? kNone : b_off[i]);
-    const u32x4_t frs = descriptor(p.reset ? p.reset + (long long)b * p.reset_sb + t : reinterpret_cast<const uint8_t *>(p.d_wx), p.reset ? (uint32_t)nrows : 0u);
-    if (lane < 4) bwd_fetch_to_lds_u8(frs, uniform(dst + FOFF + (uint32_t)(wave * 16)), (uint32_t)(4 * wave + lane));
-    ++f_chunk;
-    if (++f_t == p.tchunks) { f_t = 0; ++f_b; }
-    if (++f_stage == S) f_stage = 0;
+        bwd_fetch_to_lds_b128(brs, uniform(f_dst + BOFF + (uint32_t)(wave * BLANES * 16 + 8192 * i)), f_t == 0 && b_row[i] == 0 ? kNone : b_off[i]);
+    const u32x4_t frs = descriptor(r_at, p.reset && there ? (uint32_t)(last ? tail : KC) : 0u);
+    if (lane < 4) bwd_fetch_to_lds_u8(frs, uniform(f_dst + FOFF + (uint32_t)(wave * 16)), (uint32_t)(4 * wave + lane));
+    --f_left;
+    a_at += a_step; b_at += b_step; r_at += KC;
+    if (++f_t == p.tchunks) {
+      f_t = 0; ++f_b;
+      row_start(0);
+    }
+    f_dst = f_dst == lds0 + (S - 1) * STAGE ? lds0 : f_dst + STAGE;
   };
 
   // ---- fragments: lane (q, r16) takes k = 8 q .. 8 q + 7 of column r16 of a 16 x 16 tile
@@ -163,8 +175,8 @@ __global__ __launch_bounds__(512) void slstm_bwd_param_slab_kernel(BwdParamParam
   for (int c = c_lo; c < c_hi; ++c) {
     asm volatile("s_waitcnt vmcnt(%0)" :: "n"((S - 2) * LOADS) : "memory");  // (this wave's part of chunk c has landed)
     lds_barrier();  // ... and everybody's; the stage of chunk c - 1 has been read
-    request();      // chunk c + S - 1, into that stage
     compute(stage, flags, counts);
+    request();      // chunk c + S - 1, into that stage, while the last MFMAs run (in front of them: 359 us where 355 now)
     if (++stage == S) stage = 0;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -1118,7 +1118,10 @@ int run_backward_params(const xs_slstm_bwd_args *a) {
     // shorter than four chunks
     const int cus = device_cus() > 0 ? device_cus() : 256;
     const long long base = (long long)a->NH * tiles;
-    long long ks = slab ? cus / base : (2ll * cus + base - 1) / base;  // (4 or 8 per compute unit: 10 to 30 % slower)
+    // (4 or 8 per compute unit: 10 to 30 % slower.  float32, where one per compute unit fills the device, one: half the atomics; a training call
+    // at B 16 T 256 4 x 256 787 -> 761 us, B 30 T 100 4 x 512 1318 -> 1293; where the tiles alone are more, two: B 101 T 10 16 x 136 820 with one,
+    // 759 with two)
+    long long ks = slab || (!bf16 && base <= cus) ? cus / base : (2ll * cus + base - 1) / base;
     if (ks < 1) ks = 1;
     // (head, slice) groups are dealt out over the XCDs, group i on XCD i % 8: a multiple of 8 of them keeps every XCD
     // busy (4 heads of 1024 are 512 tiles and one slice each by the rule above: four XCDs idle, twice the time)
