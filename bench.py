@@ -523,9 +523,20 @@ def phase_profile(device):
                         "barrier": round(float(st[4][2] / T))},
         "drainer wave": {"h to HBM": round(float(st[5][0] / T)), "barrier": round(float(st[5][1] / T))},
     }
-    # config 5 at a quarter of its length and config 3's prefill: slstm_seq_roles_kernel; per tile iteration (4 per step)
-    for label, (B, T, NH, dh) in (("config 5, T = 1024 (slstm_seq_roles_kernel<bf16,NCH=8,FULL>)", (64, 1024, 4, 1024)),
-                                  ("config 3 prefill, T = 128 (slstm_seq_roles_kernel<bf16,NCH=2,FULL>)", (256, 128, 8, 256))):
+    # config 5 at a quarter of its length: slstm_seq_pair_kernel; per tile iteration (2 per step)
+    B, T, NH, dh = 64, 1024, 4, 1024
+    st, ms = run(B, T, NH, dh, 0)
+    n = 2.0 * T
+    pnames = {7: "loop top", 0: "wait for the operand tile", 1: "arrival test, polls repeated", 2: "MFMAs, W.x, partial sums to LDS", 3: "barrier",
+              4: "sums + gating + request of the other tile", 5: "publish + re-arm + h + fetch of W.x"}
+    out["config 5, T = 1024 (slstm_seq_pair_kernel<MT=2,RT=16>), cycles per tile iteration, workgroup 0"] = {
+        "ms_per_call_with_stamps": ms,
+        "waves 0-3": {nm: [round(float(st[w][i] / n)) for w in range(4)] for i, nm in pnames.items()},
+        "sum": [round(float((st[w][:6].sum() + st[w][7]) / n)) for w in range(4)],
+        "polls repeated": [round(float(st[w][6] / n), 2) for w in range(4)],
+    }
+    # config 3's prefill: slstm_seq_roles_kernel; per tile iteration (4 per step)
+    for label, (B, T, NH, dh) in (("config 3 prefill, T = 128 (slstm_seq_roles_kernel<bf16,NCH=2,FULL>)", (256, 128, 8, 256)),):
         st, ms = run(B, T, NH, dh, 0)
         n = 4.0 * T
         mnames = ["loop top", "wait for the operand tile", "request next tile + arrival test", "mfma", "partial sums to LDS", "barrier"]
@@ -781,7 +792,7 @@ def main():
         c5 = bench_config(device, CONFIG5_NAME, 64, 4096, 4, 1024, True, 0, iters=max(1, min(args.steps, 5)))
         c5["roofline"] = {"bound": "mfma", "achieved": c5["tflops"], "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                           "frac": c5["tflops"] / MFMA_BF16_PEAK_TFLOPS, "traffic": None,
-                          "kernel": "slstm_seq_roles_kernel<bf16,NCH=8,FULL>",
+                          "kernel": "slstm_seq_pair_kernel<MT=2,RT=16>",
                           "algorithmic_flops_per_launch": 8.0 * 64 * 4096 * 4096 * 1024}
         print(json.dumps({"config5": c5}))
         return
@@ -864,7 +875,7 @@ def main():
         out["other_configs"] = [
             {"workload": c["workload"], "ms": c["ms"], "us_per_timestep": c["us_per_timestep"], "aborted": c["aborted"],
              "roofline": ({"bound": "mfma", "frac": c["tflops"] / MFMA_BF16_PEAK_TFLOPS, "achieved": c["tflops"], "unit": "TFLOP/s",
-                           "peak": MFMA_BF16_PEAK_TFLOPS, "kernel": "slstm_seq_roles_kernel<bf16,NCH=8,FULL>"} if c is c5 else
+                           "peak": MFMA_BF16_PEAK_TFLOPS, "kernel": "slstm_seq_pair_kernel<MT=2,RT=16>"} if c is c5 else
                           {"bound": "hbm", "frac": c["hbm_GBs"] / HBM_PEAK_GBS, "achieved": c["hbm_GBs"], "unit": "GB/s",
                            "peak": HBM_PEAK_GBS})}
             for c in (c1, c4, c5)]
