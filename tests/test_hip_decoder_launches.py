@@ -20,6 +20,12 @@ def test_direct_steps_and_replays_may_be_mixed(monkeypatch, B, NH, dh):
     decoders = [GraphedLayerDecoder(layer, B) for _ in range(2)]
     for dec in decoders:
         dec.load_state(ring, state)
+    first = None
+    if dh <= 512:  # (float32: PyTorch's convolution, products and norm around the cell, up to the cell's largest head)
+        plain = sLSTMLayer(layer.config).to(DEV).eval()
+        plain.load_state_dict(layer.state_dict())
+        with torch.no_grad():
+            first = plain.step(x[0].float(), conv_state=ring.float(), slstm_state=state.clone())[0]
     launch, launched = GraphedLayerDecoder._launch, []
     monkeypatch.setattr(GraphedLayerDecoder, "_launch", lambda self, t: launched.append(launch(self, t)) or launched[-1])
     replayed = decoders[0]
@@ -33,6 +39,8 @@ def test_direct_steps_and_replays_may_be_mixed(monkeypatch, B, NH, dh):
         monkeypatch.undo()
         monkeypatch.setattr(GraphedLayerDecoder, "_launch", lambda self, t: launched.append(launch(self, t)) or launched[-1])
         got = decoders[1].step(decoders[1].out if t == 6 else token)  # (t 6: the output fed back is read before it is written)
+        if t == 0 and first is not None:  # (the layer's bfloat16 kernels: 2e-2)
+            assert float((got.float() - first).norm() / first.norm()) < 2e-2
         assert torch.equal(got, want), t
         assert torch.equal(decoders[1].state()["slstm_state"], replayed.state()["slstm_state"]), t
         assert torch.equal(decoders[1].state()["conv_state"][0], replayed.state()["conv_state"][0]), t

@@ -1,5 +1,5 @@
-"""The sequence kernel with two workgroups per compute unit (``slstm_seq_pair_kernel``: bfloat16 heads of more than 512 units, 32 steps and
-more) at the sizes where it can go wrong: 33 workgroups per head and a last one half filled, row tiles of 4, 8 and 16 rows and two of
+"""The sequence kernel with two workgroups per compute unit (``slstm_seq_pair_kernel``: bfloat16 heads of more than 512 units, and smaller
+ones whose batch fills the device, 32 steps and more) at the sizes where it can go wrong: 33 workgroups per head and a last one half filled, row tiles of 4, 8 and 16 rows and two of
 16, batches that leave rows over, more heads and rows than one launch holds, numbers of steps around its round of four tiles.
 
 The same call in pieces of fewer than 32 steps runs in other kernels, which form every sum in the same order: the same bits."""
@@ -22,6 +22,9 @@ CASES = [
     (40, 64, 4, 1024, 32),    # two row tiles, the last with 8 rows
     (61, 67, 4, 1000, 32),    # ... a last workgroup with 8 units, a row tile with 13 rows
     (70, 65, 4, 528, 32),     # ... and a second launch of 6 rows
+    (61, 33, 4, 512, 16),     # head dims that fit an XCD at one workgroup per compute unit: one row tile in place of two
+    (115, 34, 4, 248, 16),    # ... a last workgroup with 8 units, two chunks of K per wave
+    (150, 65, 3, 328, 32),    # ... one launch in place of two
     (9, 36, 9, 536, 4),       # eight heads and one: two launches, the second in row tiles of 4
 ]
 
@@ -44,7 +47,7 @@ def test_same_bits_as_in_short_pieces(B, T, NH, dh, rows, masked):
     np.testing.assert_array_equal(s, state)
 
 
-@pytest.mark.parametrize("B,T,NH,dh", [(3, 33, 1, 520), (11, 32, 4, 1024), (41, 34, 3, 768), (70, 33, 4, 528)])
+@pytest.mark.parametrize("B,T,NH,dh", [(3, 33, 1, 520), (11, 32, 4, 1024), (41, 34, 3, 768), (70, 33, 4, 528), (70, 32, 4, 504), (130, 33, 12, 144)])
 def test_training_forward_leaves_the_same_coefficients(B, T, NH, dh):
     from xlstm_amd import functional as F
 

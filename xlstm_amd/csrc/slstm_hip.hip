@@ -528,21 +528,33 @@ std::mutex &launches_into(const void *workspace) {
   return mu[((uintptr_t)workspace >> 8) % 64];
 }
 
-SeqKernel pick_pair(int MT, int rows, bool coef) {
-  if (MT == 2) return coef ? slstm_seq_pair_kernel<2, 16, 2> : slstm_seq_pair_kernel<2, 16, 0>;
-  if (rows == 4) return coef ? slstm_seq_pair_kernel<1, 4, 2> : slstm_seq_pair_kernel<1, 4, 0>;
-  if (rows == 8) return coef ? slstm_seq_pair_kernel<1, 8, 2> : slstm_seq_pair_kernel<1, 8, 0>;
-  return coef ? slstm_seq_pair_kernel<1, 16, 2> : slstm_seq_pair_kernel<1, 16, 0>;
+template <int NCH>
+SeqKernel pick_pair_n(int MT, int rows, bool coef) {
+  if (MT == 2) return coef ? slstm_seq_pair_kernel<NCH, 2, 16, 2> : slstm_seq_pair_kernel<NCH, 2, 16, 0>;
+  if constexpr (NCH == 8) {  // (smaller heads come here with full tiles only)
+    if (rows == 4) return coef ? slstm_seq_pair_kernel<NCH, 1, 4, 2> : slstm_seq_pair_kernel<NCH, 1, 4, 0>;
+    if (rows == 8) return coef ? slstm_seq_pair_kernel<NCH, 1, 8, 2> : slstm_seq_pair_kernel<NCH, 1, 8, 0>;
+  }
+  return coef ? slstm_seq_pair_kernel<NCH, 1, 16, 2> : slstm_seq_pair_kernel<NCH, 1, 16, 0>;
+}
+SeqKernel pick_pair(int nch, int MT, int rows, bool coef) {
+  switch (nch) {
+    case 2: return pick_pair_n<2>(MT, rows, coef);
+    case 4: return pick_pair_n<4>(MT, rows, coef);
+    case 8: return pick_pair_n<8>(MT, rows, coef);
+    default: return nullptr;
+  }
 }
 
 // Do two workgroups of every form of slstm_seq_pair_kernel share a compute unit, as its placement needs?
 bool pair_resident() {
   static const bool resident = [] {
-    for (int form = 0; form < 8; ++form) {
-      const SeqKernel k = pick_pair(form >> 1 == 3 ? 2 : 1, 4 << (form >> 1), form & 1);
-      int n = 0;
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(k), kPairThreads, 0) != hipSuccess || n < 2) return false;
-    }
+    for (int nch = 2; nch <= 8; nch *= 2)
+      for (int form = 0; form < 8; ++form) {
+        const SeqKernel k = pick_pair(nch, form >> 1 == 3 ? 2 : 1, 4 << (form >> 1), form & 1);
+        int n = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(k), kPairThreads, 0) != hipSuccess || n < 2) return false;
+      }
     return true;
   }();
   return resident;
@@ -596,9 +608,20 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
   // hands: 4 heads of 1024, us a call, on XCD pairs / on one XCD: B 64 T 40 143 / 151, T 100 361 / 346, T 300 1016 / 937; B 16 T 17 68 / 76, T 40
   // 119 / 114, T 300 700 / 514; B 2 T 9 49 / 47; 4 x 768 B 64 T 40 161 / 137.  (A training forward takes one row tile per workgroup on XCD
   // pairs, four times the launches.)
-  const int pair_groups = 8 * (2 * cus_per_xcd / G), pair_heads = NH < pair_groups ? NH : pair_groups;
-  const bool pair = bf16 && G > 32 && pair_groups > 0 && offsets_fit &&
-                    T >= (train_coef || (B + 15) / 16 <= pair_groups / pair_heads ? 32 : 64) && pair_resident();
+  // Smaller heads, batches that fill the device with more than one row tile per workgroup at one workgroup per compute unit: two of them
+  // where that makes one row tile per workgroup of two, or fewer launches (T 300, us a call, one / two workgroups per compute unit: B 64 4 x 512
+  // 697 / 538, B 128 4 x 256 631 / 453, B 200 3 x 320 1291 / 749; but B 128 4 x 512, two row tiles of 16 in place of four, 671 / 761, B 256 8 x 256
+  // 1160 / 1390; T 20 the same, T 64 B 64 4 x 512 165 / 125), and in training, where a workgroup has one row tile otherwise (B 112 T 100 12 x 144
+  // 1222 / 1038 with the backward pass, B 64 T 100 4 x 512 845 / 802).
+  const int pair_groups = 8 * (2 * cus_per_xcd / G), row_tiles = (B + 15) / 16;
+  const int per_pair = pair_groups > 0 ? pair_groups / (NH < pair_groups ? NH : pair_groups) : 0;  // row tiles of a head at once
+  bool pair = bf16 && nch >= 2 && per_pair > 0 && offsets_fit && !a->coef_out && T >= (train_coef || row_tiles <= per_pair ? 32 : 64);
+  if (pair && G <= 32) {
+    const int groups = 8 * (cus_per_xcd / G), per_one = groups > 0 ? groups / (NH < groups ? NH : groups) : 0;
+    pair = per_one > 0 && row_tiles > per_one && (train_coef || row_tiles <= per_pair ||
+                                   (row_tiles + 2 * per_pair - 1) / (2 * per_pair) < (row_tiles + 4 * per_one - 1) / (4 * per_one));
+  }
+  pair = pair && pair_resident();
   const int span = pair ? 64 : 32;
   int capacity;  // head groups per launch
   if (pair) capacity = pair_groups;
@@ -634,7 +657,7 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
   // one size: where the first goes to that kernel, a last one of fewer heads may still come here.)
   if (MT < 4 && !a->coef_out && !train_coef && local_head(dh, bf16)) return dry ? XS_OK : run_local(a, nullptr, head0);
   int rows_per_wg = 16 * MT;
-  if (MT == 1) {  // spare compute units: smaller row tiles, smaller exchanges
+  if (MT == 1 && (!pair || nch == 8)) {  // spare compute units: smaller row tiles, smaller exchanges
     for (int r = 4; r < 16; r *= 2)
       if ((B + r - 1) / r <= max_groups_per_head) { rows_per_wg = r; break; }
   }
@@ -659,7 +682,7 @@ int run_forward(const xs_slstm_args *a, size_t *need = nullptr, uint32_t *abort_
     // row tiles of at most 4 rows: the compute waves split the columns by unit, not K (head groups on one XCD)
     const bool quad = MT == 1 && rows_per_wg == 4 && G <= 32;
     if (quad) kern = bf16 ? (full ? pick_quad<true, true>(nch) : pick_quad<true, false>(nch)) : (full ? pick_quad<false, true>(nch) : pick_quad<false, false>(nch));
-    if (pair) kern = pick_pair(MT, rows_per_wg, train_coef != nullptr);
+    if (pair) kern = pick_pair(nch, MT, rows_per_wg, train_coef != nullptr);
     else if (train_coef) kern = bf16 ? (full ? pick_train<true, true>(nch, quad, burst) : pick_train<true, false>(nch, quad, burst))
                                 : (full ? pick_train<false, true>(nch, quad, burst) : pick_train<false, false>(nch, quad, burst));
     if (a->coef_out) {  // a training forward: the same kernel, leaving the backward pass its coefficients

@@ -1,5 +1,5 @@
-// The persistent sequence kernel for heads of more than 512 units (bf16): two workgroups per compute unit, a head group on ONE
-// XCD.  Included by slstm_hip.hip only, after slstm_seq_kernel.h (same parameters, same exchange ring, same bits).
+// The persistent sequence kernel with two workgroups per compute unit (bf16): heads of more than 512 units, whose group it keeps on ONE
+// XCD, and batches of smaller heads that fill the device.  Included by slstm_hip.hip only, after slstm_seq_kernel.h (same parameters, same exchange ring, same bits).
 //
 // At 16 units a workgroup such a head has 33 to 64 members.  With one workgroup per compute unit they sit on an XCD pair, half of
 // every poll crosses the fabric between the two (the exchange alone: 1.72 us a step against 0.58 inside an XCD), and four
@@ -24,6 +24,9 @@
 // and more), B 32 3.35 -> 2.29, B 16 2.40 -> 1.87, B 1 1.91 -> 1.38; 4 x 768 B 64 3.78 -> 2.96, B 16 2.29 -> 1.71; training 3 x 768
 // B 200 T 52 87 -> 63 with the backward pass.
 //
+// Smaller heads (NCH 2 and 4: head dims 136 to 512) come here where two workgroups per compute unit make one row tile per workgroup of two, or
+// fewer launches; see the dispatch for both sides.
+//
 // Bound, at B 64 x 4 heads of 1024: a tile goes round once in two iterations of 3,500 cycles.  The compute unit's vector issue is busy for 2,000
 // of them (two workgroups' arrival tests, sums and gating), its matrix cores 1,024, its texture path 1,024 (64 KiB of operand).  The
 // later of two workgroups on a compute unit has no slack (300 arrival test, 900 MFMA, 850 sums and gating with the request, 650 stores and
@@ -35,15 +38,15 @@
 namespace {
 
 constexpr int kPairThreads = 256;
-template <int MT, int RT, int COEF>
+template <int NCH, int MT, int RT, int COEF>  // NCH: 16-byte chunks of an operand row per lane and wave
 __global__ __launch_bounds__(kPairThreads, 2) void slstm_seq_pair_kernel(SeqParams p) {
-  constexpr int NCH = 8;                 // 16-byte chunks of an operand row per lane and wave
   constexpr int KW = NCH * 32;           // input units per wave
   constexpr int PK = 16 / RT;            // chunks per load: the MFMA rows of batch rows that do not exist bring other chunks of those that do
   constexpr int NL = NCH / PK;           // loads per wave and tile
   constexpr int D = 4;                   // iterations W.x is fetched ahead
   static_assert(RT == 4 || RT == 8 || RT == 16, "rows of a tile");
   static_assert(MT == 1 || RT == 16, "two row tiles are of 16 rows");
+  static_assert(NCH % PK == 0, "whole loads");
   static_assert(D % MT == 0, "the ring of W.x turns over in whole steps");
   __shared__ float part[2][4][4][kTileFloats];  // [buffer][wave][gate][unit*stride + row]
   __shared__ __attribute__((aligned(16))) uint16_t wxt[4][16][16];  // [wave][row * 4 + gate][unit]
