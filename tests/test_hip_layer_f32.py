@@ -277,3 +277,30 @@ def test_what_wants_the_modules_one_by_one_gets_them():
     out.sum().backward()
     with pytest.raises(RuntimeError, match="second time"):
         out.sum().backward()
+
+
+@pytest.mark.parametrize("chain", ["state", "input", "tied"])
+def test_recorded_backward_of_calls_that_depend_on_the_layer(chain):
+    """A backward pass that is itself recorded, where x or the state of a call comes from an earlier call of the same layer, or one weight
+    serves two gates: every call's share is counted once."""
+    print("case layer create_graph", chain, flush=True)
+    layer = _layer(2, 64)
+    if chain == "tied":
+        layer.zgate.weight = layer.ogate.weight
+    x0, x1 = (torch.randn(2, 6, 128, device=DEV, requires_grad=True) for _ in range(2))
+    d = torch.randn(2, 6, 128, device=DEV)
+
+    def gradients(fused, create_graph):
+        layer.fused_pre_ops = fused
+        first, states = layer(x0, return_last_state=True)
+        out = layer(first) if chain == "input" else layer(x1, slstm_state=states["slstm_state"])
+        assert _one_node(out) is fused
+        leaves = [x0, x1, *layer.parameters()]
+        return torch.autograd.grad([first, out], leaves, [d, d], create_graph=create_graph, allow_unused=True)
+
+    want = gradients(False, False)
+    for got in (gradients(True, True), gradients(True, False)):
+        for a, b in zip(got, want):
+            assert (a is None) == (b is None)
+            if a is not None:  # (float32 on both sides: sums over dh units, then over 12 steps of a recurrence)
+                torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-4 * float(b.detach().abs().max()))

@@ -260,13 +260,17 @@ class sLSTMLayer(nn.Module):
 
     def _gradients_with_graph(self, inputs, reset_mask, d_y, d_state):
         """The gradients of a training call for a backward pass that is itself recorded: its operations once more with the
-        call's own tensors (x, convolution weight and bias, the gates', R, b, state), one by one."""
-        x, state = inputs[0], inputs[-1]
+        call's own tensors (x, convolution weight and bias, the gates', R, b, state), one by one.  They are taken at aliases
+        made here, one per place: x or the state may come from an earlier call of the same layer and a weight may stand
+        in two places, and a gradient taken at the tensors themselves would run on through those - a part that the
+        surrounding backward pass adds by itself."""
         names = ("conv1d.conv.weight", "conv1d.conv.bias", "fgate.weight", "igate.weight", "zgate.weight", "ogate.weight",
                  "slstm_cell._recurrent_kernel_", "slstm_cell._bias_")
-        params = {"layer." + n: t for n, t in zip(names, inputs[1:-1]) if t is not None}
         with torch.enable_grad():
-            y, new_state = torch.func.functional_call(_UpToTheCell(self), params, (x, state, reset_mask))
+            inputs = [None if t is None else t.view_as(t) for t in inputs]
+            x, state = inputs[0], inputs[-1]
+            params = {"layer." + n: t for n, t in zip(names, inputs[1:-1]) if t is not None}
+            y, new_state = torch.func.functional_call(_UpToTheCell(self), params, (x, state, reset_mask), tie_weights=False)
             pairs = [(o, g) for o, g in ((y, d_y), (new_state, d_state)) if g is not None]
             wanted = [t for t in inputs if t is not None and t.requires_grad]
             grads = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs], create_graph=True, allow_unused=True))
