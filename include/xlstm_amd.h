@@ -294,7 +294,7 @@ int xs_headwise_group_norm(const xs_norm_args *args);
  * of xs_causal_conv_silu, xs_headwise_gates and xs_slstm_step called one behind the other.  XS_ERR_UNSUPPORTED, with nothing launched,
  * where xs_layer_step_fits() is 0: those three are the faster way there.
  *   cell         as for xs_slstm_step with bf16 wx and r, a state (s0) and no mask; wx and its strides are not read
- *   x            [B,D] contiguous, not overlapping ring_out;  conv_state, conv_w, conv_b, ring_out (required) as for
+ *   x            [B,D] contiguous;  neither x nor conv_state may overlap ring_out, cell.h_out or cell.s_out;  conv_state, conv_w, conv_b, ring_out (required) as for
  *                xs_causal_conv_silu, K = 4;  gate_w as for xs_headwise_gates
  */
 typedef struct xs_layer_step_args {

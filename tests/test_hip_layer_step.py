@@ -96,5 +96,46 @@ def test_layer_step_refuses_what_its_parts_refuse():
     a.conv_w, a.K = w.data_ptr(), 3
     assert lib.xs_layer_step(ctypes.byref(a)) == -5 and not lib.xs_layer_step_fits(2, 2, 64, 3)  # three taps: its parts
     a.K = 4
+    # h_out or s_out in the memory of x or of the taps (rows of 2 x 128, taps of 3 x 128 each), at both ends
+    free, taps = torch.zeros(8, 2, 128, dtype=torch.bfloat16, device=DEV), torch.zeros(2, 3, 128, dtype=torch.bfloat16, device=DEV)
+    h, s_out, x = c.h_out, c.s_out, a.x
+    for moved in (dict(h=x), dict(h=x + 496), dict(x=s_out), dict(x=s_out + 16 * 256 - 16), dict(taps=h + 496), dict(taps=h - 3 * 512 + 16),
+                  dict(taps=s_out + 16 * 256 - 16)):
+        c.h_out, a.x, a.conv_state = moved.get("h", h), moved.get("x", x), moved.get("taps")
+        a.conv_state_stride_b = 0
+        assert lib.xs_layer_step(ctypes.byref(a)) == -2 and b"overlap" in lib.xs_last_error(), moved
+    c.h_out, a.x, a.conv_state = free[0].data_ptr(), free[1].data_ptr(), taps.data_ptr()  # next to each other
     assert lib.xs_layer_step(ctypes.byref(a)) == 0 and lib.xs_layer_step_fits(2, 2, 64, 4)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("shared", ["h over x", "state over x", "h over taps", "state over taps"])
+def test_buffers_that_share_memory_give_what_the_parts_give(shared):
+    """h_out or slstm_state_out in the memory of x or of the convolution's state: the convolution and the projections have read both before
+    the cell's step writes."""
+    from xlstm_amd.layer import sLSTMLayer, sLSTMLayerConfig
+
+    print("case layer step shared", shared, flush=True)
+    B, NH, dh = 48, 4, 256
+    D = NH * dh
+    torch.manual_seed(1)
+    layer = sLSTMLayer(sLSTMLayerConfig(embedding_dim=D, num_heads=NH, backend="hip", recurrent_weight_init="standard")).to(DEV).bfloat16().eval()
+    layer.slstm_cell.keep_state_fp32 = True
+    x, taps = torch.randn(B, 1, D, device=DEV).bfloat16(), torch.randn(B, 3, D, device=DEV).bfloat16()
+    state = torch.rand(4, B, D, device=DEV) + 0.5
+    memory = torch.zeros(16 * B * D, dtype=torch.uint8, device=DEV)  # (as large as a state)
+
+    def at(t):  # t's values at the start of that memory
+        v = memory[:t.numel() * t.element_size()].view(t.dtype).view(t.shape)
+        v.copy_(t)
+        return v
+
+    with torch.no_grad():
+        layer.slstm_cell.step(torch.zeros(B, 1, 4 * D, device=DEV, dtype=torch.bfloat16), state)  # (plans steps of B rows)
+        want, want_st = layer.step(x, conv_state=(taps,), slstm_state=state)
+        tokens, ring = (at(x), taps) if "x" in shared else (x, at(taps))
+        out = {"h_out": memory[:2 * B * D].view(torch.bfloat16).view(1, B, D)} if shared.startswith("h") else \
+              {"slstm_state_out": memory.view(torch.float32).view(4, B, D)}
+        got, got_st = layer.step(tokens, conv_state=(ring,), slstm_state=state, **out)
+    assert torch.equal(got, want) and torch.equal(got_st["slstm_state"], want_st["slstm_state"])
+    assert torch.equal(got_st["conv_state"][0], want_st["conv_state"][0])

@@ -359,6 +359,9 @@ struct Step {
   // wx: contiguous [B,1,4H]; everything else as step_fits has found it
   void run(const at::Tensor &wx, const at::Tensor &s0, const StepBuffers &s, const Shape4 *h_shape) {
     fill(wx.options(), s0, s, h_shape);
+    launch(wx);
+  }
+  void launch(const at::Tensor &wx) {
     a.wx = wx.data_ptr();
     launched(g_engine.step(&a));
   }
@@ -982,9 +985,9 @@ bool taps_of(const LayerParts &p, const at::Tensor &t, int64_t B, const void *&t
   return true;
 }
 
-bool overlap(const at::Tensor &a, const at::Tensor &b) {  // contiguous tensors
-  const char *pa = (const char *)a.data_ptr(), *pb = (const char *)b.data_ptr();
-  return pa < pb + b.nbytes() && pb < pa + a.nbytes();
+bool overlap(const void *a, int64_t a_bytes, const at::Tensor &b) {  // (b: contiguous)
+  const char *pa = (const char *)a, *pb = (const char *)b.data_ptr();
+  return a && pa < pb + b.nbytes() && pb < pa + a_bytes;
 }
 
 PyObject *states_dict(PyObject *conv_state, const at::Tensor &state) {
@@ -1034,8 +1037,13 @@ PyObject *layer_step_(PyObject *const *args) {
     void *stream = stream_of(x.device());
     ring = ring_out ? *ring_out : at::empty({B, p.K, p.D}, opts);
     out = out_given ? *out_given : at::empty({B, 1, p.D}, opts);
-    if (g_engine.own_parts && g_engine.layer_step_fits((int32_t)B, (int32_t)p.NH, (int32_t)p.dh, (int32_t)p.K) && !overlap(x, ring)) {
-      step.fill(opts, state, buffers, nullptr);
+    step.fill(opts, state, buffers, nullptr);
+    // (one kernel: its workgroups read a head's inputs while others write their units' results.  The parts have read x and the
+    // taps before the step writes h and the state, so buffers that share memory go to them)
+    const int64_t taps_bytes = taps ? 2 * ((B - 1) * taps_stride + (p.K - 1) * p.D) : 0;
+    const bool shared = overlap(x.data_ptr(), x.nbytes(), ring) || overlap(x.data_ptr(), x.nbytes(), step.h) || overlap(x.data_ptr(), x.nbytes(), step.state) ||
+                        overlap(taps, taps_bytes, step.h) || overlap(taps, taps_bytes, step.state);
+    if (g_engine.own_parts && !shared && g_engine.layer_step_fits((int32_t)B, (int32_t)p.NH, (int32_t)p.dh, (int32_t)p.K)) {
       xs_layer_step_args a{};
       a.cell = step.a;
       a.x = x.data_ptr();
@@ -1048,7 +1056,7 @@ PyObject *layer_step_(PyObject *const *args) {
       at::Tensor wx = at::empty({B, 1, 4 * p.D}, opts), x_conv = at::empty({B, 1, p.D}, opts);
       run_conv(p, x, taps, taps_stride, nullptr, x_conv.data_ptr(), ring.data_ptr(), stream);
       run_gates(p, x, x_conv.data_ptr(), wx.data_ptr(), stream);
-      step.run(wx, state, buffers, nullptr);
+      step.launch(wx);
     }
     run_norm(p, step.h, B, 1, out.data_ptr(), stream);
     state_out = p.keep_state ? step.state : step.state.to(at::kBFloat16);

@@ -1386,8 +1386,13 @@ int run_layer_step(const xs_layer_step_args *a) {
   for (int g = 0; g < 4; ++g) gates.w[g] = a->gate_w[g];
   gates.out = a->ring_out; gates.out_stride_row = 4 * D;
   if ((rc = check_conv(&conv)) != XS_OK || (rc = check_gates(&gates)) != XS_OK) return rc;
-  const uintptr_t x0 = (uintptr_t)a->x, r0 = (uintptr_t)a->ring_out, nx = (uintptr_t)B * D * 2;
-  if (x0 < r0 + 4 * nx && r0 < x0 + nx) return fail(XS_ERR_SHAPE, "ring_out must not overlap x");  // (other workgroups still read it)
+  // other workgroups of a head still read its x and its taps while the first ones write
+  const long long row = D * 2, taps_sb = a->conv_state_stride_b ? a->conv_state_stride_b * 2 : 3 * row;
+  const struct { const char *name; const void *p; long long bytes; } in[2] = {{"x", a->x, B * row}, {"conv_state", a->conv_state, a->conv_state ? (B - 1) * taps_sb + 3 * row : 0}},
+      out[3] = {{"ring_out", a->ring_out, 4 * B * row}, {"h_out", cell.h_out, B * row}, {"s_out", cell.s_out, 8 * B * row}};
+  for (const auto &i : in)
+    for (const auto &o : out)
+      if ((uintptr_t)i.p < (uintptr_t)o.p + o.bytes && (uintptr_t)o.p < (uintptr_t)i.p + i.bytes) return fail(XS_ERR_SHAPE, "%s must not overlap %s", o.name, i.name);
   LayerStepParams p;
   p.step = step_params(&cell);
   p.step.n_unit_tiles = dh / (16 * split.ut);
