@@ -258,3 +258,38 @@ def test_layer_ops_accept_empty_inputs():
     assert tuple(hipF.headwise_gates(e, e, ws, 1).shape) == (0, 3, 256)
     assert tuple(hipF.headwise_group_norm(torch.zeros(2, 1, 0, 64, dtype=torch.bfloat16, device=DEV)).shape) == (2, 0, 64)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T", [1, 2, 7])
+def test_gradient_of_the_inputs_before_x(dtype, T):
+    """A layer whose parameters are frozen: the convolution's state and the cell's may still want their gradients."""
+    from xlstm_amd.layer import sLSTMLayer, sLSTMLayerConfig
+
+    print("case conv_state gradient", dtype, T, flush=True)
+    torch.manual_seed(T)
+    layer = sLSTMLayer(sLSTMLayerConfig(embedding_dim=128, num_heads=2, backend="hip", recurrent_weight_init="standard")).to(DEV).to(dtype)
+    layer.requires_grad_(False)
+    x = torch.randn(3, T, 128, device=DEV).to(dtype)
+    before = torch.randn(3, 3, 128, device=DEV).to(dtype).requires_grad_(True)
+    state = (torch.rand(4, 3, 128, device=DEV) + 0.5).to(dtype).requires_grad_(True)
+    d = torch.randn(3, T, 128, device=DEV).to(dtype)
+    buffer = torch.empty(3, 1, 128, device=DEV, dtype=dtype)
+    with torch.no_grad():  # (plans steps of 3 rows, so that the native host path is asked)
+        layer.step(x[:, :1].contiguous(), (before,), state.float())
+
+    def call(wanted):
+        ring, s = (t if any(t is w for w in wanted) else t.detach() for t in (before, state))
+        return layer.step(x, (ring,), s.float(), out=buffer)[0] if T == 1 else layer(x, conv_state=ring, slstm_state=s)
+
+    for wanted in ((before,), (state,), (before, state)):
+        got = torch.autograd.grad(call(wanted), wanted, d)
+        layer.fused_pre_ops = False
+        want = torch.autograd.grad(call(wanted), wanted, d)
+        layer.fused_pre_ops = True
+        for a, b in zip(got, want):
+            assert a.shape == b.shape and float(b.float().norm()) > 0
+            # Where the state alone wants one, the engine's kernels run in front of the cell on one side and PyTorch's on the other.  bfloat16:
+            # each of about ten operations rounds to 8 bits, 2^-9 each at worst; float32: sums of 64 products, 2^-24 a term
+            bound = 10 * 2.0 ** -9 if dtype == torch.bfloat16 else 10 * 64 * 2.0 ** -24
+            assert float((a.float() - b.float()).norm() / b.float().norm()) <= bound

@@ -973,6 +973,9 @@ xs_layer_args float32_args(const LayerParts &p, const at::Tensor &x, const at::T
   return a;
 }
 
+// (the kernels around the cell record no graph in inference calls)
+bool wants_gradient(const at::Tensor &t) { return at::GradMode::is_enabled() && t.requires_grad(); }
+
 // the taps in front of the first token: a [B,n,D] tensor of which the last K-1 inputs count
 bool taps_of(const LayerParts &p, const at::Tensor &t, int64_t B, const void *&taps, int64_t &stride) {
   const int64_t n = t.dim() == 3 ? t.size(1) : 0;
@@ -1021,7 +1024,7 @@ PyObject *layer_step_(PyObject *const *args) {
   PyObject *prev = absent(args[3]) ? nullptr : first_of(args[3]);
   if (!absent(prev)) {
     const at::Tensor *t = tensor_of(prev);
-    if (!t || t->dim() != 3 || (t->size(1) != p.K && t->size(1) != p.K - 1) || !taps_of(p, *t, B, taps, taps_stride)) Py_RETURN_NONE;  // (the general path asserts)
+    if (!t || wants_gradient(*t) || t->dim() != 3 || (t->size(1) != p.K && t->size(1) != p.K - 1) || !taps_of(p, *t, B, taps, taps_stride)) Py_RETURN_NONE;  // (the general path asserts)
     before = *t;
   }
   const auto opts = x.options();
@@ -1084,7 +1087,7 @@ PyObject *layer_forward_(PyObject *const *args) {
   PyObject *prev = absent(args[3]) ? nullptr : first_of(args[3]);
   if (!absent(prev)) {
     const at::Tensor *t = tensor_of(prev);
-    if (!t || !taps_of(p, *t, B, taps, taps_stride)) Py_RETURN_NONE;
+    if (!t || wants_gradient(*t) || !taps_of(p, *t, B, taps, taps_stride)) Py_RETURN_NONE;
     before = *t;
   }
   const bool last = args[5] == Py_True;

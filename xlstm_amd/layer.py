@@ -209,7 +209,7 @@ class sLSTMLayer(nn.Module):
 
     def _gates(self, x, x_conv):
         # the module named fgate feeds the i slot, igate the f slot (layer.py:144-149)
-        if self._fused(x):
+        if self._fused(x) and not (torch.is_grad_enabled() and x_conv.requires_grad):
             return hipF.headwise_gates(x, x_conv, (self.fgate.weight, self.igate.weight, self.zgate.weight, self.ogate.weight),
                                        self.config.num_heads)
         return torch.cat([self.fgate(x_conv), self.igate(x_conv), self.zgate(x), self.ogate(x)], dim=-1)
@@ -276,14 +276,15 @@ class sLSTMLayer(nn.Module):
             grads = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs], create_graph=True, allow_unused=True))
         return tuple(next(grads) if t is not None and t.requires_grad else None for t in inputs)
 
-    def _engine_ops_allowed(self, t) -> bool:
-        # the engine's kernels record no autograd graph: under grad mode the PyTorch ops run, and a backward pass
-        # reaches the cell, which raises (inference engine)
+    def _engine_ops_allowed(self, t, conv_state=None) -> bool:
+        # the engine's kernels record no autograd graph: where a gradient is wanted, of the inputs before x as well, the PyTorch
+        # ops run around the cell
         return self.fused_pre_ops and t.is_cuda and t.dtype == torch.bfloat16 and not (
-            torch.is_grad_enabled() and (t.requires_grad or any(q.requires_grad for q in self.parameters())))
+            torch.is_grad_enabled() and (t.requires_grad or (conv_state is not None and conv_state.requires_grad)
+                                         or any(q.requires_grad for q in self.parameters())))
 
-    def _fused(self, x) -> bool:
-        return (self._engine_ops_allowed(x) and self.fgate.weight.dtype == torch.bfloat16
+    def _fused(self, x, conv_state=None) -> bool:
+        return (self._engine_ops_allowed(x, conv_state) and self.fgate.weight.dtype == torch.bfloat16
                 and hipF.fused_layer_ops_supported(x, self.config.num_heads, self.config.conv1d_kernel_size))
 
     def forward(self, x: torch.Tensor, conv_state: Optional[torch.Tensor] = None,
@@ -310,7 +311,7 @@ class sLSTMLayer(nn.Module):
         B, S, _ = x.shape
         if isinstance(conv_state, (tuple, list)):  # the ring a step returned (conv.py:131-157): oldest input first
             conv_state = conv_state[0]
-        if self.config.conv1d_kernel_size > 0 and self._fused(x):
+        if self.config.conv1d_kernel_size > 0 and self._fused(x, conv_state):
             conv = self.conv1d.conv
             pad = self.conv1d.pad
             taps = conv_state
@@ -350,11 +351,11 @@ class sLSTMLayer(nn.Module):
                 cell._rt.last_workspace = cell._rt.step_plan[1].workspace
                 return fast
         B, S, _ = x.shape
-        fused = self._fused(x)
+        prev = conv_state[0] if isinstance(conv_state, (tuple, list)) else conv_state
+        fused = self._fused(x, prev)
         if self.config.conv1d_kernel_size > 0 and fused:
             conv = self.conv1d.conv
             k = self.config.conv1d_kernel_size
-            prev = conv_state[0] if isinstance(conv_state, (tuple, list)) else conv_state
             if prev is not None:
                 assert prev.shape[1] in (k, k - 1), f"conv state holds {prev.shape[1]} inputs, expected {k} or {k - 1}"
                 if prev.shape[1] == k:
@@ -370,7 +371,7 @@ class sLSTMLayer(nn.Module):
         y, slstm_state = self.slstm_cell.step(self._gates(x, x_conv), slstm_state, state_out=slstm_state_out,
                                               h_out=h_out, h_prev=h_prev)
         y = self.dropout(y)
-        if fused and out is not None:
+        if fused and out is not None and self._engine_ops_allowed(y):
             out = hipF.headwise_group_norm(y, self.group_norm.weight, self.group_norm.eps, out=out)
         else:
             out = self._norm(y, B, S)
