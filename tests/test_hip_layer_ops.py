@@ -293,3 +293,26 @@ def test_gradient_of_the_inputs_before_x(dtype, T):
             # each of about ten operations rounds to 8 bits, 2^-9 each at worst; float32: sums of 64 products, 2^-24 a term
             bound = 10 * 2.0 ** -9 if dtype == torch.bfloat16 else 10 * 64 * 2.0 ** -24
             assert float((a.float() - b.float()).norm() / b.float().norm()) <= bound
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_a_norm_without_weights_takes_the_native_host_path(dtype):
+    from xlstm_amd import _lib
+    from xlstm_amd.layer import sLSTMLayer, sLSTMLayerConfig
+
+    print("case norm without weights", dtype, flush=True)
+    torch.manual_seed(0)
+    layer = sLSTMLayer(sLSTMLayerConfig(embedding_dim=128, num_heads=2, backend="hip", group_norm_weight=False, recurrent_weight_init="standard"))
+    layer = layer.to(DEV).to(dtype).eval()
+    assert layer.group_norm.weight is None and "group_norm.weight" not in layer.state_dict()
+    layer.slstm_cell.keep_state_fp32 = True
+    x = torch.randn(3, 6, 128, device=DEV).to(dtype)
+    with torch.no_grad():
+        want, states = layer(x, return_last_state=True)
+        got = _lib.host().layer_forward(layer, layer.slstm_cell._native(), x, None, None, False, None)
+        assert got is not None and torch.equal(got, want)
+        if dtype == torch.bfloat16:  # (a float32 layer's step is not one of the native path's)
+            token = x[:, :1].contiguous()
+            want, want_states = layer.step(token, (states["conv_state"],), states["slstm_state"])  # (plans steps of 3 rows)
+            got = _lib.host().layer_step(layer, layer.slstm_cell._native(), token, states["conv_state"], states["slstm_state"], *5 * [None])
+            assert got is not None and torch.equal(got[0], want) and torch.equal(got[1]["slstm_state"], want_states["slstm_state"])

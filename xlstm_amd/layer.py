@@ -145,7 +145,7 @@ class MultiHeadLayerNorm(nn.Module):
 
     def __init__(self, ndim: int, weight: bool = True, eps: float = 1e-5):
         super().__init__()
-        self.weight = nn.Parameter(torch.zeros(ndim)) if weight else None
+        self.register_parameter("weight", nn.Parameter(torch.zeros(ndim)) if weight else None)  # (None: the native host path looks here)
         self.eps = eps
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
