@@ -20,7 +20,7 @@
 extern "C" {
 #endif
 
-#define XS_ABI_VERSION 19
+#define XS_ABI_VERSION 20
 
 /* element types */
 enum { XS_F32 = 0, XS_BF16 = 1 };
@@ -296,6 +296,7 @@ int xs_headwise_group_norm(const xs_norm_args *args);
  *   cell         as for xs_slstm_step with bf16 wx and r, a state (s0) and no mask; wx and its strides are not read
  *   x            [B,D] contiguous;  neither x nor conv_state may overlap ring_out, cell.h_out or cell.s_out;  conv_state, conv_w, conv_b, ring_out (required) as for
  *                xs_causal_conv_silu, K = 4;  gate_w as for xs_headwise_gates
+ *   x_out        x once more ([B,D] contiguous, overlapping no other operand), or NULL
  */
 typedef struct xs_layer_step_args {
   xs_slstm_args cell;
@@ -304,6 +305,7 @@ typedef struct xs_layer_step_args {
   int64_t conv_state_stride_b;
   const void *conv_w, *conv_b;
   void *ring_out;
+  void *x_out;
   const void *gate_w[4];
   int32_t K;
 } xs_layer_step_args;

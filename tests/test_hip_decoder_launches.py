@@ -53,3 +53,31 @@ def test_direct_steps_and_replays_may_be_mixed(monkeypatch, B, NH, dh):
     got, want = decoders[1].step(x[0]), decoders[0].step(x[0])
     handle.remove()
     assert not launched[-1] and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("B,NH,dh", [(3, 2, 64), (600, 2, 128), (70, 4, 256), (33, 2, 1024)])
+def test_the_token_is_in_the_decoders_buffer(B, NH, dh):
+    """``step(x)`` leaves the token in ``dec.x``: whoever holds that buffer reads it there, and ``step()`` behind it takes it
+    once more."""
+    from xlstm_amd.decode import GraphedLayerDecoder
+    from xlstm_amd.layer import sLSTMLayer, sLSTMLayerConfig
+
+    print("case decoder token", B, NH, dh, flush=True)
+    D = NH * dh
+    torch.manual_seed(B)
+    layer = sLSTMLayer(sLSTMLayerConfig(embedding_dim=D, num_heads=NH, backend="hip", recurrent_weight_init="standard")).to(DEV).bfloat16().eval()
+    x = torch.randn(3, B, 1, D, device=DEV).bfloat16()
+    dec, twice = GraphedLayerDecoder(layer, B), GraphedLayerDecoder(layer, B)
+    held = dec.x
+    for token in (x[0], x[1], x[2].float()):
+        got = dec.step(token).clone()
+        assert torch.equal(held, token.bfloat16()) and dec.x is held
+        assert torch.equal(got, twice.step(token))
+        got = dec.step().clone()
+        assert torch.equal(got, twice.step(token))
+        assert torch.equal(held, token.bfloat16())
+    held[:2].copy_(x[0][:2])  # (its producer writes a part of it)
+    mixed = held.clone()
+    assert torch.equal(dec.step(), twice.step(mixed))
+    assert torch.equal(dec.step(x[1][:1]), twice.step(x[1][:1].expand(B, 1, D)))  # (one token for all rows)
+    assert torch.equal(held, x[1][:1].expand(B, 1, D))

@@ -105,8 +105,14 @@ def test_layer_step_refuses_what_its_parts_refuse():
         a.conv_state_stride_b = 0
         assert lib.xs_layer_step(ctypes.byref(a)) == -2 and b"overlap" in lib.xs_last_error(), moved
     c.h_out, a.x, a.conv_state = free[0].data_ptr(), free[1].data_ptr(), taps.data_ptr()  # next to each other
+    for at, error in ((a.x + 496, -2), (taps.data_ptr() + 3 * 512 - 16, -2), (free[2].data_ptr() + 8, -4)):
+        a.x_out = at
+        assert lib.xs_layer_step(ctypes.byref(a)) == error
+    a.x_out = free[2].data_ptr()
+    free[1].fill_(3.0)
     assert lib.xs_layer_step(ctypes.byref(a)) == 0 and lib.xs_layer_step_fits(2, 2, 64, 4)
     torch.cuda.synchronize()
+    assert torch.equal(free[2], free[1]) and not free[3].any()
 
 
 @pytest.mark.parametrize("shared", ["h over x", "state over x", "h over taps", "state over taps"])

@@ -17,7 +17,7 @@ LIB_PATH = os.environ.get("XLSTM_AMD_LIB", os.path.join(PKG, "lib", "libxlstm_am
 XS_F32, XS_BF16 = 0, 1
 XS_ERR_UNSUPPORTED = -5
 STATIC_SCRATCH_BYTES = (4 << 20) + (64 << 10)
-ABI_VERSION = 19
+ABI_VERSION = 20
 
 EXPORTS = (
     "xs_abi_version",
@@ -172,6 +172,7 @@ class LayerStepArgs(ctypes.Structure):
         ("conv_w", ctypes.c_void_p),
         ("conv_b", ctypes.c_void_p),
         ("ring_out", ctypes.c_void_p),
+        ("x_out", ctypes.c_void_p),
         ("gate_w", ctypes.c_void_p * 4),
         ("K", ctypes.c_int32),
     ]

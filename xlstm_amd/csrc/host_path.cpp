@@ -1004,14 +1004,14 @@ PyObject *first_of(PyObject *o) {  // a state that may come in a tuple or list o
   return o;
 }
 
-// layer_step(layer, cell path, x, conv_state, slstm_state, slstm_state_out, conv_state_out, h_out, h_prev, out)
-//   -> (out, {"conv_state": (ring,), "slstm_state": state}) or None
+// layer_step(layer, cell path, x, conv_state, slstm_state, slstm_state_out, conv_state_out, h_out, h_prev, out[, x_out])
+//   -> (out, {"conv_state": (ring,), "slstm_state": state}) or None.  x_out: a buffer that x is left in as well
 PyObject *layer_step_(PyObject *const *args) {
-  const at::Tensor *xp = tensor_of(args[2]), *statep = tensor_of(args[4]), *ring_out, *out_given;
+  const at::Tensor *xp = tensor_of(args[2]), *statep = tensor_of(args[4]), *ring_out, *out_given, *x_out;
   CellPath &c = *((CellPathObject *)args[1])->c;
   StepBuffers buffers;
   if (!xp || !statep || !c.plan || !step_buffers(args[5], args[7], args[8], buffers) || !optional_tensor(args[6], ring_out) ||
-      !optional_tensor(args[9], out_given))
+      !optional_tensor(args[9], out_given) || !optional_tensor(args[10], x_out))
     Py_RETURN_NONE;
   const at::Tensor &x = *xp, &state = *statep;
   LayerParts p;
@@ -1032,6 +1032,10 @@ PyObject *layer_step_(PyObject *const *args) {
                    ring_out->size(2) != p.D || !ring_out->is_contiguous()))
     Py_RETURN_NONE;
   if (out_given && (out_given->scalar_type() != at::kBFloat16 || out_given->numel() != B * p.D || !out_given->is_contiguous())) Py_RETURN_NONE;
+  if (x_out && x_out->data_ptr() == x.data_ptr()) x_out = nullptr;
+  if (x_out && (x_out->scalar_type() != at::kBFloat16 || x_out->sizes() != x.sizes() || !x_out->is_contiguous() || x_out->device() != x.device() ||
+                !aligned(x_out->data_ptr(), 16) || overlap(x.data_ptr(), x.nbytes(), *x_out)))
+    Py_RETURN_NONE;
   c10::OptionalDeviceGuard guard(x.device());
   Step step(c);
   at::Tensor ring, out, state_out;
@@ -1045,14 +1049,14 @@ PyObject *layer_step_(PyObject *const *args) {
     // taps before the step writes h and the state, so buffers that share memory go to them)
     const int64_t taps_bytes = taps ? 2 * ((B - 1) * taps_stride + (p.K - 1) * p.D) : 0;
     const bool shared = overlap(x.data_ptr(), x.nbytes(), ring) || overlap(x.data_ptr(), x.nbytes(), step.h) || overlap(x.data_ptr(), x.nbytes(), step.state) ||
-                        overlap(taps, taps_bytes, step.h) || overlap(taps, taps_bytes, step.state);
+                        overlap(taps, taps_bytes, step.h) || overlap(taps, taps_bytes, step.state) || (x_out && overlap(taps, taps_bytes, *x_out));
     if (g_engine.own_parts && !shared && g_engine.layer_step_fits((int32_t)B, (int32_t)p.NH, (int32_t)p.dh, (int32_t)p.K)) {
       xs_layer_step_args a{};
       a.cell = step.a;
       a.x = x.data_ptr();
       a.conv_state = taps; a.conv_state_stride_b = taps && B > 1 ? taps_stride : 0;
       a.conv_w = p.conv_w.data_ptr(); a.conv_b = p.conv_b.defined() ? p.conv_b.data_ptr() : nullptr;
-      a.ring_out = ring.data_ptr(); a.K = (int32_t)p.K;
+      a.ring_out = ring.data_ptr(); a.x_out = x_out ? x_out->data_ptr() : nullptr; a.K = (int32_t)p.K;
       for (int g = 0; g < 4; ++g) a.gate_w[g] = p.gate[g].data_ptr();
       launched(g_engine.layer_step(&a));
     } else {
@@ -1060,6 +1064,10 @@ PyObject *layer_step_(PyObject *const *args) {
       run_conv(p, x, taps, taps_stride, nullptr, x_conv.data_ptr(), ring.data_ptr(), stream);
       run_gates(p, x, x_conv.data_ptr(), wx.data_ptr(), stream);
       step.launch(wx);
+      if (x_out) {
+        at::NoGradGuard no_grad;
+        x_out->copy_(x);
+      }
     }
     run_norm(p, step.h, B, 1, out.data_ptr(), stream);
     state_out = p.keep_state ? step.state : step.state.to(at::kBFloat16);
@@ -1320,9 +1328,11 @@ PyObject *layer_train_(PyObject *const *args) {
   return PyTuple_Pack(2, ph.o, ps.o);
 }
 
-template <PyObject *(*F)(PyObject *const *), int N>
-PyObject *layer_call(PyObject *, PyObject *const *args, Py_ssize_t n) {
-  if (n != N) { PyErr_Format(PyExc_TypeError, "%d arguments expected, got %zd", N, n); return nullptr; }
+template <PyObject *(*F)(PyObject *const *), int N, int OPTIONAL = 0>
+PyObject *layer_call(PyObject *, PyObject *const *given, Py_ssize_t n) {
+  if (n < N || n > N + OPTIONAL) { PyErr_Format(PyExc_TypeError, "%d arguments expected, got %zd", N, n); return nullptr; }
+  PyObject *args[N + OPTIONAL] = {};  // (what is not given: null)
+  std::copy(given, given + n, args);
   if (!PyObject_TypeCheck(args[1], g_cell_type)) Py_RETURN_NONE;
   try {
     return F(args);
@@ -1388,7 +1398,7 @@ PyMethodDef module_methods[] = {
     {"bind", (PyCFunction)(void *)bind, METH_FASTCALL, nullptr},
     {"keep", (PyCFunction)(void *)keep, METH_FASTCALL, nullptr},
     {"kept", (PyCFunction)(void *)kept, METH_FASTCALL, nullptr},
-    {"layer_step", (PyCFunction)(void *)layer_call<layer_step_, 10>, METH_FASTCALL, nullptr},
+    {"layer_step", (PyCFunction)(void *)layer_call<layer_step_, 10, 1>, METH_FASTCALL, nullptr},
     {"layer_forward", (PyCFunction)(void *)layer_call<layer_forward_, 7>, METH_FASTCALL, nullptr},
     {"layer_train", (PyCFunction)(void *)layer_call<layer_train_, 6>, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};

@@ -1386,10 +1386,11 @@ int run_layer_step(const xs_layer_step_args *a) {
   for (int g = 0; g < 4; ++g) gates.w[g] = a->gate_w[g];
   gates.out = a->ring_out; gates.out_stride_row = 4 * D;
   if ((rc = check_conv(&conv)) != XS_OK || (rc = check_gates(&gates)) != XS_OK) return rc;
+  if ((uintptr_t)a->x_out % 16) return fail(XS_ERR_ALIGN, "x_out must be 16-byte aligned");
   // other workgroups of a head still read its x and its taps while the first ones write
   const long long row = D * 2, taps_sb = a->conv_state_stride_b ? a->conv_state_stride_b * 2 : 3 * row;
   const struct { const char *name; const void *p; long long bytes; } in[2] = {{"x", a->x, B * row}, {"conv_state", a->conv_state, a->conv_state ? (B - 1) * taps_sb + 3 * row : 0}},
-      out[3] = {{"ring_out", a->ring_out, 4 * B * row}, {"h_out", cell.h_out, B * row}, {"s_out", cell.s_out, 8 * B * row}};
+      out[4] = {{"ring_out", a->ring_out, 4 * B * row}, {"h_out", cell.h_out, B * row}, {"s_out", cell.s_out, 8 * B * row}, {"x_out", a->x_out, a->x_out ? B * row : 0}};
   for (const auto &i : in)
     for (const auto &o : out)
       if ((uintptr_t)i.p < (uintptr_t)o.p + o.bytes && (uintptr_t)o.p < (uintptr_t)i.p + i.bytes) return fail(XS_ERR_SHAPE, "%s must not overlap %s", o.name, i.name);
@@ -1404,7 +1405,7 @@ int run_layer_step(const xs_layer_step_args *a) {
   p.state_sb = a->conv_state_stride_b ? a->conv_state_stride_b : 3 * D;
   p.conv_w = (const uint16_t *)a->conv_w; p.conv_b = (const uint16_t *)a->conv_b;
   for (int g = 0; g < 4; ++g) p.gate_w[g] = (const uint16_t *)a->gate_w[g];
-  p.ring_out = (uint16_t *)a->ring_out;
+  p.ring_out = (uint16_t *)a->ring_out; p.x_out = (uint16_t *)a->x_out;
   const LayerStepKernel kern = cell.h_prev ? pick_layer_step<true>(split.nch, split.ut, split.loop) : pick_layer_step<false>(split.nch, split.ut, split.loop);
   const size_t lds = (size_t)layer_step_lds_bytes(split.nch);
   if (lds + 25600 * split.ut > 64 * 1024 && (rc = ensure_dynamic_lds(reinterpret_cast<const void *>(kern), lds)) != XS_OK) return rc;

@@ -13,6 +13,7 @@ struct LayerStepParams {
   const uint16_t *conv_b;   // [D] or null
   const uint16_t *gate_w[4];  // each [NH, dh, dh]
   uint16_t *ring_out;       // [B, 4, D]: the inputs before x, then x
+  uint16_t *x_out;          // [B, D]: x, or null
   int row_tiles;            // of the batch; step.n_row_tiles: of the grid, a workgroup takes every n_row_tiles-th
 };
 
@@ -145,6 +146,7 @@ __global__ __launch_bounds__(256 * UT, UT == 2 ? (NQ == 1 && !LOOP ? 4 : 2) : (N
           uint16_t *ring = p.ring_out + (long long)(row0 + r16) * 4 * H + head * dh + k;
 #pragma unroll
           for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4 *>(ring + (long long)j * H) = j == 3 ? rows.x[s0 + s] : rows.taps[s0 + s][j];
+          if (p.x_out) *reinterpret_cast<uint4 *>(p.x_out + (long long)(row0 + r16) * H + head * dh + k) = rows.x[s0 + s];
         }
         const bool there = k < dh;
         unsigned char *dst = layer_step_lds + r16 * RB + 2 * k;

@@ -87,7 +87,7 @@ class GraphedLayerDecoder:
     def step(self, x: Optional[torch.Tensor] = None) -> torch.Tensor:
         """``x`` [B,1,D] -> the layer's output for this token (a buffer that the next call overwrites).
         With ``x=None`` the token is taken from ``self.x``, where its producer has written it (from the graphs: one copy
-        kernel and the gap in front of the graph less per token)."""
+        kernel and the gap in front of the graph less per token).  Afterwards ``self.x`` holds the token either way."""
         if not torch.cuda.is_current_stream_capturing() and self._launch(self.x if x is None else x):
             return self.out
         if x is not None and x.data_ptr() != self.x.data_ptr():
@@ -107,7 +107,7 @@ class GraphedLayerDecoder:
             return False
         with torch.no_grad():
             done = _lib.host().layer_step(layer, cell._native(), x, self.conv[k], self.slstm[k], self.slstm[1 - k], self.conv[1 - k],
-                                          self.h[1 - k], self.h[k], self.out)
+                                          self.h[1 - k], self.h[k], self.out, self.x)
         if done is None:
             return False
         cell._rt.last_workspace = cell._rt.step_plan[1].workspace
