@@ -304,3 +304,26 @@ def test_recorded_backward_of_calls_that_depend_on_the_layer(chain):
             assert (a is None) == (b is None)
             if a is not None:  # (float32 on both sides: sums over dh units, then over 12 steps of a recurrence)
                 torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-4 * float(b.detach().abs().max()))
+
+
+def test_recorded_backward_leaves_the_layers_parameters_in_place(monkeypatch):
+    """Other threads may be in the layer while a recorded backward makes a call's operations once more."""
+    from xlstm_amd import layer as layer_module
+
+    print("case layer create_graph in place", flush=True)
+    layer = _layer(2, 64)
+    mine = dict(layer.named_parameters())
+    x = torch.randn(2, 6, 128, device=DEV, requires_grad=True)
+    out = layer(x)
+    assert _one_node(out)
+    forward, seen = layer_module.CausalConv1d.forward, []
+
+    def watched(self, *args, **kwargs):
+        now = dict(layer.named_parameters())
+        seen.append(self is not layer.conv1d and set(now) == set(mine) and all(now[n] is mine[n] for n in mine))
+        return forward(self, *args, **kwargs)
+
+    monkeypatch.setattr(layer_module.CausalConv1d, "forward", watched)
+    grads = torch.autograd.grad(out, [x, *mine.values()], torch.ones_like(out), create_graph=True)
+    assert seen == [True] and all(g.isfinite().all() for g in grads)
+    layer.slstm_cell.check_status()

@@ -304,6 +304,19 @@ class sLSTMCell_hip(nn.Module):
 
             _lib.host()  # fail loudly here, not at the first forward, if the engine or its host path is missing
 
+    @classmethod
+    def around(cls, config: sLSTMCellConfig, r: torch.Tensor, bias: torch.Tensor, reports) -> "sLSTMCell_hip":
+        """A cell for a call with the given tensors in place of parameters.  ``reports``: the native host path's handle of
+        another cell's abort word and calls in flight, which takes this one's."""
+        cell = cls.__new__(cls)
+        nn.Module.__init__(cell)
+        cell.config = config
+        cell._parameters.update(_recurrent_kernel_=r, _bias_=bias)
+        cell.keep_state_fp32 = False
+        cell._rt = _Runtime()
+        cell._native().report_to(reports)
+        return cell
+
     def __repr__(self):
         return (
             f"{self.__class__.__name__}(function={self.config.function}, "

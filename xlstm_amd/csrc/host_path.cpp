@@ -770,6 +770,15 @@ PyObject *cell_workspace_(CellPath &c, PyObject *const *args) {
   if (!like) { PyErr_SetString(PyExc_TypeError, "workspace: a tensor on the device"); throw PythonError{}; }
   return THPVariable_Wrap(c.workspace(PyLong_AsLongLong(args[0]), like->device()));
 }
+// report_to(handle): the abort word and the calls in flight of another cell (a capsule that owns a Reports) take this one's
+struct Reports { AbortWord word; std::shared_ptr<CallsInFlight> calls; };
+constexpr const char *kReports = "reports";
+PyObject *cell_report_to_(CellPath &c, PyObject *const *args) {
+  const Reports *r = (const Reports *)PyCapsule_GetPointer(args[0], kReports);
+  if (!r) throw PythonError{};
+  c.abort_word = r->word; c.calls = r->calls;
+  Py_RETURN_NONE;
+}
 // last_workspace() -> the workspace of the latest sequence call
 PyObject *cell_last_workspace_(CellPath &c, PyObject *const *) {
   if (!c.last_workspace.defined()) Py_RETURN_NONE;
@@ -837,6 +846,7 @@ PyMethodDef cell_methods[] = {
     {"workspace", (PyCFunction)(void *)cell_call<cell_workspace_, 2>, METH_FASTCALL, nullptr},
     {"last_workspace", (PyCFunction)(void *)cell_call<cell_last_workspace_, 0>, METH_FASTCALL, nullptr},
     {"poll", (PyCFunction)(void *)cell_call<cell_poll_, 1>, METH_FASTCALL, nullptr},
+    {"report_to", (PyCFunction)(void *)cell_call<cell_report_to_, 1>, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyType_Slot cell_slots[] = {{Py_tp_new, (void *)cell_new}, {Py_tp_dealloc, (void *)cell_dealloc},
                             {Py_tp_traverse, (void *)cell_traverse}, {Py_tp_clear, (void *)cell_clear}, {Py_tp_methods, cell_methods}, {0, nullptr}};
@@ -1180,7 +1190,7 @@ struct LayerBackward : public torch::autograd::Node {
   }
 
   // A backward that is itself recorded (create_graph): the layer's operations once more, one by one, and their gradients
-  variable_list with_graph(PyObject *module, const at::Tensor (&t)[INPUTS], const at::Tensor &reset, const variable_list &grads) {
+  variable_list with_graph(PyObject *module, const at::Tensor (&t)[INPUTS], const ReverseInputs &call, const variable_list &grads) {
     struct Gil { PyGILState_STATE g = PyGILState_Ensure(); ~Gil() { PyGILState_Release(g); } } gil;
     PyRef held(module);
     auto wrapped = [](const at::Tensor &v) {
@@ -1188,10 +1198,11 @@ struct LayerBackward : public torch::autograd::Node {
       Py_INCREF(Py_None);
       return Py_None;
     };
-    PyRef list(PyTuple_New(INPUTS)), d_out(wrapped(grads[0])), d_state(wrapped(grads[1])), mask(wrapped(reset));
+    PyRef list(PyTuple_New(INPUTS)), d_out(wrapped(grads[0])), d_state(wrapped(grads[1])), mask(wrapped(call.mask));
+    PyRef reports(PyCapsule_New(new Reports{call.word, call.calls}, kReports, [](PyObject *o) { delete (Reports *)PyCapsule_GetPointer(o, kReports); }));
     if (list.o)
       for (int i = 0; i < INPUTS; ++i) PyTuple_SET_ITEM(list.o, i, wrapped(t[i]));
-    PyRef result(list.o && module ? PyObject_CallMethodObjArgs(module, g_names.gradients_with_graph, list.o, mask.o, d_out.o, d_state.o, nullptr) : nullptr);
+    PyRef result(list.o && reports.o && module ? PyObject_CallMethodObjArgs(module, g_names.gradients_with_graph, list.o, mask.o, d_out.o, d_state.o, reports.o, nullptr) : nullptr);
     variable_list out(INPUTS);
     if (!result.o || !PyTuple_Check(result.o) || PyTuple_GET_SIZE(result.o) != INPUTS) {
       if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "the gradients of the layer are missing");
@@ -1224,7 +1235,7 @@ struct LayerBackward : public torch::autograd::Node {
       }
     }
     c10::OptionalDeviceGuard guard(call.h.device());
-    if (at::GradMode::is_enabled()) return with_graph(module, t, call.mask, grads);
+    if (at::GradMode::is_enabled()) return with_graph(module, t, call, grads);
     at::NoGradGuard no_grad;
     call.r = t[R];
     if (given[STATE]) call.state = t[STATE];

@@ -132,9 +132,13 @@ class LinearHeadwiseExpand(nn.Module):
         nn.init.normal_(self.weight, mean=0.0, std=sqrt(2 / 5 / d))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        shape = x.shape
-        y = torch.einsum("...hd,hod->...ho", x.view(*shape[:-1], self.num_heads, -1), self.weight)
-        return y.reshape(*shape[:-1], -1)
+        return _headwise(x, self.weight, self.num_heads)
+
+
+def _headwise(x: torch.Tensor, weight: torch.Tensor, num_heads: int) -> torch.Tensor:
+    shape = x.shape
+    y = torch.einsum("...hd,hod->...ho", x.view(*shape[:-1], num_heads, -1), weight)
+    return y.reshape(*shape[:-1], -1)
 
 
 class MultiHeadLayerNorm(nn.Module):
@@ -155,19 +159,6 @@ class MultiHeadLayerNorm(nn.Module):
         w = None if self.weight is None else 1.0 + self.weight
         out = F.group_norm(gn_in, num_groups=NH, weight=w, bias=None, eps=self.eps)
         return out.view(B, S, NH, DH).transpose(1, 2)
-
-
-class _UpToTheCell(nn.Module):
-    """A layer's modules up to the cell, one by one, for calls with other tensors in place of its parameters
-    (``torch.func.functional_call``)."""
-
-    def __init__(self, layer: "sLSTMLayer"):
-        super().__init__()
-        self.layer = layer
-
-    def forward(self, x, slstm_state, reset_mask):
-        x_conv = self.layer.conv_act_fn(self.layer.conv1d(x, reset_mask=reset_mask))
-        return self.layer._cell_output(x, x_conv, slstm_state, reset_mask)
 
 
 # the modules that the float32 path of a layer stands in for, and their methods
@@ -255,22 +246,22 @@ class sLSTMLayer(nn.Module):
         cell = modules["slstm_cell"]
         return not (cell._backward_hooks or cell._backward_pre_hooks)
 
-    def _cell_output(self, x, x_conv, slstm_state, reset_mask):
-        return self.slstm_cell(self._gates(x, x_conv), state=slstm_state, reset_mask=reset_mask)
-
-    def _gradients_with_graph(self, inputs, reset_mask, d_y, d_state):
+    def _gradients_with_graph(self, inputs, reset_mask, d_y, d_state, reports):
         """The gradients of a training call for a backward pass that is itself recorded: its operations once more with the
-        call's own tensors (x, convolution weight and bias, the gates', R, b, state), one by one.  They are taken at aliases
-        made here, one per place: x or the state may come from an earlier call of the same layer and a weight may stand
-        in two places, and a gradient taken at the tensors themselves would run on through those - a part that the
-        surrounding backward pass adds by itself."""
-        names = ("conv1d.conv.weight", "conv1d.conv.bias", "fgate.weight", "igate.weight", "zgate.weight", "ogate.weight",
-                 "slstm_cell._recurrent_kernel_", "slstm_cell._bias_")
+        call's own tensors (x, convolution weight and bias, the gates', R, b, state), one by one, in modules made for this
+        (other threads may be in the layer's).  They are taken at aliases made here, one per place: x or the state may come
+        from an earlier call of the same layer and a weight may stand in two places, and a gradient taken at the
+        tensors themselves would run on through those - a part that the surrounding backward pass adds by itself.
+        ``reports``: where the layer's cell learns of calls that gave up."""
         with torch.enable_grad():
             inputs = [None if t is None else t.view_as(t) for t in inputs]
-            x, state = inputs[0], inputs[-1]
-            params = {"layer." + n: t for n, t in zip(names, inputs[1:-1]) if t is not None}
-            y, new_state = torch.func.functional_call(_UpToTheCell(self), params, (x, state, reset_mask), tie_weights=False)
+            x, conv_weight, conv_bias, fgate, igate, zgate, ogate, r, bias, state = inputs
+            with torch.device("meta"):
+                conv1d = CausalConv1d(x.shape[-1], conv_weight.shape[-1])
+            conv1d.conv._parameters.update(weight=conv_weight, bias=conv_bias)
+            x_conv = F.silu(conv1d(x, reset_mask=reset_mask))
+            wx = torch.cat([_headwise(t, w, w.shape[0]) for t, w in ((x_conv, fgate), (x_conv, igate), (x, zgate), (x, ogate))], dim=-1)
+            y, new_state = sLSTMCell_hip.around(self.slstm_cell.config, r, bias, reports)(wx, state=state, reset_mask=reset_mask)
             pairs = [(o, g) for o, g in ((y, d_y), (new_state, d_state)) if g is not None]
             wanted = [t for t in inputs if t is not None and t.requires_grad]
             grads = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs], create_graph=True, allow_unused=True))
@@ -329,7 +320,7 @@ class sLSTMLayer(nn.Module):
             x_conv = self.conv_act_fn(x_conv)
         else:
             x_conv = x
-        y, slstm_state = self._cell_output(x, x_conv, slstm_state, reset_mask)
+        y, slstm_state = self.slstm_cell(self._gates(x, x_conv), state=slstm_state, reset_mask=reset_mask)
         out = self._norm(self.dropout(y), B, S)
         if return_last_state:
             return out, {"conv_state": conv_state, "slstm_state": slstm_state}
