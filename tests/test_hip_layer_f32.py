@@ -327,3 +327,25 @@ def test_recorded_backward_leaves_the_layers_parameters_in_place(monkeypatch):
     grads = torch.autograd.grad(out, [x, *mine.values()], torch.ones_like(out), create_graph=True)
     assert seen == [True] and all(g.isfinite().all() for g in grads)
     layer.slstm_cell.check_status()
+
+
+def test_what_a_training_call_returned_does_not_hold_the_layer():
+    """An output kept on the layer goes with it, and its graph outlives the layer."""
+    import gc
+    import weakref
+
+    print("case layer kept output", flush=True)
+    layer = _layer(2, 64)
+    x = torch.randn(2, 6, 128, device=DEV, requires_grad=True)
+    out = layer(x)
+    assert _one_node(out)
+    layer.last, gone = layer(x), weakref.ref(layer)
+    leaves = [x, *layer.parameters()]
+    want = torch.autograd.grad(layer(x), leaves, torch.ones_like(out))
+    kept = weakref.ref(layer.last)
+    del layer
+    gc.collect()
+    assert gone() is None and kept() is None
+    got = torch.autograd.grad(out, leaves, torch.ones_like(out), create_graph=True)
+    for a, b in zip(got, want):  # (float32 on both sides: sums over dh units, then over 6 steps of a recurrence)
+        torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-4 * float(b.abs().max()))

@@ -1176,7 +1176,7 @@ struct LayerBackward : public torch::autograd::Node {
   ReverseInputs in;  // (its saved tensors are filled in when the backward runs)
   int64_t K = 0;
   at::ScalarType r_dtype = at::kFloat, b_dtype = at::kFloat, s_dtype = at::kFloat;
-  std::unique_ptr<PythonObject> layer;
+  std::unique_ptr<PythonObject> recorded_backward;  // (sLSTMLayer._gradients_with_graph, the cell's config)
 
   std::string name() const override { return "sLSTMLayerBackward"; }
   void release_variables() override {
@@ -1186,13 +1186,13 @@ struct LayerBackward : public torch::autograd::Node {
     for (SavedVariable *v : {&x_conv, &h, &coef}) v->reset_data();
     in.mask.reset();
     share.reset();
-    last = std::move(layer);
+    last = std::move(recorded_backward);
   }
 
   // A backward that is itself recorded (create_graph): the layer's operations once more, one by one, and their gradients
-  variable_list with_graph(PyObject *module, const at::Tensor (&t)[INPUTS], const ReverseInputs &call, const variable_list &grads) {
+  variable_list with_graph(PyObject *function_and_config, const at::Tensor (&t)[INPUTS], const ReverseInputs &call, const variable_list &grads) {
     struct Gil { PyGILState_STATE g = PyGILState_Ensure(); ~Gil() { PyGILState_Release(g); } } gil;
-    PyRef held(module);
+    PyRef held(function_and_config);
     auto wrapped = [](const at::Tensor &v) {
       if (v.defined()) return THPVariable_Wrap(v);
       Py_INCREF(Py_None);
@@ -1202,7 +1202,8 @@ struct LayerBackward : public torch::autograd::Node {
     PyRef reports(PyCapsule_New(new Reports{call.word, call.calls}, kReports, [](PyObject *o) { delete (Reports *)PyCapsule_GetPointer(o, kReports); }));
     if (list.o)
       for (int i = 0; i < INPUTS; ++i) PyTuple_SET_ITEM(list.o, i, wrapped(t[i]));
-    PyRef result(list.o && reports.o && module ? PyObject_CallMethodObjArgs(module, g_names.gradients_with_graph, list.o, mask.o, d_out.o, d_state.o, reports.o, nullptr) : nullptr);
+    PyRef result(list.o && reports.o && held.o ? PyObject_CallFunctionObjArgs(PyTuple_GET_ITEM(held.o, 0), PyTuple_GET_ITEM(held.o, 1), list.o, mask.o, d_out.o, d_state.o,
+                                                                              reports.o, nullptr) : nullptr);
     variable_list out(INPUTS);
     if (!result.o || !PyTuple_Check(result.o) || PyTuple_GET_SIZE(result.o) != INPUTS) {
       if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "the gradients of the layer are missing");
@@ -1218,7 +1219,7 @@ struct LayerBackward : public torch::autograd::Node {
   variable_list apply(variable_list &&grads) override {
     at::Tensor t[INPUTS], xc;
     ReverseInputs call;
-    PyObject *module = nullptr;
+    PyObject *function_and_config = nullptr;
     {
       std::lock_guard<std::mutex> lock(mutex_);
       for (int i = 0; i < INPUTS; ++i)
@@ -1227,15 +1228,15 @@ struct LayerBackward : public torch::autograd::Node {
       call.h = h.unpack(shared_from_this());
       call.coef = coef.unpack();
       xc = x_conv.unpack();
-      if (at::GradMode::is_enabled() && layer) {
+      if (at::GradMode::is_enabled() && recorded_backward) {
         PyGILState_STATE gil = PyGILState_Ensure();
-        module = layer->o;
-        Py_INCREF(module);
+        function_and_config = recorded_backward->o;
+        Py_INCREF(function_and_config);
         PyGILState_Release(gil);
       }
     }
     c10::OptionalDeviceGuard guard(call.h.device());
-    if (at::GradMode::is_enabled()) return with_graph(module, t, call, grads);
+    if (at::GradMode::is_enabled()) return with_graph(function_and_config, t, call, grads);
     at::NoGradGuard no_grad;
     call.r = t[R];
     if (given[STATE]) call.state = t[STATE];
@@ -1298,7 +1299,9 @@ PyObject *layer_train_(PyObject *const *args) {
   std::shared_ptr<Share> share = Share::take(x_in.device().index(), 4 * (int64_t)g_engine.coef_floats((int32_t)B, (int32_t)T, (int32_t)p.NH, (int32_t)p.dh, XS_F32), limit);
   if (!share) Py_RETURN_NONE;
   Sequence s(c, x_in.device(), B);
-  auto layer = std::make_unique<PythonObject>(args[0]);
+  PyRef function(attribute(args[0], g_names.gradients_with_graph)), pair(PyTuple_Pack(2, function.o, p.cell_config.o));
+  if (!pair.o) throw PythonError{};
+  auto recorded_backward = std::make_unique<PythonObject>(pair.o);
   {
     WithoutGil no_gil;
     at::Tensor x_conv;
@@ -1328,7 +1331,7 @@ PyObject *layer_train_(PyObject *const *args) {
     node->in.mask = s.mask; node->in.word = s.word; node->in.calls = c.calls;
     node->in.B = B; node->in.T = T; node->in.NH = p.NH; node->in.dh = p.dh;
     node->in.cut = cut_on != 0; node->in.clip = clipval;
-    node->layer = std::move(layer);
+    node->recorded_backward = std::move(recorded_backward);
     torch::autograd::set_history(s.h, node);
     torch::autograd::set_history(s.state, node);
     node->h = SavedVariable(s.h, true);

@@ -246,13 +246,15 @@ class sLSTMLayer(nn.Module):
         cell = modules["slstm_cell"]
         return not (cell._backward_hooks or cell._backward_pre_hooks)
 
-    def _gradients_with_graph(self, inputs, reset_mask, d_y, d_state, reports):
+    @staticmethod
+    def _gradients_with_graph(config, inputs, reset_mask, d_y, d_state, reports):
         """The gradients of a training call for a backward pass that is itself recorded: its operations once more with the
         call's own tensors (x, convolution weight and bias, the gates', R, b, state), one by one, in modules made for this
         (other threads may be in the layer's).  They are taken at aliases made here, one per place: x or the state may come
         from an earlier call of the same layer and a weight may stand in two places, and a gradient taken at the
         tensors themselves would run on through those - a part that the surrounding backward pass adds by itself.
-        ``reports``: where the layer's cell learns of calls that gave up."""
+        ``config``: the cell's (the call's node holds no more of the layer: what hangs on the node may hang on the layer too);
+        ``reports``: where the cell learns of calls that gave up."""
         with torch.enable_grad():
             inputs = [None if t is None else t.view_as(t) for t in inputs]
             x, conv_weight, conv_bias, fgate, igate, zgate, ogate, r, bias, state = inputs
@@ -261,7 +263,7 @@ class sLSTMLayer(nn.Module):
             conv1d.conv._parameters.update(weight=conv_weight, bias=conv_bias)
             x_conv = F.silu(conv1d(x, reset_mask=reset_mask))
             wx = torch.cat([_headwise(t, w, w.shape[0]) for t, w in ((x_conv, fgate), (x_conv, igate), (x, zgate), (x, ogate))], dim=-1)
-            y, new_state = sLSTMCell_hip.around(self.slstm_cell.config, r, bias, reports)(wx, state=state, reset_mask=reset_mask)
+            y, new_state = sLSTMCell_hip.around(config, r, bias, reports)(wx, state=state, reset_mask=reset_mask)
             pairs = [(o, g) for o, g in ((y, d_y), (new_state, d_state)) if g is not None]
             wanted = [t for t in inputs if t is not None and t.requires_grad]
             grads = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs], create_graph=True, allow_unused=True))
