@@ -197,3 +197,55 @@ def test_a_stack_keeps_what_a_device_may_hold(monkeypatch, native, dtype, dh):
         # (other row tiles sum in another order; bfloat16 deltas round once, 2^-8, and so do the gradients between layers)
         tol = (1e-4 if dtype == torch.float32 else 3e-2) * float(a.abs().max())
         torch.testing.assert_close(a, b, rtol=0, atol=tol)
+
+
+def _contiguous(t):
+    return t.clone(memory_format=torch.contiguous_format)
+
+
+def _misaligned(t):
+    return torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape).copy_(t)
+
+
+def _other_order(t):
+    return t if t.dim() < 2 else t.transpose(0, -1).contiguous().transpose(0, -1)
+
+
+@pytest.mark.parametrize("kind,dtype,repack", [
+    (k, t, r) for k in ("BNSH", "BSH", "SBNH", "general", "layer") for t in (torch.float32, torch.bfloat16) for r in (_contiguous, _misaligned, _other_order)
+    if not (k == "general" and r is _misaligned)  # (the entry points called from Python refuse misaligned tensors with an error)
+    and not (k == "layer" and t == torch.bfloat16)])
+def test_hooks_may_hand_back_other_layouts(monkeypatch, kind, dtype, repack):
+    """What hooks on saved tensors return has the values that were packed, in any memory layout (``save_on_cpu(pin_memory=True)``:
+    contiguous in the order of the dimensions)."""
+    from xlstm_amd import cell as cell_module
+    from xlstm_amd.layer import sLSTMLayer, sLSTMLayerConfig
+
+    print("case saved layouts", kind, dtype, repack.__name__, flush=True)
+    if kind == "general":
+        monkeypatch.setattr(cell_module.sLSTMCell_hip, "_trains_natively", lambda self, input: False)
+    torch.manual_seed(1)
+    NH, dh, B, T = 2, 128, 3, 5
+    H = NH * dh
+    s0 = torch.randn(4, B, H, device=DEV)
+    s0[2] = s0[2].abs() + 1.0
+    if kind == "layer":
+        module = sLSTMLayer(sLSTMLayerConfig(embedding_dim=H, num_heads=NH, backend="hip", recurrent_weight_init="standard")).to(DEV).to(dtype)
+        module._norm = lambda y, B, S: y.transpose(1, 2).reshape(B, S, -1)  # (PyTorch's own reads what it saved as dense)
+        call = lambda: module(x, slstm_state=s0)
+    else:
+        module = cell_module.sLSTMCell(cell_module.sLSTMCellConfig(hidden_size=H, num_heads=NH, backend="hip", recurrent_weight_init="standard",
+                                                                   output_shape="BNSH" if kind == "general" else kind)).to(DEV)
+        call = lambda: module(x, s0)[0]
+    x = torch.randn(B, T, H if kind == "layer" else 4 * H, device=DEV).to(dtype).requires_grad_(True)
+    leaves = [x, *(p for n, p in module.named_parameters() if n != "group_norm.weight")]
+    out = call()
+    d = torch.randn_like(out)
+    want = torch.autograd.grad(out, leaves, d)
+    with torch.autograd.graph.saved_tensors_hooks(repack, lambda t: t):
+        out = call()
+    got = torch.autograd.grad(out, leaves, d)
+    for a, b in zip(want, got):
+        # (the same kernels on the same values; sums over 15 tokens by float atomics)
+        tol = 2.0 ** -7 if a.dtype == torch.bfloat16 else 1e-5
+        torch.testing.assert_close(a, b, rtol=tol, atol=tol * float(a.abs().max()))

@@ -630,6 +630,23 @@ at::Tensor output_gradient(const ReverseInputs &in, OutShape shape, const at::Te
 using torch::autograd::SavedVariable;
 using torch::autograd::variable_list;
 
+// What a call saved, as its kernels left it: hooks on saved tensors may hand back the same values in another memory layout
+// (torch.autograd.graph.save_on_cpu(pin_memory=True): contiguous in the order of the dimensions)
+at::Tensor laid_out(const at::Tensor &t, at::IntArrayRef stride) {
+  if (t.strides() == stride && aligned(t.data_ptr(), 16)) return t;
+  at::Tensor out = at::empty_strided(t.sizes(), stride, t.options());
+  return out.copy_(t);
+}
+at::Tensor laid_out(const at::Tensor &t) {  // contiguous
+  if (t.is_contiguous() && aligned(t.data_ptr(), 16)) return t;
+  return t.clone(at::MemoryFormat::Contiguous);
+}
+at::Tensor laid_out(const at::Tensor &h, OutShape shape, const ReverseInputs &in) {  // [T,B,H] memory
+  const Shape4 s = shape_of(shape, in.T, in.B, in.NH, in.dh);
+  TORCH_CHECK(h.sizes() == at::IntArrayRef(s.size.data(), s.n), "the hidden states of a call came back from a saved-tensor hook in another shape");
+  return laid_out(h, at::IntArrayRef(s.stride.data(), s.n));
+}
+
 struct CellBackward : public torch::autograd::Node {
   // (input and bias are not read again: a change of theirs in front of the backward is refused like one of R.  The
   // coefficients are saved like a tensor of the caller's, so that checkpointing and offloading hooks see them)
@@ -655,9 +672,10 @@ struct CellBackward : public torch::autograd::Node {
     b.unpack();
     call.h = h.unpack(shared_from_this());
     c10::OptionalDeviceGuard guard(call.h.device());
-    call.r = r.unpack();
-    call.coef = coef.unpack();
-    if (has_state) call.state = state.unpack();
+    call.h = laid_out(call.h, shape, call);
+    call.r = laid_out(r.unpack());
+    call.coef = laid_out(coef.unpack());
+    if (has_state) call.state = laid_out(state.unpack());
     int64_t sb, st;
     const at::Tensor d = output_gradient(call, shape, grads[0], sb, st);
     CellGradients g = run_reverse(call, d, sb, st, grads[1]);
@@ -1238,14 +1256,19 @@ struct LayerBackward : public torch::autograd::Node {
     c10::OptionalDeviceGuard guard(call.h.device());
     if (at::GradMode::is_enabled()) return with_graph(function_and_config, t, call, grads);
     at::NoGradGuard no_grad;
+    call.h = laid_out(call.h, OutShape::BNSH, call);
+    call.coef = laid_out(call.coef);
+    xc = laid_out(xc);
+    for (int i = CONV_W; i <= R; ++i)
+      if (given[i]) t[i] = laid_out(t[i]);
     call.r = t[R];
-    if (given[STATE]) call.state = t[STATE];
+    if (given[STATE]) call.state = laid_out(t[STATE]);
     const int64_t B = in.B, T = in.T, D = in.NH * in.dh;
     int64_t sb, st;
     const at::Tensor d = output_gradient(call, OutShape::BNSH, grads[0], sb, st);
     CellGradients g = run_reverse(call, d, sb, st, grads[1]);
     const auto f32 = call.h.options();
-    const at::Tensor x = t[X].is_contiguous() && aligned(t[X].data_ptr(), 16) ? t[X] : t[X].clone(at::MemoryFormat::Contiguous);
+    const at::Tensor x = laid_out(t[X]);
     LayerParts p;
     p.NH = in.NH; p.dh = in.dh; p.D = D; p.K = K;
     p.conv_w = t[CONV_W]; p.conv_b = t[CONV_B];
