@@ -318,8 +318,9 @@ int xs_layer_step(const xs_layer_step_args *args);
  * summed in float32): what a layer's training call and its float32 inference call consist of besides the cell's own calls.
  *   xs_layer_front           x_conv = silu(conv(x)) and the cell's input wx = the four projections.  Two kernels.
  *   xs_layer_norm            out = group norm of h.  One kernel.
- *   xs_layer_front_backward  from d_wx (what xs_slstm_train_backward left): d_x, d_gate_w, d_conv_w and d_conv_b.  Four kernels.
- *                            d_x_conv is its intermediate, scratch holds xs_layer_scratch_floats floats.
+ *   xs_layer_front_backward  from d_wx (what xs_slstm_train_backward left): d_x, d_gate_w, d_conv_w and d_conv_b, those that are not
+ *                            NULL.  Up to four kernels.  d_x_conv is the intermediate of d_x and of the convolution's gradients,
+ *                            scratch holds xs_layer_scratch_floats floats.
  * The reference leaves these gradients to PyTorch's autograd (xlstm/blocks/slstm/layer.py:123-155).  Sums over tokens are added
  * up in a fixed order.
  */
@@ -344,7 +345,7 @@ typedef struct xs_layer_args {
   const float *d_wx;         /* [B,T,4D] contiguous (front_backward) */
   float *d_x_conv;           /* [B,T,D] contiguous (front_backward) */
   float *d_x;                /* [B,T,D] contiguous (front_backward) */
-  float *d_conv_w, *d_conv_b, *d_gate_w[4]; /* in the parameters' layouts; d_conv_b NULL where there is no bias */
+  float *d_conv_w, *d_conv_b, *d_gate_w[4]; /* in the parameters' layouts; d_conv_b not used where there is no bias */
   float *scratch;
   void *stream;
 } xs_layer_args;

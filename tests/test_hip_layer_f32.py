@@ -133,6 +133,23 @@ def test_kernels_around_the_cell_equal_float64(B, T, NH, dh, K, masked, bias, st
         _close(t["d_conv_b"], cb64.grad, "d_conv_b", 2 * dh + B * T)
     else:
         assert bool((t["d_conv_b"] == 7.0).all())
+    # what is not wanted is not made; the rest comes out the same
+    results = {"d_x": t["d_x"], "d_conv_w": t["d_conv_w"], "d_conv_b": t["d_conv_b"], **{i: d_gates[i] for i in range(4)}}
+    whole = {k: v.clone() for k, v in results.items()}
+    for wanted in (("d_x",), ("d_conv_w",), ("d_conv_b",), (0, 3), (2, "d_conv_w"), ("d_x", 1), ()):
+        for k, v in [*results.items(), *t.items()]:
+            if k in results or k in ("d_x_conv", "scratch"):
+                v.fill_(7.0)
+            if k in results and isinstance(k, str):
+                setattr(a, k, v.data_ptr() if k in wanted else None)
+            elif k in results:
+                a.d_gate_w[k] = v.data_ptr() if k in wanted else None
+        call(lib.xs_layer_front_backward)
+        for k, v in results.items():
+            made = k in wanted and (k != "d_conv_b" or bias)
+            assert torch.equal(v, whole[k]) if made else bool((v == 7.0).all()), (wanted, k)
+        if not any(isinstance(k, str) for k in wanted):
+            assert bool((t["d_x_conv"] == 7.0).all())
 
 
 def _layer(NH, dh, **kw):
@@ -349,3 +366,29 @@ def test_what_a_training_call_returned_does_not_hold_the_layer():
     got = torch.autograd.grad(out, leaves, torch.ones_like(out), create_graph=True)
     for a, b in zip(got, want):  # (float32 on both sides: sums over dh units, then over 6 steps of a recurrence)
         torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-4 * float(b.abs().max()))
+
+
+@pytest.mark.parametrize("frozen", [("x",), ("fgate", "igate", "zgate", "ogate"), ("conv1d", "x"), ("zgate", "conv1d"), ("conv1d", "fgate", "igate", "zgate", "ogate", "x")])
+def test_frozen_parts_of_a_layer(frozen):
+    """The gradients of what is not frozen, and of what a call of torch.autograd.grad asks for, are those of the whole."""
+    print("case layer frozen", frozen, flush=True)
+    layer = _layer(2, 64)
+    x = torch.randn(3, 90, 128, device=DEV, requires_grad=True)
+    d = torch.randn(3, 90, 128, device=DEV)
+    named = {"x": x, **dict(layer.named_parameters())}
+    out = layer(x)
+    assert _one_node(out)
+    whole = dict(zip(named, torch.autograd.grad(out, list(named.values()), d, retain_graph=True)))
+    wanted = [n for n in named if n.split(".")[0] not in frozen]
+    asked = torch.autograd.grad(out, [named[n] for n in wanted], d)
+    for n in named:
+        named[n].requires_grad_(n in wanted)
+    out = layer(x)
+    assert _one_node(out)
+    out.backward(d)
+    for n, got in zip(wanted, asked):
+        # (R and bias are summed by float atomics; the rest has a fixed order)
+        tol = 1e-5 * float(whole[n].abs().max()) if "slstm_cell" in n else 0.0
+        torch.testing.assert_close(got, whole[n], rtol=0, atol=tol)
+        torch.testing.assert_close(named[n].grad, whole[n], rtol=0, atol=tol)
+    assert all(named[n].grad is None for n in named if n not in wanted)

@@ -1275,10 +1275,18 @@ struct LayerBackward : public torch::autograd::Node {
     for (int i = 0; i < 4; ++i) p.gate[i] = t[GATE + i];
     xs_layer_args a = float32_args(p, x, xc, call.mask.defined() ? &call.mask : nullptr);
     variable_list out(INPUTS);
-    for (int i = CONV_W; i < R; ++i)
-      if (given[i]) out[i] = at::empty(t[i].sizes(), f32);
-    out[X] = at::empty({B, T, D}, f32);
-    const at::Tensor d_x_conv = at::empty({B, T, D}, f32);
+    out[R] = g.d_r.to(r_dtype);
+    out[BIAS] = g.d_bias.to(b_dtype);
+    if (given[STATE]) out[STATE] = g.d_s0.to(s_dtype);
+    bool any = false;  // (what is frozen costs nothing)
+    for (int i = X; i < R; ++i)
+      if (given[i] && task_should_compute_output(i)) {
+        out[i] = at::empty(t[i].sizes(), f32);
+        any = true;
+      }
+    if (!any) return out;
+    at::Tensor d_x_conv;
+    if (out[X].defined() || out[CONV_W].defined() || out[CONV_B].defined()) d_x_conv = at::empty({B, T, D}, f32);
     const at::Tensor scratch = at::empty({(int64_t)g_engine.layer_scratch((int32_t)B, (int32_t)T, (int32_t)in.NH, (int32_t)in.dh, (int32_t)K)}, f32);
     auto ptr = [](const at::Tensor &v) { return v.defined() ? (float *)v.data_ptr() : nullptr; };
     a.scratch = ptr(scratch);
@@ -1288,9 +1296,6 @@ struct LayerBackward : public torch::autograd::Node {
     for (int i = 0; i < 4; ++i) a.d_gate_w[i] = ptr(out[GATE + i]);
     const int rc = g_engine.layer_front_backward(&a);
     if (rc != XS_OK) engine_failed_in_backward(rc);
-    out[R] = g.d_r.to(r_dtype);
-    out[BIAS] = g.d_bias.to(b_dtype);
-    if (given[STATE]) out[STATE] = g.d_s0.to(s_dtype);
     return out;
   }
 };

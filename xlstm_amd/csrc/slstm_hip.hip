@@ -1470,7 +1470,8 @@ LayerProductParams layer_product_params(const xs_layer_args *a) {
 template <LayerProduct MODE>
 int launch_layer_product(LayerProductParams p, hipStream_t stream) {
   const int up = (p.dh + 63) / 64;
-  p.tiles = MODE == LayerProduct::WEIGHTS ? 4 * up * up : (MODE == LayerProduct::INPUTS ? 2 : 4) * up;
+  // (INPUTS: the operand x behind x_conv, and not at all where its gradient is not wanted)
+  p.tiles = MODE == LayerProduct::WEIGHTS ? 4 * up * up : (MODE == LayerProduct::INPUTS ? (p.d_a[1] ? 2 : 1) : 4) * up;
   const long long pairs = (long long)p.NH * (MODE == LayerProduct::WEIGHTS ? p.slices : p.m_tiles);
   const long long grid = 8 * ((pairs + 7) / 8) * p.tiles;
   if (grid > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many tiles for one launch");
@@ -1535,9 +1536,8 @@ int run_layer_front_backward(const xs_layer_args *a) {
   int rc = layer_check(a);
   if (rc != XS_OK || a->B == 0 || a->T == 0) return rc;
   if ((rc = layer_front_check(a)) != XS_OK) return rc;
-  if (!a->d_wx || !a->d_x_conv || !a->d_x || !a->scratch || !a->d_conv_w || (a->conv_b && !a->d_conv_b) ||
-      !a->d_gate_w[0] || !a->d_gate_w[1] || !a->d_gate_w[2] || !a->d_gate_w[3])
-    return fail(XS_ERR_NULL, "d_wx, d_x_conv, d_x, scratch and the gradients of the parameters are required");
+  const bool gates = a->d_gate_w[0] || a->d_gate_w[1] || a->d_gate_w[2] || a->d_gate_w[3], conv = a->d_conv_w || a->d_conv_b, inputs = a->d_x || conv;
+  if (!a->d_wx || !a->scratch || (inputs && !a->d_x_conv)) return fail(XS_ERR_NULL, "d_wx, scratch and, for d_x and the convolution's gradients, d_x_conv are required");
   if (a->conv_state) return fail(XS_ERR_UNSUPPORTED, "no gradient through a convolution that continues from a state");
   if (layer_misaligned({a->d_wx, a->d_x_conv, a->d_x, a->scratch, a->d_gate_w[0], a->d_gate_w[1], a->d_gate_w[2], a->d_gate_w[3]}))
     return fail(XS_ERR_ALIGN, "d_wx, d_x_conv, d_x, scratch and d_gate_w must be 16-byte aligned");
@@ -1545,21 +1545,25 @@ int run_layer_front_backward(const xs_layer_args *a) {
   hipStream_t stream = (hipStream_t)a->stream;
   const long long D = (long long)a->NH * a->dh;
   LayerProductParams g = layer_product_params(a);
-  if ((rc = launch_layer_product<LayerProduct::INPUTS>(g, stream)) != XS_OK) return rc;
+  if (inputs && (rc = launch_layer_product<LayerProduct::INPUTS>(g, stream)) != XS_OK) return rc;
   g.slices = split.slices; g.slice_tokens = split.slice_tokens; g.partial = a->scratch;
-  if ((rc = launch_layer_product<LayerProduct::WEIGHTS>(g, stream)) != XS_OK) return rc;
-  LayerConvParams c = layer_conv_params(a);
-  c.state = nullptr;
-  c.d_out = a->d_x_conv; c.d_x = a->d_x; c.partial = a->scratch + split.gate_floats;
-  const int piece_blocks = (int)((D / 4 + 31) / 32);
-  if ((long long)piece_blocks * split.conv_blocks > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many tokens for one launch");
-  void (*kern)(LayerConvParams, int) = a->K == 2 ? layer_conv_backward_f32_kernel<2> : (a->K == 3 ? layer_conv_backward_f32_kernel<3> : layer_conv_backward_f32_kernel<4>);
-  hipLaunchKernelGGL(kern, dim3((unsigned)(piece_blocks * split.conv_blocks)), dim3(256), 0, stream, c, piece_blocks);
-  if ((rc = layer_launched("convolution gradient kernel")) != XS_OK) return rc;
+  if (gates && (rc = launch_layer_product<LayerProduct::WEIGHTS>(g, stream)) != XS_OK) return rc;
+  float *const conv_partial = a->scratch + split.gate_floats;
+  if (inputs) {
+    LayerConvParams c = layer_conv_params(a);
+    c.state = nullptr;
+    c.d_out = a->d_x_conv; c.d_x = a->d_x; c.partial = conv ? conv_partial : nullptr;
+    const int piece_blocks = (int)((D / 4 + 31) / 32);
+    if ((long long)piece_blocks * split.conv_blocks > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many tokens for one launch");
+    void (*kern)(LayerConvParams, int) = a->K == 2 ? layer_conv_backward_f32_kernel<2> : (a->K == 3 ? layer_conv_backward_f32_kernel<3> : layer_conv_backward_f32_kernel<4>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(piece_blocks * split.conv_blocks)), dim3(256), 0, stream, c, piece_blocks);
+    if ((rc = layer_launched("convolution gradient kernel")) != XS_OK) return rc;
+  }
   LayerReduceParams r{};
   auto region = [](const float *partial, long long n, int parts) { return LayerReduceParams::Region{partial, n, parts, (int)((n + 63) / 64)}; };
-  r.region[0] = region(a->scratch, split.slices > 1 ? 4 * D * a->dh : 0, split.slices);
-  r.region[1] = region(c.partial, D * (a->K + 1), split.conv_blocks);
+  r.region[0] = region(a->scratch, gates && split.slices > 1 ? 4 * D * a->dh : 0, split.slices);
+  r.region[1] = region(conv_partial, conv ? D * (a->K + 1) : 0, split.conv_blocks);
+  if (!r.region[0].blocks && !r.region[1].blocks) return XS_OK;
   for (int i = 0; i < 4; ++i) r.d_w[i] = a->d_gate_w[i];
   r.d_conv_w = a->d_conv_w; r.d_conv_b = a->conv_b ? a->d_conv_b : nullptr;
   r.per_gate = D * a->dh; r.taps = a->K;

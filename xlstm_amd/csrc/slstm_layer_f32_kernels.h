@@ -17,8 +17,8 @@ struct LayerConvParams {
   long long reset_sb;
   float *out;          // [B, T, D]: the forward's result
   const float *d_out;  // [B, T, D]: gradient of that result (backward)
-  float *d_x;          // [B, T, D]: on entry the gradient that reaches x past the convolution (backward)
-  float *partial;      // [workgroups over tokens][D][KS+1]: sums over a workgroup's tokens (backward)
+  float *d_x;          // [B, T, D]: on entry the gradient that reaches x past the convolution (backward); null: not wanted
+  float *partial;      // [workgroups over tokens][D][KS+1]: sums over a workgroup's tokens (backward); null: not wanted
   int B, T, D;
 };
 
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) void layer_conv_backward_f32_kernel(LayerConvP
     for (int i = 0; i < N; ++i) d[i] = t0 + i < p.T ? load4(drow + (long long)(t0 + i) * p.D) : zero4();
     f32x4 dx[R];
 #pragma unroll
-    for (int i = 0; i < R; ++i) dx[i] = t0 + i < p.T ? load4(dxrow + (long long)(t0 + i) * p.D) : zero4();
+    for (int i = 0; i < R; ++i) dx[i] = p.d_x && t0 + i < p.T ? load4(dxrow + (long long)(t0 + i) * p.D) : zero4();
     f32x4 taps[KS];
     load_taps<KS>(p.w + (long long)c0 * KS, taps);
     const f32x4 bias = p.bias ? load4(p.bias + c0) : zero4();
@@ -166,8 +166,9 @@ __global__ __launch_bounds__(256) void layer_conv_backward_f32_kernel(LayerConvP
     }
 #pragma unroll
     for (int i = 0; i < R; ++i)
-      if (t0 + i < p.T) *reinterpret_cast<f32x4 *>(dxrow + (long long)(t0 + i) * p.D) = dx[i];
+      if (p.d_x && t0 + i < p.T) *reinterpret_cast<f32x4 *>(dxrow + (long long)(t0 + i) * p.D) = dx[i];
   }
+  if (!p.partial) return;
 #pragma unroll
   for (int j = 0; j < G; ++j)
 #pragma unroll
@@ -208,7 +209,7 @@ struct LayerProductParams {
   const float *d_wx;       // [M, 4H]
   float *wx;               // [M, 4H] (PROJECT)
   float *d_a[2];           // [M, H] (INPUTS)
-  float *d_w[4];           // [NH, dh, dh] (WEIGHTS, one slice)
+  float *d_w[4];           // [NH, dh, dh] (WEIGHTS; written here with one slice), null: not wanted
   float *partial;          // [slices][4][NH][dh][dh] (WEIGHTS, several)
   int M, T, NH, dh, slices, slice_tokens;
   int m_tiles, tiles, pairs, pairs_per_xcd;
@@ -247,6 +248,9 @@ __global__ __launch_bounds__(256) void layer_product_f32_kernel(LayerProductPara
       m0 = pair % p.m_tiles * 64;
     }
     slot = tile;  // INPUTS: the operand instead (0: x_conv, slots i and f; 1: x, slots z and o)
+  }
+  if constexpr (MODE == LayerProduct::WEIGHTS) {
+    if (!p.d_w[slot]) return;
   }
   const int which = MODE == LayerProduct::INPUTS ? slot : slot >> 1;
   const int k_first = MODE == LayerProduct::WEIGHTS ? slice * p.slice_tokens : 0;
@@ -430,7 +434,7 @@ __global__ __launch_bounds__(256) void layer_norm_f32_kernel(LayerNormParams p) 
 // parts each.  Two regions in one launch (a launch costs more than either of them).
 struct LayerReduceParams {
   struct Region { const float *partial; long long n; int parts, blocks; } region[2];  // gate weights, convolution
-  float *d_w[4], *d_conv_w, *d_conv_b;
+  float *d_w[4], *d_conv_w, *d_conv_b;  // null: not wanted
   long long per_gate;
   int taps;
 };
@@ -451,12 +455,15 @@ __global__ __launch_bounds__(256) void layer_reduce_kernel(LayerReduceParams p) 
   if (wave || i >= r.n) return;
   s = (s + sums[0][lane]) + (sums[1][lane] + sums[2][lane]);
   if (which == 0) {
-    p.d_w[i / p.per_gate][i % p.per_gate] = s;
+    if (float *d_w = p.d_w[i / p.per_gate]) d_w[i % p.per_gate] = s;
   } else {
     const long long c = i / (p.taps + 1);
     const int j = (int)(i % (p.taps + 1));
-    if (j < p.taps) p.d_conv_w[c * p.taps + j] = s;
-    else if (p.d_conv_b) p.d_conv_b[c] = s;
+    if (j < p.taps) {
+      if (p.d_conv_w) p.d_conv_w[c * p.taps + j] = s;
+    } else if (p.d_conv_b) {
+      p.d_conv_b[c] = s;
+    }
   }
 }
 
