@@ -249,10 +249,16 @@ def test_out_of_memory_is_reported_as_such(trains):
     total = torch.cuda.get_device_properties(0).total_memory
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
+    large = torch.empty(2 << 30, dtype=torch.uint8, device=DEV)
+    del large
+    kept = torch.empty(2 << 20, dtype=torch.uint8, device=DEV)  # (a block with a tensor in it stays, whatever else of it is free)
+    torch.cuda.empty_cache()
+    free = torch.cuda.memory_reserved() - torch.cuda.memory_allocated()
+    assert free > kept.numel()
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)
     try:
         with torch.set_grad_enabled(trains), pytest.raises(torch.OutOfMemoryError):
-            held = [cell(x) for _ in range(64)]  # (16 MiB of outputs each)
+            held = [cell(x) for _ in range(64 + free // (16 << 20))]  # (16 MiB of outputs each)
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     with torch.set_grad_enabled(trains):
