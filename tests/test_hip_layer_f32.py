@@ -392,3 +392,44 @@ def test_frozen_parts_of_a_layer(frozen):
         torch.testing.assert_close(got, whole[n], rtol=0, atol=tol)
         torch.testing.assert_close(named[n].grad, whole[n], rtol=0, atol=tol)
     assert all(named[n].grad is None for n in named if n not in wanted)
+
+
+@pytest.mark.parametrize("own", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,S", [(1, 3), (4, 32), (3, 43), (8, 512)])
+def test_gradients_of_the_norm(B, S, dtype, own):
+    """A group norm's gradients against float64 on the CPU.  That of the weight is PyTorch's up to 128 tokens and wrong there beyond, of
+    which the call warns; with own_weight_gradient it is right at any number of them."""
+    import warnings
+
+    from xlstm_amd import layer as layer_module
+
+    print("case norm gradients", B, S, dtype, own, flush=True)
+    NH, dh = 2, 64
+    torch.manual_seed(B * S)
+    norm = layer_module.MultiHeadLayerNorm(NH * dh).to(DEV).to(dtype)
+    with torch.no_grad():
+        norm.weight.normal_(std=0.2)
+    norm.own_weight_gradient = own
+    y = torch.randn(S, B, NH, dh, device=DEV).to(dtype).permute(1, 2, 0, 3).requires_grad_(True)
+    d = torch.randn(B, NH, S, dh, device=DEV).to(dtype)
+    layer_module._warn_of_the_weight_gradient.cache_clear()
+    with warnings.catch_warnings(record=True) as said:
+        warnings.simplefilter("always")
+        for _ in range(2):
+            out = norm(y)
+        with torch.no_grad():
+            assert torch.equal(norm(y), out)  # (the same bits, whatever makes the gradient)
+    wrong = B * S > 128 and not own
+    assert sum("group norm" in str(w.message) for w in said) == wrong  # (once)
+    got = torch.autograd.grad(out, (y, norm.weight), d)
+    y64 = y.detach().double().cpu().requires_grad_(True)
+    scale = 1.0 + norm.weight.detach().cpu()  # (rounded to the module's type, as the module does)
+    w64 = scale.double().requires_grad_(True)
+    want64 = _norm64(y64.permute(2, 0, 1, 3).reshape(S, B, NH * dh), w64 - 1.0, norm.eps, NH).reshape(B, S, NH, dh).transpose(1, 2)
+    want = torch.autograd.grad(want64, (y64, w64), d.double().cpu())
+    # float32: a few sums of 64 products, then over 4096 tokens, whose rounding errors grow with the square root: 2^-24 times 8 + 64.
+    # bfloat16: results of float32 sums, rounded once
+    bound = 2.0 ** -24 * 72 if dtype == torch.float32 else 2.0 ** -8
+    for a, b in list(zip(got, want))[: 1 if wrong else 2]:
+        assert float((a.double().cpu() - b).norm() / b.norm()) <= bound

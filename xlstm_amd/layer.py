@@ -21,6 +21,8 @@ the causal convolution does not look across a document start either.
 """
 from __future__ import annotations
 
+import functools
+import warnings
 from dataclasses import dataclass
 from math import sqrt
 from typing import Optional
@@ -141,11 +143,40 @@ def _headwise(x: torch.Tensor, weight: torch.Tensor, num_heads: int) -> torch.Te
     return y.reshape(*shape[:-1], -1)
 
 
+#: Tokens (B*S) up to which the gradient of the weight that ``F.group_norm`` hands back on the GPU is right (PyTorch 2.10 on ROCm 7)
+_GROUP_NORM_GRADIENT_TOKENS = 128
+
+
+@functools.lru_cache(maxsize=None)
+def _warn_of_the_weight_gradient() -> None:
+    warnings.warn(f"the gradient of a group norm's weight that PyTorch hands back on this GPU is wrong beyond {_GROUP_NORM_GRADIENT_TOKENS} tokens "
+                  "(its error is as large as it is itself); set own_weight_gradient on the layer's group_norm, or freeze its weight", RuntimeWarning, stacklevel=4)
+
+
+class _WeightOfNorm(torch.autograd.Function):
+    """``out`` as it is; the gradient of the weight from the normalised input, in float32."""
+
+    @staticmethod
+    def forward(ctx, out, gn_in, weight, num_heads, eps):
+        ctx.save_for_backward(gn_in)
+        ctx.num_heads, ctx.eps, ctx.dtype = num_heads, eps, weight.dtype
+        return out.view_as(out)
+
+    @staticmethod
+    def backward(ctx, d_out):
+        gn_in, = ctx.saved_tensors
+        normed = F.group_norm(gn_in.float(), num_groups=ctx.num_heads, eps=ctx.eps)
+        return d_out, None, (d_out.float() * normed).sum(0).to(ctx.dtype), None, None
+
+
 class MultiHeadLayerNorm(nn.Module):
     """Per-head group norm of [B,NH,S,DH] with residual weight (components/ln.py:8-68).  Its gradients are PyTorch's.
     Measured with PyTorch 2.10 on ROCm 7: beyond 128 tokens (B*S) the gradient of the WEIGHT that ``F.group_norm`` hands back
-    on the GPU is off by its own size (relative 2-norm error 0.9 to 1.05 against float64 on the CPU; up to 128 tokens
-    2e-7; the gradient of the input is right throughout)."""
+    on the GPU is off by its own size (relative 2-norm error 0.95 to 1 against float64 on the CPU; up to 128 tokens
+    2e-7; the gradient of the input is right throughout).  A call that this would reach warns once per process."""
+
+    #: True: the gradient of the weight is not PyTorch's but a product and a sum over the tokens (6e-8 of float64's norm at 129 tokens)
+    own_weight_gradient: bool = False
 
     def __init__(self, ndim: int, weight: bool = True, eps: float = 1e-5):
         super().__init__()
@@ -157,6 +188,12 @@ class MultiHeadLayerNorm(nn.Module):
         B, NH, S, DH = x.shape
         gn_in = x.transpose(1, 2).reshape(B * S, NH * DH)
         w = None if self.weight is None else 1.0 + self.weight
+        if w is not None and w.requires_grad and gn_in.is_cuda:
+            if self.own_weight_gradient:
+                out = _WeightOfNorm.apply(F.group_norm(gn_in, num_groups=NH, weight=w.detach(), eps=self.eps), gn_in, w, NH, self.eps)
+                return out.view(B, S, NH, DH).transpose(1, 2)
+            if B * S > _GROUP_NORM_GRADIENT_TOKENS:
+                _warn_of_the_weight_gradient()
         out = F.group_norm(gn_in, num_groups=NH, weight=w, bias=None, eps=self.eps)
         return out.view(B, S, NH, DH).transpose(1, 2)
 
