@@ -66,3 +66,24 @@ def test_a_wait_that_runs_out_is_reported(bf16, B, NH, dh):
     h, _ = F.slstm_forward(*dev, train_coef=coef)
     with pytest.raises(F.EngineError):
         F.slstm_backward(*dev, h, d_h, d_sf, coef=coef, spin_limit=-1)
+
+
+@pytest.mark.parametrize("B,T,NH,dh", [(32, 256, 4, 1024), (12, 128, 8, 640)])
+def test_no_wait_goes_on_until_the_abort_word_is_read(B, T, NH, dh):
+    """Row tiles of 16 rows, head dims beyond 512: every wait ends with a look at the deltas, long before the 256th, behind which a
+    wave reads the abort word (16 looks suffice; a line left in the vector cache had waves wait for that)."""
+    from xlstm_amd import functional as F
+
+    print("case looks", B, T, NH, dh, flush=True)
+    H = NH * dh
+    torch.manual_seed(dh)
+    wx = torch.randn(B, T, 4 * H, device=DEV, dtype=torch.bfloat16)
+    r = ((torch.rand(NH, 4 * dh, dh, device=DEV) * 2 - 1) / H ** 0.5).bfloat16()
+    b = torch.zeros(NH, 4, dh, device=DEV)
+    d_h = torch.randn(T, B, H, device=DEV).bfloat16()
+    coef = F.training_coefficients(wx, NH)
+    h, _ = F.slstm_forward(wx, r, b, train_coef=coef)
+    want = F.slstm_backward(wx, r, b, None, None, h, d_h, coef=coef, d_wx_dtype=torch.bfloat16)
+    for _ in range(5):
+        got = F.slstm_backward(wx, r, b, None, None, h, d_h, coef=coef, d_wx_dtype=torch.bfloat16, spin_limit=200)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[3], want[3])

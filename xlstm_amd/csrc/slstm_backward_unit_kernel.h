@@ -66,6 +66,15 @@ constexpr int unit_bwd_lds_bytes(int rt, int ct, bool bf16) {
 // (6, 20) 2905, (9, 24) 2933; the others lose with more than (2, 8): 4 heads of 256, 6 rows, T 300 (2, 8) 558, (4, 10) 570, (6, 16) 597.
 constexpr int unit_bwd_sleep(int rt, int ct, int gq, bool published) { return rt == 8 && ct == 2 && gq == 4 ? (published ? 6 : 16) : (published ? 2 : 8); }
 
+// Whether a wave's own publication has to have reached the L2 before it looks, and a look that came back incomplete clears the compute
+// unit's vector cache.  A look that is under way while a store of the same compute unit goes through the same lines can leave
+// the old ones there, and looks that follow find those again: measured in row tiles of 16 rows at head dims beyond 512 (16 loads a
+// look), where such a wave went on until its 256th look read the abort word, 420 us (1,740 with that read every 1,024th, 60
+// every 32nd), in one of some hundred steps.  us a backward call of 128 steps, without / with both (the wait alone prevents it, the
+// clearing alone ends it with the next look): 4 heads of 1024 B 32 1452-1911 / 977-1000, B 128 5463-8569 / 3580-3640, 8 of 640 B 12
+// 4889-9293 / 700-720.  No other form showed it, and with both they gain nothing.
+constexpr bool unit_bwd_settles(bool bf16, int gq, int rt) { return bf16 && gq == 4 && rt == 16; }
+
 template <bool BF16, int GQ, int RT, int CT, bool DWX16>  // GQ: members of a wave's share of K (rounded up)
 __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(UnitBwdParams p) {
   static_assert(RT == 4 || (RT == 16 && BF16 == (CT == 2)) || (RT == 8 && CT == 2), "row tiles of 4, 8 (bf16) or 16 rows");
@@ -283,6 +292,7 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
           *reinterpret_cast<uint4 *>(old) = uint4{kSentinel32, kSentinel32, kSentinel32, kSentinel32};
         }
       }
+      if constexpr (unit_bwd_settles(BF16, GQ, RT)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       if (mine) {
         const long long o = wo + (long long)t * p.d_wx_st;
 #pragma unroll
@@ -321,6 +331,7 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
 #pragma unroll
             for (int i = 0; i < BATCH; ++i) mark = mark_join<BF16>(mark, chunk_mark<BF16>(areg[i]));
             if ((__builtin_amdgcn_ballot_w64(mark_has_sentinel<BF16>(mark)) == 0ull && p.spin_limit >= 0) || gave_up) break;
+            if constexpr (unit_bwd_settles(BF16, GQ, RT)) asm volatile("buffer_inv sc0" ::: "memory");
             if (++spins > p.spin_limit || ((spins & 255) == 0 && __hip_atomic_load(p.abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
               __hip_atomic_store(p.abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
               gave_up = true;
