@@ -1141,14 +1141,23 @@ int run_backward_params(const xs_slstm_bwd_args *a) {
     // shorter than four chunks
     const int cus = device_cus() > 0 ? device_cus() : 256;
     const long long base = (long long)a->NH * tiles;
-    // (4 or 8 per compute unit: 10 to 30 % slower.  float32, where one per compute unit fills the device, one: half the atomics; a training call
-    // at B 16 T 256 4 x 256 787 -> 761 us, B 30 T 100 4 x 512 1318 -> 1293; where the tiles alone are more, two: B 101 T 10 16 x 136 820 with one,
-    // 759 with two)
-    long long ks = slab || (!bf16 && base <= cus) ? cus / base : (2ll * cus + base - 1) / base;
-    if (ks < 1) ks = 1;
+    // (4 or 8 per compute unit: 10 to 30 % slower.)
     // (head, slice) groups are dealt out over the XCDs, group i on XCD i % 8: a multiple of 8 of them keeps every XCD
     // busy (4 heads of 1024 are 512 tiles and one slice each by the rule above: four XCDs idle, twice the time)
-    while ((a->NH * ks) % 8 != 0 && a->NH * ks < 64) ++ks;
+    auto whole_xcds = [&](long long k) {
+      if (k < 1) k = 1;
+      while ((a->NH * k) % 8 != 0 && a->NH * k < 64) ++k;
+      return k;
+    };
+    long long ks = whole_xcds(slab ? cus / base : (2ll * cus + base - 1) / base);
+    // float32, one per compute unit, half the atomics: with 256 columns a tile wherever the tiles alone are no more than that; with fewer columns
+    // where it fills the device exactly and a slice is short.  us, two -> one per compute unit: 4 x 256 B 32 T 256 206 -> 181, 6 x 256 373 -> 328,
+    // 8 x 512 1177 -> 1170; 8 x 128 B 6 T 250 (6 chunks a slice) 45.8 -> 38.5, 4 x 128 B 32 T 256 (16) 72.2 -> 69.0, B 100 T 128 (25) 80 -> 86, 16 x 128
+    // B 32 T 256 (64) 176 -> 183; not filled, or with a last round that is nearly empty: 8 x 192 283 -> 429, 4 x 384 452 -> 588
+    if (!slab && !bf16 && base <= cus) {
+      const long long one = whole_xcds(cus / base);
+      if (nt == 256 || (base * one == cus && nchunks < 20 * one)) ks = one;
+    }
     if (ks > nchunks / 4) ks = nchunks / 4;
     if (ks < 1) ks = 1;
     p.ksplit = (int)ks;
