@@ -1427,7 +1427,8 @@ PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
     PyErr_SetString(PyExc_KeyError, "an entry point of the engine is missing");
     return nullptr;
   }
-  // (whoever binds other entry points for the parts of a layer's step, to watch them or to stand in for them, has them called)
+  // (whoever binds other entry points for the parts of a layer's step that the one kernel stands for, to watch them or to stand in for
+  // them, has them called; the norm behind it is called either way)
   static const Engine first = g_engine;
   g_engine.own_parts = g_engine.step == first.step && g_engine.conv == first.conv && g_engine.gates == first.gates;
   for (int i = 1; i < 4; ++i) Py_INCREF(args[i]);

@@ -62,8 +62,10 @@ constexpr int unit_bwd_lds_bytes(int rt, int ct, bool bf16) {
 
 // s_sleep units (64 cycles each) in front of a wave's first look at the step's deltas: of the waves that have just published,
 // and of the others.  A look that comes back incomplete costs its whole round trip.  Head dim 1024 in row tiles of 8 rows has
-// the longest step (B 16 x T 512 x 4 heads, us a training call): (2, 8) 3006, (2, 12) 2924, (4, 12) 2917, (6, 16) 2881, (9, 16) 2883,
-// (6, 20) 2905, (9, 24) 2933; the others lose with more than (2, 8): 4 heads of 256, 6 rows, T 300 (2, 8) 558, (4, 10) 570, (6, 16) 597.
+// the longest step (us a training call; B 16 x T 512 x 4 heads: (2, 8) 3006, (2, 12) 2924, (4, 12) 2917, (6, 16) 2881, (9, 16) 2883,
+// (6, 20) 2905, (9, 24) 2933; other batches, lengths and head dims that run in this form, (2, 8) / (4, 12) / (6, 16) / (9, 24): B 16 T 128 872 / 857 /
+// 847 / 862, B 9 T 300 1630 / 1593 / 1563 / 1597, 4 heads of 768 B 16 T 512 2506 / 2476 / 2455 / 2542); the others lose with more than (2, 8):
+// 4 heads of 256, 6 rows, T 300 (2, 8) 558, (4, 10) 570, (6, 16) 597.
 constexpr int unit_bwd_sleep(int rt, int ct, int gq, bool published) { return rt == 8 && ct == 2 && gq == 4 ? (published ? 6 : 16) : (published ? 2 : 8); }
 
 // Whether a wave's own publication has to have reached the L2 before it looks, and a look that came back incomplete clears the compute

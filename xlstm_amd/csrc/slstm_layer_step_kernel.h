@@ -31,8 +31,10 @@ constexpr int layer_step_lds_bytes(int nq) { return 2 * 16 * layer_step_row_byte
 // UT 2: 32 units, eight waves; the convolution is made half as often, which counts where a compute unit has more than one
 // workgroup of UT 1.  LOOP: a workgroup keeps its weights and R in registers for several row tiles, the rows of the next one
 // on their way while this one is multiplied and gated.
-// What bounds it is the arithmetic of the convolution (150 instructions a wave and k-step) behind one latency of memory; the
-// times of both sides stand at layer_step_split.
+// What bounds it, 8 heads of 256 with the norm behind it, us a token at 256 / 64 rows: 20.6 / 10.9; without the convolution's arithmetic (150
+// instructions a wave and k-step) 20.0 / 10.6, without the products and the reads of their weights 16.4 / 8.1, without either 15.5 / 7.6.  So
+// most of it is the way in and out: a latency of memory in front of each row tile's work, x and the taps read once per unit tile, 34 MB
+// of states, ring and weights.  The times of both sides stand at layer_step_split.
 template <int NQ, int UT, bool HB, bool LOOP>  // NQ: MFMA k-steps of a quarter of K; HB: the recurrent operand comes from h_prev, in bf16
 __global__ __launch_bounds__(256 * UT, UT == 2 ? (NQ == 1 && !LOOP ? 4 : 2) : (NQ >= 4 ? 1 : 2)) void slstm_layer_step_kernel(LayerStepParams p) {
   constexpr int QS = 20;  // (see slstm_step_small_kernel)

@@ -27,8 +27,9 @@
 // Smaller heads (NCH 2 and 4: head dims 136 to 512) come here where two workgroups per compute unit make one row tile per workgroup of two, or
 // fewer launches; see the dispatch for both sides.
 //
-// Bound, at B 64 x 4 heads of 1024: a tile goes round once in two iterations of 3,500 cycles.  The compute unit's vector issue is busy for 2,000
-// of them (two workgroups' arrival tests, sums and gating), its matrix cores 1,024, its texture path 1,024 (64 KiB of operand).  The
+// Bound, at B 64 x 4 heads of 1024: a tile goes round once in two iterations of 3,400 cycles.  By its counters a SIMD's matrix unit is busy for
+// 1,023 of them and its vector unit issues for 1,200 (141 instructions a wave, arrival tests, sums and gating of two workgroups), and the data path of
+// the texture unit has something under way for 2,860 (64 KiB of operand a compute unit, waiting included): latencies, one behind the other.  The
 // later of two workgroups on a compute unit has no slack (300 arrival test, 900 MFMA, 850 sums and gating with the request, 650 stores and
 // W.x, 300 to 600 at the barrier), the earlier waits for its h.  Dropped: ONE workgroup of eight waves and 32 units with the operand
 // polled once and shared through LDS (half the texture traffic): 3.83 at B 64, 2.14 at B 16, because all eight waves then multiply,
