@@ -20,7 +20,7 @@
 extern "C" {
 #endif
 
-#define XS_ABI_VERSION 20
+#define XS_ABI_VERSION 21
 
 /* element types */
 enum { XS_F32 = 0, XS_BF16 = 1 };
@@ -242,6 +242,9 @@ typedef struct xs_conv_args {
 } xs_conv_args;
 
 int xs_causal_conv_silu(const xs_conv_args *args);
+/* the same for a token (ring_out required), which is left in x_out as well: [B,D] contiguous, overlapping x, conv_state,
+ * out and ring_out nowhere */
+int xs_causal_conv_silu_token(const xs_conv_args *args, void *x_out);
 
 /*
  * xs_headwise_gates: the four block-diagonal gate projections and their concatenation,

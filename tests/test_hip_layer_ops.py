@@ -106,6 +106,40 @@ def test_causal_conv_silu_step_writes_the_next_ring():
         hipF.causal_conv_silu(x, w, None, ring[:, 1:], ring_out=ring)  # in place is refused
 
 
+@pytest.mark.parametrize("B,D,K", [(1, 8, 2), (3, 64, 3), (37, 520, 4)])
+def test_a_token_is_left_in_another_buffer_too(B, D, K):
+    import ctypes
+
+    from xlstm_amd import _lib
+    from xlstm_amd import functional as hipF
+
+    print("case token out", B, D, K, flush=True)
+    torch.manual_seed(B)
+    memory = torch.randn(8 * B * K, D, device=DEV).bfloat16()  # (one allocation: what overlaps is known)
+    x, taps, out, ring, free = (memory[i * B * K:(i + 1) * B * K] for i in range(5))
+    w = torch.randn(D, K, device=DEV).bfloat16()
+    a = _lib.ConvArgs()
+    a.B, a.T, a.D, a.K, a.dtype = B, 1, D, K, _lib.XS_BF16
+    a.x, a.x_stride_b, a.x_stride_t, a.conv_state, a.weight, a.out = x.data_ptr(), D, D, taps.data_ptr(), w.data_ptr(), out.data_ptr()
+    a.stream = torch.cuda.current_stream().cuda_stream
+    call = _lib.load().xs_causal_conv_silu_token
+    assert call(ctypes.byref(a), free.data_ptr()) == -1  # goes with a ring
+    a.ring_out = ring.data_ptr()
+    assert call(ctypes.byref(a), None) == -1 and call(ctypes.byref(a), free.data_ptr() + 2) == -4
+    before = memory.clone()
+    last = {"x": x[B - 1:], "conv_state": taps[B * (K - 1) - 1:], "out": out[B - 1:], "ring_out": ring[B * K - 1:]}
+    for name, rows in last.items():
+        assert call(ctypes.byref(a), rows.data_ptr()) == -2 and name.encode() in _lib.load().xs_last_error(), name
+    torch.cuda.synchronize()
+    assert torch.equal(memory, before)
+    assert call(ctypes.byref(a), free.data_ptr()) == 0
+    torch.cuda.synchronize()
+    states = taps[:B * (K - 1)].view(B, K - 1, D)
+    want = hipF.causal_conv_silu(x[:B].view(B, 1, D), w, None, states)
+    assert torch.equal(free[:B], x[:B]) and torch.equal(free[B:], before[4 * B * K + B:5 * B * K])
+    assert torch.equal(out[:B], want[:, 0]) and torch.equal(ring.view(B, K, D), torch.cat([states, x[:B].view(B, 1, D)], 1))
+
+
 @pytest.mark.parametrize("lead,NH,dh", [
     ((2, 37), 4, 64),      # 64-token x 64-unit tiles, ragged token count
     ((3, 50), 2, 256),     # 64 x 128

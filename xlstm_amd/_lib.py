@@ -17,7 +17,7 @@ LIB_PATH = os.environ.get("XLSTM_AMD_LIB", os.path.join(PKG, "lib", "libxlstm_am
 XS_F32, XS_BF16 = 0, 1
 XS_ERR_UNSUPPORTED = -5
 STATIC_SCRATCH_BYTES = (4 << 20) + (64 << 10)
-ABI_VERSION = 20
+ABI_VERSION = 21
 
 EXPORTS = (
     "xs_abi_version",
@@ -33,6 +33,7 @@ EXPORTS = (
     "xs_slstm_backward_params",
     "xs_slstm_backward_tile_r",
     "xs_causal_conv_silu",
+    "xs_causal_conv_silu_token",
     "xs_headwise_gates",
     "xs_headwise_group_norm",
     "xs_layer_step_fits",
@@ -270,6 +271,8 @@ def load() -> ctypes.CDLL:
     lib.xs_slstm_tile_r_for_steps.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p]
     lib.xs_causal_conv_silu.restype = ctypes.c_int
     lib.xs_causal_conv_silu.argtypes = [ctypes.POINTER(ConvArgs)]
+    lib.xs_causal_conv_silu_token.restype = ctypes.c_int
+    lib.xs_causal_conv_silu_token.argtypes = [ctypes.POINTER(ConvArgs), ctypes.c_void_p]
     lib.xs_headwise_gates.restype = ctypes.c_int
     lib.xs_headwise_gates.argtypes = [ctypes.POINTER(GatesArgs)]
     lib.xs_headwise_group_norm.restype = ctypes.c_int
@@ -323,6 +326,7 @@ def host():
     mod = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(mod)
     names = ("xs_slstm_step", "xs_slstm_forward_watched", "xs_slstm_workspace_bytes", "xs_last_error", "xs_causal_conv_silu",
+             "xs_causal_conv_silu_token",
              "xs_headwise_gates", "xs_headwise_group_norm", "xs_slstm_train_coef_floats", "xs_slstm_train_exchange_bytes",
              "xs_slstm_train_forward", "xs_slstm_train_backward", "xs_slstm_backward_params", "xs_layer_step_fits", "xs_layer_step",
              "xs_layer_front", "xs_layer_norm",

@@ -43,6 +43,7 @@ struct Engine {
   decltype(&xs_slstm_workspace_bytes) workspace_bytes = nullptr;
   decltype(&xs_last_error) last_error = nullptr;
   decltype(&xs_causal_conv_silu) conv = nullptr;
+  decltype(&xs_causal_conv_silu_token) conv_token = nullptr;
   decltype(&xs_headwise_gates) gates = nullptr;
   decltype(&xs_headwise_group_norm) norm = nullptr;
   decltype(&xs_slstm_train_coef_floats) coef_floats = nullptr;
@@ -956,7 +957,7 @@ bool collect(PyObject *layer, PyObject *cell_path, const at::Tensor &x, LayerPar
   return p.K >= 2 && p.K <= 4 && records == train;
 }
 
-void run_conv(const LayerParts &p, const at::Tensor &x, const void *taps, int64_t taps_stride, const at::Tensor *mask, void *out, void *ring, void *stream) {
+void run_conv(const LayerParts &p, const at::Tensor &x, const void *taps, int64_t taps_stride, const at::Tensor *mask, void *out, void *ring, void *stream, void *x_out = nullptr) {
   xs_conv_args a{};
   a.B = (int32_t)x.size(0); a.T = (int32_t)x.size(1); a.D = (int32_t)p.D; a.K = (int32_t)p.K;
   a.dtype = XS_BF16;
@@ -965,7 +966,7 @@ void run_conv(const LayerParts &p, const at::Tensor &x, const void *taps, int64_
   a.weight = p.conv_w.data_ptr(); a.bias = p.conv_b.defined() ? p.conv_b.data_ptr() : nullptr;
   a.reset = mask ? (const uint8_t *)mask->data_ptr() : nullptr; a.reset_stride_b = mask ? mask->stride(0) : 0;
   a.out = out; a.ring_out = ring; a.stream = stream;
-  launched(g_engine.conv(&a));
+  launched(x_out ? g_engine.conv_token(&a, x_out) : g_engine.conv(&a));
 }
 void run_gates(const LayerParts &p, const at::Tensor &x, const void *x_conv, void *out, void *stream) {
   xs_gates_args a{};
@@ -1089,10 +1090,11 @@ PyObject *layer_step_(PyObject *const *args) {
       launched(g_engine.layer_step(&a));
     } else {
       at::Tensor wx = at::empty({B, 1, 4 * p.D}, opts), x_conv = at::empty({B, 1, p.D}, opts);
-      run_conv(p, x, taps, taps_stride, nullptr, x_conv.data_ptr(), ring.data_ptr(), stream);
+      const bool with_x = x_out && !overlap(taps, taps_bytes, *x_out);
+      run_conv(p, x, taps, taps_stride, nullptr, x_conv.data_ptr(), ring.data_ptr(), stream, with_x ? x_out->data_ptr() : nullptr);
       run_gates(p, x, x_conv.data_ptr(), wx.data_ptr(), stream);
       step.launch(wx);
-      if (x_out) {
+      if (x_out && !with_x) {
         at::NoGradGuard no_grad;
         x_out->copy_(x);
       }
@@ -1417,7 +1419,7 @@ PyObject *bind(PyObject *, PyObject *const *args, Py_ssize_t n) {
   };
   if (!get("xs_slstm_step", g_engine.step) || !get("xs_slstm_forward_watched", g_engine.forward) ||
       !get("xs_slstm_workspace_bytes", g_engine.workspace_bytes) || !get("xs_last_error", g_engine.last_error) ||
-      !get("xs_causal_conv_silu", g_engine.conv) || !get("xs_headwise_gates", g_engine.gates) || !get("xs_headwise_group_norm", g_engine.norm) ||
+      !get("xs_causal_conv_silu", g_engine.conv) || !get("xs_causal_conv_silu_token", g_engine.conv_token) || !get("xs_headwise_gates", g_engine.gates) || !get("xs_headwise_group_norm", g_engine.norm) ||
       !get("xs_slstm_train_coef_floats", g_engine.coef_floats) || !get("xs_slstm_train_exchange_bytes", g_engine.exchange_bytes) ||
       !get("xs_slstm_train_forward", g_engine.train_forward) || !get("xs_slstm_train_backward", g_engine.train_backward) ||
       !get("xs_slstm_backward_params", g_engine.backward_params) || !get("xs_layer_front", g_engine.layer_front) ||

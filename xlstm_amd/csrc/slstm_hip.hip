@@ -1209,9 +1209,18 @@ int check_conv(const xs_conv_args *a) {
   return XS_OK;
 }
 
-int run_conv(const xs_conv_args *a) {
+int run_conv(const xs_conv_args *a, void *x_out = nullptr) {
   const int rc = check_conv(a);
   if (rc != XS_OK || a->B == 0 || a->T == 0) return rc;
+  if (x_out) {
+    if (!a->ring_out) return fail(XS_ERR_NULL, "x_out goes with ring_out");
+    if ((uintptr_t)x_out % 16) return fail(XS_ERR_ALIGN, "x_out must be 16-byte aligned");
+    const long long row = 2ll * a->D, x_sb = a->B > 1 ? 2 * a->x_stride_b : 0, taps = (a->K - 1) * row, taps_sb = a->conv_state_stride_b ? 2 * a->conv_state_stride_b : taps;
+    const struct { const char *name; const void *p; long long bytes; } others[4] = {
+        {"x", a->x, (a->B - 1) * x_sb + row}, {"conv_state", a->conv_state, a->conv_state ? (a->B - 1) * taps_sb + taps : 0}, {"out", a->out, a->B * row}, {"ring_out", a->ring_out, a->B * a->K * row}};
+    for (const auto &o : others)
+      if ((uintptr_t)x_out < (uintptr_t)o.p + o.bytes && (uintptr_t)o.p < (uintptr_t)x_out + a->B * row) return fail(XS_ERR_SHAPE, "x_out must not overlap %s", o.name);
+  }
   const long long threads = (long long)a->B * a->T * (a->D / 8);
   const long long blocks = ((threads + 255) / 256 + 7) / 8 * 8;  // a multiple of 8: the kernel deals them out by XCD
   if (blocks > 0x7FFFFFFF) return fail(XS_ERR_UNSUPPORTED, "too many tokens for one launch");
@@ -1222,7 +1231,7 @@ int run_conv(const xs_conv_args *a) {
   p.w = (const uint16_t *)a->weight; p.bias = (const uint16_t *)a->bias;
   p.reset = a->reset; p.reset_sb = a->reset_stride_b;
   p.out = (uint16_t *)a->out;
-  p.ring_out = (uint16_t *)a->ring_out;
+  p.ring_out = (uint16_t *)a->ring_out; p.x_out = (uint16_t *)x_out;
   p.B = a->B; p.T = a->T; p.D = a->D;
   hipStream_t stream = (hipStream_t)a->stream;
   void (*kern)(ConvParams) = a->K == 2 ? causal_conv_silu_kernel<2> : (a->K == 3 ? causal_conv_silu_kernel<3> : causal_conv_silu_kernel<4>);
@@ -1788,6 +1797,12 @@ int xs_slstm_backward_tile_r(const xs_slstm_bwd_args *args) {
 int xs_causal_conv_silu(const xs_conv_args *args) {
   g_err[0] = 0;
   return run_conv(args);
+}
+
+int xs_causal_conv_silu_token(const xs_conv_args *args, void *x_out) {
+  g_err[0] = 0;
+  if (!x_out) return fail(XS_ERR_NULL, "x_out is required");
+  return run_conv(args, x_out);
 }
 
 int xs_headwise_gates(const xs_gates_args *args) {

@@ -27,6 +27,7 @@ struct ConvParams {
   long long reset_sb;
   uint16_t *out;          // [B, T, D]
   uint16_t *ring_out;     // [B, KS, D] or null (T == 1): the inputs of the taps, oldest first
+  uint16_t *x_out;        // [B, D] or null (with ring_out): x
   int B, T, D;
 };
 
@@ -89,6 +90,7 @@ __global__ __launch_bounds__(256) void causal_conv_silu_kernel(ConvParams p) {
     if (p.ring_out) {  // (T == 1, no mask: `alive` holds; a missing state reads as zeros)
       const uint4 v = src ? *reinterpret_cast<const uint4 *>(src) : make_uint4(0, 0, 0, 0);
       *reinterpret_cast<uint4 *>(p.ring_out + ((long long)b * KS + j) * p.D + c0) = v;
+      if (back == 0 && p.x_out) *reinterpret_cast<uint4 *>(p.x_out + (long long)b * p.D + c0) = v;
     }
     if (src) {
       const uint4 v = *reinterpret_cast<const uint4 *>(src);
