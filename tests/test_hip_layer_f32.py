@@ -244,6 +244,23 @@ def test_inference_continues_from_states():
     torch.testing.assert_close(torch.cat([first, second], 1), whole, rtol=1e-5, atol=1e-5)
 
 
+def test_inputs_off_the_16_bytes_of_the_kernels():
+    """x as a contiguous view that starts 4 bytes into an allocation: laid out again, as a view with other strides is."""
+    from xlstm_amd.layer import sLSTMLayer, sLSTMLayerConfig
+
+    print("case misaligned", flush=True)
+    torch.manual_seed(3)
+    layer = sLSTMLayer(sLSTMLayerConfig(embedding_dim=96, num_heads=3, backend="hip", recurrent_weight_init="standard")).to(DEV).eval()
+    x = torch.randn(2, 9, 96, device=DEV)
+    off = torch.empty(x.numel() + 1, device=DEV)[1:].view(x.shape).copy_(x)
+    assert off.is_contiguous() and off.data_ptr() % 16
+    with torch.no_grad():
+        want, states = layer(x, return_last_state=True)
+        got, got_states = layer(off, return_last_state=True)
+    assert torch.equal(got, want) and torch.equal(got_states["slstm_state"], states["slstm_state"])
+    assert torch.equal(got_states["conv_state"], states["conv_state"])
+
+
 def test_what_wants_the_modules_one_by_one_gets_them():
     print("case layer f32 modules", flush=True)
     layer = _layer(2, 64)

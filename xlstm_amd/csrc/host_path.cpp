@@ -1139,7 +1139,7 @@ PyObject *layer_forward_(PyObject *const *args) {
     at::Tensor mask;
     if (mask_in) mask = mask_bytes(*mask_in);
     const at::Tensor *maskp = mask_in ? &mask : nullptr;
-    at::Tensor x = x_in.is_contiguous() && aligned(x_in.data_ptr(), 16) ? x_in : x_in.contiguous();
+    const at::Tensor x = p.float32 ? laid_out(x_in) : x_in.contiguous();  // (bf16: a misaligned x is refused, as by the kernels' own entry points)
     void *stream = stream_of(x.device());
     at::Tensor wx = at::empty({B, T, 4 * p.D}, x.options()), x_conv = at::empty({B, T, p.D}, x.options());
     out = x_conv;  // (its last reader has been launched in front of the norm)
