@@ -106,6 +106,35 @@ def test_causal_conv_silu_step_writes_the_next_ring():
         hipF.causal_conv_silu(x, w, None, ring[:, 1:], ring_out=ring)  # in place is refused
 
 
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("dtype,NH,dh,K", [(torch.float32, 3, 40, 4), (torch.float32, 2, 64, 2), (torch.bfloat16, 2, 64, 4), (torch.bfloat16, 1, 128, 3)])
+def test_one_convolution_state_for_all_rows(dtype, NH, dh, K, native, monkeypatch):
+    """A state expanded over the batch (rows of stride 0): the same as its copies, in sequences and in steps, through the native host path
+    and the kernels of the parts.  (float32: such a call takes PyTorch's operations around the cell, whose sums round in another order.)"""
+    from xlstm_amd.layer import sLSTMLayer, sLSTMLayerConfig
+
+    print("case shared conv state", dtype, NH, dh, K, native, flush=True)
+    torch.manual_seed(K)
+    B, D = 5, NH * dh
+    layer = sLSTMLayer(sLSTMLayerConfig(embedding_dim=D, num_heads=NH, conv1d_kernel_size=K, backend="hip", recurrent_weight_init="standard")).to(DEV, dtype).eval()
+    layer.slstm_cell.keep_state_fp32 = True
+    if not native:
+        monkeypatch.setattr(layer, "_own_modules", lambda: False)
+    x = torch.randn(B, 6, D, device=DEV).to(dtype)
+    token = torch.randn(B, 1, D, device=DEV).to(dtype)
+    rows = [torch.randn(1, n, D, device=DEV).to(dtype).expand(B, n, D) for n in (K - 1, K)]
+    overlapping = torch.randn((B + K) * D, device=DEV).to(dtype).as_strided((B, K - 1, D), (max(D // 8 * 8, 8), D, 1))
+    tolerance = dict(rtol=1e-5, atol=1e-5) if dtype == torch.float32 else dict(rtol=0, atol=0)
+    with torch.no_grad():
+        state = layer(x, return_last_state=True)[1]["slstm_state"].float()
+        for taps in (*rows, overlapping):
+            torch.testing.assert_close(layer(x, conv_state=taps), layer(x, conv_state=taps.contiguous()), **tolerance)
+            for _ in range(2):  # (the second on the plan of the first)
+                got, want = (layer.step(token, conv_state=(t,), slstm_state=state) for t in (taps, taps.contiguous()))
+                torch.testing.assert_close(got[0], want[0], **tolerance)
+                assert torch.equal(got[1]["conv_state"][0], want[1]["conv_state"][0])
+
+
 @pytest.mark.parametrize("B,D,K", [(1, 8, 2), (3, 64, 3), (37, 520, 4)])
 def test_a_token_is_left_in_another_buffer_too(B, D, K):
     import ctypes

@@ -1012,6 +1012,7 @@ bool taps_of(const LayerParts &p, const at::Tensor &t, int64_t B, const void *&t
   if (t.scalar_type() != (p.float32 ? at::kFloat : at::kBFloat16) || n < p.K - 1 || t.size(0) != B || t.size(2) != p.D || t.stride(2) != 1 ||
       t.stride(1) != p.D || t.stride(0) * esz % 16 || !t.is_cuda() || !aligned(t.data_ptr(), 16))
     return false;
+  if (B > 1 && t.stride(0) < (p.K - 1) * p.D) return false;  // (rows that share memory, one state for all of them: laid out by the general path)
   stride = t.stride(0);
   taps = (const char *)t.data_ptr() + (n - (p.K - 1)) * p.D * esz;
   return true;

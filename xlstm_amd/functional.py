@@ -749,7 +749,8 @@ def causal_conv_silu(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
         if tuple(conv_state.shape) != (B, K - 1, D):
             raise ValueError(f"conv_state must be [B, K-1, D] = {(B, K - 1, D)}, got {tuple(conv_state.shape)}")
         if (conv_state.dtype != torch.bfloat16 or conv_state.stride(2) != 1 or conv_state.stride(1) != D
-                or conv_state.stride(0) % 8 or conv_state.data_ptr() % 16):  # a [:, :K-1] view of a ring is taken as it is
+                or conv_state.stride(0) % 8 or (B > 1 and conv_state.stride(0) < (K - 1) * D)
+                or conv_state.data_ptr() % 16):  # a [:, :K-1] view of a ring is taken as it is, rows that share memory are not
             conv_state = conv_state.to(torch.bfloat16).contiguous()
     if reset_mask is not None:
         reset_mask = _mask_u8(reset_mask, B, T)
