@@ -8,8 +8,8 @@
 // `member` owns 16 CT output units of a tile of RT = 4, 8 or 16 batch rows: SIXTEEN with four compute waves (CT 1), or in
 // bf16 32 with eight (CT 2), which keeps a head of 1024 on one XCD and halves what a larger batch polls.  Per step:
 //   - the lanes that own an element (row, unit) add up the waves' partial sums of what reached its y from the step
-//     behind, form the step's gradient and publish the four gate deltas in the group's slot of an exchange ring:
-//     [member][row][unit][gate], so K is ordered (unit, gate);
+//     behind, form the step's gradient and publish the four gate deltas in the group's slot of an exchange ring, in the order
+//     in which a look's lanes take them (unit_bwd_word; K is ordered (unit, gate));
 //   - wave w polls the deltas of a quarter (CT 2: an eighth) of the members straight into MFMA operand registers (a word is
 //     data or the "not written yet" pattern; the publisher re-arms its words of two steps ago, as in the forward's ring),
 //     multiplies them by its share of R transposed and leaves its partial sums in LDS (two sets of tiles, one barrier a step).
@@ -41,7 +41,7 @@ struct UnitBwdParams {
   void *d_wx;
   long long d_wx_sb, d_wx_st;
   float *d_s0;
-  char *xch;                 // exchange ring [kBwdRing][groups of the launch][member][RT rows][16 CT units][4 gates]
+  char *xch;                 // exchange ring [kBwdRing][groups of the launch][slot]: unit_bwd_slot_members() x RT rows x 16 CT units x 4 gates
   unsigned int *abort_word, *placement;
   unsigned int *abort_host;  // a pinned host word that a wait that ran out is reported in, or null
   long long spin_limit;
@@ -58,6 +58,27 @@ constexpr int unit_bwd_burst(int rt, int ct) { return rt * ct <= 4 ? 8 : (rt * c
 constexpr int unit_bwd_slot(int rt, int ct, bool bf16) { return rt / 4 * ct * 2304 + rt * 16 * ct * (bf16 ? 2 : 4) + rt * 4; }
 constexpr int unit_bwd_lds_bytes(int rt, int ct, bool bf16) {
   return 2 * 4 * ct * rt * unit_part_stride(ct) * 4 + 2 * unit_bwd_burst(rt, ct) * unit_bwd_slot(rt, ct, bf16);
+}
+
+// A slot of the exchange ring: pieces of 1 KiB, each what ONE load of a look brings, lane after lane.  (With the words as [member][row]
+// [unit][gate] the lanes of a load lay 256 bytes apart, and a compute unit's address path, which takes a line a cycle, was what a
+// step waited for: float32 at 8 x 512, 10 rows, looks of 10,200 of 14,600 cycles, 6,300 now.  us a training call, that order -> this one: bf16
+4 x 1024 B 16 T 512 2,724 -> 2,585, 4 x 768 B 20 T 384 3,046 -> 2,295, 3 x 768 B 200 T 52 3,149 -> 2,418, float32 8 x 512 B 10 T 384 4,264 -> 3,561,
+3 x 256 B 4 T 130 381 -> 327, 4 x 96 B 6 T 250 459 -> 434, of these two 128 and 64 cycles a step by the second chain of MFMAs.)  bf16: a piece of K is 8 units = an MFMA's 32
+// inputs, PK = 16 / RT of them share a load: lane (unit pair q, row x PK + piece % PK), 16 bytes.  float32: 16 units of a set of
+// four rows: lane (unit / 4, unit % 4, row), 16 bytes.
+__host__ __device__ constexpr int unit_bwd_slot_members(int members, int rt, int ct, bool bf16) {
+  return bf16 && rt * ct == 4 ? members + (members & 1) : members;  // (a load brings two members there: an odd last one has an empty neighbour)
+}
+template <bool BF16, int RT, int CT>
+__device__ __forceinline__ int unit_bwd_word(int member, int row, int pu) {  // where the deltas of (row, unit pu of a member) lie in a slot
+  if constexpr (BF16) {
+    constexpr int PK = 16 / RT;
+    const int piece = member * 2 * CT + (pu >> 3);
+    return piece / PK * 1024 + (((pu >> 1) & 3) * 16 + row * PK + piece % PK) * 16 + (pu & 1) * 8;
+  } else {
+    return (member * (RT / 4) + (row >> 2)) * 1024 + (pu * 4 + (row & 3)) * 16;
+  }
 }
 
 // s_sleep units (64 cycles each) in front of a wave's first look at the step's deltas: of the waves that have just published,
@@ -85,8 +106,7 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
   constexpr int ESZ = BF16 ? 2 : 4;
   constexpr int NW = 4 * CT;                  // compute waves
   constexpr int UW = 16 * CT;                 // units of a member
-  constexpr int EB = UW * 4 * ESZ;            // bytes of a member's row: its units x 4 gates
-  constexpr int MB = RT * EB;                 // ... of a member
+  constexpr int MB = RT * UW * 4 * ESZ;       // bytes a member publishes a step
   constexpr int SETS = RT / 4;
   constexpr int BL = unit_bwd_burst(RT, CT), SLOTB = unit_bwd_slot(RT, CT, BF16);
   constexpr int PSTRIDE = unit_part_stride(CT), PWAVE = RT * PSTRIDE;
@@ -94,7 +114,8 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
   constexpr int NLD = BF16 ? 2 * CT * GQ : GQ;  // 16-byte pieces of deltas a lane polls per step (float32: per set of four rows)
   // bf16, row tiles of fewer than 16 rows: PK MFMA rows per batch row, each of which takes another piece, so that a load has
   // no lane without a row; NPL loads for the NLD pieces
-  constexpr int PK = BF16 ? 16 / RT : 1, NPL = (NLD + PK - 1) / PK;
+  constexpr int PK = BF16 ? 16 / RT : 1, NPL = NLD / PK;
+  static_assert(NLD % PK == 0, "whole loads");
   constexpr int BATCH = NPL < 16 ? NPL : 16;  // ... in one go
   constexpr int NPASS = BF16 ? 1 : SETS;
   extern __shared__ __attribute__((aligned(1024))) unsigned char unit_lds[];
@@ -216,21 +237,18 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
   if (mine && p.d_s_final) { dy = p.d_s_final[so]; dc = p.d_s_final[BH + so]; dn = p.d_s_final[2 * BH + so]; }
   const long long wo = (long long)(row < p.B ? row : p.B - 1) * p.d_wx_sb + head * dh + (a < dh ? a : dh - 1);
 
-  const int xslot = p.G * MB;
+  const int xslot = unit_bwd_slot_members(p.G, RT, CT, BF16) * MB;
   char *const ring = p.xch + (long long)gi * xslot;
   const long long ring_stride = (long long)ngroups * xslot;
-  const int pub = member * MB + prow * EB + pu * 4 * ESZ;
-  // poll: bf16: piece j: member wave GQ + j / (2 CT), units 8 (j % (2 CT)) + 2 q, + 1 of a batch row; MFMA row r16 holds pieces
-  // r16 % PK, + PK, ... of batch row r16 / PK; float32: piece c: member wave GQ + c, unit 4 q + r16 / 4 of row r16 % 4.  Members
-  // past the last one and pieces that are another wave's lie past the end of the descriptor: zeros
-  int vo;
-  if constexpr (BF16) {
-    const int j = r16 % PK;
-    vo = j < NLD ? r16 / PK * EB + q * 16 + j / (2 * CT) * MB + j % (2 * CT) * 64 : 0x40000000;
-  } else {
-    vo = (r16 & 3) * EB + q * 64 + (r16 >> 2) * 16;
+  const int pub = unit_bwd_word<BF16, RT, CT>(member, prow, pu);
+  // poll: bf16: load i: pieces PK i, + 1, ... of the wave's share, MFMA row r16 holds piece r16 % PK of batch row r16 / PK; float32: piece c of
+  // set s: member wave GQ + c, unit 4 q + r16 / 4 of row r16 % 4.  Members past the last one lie past the end of the descriptor: zeros
+  const int vo = wave * GQ * MB + lane * 16;
+  if (BF16 && unit_bwd_slot_members(p.G, RT, CT, BF16) != p.G && member == p.G - 1 && grad_wave) {
+    // (the empty neighbour's words are polled like the others: zeros)
+#pragma unroll
+    for (int i = 0; i < kBwdRing; ++i) *reinterpret_cast<unsigned long long *>(ring + i * ring_stride + unit_bwd_word<BF16, RT, CT>(p.G, prow, pu)) = 0ull;
   }
-  vo += wave * GQ * MB;
 
   f32x4 cA{0, 0, 0, 0}, cB{0, 0, 0, 0};
   float cC = 0.0f, dht = 0.0f;
@@ -315,9 +333,10 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
       for (int ps = 0; ps < NPASS; ++ps) {
         // bf16: a chain per column tile and MFMA row of a batch row (RT 16: four chains, CT 2: two per column tile)
         constexpr int CH = PK == 1 ? 4 / CT : PK;
-        f32x4 acc[BF16 ? CT * CH : 1];
+        // (float32: two, a v_mfma_f32_4x4x1 behind one that it adds to issues after 12 cycles instead of 8)
+        f32x4 acc[BF16 ? CT * CH : 2];
 #pragma unroll
-        for (int i = 0; i < (BF16 ? CT * CH : 1); ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int i = 0; i < (BF16 ? CT * CH : 2); ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int b0 = 0; b0 < NPL; b0 += BATCH) {
           uint4 areg[BATCH];
@@ -325,8 +344,7 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
           for (;;) {
 #pragma unroll
             for (int i = 0; i < BATCH; ++i) {
-              const int j = (b0 + i) * PK;
-              const int off = BF16 ? j / (2 * CT) * MB + j % (2 * CT) * 64 : j * MB + ps * 4 * EB;
+              const int off = BF16 ? (b0 + i) * 1024 : (b0 + i) * MB + ps * 1024;
               areg[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, vo + off, 0, 16));
             }
             uint32_t mark = 0u;
@@ -359,9 +377,9 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
 #pragma unroll
               for (int g = 0; g < 4; ++g) {
                 acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(dv[g], rr[g], acc[0], 2, 0, 0);
-                acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(dv[g], rr[4 + g], acc[0], 2, 1, 0);
+                acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(dv[g], rr[4 + g], acc[1], 2, 1, 0);
                 acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(dv[g], rr[8 + g], acc[0], 2, 2, 0);
-                acc[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(dv[g], rr[12 + g], acc[0], 2, 3, 0);
+                acc[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(dv[g], rr[12 + g], acc[1], 2, 3, 0);
               }
             }
           }
@@ -383,7 +401,7 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
               tiles[(4 * q + i) / PK * PSTRIDE + 16 * ct + r16] = sum;
             }
         } else {
-          float x0 = acc[0][0], x1 = acc[0][1], x2 = acc[0][2], x3 = acc[0][3];
+          float x0 = acc[0][0] + acc[1][0], x1 = acc[0][1] + acc[1][1], x2 = acc[0][2] + acc[1][2], x3 = acc[0][3] + acc[1][3];
           transpose_lane_groups(x0, x1, x2, x3);
           tiles[(4 * ps + q) * PSTRIDE + r16] = ((x0 + x1) + x2) + x3;
         }

@@ -419,7 +419,8 @@ int unit_plan(int B, int NH, int dh, bool bf16, UnitPlan &u) {
   if (!found) return fail(XS_ERR_DEVICE, "a head of %d units does not fit the compute units of this device's XCDs", dh);
   return XS_OK;
 }
-inline size_t unit_ring_bytes(const UnitPlan &u, int esz) { return (size_t)kBwdRing * u.heads * u.groups * u.G * u.RT * 64 * u.CT * esz; }
+inline size_t unit_slot_bytes(const UnitPlan &u, int esz) { return (size_t)unit_bwd_slot_members(u.G, u.RT, u.CT, esz == 2) * u.RT * 64 * u.CT * esz; }
+inline size_t unit_ring_bytes(const UnitPlan &u, int esz) { return kBwdRing * u.heads * u.groups * unit_slot_bytes(u, esz); }
 
 template <bool BF16, int RT, int CT, bool DWX16>
 void (*pick_unit_bwd(int gq))(UnitBwdParams) {
@@ -477,7 +478,7 @@ int run_unit_backward(const xs_slstm_bwd_args *a, int64_t d_h_sb, int64_t d_h_st
       p.b0 = b0; p.bend = b0 + u.RT * u.groups < a->B ? b0 + u.RT * u.groups : a->B;
       p.NBT = (p.bend - b0 + u.RT - 1) / u.RT;
       const int ng = p.NHL * p.NBT;
-      const long long n16 = (long long)kBwdRing * ng * u.G * u.RT * 64 * u.CT * esz / 16;
+      const long long n16 = (long long)kBwdRing * ng * (long long)unit_slot_bytes(u, esz) / 16;
       hipLaunchKernelGGL(slstm_bwd_arm_kernel, dim3((unsigned)((n16 + 255) / 256 < 1024 ? (n16 + 255) / 256 : 1024)), dim3(256), 0, stream,
                          (uint4 *)p.xch, n16, first ? p.abort_word : p.placement, ng + (first ? 1 : 0));
       first = false;
