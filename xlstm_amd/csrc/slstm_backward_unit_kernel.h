@@ -63,8 +63,8 @@ constexpr int unit_bwd_lds_bytes(int rt, int ct, bool bf16) {
 // A slot of the exchange ring: pieces of 1 KiB, each what ONE load of a look brings, lane after lane.  (With the words as [member][row]
 // [unit][gate] the lanes of a load lay 256 bytes apart, and a compute unit's address path, which takes a line a cycle, was what a
 // step waited for: float32 at 8 x 512, 10 rows, looks of 10,200 of 14,600 cycles, 6,300 now.  us a training call, that order -> this one: bf16
-4 x 1024 B 16 T 512 2,724 -> 2,585, 4 x 768 B 20 T 384 3,046 -> 2,295, 3 x 768 B 200 T 52 3,149 -> 2,418, float32 8 x 512 B 10 T 384 4,264 -> 3,561,
-3 x 256 B 4 T 130 381 -> 327, 4 x 96 B 6 T 250 459 -> 434, of these two 128 and 64 cycles a step by the second chain of MFMAs.)  bf16: a piece of K is 8 units = an MFMA's 32
+// 4 x 1024 B 16 T 512 2,724 -> 2,585, 4 x 768 B 20 T 384 3,046 -> 2,295, 3 x 768 B 200 T 52 3,149 -> 2,418, float32 8 x 512 B 10 T 384 4,264 -> 3,561,
+// 3 x 256 B 4 T 130 381 -> 327, 4 x 96 B 6 T 250 459 -> 434, of these two 128 and 64 cycles a step by the second chain of MFMAs.)  bf16: a piece of K is 8 units = an MFMA's 32
 // inputs, PK = 16 / RT of them share a load: lane (unit pair q, row x PK + piece % PK), 16 bytes.  float32: 16 units of a set of
 // four rows: lane (unit / 4, unit % 4, row), 16 bytes.
 __host__ __device__ constexpr int unit_bwd_slot_members(int members, int rt, int ct, bool bf16) {
