@@ -144,6 +144,15 @@ __device__ __forceinline__ uint32_t seq_handshake(const SeqParams &p, int wg, in
   return cross ? 1u : 0u;
 }
 
+// Row tiles of 4 rows (QUAD): the byte of a ring slot at which the h of (unit of the head, row of the tile) lies.  Piece c holds chunk c of each
+// quarter of K, 16 bytes per (unit group q, row, quarter) in bf16 and per (quarter, unit group, row) in float32.
+template <bool BF16, int NCH>
+__device__ __forceinline__ int quad_word(int unit, int row) {
+  const int chunk = unit >> (BF16 ? 5 : 4), quarter = chunk / NCH, piece = chunk % NCH;
+  if constexpr (BF16) return piece * 1024 + (((unit >> 3) & 3) * 16 + row * 4 + quarter) * 16 + (unit & 7) * 2;
+  else return piece * 1024 + (quarter * 16 + ((unit >> 2) & 3) * 4 + row) * 16 + (unit & 3) * 4;
+}
+
 // FULL: the head dim fills the K range of the four waves exactly (dh == 16 * NCH * elements per chunk) and, with
 // more than one row tile, every batch row of every tile exists.  The per-chunk "is this chunk needed" masks of
 // the arrival test are then compiled out (with one row tile, lanes of rows that do not exist read zeros from
@@ -480,10 +489,11 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
   // with the batch rows at MFMA rows 0, 4, 8, 12 and zeros between it was 8, three quarters of their lanes empty, and the
   // loads of the four waves held each other up in the compute unit's one return path (us a call, before -> after: B 16 x T 2048 x 4 heads
   // of 256 1527 -> 1464, a layer at B 7 x T 333 x 4 heads of 192 286 -> 257, B 1 x T 500 x 8 heads of 256 379 -> 310).  The barrier of the step (the
-  // feeder's W.x, the drainer's h) is passed in front of the poll.  The exchange ring is [slot][member][4 rows]
-  // [16 units]: the group's h of a step is 8 dh bytes (float32: 16 dh) in a row.
-  // Without FULL the K range ends inside the four quarters: members past the last one lie past the end of the descriptor
-  // and read zeros, and units past the head dim publish zeros (they are polled like the others).
+  // feeder's W.x, the drainer's h) is passed in front of the poll.  A slot of the exchange ring is NCH pieces of 1 KiB, each what
+  // one load of a poll brings, lane after lane (quad_word): with [member][4 rows][16 units], where the lanes of a load lay 32 or
+  // more bytes apart, a load took the address path of a compute unit up to four times as long.
+  // Without FULL the K range ends inside the four quarters: lanes whose member is past the last one read past the end of the descriptor,
+  // zeros, and units past the head dim publish zeros (they are polled like the others).
   // float32 multiplies with v_mfma_f32_4x4x1, whose 16 blocks are 4 groups of columns x 4 quarters of K: a tile of 4 rows
   // without padding takes a quarter of the cycles of v_mfma_f32_16x16x4 (head dim 128: 256 instead of 1,024 per wave and
   // step), the operand is broadcast inside a quarter by the instruction, so that a lane polls only its own 16 bytes per 16
@@ -573,10 +583,8 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
 #endif
     lds_barrier();  // prologue barrier
     const bool cross = cross_s != 0u;
-    constexpr int QTILE = 4 * 16 * ESZ;        // bytes a member publishes per step
     constexpr int NP = NCH;                    // 16-byte pieces of the group's h a lane polls per step
-    constexpr int PSTEP = BF16 ? 2 * QTILE : QTILE;  // ... and the distance between them
-    const int xslot = p.G * QTILE;
+    constexpr int xslot = NP * 1024;           // (the host's G members of 16 rows are more)
     char *const xbase = reinterpret_cast<char *>(p.xbuf) + (long long)gi * kRing * xslot;
     // operand: lane (q, MFMA row r16) holds batch row r16 / 4 and quarter r16 % 4 of K: chunk c of the quarter, units
     // 32 (NCH (r16 % 4) + c) + 8 q .. + 7 = member 2 (NCH (r16 % 4) + c) + q / 2, its units 8 (q % 2) .. + 7
@@ -584,12 +592,18 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
     const int orow = BF16 ? r16 >> 2 : r16 & 3;   // the batch row of the tile in this lane's operand
     const int arow = rowbase + orow;
     const bool a_lane = arow < rend;
-    const int xl = !a_lane ? 0x7FFFFF00 : (BF16 ? (2 * NCH * (r16 & 3) + (q >> 1)) * QTILE + orow * 32 + (q & 1) * 16 : q * NCH * QTILE + orow * 64 + (r16 >> 2) * 16);
-    const long long xo = (long long)member * (QTILE / ESZ) + gb * 16 + gu;
+    int xl[FULL ? 1 : NP];
+#pragma unroll
+    for (int c = 0; c < (FULL ? 1 : NP); ++c)
+      xl[c] = a_lane && (FULL || (BF16 ? 2 * (NCH * (r16 & 3) + c) + (q >> 1) : q * NCH + c) < p.G) ? c * 1024 + lane * 16 : 0x7FFFFF00;
+    auto poll = [&](const __amdgpu_buffer_rsrc_t &rs, int c) {
+      return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, xl[FULL ? 0 : c], FULL ? c * 1024 : 0, 16));
+    };
+    const int xo = quad_word<BF16, NCH>(a0 + gu, gb) / ESZ;
     typedef typename std::conditional<BF16, uint16_t, uint32_t>::type word_t;
     constexpr word_t kMissing = BF16 ? (word_t)kSentinel16 : (word_t)kSentinel32;
 #ifndef XS_QUAD_PAD
-#define XS_QUAD_PAD 4
+#define XS_QUAD_PAD (BF16 ? 6 : 0)
 #endif
     asm volatile(".p2align 5\n\t.rept %0\n\ts_nop 0\n\t.endr" :: "n"(XS_QUAD_PAD));
     for (int t = 0; t < p.T; ++t) {
@@ -605,9 +619,12 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
       // barrier (1.52 - 1.53) - but the issue slots: a wave asleep leaves its SIMD to the feeder, drainer and prefetch
       // waves, which these waves' raised priority otherwise keeps waiting (no s_sleep but priority 0 from the barrier
       // to the poll: 1.53).  Then the loop's start moved over the eight phases of a 32-byte line of code:
-      // 1.517 .. 1.573, the best one taken.  (K split over the waves, below: 1.70.)  With the shorter polls, ms: 1.457 with one
-      // s_sleep, 1.52 with two, 1.60 with three; head dim 512 (B 4 x T 700), whose peers come later, 0.77, 0.73 and 0.76.  One
-      // barrier for two or four steps, W.x and h in rings of as many: 1.51 and 1.55 (the waves beside these then come in bursts).
+      // 1.517 .. 1.573, the best one taken.  (K split over the waves, below: 1.70.)  One barrier for two or four steps, W.x and h in
+      // rings of as many: 1.51 and 1.55 (the waves beside these then come in bursts).  With polls of lanes side by side (quad_word) a
+      // call takes 1.163 ms instead of 1.450 (bf16 4 x 512 B 4 T 600 0.622 -> 0.451, float32 4 x 128 B 4 T 256 0.196 -> 0.174), the eight
+      // phases 1.163 .. 1.195; s_sleeps none / 1 / 2: bf16 1.212 / 1.169 / 1.203, with coefficients for slstm_bwd_quad_kernel (a training
+      // call) 3.581 / 3.511 / 3.461, head dim 512 0.451 / 0.452 / 0.461; float32 head dim 128 0.174 / 0.181 / 0.184, 200 (B 9 T 500)
+      // 0.525 / 0.517 / 0.501.
       const int buf = t & 1;
       float wxv[4];
       XS_QTICK(5);
@@ -618,7 +635,7 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
       const bool row_reset = rfl[t & 3][orow] != 0u;       // (the operand's row: it contributes R.0 = 0 exactly)
       const bool gate_reset = rfl[t & 3][gb] != 0u;
 #ifndef XS_QUAD_SLEEP
-#define XS_QUAD_SLEEP (BF16 && NCH == 4 ? 2 : 1)
+#define XS_QUAD_SLEEP (BF16 ? (COEF == 1 ? 2 : 1) : (NCH == 2 ? 0 : (NCH == 4 && !COEF ? 2 : 1)))
 #endif
       if (XS_QUAD_SLEEP > 0) __builtin_amdgcn_s_sleep(XS_QUAD_SLEEP);
       asm volatile("");  // (the compiler keeps what stands in front of this statement in front of the poll)
@@ -629,7 +646,7 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
       if (t > 0) {
 #pragma unroll
         for (int ks = 0; ks < NP; ++ks)
-          areg[ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(hrs, xl, ks * PSTEP, 16));
+          areg[ks] = poll(hrs, ks);
         stage_coefficients(t - 1);  // (COEF; while the poll is on its way)
       } else {
 #pragma unroll
@@ -657,7 +674,7 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
           if (__builtin_amdgcn_ballot_w64(mark_has_sentinel<BF16>(ma)) == 0ull) break;
 #pragma unroll
           for (int ks = 0; ks < NP; ++ks)
-            areg[ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(hrs, xl, ks * PSTEP, 16));
+            areg[ks] = poll(hrs, ks);
           spins += 1;
           if ((spins & 1023u) == 0u && __hip_atomic_load(&p.status->aborted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
             aborted = true;

@@ -90,7 +90,7 @@ __global__ __launch_bounds__(256) void stage_exchange_kernel(StageParams p) {
   if (member == 0 && tid == 0) p.words[8] = carry;
 }
 
-// ---- (1b) the exchange as the kernel for row tiles of 4 rows makes it: [slot][member][4 rows][16 units], EVERY wave
+// ---- (1b) the exchange as the kernel for row tiles of 4 rows makes it: a slot in the order of a poll's lanes (quad_word), EVERY wave
 //      polls the group's whole tile (NK / 4 chunks of 16 bytes a lane) and publishes its own 16 values; the step's barrier
 //      and a pause of 64 cycles in front of the poll
 template <int NK>
@@ -98,11 +98,9 @@ __global__ __launch_bounds__(256) void stage_exchange_quad_kernel(StageParams p)
   const int wg = blockIdx.x, xcd = wg & 7, member = wg >> 3;
   if (xcd != 0 || member >= p.members) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, r16 = lane & 15;
-  constexpr int QTILE = 4 * 16 * 2, NCH = NK / 4;
-  const int xslot = p.members * QTILE;
-  const bool a_lane = (r16 >> 2) < p.rows;
-  const int xl = a_lane ? (2 * NCH * (r16 & 3) + (q >> 1)) * QTILE + (r16 >> 2) * 32 + (q & 1) * 16 : 0x7FFFFF00;
-  const long long xo = (long long)member * (QTILE / 2) + q * 16 + 4 * wave + (r16 & 3);
+  constexpr int NCH = NK / 4, xslot = NCH * 1024;
+  const int xl = (r16 >> 2) < p.rows ? lane * 16 : 0x7FFFFF00;
+  const int xo = quad_word<true, NCH>(member * 16 + 4 * wave + (r16 & 3), q) / 2;
   uint32_t carry = (uint32_t)tid, max_spins = 0;
   bool dead = false;
   for (int t = 0; t < p.steps; ++t) {
@@ -120,7 +118,7 @@ __global__ __launch_bounds__(256) void stage_exchange_quad_kernel(StageParams p)
     for (;;) {
 #pragma unroll
       for (int ks = 0; ks < NCH; ++ks)
-        areg[ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, xl, ks * 2 * QTILE, 16));
+        areg[ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, xl, ks * 1024, 16));
       uint32_t ma = 0u;
 #pragma unroll
       for (int ks = 0; ks < NCH; ++ks) ma = mark_join<true>(ma, chunk_mark<true>(areg[ks]));
@@ -198,16 +196,14 @@ __global__ __launch_bounds__(256) void stage_gating_kernel(StageParams p) {
 //      output tensor, no feeder, drainer or prefetch waves.  Head groups of 16 members placed as the product places
 //      them (consecutive slots of one XCD).
 __global__ __launch_bounds__(256) void stage_chain_kernel(StageParams p) {
-  constexpr int NCH = 2, NK = 4 * NCH, QTILE = 4 * 16 * 2;
+  constexpr int NCH = 2, NK = 4 * NCH, xslot = NCH * 1024;
   const int wg = blockIdx.x, xcd = wg & 7, local = wg >> 3;
   const int slot = local / p.members, member = local - slot * p.members;
   const int group = slot * 8 + xcd;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, r16 = lane & 15;
-  const int xslot = p.members * QTILE;
   char *const xbase = p.ring + (long long)group * kRing * xslot;
-  const bool a_lane = (r16 >> 2) < p.rows;
-  const int xl = a_lane ? (2 * NCH * (r16 & 3) + (q >> 1)) * QTILE + (r16 >> 2) * 32 + (q & 1) * 16 : 0x7FFFFF00;
-  const long long xo = (long long)member * (QTILE / 2) + q * 16 + 4 * wave + (r16 & 3);
+  const int xl = (r16 >> 2) < p.rows ? lane * 16 : 0x7FFFFF00;
+  const int xo = quad_word<true, NCH>(member * 16 + 4 * wave + (r16 & 3), q) / 2;
   uint4 rreg[NK];
 #pragma unroll
   for (int ks = 0; ks < NK; ++ks) {
@@ -239,7 +235,7 @@ __global__ __launch_bounds__(256) void stage_chain_kernel(StageParams p) {
       for (;;) {
 #pragma unroll
         for (int ks = 0; ks < NCH; ++ks)
-          areg[ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, xl, ks * 2 * QTILE, 16));
+          areg[ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, xl, ks * 1024, 16));
         uint32_t ma = 0u;
 #pragma unroll
         for (int ks = 0; ks < NCH; ++ks) ma = mark_join<true>(ma, chunk_mark<true>(areg[ks]));
