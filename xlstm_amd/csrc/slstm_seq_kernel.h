@@ -144,6 +144,13 @@ __device__ __forceinline__ uint32_t seq_handshake(const SeqParams &p, int wg, in
   return cross ? 1u : 0u;
 }
 
+// Row tiles of 8 or 16 rows: the byte of a member's tile at which the h of (unit of the member, row) lies.  SIDE_BY_SIDE: the lanes of a
+// poll's load (group q, row r16) lie side by side; else [row][unit].
+template <int ESZ, bool SIDE_BY_SIDE>
+__device__ __forceinline__ int tile_word(int unit, int row) {
+  return SIDE_BY_SIDE ? unit * ESZ / 16 * 256 + row * 16 + unit * ESZ % 16 : (row * 16 + unit) * ESZ;
+}
+
 // Row tiles of 4 rows (QUAD): the byte of a ring slot at which the h of (unit of the head, row of the tile) lies.  Piece c holds chunk c of each
 // quarter of K, 16 bytes per (unit group q, row, quarter) in bf16 and per (quarter, unit group, row) in float32.
 template <bool BF16, int NCH>
@@ -873,7 +880,7 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
   lds_barrier();  // prologue barrier: reset flags of iteration 0 and the placement verdict are in LDS
   const bool cross = cross_s != 0u;
 
-  // exchange ring layout [head group][slot][row tile][member][16 rows][16 units]: what a group
+  // exchange ring layout [head group][slot][row tile][member][tile_word]: what a group
   // publishes for one row tile is contiguous (512 B per member for bf16), which spreads the polls
   // of an iteration over all L2 channels (measured: lines 256 B .. 2 KiB apart are served 1.5x
   // faster than lines 4 KiB or more apart)
@@ -892,8 +899,13 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
   uint4 areg[NCH];
   bool prefetched = false;
   // poll address of chunk c of row tile mt = per-lane part (one register) + a compile-time constant:
-  // unit k of row r of row tile mt lives at [mt][member k/16][r][k%16]
-  const int xlane = ((wave * KW + q * EPC) >> 4) * XTILE + (r16 * 16 + ((q * EPC) & 15)) * ESZ;
+  // unit k of row r of row tile mt lives at [mt][member k/16], there at tile_word(k%16, r)
+  // (float32, one row tile: side by side; the lanes of a load lay 64 bytes apart, every load a line a lane.  us a call of T 200, before ->
+  // after: 4 x 256 B 64 423 -> 403, B 30 371 -> 366, 4 x 512 B 16 616 -> 587, 6 x 320 B 16 661 -> 632, 4 x 200 B 64 404 -> 389.  bf16, whose lanes
+  // lie 32 bytes apart, does not gain: 4 x 256 T 300 B 64 383.7 / 384.2, T 500 B 30 492 / 495; nor do two row tiles, which are asked for
+  // an iteration ahead: float32 4 x 256 B 120 771 / 780.)
+  constexpr bool LANES = !BF16 && MT == 1;
+  const int xlane = ((wave * KW + q * EPC) >> 4) * XTILE + tile_word<ESZ, LANES>((q * EPC) & 15, r16);
   const int xtile_stride = p.G * XTILE;
   auto xconst = [&](int c, int mt_) { return ((c * 4 * EPC) >> 4) * XTILE + mt_ * xtile_stride; };
   // Where the time loop of the compute waves starts relative to a 32-byte boundary of the code moves the time per step
@@ -1207,7 +1219,7 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
       if (!BF16 && y != y) y = __uint_as_float(0x7FC00000u);  // keep the "not written yet" NaN pattern unique
       // Every lane stores, every iteration: lanes outside the batch or the head write words of their own
       // block that nobody polls, and the re-arm of steps 0 and 1 hits slots that still hold the pattern.
-      const long long xo = ((long long)mt * p.G + member) * (XTILE / ESZ) + pb * 16 + pa;
+      const long long xo = ((long long)mt * p.G + member) * (XTILE / ESZ) + tile_word<ESZ, LANES>(pa, pb) / ESZ;
       if (BF16) {
         const uint16_t v = (uint16_t)float_to_bf16_bits(y);
         uint16_t *dst = reinterpret_cast<uint16_t *>(hcur) + xo;
