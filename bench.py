@@ -576,13 +576,12 @@ def backward_phase_profile(device):
         out = F.slstm_backward(wx, r, bias, None, mask, h, d_h, timings=tm)
         torch.cuda.synchronize()
         ms.append(tm["events"][1].elapsed_time(tm["events"][2]))
-    words = out[3][3].reshape(-1)[:60].view(torch.int64).cpu().double()
-    st, fd = words[:24].view(3, 8) / T, words[24:30]
+    words = out[3][3].reshape(B, H)[:4, :16].contiguous().view(torch.int64).cpu().double()  # a row of the m plane per wave
+    st, fd = words[:3] / T, words[3]
     points = ["partial results added up", "deltas published", "first look issued at the earliest", "deltas complete",
               "partial tile written", "barrier left (= the step)"]
     res = {"reverse_kernel_ms_with_stamps": sorted(ms)[1]}
-    for w, row in zip(("wave 0 (forms the gradient; polls its own workgroup)", "wave 4 (polls its own workgroup)",
-                       "wave 6 (polls another workgroup)"), st):
+    for w, row in zip(("first gradient wave", "first matrix wave", "last matrix wave"), st):
         res[w] = {n: round(float(v)) for n, v in zip(points, row[:6])}
         res[w]["looks repeated per step"] = round(float(row[6]), 2)
         res[w]["the look that found them issued"] = round(float(row[7]))

@@ -590,15 +590,22 @@ __global__ __launch_bounds__(256) void slstm_bwd_arm_kernel(uint4 *xch, long lon
 // than two or three groups; the feeder waves then missed to HBM, every poll of their compute unit came back behind those
 // misses, and at the end the prefetch kept the kernel alive for as long again: 5 us per step at B 64 x 4 heads of 256
 // instead of 2, 16 at B 192.)
-constexpr int kBwdAhead = 12;  // steps the prefetch may run ahead at most (1.2 MiB of a 4 MiB L2 at config 2)
+// Steps the prefetch may run ahead at most, and between two looks at the progress.  A look comes back behind the touches issued in front of
+// it, a trip to memory: with row tiles of 4 rows it is made every eighth step (every fourth, 16 steps ahead: 1.75 ms a training call at B 16 x T
+// 1024 x 4 heads of 256, every second 1.73, every one 1.89; 1.70 with this).
+constexpr int bwd_ahead(int rows) { return rows == 4 ? 24 : 12; }
+constexpr int bwd_look_every(int rows) { return rows == 4 ? 8 : 2; }
+// Bytes between two touches: a miss of the L2 brings 64 bytes, half a line (the same call with 128: 1.85 -> 1.73).
+constexpr int bwd_touch(int rows) { return rows == 4 ? 64 : 128; }
 // ROWS: batch rows of a row tile; DEPTH: steps the feeder waves ask ahead
 template <bool BF16, int S, int ROWS, int DEPTH>
 __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int xcd, int which, int of) {
   constexpr int ESZ = BF16 ? 2 : 4;
   constexpr int dh = 64 * S;
   constexpr int PIECE = ROWS * 9 * 64 * 4;          // bytes of a workgroup's coefficients of one step
-  constexpr int CL = S * PIECE / 128;               // lines of a group's coefficients of one step (its S workgroups' pieces lie in a row)
-  constexpr int PER_ROW = dh * ESZ / 128;           // lines of a row of d_h
+  constexpr int TOUCH = bwd_touch(ROWS), EVERY = bwd_look_every(ROWS);
+  constexpr int CL = S * PIECE / TOUCH;             // touches of a group's coefficients of one step (its S workgroups' pieces lie in a row)
+  constexpr int PER_ROW = dh * ESZ / TOUCH;         // touches of a row of d_h
   constexpr int DL = ROWS * PER_ROW;
   const int H = p.NH * dh, ntiles = (p.B + ROWS - 1) / ROWS, ngroups = p.NH * ntiles;
   const int tid = threadIdx.x, nthreads = blockDim.x, lane = tid & 63;
@@ -606,8 +613,8 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
   const int G = (ngroups - xcd + 7) >> 3;           // groups of this XCD: xcd, xcd + 8, ...
   // steps the prefetch may run ahead of the groups' progress: about 2 MiB of the XCD's 4 MiB L2, and more than the
   // feeder waves run ahead
-  int ahead = (2 << 20) / (G * (CL + DL) * 128);
-  ahead = ahead > kBwdAhead ? kBwdAhead : (ahead < DEPTH + 2 ? DEPTH + 2 : ahead);
+  int ahead = (2 << 20) / (G * (CL + DL) * TOUCH);
+  ahead = ahead > bwd_ahead(ROWS) ? bwd_ahead(ROWS) : (ahead < DEPTH + 2 ? DEPTH + 2 : ahead);
   // A touch is a load that writes LDS, not a register: nothing waits for these loads before the end, and a register
   // that a load in flight is going to write would be handed out again by the compiler in the meantime.  Every touch of
   // every wave lands in the same kilobyte, which nobody reads.
@@ -617,7 +624,7 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
   const long long coef_step = (long long)ngroups * S * PIECE;  // bytes of one step's coefficients, all groups
   const long long dh_step = (long long)p.B * H * ESZ;
   for (int m = 0; m < p.T; ++m) {
-    if (m >= ahead && (m & 1) == 0) {  // (every other step: the groups' progress is read through the L2)
+    if (m >= ahead && m % EVERY == 0) {  // (the groups' progress is read through the L2)
       if (tid == 0) slowest = 0x7FFFFFFF;
       __syncthreads();
       if (tid < 64) {
@@ -643,7 +650,7 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
       const int at = slowest;
       if (at < 0) break;
       // (fallen behind what the feeder waves have already asked for: skip to where a touch can still come first)
-      if (m < at + DEPTH + 1) m = (at + DEPTH + 1) & ~1;
+      if (m < at + DEPTH + 1) m = (at + DEPTH + 1) / EVERY * EVERY;
       if (m >= p.T) break;
     }
     const int t = p.T - 1 - m;
@@ -656,7 +663,7 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
       const int i = i0 + tid;
       const int j = i / CL, l = i - j * CL;
       const int g = xcd + 8 * j, head = g % p.NH, tile = g / p.NH;
-      const uint32_t coff = i < G * CL ? (uint32_t)(((tile * p.NH + head) * S) * PIECE + l * 128) : 0xFFFFFF00u;
+      const uint32_t coff = i < G * CL ? (uint32_t)(((tile * p.NH + head) * S) * PIECE + l * TOUCH) : 0xFFFFFF00u;
       bwd_fetch_to_lds_b128(crs, uniform(dump_lds), coff);
     }
     for (int i0 = which * nthreads; i0 < G * DL; i0 += of * nthreads) {
@@ -664,7 +671,7 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
       const int j = i / DL, l = i - j * DL;
       const int g = xcd + 8 * j, head = g % p.NH, tile = g / p.NH;
       const int row = tile * ROWS + l / PER_ROW;
-      const uint32_t doff = (i < G * DL && row < p.B) ? (uint32_t)(((long long)row * H + head * dh) * ESZ + (l % PER_ROW) * 128) : 0xFFFFFF00u;
+      const uint32_t doff = (i < G * DL && row < p.B) ? (uint32_t)(((long long)row * H + head * dh) * ESZ + (l % PER_ROW) * TOUCH) : 0xFFFFFF00u;
       bwd_fetch_to_lds_b128(drs, uniform(dump_lds), doff);
     }
   }

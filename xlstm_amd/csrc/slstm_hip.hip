@@ -422,6 +422,12 @@ int unit_plan(int B, int NH, int dh, bool bf16, UnitPlan &u) {
 inline size_t unit_slot_bytes(const UnitPlan &u, int esz) { return (size_t)unit_bwd_slot_members(u.G, u.RT, u.CT, esz == 2) * u.RT * 64 * u.CT * esz; }
 inline size_t unit_ring_bytes(const UnitPlan &u, int esz) { return kBwdRing * u.heads * u.groups * unit_slot_bytes(u, esz); }
 
+template <int UW>
+void (*pick_bwd_quad(int dh, bool dwx_bf16))(BwdSplitParams) {
+  if (dwx_bf16) return dh == 64 ? slstm_bwd_quad_kernel<1, UW, true> : (dh == 128 ? slstm_bwd_quad_kernel<2, UW, true> : slstm_bwd_quad_kernel<4, UW, true>);
+  return dh == 64 ? slstm_bwd_quad_kernel<1, UW> : (dh == 128 ? slstm_bwd_quad_kernel<2, UW> : slstm_bwd_quad_kernel<4, UW>);
+}
+
 template <bool BF16, int RT, int CT, bool DWX16>
 void (*pick_unit_bwd(int gq))(UnitBwdParams) {
   if constexpr (!BF16) {
@@ -908,7 +914,14 @@ int run_backward(const xs_slstm_bwd_args *a, bool prepare) {
       if (3 * H * 2 + 1024 >= 0x7FFFFF00ll) return fail(XS_ERR_UNSUPPORTED, "rows too long for row tiles of 4 rows");
       const int S = a->dh / 64;
       const long long ngroups = (long long)a->NH * ((a->B + 3) / 4);
-      const long long grid = (ngroups + 7) / 8 * 8 * S;
+      const long long groups_per_xcd = (ngroups + 7) / 8;
+      // prefetching workgroups per XCD: one per 40 KB that the XCD's groups read per step (a compute unit draws some
+      // 65 GB/s from memory, a step takes about a microsecond; one per 20 or 10 KB gains nothing), as far as there are compute units left
+      const long long step_bytes = groups_per_xcd * S * (4 * 9 * 64 * 4 + 4 * 64 * 2);
+      const long long want = step_bytes > 280000 ? 8 : (step_bytes + 39999) / 40000;
+      // 32 units a workgroup where twice the workgroups leave these their room, else 64 (figures at the kernel)
+      const int uw = 8 * (groups_per_xcd * (a->dh / 32) + want) <= device_cus() ? 32 : 64;
+      const long long grid = groups_per_xcd * 8 * (a->dh / uw);
       if (grid > device_cus()) return fail(XS_ERR_DEVICE, "%lld workgroups of the backward pass with row tiles of 4 rows do not fit %d compute units at once", grid, device_cus());
       BwdSplitParams q;
       q.B = a->B; q.T = a->T; q.NH = a->NH; q.dh = a->dh;
@@ -917,31 +930,20 @@ int run_backward(const xs_slstm_bwd_args *a, bool prepare) {
       q.d_wx = (float *)a->d_wx; q.d_wx_sb = a->d_wx_stride_b; q.d_wx_st = a->d_wx_stride_t; q.d_s0 = a->d_s0;
       q.xch = a->exchange; q.abort_word = a->counters; q.progress = a->counters + 1; q.placement = a->counters + 1 + ngroups;
       q.main_locals = (int)(grid / 8);
-      // prefetching workgroups per XCD: one per 40 KB that the XCD's groups read per step (a compute unit draws some
-      // 65 GB/s from memory, a step takes about a microsecond), as far as there are compute units left
-      int prefetchers = 0;
-      {
-        const long long groups_per_xcd = (ngroups + 7) / 8;
-        const long long step_bytes = groups_per_xcd * S * (kBwdQuadCoefBytes + 4 * 64 * 2);
-        long long want = (step_bytes + 39999) / 40000;
-        const long long room = (device_cus() - grid) / 8;
-        if (want > room) want = room;
-        if (want > 8) want = 8;
-        prefetchers = (int)(want < 0 ? 0 : want);
-      }
+      const long long room = (device_cus() - grid) / 8;
+      const int prefetchers = (int)(want < room ? want : room);
       q.spin_limit = a->spin_limit != 0 ? a->spin_limit : kDefaultSpinLimit;
       q.cut = a->recurrent_cut != 0; q.clip = clip;
       const long long n16 = (long long)kBwdRing * ngroups * 4 * 4 * a->dh * 2 / 16;
       hipLaunchKernelGGL(slstm_bwd_arm_kernel, dim3((unsigned)((n16 + 255) / 256 < 1024 ? (n16 + 255) / 256 : 1024)), dim3(256), 0, stream,
                          (uint4 *)a->exchange, n16, a->counters, (int)(1 + 2 * ngroups));
-      void (*kq)(BwdSplitParams) = a->dh == 64 ? slstm_bwd_quad_kernel<1> : (a->dh == 128 ? slstm_bwd_quad_kernel<2> : slstm_bwd_quad_kernel<4>);
-      if (dwx_bf16) kq = a->dh == 64 ? slstm_bwd_quad_kernel<1, true> : (a->dh == 128 ? slstm_bwd_quad_kernel<2, true> : slstm_bwd_quad_kernel<4, true>);
-      const int lds = bwd_quad_lds_bytes();
+      void (*kq)(BwdSplitParams) = uw == 32 ? pick_bwd_quad<32>(a->dh, dwx_bf16) : pick_bwd_quad<64>(a->dh, dwx_bf16);
+      const int lds = bwd_quad_lds_bytes(uw);
       {
         const int rc = ensure_dynamic_lds((const void *)kq, (size_t)lds);
         if (rc != XS_OK) return rc;
       }
-      hipLaunchKernelGGL(kq, dim3((unsigned)(grid + 8 * prefetchers)), dim3(kBwdQuadThreads), lds, stream, q);
+      hipLaunchKernelGGL(kq, dim3((unsigned)(grid + 8 * prefetchers)), dim3(bwd_quad_threads(uw)), lds, stream, q);
       const hipError_t es = hipGetLastError();
       if (es != hipSuccess) return fail(XS_ERR_LAUNCH, "backward kernel launch failed: %s", hipGetErrorString(es));
       return XS_OK;
