@@ -586,8 +586,8 @@ class sLSTMCell_hip(nn.Module):
 
     def _trains_natively(self, input: torch.Tensor) -> bool:
         """Whether a training call takes the native host path.  Not where the coefficients are not to be kept, and for long
-        bfloat16 sequences at head dim 256: forward and backward in row tiles of 4 rows x 64 units save 0.07 us a step there
-        and take three more launches."""
+        bfloat16 sequences at head dim 256: forward and backward in row tiles of 4 rows save 0.1 to 0.2 us a step there and take
+        three more launches (us a call, native / those: 4 heads B 16 T 320 584 / 588, T 383 682 / 673; B 4 T 256 441 / 439)."""
         return (self.keep_backward_coefficients and 9 * input.numel() <= F_hip.KEPT_COEFFICIENT_BYTES
                 and not (self.head_dim == 256 and input.dtype == torch.bfloat16
                          and input.shape[1 if self.config.input_shape == "BSGNH" else 0] >= 384))
