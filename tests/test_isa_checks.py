@@ -112,3 +112,34 @@ def test_the_backward_kernel_with_feeder_waves_keeps_its_registers_and_polls_wit
         for i in polls:
             assert not any("v_readfirstlane" in line for line in body[max(0, i - 6): i]), (name.group(1), body[i - 6: i + 1])
     assert seen == 8  # bf16 at head dims 64, 128, 256 with the gate deltas in float32 and in bf16; float32 at 64, 128
+
+
+def test_the_reverse_kernel_for_row_tiles_of_4_rows_publishes_behind_the_acknowledgement_of_what_it_rearmed(tmp_path):
+    """The gradient waves of slstm_bwd_quad_kernel publish a step's deltas and re-arm the words of two steps ago with plain
+    stores, and never load: without a wait between a re-arm and the next publication a peer that has seen the latter may poll
+    re-armed words before they are there and take the deltas of four steps ago.  A publication is two stores of 8 bytes in
+    one basic block; a wait for everything in flight has to stand in front of them in that block."""
+    import re
+
+    listing = _compiled_listing(tmp_path)
+    kernels = re.findall(r"^(_Z\w*slstm_bwd_quad_kernelILi\d+ELi\d+ELb[01]E\w*):", listing, re.M)
+    for name in kernels:
+        body = listing[listing.index("\n" + name + ":"):]
+        body = [line.strip() for line in body[: body.index(".end_amdhsa_kernel")].split("\n")]
+        blocks, block = [], []
+        for ins in body:
+            if re.match(r"^\.LBB\w+:|^s_c?branch", ins):
+                blocks.append(block)
+                block = []
+            elif _is_instruction(ins):
+                block.append(ins)
+        publications = [b for b in blocks if sum(i.startswith("global_store_dwordx2") for i in b) == 2]
+        assert publications, name
+        for b in publications:
+            first = next(i for i, ins in enumerate(b) if ins.startswith("global_store_dwordx2"))
+            assert any(re.match(r"s_waitcnt\b.*vmcnt\(0\)", ins) for ins in b[:first]), (name, b)
+    assert len(kernels) == 12  # head dims 64, 128, 256; 32 and 64 units a workgroup; gate deltas in float32 and in bf16
+
+
+def _is_instruction(ins):
+    return bool(ins) and not ins.startswith((";", ".")) and not ins.endswith(":")

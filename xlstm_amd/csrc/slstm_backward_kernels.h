@@ -532,9 +532,10 @@ __global__ __launch_bounds__(NW * 64) void slstm_bwd_kernel(BwdParams p) {
 // a NaN that would is changed into another NaN).  A reader polls its 16-byte chunks until none holds the pattern.  A workgroup that
 // publishes step n also re-arms its words of step n - 2: it has read all deltas of step n - 1, which every peer
 // computed from a complete set of step n - 2.  The re-arm is acknowledged before the workgroup's poll of step n
-// returns (accesses of a wave complete in order), so before it publishes step n + 1; a peer that polls the slot again
-// for step n - 2 + kBwdRing has seen that publication and finds the pattern or the new data, never the old.  The
-// library fills the ring with the pattern in front of the kernel.
+// returns (accesses of a wave complete in order: this holds for a wave that publishes AND polls; slstm_bwd_quad_kernel,
+// whose publishing waves do not poll, waits for the acknowledgement), so before it publishes step n + 1; a peer that polls
+// the slot again for step n - 2 + kBwdRing has seen that publication and finds the pattern or the new data, never the
+// old.  The library fills the ring with the pattern in front of the kernel.
 //
 // All workgroups of a group run on one XCD (workgroup i is dispatched to XCD i % 8): plain stores reach the XCD's L2,
 // and the polls read past the first-level cache.  All workgroups must be resident at once; the host launches at most
