@@ -355,7 +355,7 @@ def test_the_gradient_of_the_final_state_by_the_chain_rule(bf16, B, T, NH, dh, s
 
 @pytest.mark.parametrize("bf16,B,T,NH,dh,split", [(False, 5, 9, 2, 64, True), (False, 20, 7, 2, 128, True), (True, 16, 10, 4, 256, True),
                                                   (False, 4, 12, 4, 256, False), (True, 9, 7, 2, 512, True), (True, 6, 9, 2, 128, False),
-                                                  (False, 7, 6, 2, 256, True), (True, 16, 10, 4, 256, 4), (True, 5, 9, 2, 64, 4)])
+                                                  (False, 7, 6, 2, 256, True), (True, 16, 10, 4, 256, 4), (True, 25, 10, 4, 256, 4), (True, 5, 9, 2, 64, 4)])
 @pytest.mark.parametrize("opts", [dict(recurrent_cut=True), dict(recurrent_clipval=0.05), dict(recurrent_clipval=1.0),
                                   dict(recurrent_cut=True, recurrent_clipval=0.05)],
                          ids=["cut", "clip0.05", "clip1", "cut+clip"])

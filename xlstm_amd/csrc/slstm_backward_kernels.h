@@ -686,9 +686,10 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
 __device__ __forceinline__ void bwd_note_placement(const BwdSplitParams &p, int group) {
   if (threadIdx.x == 0) atomicOr(p.placement + group, 1u << (__builtin_amdgcn_s_getreg(20 | (3 << 11)) & 0xFu));  // XCC_ID, bits [3:0]
 }
-__device__ __forceinline__ bool bwd_placement_mixed(const BwdSplitParams &p, int group) {
+__device__ __forceinline__ bool bwd_placement_mixed(const BwdSplitParams &p, int group, int members) {
+  if (members == 1 || p.cut != 0) return false;  // (nothing to look at: bwd_exchange_torn)
   const unsigned int seen = __hip_atomic_load(p.placement + group, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const bool mixed = (seen & (seen - 1u)) != 0u;
+  const bool mixed = bwd_exchange_torn(members, p.cut != 0, seen);
   if (mixed && threadIdx.x == 0) __hip_atomic_store(p.abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return mixed;
 }
@@ -991,7 +992,7 @@ __global__ __launch_bounds__(FEED ? 768 : 512) void slstm_bwd_split_kernel(BwdSp
     if (t > 0) step(in1, t - 1);
   }
   // ---- gradient w.r.t. the initial state (the stabiliser's part is zero by the rule; NaN all over when a wait ran out)
-  const bool mixed = S > 1 && p.cut == 0 && bwd_placement_mixed(p, group);
+  const bool mixed = bwd_placement_mixed(p, group, S);
   if (there) {
     const bool poisoned = gave_up || mixed || __hip_atomic_load(p.abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const long long o = (long long)row * H + ecol;

@@ -297,7 +297,7 @@ __global__ __launch_bounds__(bwd_quad_threads(UW)) void slstm_bwd_quad_kernel(Bw
       lds_barrier();  // A(n)
       XS_BTICK(5);
     }
-    bwd_placement_mixed(p, group);  // (thread 0 flags the call)
+    bwd_placement_mixed(p, group, M);  // (thread 0 flags the call)
 #ifdef XS_PROFILE
     __syncthreads();
     if (tid == 0 && member == 0) p.progress[group] = 0x40000000u + (unsigned int)(wall_clock64() - wg_start);  // (how long the group took, in 10 ns)
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(bwd_quad_threads(UW)) void slstm_bwd_quad_kernel(Bw
     XS_BTICK(5);
   }
   // ---- gradient w.r.t. the initial state (the stabiliser's part is zero by the rule; NaN all over when a wait ran out)
-  const bool mixed = M > 1 && !cut && bwd_placement_mixed(p, group);
+  const bool mixed = bwd_placement_mixed(p, group, M);
   dy = (cut || zero_dy) ? 0.0f : add_up(p.T - 1);
   if (there) {
     const bool poisoned = mixed || __hip_atomic_load(p.abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;

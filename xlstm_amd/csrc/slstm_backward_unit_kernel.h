@@ -420,7 +420,7 @@ __global__ __launch_bounds__(unit_bwd_threads(CT)) void slstm_bwd_unit_kernel(Un
   // ---- the gradient of the initial state (the stabiliser's part is zero by the rule; NaN when a wait ran out)
   if (grad_wave) {
     const unsigned int seen = __hip_atomic_load(p.placement + gi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const bool mixed = !p.cut && (seen & (seen - 1u)) != 0u;  // (the plain stores reach one XCD's L2 only)
+    const bool mixed = bwd_exchange_torn(p.G, p.cut != 0, seen);
     if (mixed && tid == 0) __hip_atomic_store(p.abort_word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     dy = (p.cut || after) ? 0.0f : add_up(p.T - 1);
     const bool poisoned = mixed || __hip_atomic_load(p.abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;

@@ -38,6 +38,7 @@
 #include "slstm_step_pipe_kernel.h"
 #include "slstm_step_small_kernel.h"
 #include "slstm_layer_step_kernel.h"
+#include "slstm_backward_rules.h"
 #include "slstm_backward_kernels.h"
 #include "slstm_layer_kernels.h"
 #include "slstm_layer_f32_kernels.h"
