@@ -42,3 +42,50 @@ int main() {
             assert "seen - 1" not in text, name  # (nobody decides this for itself)
             asked += len(re.findall(r"bwd_exchange_torn\([^;]*p\.cut != 0", text))
     assert asked == 2  # bwd_placement_mixed (split and quad kernels) and the unit kernel
+
+
+_WALK = r"""
+#include <cstdlib>
+// the prefetching workgroups' walk of slstm_backward_kernels.h over groups whose slowest moves on by chance; what is touched must be
+// neither too far in front of the groups nor, right behind a look, what their feeder waves have asked for already
+static int walk(int rows, long long step_bytes, int depth, int T, int slow) {
+  const BwdPace pace = bwd_pace(rows, step_bytes, depth);
+  if (pace.every < 2 || pace.ahead < depth + 2) return 1;
+  const long long most = 2 << 20 > (depth + 3) * step_bytes ? 2 << 20 : (depth + 3) * step_bytes;
+  int at = 0, next_look = pace.ahead;
+  for (int m = 0; m < T; ++m) {
+    at += rand() % 100 < slow ? 0 : rand() % 3;
+    if (m >= next_look) {
+      while (at < m - pace.ahead) at += rand() % 2;
+      if (rand() % 50 == 0) at += rand() % 40;  // (the prefetch is late)
+      m = bwd_pace_resume(m, at, depth);
+      if (m >= T) break;
+      if (m <= at + depth) return 2;
+      if (m > at + depth + 1 && m > at + pace.ahead) return 3;
+      next_look = m + pace.every;
+    }
+    if ((m - at) * step_bytes > most) return 4;
+  }
+  return 0;
+}
+int main() {
+  for (int rows : {4, 16})
+    for (int groups = 1; groups <= 64; ++groups)
+      for (int S : {1, 2, 4, 8})
+        for (int slow : {0, 30, 60, 95}) {
+          const int depth = rows == 4 ? 6 : 2;
+          const long long bytes = (long long)groups * S * rows * (9 * 64 * 4 + 64 * 2);
+          if (int why = walk(rows, bytes, depth, 4000, slow)) { printf("%d rows, %d groups of %d: %d\n", rows, groups, S, why); return 1; }
+        }
+  return 0;
+}
+"""
+
+
+def test_the_prefetch_stays_in_its_share_of_the_cache_and_ahead_of_the_feeder_waves(tmp_path):
+    """However the groups move: what the prefetching workgroups have brought and no group has reached is at most 2 MiB of an
+    XCD's 4 MiB L2 (or three steps more than the feeder waves run ahead), also between two looks, and a prefetch that is late goes
+    on at the first step that nobody has asked for."""
+    _run(tmp_path, _WALK)
+    kernel = open(os.path.join(CSRC, "slstm_backward_kernels.h")).read()
+    assert "= bwd_pace(ROWS, " in kernel and "m = bwd_pace_resume(m, at, DEPTH);" in kernel and "next_look = m + pace.every;" in kernel

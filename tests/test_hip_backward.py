@@ -137,7 +137,8 @@ def test_backward_against_the_oracle(bf16, B, T, NH, dh, masked, kernel):
 
 @pytest.mark.parametrize("B,T,NH,dh", [(23, 40, 4, 256), (25, 40, 4, 256),   # 32 units a workgroup, three groups per XCD; 64, four
                                        (28, 33, 7, 128), (33, 9, 7, 128),    # 32: every compute unit taken; 64, eight groups per XCD
-                                       (30, 9, 12, 64), (61, 9, 16, 64)])    # 32; 64: one workgroup per group, every compute unit taken
+                                       (30, 9, 12, 64), (61, 9, 16, 64),     # 32; 64: one workgroup per group, every compute unit taken
+                                       (15, 150, 4, 256), (45, 150, 4, 256)])  # the prefetch looks every eighth and every second step
 def test_both_widths_of_the_reverse_kernel_for_row_tiles_of_4_rows(B, T, NH, dh):
     """Calls on both sides of where a workgroup takes 32 units instead of 64, last row tiles that are not whole: as above."""
     test_backward_against_the_oracle(True, B, T, NH, dh, True, "quad")

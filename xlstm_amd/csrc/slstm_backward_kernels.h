@@ -591,11 +591,6 @@ __global__ __launch_bounds__(256) void slstm_bwd_arm_kernel(uint4 *xch, long lon
 // than two or three groups; the feeder waves then missed to HBM, every poll of their compute unit came back behind those
 // misses, and at the end the prefetch kept the kernel alive for as long again: 5 us per step at B 64 x 4 heads of 256
 // instead of 2, 16 at B 192.)
-// Steps the prefetch may run ahead at most, and between two looks at the progress.  A look comes back behind the touches issued in front of
-// it, a trip to memory: with row tiles of 4 rows it is made every eighth step (every fourth, 16 steps ahead: 1.75 ms a training call at B 16 x T
-// 1024 x 4 heads of 256, every second 1.73, every one 1.89; 1.70 with this).
-constexpr int bwd_ahead(int rows) { return rows == 4 ? 24 : 12; }
-constexpr int bwd_look_every(int rows) { return rows == 4 ? 8 : 2; }
 // Bytes between two touches: a miss of the L2 brings 64 bytes, half a line (the same call with 128: 1.85 -> 1.73).
 constexpr int bwd_touch(int rows) { return rows == 4 ? 64 : 128; }
 // ROWS: batch rows of a row tile; DEPTH: steps the feeder waves ask ahead
@@ -604,7 +599,7 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
   constexpr int ESZ = BF16 ? 2 : 4;
   constexpr int dh = 64 * S;
   constexpr int PIECE = ROWS * 9 * 64 * 4;          // bytes of a workgroup's coefficients of one step
-  constexpr int TOUCH = bwd_touch(ROWS), EVERY = bwd_look_every(ROWS);
+  constexpr int TOUCH = bwd_touch(ROWS);
   constexpr int CL = S * PIECE / TOUCH;             // touches of a group's coefficients of one step (its S workgroups' pieces lie in a row)
   constexpr int PER_ROW = dh * ESZ / TOUCH;         // touches of a row of d_h
   constexpr int DL = ROWS * PER_ROW;
@@ -612,10 +607,7 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
   const int tid = threadIdx.x, nthreads = blockDim.x, lane = tid & 63;
   if (xcd >= ngroups || of < 1) return;
   const int G = (ngroups - xcd + 7) >> 3;           // groups of this XCD: xcd, xcd + 8, ...
-  // steps the prefetch may run ahead of the groups' progress: about 2 MiB of the XCD's 4 MiB L2, and more than the
-  // feeder waves run ahead
-  int ahead = (2 << 20) / (G * (CL + DL) * TOUCH);
-  ahead = ahead > bwd_ahead(ROWS) ? bwd_ahead(ROWS) : (ahead < DEPTH + 2 ? DEPTH + 2 : ahead);
+  const BwdPace pace = bwd_pace(ROWS, (long long)G * (CL + DL) * TOUCH, DEPTH);
   // A touch is a load that writes LDS, not a register: nothing waits for these loads before the end, and a register
   // that a load in flight is going to write would be handed out again by the compiler in the meantime.  Every touch of
   // every wave lands in the same kilobyte, which nobody reads.
@@ -624,8 +616,9 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
   __shared__ int slowest;      // the least progress among the XCD's groups; -1: stop
   const long long coef_step = (long long)ngroups * S * PIECE;  // bytes of one step's coefficients, all groups
   const long long dh_step = (long long)p.B * H * ESZ;
+  int next_look = pace.ahead;
   for (int m = 0; m < p.T; ++m) {
-    if (m >= ahead && m % EVERY == 0) {  // (the groups' progress is read through the L2)
+    if (m >= next_look) {  // (the groups' progress is read through the L2)
       if (tid == 0) slowest = 0x7FFFFFFF;
       __syncthreads();
       if (tid < 64) {
@@ -636,7 +629,7 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
             const int at = (int)__hip_atomic_load(p.progress + xcd + 8 * j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             least = at < least ? at : least;
           }
-          if (__builtin_amdgcn_ballot_w64(least < m - ahead) == 0ull) {  // (lanes without a group: the largest int)
+          if (__builtin_amdgcn_ballot_w64(least < m - pace.ahead) == 0ull) {  // (lanes without a group: the largest int)
             if (lane < G) atomicMin(&slowest, least);
             break;
           }
@@ -651,8 +644,9 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
       const int at = slowest;
       if (at < 0) break;
       // (fallen behind what the feeder waves have already asked for: skip to where a touch can still come first)
-      if (m < at + DEPTH + 1) m = (at + DEPTH + 1) / EVERY * EVERY;
+      m = bwd_pace_resume(m, at, DEPTH);
       if (m >= p.T) break;
+      next_look = m + pace.every;
     }
     const int t = p.T - 1 - m;
     const unsigned long long cb = reinterpret_cast<unsigned long long>(p.coef) + (unsigned long long)(t * coef_step);
