@@ -141,5 +141,39 @@ def test_the_reverse_kernel_for_row_tiles_of_4_rows_publishes_behind_the_acknowl
     assert len(kernels) == 12  # head dims 64, 128, 256; 32 and 64 units a workgroup; gate deltas in float32 and in bf16
 
 
+def test_the_feeder_waves_of_that_kernel_wait_only_where_they_say_so(tmp_path):
+    """The compiler sees one function, not roles: a load at the head of one role that it takes for pending where another role
+    uses the register is waited for there, in the feeder waves' loop at the cost of a request's whole latency every step.
+    In the loops that make requests every wait for memory is one written by hand (or that of a load in the loop itself)."""
+    import re
+
+    listing = _compiled_listing(tmp_path)
+    kernels = re.findall(r"^(_Z\w*slstm_bwd_quad_kernelILi\d+ELi\d+ELb[01]E\w*):", listing, re.M)
+    for name in kernels:
+        body = listing[listing.index("\n" + name + ":"):]
+        blocks, in_asm = [], False
+        for line in body[: body.index(".end_amdhsa_kernel")].split("\n"):
+            label = re.match(r"^\.L(BB\w+):(.*)", line)
+            if label:
+                blocks.append((label.group(1), label.group(2), []))
+            elif line.lstrip().startswith("; ") and blocks and not blocks[-1][2]:  # (the loops around a block, over several lines)
+                blocks[-1] = (blocks[-1][0], blocks[-1][1] + line, [])
+            elif "ASMSTART" in line or "ASMEND" in line:
+                in_asm = "ASMSTART" in line
+            elif blocks and _is_instruction(line.strip()):
+                blocks[-1][2].append((line.strip(), in_asm))
+        loops = set()
+        for label, where, code in blocks:
+            if any(ins.startswith("buffer_load_ubyte") for ins, _ in code):
+                loops.add(label if "Loop Header" in where else re.search(r"Header=(BB\w+)", where).group(1))
+        assert len(loops) == 2, (name, loops)  # the requests in front of the first step, and those of the steps
+        for label, where, code in blocks:
+            if label in loops or any(re.search(r"(Header=|Parent Loop )%s\b" % loop, where) for loop in loops):
+                for i, (ins, hand) in enumerate(code):
+                    if ins.startswith("s_waitcnt") and "vmcnt" in ins and not hand:
+                        assert i and re.match(r"(global|flat)_load", code[i - 1][0]), (name, label, ins)
+    assert len(kernels) == 12
+
+
 def _is_instruction(ins):
     return bool(ins) and not ins.startswith((";", ".")) and not ins.endswith(":")

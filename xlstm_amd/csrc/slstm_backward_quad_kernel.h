@@ -53,6 +53,12 @@ constexpr int bwd_quad_lds_bytes(int uw) {
 // several states of the kernel, each pair to be read by itself.  Raised priorities of the matrix or the gradient waves: no difference.)
 constexpr int kBwdQuadSleep = 9;
 
+// What a wave has asked for in front of its loop is there, and the compiler knows it (it reads this builtin, not a wait in inline assembly).  All
+// roles are one function to it: left open, the loads of R at the head of the matrix waves were waited for in the loop of the feeder waves,
+// where another use of the registers stands, that is, every step waited for the requests just made (64 units a workgroup).
+// us of the reverse kernel at 4 heads of 256, T 512, B 25 / 32 / 48 / 64: 615 / 643 / 665 / 740 -> 550 / 580 / 607 / 668.
+__device__ __forceinline__ void settle_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }  // vmcnt(0)
+
 template <int S, int UW, bool DWX16 = false>  // dh = 64 S; UW units a workgroup; DWX16: d_wx takes the gate deltas rounded to bf16
 __global__ __launch_bounds__(bwd_quad_threads(UW)) void slstm_bwd_quad_kernel(BwdSplitParams p) {
   constexpr int dh = S * 64;
@@ -237,6 +243,7 @@ __global__ __launch_bounds__(bwd_quad_threads(UW)) void slstm_bwd_quad_kernel(Bw
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb) bq[ks][cb] = *reinterpret_cast<const uint4 *>(base + ((cb * 64 + lane) << 4));
     }
+    settle_loads();
     // MFMA row r16 holds k-step r16 % 4 (+ 4 a load) of batch row r16 / 4: a load brings PK k-steps, no lane of it is a row that
     // is not there (one k-step a load, its rows at MFMA rows 0, 4, 8, 12: 2.11 ms at B 16 x T 2048 x 4 heads of 256, 2.01 with this)
     const int poll_off = (r16 & 3) < PK ? ((q * 4 + (r16 >> 2)) * PK + (r16 & 3)) * 16 : 0x7FFFFF00;
@@ -320,6 +327,7 @@ __global__ __launch_bounds__(bwd_quad_threads(UW)) void slstm_bwd_quad_kernel(Bw
     const long long o = (long long)row * H + ecol;
     dy = p.d_s_final[o]; dc = p.d_s_final[BH + o]; dn = p.d_s_final[2 * BH + o];
   }
+  settle_loads();
   const int pub_off = member * (UW * 32) + e * 8;
   float c9[9], dht = 0.0f;
   bool restart = false, zero_dy = false;
