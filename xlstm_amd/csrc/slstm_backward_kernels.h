@@ -593,8 +593,8 @@ __global__ __launch_bounds__(256) void slstm_bwd_arm_kernel(uint4 *xch, long lon
 // instead of 2, 16 at B 192.)
 // Bytes between two touches: a miss of the L2 brings 64 bytes, half a line (the same call with 128: 1.85 -> 1.73).
 constexpr int bwd_touch(int rows) { return rows == 4 ? 64 : 128; }
-// ROWS: batch rows of a row tile; DEPTH: steps the feeder waves ask ahead
-template <bool BF16, int S, int ROWS, int DEPTH>
+// ROWS: batch rows of a row tile; DEPTH: steps the feeder waves ask ahead; THREADS: those of a workgroup that come here
+template <bool BF16, int S, int ROWS, int DEPTH, int THREADS>
 __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int xcd, int which, int of) {
   constexpr int ESZ = BF16 ? 2 : 4;
   constexpr int dh = 64 * S;
@@ -604,7 +604,7 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
   constexpr int PER_ROW = dh * ESZ / TOUCH;         // touches of a row of d_h
   constexpr int DL = ROWS * PER_ROW;
   const int H = p.NH * dh, ntiles = (p.B + ROWS - 1) / ROWS, ngroups = p.NH * ntiles;
-  const int tid = threadIdx.x, nthreads = blockDim.x, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
   if (xcd >= ngroups || of < 1) return;
   const int G = (ngroups - xcd + 7) >> 3;           // groups of this XCD: xcd, xcd + 8, ...
   const BwdPace pace = bwd_pace(ROWS, (long long)G * (CL + DL) * TOUCH, DEPTH);
@@ -654,14 +654,14 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
     const u32x4_t crs = {uniform((uint32_t)cb), uniform((uint32_t)(cb >> 32) & 0xFFFFu), uniform((uint32_t)coef_step), 0x00020000u};
     const u32x4_t drs = {uniform((uint32_t)db), uniform((uint32_t)(db >> 32) & 0xFFFFu), uniform((uint32_t)dh_step), 0x00020000u};
     // (uniform trip counts: lanes past the end ask past the buffer's end)
-    for (int i0 = which * nthreads; i0 < G * CL; i0 += of * nthreads) {
+    for (int i0 = which * THREADS; i0 < G * CL; i0 += of * THREADS) {
       const int i = i0 + tid;
       const int j = i / CL, l = i - j * CL;
       const int g = xcd + 8 * j, head = g % p.NH, tile = g / p.NH;
       const uint32_t coff = i < G * CL ? (uint32_t)(((tile * p.NH + head) * S) * PIECE + l * TOUCH) : 0xFFFFFF00u;
       bwd_fetch_to_lds_b128(crs, uniform(dump_lds), coff);
     }
-    for (int i0 = which * nthreads; i0 < G * DL; i0 += of * nthreads) {
+    for (int i0 = which * THREADS; i0 < G * DL; i0 += of * THREADS) {
       const int i = i0 + tid;
       const int j = i / DL, l = i - j * DL;
       const int g = xcd + 8 * j, head = g % p.NH, tile = g / p.NH;
@@ -728,7 +728,7 @@ __global__ __launch_bounds__(FEED ? 768 : 512) void slstm_bwd_split_kernel(BwdSp
   const int ngroups = p.NH * ((p.B + 15) / 16);
   const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
   if (local >= p.main_locals) {
-    bwd_tile_prefetch<BF16, S, 16, 2>(p, xcd, local - p.main_locals, (int)(gridDim.x >> 3) - p.main_locals);
+    bwd_tile_prefetch<BF16, S, 16, 2, FEED ? 768 : 512>(p, xcd, local - p.main_locals, (int)(gridDim.x >> 3) - p.main_locals);
     return;
   }
   const int group = (local / S) * 8 + xcd, s = local % S;

@@ -32,6 +32,12 @@ namespace {
 constexpr int kBwdQuadSlots = 8;
 constexpr int kBwdQuadFeeders = 4;                 // feeder wave f brings the inputs of the steps n = f (mod 4)
 constexpr int kBwdQuadDepth = 6;                   // steps the feeder waves request ahead
+// Threads of a prefetching workgroup that do so, whatever a computing one has: what many waves touch at once stands in front of the
+// polls and requests of the other compute units.  us of the reverse kernel with 64 / 128 / 192 / 256 / 512 / all (704 with 32 units a
+// workgroup, 1,024 with 64) threads: 4 heads of 256, B 16 x T 2048 1,820 / 1,608 / 1,568 / 1,636 / 1,710 / 1,762, T 512, B 8 441 / 384 / 384 /
+// 384 / 386 / 385, B 28 466 / 477 / 467 / 495 / 519 / 565, B 48 552 / 545 / 541 / 554 / 562 / 604, B 56 (no room for more than four per XCD)
+// 622 / 617 / 615 / 613 / 613 / 617; 8 of 128, B 28 422 / 419 / 439 / 425 / 448 / 478.
+constexpr int kBwdQuadPrefetchThreads = 192;
 static_assert(kBwdQuadDepth >= 3 && kBwdQuadDepth <= kBwdQuadSlots && kBwdQuadDepth <= kBwdQuadFeeders + 2, "feeder depth");
 // a slot of the feeder waves: the coefficients [4 rows][9][UW] in whole loads, d_h (4 rows in a landing zone of 1 KiB), the reset
 // flags of the 4 rows as words (in a landing zone of 256 bytes)
@@ -84,7 +90,8 @@ __global__ __launch_bounds__(bwd_quad_threads(UW)) void slstm_bwd_quad_kernel(Bw
   const long long wg_start = wall_clock64();
 #endif
   if (local >= p.main_locals) {
-    bwd_tile_prefetch<true, S, 4, kBwdQuadDepth>(p, xcd, local - p.main_locals, (int)(gridDim.x >> 3) - p.main_locals);
+    if (threadIdx.x < kBwdQuadPrefetchThreads)  // (the others end here: a barrier waits for the waves that are left)
+      bwd_tile_prefetch<true, S, 4, kBwdQuadDepth, kBwdQuadPrefetchThreads>(p, xcd, local - p.main_locals, (int)(gridDim.x >> 3) - p.main_locals);
     return;
   }
   const int group = (local / M) * 8 + xcd, member = local % M;
