@@ -89,3 +89,19 @@ def test_the_prefetch_stays_in_its_share_of_the_cache_and_ahead_of_the_feeder_wa
     _run(tmp_path, _WALK)
     kernel = open(os.path.join(CSRC, "slstm_backward_kernels.h")).read()
     assert "= bwd_pace(ROWS, " in kernel and "m = bwd_pace_resume(m, at, DEPTH);" in kernel and "next_look = m + pace.every;" in kernel
+
+
+def test_a_look_leaves_its_result_where_no_wave_still_reads_the_one_before(tmp_path):
+    """Look k: a first barrier, the result, a second barrier, everybody reads.  A wave may read as late as its first barrier of
+    look k + 1, and the looking wave writes look k + 1's word in front of that barrier: not the same word.  Its write for look
+    k + 2 is behind it."""
+    _run(tmp_path, r"""
+int main() {
+  for (int k = 0; k < 1000; ++k)
+    if (bwd_look_word(k) == bwd_look_word(k + 1) || bwd_look_word(k) < 0 || bwd_look_word(k) > 1) return 1;
+  return 0;
+}
+""")
+    kernel = open(os.path.join(CSRC, "slstm_backward_kernels.h")).read()
+    assert "int *const found = &slowest[bwd_look_word(looks++)];" in kernel and "int slowest[2];" in kernel
+    assert len(re.findall(r"\bslowest\b(?!\[)", kernel)) == 0  # (nothing goes past the rule)

@@ -613,13 +613,14 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
   // every wave lands in the same kilobyte, which nobody reads.
   __shared__ uint4 dump[64];
   const uint32_t dump_lds = (uint32_t)(unsigned long long)((__attribute__((address_space(3))) unsigned char *)dump);
-  __shared__ int slowest;      // the least progress among the XCD's groups; -1: stop
+  __shared__ int slowest[2];   // the least progress among the XCD's groups; -1: stop (bwd_look_word)
   const long long coef_step = (long long)ngroups * S * PIECE;  // bytes of one step's coefficients, all groups
   const long long dh_step = (long long)p.B * H * ESZ;
-  int next_look = pace.ahead;
+  int next_look = pace.ahead, looks = 0;
   for (int m = 0; m < p.T; ++m) {
     if (m >= next_look) {  // (the groups' progress is read through the L2)
-      if (tid == 0) slowest = 0x7FFFFFFF;
+      int *const found = &slowest[bwd_look_word(looks++)];
+      if (tid == 0) *found = 0x7FFFFFFF;
       __syncthreads();
       if (tid < 64) {
         int spins = 0;
@@ -630,18 +631,18 @@ __device__ __forceinline__ void bwd_tile_prefetch(const BwdSplitParams &p, int x
             least = at < least ? at : least;
           }
           if (__builtin_amdgcn_ballot_w64(least < m - pace.ahead) == 0ull) {  // (lanes without a group: the largest int)
-            if (lane < G) atomicMin(&slowest, least);
+            if (lane < G) atomicMin(found, least);
             break;
           }
           if (++spins > (1 << 16) || __hip_atomic_load(p.abort_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-            if (lane == 0) slowest = -1;
+            if (lane == 0) *found = -1;
             break;
           }
           __builtin_amdgcn_s_sleep(8);
         }
       }
       __syncthreads();
-      const int at = slowest;
+      const int at = *found;
       if (at < 0) break;
       // (fallen behind what the feeder waves have already asked for: skip to where a touch can still come first)
       m = bwd_pace_resume(m, at, DEPTH);

@@ -43,4 +43,8 @@ XS_RULE BwdPace bwd_pace(int rows, long long step_bytes, int depth) {
 // by then (up to step at + depth) is past help.
 XS_RULE int bwd_pace_resume(int m, int at, int depth) { return m < at + depth + 1 ? at + depth + 1 : m; }
 
+// Which of the two words the k-th look leaves its result in for the other waves: while one of them may still have to read a word, the wave
+// that looks writes the other (between two looks it passes no barrier that they have not).
+XS_RULE int bwd_look_word(int k) { return k & 1; }
+
 }  // namespace
