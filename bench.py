@@ -220,7 +220,8 @@ def serial_bound(device):
     """The dependency chain of one timestep, measured by ``xs_measure_stage`` (the product kernel's instructions, layouts
     and exchange protocol; every iteration needs the result of the one before).  ``config2_chain``: the whole chain as
     one loop - barrier, poll, MFMAs, fold and row shifts, gating, publication - on 16 head groups of 16 compute
-    units, with none of the product kernel's other work: the serial bound of a step of this structure.  The stages alone
+    units, with none of the product kernel's other work: what the chain takes by itself (no lower bound: where its loop
+    starts in the code and when it polls move it by 0.05 us, and the product kernel may do better).  The stages alone
     (each its own loop, so their sum is more than the chain: every loop pays its own entry and waits) say where it
     goes.  Per-iteration times are differences between two step counts, so launches and set-up cancel.  Also the floor
     of a dependent launch (the decode step's)."""
@@ -737,7 +738,7 @@ def main():
     ap.add_argument("--serial-bound", action="store_true",
                     help="only measure the stages of a timestep's dependency chain and the launch floor (their own JSON line)")
     ap.add_argument("--headline-only", action="store_true",
-                    help="leave out the other BASELINE configs, the backward pass and the serial bound (profiling runs)")
+                    help="leave out the other BASELINE configs, the backward pass and the chain alone (profiling runs)")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="only run a plain 1 GiB device copy 5 times (scales the rocprofv3 FETCH_SIZE/WRITE_SIZE counters)")
     args = ap.parse_args()
@@ -770,7 +771,7 @@ def main():
         print(json.dumps({"copy_bytes_each_way": src.numel() * 4, "copies": 5}))
         return
     if args.serial_bound:
-        print(json.dumps({"serial_bound": serial_bound(device)}))
+        print(json.dumps({"chain_alone": serial_bound(device)}))
         return
     if args.decode_only:
         dec = bench_decode(device)
@@ -858,14 +859,13 @@ def main():
         out["roofline"]["traffic_source"] = "profiles/traffic_seq_cfg2.json (rocprofv3 counters of a separate run, not of this one)"
     lean = args.headline_only or args.no_decode  # (profiling runs want the one kernel)
     if not lean:
-        # the stages of the chain measured in this run, and what the measured step is against their sum
+        # the chain of a step and its stages, each measured alone in this run
         sb = serial_bound(device)
-        out["roofline"]["serial_bound_stages_us"] = sb
+        out["roofline"]["chain_alone_stages_us"] = sb
         if sb.get("config2_chain_us_per_step"):
-            out["roofline"]["serial_bound_us_per_step"] = sb["config2_chain_us_per_step"]
-            out["roofline"]["frac_of_serial_bound"] = sb["config2_chain_us_per_step"] / (kern_ms * 1e3 / T)
-            out["roofline"]["serial_bound_source"] = ("measured in this run: xs_measure_stage(XS_STAGE_CHAIN), the step's "
-                                                      "dependency chain alone on 16 head groups of 16 compute units")
+            out["roofline"]["chain_alone_us_per_step"] = sb["config2_chain_us_per_step"]
+            out["roofline"]["chain_alone_source"] = ("measured in this run: xs_measure_stage(XS_STAGE_CHAIN), the step's "
+                                                     "dependency chain alone on 16 head groups of 16 compute units; no lower bound")
         # the other BASELINE configurations and the backward pass, compact (full rows: --all-configs)
         c1 = bench_config(device, "config 1: B=4 T=256 D=512 NH=4 fp32, no resets", 4, 256, 4, 128, False, 0)
         c4 = bench_config(device, "config 4 (one sLSTM cell): B=8 T=2048 D=1024 NH=4 bf16, documents mean 768", 8, 2048, 4, 256, True, 768)
@@ -903,7 +903,7 @@ def main():
             out["decode"]["other_head_dims"] = bench_decode_other_head_dims(device)
         if not lean:
             # a decode step is one dependent launch: its floor is the launch itself plus the step's bytes at the HBM peak
-            launch = out["roofline"]["serial_bound_stages_us"].get("dependent_launch_us")
+            launch = out["roofline"]["chain_alone_stages_us"].get("dependent_launch_us")
             if launch:
                 dr = out["decode"]["roofline"]
                 dr["dependent_launch_floor_us"] = launch

@@ -501,7 +501,7 @@ int xs_slstm_backward_tile_r(const xs_slstm_bwd_args *args);
  * Measurement (no counterpart in the reference): one stage of the dependency chain of a timestep of the sequence
  * kernel, run alone for `steps` iterations in which every iteration needs the result of the one before, with the
  * product kernel's instructions, layouts and exchange protocol.  The caller times the call (events on `stream`) at two
- * step counts and divides the difference; the sum of the three stages is the serial bound of a step.
+ * step counts and divides the difference.  (The three stages add up to more than the chain; neither bounds a step from below.)
  *   XS_STAGE_EXCHANGE     `members` compute units (8, 16, 32 or 64; one XCD, or with two_xcds != 0 half each on XCDs 0
  *                         and 4 with device-scope stores) publish a 16 x 16 bf16 tile each and poll the group's tile of
  *                         `rows` batch rows until it is complete.  Workspace: 256 + 8 * members * 512 bytes; word 0 is

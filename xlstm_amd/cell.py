@@ -536,7 +536,7 @@ class sLSTMCell_hip(nn.Module):
         args = (x, r, self._bias_.detach().view(self.config.num_heads, 4, self.head_dim), state, reset_mask)
         coef = h = s = None
         if wants_grad and self.keep_backward_coefficients and x.is_cuda and not step:
-            if self.head_dim == 256:  # (bfloat16: row tiles of 4 rows x 64 units in the backward, where they fit)
+            if self.head_dim == 256:  # (bfloat16: row tiles of 4 rows in the backward, where they fit)
                 coef = F_hip.backward_coefficients_buffer(x, self.config.num_heads, kept=True)
             if coef is None and 9 * x.numel() <= F_hip.KEPT_COEFFICIENT_BYTES:
                 coef = F_hip.training_coefficients(x, self.config.num_heads, kept=True)
@@ -586,8 +586,10 @@ class sLSTMCell_hip(nn.Module):
 
     def _trains_natively(self, input: torch.Tensor) -> bool:
         """Whether a training call takes the native host path.  Not where the coefficients are not to be kept, and for long
-        bfloat16 sequences at head dim 256: forward and backward in row tiles of 4 rows save 0.1 to 0.2 us a step there and take
-        three more launches (us a call, native / those: 4 heads B 16 T 320 584 / 588, T 383 682 / 673; B 4 T 256 441 / 439)."""
+        bfloat16 sequences at head dim 256: forward and backward in row tiles of 4 rows save 0.2 to 0.3 us a step there, and their
+        host path takes 0.40 to 0.45 ms a call (us a call, native / those, T 256, 320, 383: 4 heads B 16 489 / 499, 589 / 592, 688 / 680, B 8
+        476 / 483, 571 / 573, 668 / 649, B 4 445 / 445, 547 / 544, 648 / 633; 8 heads B 8 489 / 506, 588 / 593, 688 / 684; 1 head B 1 420 / 420,
+        515 / 501, 608 / 585: a few per cent are left between 320 and 383 steps)."""
         return (self.keep_backward_coefficients and 9 * input.numel() <= F_hip.KEPT_COEFFICIENT_BYTES
                 and not (self.head_dim == 256 and input.dtype == torch.bfloat16
                          and input.shape[1 if self.config.input_shape == "BSGNH" else 0] >= 384))

@@ -628,10 +628,12 @@ __global__ __launch_bounds__(kThreads + 64 * max_prefetch_waves(NCH)) void slstm
       // to the poll: 1.53).  Then the loop's start moved over the eight phases of a 32-byte line of code:
       // 1.517 .. 1.573, the best one taken.  (K split over the waves, below: 1.70.)  One barrier for two or four steps, W.x and h in
       // rings of as many: 1.51 and 1.55 (the waves beside these then come in bursts).  With polls of lanes side by side (quad_word) a
-      // call takes 1.163 ms instead of 1.450 (bf16 4 x 512 B 4 T 600 0.622 -> 0.451, float32 4 x 128 B 4 T 256 0.196 -> 0.174), the eight
-      // phases 1.163 .. 1.195; s_sleeps none / 1 / 2: bf16 1.212 / 1.169 / 1.203, with coefficients for slstm_bwd_quad_kernel (a training
-      // call) 3.581 / 3.511 / 3.461, head dim 512 0.451 / 0.452 / 0.461; float32 head dim 128 0.174 / 0.181 / 0.184, 200 (B 9 T 500)
-      // 0.525 / 0.517 / 0.501.
+      // call takes 1.163 ms instead of 1.450 (bf16 4 x 512 B 4 T 600 0.629 -> 0.453; float32 4 x 128 B 4 T 256 with inputs of its own, us, 213 -> 201,
+      // with the same inputs call after call 196 -> 173: W.x from memory is what the difference waits for), the eight
+      // phases 1.163 .. 1.195.  s_sleeps none / 1 / 2, us a call with inputs of its own (the same order with the same inputs): bf16 1205 / 1164 / 1205,
+      // with coefficients for slstm_bwd_quad_kernel (a training call of T 1024) 1621 / 1596 / 1571, head dim 512 (B 4 T 600) 455 / 453 / 463; float32
+      // head dim 128 200.6 / 206.7 / 209.4, 96 in training (B 6 T 250) 429.5 / 432.5 / 438.4, 200 (B 4 T 256) 295.7 / 295.2 / 292.8, 256 in
+      // training (B 4 T 200) 473.9 / 474.8 / 478.0, 512 forward (2 heads, B 4 T 128) 233.4 / 234.0 / 233.6 and in training 462.6 / 461.6 / 463.4.
       const int buf = t & 1;
       float wxv[4];
       XS_QTICK(5);

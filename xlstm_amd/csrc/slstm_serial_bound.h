@@ -4,8 +4,9 @@
 // A timestep of slstm_seq_kernel is a chain: the peers' h arrives -> MFMAs over this workgroup's 64 columns -> the
 // gates of a unit brought together -> exponential gating -> h published -> it arrives at the peers.  stage_chain_kernel
 // runs that chain, as the kernel for row tiles of 4 rows makes it, with the same instructions, layouts and protocol
-// and nothing else: what a step of this structure costs when only the chain is left, the serial bound that bench.py
-// reports next to the measured time per step.  The other kernels run its stages alone (each its own loop: their sum is
+// and nothing else: what a step of this structure costs when only the chain is left, at the pause and the phase of its loop
+// that are best for it (it is measured, not derived: a chain with other ones takes up to 0.08 us more).  bench.py reports it next to the
+// measured time per step.  The other kernels run its stages alone (each its own loop: their sum is
 // more than the chain) and the exchange in the layouts of the other sequence kernels.
 #pragma once
 
@@ -214,17 +215,18 @@ __global__ __launch_bounds__(256) void stage_chain_kernel(StageParams p) {
   CellState st{0.0f, 0.0f, 0.0f, 0.0f};
   uint32_t max_spins = 0;
   bool dead = false;
-  // (the loop's start relative to a 32-byte line of code, chosen like the product kernel's: the best of the eight,
-  // 0.638 us per step; five others 0.64, two 0.81)
+  // (pause and start of the loop relative to a 32-byte line of code, each measured with the other, us a step over the eight
+  // phases: no pause 0.574 .. 0.621, one unit 0.584 .. 0.618, three 0.569 .. 0.615, four 0.568 .. 0.607, five 0.596 .. 0.618, eight 0.679 ..
+  // 0.699; the product kernel reads its W.x from LDS in front of its one unit)
 #ifndef XS_CHAIN_PAD
-#define XS_CHAIN_PAD 6
+#define XS_CHAIN_PAD 4
 #endif
   asm volatile(".p2align 5\n\t.rept %0\n\ts_nop 0\n\t.endr" :: "n"(XS_CHAIN_PAD));
   for (int t = 0; t < p.steps; ++t) {
     uint16_t *const cur = reinterpret_cast<uint16_t *>(xbase + (t % kRing) * xslot);
     uint16_t *const old = reinterpret_cast<uint16_t *>(xbase + ((t + kRing - 2) % kRing) * xslot);
     lds_barrier();
-    __builtin_amdgcn_s_sleep(1);
+    __builtin_amdgcn_s_sleep(4);
     uint4 areg[NCH];
     if (t == 0) {
 #pragma unroll

@@ -281,7 +281,7 @@ def slstm_backward(
     if tuple(h_out.shape) != (T, B, H) or tuple(d_h.shape) != (T, B, H):
         raise ValueError(f"h_out and d_h must be [S, B, H] = {(T, B, H)}")
     # Unless a kernel is asked for by name: the reverse pass of one launch from a training forward's coefficients.  bf16 at
-    # head dim 256 keeps the kernel for row tiles of 4 rows x 64 units (its prefetching workgroups: 1.03 us a step) where it fits
+    # head dim 256 keeps the kernel for row tiles of 4 rows (its prefetching workgroups: 0.76 us a step) where it fits
     from_training = ((coef is None or coef.dim() == 1) and split_override is None and row_tile_override is None and not stepwise_override
                      and not (coef is None and bf16 and dh == 256 and _quad_fits(B, T, NH, dh, wx.device))
                      and lib.xs_slstm_train_coef_floats(B, T, NH, dh, _DTYPE_CODE[wx.dtype]))
@@ -385,7 +385,7 @@ def slstm_backward(
     if stepwise:
         split = False
     # row tiles of 4 rows (bf16, head dims up to 256) where four times the workgroups still fit (the prefetching ones
-    # take what room is left: without any, at B 64 x 4 heads of 256, the reverse kernel still takes 2.6 ms against 4.2
+    # take what room is left: without any, at B 64 x T 512 x 4 heads of 256, the reverse kernel still takes 0.66 ms against 1.05
     # with row tiles of 16 rows)
     groups4 = NH * ((B + 3) // 4)
     quad = (split and bf16 and dh <= 256 and (groups4 + 7) // 8 * 8 * S <= _compute_units(dev)
