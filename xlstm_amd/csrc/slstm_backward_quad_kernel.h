@@ -17,8 +17,9 @@
 // multiply as well, their first look left 280 cycles after the others'), and the MFMAs, of which a tile of 4 rows leaves three quarters
 // empty, are split over twice the workgroups (UW 32) where these fit: 128 of 16 cycles a step and workgroup at head dim 256 with UW 64.
 // ms a training call at 4 heads of 256, one form of wave and UW 64 -> these roles and UW 64 -> UW 32: B 16 x T 1024 1.757 -> 1.751 -> 1.694, B 8 x T 512
-// 0.904 -> 0.866 -> 0.816, 2 heads B 5 x T 600 1.010 -> 0.967 -> 0.910, 3 heads B 16 x T 400 0.766 -> 0.736 -> 0.720.  What is left at B 16 is coefficients
-// that are not in the L2 yet when a feeder wave asks (1.56 when they always are): its loads then hold up the looks behind them.
+// 0.904 -> 0.866 -> 0.816, 2 heads B 5 x T 600 1.010 -> 0.967 -> 0.910, 3 heads B 16 x T 400 0.766 -> 0.736 -> 0.720.  (Each pair with the
+// prefetch of then; with its pace, its threads and the waits as they are now 1.567, 0.818, 0.909, 0.700.  Where the coefficients always are in
+// the L2, B 16 x T 1024 takes 1.56.)
 //
 // K is ordered (unit of the head, gate): the four deltas of an element are 8 bytes and a thread publishes them with one store.  Matrix
 // wave w multiplies KS k-steps (of 32 inputs, 8 units) of the head.  Batch row b takes the MFMA rows 4 b .. 4 b + 3, each with another of
@@ -100,7 +101,7 @@ __global__ __launch_bounds__(bwd_quad_threads(UW)) void slstm_bwd_quad_kernel(Bw
   const int row0 = (group / p.NH) * 4;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, r16 = lane & 15;
   char *const feed = reinterpret_cast<char *>(part + 2 * NMW * PART);
-  // the deltas of the step before, for the feeder waves to write to d_wx: [2][row][UW units][4 gates].  (Stores of the waves
+  // the deltas of the step before, for the drainer wave (or the feeder waves) to write to d_wx: [2][row][UW units][4 gates].  (Stores of the waves
   // that form the gradient stood in front of their look at the peers' deltas, which waits for their acknowledgement.)
   typedef typename std::conditional<DWX16, uint16_t, float>::type wx_t;
   wx_t *const stash = reinterpret_cast<wx_t *>(feed + kBwdQuadSlots * FSLOT);
@@ -111,8 +112,8 @@ __global__ __launch_bounds__(bwd_quad_threads(UW)) void slstm_bwd_quad_kernel(Bw
   const int rows_there = p.B - row0 < 4 ? p.B - row0 : 4;
   constexpr bool DRAINS = bwd_quad_drains(UW);
   if (DRAINS && wave == NMW + NGW + kBwdQuadFeeders) {
-    // ---- the drainer wave: the step's deltas to d_wx, and the group's progress.  (Nothing waits for its stores; From the feeder waves
-    //      their wait for their loads was one for these stores too.)
+    // ---- the drainer wave: the step's deltas to d_wx, and the group's progress.  (Nothing waits for its stores; from the feeder waves,
+    //      whose waits for their loads were waits for these stores too, they held up the requests.)
     __syncthreads();  // P
     typedef wx_t pair_t __attribute__((ext_vector_type(2)));
     const int unit = 2 * (lane & 15), g = lane >> 4;
@@ -388,7 +389,7 @@ __global__ __launch_bounds__(bwd_quad_threads(UW)) void slstm_bwd_quad_kernel(Bw
       *reinterpret_cast<uint2 *>(ring + ((n + kBwdRing - 2) % kBwdRing) * ring_stride + pub_off) = uint2{0xFFFFFFFFu, 0xFFFFFFFFu};
     }
     XS_BTICK(1);
-    // ---- while the deltas are on their way: their copies for the feeder waves, the next step's inputs
+    // ---- while the deltas are on their way: their copies for d_wx, the next step's inputs
     wx_t *const copy = stash + (((n & 1) * 4 + prow) * UW + pu) * 4;
     if constexpr (DWX16) *reinterpret_cast<uint2 *>(copy) = uint2{pack_bf16x2(delta[0], delta[1]), pack_bf16x2(delta[2], delta[3])};
     else *reinterpret_cast<f32x4 *>(copy) = f32x4{delta[0], delta[1], delta[2], delta[3]};
